@@ -31,11 +31,16 @@ SIGNATURES = {
     "fmoe_routing_workspace_bytes": (_i64, [_i64, _i64]),
     "fmoe_assign_pos": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp]),
     "fmoe_route": (_int, [_vp, _i64, _i64, _vp, _vp, _vp, _vp, _i64, _vp]),
+    "fmoe_route_table": (_int, [_vp, _i64, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _vp]),
     "fmoe_route_static": (_int, [_vp, _i64, _i64, _vp, _vp, _vp, _vp]),
     "fmoe_gate_topk_route": (_int, [_vp, _i64, _i64, _i64, _int, _int, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
+    "fmoe_gate_topk_route_table": (_int, [_vp, _i64, _i64, _i64, _int, _int, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64,
+                                          _vp]),
     "fmoe_gate_linear_supported": (_int, [_i64, _i64, _i64, _int]),
     "fmoe_gate_linear_topk_route": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp, _vp, _vp, _vp, _vp, _vp,
                                            _i64, _vp]),
+    "fmoe_gate_linear_topk_route_table": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp, _vp, _vp, _vp, _vp,
+                                                 _vp, _i64, _vp, _i64, _vp]),
     "fmoe_gate_topk_backward": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _int, _vp]),
     "fmoe_noisy_gate_forward": (_int, [_vp, _vp, _vp, ctypes.c_double, _i64, _i64, _i64, _int, _vp, _vp, _vp, _vp, _vp,
                                        _vp, _vp, _vp, _vp, _i64, _vp]),

@@ -15,8 +15,10 @@
 //
 // The index arrays are a few hundred KB at most, so these kernels are bound by
 // launch and memory latency, not by HBM bandwidth; the design keeps them to
-// three short launches with coalesced 8-byte loads.
+// three short launches with coalesced 8-byte loads, and for few slots (fmoe_route
+// and the gates) to a single one.
 #include "common.hpp"
+#include "segment_table.hpp"
 
 #include <mutex>
 #include <type_traits>
@@ -154,24 +156,33 @@ __global__ __launch_bounds__(kBlock) void block_scan_kernel(
 }
 
 // fmoe_route: a single 1024-thread workgroup does the per-expert prefix over
-// workgroups and then the inclusive cumsum over experts.
-constexpr int kRouteScanBlock = 1024;
+// workgroups and then the inclusive cumsum over experts, and, for at most
+// segtab::kSmallExperts experts, the segment table of the counts (`table`, may be null)
+// that the grouped GEMMs read.
+constexpr int kRouteScanBlock = segtab::kThreads;
 __global__ __launch_bounds__(kRouteScanBlock) void route_scan_kernel(
     int32_t *__restrict__ block_hist, int n_blocks, int n_expert,
-    int64_t *__restrict__ expert_count, int32_t *__restrict__ cum_incl) {
+    int64_t *__restrict__ expert_count, int32_t *__restrict__ cum_incl, int rows_cap, int32_t *__restrict__ table) {
     __shared__ int32_t wave_sum[kRouteScanBlock / kWave];
     __shared__ int32_t carry_s;
+    __shared__ segtab::SmallLds table_lds;
     if (threadIdx.x == 0) carry_s = 0;
     __syncthreads();
+    int32_t run = 0;
     for (int e0 = 0; e0 < n_expert; e0 += kRouteScanBlock) {
         const int e = e0 + threadIdx.x;
-        int32_t run = 0;
+        run = 0;
         if (e < n_expert) {
-            for (int b = 0; b < n_blocks; ++b) {
-                int32_t *cell = block_hist + (int64_t)b * n_expert + e;
-                const int32_t c = *cell;
-                *cell = run;
-                run += c;
+            // the cells go out eight at a time: one by one, each waits for the store before it
+            for (int b0 = 0; b0 < n_blocks; b0 += 8) {
+                int32_t c[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) c[j] = b0 + j < n_blocks ? block_hist[(int64_t)(b0 + j) * n_expert + e] : 0;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    if (b0 + j < n_blocks) block_hist[(int64_t)(b0 + j) * n_expert + e] = run;
+                    run += c[j];
+                }
             }
             expert_count[e] = run;
         }
@@ -192,6 +203,88 @@ __global__ __launch_bounds__(kRouteScanBlock) void route_scan_kernel(
         if (threadIdx.x == kRouteScanBlock - 1) carry_s = v + before;
         __syncthreads();
     }
+    if (table != nullptr) segtab::small_table(run, n_expert, rows_cap, table, table_lds);
+}
+
+// Few slots: histogram, scan, placement and segment table in one launch of one workgroup.  Wave w owns
+// the slots [w * 64 steps, (w + 1) * 64 steps) and keeps its keys and match masks in registers between
+// the passes; its table in LDS is a histogram first and the running ranks afterwards, as in
+// block_hist_kernel and rank_apply_kernel.  The four separate launches took 26 us for 64 slots, 34 us for
+// 509 and 25 us for 8192, nearly all of it launch and memory latency; this one takes 8, 10 and 13 us.
+// Up to kSmallSlots a wave has no more steps to walk than one of rank_apply_kernel's.
+constexpr int kSmallBlock = segtab::kThreads, kSmallWaves = kSmallBlock / kWave;
+constexpr int kSmallSlots = kSmallBlock * kStepsPerWave;   // 8192
+__global__ __launch_bounds__(kSmallBlock) void route_small_kernel(
+    const int64_t *__restrict__ gate, int n_slots, int n_expert, int nbits, int64_t *__restrict__ expert_count,
+    int64_t *__restrict__ pos, int64_t *__restrict__ slot_to_row, int32_t *__restrict__ table) {
+    extern __shared__ int32_t bins[];  // [kSmallWaves][n_expert], then the inclusive cumsum [n_expert]
+    __shared__ segtab::SmallLds table_lds;
+    __shared__ int32_t wave_sum[kSmallWaves];
+    int32_t *cum = bins + kSmallWaves * n_expert;
+    const int wave = threadIdx.x / kWave;
+    int32_t *mine = bins + wave * n_expert;
+    const int steps = (n_slots + kSmallBlock - 1) / kSmallBlock;
+    const int wave_base = wave * steps * kWave;
+    int keys[kStepsPerWave];
+#pragma unroll
+    for (int s = 0; s < kStepsPerWave; ++s) {
+        const int i = wave_base + s * kWave + lane_id();
+        int64_t g = -1;
+        if (s < steps && i < n_slots) g = gate[i];
+        keys[s] = (g >= 0 && g < n_expert) ? (int)g : -1;
+    }
+    for (int e = threadIdx.x; e < kSmallWaves * n_expert; e += kSmallBlock) bins[e] = 0;
+    __syncthreads();
+    uint64_t peers[kStepsPerWave];
+#pragma unroll
+    for (int s = 0; s < kStepsPerWave; ++s) {
+        peers[s] = 0;
+        if (s < steps) {
+            peers[s] = match_mask(keys[s], keys[s] >= 0, nbits);
+            wave_bins_add(mine, keys[s], keys[s] >= 0, peers[s]);
+        }
+    }
+    __syncthreads();
+    // thread e: expert e's counts per wave -> starting ranks, its total, and the cumsum over the experts
+    const int e = threadIdx.x;
+    int32_t total = 0;
+    if (e < n_expert) {
+#pragma unroll
+        for (int w = 0; w < kSmallWaves; ++w) {
+            const int32_t c = bins[w * n_expert + e];
+            bins[w * n_expert + e] = total;
+            total += c;
+        }
+        expert_count[e] = total;
+    }
+    int32_t v = total;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int32_t up = __shfl_up(v, off, kWave);
+        if (lane_id() >= off) v += up;
+    }
+    if (lane_id() == kWave - 1) wave_sum[wave] = v;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) v += wave_sum[w];
+    if (e < n_expert) cum[e] = v;
+    __syncthreads();
+    const int routed = cum[n_expert - 1];
+#pragma unroll
+    for (int s = 0; s < kStepsPerWave; ++s) {
+        if (s >= steps) break;
+        const int i = wave_base + s * kWave + lane_id();
+        const int key = keys[s];
+        const bool valid = key >= 0;
+        int32_t rank = 0;
+        if (valid) rank = mine[key] + __popcll(peers[s] & lanes_below());
+        wave_lds_sync();
+        wave_bins_add(mine, key, valid, peers[s]);
+        const int row = valid ? cum[key] - 1 - rank : -1;
+        if (valid) pos[row] = i;
+        if (slot_to_row && i < n_slots) slot_to_row[i] = row;
+        if (i < n_slots && i >= routed) pos[i] = -1;
+    }
+    if (table != nullptr) segtab::small_table(total, n_expert, n_slots, table, table_lds);
 }
 
 // ---------------------------------------------------------------- apply ----
@@ -288,78 +381,100 @@ __device__ __forceinline__ void topk_insert(float (&val)[K], int (&idx)[K], floa
     }
 }
 
-// Top-k of the gate logits, the scores of the selected experts and the per-workgroup expert
-// histogram that the routing scan starts from, in one pass over the logits.
-//
-// A workgroup owns kSlotsPerBlock consecutive (token, choice) slots -- the same slots as
-// workgroup b of rank_apply_kernel -- i.e. kSlotsPerBlock / K tokens, 8 / K per thread.  A lane
-// reads its token's row of logits (16 bytes at a time when the rows are aligned) and keeps the K
-// largest in a sorted register list: an insertion is K compare-selects, there is no traffic
-// between lanes, and a later logit only displaces a strictly smaller one, so ties go to the
-// lower expert index.  The choices come out in descending order of the logit.  The wave then
-// adds the selected experts to its private table, one 64-key step per choice.
-// score_mode 0: the selected logit itself; 1: softmax over the K selected logits.
-template <typename T, int K>
-__global__ __launch_bounds__(kBlock) void gate_topk_hist_kernel(
-    const T *__restrict__ logits, int64_t n_tokens, int n_expert, int score_mode, int vector_rows,
-    int64_t *__restrict__ topk_idx, T *__restrict__ topk_score, int32_t *__restrict__ block_hist, int nbits) {
-    extern __shared__ int32_t bins[];  // [kWavesPerBlock][n_expert]
-    int32_t *mine = bins + (threadIdx.x / kWave) * n_expert;
-    for (int e = threadIdx.x; e < kWavesPerBlock * n_expert; e += kBlock) bins[e] = 0;
-    __syncthreads();
+// Merges the sorted lists of the G lanes of a group (G consecutive lanes, a power of two of at least K):
+// K rounds of taking the best head of all lists -- the larger value, of equal ones the lower expert --
+// after which every lane of the group holds the group's K best in out_val / out_idx.  That is the
+// order topk_insert gives a single lane that sees all the experts in ascending order.
+template <int K, int G>
+__device__ __forceinline__ void topk_merge(float (&val)[K], int (&idx)[K], float (&out_val)[K], int (&out_idx)[K]) {
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        float bv = idx[0] >= 0 ? val[0] : -__builtin_inff();
+        int bi = idx[0] >= 0 ? idx[0] : INT32_MAX;
+#pragma unroll
+        for (int off = 1; off < G; off <<= 1) {
+            const float ov = __shfl_xor(bv, off, kWave);
+            const int oi = __shfl_xor(bi, off, kWave);
+            const bool take = ov > bv || (ov == bv && oi < bi);
+            bv = take ? ov : bv;
+            bi = take ? oi : bi;
+        }
+        out_val[j] = bv;
+        out_idx[j] = bi == INT32_MAX ? -1 : bi;
+        const bool pop = idx[0] >= 0 && idx[0] == bi;
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            const float nv = i + 1 < K ? val[i + 1 < K ? i + 1 : i] : -__builtin_inff();
+            const int ni = i + 1 < K ? idx[i + 1 < K ? i + 1 : i] : -1;
+            val[i] = pop ? nv : val[i];
+            idx[i] = pop ? ni : idx[i];
+        }
+    }
+}
 
-    constexpr int kTokensPerBlock = kSlotsPerBlock / K, kTokensPerThread = kTokensPerBlock / kBlock;
+// Scores of a token's K selected experts (descending logits): the logits themselves (score_mode 0) or
+// their softmax (1).
+template <int K>
+__device__ __forceinline__ void topk_scores(const float (&val)[K], const int (&idx)[K], int score_mode, float (&score)[K]) {
+#pragma unroll
+    for (int j = 0; j < K; ++j) score[j] = val[j];
+    if (score_mode == 1) {
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < K; ++j) { score[j] = idx[j] >= 0 ? __expf(val[j] - val[0]) : 0.f; sum += score[j]; }
+#pragma unroll
+        for (int j = 0; j < K; ++j) score[j] /= sum;
+    }
+}
+
+// Lane `sub` < K of a token's group of lanes writes the token's choice number `sub`.
+template <typename T, int K>
+__device__ __forceinline__ void topk_store(int sub, int64_t token, const int (&idx)[K], const float (&score)[K],
+                                           int64_t *__restrict__ topk_idx, T *__restrict__ topk_score) {
+    int i = idx[0];
+    float s = score[0];
+#pragma unroll
+    for (int j = 1; j < K; ++j) { i = sub == j ? idx[j] : i; s = sub == j ? score[j] : s; }
+    if (sub < K) {
+        topk_idx[token * K + sub] = i;
+        topk_score[token * K + sub] = (T)(i >= 0 ? s : 0.f);
+    }
+}
+
+// Top-k of the gate logits and the scores of the selected experts.
+//
+// G lanes share a token: each keeps the K largest of its part of the row (16-byte pieces when the rows
+// are aligned) in a sorted register list -- an insertion is K compare-selects, and a later logit
+// only displaces a strictly smaller one -- and the G lists are merged in K rounds of lane exchanges, so
+// the choices come out in descending order of the logit, ties to the lower expert.  With one lane per token
+// (the routing histogram in the same kernel, 2048 slots per workgroup) a row of 256 logits was a chain
+// of 256 insertions on a few waves: 71 us for 64 tokens and 77 us for 8192 at top-8; 16 lanes per token take
+// 13 us for either, and the histogram is left to the routing kernels.
+template <typename T, int K, int G>
+__global__ __launch_bounds__(kBlock) void gate_topk_kernel(
+    const T *__restrict__ logits, int64_t n_tokens, int n_expert, int score_mode, int vector_rows,
+    int64_t *__restrict__ topk_idx, T *__restrict__ topk_score) {
     constexpr int kVec = 16 / (int)sizeof(T);
-    const float kLowest = -__builtin_inff();
-    for (int it = 0; it < kTokensPerThread; ++it) {
-        const int64_t token = (int64_t)blockIdx.x * kTokensPerBlock + it * kBlock + threadIdx.x;
-        const bool live = token < n_tokens;
-        float val[K];
-        int idx[K];
+    const int sub = threadIdx.x % G;
+    const int64_t token = (int64_t)blockIdx.x * (kBlock / G) + threadIdx.x / G;
+    const T *row = logits + (token < n_tokens ? token : n_tokens - 1) * n_expert;
+    float val[K], best[K], score[K];
+    int idx[K], chosen[K];
 #pragma unroll
-        for (int j = 0; j < K; ++j) { val[j] = kLowest; idx[j] = -1; }
-        auto insert = [&](float x, int e) { topk_insert<K>(val, idx, x, e); };
-        if (live) {
-            const T *row = logits + token * n_expert;
-            int e = 0;
-            if (vector_rows) {
-                for (; e + kVec <= n_expert; e += kVec) {
-                    alignas(16) T chunk[kVec];
-                    *(uint4 *)chunk = *(const uint4 *)(row + e);
+    for (int j = 0; j < K; ++j) { val[j] = -__builtin_inff(); idx[j] = -1; }
+    if (vector_rows) {
+        for (int e = sub * kVec; e < n_expert; e += G * kVec) {
+            alignas(16) T chunk[kVec];
+            *(uint4 *)chunk = *(const uint4 *)(row + e);
 #pragma unroll
-                    for (int c = 0; c < kVec; ++c) insert((float)chunk[c], e + c);
-                }
-            }
-            for (; e < n_expert; ++e) insert((float)row[e], e);
+            for (int c = 0; c < kVec; ++c) topk_insert<K>(val, idx, (float)chunk[c], e + c);
         }
-        float score[K];
-#pragma unroll
-        for (int j = 0; j < K; ++j) score[j] = val[j];
-        if (score_mode == 1) {
-            float sum = 0.f;
-#pragma unroll
-            for (int j = 0; j < K; ++j) { score[j] = idx[j] >= 0 ? __expf(val[j] - val[0]) : 0.f; sum += score[j]; }
-#pragma unroll
-            for (int j = 0; j < K; ++j) score[j] /= sum;
-        }
-#pragma unroll
-        for (int j = 0; j < K; ++j) {
-            const bool chosen = live && idx[j] >= 0;
-            if (live) {
-                topk_idx[token * K + j] = idx[j];
-                topk_score[token * K + j] = (T)(chosen ? score[j] : 0.f);
-            }
-            wave_bins_add(mine, chosen ? idx[j] : 0, chosen, match_mask(chosen ? idx[j] : 0, chosen, nbits));
-        }
+    } else {
+        for (int e = sub; e < n_expert; e += G) topk_insert<K>(val, idx, (float)row[e], e);
     }
-    __syncthreads();
-    int32_t *dst = block_hist + (int64_t)blockIdx.x * n_expert;
-    for (int e = threadIdx.x; e < n_expert; e += kBlock) {
-        int32_t c = 0;
-#pragma unroll
-        for (int w = 0; w < kWavesPerBlock; ++w) c += bins[w * n_expert + e];
-        dst[e] = c;
-    }
+    topk_merge<K, G>(val, idx, best, chosen);
+    topk_scores<K>(best, chosen, score_mode, score);
+    if (token < n_tokens) topk_store<T, K>(sub, token, chosen, score, topk_idx, topk_score);
 }
 
 // The gate's linear layer, its top-k and the scores in one kernel, for up to 64 experts: the logits
@@ -368,11 +483,13 @@ __global__ __launch_bounds__(kBlock) void gate_topk_hist_kernel(
 // takes the steps w, w + 4, ... of 128 bytes per row) and feed the MFMA straight from global
 // memory -- for the 16 x 16 block shapes a lane's operand is 16 contiguous bytes of one row of W
 // (expert lb of a 16-expert block) or of x (token lb of a 16-token block), so there is no staging
-// -- then leave their partial [expert][token] tiles in LDS.  Thread t < kGateTokens adds the four
-// partials of its token's logits in wave order (a fixed order), adds the bias, rounds to the
-// element type (what the layer's own output would have been) and keeps the K largest exactly as
-// gate_topk_hist_kernel does.  The routing histogram is left to the routing kernels that follow:
+// -- then leave their partial [expert][token] tiles in LDS.  Eight lanes per token add the four
+// partials of the token's logits in wave order (a fixed order), add the bias, round to the
+// element type (what the layer's own output would have been) and keep the K largest exactly as
+// gate_topk_kernel does.  The routing histogram is left to the routing kernels that follow:
 // the contraction wants many small workgroups, the histogram few large ones.
+// For few tokens the kernel is one chain of load latencies per workgroup, so a group's loads go out
+// before the group ahead of it is multiplied.
 constexpr int kGateTokens = 32, kGateMaxExpert = 64, kGateStride = kGateTokens + 4;
 
 template <typename T, int K, int kEB>
@@ -438,40 +555,49 @@ __global__ __launch_bounds__(kBlock) void gate_linear_topk_kernel(
     // then depends on where in the batch a token stands; the result stays a fixed function of the input.)
     const int n_groups = (d + kUnroll * kStride - 1) / (kUnroll * kStride);
     const int first = (int)((blockIdx.x * 7u) % (unsigned)n_groups);
-    for (int gi = 0; gi < n_groups; ++gi) {
+    u32x4 a[2][kUnroll][2][kEB], b[2][kUnroll][2][kTB];
+    auto load_group = [&](int gi, u32x4 (&ga)[kUnroll][2][kEB], u32x4 (&gb)[kUnroll][2][kTB]) {
         const int g = gi + first < n_groups ? gi + first : gi + first - n_groups;
         const int k0 = g * (kUnroll * kStride) + wave * kStep;
         if (k0 + (kUnroll - 1) * kStride + kStep <= d) {
-            // a whole group of kUnroll steps: every load goes out before the first product needs one
-            u32x4 a[kUnroll][2][kEB], b[kUnroll][2][kTB];
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u)
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
                     const int k = k0 + u * kStride + (c * 4 + hq) * kPer;
 #pragma unroll
-                    for (int tb = 0; tb < kTB; ++tb) b[u][c][tb] = *(const u32x4 *)(xrow[tb] + k);
+                    for (int tb = 0; tb < kTB; ++tb) gb[u][c][tb] = *(const u32x4 *)(xrow[tb] + k);
 #pragma unroll
-                    for (int eb = 0; eb < kEB; ++eb) a[u][c][eb] = eb < n_eb ? *(const u32x4 *)(wrow[eb] + k) : zero4;
+                    for (int eb = 0; eb < kEB; ++eb) ga[u][c][eb] = eb < n_eb ? *(const u32x4 *)(wrow[eb] + k) : zero4;
                 }
+        } else {
+            // the last group of the contraction: d is a multiple of kPer, so a chunk lies inside the row or
+            // outside it (zeros: a product that adds nothing)
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u)
 #pragma unroll
-                for (int c = 0; c < 2; ++c) mma(a[u][c], b[u][c]);
-        } else {
-            for (int ks = k0; ks < d && ks < k0 + kUnroll * kStride; ks += kStride) {
-#pragma unroll
                 for (int c = 0; c < 2; ++c) {
-                    const int k = ks + (c * 4 + hq) * kPer;   // d is a multiple of kPer: a chunk lies inside the row or outside it
-                    u32x4 a[kEB], b[kTB];
+                    const int k = k0 + u * kStride + (c * 4 + hq) * kPer;
 #pragma unroll
-                    for (int tb = 0; tb < kTB; ++tb) b[tb] = k < d ? *(const u32x4 *)(xrow[tb] + k) : zero4;
+                    for (int tb = 0; tb < kTB; ++tb) gb[u][c][tb] = k < d ? *(const u32x4 *)(xrow[tb] + k) : zero4;
 #pragma unroll
-                    for (int eb = 0; eb < kEB; ++eb) a[eb] = (eb < n_eb && k < d) ? *(const u32x4 *)(wrow[eb] + k) : zero4;
-                    mma(a, b);
+                    for (int eb = 0; eb < kEB; ++eb) ga[u][c][eb] = (eb < n_eb && k < d) ? *(const u32x4 *)(wrow[eb] + k) : zero4;
                 }
-            }
         }
+    };
+    auto mma_group = [&](const u32x4 (&ga)[kUnroll][2][kEB], const u32x4 (&gb)[kUnroll][2][kTB]) {
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) mma(ga[u][c], gb[u][c]);
+    };
+    load_group(0, a[0], b[0]);
+    for (int gi = 0; gi < n_groups; gi += 2) {
+        if (gi + 1 < n_groups) load_group(gi + 1, a[1], b[1]);
+        mma_group(a[0], b[0]);
+        if (gi + 1 >= n_groups) break;
+        if (gi + 2 < n_groups) load_group(gi + 2, a[0], b[0]);
+        mma_group(a[1], b[1]);
     }
     // lane (lb, hq) holds, per block pair, experts 4 hq .. 4 hq + 3 of the expert block for token lb of the token block
 #pragma unroll
@@ -483,35 +609,23 @@ __global__ __launch_bounds__(kBlock) void gate_linear_topk_kernel(
                 if (eb < n_eb) part_lds[((wave * n_eb + eb) * 16 + 4 * hq + r) * kGateStride + tb * 16 + lb] = acc[eb][tb][r];
     __syncthreads();
 
-    const int t = threadIdx.x;
+    constexpr int kSub = kBlock / kGateTokens;   // lanes per token
+    const int t = threadIdx.x / kSub, sub = threadIdx.x % kSub;
     const int64_t token = token0 + t;
-    if (t >= kGateTokens || token >= n_tokens) return;
-    float val[K];
-    int idx[K];
+    float val[K], best[K], score[K];
+    int idx[K], chosen[K];
 #pragma unroll
     for (int j = 0; j < K; ++j) { val[j] = -__builtin_inff(); idx[j] = -1; }
-    for (int e = 0; e < n_expert; ++e) {
+    const int ws = n_eb * 16 * kGateStride;   // one wave's tile
+    for (int e = sub; e < n_expert; e += kSub) {
         const float *p = part_lds + e * kGateStride + t;
-        const int ws = n_eb * 16 * kGateStride;   // one wave's tile
         float logit = ((p[0] + p[ws]) + p[2 * ws]) + p[3 * ws];
         if (bias != nullptr) logit += (float)bias[e];
         topk_insert<K>(val, idx, (float)(T)logit, e);
     }
-    float score[K];
-#pragma unroll
-    for (int j = 0; j < K; ++j) score[j] = val[j];
-    if (score_mode == 1) {
-        float sum = 0.f;
-#pragma unroll
-        for (int j = 0; j < K; ++j) { score[j] = idx[j] >= 0 ? __expf(val[j] - val[0]) : 0.f; sum += score[j]; }
-#pragma unroll
-        for (int j = 0; j < K; ++j) score[j] /= sum;
-    }
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        topk_idx[token * K + j] = idx[j];
-        topk_score[token * K + j] = (T)(idx[j] >= 0 ? score[j] : 0.f);
-    }
+    topk_merge<K, kSub>(val, idx, best, chosen);
+    topk_scores<K>(best, chosen, score_mode, score);
+    if (token < n_tokens) topk_store<T, K>(sub, token, chosen, score, topk_idx, topk_score);
 }
 
 // ----------------------------------------------------------- noisy gate ----
@@ -522,7 +636,7 @@ __global__ __launch_bounds__(kBlock) void gate_linear_topk_kernel(
 //   v_0 >= ... >= v_K : the K + 1 largest noisy logits (ties to the lower expert), experts i_0 .. i_K
 //   gates_j = softmax(v_0 .. v_{K-1})_j
 //   P_e     = Phi((clean_e - (noisy_e > v_K ? v_K : v_{K-1})) / std_e)      load_e = sum over tokens of P_e
-// A workgroup owns the same kSlotsPerBlock / K tokens as in gate_topk_hist_kernel and leaves the
+// A workgroup owns kSlotsPerBlock / K tokens (the slots of a workgroup of rank_apply_kernel) and leaves the
 // routing histogram of its selections for route_scan_kernel.  The load is summed without atomics:
 // a wave adds its 64 tokens' P_e by a butterfly of lane exchanges, wave-private LDS tables take
 // the sums, the four tables are added in wave order and written per workgroup; the caller adds
@@ -841,19 +955,54 @@ extern "C" int fmoe_assign_pos(int32_t *cum_count, const int64_t *gate, int64_t 
 namespace fmoe {
 namespace {
 
-// histogram -> scan over workgroups and experts -> placement, on scratch carved by the caller
-int route_launch(const int64_t *gate, int64_t n_slots, int64_t n_expert, int64_t *expert_count, int64_t *pos,
-                 int64_t *slot_to_row, const RouteScratch &s, hipStream_t st) {
+// Scan and placement after the per-workgroup histograms are in s.block_hist; the segment table of the
+// counts (for up to n_slots rows) goes to `table` unless that is null.
+int scan_and_place(const int64_t *gate, int64_t n_slots, int64_t n_expert, int64_t *expert_count, int64_t *pos,
+                   int64_t *slot_to_row, int32_t *table, const RouteScratch &s, hipStream_t st) {
     const int E = (int)n_expert;
-    if (int rc = allow_lds((const void *)block_hist_kernel, kWavesPerBlock * E * sizeof(int32_t))) return rc;
-    block_hist_kernel<<<s.n_blocks, kBlock, kWavesPerBlock * E * sizeof(int32_t), st>>>(gate, s.block_hist, n_slots, E, ilog2_ceil(n_expert));
+    const bool table_in_scan = E <= segtab::kSmallExperts;
+    route_scan_kernel<<<1, kRouteScanBlock, 0, st>>>(s.block_hist, s.n_blocks, E, expert_count, s.cum, (int)n_slots,
+                                                     table_in_scan ? table : nullptr);
     FMOE_LAUNCH_CHECK();
-    route_scan_kernel<<<1, kRouteScanBlock, 0, st>>>(s.block_hist, s.n_blocks, E, expert_count, s.cum);
-    FMOE_LAUNCH_CHECK();
+    if (table != nullptr && !table_in_scan)
+        if (int rc = fmoe_segment_table_build(expert_count, n_expert, n_slots, table,
+                                              fmoe_segment_table_bytes(n_slots, n_expert), st)) return rc;
     if (int rc = allow_lds((const void *)rank_apply_kernel<kApplyAssign>, kWavesPerBlock * E * sizeof(int32_t))) return rc;
     rank_apply_kernel<kApplyAssign><<<s.n_blocks, kBlock, kWavesPerBlock * E * sizeof(int32_t), st>>>(
         gate, s.block_hist, s.cum, pos, slot_to_row, n_slots, n_slots, E, ilog2_ceil(n_expert), 1);
     FMOE_LAUNCH_CHECK();
+    return FMOE_OK;
+}
+
+// Counts, positions, their inverse and (unless `table` is null) the segment table of a gate index:
+// one workgroup for few slots, else histogram -> scan over workgroups and experts -> placement, on
+// scratch carved by the caller.
+int route_launch(const int64_t *gate, int64_t n_slots, int64_t n_expert, int64_t *expert_count, int64_t *pos,
+                 int64_t *slot_to_row, int32_t *table, const RouteScratch &s, hipStream_t st) {
+    const int E = (int)n_expert;
+    // (the single workgroup's tables: 17 int32 per expert, 35 KiB of LDS at 512 experts beside the segment table's)
+    if (n_slots <= kSmallSlots && E <= 512) {
+        route_small_kernel<<<1, kSmallBlock, (kSmallWaves + 1) * E * sizeof(int32_t), st>>>(
+            gate, (int)n_slots, E, ilog2_ceil(n_expert), expert_count, pos, slot_to_row, table);
+        FMOE_LAUNCH_CHECK();
+        return FMOE_OK;
+    }
+    if (int rc = allow_lds((const void *)block_hist_kernel, kWavesPerBlock * E * sizeof(int32_t))) return rc;
+    block_hist_kernel<<<s.n_blocks, kBlock, kWavesPerBlock * E * sizeof(int32_t), st>>>(gate, s.block_hist, n_slots, E, ilog2_ceil(n_expert));
+    FMOE_LAUNCH_CHECK();
+    return scan_and_place(gate, n_slots, n_expert, expert_count, pos, slot_to_row, table, s, st);
+}
+
+// checks of the optional segment table of an entry point
+int check_table(const char *who, int64_t n_slots, int64_t n_expert, void *table, int64_t table_bytes) {
+    if (table == nullptr) return FMOE_OK;
+    FMOE_REQUIRE((reinterpret_cast<uintptr_t>(table) & 15u) == 0, "%s: the segment table must be 16-byte aligned", who);
+    if (n_slots > (int64_t)INT32_MAX - 65536)
+        return fail(FMOE_ELIMIT, "%s: %lld rows exceed the segment table's range", who, (long long)n_slots);
+    const int64_t need = fmoe_segment_table_bytes(n_slots, n_expert);
+    if (table_bytes < need)
+        return fail(FMOE_EWORKSPACE, "%s: the segment table needs %lld bytes, got %lld", who, (long long)need,
+                    (long long)table_bytes);
     return FMOE_OK;
 }
 
@@ -895,14 +1044,25 @@ int static_scratch_address(void **out) {
 extern "C" int fmoe_route(const int64_t *gate, int64_t n_slots, int64_t n_expert, int64_t *expert_count,
                           int64_t *pos, int64_t *slot_to_row, void *workspace, int64_t workspace_bytes,
                           void *stream) {
+    return fmoe_route_table(gate, n_slots, n_expert, expert_count, pos, slot_to_row, nullptr, 0, workspace,
+                            workspace_bytes, stream);
+}
+
+extern "C" int fmoe_route_table(const int64_t *gate, int64_t n_slots, int64_t n_expert, int64_t *expert_count,
+                                int64_t *pos, int64_t *slot_to_row, void *segment_table, int64_t table_bytes,
+                                void *workspace, int64_t workspace_bytes, void *stream) {
     if (int rc = check_sizes(n_slots, n_expert)) return rc;
     FMOE_REQUIRE(expert_count, "fmoe_route: NULL expert_count");
+    if (int rc = check_table("fmoe_route_table", n_slots, n_expert, segment_table, table_bytes)) return rc;
     hipStream_t st = (hipStream_t)stream;
-    if (n_slots == 0) return route_empty(n_expert, expert_count, st);
+    if (n_slots == 0) {
+        if (int rc = route_empty(n_expert, expert_count, st)) return rc;
+        return segment_table ? fmoe_segment_table_build(expert_count, n_expert, 0, segment_table, table_bytes, stream) : FMOE_OK;
+    }
     FMOE_REQUIRE(gate && pos, "fmoe_route: NULL pointer");
     RouteScratch s;
     if (int rc = carve(workspace, workspace_bytes, n_slots, n_expert, &s)) return rc;
-    return route_launch(gate, n_slots, n_expert, expert_count, pos, slot_to_row, s, st);
+    return route_launch(gate, n_slots, n_expert, expert_count, pos, slot_to_row, (int32_t *)segment_table, s, st);
 }
 
 extern "C" int fmoe_route_static(const int64_t *gate, int64_t n_slots, int64_t n_expert, int64_t *expert_count,
@@ -924,7 +1084,7 @@ extern "C" int fmoe_route_static(const int64_t *gate, int64_t n_slots, int64_t n
     if (int rc = carve(scratch_dev, kStaticScratchBytes, n_slots, n_expert, &s)) return rc;
     // Every cell of the scratch that the scan and the placement read is written by the
     // histogram / scan launched just before them, so nothing has to be cleared between calls.
-    return route_launch(gate, n_slots, n_expert, expert_count, pos, slot_to_row, s, st);
+    return route_launch(gate, n_slots, n_expert, expert_count, pos, slot_to_row, nullptr, s, st);
 }
 
 extern "C" int fmoe_limit_by_capacity(const int64_t *ec, int32_t *cap, int64_t *eca, int64_t n_expert,
@@ -964,28 +1124,34 @@ extern "C" int fmoe_prune_gate_by_capacity(const int64_t *gate_idx, int64_t *new
 namespace fmoe {
 namespace {
 
-template <typename T>
-int launch_gate_topk(const void *logits, int64_t n_tokens, int E, int top_k, int score_mode, int64_t *topk_idx,
-                     void *topk_score, int32_t *block_hist, int n_blocks, hipStream_t st) {
-    const size_t lds = kWavesPerBlock * E * sizeof(int32_t);
-    const int nbits = ilog2_ceil(E);
+template <typename T, int K>
+void launch_gate_topk_lanes(const T *logits, int64_t n_tokens, int E, int score_mode, int64_t *topk_idx, T *topk_score,
+                            hipStream_t st) {
     // rows start on 16-byte boundaries: vector loads
     const int vector_rows = (E * sizeof(T)) % 16 == 0 && (reinterpret_cast<uintptr_t>(logits) & 15u) == 0;
-#define FMOE_GATE_LAUNCH(KK)                                                                                      \
-    do {                                                                                                          \
-        if (int rc = allow_lds((const void *)gate_topk_hist_kernel<T, KK>, lds)) return rc;                       \
-        gate_topk_hist_kernel<T, KK><<<n_blocks, kBlock, lds, st>>>((const T *)logits, n_tokens, E, score_mode,   \
-                                                                    vector_rows, topk_idx, (T *)topk_score,       \
-                                                                    block_hist, nbits);                           \
-    } while (0)
+    // lanes per token: 8 for short rows, 64 for long ones, so that a lane's chain stays at 8 to 32 logits
+    // (and at least K, since lane j writes choice j)
+    if (E <= 64)
+        gate_topk_kernel<T, K, 8><<<(unsigned)ceil_div(n_tokens, kBlock / 8), kBlock, 0, st>>>(
+            logits, n_tokens, E, score_mode, vector_rows, topk_idx, topk_score);
+    else if (E <= 512)
+        gate_topk_kernel<T, K, 16><<<(unsigned)ceil_div(n_tokens, kBlock / 16), kBlock, 0, st>>>(
+            logits, n_tokens, E, score_mode, vector_rows, topk_idx, topk_score);
+    else
+        gate_topk_kernel<T, K, 64><<<(unsigned)ceil_div(n_tokens, kBlock / 64), kBlock, 0, st>>>(
+            logits, n_tokens, E, score_mode, vector_rows, topk_idx, topk_score);
+}
+
+template <typename T>
+int launch_gate_topk(const void *logits, int64_t n_tokens, int E, int top_k, int score_mode, int64_t *topk_idx,
+                     void *topk_score, hipStream_t st) {
     switch (top_k) {
-        case 1: FMOE_GATE_LAUNCH(1); break;
-        case 2: FMOE_GATE_LAUNCH(2); break;
-        case 4: FMOE_GATE_LAUNCH(4); break;
-        case 8: FMOE_GATE_LAUNCH(8); break;
+        case 1: launch_gate_topk_lanes<T, 1>((const T *)logits, n_tokens, E, score_mode, topk_idx, (T *)topk_score, st); break;
+        case 2: launch_gate_topk_lanes<T, 2>((const T *)logits, n_tokens, E, score_mode, topk_idx, (T *)topk_score, st); break;
+        case 4: launch_gate_topk_lanes<T, 4>((const T *)logits, n_tokens, E, score_mode, topk_idx, (T *)topk_score, st); break;
+        case 8: launch_gate_topk_lanes<T, 8>((const T *)logits, n_tokens, E, score_mode, topk_idx, (T *)topk_score, st); break;
         default: return fail(FMOE_ELIMIT, "gate top-k: top_k=%d is not 1, 2, 4 or 8", top_k);
     }
-#undef FMOE_GATE_LAUNCH
     FMOE_LAUNCH_CHECK();
     return FMOE_OK;
 }
@@ -997,6 +1163,14 @@ extern "C" int fmoe_gate_topk_route(const void *logits, int64_t n_tokens, int64_
                                     int score_mode, int64_t *topk_idx, void *topk_score, int64_t *expert_count,
                                     int64_t *pos, int64_t *slot_to_row, void *workspace, int64_t workspace_bytes,
                                     void *stream) {
+    return fmoe_gate_topk_route_table(logits, n_tokens, n_expert, top_k, dtype, score_mode, topk_idx, topk_score,
+                                      expert_count, pos, slot_to_row, nullptr, 0, workspace, workspace_bytes, stream);
+}
+
+extern "C" int fmoe_gate_topk_route_table(const void *logits, int64_t n_tokens, int64_t n_expert, int64_t top_k, int dtype,
+                                          int score_mode, int64_t *topk_idx, void *topk_score, int64_t *expert_count,
+                                          int64_t *pos, int64_t *slot_to_row, void *segment_table, int64_t table_bytes,
+                                          void *workspace, int64_t workspace_bytes, void *stream) {
     FMOE_REQUIRE(n_tokens >= 0 && top_k >= 1, "fmoe_gate_topk_route: n_tokens=%lld top_k=%lld", (long long)n_tokens,
                  (long long)top_k);
     FMOE_REQUIRE(dtype == FMOE_F32 || dtype == FMOE_BF16 || dtype == FMOE_F16, "fmoe_gate_topk_route: dtype %d", dtype);
@@ -1007,26 +1181,24 @@ extern "C" int fmoe_gate_topk_route(const void *logits, int64_t n_tokens, int64_
     const int64_t n_slots = n_tokens * top_k;
     if (int rc = check_sizes(n_slots, n_expert)) return rc;
     FMOE_REQUIRE(expert_count, "fmoe_gate_topk_route: NULL expert_count");
+    if (int rc = check_table("fmoe_gate_topk_route_table", n_slots, n_expert, segment_table, table_bytes)) return rc;
     hipStream_t st = (hipStream_t)stream;
-    if (n_slots == 0) return route_empty(n_expert, expert_count, st);
+    if (n_slots == 0) {
+        if (int rc = route_empty(n_expert, expert_count, st)) return rc;
+        return segment_table ? fmoe_segment_table_build(expert_count, n_expert, 0, segment_table, table_bytes, stream) : FMOE_OK;
+    }
     FMOE_REQUIRE(logits && topk_idx && topk_score && pos, "fmoe_gate_topk_route: NULL pointer");
     RouteScratch s;
     if (int rc = carve(workspace, workspace_bytes, n_slots, n_expert, &s)) return rc;
     const int E = (int)n_expert;
     int rc = FMOE_OK;
     switch (dtype) {
-        case FMOE_F32: rc = launch_gate_topk<float>(logits, n_tokens, E, (int)top_k, score_mode, topk_idx, topk_score, s.block_hist, s.n_blocks, st); break;
-        case FMOE_BF16: rc = launch_gate_topk<__bf16>(logits, n_tokens, E, (int)top_k, score_mode, topk_idx, topk_score, s.block_hist, s.n_blocks, st); break;
-        default: rc = launch_gate_topk<_Float16>(logits, n_tokens, E, (int)top_k, score_mode, topk_idx, topk_score, s.block_hist, s.n_blocks, st); break;
+        case FMOE_F32: rc = launch_gate_topk<float>(logits, n_tokens, E, (int)top_k, score_mode, topk_idx, topk_score, st); break;
+        case FMOE_BF16: rc = launch_gate_topk<__bf16>(logits, n_tokens, E, (int)top_k, score_mode, topk_idx, topk_score, st); break;
+        default: rc = launch_gate_topk<_Float16>(logits, n_tokens, E, (int)top_k, score_mode, topk_idx, topk_score, st); break;
     }
     if (rc) return rc;
-    route_scan_kernel<<<1, kRouteScanBlock, 0, st>>>(s.block_hist, s.n_blocks, E, expert_count, s.cum);
-    FMOE_LAUNCH_CHECK();
-    if (int rc2 = allow_lds((const void *)rank_apply_kernel<kApplyAssign>, kWavesPerBlock * E * sizeof(int32_t))) return rc2;
-    rank_apply_kernel<kApplyAssign><<<s.n_blocks, kBlock, kWavesPerBlock * E * sizeof(int32_t), st>>>(
-        topk_idx, s.block_hist, s.cum, pos, slot_to_row, n_slots, n_slots, E, ilog2_ceil(n_expert), 1);
-    FMOE_LAUNCH_CHECK();
-    return FMOE_OK;
+    return route_launch(topk_idx, n_slots, n_expert, expert_count, pos, slot_to_row, (int32_t *)segment_table, s, st);
 }
 
 namespace fmoe {
@@ -1077,6 +1249,17 @@ extern "C" int fmoe_gate_linear_topk_route(const void *x, const void *w, const v
                                            int64_t *topk_idx, void *topk_score, int64_t *expert_count, int64_t *pos,
                                            int64_t *slot_to_row, void *workspace, int64_t workspace_bytes,
                                            void *stream) {
+    return fmoe_gate_linear_topk_route_table(x, w, bias, n_tokens, d_model, n_expert, top_k, dtype, score_mode, topk_idx,
+                                             topk_score, expert_count, pos, slot_to_row, nullptr, 0, workspace,
+                                             workspace_bytes, stream);
+}
+
+extern "C" int fmoe_gate_linear_topk_route_table(const void *x, const void *w, const void *bias, int64_t n_tokens,
+                                                 int64_t d_model, int64_t n_expert, int64_t top_k, int dtype,
+                                                 int score_mode, int64_t *topk_idx, void *topk_score,
+                                                 int64_t *expert_count, int64_t *pos, int64_t *slot_to_row,
+                                                 void *segment_table, int64_t table_bytes, void *workspace,
+                                                 int64_t workspace_bytes, void *stream) {
     FMOE_REQUIRE(n_tokens >= 0 && top_k >= 1, "fmoe_gate_linear_topk_route: n_tokens=%lld top_k=%lld",
                  (long long)n_tokens, (long long)top_k);
     FMOE_REQUIRE(score_mode == 0 || score_mode == 1, "fmoe_gate_linear_topk_route: score_mode %d", score_mode);
@@ -1088,8 +1271,12 @@ extern "C" int fmoe_gate_linear_topk_route(const void *x, const void *w, const v
     const int64_t n_slots = n_tokens * top_k;
     if (int rc = check_sizes(n_slots, n_expert)) return rc;
     FMOE_REQUIRE(expert_count, "fmoe_gate_linear_topk_route: NULL expert_count");
+    if (int rc = check_table("fmoe_gate_linear_topk_route_table", n_slots, n_expert, segment_table, table_bytes)) return rc;
     hipStream_t st = (hipStream_t)stream;
-    if (n_slots == 0) return route_empty(n_expert, expert_count, st);
+    if (n_slots == 0) {
+        if (int rc = route_empty(n_expert, expert_count, st)) return rc;
+        return segment_table ? fmoe_segment_table_build(expert_count, n_expert, 0, segment_table, table_bytes, stream) : FMOE_OK;
+    }
     FMOE_REQUIRE(x && w && topk_idx && topk_score && pos, "fmoe_gate_linear_topk_route: NULL pointer");
     FMOE_REQUIRE(aligned16(x) && aligned16(w), "fmoe_gate_linear_topk_route: x and w must be 16-byte aligned");
     RouteScratch s;
@@ -1101,7 +1288,7 @@ extern "C" int fmoe_gate_linear_topk_route(const void *x, const void *w, const v
         default: rc = launch_gate_linear<_Float16>(x, w, bias, n_tokens, (int)d_model, (int)n_expert, (int)top_k, score_mode, topk_idx, topk_score, st); break;
     }
     if (rc) return rc;
-    return route_launch(topk_idx, n_slots, n_expert, expert_count, pos, slot_to_row, s, st);
+    return route_launch(topk_idx, n_slots, n_expert, expert_count, pos, slot_to_row, (int32_t *)segment_table, s, st);
 }
 
 extern "C" int fmoe_noisy_gate_forward(const void *clean, const void *raw, const void *noise, double eps,
@@ -1148,13 +1335,7 @@ extern "C" int fmoe_noisy_gate_forward(const void *clean, const void *raw, const
 #undef FMOE_NOISY_FWD_K
 #undef FMOE_NOISY_FWD
     FMOE_LAUNCH_CHECK();
-    route_scan_kernel<<<1, kRouteScanBlock, 0, st>>>(s.block_hist, s.n_blocks, E, expert_count, s.cum);
-    FMOE_LAUNCH_CHECK();
-    if (int rc2 = allow_lds((const void *)rank_apply_kernel<kApplyAssign>, kWavesPerBlock * E * sizeof(int32_t))) return rc2;
-    rank_apply_kernel<kApplyAssign><<<s.n_blocks, kBlock, kWavesPerBlock * E * sizeof(int32_t), st>>>(
-        topk_idx, s.block_hist, s.cum, pos, slot_to_row, n_slots, n_slots, E, nbits, 1);
-    FMOE_LAUNCH_CHECK();
-    return FMOE_OK;
+    return scan_and_place(topk_idx, n_slots, n_expert, expert_count, pos, slot_to_row, nullptr, s, st);
 }
 
 extern "C" int fmoe_noisy_gate_backward(const void *clean, const void *raw, const void *noise, double eps,

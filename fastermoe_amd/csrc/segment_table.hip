@@ -7,14 +7,21 @@
 // and the first GEMM.  Here one small kernel builds the same table on the device, straight from
 // the counts the routing kernels left there; the GEMMs launched over it are sized for the most
 // tiles the rows can make and read the real numbers themselves.
-#include "grouped_gemm.hpp"
+#include "segment_table.hpp"
 
 namespace fmoe {
 namespace {
 
-constexpr int kTabBlock = 1024;
+constexpr int kTabBlock = segtab::kThreads;
 
-// One workgroup.  Pass 1: per expert (in chunks of kTabBlock, carrying the running sums) the
+// Up to segtab::kSmallExperts experts: everything in LDS.
+__global__ __launch_bounds__(kTabBlock) void small_table_kernel(const int64_t *__restrict__ counts, int n_expert,
+                                                                int rows_cap, int32_t *__restrict__ tab) {
+    __shared__ segtab::SmallLds lds;
+    segtab::small_table((int)threadIdx.x < n_expert ? counts[threadIdx.x] : 0, n_expert, rows_cap, tab, lds);
+}
+
+// More experts: one workgroup.  Pass 1: per expert (in chunks of kTabBlock, carrying the running sums) the
 // exclusive prefixes of rows, 256-row tiles and 128-row tiles.  Counts are clamped so that their
 // sum never exceeds rows_cap: the tile maps then never outgrow the space laid out for them,
 // whatever the counts hold.  Pass 2: one thread per row tile finds its expert by binary search
@@ -147,8 +154,12 @@ extern "C" int fmoe_segment_table_build(const int64_t *expert_count, int64_t n_e
     if (table_bytes < need)
         return fail(FMOE_EWORKSPACE, "fmoe_segment_table_build: the table needs %lld bytes, got %lld", (long long)need,
                     (long long)table_bytes);
-    segment_table_kernel<<<1, kTabBlock, 0, (hipStream_t)stream>>>(expert_count, (int)n_expert, (int)rows_cap,
-                                                                  (int32_t *)segment_table);
+    if (n_expert <= segtab::kSmallExperts)
+        small_table_kernel<<<1, kTabBlock, 0, (hipStream_t)stream>>>(expert_count, (int)n_expert, (int)rows_cap,
+                                                                    (int32_t *)segment_table);
+    else
+        segment_table_kernel<<<1, kTabBlock, 0, (hipStream_t)stream>>>(expert_count, (int)n_expert, (int)rows_cap,
+                                                                      (int32_t *)segment_table);
     FMOE_LAUNCH_CHECK();
     return FMOE_OK;
 }

@@ -1,0 +1,102 @@
+// Device side of the segment table (layout: grouped_gemm.hpp, namespace segtab): the part that the
+// stand-alone kernel of segment_table.hip and the routing kernels share.
+#pragma once
+#include "grouped_gemm.hpp"
+
+namespace fmoe {
+namespace segtab {
+
+constexpr int kThreads = 1024;        // the workgroup that builds a table
+constexpr int kSmallExperts = 1024;   // most experts of small_table(): one per thread
+
+// LDS of small_table(): the three prefixes and the waves' sums
+struct SmallLds {
+    int64_t row_sum[kThreads / kWave];
+    int32_t wave_sum[2][kThreads / kWave];
+    int32_t seg[kSmallExperts + 1];
+    int32_t pfx[2][kSmallExperts + 1];
+};
+
+// The whole table for at most kSmallExperts experts by one workgroup of kThreads threads, thread e
+// holding expert e's row count (others: anything).  The counts are clamped so that their sum never
+// exceeds rows_cap.  The prefixes stay in LDS, where the row tiles find their expert by binary
+// search: read back from memory, the ten dependent loads of that search were most of the table's
+// 9.7 us at 8 experts.
+__device__ __forceinline__ void small_table(int64_t count, int n_expert, int rows_cap, int32_t *__restrict__ tab, SmallLds &lds) {
+    const int e = threadIdx.x, lane = e & (kWave - 1), wave = e / kWave;
+    int64_t c64 = e < n_expert ? count : 0;
+    c64 = c64 < 0 ? 0 : (c64 > rows_cap ? rows_cap : c64);
+    int64_t v = c64;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int64_t up = __shfl_up(v, off, kWave);
+        if (lane >= off) v += up;
+    }
+    if (lane == kWave - 1) lds.row_sum[wave] = v;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) v += lds.row_sum[w];
+    int64_t lo = v - c64;
+    lo = lo > rows_cap ? rows_cap : lo;
+    const int64_t hi = v > rows_cap ? rows_cap : v;
+    const int32_t rows = (int32_t)(hi - lo);
+    const int32_t t[2] = {(rows + 255) / 256, (rows + 127) / 128};
+    int32_t tv[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        int32_t s = t[k];
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+            const int32_t up = __shfl_up(s, off, kWave);
+            if (lane >= off) s += up;
+        }
+        tv[k] = s;
+        if (lane == kWave - 1) lds.wave_sum[k][wave] = s;
+    }
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) { tv[0] += lds.wave_sum[0][w]; tv[1] += lds.wave_sum[1][w]; }
+    int32_t *seg = tab + seg_off(), *pfx256 = tab + pfx256_off(n_expert), *pfx128 = tab + pfx128_off(n_expert);
+    const int map256 = (int)map256_off(n_expert), map128 = (int)map128_off(rows_cap, n_expert);
+    if (e < n_expert) {
+        lds.seg[e] = seg[e] = (int32_t)lo;
+        lds.pfx[0][e] = pfx256[e] = tv[0] - t[0];
+        lds.pfx[1][e] = pfx128[e] = tv[1] - t[1];
+    }
+    if (e == n_expert - 1) {
+        lds.seg[n_expert] = seg[n_expert] = (int32_t)hi;
+        lds.pfx[0][n_expert] = pfx256[n_expert] = tv[0];
+        lds.pfx[1][n_expert] = pfx128[n_expert] = tv[1];
+        tab[0] = n_expert;
+        tab[kRows] = (int32_t)hi;
+        tab[kTiles256] = tv[0];
+        tab[kTiles128] = tv[1];
+        tab[kMap256] = map256;
+        tab[kMap128] = map128;
+        tab[kRowsCap] = rows_cap;
+        tab[7] = 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int block_rows = k == 0 ? 256 : 128;
+        const int32_t *pfx = lds.pfx[k];
+        int32_t *map = tab + (k == 0 ? map256 : map128);
+        const int tiles = pfx[n_expert];
+        for (int i = threadIdx.x; i < tiles; i += kThreads) {
+            int a = 0, b = n_expert;  // pfx[a] <= i < pfx[b]
+            while (b - a > 1) {
+                const int mid = (a + b) >> 1;
+                if (pfx[mid] <= i) a = mid; else b = mid;
+            }
+            const int first = lds.seg[a] + (i - pfx[a]) * block_rows, left = lds.seg[a + 1] - first;
+            int4 entry;
+            entry.x = a;
+            entry.y = first;
+            entry.z = left < block_rows ? left : block_rows;
+            entry.w = 0;
+            *(int4 *)(map + 4 * (int64_t)i) = entry;
+        }
+    }
+}
+
+}  // namespace segtab
+}  // namespace fmoe

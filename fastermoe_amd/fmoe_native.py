@@ -93,11 +93,22 @@ def assign_pos(cum_count, gate, pos):
                                   _stream(gate)))
 
 
+def _table_buffer(lib, rows_cap, n_expert, device):
+    nbytes = lib.fmoe_segment_table_bytes(int(rows_cap), int(n_expert))
+    return torch.empty(nbytes // 4, dtype=torch.int32, device=device), nbytes
+
+
 def route(gate, n_expert):
     """One call for what fmoe/functions.py:19-42 does in several: returns
     ``(expert_count int64 [E], pos_buf int64 [n_slots], slot_to_row int64 [n_slots])``,
     all on the device.  Only the first ``expert_count.sum()`` entries of
     ``pos_buf`` are meaningful."""
+    return route_table(gate, n_expert, False)[:3]
+
+
+def route_table(gate, n_expert, with_table=True):
+    """:func:`route` with the segment table of the counts (:func:`segment_table`) as a fourth result,
+    built in the same launches (``None`` unless ``with_table``)."""
     _dev("gate", gate, torch.int64)
     lib = _lib.load()
     n = gate.numel()
@@ -105,10 +116,11 @@ def route(gate, n_expert):
         cnt = torch.empty(n_expert, dtype=torch.int64, device=gate.device)
         pos = torch.empty(n, dtype=torch.int64, device=gate.device)
         s2r = torch.empty(n, dtype=torch.int64, device=gate.device)
+        table, nbytes = _table_buffer(lib, n, n_expert, gate.device) if with_table else (None, 0)
         ws = _workspace(lib.fmoe_routing_workspace_bytes(n, n_expert), gate.device)
-        check(lib.fmoe_route(_ptr(gate), n, n_expert, _ptr(cnt), _ptr(pos), _ptr(s2r), _ptr(ws), ws.numel(),
-                             _stream(gate)))
-    return cnt, pos, s2r
+        check(lib.fmoe_route_table(_ptr(gate), n, n_expert, _ptr(cnt), _ptr(pos), _ptr(s2r), _ptr(table), nbytes, _ptr(ws),
+                                   ws.numel(), _stream(gate)))
+    return cnt, pos, s2r, table
 
 
 def gate_topk_supported(n_expert, top_k, dtype):
@@ -117,11 +129,12 @@ def gate_topk_supported(n_expert, top_k, dtype):
             and dtype in (torch.float32, torch.bfloat16, torch.float16))
 
 
-def gate_topk_route(logits, top_k, score_mode=0):
+def gate_topk_route(logits, top_k, score_mode=0, with_table=False):
     """Top-k of ``logits [N, E]`` with the routing bookkeeping in the same launches.  Returns
     ``(topk_idx int64 [N,k], topk_score [N,k], expert_count int64 [E], pos_buf int64 [N*k],
     slot_to_row int64 [N*k])``; ``score_mode`` 0 returns the selected logits as scores, 1 their
-    softmax over the k selected."""
+    softmax over the k selected.  ``with_table`` adds the segment table of the counts
+    (:func:`segment_table`), built in the same launches."""
     _dev("logits", logits)
     if logits.dim() != 2:
         raise ValueError(f"logits must be [n_tokens, n_expert], got {tuple(logits.shape)}")
@@ -138,9 +151,10 @@ def gate_topk_route(logits, top_k, score_mode=0):
         pos = torch.empty(n * top_k, dtype=torch.int64, device=dev)
         s2r = torch.empty(n * top_k, dtype=torch.int64, device=dev)
         ws = _workspace(lib.fmoe_routing_workspace_bytes(n * top_k, e), dev)
-        check(lib.fmoe_gate_topk_route(_ptr(logits), n, e, top_k, dt, score_mode, _ptr(idx), _ptr(score), _ptr(cnt),
-                                       _ptr(pos), _ptr(s2r), _ptr(ws), ws.numel(), _stream(logits)))
-    return idx, score, cnt, pos, s2r
+        table, nbytes = _table_buffer(lib, n * top_k, e, dev) if with_table else (None, 0)
+        check(lib.fmoe_gate_topk_route_table(_ptr(logits), n, e, top_k, dt, score_mode, _ptr(idx), _ptr(score), _ptr(cnt),
+                                       _ptr(pos), _ptr(s2r), _ptr(table), nbytes, _ptr(ws), ws.numel(), _stream(logits)))
+    return (idx, score, cnt, pos, s2r, table) if with_table else (idx, score, cnt, pos, s2r)
 
 
 def gate_linear_supported(d_model, n_expert, top_k, dtype):
@@ -149,10 +163,11 @@ def gate_linear_supported(d_model, n_expert, top_k, dtype):
                                                                        _DTYPES[dtype]) == 1
 
 
-def gate_linear_topk_route(x, weight, bias, top_k, score_mode=0):
+def gate_linear_topk_route(x, weight, bias, top_k, score_mode=0, with_table=False):
     """``gate_topk_route(x @ weight.T + bias, ...)`` without the logits ever reaching memory: the gate's
     linear layer, its top-k, the scores and the routing in one call.  ``weight`` is ``[E, d_model]``
-    (``nn.Linear.weight``), ``bias`` ``[E]`` or ``None``.  Same results tuple as :func:`gate_topk_route`."""
+    (``nn.Linear.weight``), ``bias`` ``[E]`` or ``None``.  Same results tuple as :func:`gate_topk_route`
+    (with the segment table appended by ``with_table``)."""
     dt = _rows("x", x)
     _dev("weight", weight, x.dtype)
     if weight.dim() != 2 or weight.shape[1] != x.shape[1]:
@@ -174,10 +189,11 @@ def gate_linear_topk_route(x, weight, bias, top_k, score_mode=0):
         pos = torch.empty(n * top_k, dtype=torch.int64, device=dev)
         s2r = torch.empty(n * top_k, dtype=torch.int64, device=dev)
         ws = _workspace(lib.fmoe_routing_workspace_bytes(n * top_k, e), dev)
-        check(lib.fmoe_gate_linear_topk_route(_ptr(x), _ptr(weight), _ptr(bias), n, d, e, top_k, dt, score_mode, _ptr(idx),
-                                              _ptr(score), _ptr(cnt), _ptr(pos), _ptr(s2r), _ptr(ws), ws.numel(),
+        table, nbytes = _table_buffer(lib, n * top_k, e, dev) if with_table else (None, 0)
+        check(lib.fmoe_gate_linear_topk_route_table(_ptr(x), _ptr(weight), _ptr(bias), n, d, e, top_k, dt, score_mode, _ptr(idx),
+                                              _ptr(score), _ptr(cnt), _ptr(pos), _ptr(s2r), _ptr(table), nbytes, _ptr(ws), ws.numel(),
                                               _stream(x)))
-    return idx, score, cnt, pos, s2r
+    return (idx, score, cnt, pos, s2r, table) if with_table else (idx, score, cnt, pos, s2r)
 
 
 def noisy_gate_supported(n_expert, top_k, dtype):

@@ -33,11 +33,12 @@ class GateTopK(Function):
     @staticmethod
     def forward(ctx, logits, top_k, score_mode):
         logits = logits.contiguous()
-        idx, score, cnt, pos_buf, s2r = fmoe_native.gate_topk_route(logits, top_k, score_mode)
+        idx, score, cnt, pos_buf, s2r, table = fmoe_native.gate_topk_route(logits, top_k, score_mode, with_table=True)
         ctx.save_for_backward(idx, score)
         ctx.moe_args = logits.shape[1], score_mode
         ctx.mark_non_differentiable(idx)
         idx._fmoe_route = (idx._version, logits.shape[1], cnt, pos_buf, s2r)
+        idx._fmoe_table = table
         return idx, score
 
     @staticmethod
@@ -57,11 +58,13 @@ class GateLinearTopK(Function):
     def forward(ctx, x, weight, bias, top_k, score_mode):
         x = x.contiguous()
         weight = weight.contiguous()
-        idx, score, cnt, pos_buf, s2r = fmoe_native.gate_linear_topk_route(x, weight, bias, top_k, score_mode)
+        idx, score, cnt, pos_buf, s2r, table = fmoe_native.gate_linear_topk_route(x, weight, bias, top_k, score_mode,
+                                                                                  with_table=True)
         ctx.save_for_backward(x, weight, idx, score)
         ctx.moe_args = score_mode, bias is not None
         ctx.mark_non_differentiable(idx)
         idx._fmoe_route = (idx._version, weight.shape[0], cnt, pos_buf, s2r)
+        idx._fmoe_table = table
         return idx, score
 
     @staticmethod
@@ -131,15 +134,22 @@ def gate_topk(logits, top_k, score_mode=0):
     return idx, (torch.softmax(val, dim=-1) if score_mode == 1 else val)
 
 
-def _route_launch(gate, num_expert):
+def _route_launch(gate, num_expert, with_table=False):
     """Enqueues the routing of ``gate`` (or picks up the one its :class:`GateTopK` call made) and
     returns the device tensors ``(counts [E], pos_buf [n_slots], slot_to_row [n_slots])``; nothing
-    is read back.  ``pos_buf`` holds the routed slots first and -1 after them."""
+    is read back.  ``pos_buf`` holds the routed slots first and -1 after them.  ``with_table`` appends
+    the segment table of the counts that the grouped GEMMs read."""
     with torch.no_grad():
         cached = getattr(gate, "_fmoe_route", None)
         if cached is not None and cached[0] == gate._version and cached[1] == num_expert:
-            return cached[2:]
-        return fmoe_native.route(gate.contiguous(), num_expert)
+            if not with_table:
+                return cached[2:]
+            table = getattr(gate, "_fmoe_table", None)
+            if table is None:
+                table = fmoe_native.segment_table(cached[2], cached[3].numel())
+            return cached[2:] + (table,)
+        routed = fmoe_native.route_table(gate.contiguous(), num_expert, with_table)
+        return routed if with_table else routed[:3]
 
 
 def _route(gate, num_expert, world_size):

@@ -84,9 +84,10 @@ def _fmoe_general_global_forward(inp, gate, expert_fn, policy_fn, experts, num_e
            and gate.numel() == inp.shape[0] * topk and fused and _own_expert_path(expert_fn, experts))
     if own:
         _single_worker(world_size, "count_by_gate")
-        counts_dev, pos_buf, slot_to_row = _route_launch(gate, num_expert)
+        routed = _route_launch(gate, num_expert, with_table=not enable_fuse)
+        counts_dev, pos_buf, slot_to_row = routed[:3]
         if not enable_fuse:
-            x = experts.routed_forward(inp, pos_buf, slot_to_row, counts_dev, topk)
+            x = experts.routed_forward(inp, pos_buf, slot_to_row, counts_dev, topk, routed[3])
             if x is not None:
                 stored_models = torch.zeros(world_size * num_expert, dtype=torch.bool)
                 if combine_score is not None:

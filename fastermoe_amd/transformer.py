@@ -33,11 +33,12 @@ class _Expert(nn.Module):
         x = self.activation(x)
         return self.h4toh(x, fwd_expert_count)
 
-    def routed_forward(self, inp, pos_buf, slot_to_row, counts_dev, top_k):
+    def routed_forward(self, inp, pos_buf, slot_to_row, counts_dev, top_k, table=None):
         r"""The experts over token rows ``inp [N, d_model]`` routed by ``pos_buf`` / ``slot_to_row`` /
-        ``counts_dev`` (the device tensors of the routing call), without any of them being read on
-        the host: returns the experts' output in expert-sorted order, one row per slot, or ``None``
-        when this shape or activation needs the module-by-module path."""
+        ``counts_dev`` (the device tensors of the routing call, and ``table``, the segment table of the
+        counts, where the call made one), without any of them being read on the host: returns the
+        experts' output in expert-sorted order, one row per slot, or ``None`` when this shape or
+        activation needs the module-by-module path."""
         code = self._epilogue_activation()
         d_hidden, d_model = self.htoh4.weight.shape[1:]
         if (code is None or not inp.is_cuda or inp.dtype not in (torch.float32, torch.bfloat16, torch.float16)
@@ -46,7 +47,8 @@ class _Expert(nn.Module):
                 or os.environ.get("FMOE_DEVICE_TABLES", "1") == "0"
                 or not fmoe_native.linear_dev_supported(d_model, d_hidden, inp.dtype)):
             return None
-        table = fmoe_native.segment_table(counts_dev, pos_buf.numel())
+        if table is None:
+            table = fmoe_native.segment_table(counts_dev, pos_buf.numel())
         return MOERoutedMLP.apply(inp, self.htoh4.weight, self.htoh4.bias, self.h4toh.weight, self.h4toh.bias,
                                   pos_buf, slot_to_row, table, top_k, code)
 

@@ -78,6 +78,17 @@ int fmoe_route(const int64_t *gate, int64_t n_slots, int64_t n_expert,
                int64_t *expert_count, int64_t *pos, int64_t *slot_to_row,
                void *workspace, int64_t workspace_bytes, void *stream);
 
+/* fmoe_route that also leaves the segment table of the counts for up to n_slots
+ * rows (fmoe_segment_table_build(expert_count, n_expert, n_slots, ...)) in
+ * segment_table, for the *_dev products below; NULL: no table.  table_bytes: at
+ * least fmoe_segment_table_bytes(n_slots, n_expert).  Few slots take one launch
+ * for all of it. */
+int fmoe_route_table(const int64_t *gate, int64_t n_slots, int64_t n_expert,
+                     int64_t *expert_count, int64_t *pos,
+                     int64_t *slot_to_row, void *segment_table,
+                     int64_t table_bytes, void *workspace,
+                     int64_t workspace_bytes, void *stream);
+
 /* fmoe_route for callers that must not allocate (code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc): same inputs, outputs and
  * results as fmoe_route, but the scratch is a fixed array of
@@ -101,8 +112,7 @@ int fmoe_route_static(const int64_t *gate, int64_t n_slots, int64_t n_expert,
  *   topk_score [n_tokens, top_k] (dtype)  score_mode 0: the selected logits
  *              (what NaiveGate returns, fmoe/gates/naive_gate.py:32-42);
  *              1: softmax over the top_k selected logits
- * and, from the per-workgroup histograms the same pass leaves behind,
- * expert_count / pos / slot_to_row exactly as fmoe_route(topk_idx) gives them.
+ * and expert_count / pos / slot_to_row exactly as fmoe_route(topk_idx) gives them.
  * logits [n_tokens, n_expert] in FMOE_F32 / FMOE_BF16 / FMOE_F16; top_k 1, 2, 4
  * or 8 (FMOE_ELIMIT otherwise: use torch.topk and fmoe_route).  workspace: fmoe_routing_workspace_bytes(n_tokens*top_k, n_expert).
  * Replaces torch.topk (+ softmax) of fmoe/gates/naive_gate.py:26-42 followed by
@@ -113,6 +123,16 @@ int fmoe_gate_topk_route(const void *logits, int64_t n_tokens, int64_t n_expert,
                          int64_t *expert_count, int64_t *pos,
                          int64_t *slot_to_row, void *workspace,
                          int64_t workspace_bytes, void *stream);
+
+/* ... with the segment table of fmoe_route_table (NULL: none). */
+int fmoe_gate_topk_route_table(const void *logits, int64_t n_tokens,
+                               int64_t n_expert, int64_t top_k, int dtype,
+                               int score_mode, int64_t *topk_idx,
+                               void *topk_score, int64_t *expert_count,
+                               int64_t *pos, int64_t *slot_to_row,
+                               void *segment_table, int64_t table_bytes,
+                               void *workspace, int64_t workspace_bytes,
+                               void *stream);
 
 /* The gate's linear layer folded into the same call, for small expert counts:
  * logits = x . w^T + bias are formed on chip (rounded to the element type as the
@@ -135,6 +155,15 @@ int fmoe_gate_linear_topk_route(const void *x, const void *w, const void *bias,
                                 int64_t *pos, int64_t *slot_to_row,
                                 void *workspace, int64_t workspace_bytes,
                                 void *stream);
+
+/* ... with the segment table of fmoe_route_table (NULL: none). */
+int fmoe_gate_linear_topk_route_table(
+    const void *x, const void *w, const void *bias, int64_t n_tokens,
+    int64_t d_model, int64_t n_expert, int64_t top_k, int dtype,
+    int score_mode, int64_t *topk_idx, void *topk_score,
+    int64_t *expert_count, int64_t *pos, int64_t *slot_to_row,
+    void *segment_table, int64_t table_bytes, void *workspace,
+    int64_t workspace_bytes, void *stream);
 
 /* Gradient of topk_score with respect to the logits, [n_tokens, n_expert]
  * (zero at experts that were not selected); score is only read in score_mode 1.

@@ -52,6 +52,28 @@ CONFIG_COUNTS = {
 CONFIG_SLOTS = {"config1": 8192, "config2": 32768, "config3": 16384, "config4": 65536, "config5": 65536}
 
 
+@pytest.mark.parametrize("n_expert", [1, 3, 64, 512, 513, 1025])
+@pytest.mark.parametrize("n_slots", [1, 63, 1024, 1025, 8192, 8193, 20000])
+def test_route_with_its_segment_table(n_slots, n_expert, device):
+    """Counts, positions, their inverse and the segment table of one call, on both sides of the limits of
+    the one-workgroup kernel (8192 slots, 512 experts) and of the table in LDS (1024 experts): integer
+    work, exact."""
+    g = torch.Generator().manual_seed(n_slots + n_expert)
+    gate = torch.randint(-1, n_expert, (n_slots,), generator=g)
+    cnt, pos, s2r, table = fmoe_native.route_table(gate.to(device), n_expert)
+    ref_pos, ref_cnt = orouting.count_by_gate(gate.numpy(), n_expert)
+    total = int(ref_cnt.sum())
+    assert np.array_equal(cnt.cpu().numpy(), ref_cnt)
+    assert np.array_equal(pos[:total].cpu().numpy(), ref_pos) and (pos[total:] == -1).all()
+    inv = np.full(n_slots, -1, dtype=np.int64)
+    inv[ref_pos] = np.arange(total)
+    assert np.array_equal(s2r.cpu().numpy(), inv)
+    got, ref = _unpack(table, n_expert), orouting.segment_table(ref_cnt, n_slots)
+    assert np.array_equal(got["seg"], ref["seg"]) and got["rows"] == total
+    for key in ("tiles256", "tiles128"):
+        assert np.array_equal(got[key][:, :3], ref[key]), key
+
+
 @pytest.mark.parametrize("name", sorted(CONFIG_COUNTS))
 def test_segment_table_at_the_configurations(name, device):
     g = torch.Generator().manual_seed(11)
