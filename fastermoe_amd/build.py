@@ -3,7 +3,7 @@
 ``python -m fastermoe_amd.build`` compiles every translation unit under
 ``csrc/`` in parallel and links them into one shared library that exports the
 C ABI declared in ``include/fmoe_hip.h``.  The grouped-GEMM template is
-compiled once per (element type, product) so that the nine variants build side
+compiled once per (element type, product) so that the variants build side
 by side.
 """
 import os
@@ -40,6 +40,9 @@ def _units():
         for p, pname in GEMM_PRODUCTS.items():
             units.append(("gemm_inst.hip", f"gemm_{tname}_{pname}.o",
                           [f"-DFMOE_GEMM_TYPE={t}", f"-DFMOE_GEMM_PRODUCT={p}"]))
+            if tname != "f32":
+                units.append(("gemm_ring_inst.hip", f"gemm_ring_{tname}_{pname}.o",
+                              [f"-DFMOE_GEMM_TYPE={t}", f"-DFMOE_GEMM_PRODUCT={p}"]))
     return units
 
 

@@ -16,7 +16,7 @@
 // kernel itself (tiling, LDS layouts, software pipeline, epilogues) is in
 // gemm_kernel.hpp and is instantiated once per element type and product by
 // gemm_inst.hip.
-#include "gemm_kernel.hpp"
+#include "gemm_ring.hpp"
 #include "profile.hpp"
 
 #include <algorithm>
@@ -239,6 +239,41 @@ int dispatch(GemmParams &prm, int dtype, int epi, bool fast, hipStream_t stream)
     return fail(FMOE_EINVAL, "unknown dtype %d", dtype);
 }
 
+// Whether a launch over a device table goes to the persistent kernel of gemm_ring.hpp: 16-bit types and enough
+// tiles for 256 x 256 ones (and no tile shape forced).  There it was at least level on every product
+// measured: 4 to 9 % faster at K = 4096, 7 to 14 % at K = 1024, 26 to 37 % on weight gradients of 64 to 256 rows per
+// expert.  32-bit tiles take four times as long per slab, so what happens between them hardly shows.
+bool use_ring(const TileShape &tile, int dtype) {
+    return tile.bm == 256 && tile.bn == 256 && (dtype == FMOE_BF16 || dtype == FMOE_F16) && !getenv("FMOE_GEMM_TILE");
+}
+
+template <int PRODUCT>
+int dispatch_ring(const GemmParams &g, int dtype, int epi, hipStream_t stream) {
+    RingParams prm{};
+    prm.P = g.P; prm.Q = g.Q; prm.C = g.C; prm.bias = g.bias; prm.bias_grad = g.bias_grad; prm.aux = g.aux;
+    prm.ldp = g.ldp; prm.ldq = g.ldq; prm.ldc = g.ldc;
+    prm.p_expert_stride = g.p_expert_stride; prm.c_expert_stride = g.c_expert_stride; prm.bias_expert_stride = g.bias_expert_stride;
+    prm.n_cols = g.n_cols; prm.n_rows = g.n_rows; prm.k_extent = g.k_extent;
+    prm.tiles_n = (int)ceil_div(g.n_cols, kRingTile);
+    prm.tiles_m = PRODUCT == kWgrad ? (int)ceil_div(g.n_rows, kRingTile) : 0;
+    prm.dev_tab = g.dev_tab;
+    prm.n_expert = g.tab.n;
+    prm.dev_map_off = (int32_t)segtab::map256_off(g.tab.n);
+    const int64_t order = segtab::order_off(g.dev_rows_cap, g.tab.n);
+    const int64_t tiles = PRODUCT == kWgrad ? (int64_t)g.tab.n * prm.tiles_m * prm.tiles_n
+                                            : segtab::cap_tiles(g.dev_rows_cap, g.tab.n, kRingTile) * prm.tiles_n;
+    if (order + 4 * (int64_t)g.tab.n > (int64_t)INT32_MAX || tiles > (int64_t)INT32_MAX - 65536)
+        return fail(FMOE_ELIMIT, "grouped GEMM: %lld tiles exceed the supported range", (long long)tiles);
+    prm.dev_order_off = (int32_t)order;
+    prm.split_ws = g.dev_split_ws;
+    ProfileScope prof(g.profile_class, g.profile_work, stream);
+    if (dtype == FMOE_BF16)
+        return PRODUCT == kFwd ? launch_ring_bf16_fwd(prm, epi, g.activation, stream)
+               : PRODUCT == kDgrad ? launch_ring_bf16_dgrad(prm, epi, g.activation, stream) : launch_ring_bf16_wgrad(prm, epi, g.activation, stream);
+    return PRODUCT == kFwd ? launch_ring_f16_fwd(prm, epi, g.activation, stream)
+           : PRODUCT == kDgrad ? launch_ring_f16_dgrad(prm, epi, g.activation, stream) : launch_ring_f16_wgrad(prm, epi, g.activation, stream);
+}
+
 bool is_fast(int dtype, std::initializer_list<const void *> ptrs, std::initializer_list<int64_t> dims) {
     switch (dtype) {
         case FMOE_BF16: return fast_ok<__bf16>(ptrs, dims);
@@ -319,8 +354,9 @@ int64_t linear_dev_workspace_bytes(int64_t contraction, int dtype) {
     if (eb == 0 || dtype == FMOE_F64 || contraction < 1) return 0;
     const int64_t per_slab = kSlabBytes / eb;
     if (!tail_split_possible((int)std::min<int64_t>(ceil_div(contraction, per_slab), 1 << 24), eb == 4 ? 2 : 1)) return 0;
-    // one tile of fp32 accumulators per compute unit: a split never has more parts than that
-    return (int64_t)device_compute_units() * 256 * 256 * (int64_t)sizeof(float);
+    // one tile of fp32 accumulators per compute unit: a split never has more parts than that.  The persistent
+    // kernel's workgroups (16-bit types) leave up to two.
+    return (int64_t)device_compute_units() * 256 * 256 * (int64_t)sizeof(float) * (eb == 2 ? 2 : 1);
 }
 
 int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, int64_t n_expert, int64_t row_lo,
@@ -348,6 +384,10 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
         const int64_t ws_need = linear_dev_workspace_bytes(a.in_feat, a.dtype);
         if (a.dev_workspace != nullptr && ws_need > 0 && a.dev_workspace_bytes >= ws_need && aligned16(a.dev_workspace))
             prm.dev_split_ws = (float *)a.dev_workspace;
+        // (what the persistent kernel is built for; the erf formula, "none" and ReLU with a saved pre-activation are rare)
+        const bool ring_act = a.epilogue == kEpiStore || prm.activation == FMOE_ACT_GELU ||
+                              (prm.activation == FMOE_ACT_RELU && a.aux == nullptr);
+        if (use_ring(tile, a.dtype) && a.x_row_index == nullptr && ring_act) return dispatch_ring<kFwd>(prm, a.dtype, a.epilogue, stream);
         return dispatch<kFwd>(prm, a.dtype, a.epilogue, fast, stream);
     }
     int64_t total;
@@ -400,6 +440,8 @@ int grouped_linear_dgrad(const LinearDgradArgs &a, const int64_t *counts, int64_
         const int64_t ws_need = linear_dev_workspace_bytes(a.out_feat, a.dtype);
         if (a.dev_workspace != nullptr && ws_need > 0 && a.dev_workspace_bytes >= ws_need && aligned16(a.dev_workspace))
             prm.dev_split_ws = (float *)a.dev_workspace;
+        const bool ring_act = a.epilogue == kEpiStore || prm.activation == FMOE_ACT_GELU || prm.activation == FMOE_ACT_RELU;
+        if (use_ring(tile, a.dtype) && ring_act) return dispatch_ring<kDgrad>(prm, a.dtype, a.epilogue, stream);
         return dispatch<kDgrad>(prm, a.dtype, a.epilogue, fast, stream);
     }
     int64_t total;
@@ -445,6 +487,7 @@ int grouped_linear_wgrad(const LinearWgradArgs &a, const int64_t *counts, int64_
         prm.c_expert_stride = a.in_feat * a.out_feat;
         prm.n_cols = (int)a.in_feat; prm.n_rows = (int)a.out_feat;
         prm.accumulate_first = 0;
+        if (use_ring(tile, a.dtype)) return dispatch_ring<kWgrad>(prm, a.dtype, kEpiStore, stream);
         return dispatch<kWgrad>(prm, a.dtype, kEpiStore, fast, stream);
     }
     int64_t total;
@@ -580,6 +623,11 @@ extern "C" int fmoe_linear_dev_supported(int64_t in_feat, int64_t out_feat, int 
     if (eb == 0 || dtype == FMOE_F64 || in_feat < 1 || out_feat < 1) return 0;
     const int64_t ce = 16 / eb;
     return (in_feat % ce == 0 && out_feat % ce == 0 && in_feat * eb <= (1 << 22) && out_feat * eb <= (1 << 22)) ? 1 : 0;
+}
+
+extern "C" int fmoe_linear_dev_reads_rows(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype) {
+    if (!fmoe_linear_dev_supported(in_feat, out_feat, dtype) || rows_cap < 1 || n_expert < 1) return 0;
+    return use_ring(pick_rows_tile_estimate(rows_cap, n_expert, out_feat), dtype) ? 1 : 0;
 }
 
 extern "C" int64_t fmoe_linear_dev_workspace_bytes(int64_t contraction, int dtype) {

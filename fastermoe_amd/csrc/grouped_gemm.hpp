@@ -33,6 +33,8 @@ struct SegmentTable {
 //   [8 .. 8+E]           seg: first row of every expert, seg[E] = rows
 //   [.. +E+1] [.. +E+1]  exclusive prefix of the experts' row tiles, 256 and 128 rows high
 //   tile maps            one {expert, first row, rows, 0} per row tile, 16-byte aligned
+//   order                one {expert, first row, rows, 0} per expert, in descending order of the rows (ties: the
+//                        lower expert first; beyond segtab::kSmallExperts experts: in expert order)
 // A launch is sized for the most row tiles `rows_cap` rows can make (rows_cap / BM + E); the
 // workgroups beyond the table's tile count leave at once.
 namespace segtab {
@@ -48,8 +50,11 @@ __host__ __device__ inline int64_t map256_off(int64_t n_expert) { return (kHeade
 __host__ __device__ inline int64_t map128_off(int64_t rows_cap, int64_t n_expert) {
     return map256_off(n_expert) + 4 * cap_tiles(rows_cap, n_expert, 256);
 }
-__host__ __device__ inline int64_t total_ints(int64_t rows_cap, int64_t n_expert) {
+__host__ __device__ inline int64_t order_off(int64_t rows_cap, int64_t n_expert) {
     return map128_off(rows_cap, n_expert) + 4 * cap_tiles(rows_cap, n_expert, 128);
+}
+__host__ __device__ inline int64_t total_ints(int64_t rows_cap, int64_t n_expert) {
+    return order_off(rows_cap, n_expert) + 4 * n_expert;
 }
 }  // namespace segtab
 

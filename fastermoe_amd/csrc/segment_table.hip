@@ -80,6 +80,7 @@ __global__ __launch_bounds__(kTabBlock) void segment_table_kernel(const int64_t 
             seg[e] = (int32_t)lo;
             pfx256[e] = tb[0] + tv[0] - t[0];
             pfx128[e] = tb[1] + tv[1] - t[1];
+            *(int4 *)(tab + segtab::order_off(rows_cap, n_expert) + 4 * (int64_t)e) = make_int4(e, (int)lo, rows, 0);
         }
         __syncthreads();
         if (threadIdx.x == kTabBlock - 1) {

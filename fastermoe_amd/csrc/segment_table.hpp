@@ -15,6 +15,7 @@ struct SmallLds {
     int32_t wave_sum[2][kThreads / kWave];
     int32_t seg[kSmallExperts + 1];
     int32_t pfx[2][kSmallExperts + 1];
+    __attribute__((aligned(16))) int32_t rows[kSmallExperts];
 };
 
 // The whole table for at most kSmallExperts experts by one workgroup of kThreads threads, thread e
@@ -56,6 +57,7 @@ __device__ __forceinline__ void small_table(int64_t count, int n_expert, int row
     for (int w = 0; w < wave; ++w) { tv[0] += lds.wave_sum[0][w]; tv[1] += lds.wave_sum[1][w]; }
     int32_t *seg = tab + seg_off(), *pfx256 = tab + pfx256_off(n_expert), *pfx128 = tab + pfx128_off(n_expert);
     const int map256 = (int)map256_off(n_expert), map128 = (int)map128_off(rows_cap, n_expert);
+    lds.rows[e] = e < n_expert ? rows : -1;
     if (e < n_expert) {
         lds.seg[e] = seg[e] = (int32_t)lo;
         lds.pfx[0][e] = pfx256[e] = tv[0] - t[0];
@@ -95,6 +97,16 @@ __device__ __forceinline__ void small_table(int64_t count, int n_expert, int row
             entry.w = 0;
             *(int4 *)(map + 4 * (int64_t)i) = entry;
         }
+    }
+    // the experts by descending rows: expert e's place is the number of experts that come before it
+    if (e < n_expert) {
+        int place = 0;
+        for (int f = 0; f < n_expert; f += 4) {
+            const int4 r = *(const int4 *)(lds.rows + f);
+            place += (r.x > rows || (r.x == rows && f < e)) + (r.y > rows || (r.y == rows && f + 1 < e)) +
+                     (r.z > rows || (r.z == rows && f + 2 < e)) + (r.w > rows || (r.w == rows && f + 3 < e));
+        }
+        *(int4 *)(tab + order_off(rows_cap, n_expert) + 4 * (int64_t)place) = make_int4(e, (int)lo, rows, 0);
     }
 }
 

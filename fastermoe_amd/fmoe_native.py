@@ -600,6 +600,12 @@ def linear_dev_supported(in_feat, out_feat, dtype):
     return dtype in _DTYPES and _lib.load().fmoe_linear_dev_supported(int(in_feat), int(out_feat), _DTYPES[dtype]) == 1
 
 
+def linear_dev_reads_rows(rows_cap, n_expert, in_feat, out_feat, dtype):
+    """Whether :func:`linear_forward_dev` for these sizes is faster over sorted rows than through ``row_index``."""
+    return _lib.load().fmoe_linear_dev_reads_rows(int(rows_cap), int(n_expert), int(in_feat), int(out_feat),
+                                                  _DTYPES[dtype]) == 1
+
+
 def _dev_workspace(contraction, dt, device):
     """The caller-side workspace of the row-ragged ``*_dev`` products (``None`` when this contraction is
     never split); torch's caching allocator hands the same block back call after call."""

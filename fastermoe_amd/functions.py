@@ -349,33 +349,37 @@ class MOEExpertMLP(Function):
 class MOERoutedMLP(Function):
     r"""``MOEScatter`` -> ``Linear -> activation -> Linear`` (fmoe/functions.py:196-248,
     fmoe/transformer.py:22-30) over the rows as the routing kernels left them, with nothing read
-    back to the host: the first GEMM reads token row ``pos_buf[r] // top_k`` for sorted row ``r``
-    in its loader (no scattered copy), and all GEMMs take the experts' row segments from
-    ``table``, the device-side segment table of the routing's counts.  Returns the experts' output
-    in expert-sorted order, one row per slot (``[n_slots, d_model]``; the rows past the routed
-    ones are not written), for :class:`MOEGatherCombine` / :class:`MOEGather`.  The backward makes
-    the sorted copy of the input that the first linear's weight gradient contracts over.
+    back to the host: all GEMMs take the experts' row segments from ``table``, the device-side segment
+    table of the routing's counts.  Small first GEMMs read token row ``pos_buf[r] // top_k`` for
+    sorted row ``r`` in their loader (no scattered copy in the forward); large ones run on a kernel that wants
+    sorted rows, and the copy made for them serves the first linear's weight gradient too.  Returns the
+    experts' output in expert-sorted order, one row per slot (``[n_slots, d_model]``; the rows past the
+    routed ones are not written), for :class:`MOEGatherCombine` / :class:`MOEGather`.  With ``save`` false (nothing
+    will be differentiated) the pre-activations are not written.
     Not in the reference; same results as ``MOEScatter`` + the three modules."""
 
     @staticmethod
-    def forward(ctx, inp, w1, b1, w2, b2, pos_buf, slot_to_row, table, top_k, activation):
+    def forward(ctx, inp, w1, b1, w2, b2, pos_buf, slot_to_row, table, top_k, activation, save):
         from . import _lib
         inp = inp.contiguous()
         n_slots = pos_buf.numel()
-        keep_pre = activation == _lib.ACT_GELU  # ReLU's derivative can be read off the output
-        in_loader = inp.numel() * inp.element_size() < (1 << 31)
-        src = inp if in_loader else fmoe_native.gather_rows(inp, pos_buf, index_div=top_k)
-        mid, pre = fmoe_native.linear_forward_dev(src, w1, b1, table, n_slots, activation, keep_pre,
+        keep_pre = save and activation == _lib.ACT_GELU  # ReLU's derivative can be read off the output
+        n_expert, d_hidden, d_model = w1.shape
+        in_loader = (inp.numel() * inp.element_size() < (1 << 31)
+                     and not fmoe_native.linear_dev_reads_rows(n_slots, n_expert, d_model, d_hidden, inp.dtype))
+        rows = None if in_loader else fmoe_native.gather_rows(inp, pos_buf, index_div=top_k)
+        mid, pre = fmoe_native.linear_forward_dev(inp if in_loader else rows, w1, b1, table, n_slots, activation, keep_pre,
                                                   row_index=pos_buf if in_loader else None, index_div=top_k)
         out, _ = fmoe_native.linear_forward_dev(mid, w2, b2, table, n_slots)
-        ctx.save_for_backward(inp, w1, b1, w2, b2, pos_buf, slot_to_row, table, pre, mid)
-        ctx.moe_args = top_k, activation
+        if save:
+            ctx.save_for_backward(inp if in_loader else None, rows, w1, b1, w2, b2, pos_buf, slot_to_row, table, pre, mid)
+        ctx.moe_args = top_k, activation, inp.shape[0]
         return out
 
     @staticmethod
     def backward(ctx, grad_out):
-        inp, w1, b1, w2, b2, pos_buf, slot_to_row, table, pre, mid = ctx.saved_tensors
-        top_k, activation = ctx.moe_args
+        inp, rows, w1, b1, w2, b2, pos_buf, slot_to_row, table, pre, mid = ctx.saved_tensors
+        top_k, activation, n_tokens = ctx.moe_args
         n_slots = pos_buf.numel()
         grad_out = grad_out.contiguous()
         g_pre = fmoe_native.linear_dgrad_dev(grad_out, w2, table, n_slots, pre if pre is not None else mid, activation)
@@ -383,10 +387,11 @@ class MOERoutedMLP(Function):
         g_inp = None
         if ctx.needs_input_grad[0]:
             g_rows = fmoe_native.linear_dgrad_dev(g_pre, w1, table, n_slots)
-            g_inp = fmoe_native.reduce_slots(g_rows, slot_to_row, inp.shape[0], top_k)
-        rows = fmoe_native.gather_rows(inp, pos_buf, index_div=top_k)
+            g_inp = fmoe_native.reduce_slots(g_rows, slot_to_row, n_tokens, top_k)
+        if rows is None:
+            rows = fmoe_native.gather_rows(inp, pos_buf, index_div=top_k)
         gw1, gb1 = fmoe_native.linear_wgrad_dev(g_pre, rows, w1, table, n_slots, b1 is not None)
-        return g_inp, gw1, gb1, gw2, gb2, None, None, None, None, None
+        return g_inp, gw1, gb1, gw2, gb2, None, None, None, None, None, None
 
 
 class MOEGather(Function):

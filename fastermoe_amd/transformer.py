@@ -49,8 +49,9 @@ class _Expert(nn.Module):
             return None
         if table is None:
             table = fmoe_native.segment_table(counts_dev, pos_buf.numel())
-        return MOERoutedMLP.apply(inp, self.htoh4.weight, self.htoh4.bias, self.h4toh.weight, self.h4toh.bias,
-                                  pos_buf, slot_to_row, table, top_k, code)
+        params = (self.htoh4.weight, self.htoh4.bias, self.h4toh.weight, self.h4toh.bias)
+        save = torch.is_grad_enabled() and (inp.requires_grad or any(p is not None and p.requires_grad for p in params))
+        return MOERoutedMLP.apply(inp, *params, pos_buf, slot_to_row, table, top_k, code, save)
 
     def _epilogue_activation(self):
         from .fused_functions import _activation_code

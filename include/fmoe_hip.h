@@ -409,6 +409,12 @@ int fmoe_segment_table_build(const int64_t *expert_count, int64_t n_expert,
  * feature sizes that are multiples of 16 bytes), else 0.  Host only. */
 int fmoe_linear_dev_supported(int64_t in_feat, int64_t out_feat, int dtype);
 
+/* Whether fmoe_linear_forward_dev for these sizes runs on the kernel that reads
+ * the rows of x in order (1: sorted rows are faster than x_row_index; 0:
+ * either). */
+int fmoe_linear_dev_reads_rows(int64_t rows_cap, int64_t n_expert,
+                               int64_t in_feat, int64_t out_feat, int dtype);
+
 /* Bytes of workspace with which the two row-ragged products below can split a
  * last, partial round of tiles along the contraction (the host-count entry
  * points keep such a workspace inside the library; here it is the caller's, so

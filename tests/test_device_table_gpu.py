@@ -239,3 +239,70 @@ def test_split_tail_over_the_device_table(dtype, rows, slots, e, fin, fout, tile
             assert torch.equal(y[:rows], y_host[:rows]) and torch.equal(gx[:rows], gx_host[:rows])
         else:
             assert rel_err(y[:rows], y_host[:rows]) <= TOL[dtype] and rel_err(gx[:rows], gx_host[:rows]) <= TOL[dtype]
+
+
+# counts at the edges of the 256-row tiles and of the 64-row wave tiles, experts without rows, and a last partial round of
+# tiles; sizes that give the persistent kernel of the 16-bit types enough tiles for each of the three products
+RING_CASES = [  # counts, in, out
+    ([1, 64, 65, 127, 0, 128, 129, 255, 256, 257, 0, 511, 3000, 700, 900, 1800], 328, 4104),   # contraction and column remainders
+    ([1500, 0, 2700, 3000, 1000], 3336, 4608),   # 53 slabs, 8 or 9 whole rounds and a short tail
+    ([2300, 1900, 0, 3992], 8, 5000),            # one slab of one 16-byte chunk
+    ([9000, 300], 4096, 4096),                   # an exact number of slabs; a tail cut along the contraction
+    ([0] * 40 + [2, 1] * 30 + [700] * 12, 520, 1040),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", range(len(RING_CASES)))
+def test_persistent_kernel_products(case, dtype, device):
+    """The products of many 256 x 256 tiles (one persistent workgroup per compute unit): every epilogue against
+    float32 products of the same operands.  Bound per element: one rounding of the result to the element type
+    (2^-8 for bfloat16, 2^-11 for float16, relative) plus 1e-3 of the rms, which covers the float32 sums in another
+    order (K 2^-24 < 3e-4) and the GELU polynomials (1.4e-4)."""
+    counts, fin, fout = RING_CASES[case]
+    counts = torch.tensor(counts, dtype=torch.int64)
+    e, rows = counts.numel(), int(counts.sum())
+    slots = rows + 5
+    g = torch.Generator(device=device).manual_seed(case)
+    rnd = lambda *s: torch.randn(*s, device=device, generator=g)
+    x, gy = rnd(slots, fin).to(dtype), rnd(slots, fout).to(dtype)
+    w, b = (rnd(e, fout, fin) / fin ** 0.5).to(dtype), rnd(e, fout).to(dtype)
+    pre_in = (2 * rnd(slots, fin)).to(dtype)
+    table = fmoe_native.segment_table(counts.to(device), slots)
+    y, pre = fmoe_native.linear_forward_dev(x, w, b, table, slots, _lib.ACT_GELU, True)
+    y_np, none = fmoe_native.linear_forward_dev(x, w, b, table, slots, _lib.ACT_GELU, False)
+    y_relu, _ = fmoe_native.linear_forward_dev(x, w, b, table, slots, _lib.ACT_RELU, False)
+    y_plain, _ = fmoe_native.linear_forward_dev(x, w, None, table, slots)
+    gx = fmoe_native.linear_dgrad_dev(gy, w, table, slots)
+    gx_gelu = fmoe_native.linear_dgrad_dev(gy, w, table, slots, pre_in, _lib.ACT_GELU)
+    gx_relu = fmoe_native.linear_dgrad_dev(gy, w, table, slots, pre_in, _lib.ACT_RELU)
+    gw, gb = fmoe_native.linear_wgrad_dev(gy, x, w, table, slots, True)
+    gw_nb, none_b = fmoe_native.linear_wgrad_dev(gy, x, w, table, slots, False)
+    assert none is None and none_b is None and torch.equal(y[:rows], y_np[:rows]) and torch.equal(gw, gw_nb)
+
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    def close(got, ref, what):
+        bound = eps * ref.abs() + 1e-3 * ref.pow(2).mean().sqrt().clamp(min=1e-3)
+        assert bool(((got.float() - ref).abs() <= bound).all()), what
+    lo = 0
+    for ex, n in enumerate(counts.tolist()):
+        r = slice(lo, lo + n)
+        lo += n
+        if n == 0:
+            assert torch.count_nonzero(gw[ex]) == 0 and torch.count_nonzero(gb[ex]) == 0
+            continue
+        xs, gs, ws, ps = x[r].float(), gy[r].float(), w[ex].float(), pre_in[r].float()
+        plain = xs @ ws.t()
+        full = plain + b[ex].float()
+        close(y_plain[r], plain, f"expert {ex}: forward")
+        close(pre[r], full, f"expert {ex}: pre-activation")
+        close(y[r], torch.nn.functional.gelu(full), f"expert {ex}: gelu")
+        close(y_relu[r], torch.relu(full), f"expert {ex}: relu")
+        back = gs @ ws
+        close(gx[r], back, f"expert {ex}: data gradient")
+        ps = ps.requires_grad_(True)
+        torch.nn.functional.gelu(ps).sum().backward()
+        close(gx_gelu[r], back * ps.grad, f"expert {ex}: gelu derivative")
+        close(gx_relu[r], back * (ps > 0), f"expert {ex}: relu derivative")
+        close(gw[ex], gs.t() @ xs, f"expert {ex}: weight gradient")
+        close(gb[ex], gs.sum(dim=0), f"expert {ex}: bias gradient")
