@@ -13,8 +13,8 @@
 //   * the epilogue is staged through the Q buffer of the slab just finished (4 KiB per wave, 16 rows
 //     at a time) instead of through all of LDS, whose other buffers hold the next tile's slabs;
 //   * a tile of 128 rows or fewer leaves the waves of its lower half out of the products;
-//   * the tiles are dealt to the workgroups beforehand: row-ragged products in the XCD-contiguous order
-//     of the tile map; the weight gradient expert by expert in descending order of their rows (the table's
+//   * the tiles are dealt to the workgroups beforehand: row-ragged products in bands of row
+//     tiles shared by the XCDs; the weight gradient expert by expert in descending order of their rows (the table's
 //     order list), back and forth over the workgroups, so that every workgroup gets its share of long and
 //     short contractions;
 //   * the bias gradient is one more column of products (a block of ones times the output gradient).
@@ -76,7 +76,7 @@ inline bool ring_split_possible(int n_slabs) { return n_slabs - (n_slabs + kRing
 // the run that holds slab x of the tail's tail * n_slabs slabs; run j is [j * total / wgs, (j + 1) * total / wgs)
 __device__ __forceinline__ int ring_run_of(int x, int total, int wgs) { return ((x + 1) * wgs - 1) / total; }
 
-// tile `rem` of the logical order (groups of kGroupM row tiles per column tile): row tile and column tile
+// tile `rem` of `tm_total` row tiles x tiles_n column tiles, in groups of kGroupM row tiles per column tile
 __device__ __forceinline__ void ring_tile_coords(int rem, int tiles_n, int tm_total, int &mt, int &nt) {
     // (the compiler divides in vector registers; what depends on the quotient belongs in scalar ones)
     const int gspan = kGroupM * tiles_n;
@@ -86,6 +86,33 @@ __device__ __forceinline__ void ring_tile_coords(int rem, int tiles_n, int tm_to
     nt = __builtin_amdgcn_readfirstlane(in_grp / gsz);
     mt = grp * kGroupM + (in_grp - nt * gsz);
 }
+
+// The tiles of a row-ragged launch by XCD (each has its own L2).  Bands of kRingBand row tiles go to the eight XCDs in
+// equal parts, one group of kGroupM row tiles each, so that all of them sweep the same experts' columns at the same time
+// and a weight slab that one of them has fetched is in the memory-side cache for the others (with a
+// contiguous eighth of all row tiles per XCD each works on experts of its own: 65536 rows over 8 experts of
+// 4096 x 14336, K = 14336: 5716 us, in bands 5340).  The rows past the last whole band are dealt in contiguous eighths of their tiles.
+constexpr int kRingBand = 8 * kGroupM;
+struct RingShare {
+    int per_band, bands, rest_tiles, per_xcd;   // tiles of an XCD per band, bands, tiles past them, an XCD's share of those
+    __device__ __forceinline__ RingShare(int tm_total, int tiles_n)
+        : per_band(kGroupM * tiles_n), bands(tm_total / kRingBand), rest_tiles((tm_total % kRingBand) * tiles_n),
+          per_xcd((rest_tiles + 7) >> 3) {}
+    __device__ __forceinline__ int tiles(int xcd) const {
+        return bands * per_band + max(0, min(per_xcd, rest_tiles - xcd * per_xcd));
+    }
+    // row tile and column tile of the XCD's tile i
+    __device__ __forceinline__ void coords(int xcd, int i, int tm_total, int tiles_n, int &mt, int &nt) const {
+        const int band = __builtin_amdgcn_readfirstlane(i / per_band);
+        if (band < bands) {
+            ring_tile_coords(i - band * per_band, tiles_n, kGroupM, mt, nt);
+            mt += band * kRingBand + xcd * kGroupM;
+        } else {
+            ring_tile_coords(xcd * per_xcd + i - bands * per_band, tiles_n, tm_total - bands * kRingBand, mt, nt);
+            mt += bands * kRingBand;
+        }
+    }
+};
 
 constexpr int kRingThreads = 512, kRingWaves = 8;
 constexpr int kRingTile = 256;
@@ -219,16 +246,13 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_ring_kernel(const R
     // -- this workgroup's list of items -----------------------------------------------------
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, per = gridDim.x >> 3;
     auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
-    int n_items, tm_total, per_xcd = 0;
+    int n_items, tm_total;
     RingPlan plan{0, 0, 0};
     int run_lo = 0, run_hi = 0, k_slabs = 0;   // this workgroup's run of the tail's slabs
     if (RAGGED == kRaggedRows) {
         tm_total = dtab[segtab::kTiles256];
-        const int total = tm_total * prm.tiles_n;
-        per_xcd = (total + 7) >> 3;
-        const int mine = max(0, min(per_xcd, total - xcd * per_xcd));   // tiles of this XCD
         k_slabs = (prm.k_extent + BKE - 1) / BKE;
-        plan = ring_plan(mine, per, k_slabs, prm.split_ws != nullptr);
+        plan = ring_plan(RingShare(tm_total, prm.tiles_n).tiles(xcd), per, k_slabs, prm.split_ws != nullptr);
         plan.full = uniform(plan.full);
         plan.tail = uniform(plan.tail);
         plan.split_wgs = uniform(plan.split_wgs);
@@ -261,11 +285,11 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_ring_kernel(const R
         if (RAGGED == kRaggedRows) {
             tl.K = prm.k_extent;
             if (plan.split_wgs == 0 || r < plan.full) {
-                rem = xcd * per_xcd + r * per + slot;
+                rem = r * per + slot;
             } else {
                 const int first_tile = uniform(run_lo / k_slabs), tail_tile = first_tile + (r - plan.full);
                 const int lo = max(run_lo, tail_tile * k_slabs), hi = min(run_hi, (tail_tile + 1) * k_slabs);
-                rem = xcd * per_xcd + plan.full * per + tail_tile;
+                rem = plan.full * per + tail_tile;
                 tl.partial = hi - lo < k_slabs;
                 tl.first_slab = lo - tail_tile * k_slabs;
                 tl.K = min(prm.k_extent - tl.first_slab * BKE, (hi - lo) * BKE);
@@ -278,7 +302,8 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_ring_kernel(const R
             rem = q - ei * tpe;
             entry = *(DevTab4)(dtab + prm.dev_order_off + 4 * ei);
         }
-        ring_tile_coords(rem, prm.tiles_n, tm_total, mt, nt);
+        if (RAGGED == kRaggedRows) RingShare(tm_total, prm.tiles_n).coords(xcd, rem, tm_total, prm.tiles_n, mt, nt);
+        else ring_tile_coords(rem, prm.tiles_n, tm_total, mt, nt);
         tl.n0 = nt * kRingTile;
         tl.p_valid = min(kRingTile, prm.n_cols - tl.n0);
         if (RAGGED == kRaggedRows) {
@@ -667,16 +692,17 @@ __global__ __launch_bounds__(64) void ring_combine_kernel(const RingParams prm) 
     const DevTab dtab = (DevTab)(uintptr_t)prm.dev_tab;
     const int per = prm.ws_wgs >> 3;
     const int y = blockIdx.x & 3, wave = (blockIdx.x >> 2) & 7, unit = blockIdx.x >> 5, xcd = unit & 7, tail_tile = unit >> 3;
-    const int tm_total = dtab[segtab::kTiles256], total = tm_total * prm.tiles_n, per_xcd = (total + 7) >> 3;
+    const int tm_total = dtab[segtab::kTiles256];
+    const RingShare share(tm_total, prm.tiles_n);
     const int k_slabs = (prm.k_extent + 63) / 64;
-    const RingPlan plan = ring_plan(max(0, min(per_xcd, total - xcd * per_xcd)), per, k_slabs, true);
+    const RingPlan plan = ring_plan(share.tiles(xcd), per, k_slabs, true);
     if (plan.split_wgs == 0 || tail_tile >= plan.tail) return;
     const int slabs = plan.tail * k_slabs, wgs = plan.split_wgs;
     const int first = ring_run_of(tail_tile * k_slabs, slabs, wgs), last = ring_run_of((tail_tile + 1) * k_slabs - 1, slabs, wgs);
     if (first == last) return;   // one workgroup had all of it and has stored it
     RingTile<T> tl{};
     int mt, nt;
-    ring_tile_coords(xcd * per_xcd + plan.full * per + tail_tile, prm.tiles_n, tm_total, mt, nt);
+    share.coords(xcd, plan.full * per + tail_tile, tm_total, prm.tiles_n, mt, nt);
     const ring_i32x4 entry = *(DevTab4)(dtab + prm.dev_map_off + 4 * mt);
     tl.n0 = nt * kRingTile;
     tl.p_valid = min(kRingTile, prm.n_cols - tl.n0);

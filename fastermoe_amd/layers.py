@@ -84,6 +84,7 @@ def _fmoe_general_global_forward(inp, gate, expert_fn, policy_fn, experts, num_e
            and gate.numel() == inp.shape[0] * topk and fused and _own_expert_path(expert_fn, experts))
     if own:
         _single_worker(world_size, "count_by_gate")
+        enable_fuse = enable_fuse and not experts.unchunked_is_faster(inp, gate.numel())
         routed = _route_launch(gate, num_expert, with_table=not enable_fuse)
         counts_dev, pos_buf, slot_to_row = routed[:3]
         if not enable_fuse:

@@ -39,19 +39,32 @@ class _Expert(nn.Module):
         counts, where the call made one), without any of them being read on the host: returns the
         experts' output in expert-sorted order, one row per slot, or ``None`` when this shape or
         activation needs the module-by-module path."""
-        code = self._epilogue_activation()
-        d_hidden, d_model = self.htoh4.weight.shape[1:]
-        if (code is None or not inp.is_cuda or inp.dtype not in (torch.float32, torch.bfloat16, torch.float16)
-                or self.htoh4.weight.dtype != inp.dtype or self.h4toh.weight.dtype != inp.dtype
-                or os.environ.get("FMOE_EXPERT_EPILOGUE", "1") == "0"
-                or os.environ.get("FMOE_DEVICE_TABLES", "1") == "0"
-                or not fmoe_native.linear_dev_supported(d_model, d_hidden, inp.dtype)):
+        if not self._device_tables_apply(inp):
             return None
+        code = self._epilogue_activation()
         if table is None:
             table = fmoe_native.segment_table(counts_dev, pos_buf.numel())
         params = (self.htoh4.weight, self.htoh4.bias, self.h4toh.weight, self.h4toh.bias)
         save = torch.is_grad_enabled() and (inp.requires_grad or any(p is not None and p.requires_grad for p in params))
         return MOERoutedMLP.apply(inp, *params, pos_buf, slot_to_row, table, top_k, code, save)
+
+    def unchunked_is_faster(self, inp, n_slots):
+        r"""Whether :meth:`routed_forward` beats the chunked pipeline: where both linears run on the persistent
+        kernel and nobody asks for a number of chunks.  The pipeline hides the row permutes behind the
+        products of its chunks, but needs the counts on the host and pays every chunk's last round of tiles."""
+        n_expert, d_hidden, d_model = self.htoh4.weight.shape
+        return ("FMOE_FUSE_GRAN" not in os.environ and self._device_tables_apply(inp)
+                and fmoe_native.linear_dev_reads_rows(n_slots, n_expert, d_model, d_hidden, inp.dtype)
+                and fmoe_native.linear_dev_reads_rows(n_slots, n_expert, d_hidden, d_model, inp.dtype))
+
+    def _device_tables_apply(self, inp):
+        d_hidden, d_model = self.htoh4.weight.shape[1:]
+        return (self._epilogue_activation() is not None and inp.is_cuda
+                and inp.dtype in (torch.float32, torch.bfloat16, torch.float16)
+                and self.htoh4.weight.dtype == inp.dtype and self.h4toh.weight.dtype == inp.dtype
+                and os.environ.get("FMOE_EXPERT_EPILOGUE", "1") != "0"
+                and os.environ.get("FMOE_DEVICE_TABLES", "1") != "0"
+                and fmoe_native.linear_dev_supported(d_model, d_hidden, inp.dtype))
 
     def _epilogue_activation(self):
         from .fused_functions import _activation_code
