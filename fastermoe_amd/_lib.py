@@ -42,6 +42,10 @@ SIGNATURES = {
     "fmoe_gate_linear_topk_route_table": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp, _vp, _vp, _vp, _vp,
                                                  _vp, _i64, _vp, _i64, _vp]),
     "fmoe_gate_topk_backward": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _int, _vp]),
+    "fmoe_gate_grad_supported": (_int, [_i64, _i64, _i64, _int]),
+    "fmoe_gate_weight_grad_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "fmoe_gate_weight_grad": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _i64, _vp]),
+    "fmoe_reduce_slots_gate": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp]),
     "fmoe_noisy_gate_forward": (_int, [_vp, _vp, _vp, ctypes.c_double, _i64, _i64, _i64, _int, _vp, _vp, _vp, _vp, _vp,
                                        _vp, _vp, _vp, _vp, _i64, _vp]),
     "fmoe_noisy_gate_backward": (_int, [_vp, _vp, _vp, ctypes.c_double, _i64, _i64, _i64, _int, _vp, _vp, _vp, _vp, _vp,

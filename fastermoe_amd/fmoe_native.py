@@ -264,6 +264,57 @@ def gate_topk_backward(grad_score, score, topk_idx, n_expert, score_mode=0):
     return grad_logits
 
 
+def gate_grad_supported(d_model, n_expert, top_k, dtype):
+    """Whether :func:`gate_weight_grad` and :func:`reduce_slots_gate` take this gate."""
+    return dtype in _DTYPES and _lib.load().fmoe_gate_grad_supported(int(d_model), int(n_expert), int(top_k),
+                                                                     _DTYPES[dtype]) == 1
+
+
+def gate_weight_grad(grad_score, topk_idx, x, n_expert, with_bias):
+    """Gradients ``(grad_w [E, d_model], grad_b [E] or None)`` of the gate's linear layer from the gradient
+    ``[N, k]`` of the selected logits."""
+    dt = _rows("x", x)
+    _dev("grad_score", grad_score, x.dtype)
+    _dev("topk_idx", topk_idx, torch.int64)
+    n, d = x.shape
+    if topk_idx.dim() != 2 or topk_idx.shape[0] != n or grad_score.numel() != topk_idx.numel():
+        raise ValueError(f"grad_score and topk_idx must be [{n}, top_k]")
+    k = topk_idx.shape[1]
+    lib = _lib.load()
+    grad_w = torch.empty(n_expert, d, dtype=x.dtype, device=x.device)
+    grad_b = torch.empty(n_expert, dtype=x.dtype, device=x.device) if with_bias else None
+    if n == 0:
+        return grad_w.zero_(), grad_b.zero_() if with_bias else None
+    with torch.cuda.device(x.device):
+        ws = _workspace(lib.fmoe_gate_weight_grad_workspace_bytes(n, d, n_expert), x.device)
+        check(lib.fmoe_gate_weight_grad(_ptr(grad_score), _ptr(topk_idx), _ptr(x), _ptr(grad_w), _ptr(grad_b), n, d, n_expert, k,
+                                        dt, _ptr(ws), ws.numel(), _stream(x)))
+    return grad_w, grad_b
+
+
+def reduce_slots_gate(inp, slot_to_row, grad_score, topk_idx, weight):
+    """:func:`reduce_slots` plus the gate's part of the input gradient,
+    ``sum_j grad_score[t,j] * weight[topk_idx[t,j]]``; ``inp`` and ``slot_to_row`` ``None``: that part alone."""
+    dt = _rows("weight", weight)
+    _dev("grad_score", grad_score, weight.dtype)
+    _dev("topk_idx", topk_idx, torch.int64)
+    n, k = topk_idx.shape
+    e, d = weight.shape
+    if grad_score.numel() != n * k:
+        raise ValueError("grad_score must have one entry per slot")
+    if inp is not None:
+        _rows("inp", inp)
+        _dev("slot_to_row", slot_to_row, torch.int64)
+        if inp.dtype != weight.dtype or inp.shape[1] != d or slot_to_row.numel() != n * k:
+            raise ValueError("inp must be rows like weight's, slot_to_row must have one entry per slot")
+    out = torch.empty(n, d, dtype=weight.dtype, device=weight.device)
+    with torch.cuda.device(weight.device):
+        check(_lib.load().fmoe_reduce_slots_gate(_ptr(inp), _ptr(slot_to_row if inp is not None else None), _ptr(grad_score),
+                                                 _ptr(topk_idx), _ptr(weight), _ptr(out), n, k, 0 if inp is None else inp.shape[0],
+                                                 e, d, dt, _stream(weight)))
+    return out
+
+
 def limit_by_capacity(expert_count, capacity, n_expert, n_worker):
     """fmoe_cuda.limit_by_capacity, cuda/balancing.cu:7-20."""
     _dev("expert_count", expert_count, torch.int64)

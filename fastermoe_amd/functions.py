@@ -51,15 +51,20 @@ class GateTopK(Function):
 class GateLinearTopK(Function):
     r"""``nn.Linear`` -> ``torch.topk`` (-> softmax) of fmoe/gates/naive_gate.py:26-42 and the routing of
     ``count_by_gate`` in one call that keeps the logits on chip.  Returns ``(topk_idx, topk_score)`` like
-    :class:`GateTopK`; the routing rides on ``topk_idx``.  Backward: the sparse gradient of the logits
-    (``fmoe_gate_topk_backward``), then the linear layer's own backward as two skinny library products."""
+    :class:`GateTopK`; the routing rides on ``topk_idx``.  Gates of more experts than that call takes run the linear
+    layer as a library product first.  Backward: straight from the gradient of the selected logits; a softmax over
+    them, or a shape these kernels do not take, goes through the dense gradient of the logits and library products."""
 
     @staticmethod
     def forward(ctx, x, weight, bias, top_k, score_mode):
         x = x.contiguous()
         weight = weight.contiguous()
-        idx, score, cnt, pos_buf, s2r, table = fmoe_native.gate_linear_topk_route(x, weight, bias, top_k, score_mode,
-                                                                                  with_table=True)
+        if fmoe_native.gate_linear_supported(x.shape[1], weight.shape[0], top_k, x.dtype):
+            idx, score, cnt, pos_buf, s2r, table = fmoe_native.gate_linear_topk_route(x, weight, bias, top_k, score_mode,
+                                                                                      with_table=True)
+        else:
+            idx, score, cnt, pos_buf, s2r, table = fmoe_native.gate_topk_route(
+                torch.nn.functional.linear(x, weight, bias), top_k, score_mode, with_table=True)
         ctx.save_for_backward(x, weight, idx, score)
         ctx.moe_args = score_mode, bias is not None
         ctx.mark_non_differentiable(idx)
@@ -71,11 +76,26 @@ class GateLinearTopK(Function):
     def backward(ctx, _grad_idx, grad_score):
         x, weight, idx, score = ctx.saved_tensors
         score_mode, has_bias = ctx.moe_args
-        g = fmoe_native.gate_topk_backward(grad_score.contiguous(), score, idx, weight.shape[0], score_mode)
+        grad_score = grad_score.contiguous()
+        if score_mode == 0 and fmoe_native.gate_grad_supported(x.shape[1], weight.shape[0], idx.shape[1], x.dtype):
+            grad_x = grad_w = grad_b = None
+            if ctx.needs_input_grad[0]:
+                grad_x = fmoe_native.reduce_slots_gate(None, None, grad_score, idx, weight)
+            if ctx.needs_input_grad[1] or (has_bias and ctx.needs_input_grad[2]):
+                grad_w, grad_b = fmoe_native.gate_weight_grad(grad_score, idx, x, weight.shape[0], has_bias)
+            return grad_x, grad_w, grad_b, None, None
+        g = fmoe_native.gate_topk_backward(grad_score, score, idx, weight.shape[0], score_mode)
         grad_x = g @ weight if ctx.needs_input_grad[0] else None
         grad_w = g.t() @ x if ctx.needs_input_grad[1] else None
         grad_b = g.float().sum(dim=0).to(g.dtype) if has_bias and ctx.needs_input_grad[2] else None
         return grad_x, grad_w, grad_b, None, None
+
+
+def _plain_linear(linear):
+    """Whether calling ``linear`` is ``F.linear`` on its parameters and nothing else."""
+    return (type(linear) is torch.nn.Linear and "forward" not in linear.__dict__
+            and not (linear._forward_hooks or linear._forward_pre_hooks or linear._backward_hooks
+                     or linear._backward_pre_hooks))
 
 
 def gate_linear_topk(x, linear, top_k, score_mode=0):
@@ -86,9 +106,14 @@ def gate_linear_topk(x, linear, top_k, score_mode=0):
     w, b = linear.weight, linear.bias
     if (x.is_cuda and x.dim() == 2 and w.is_cuda and w.dtype == x.dtype and (b is None or b.dtype == x.dtype)
             and os.environ.get("FMOE_GATE_LINEAR_FUSED", "1") != "0"
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and fmoe_native.gate_linear_supported(x.shape[1], w.shape[0], top_k, x.dtype)):
-        return GateLinearTopK.apply(x, w, b, top_k, score_mode)
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+        if fmoe_native.gate_linear_supported(x.shape[1], w.shape[0], top_k, x.dtype):
+            return GateLinearTopK.apply(x, w, b, top_k, score_mode)
+        # more experts: the library makes the logits, their gradient still is never formed
+        if (_plain_linear(linear) and score_mode == 0 and x.shape[0] > 0 and not torch.is_autocast_enabled()
+                and fmoe_native.gate_topk_supported(w.shape[0], top_k, x.dtype)
+                and fmoe_native.gate_grad_supported(x.shape[1], w.shape[0], top_k, x.dtype)):
+            return GateLinearTopK.apply(x, w, b, top_k, score_mode)
     return gate_topk(linear(x), top_k, score_mode)
 
 

@@ -143,8 +143,8 @@ int fmoe_gate_topk_route_table(const void *logits, int64_t n_tokens,
  * experts, top_k 1, 2, 4 or 8, d_model a whole number of 16-byte chunks);
  * FMOE_ELIMIT otherwise.  Replaces nn.Linear + torch.topk (+ softmax) of
  * fmoe/gates/naive_gate.py:26-42 followed by count_by_gate,
- * fmoe/functions.py:19-42.  Its backward is fmoe_gate_topk_backward followed by
- * the linear layer's own (two skinny library GEMMs). */
+ * fmoe/functions.py:19-42.  Its backward: fmoe_gate_weight_grad and
+ * fmoe_reduce_slots_gate, or fmoe_gate_topk_backward and the linear layer's own. */
 int fmoe_gate_linear_supported(int64_t d_model, int64_t n_expert, int64_t top_k,
                                int dtype);
 int fmoe_gate_linear_topk_route(const void *x, const void *w, const void *bias,
@@ -172,6 +172,37 @@ int fmoe_gate_topk_backward(const void *grad_score, const void *score,
                             const int64_t *topk_idx, void *grad_logits,
                             int64_t n_tokens, int64_t n_expert, int64_t top_k,
                             int dtype, int score_mode, void *stream);
+
+/* Backward of the gate's linear layer from the gradient of the selected logits
+ * (score_mode 0), grad_score [n_tokens, top_k] at the experts topk_idx: the
+ * gradient of the logits is never formed.
+ * grad_w[e,:] = sum over (t,j) with topk_idx[t,j] == e of grad_score[t,j] x[t,:],
+ * grad_b[e] the same without x (grad_b may be NULL); summed in fp32 in a fixed
+ * order.  The experts of a token are distinct (those of a top-k are); indices
+ * outside [0, n_expert) count for nothing.  Taken where
+ * fmoe_gate_grad_supported says so (at most 256 experts, d_model a whole number
+ * of 16-byte chunks), FMOE_ELIMIT otherwise.
+ * Replaces autograd's backward of the nn.Linear of fmoe/gates/naive_gate.py:26-42. */
+int fmoe_gate_grad_supported(int64_t d_model, int64_t n_expert, int64_t top_k,
+                             int dtype);
+int64_t fmoe_gate_weight_grad_workspace_bytes(int64_t n_tokens, int64_t d_model,
+                                              int64_t n_expert);
+int fmoe_gate_weight_grad(const void *grad_score, const int64_t *topk_idx,
+                          const void *x, void *grad_w, void *grad_b,
+                          int64_t n_tokens, int64_t d_model, int64_t n_expert,
+                          int64_t top_k, int dtype, void *workspace,
+                          int64_t workspace_bytes, void *stream);
+
+/* out[t,:] = sum_j rows[slot_to_row[t*top_k+j],:]
+ *          + sum_j grad_score[t,j] * w[topk_idx[t,j],:]
+ * i.e. fmoe_reduce_slots and the gate's part of the input gradient in one pass,
+ * summed in fp32 and rounded once.  slot_to_row NULL: the gate's part alone.
+ * Same limits as fmoe_gate_weight_grad except that any n_expert is taken. */
+int fmoe_reduce_slots_gate(const void *rows, const int64_t *slot_to_row,
+                           const void *grad_score, const int64_t *topk_idx,
+                           const void *w, void *out, int64_t n_tokens,
+                           int64_t top_k, int64_t n_rows, int64_t n_expert,
+                           int64_t row_elems, int dtype, void *stream);
 
 /* Noisy top-k gating in training mode (Shazeer et al. 2017; the behaviour of
  * fmoe/gates/noisy_gate.py:113-144) after the two linear products, in one

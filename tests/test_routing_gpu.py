@@ -392,3 +392,65 @@ def test_naive_gate_uses_the_fused_linear_and_matches_the_unfused_one(device, mo
     # with all logits asked for, the gate runs the linear layer by itself
     idx3, val3, logits = gate(x, return_all_scores=True)
     assert logits.shape == (3000, 16) and torch.equal(idx3, results[1][0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,d,e,k", [
+    (1, 8, 1, 1),            # one token, one chunk, one expert
+    (31, 128, 4, 2),         # fewer tokens than a step takes, a whole column tile
+    (64, 136, 16, 2),        # a column over the tile, all experts of a block
+    (65, 120, 17, 4),        # a token over the step, an expert over the block
+    (1000, 520, 33, 8),
+    (4097, 256, 64, 1),      # several token ranges with a ragged last one
+    (2500, 384, 100, 2),
+    (3000, 1032, 256, 8),    # the most experts
+])
+def test_gate_grad_from_selected_scores(dtype, n, d, e, k, device):
+    """fmoe_gate_weight_grad and fmoe_reduce_slots_gate against the dense products in float64.  Allowed per
+    element: float32 sums (an ulp per term of the sum of absolute terms) and the rounding of the result."""
+    torch.manual_seed(n + d + e)
+    x, w = torch.randn(n, d).to(dtype), torch.randn(e, d).to(dtype)
+    g = torch.randn(n, k).to(dtype)
+    idx = torch.rand(n, e).topk(k, dim=1).indices
+    n_rows = max(1, (n * k * 3) // 4)
+    rows = torch.randn(n_rows, d).to(dtype)
+    s2r = torch.full((n * k,), -1, dtype=torch.int64)
+    s2r[torch.randperm(n * k)[:n_rows]] = torch.arange(n_rows)
+    out_eps = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -11}[dtype]
+    tiny = 2.0 ** -25 if dtype == torch.float16 else 0.0   # half of float16's smallest step
+
+    def near(got, want, mag, terms):
+        err = (got.double().cpu() - want).abs()
+        assert (err <= 2 * out_eps * want.abs() + terms * 2.0 ** -24 * mag + tiny).all(), float(err.max())
+
+    xd, wd, gd, idxd = (t.to(device) for t in (x, w, g, idx))
+    dense = torch.zeros(n, e, dtype=torch.float64).scatter_(1, idx, g.double())
+    grad_w, grad_b = fmoe_native.gate_weight_grad(gd, idxd, xd, e, True)
+    near(grad_w, dense.t() @ x.double(), dense.abs().t() @ x.double().abs(), n)
+    near(grad_b, dense.sum(0), dense.abs().sum(0), n)
+    again, none = fmoe_native.gate_weight_grad(gd, idxd, xd, e, False)
+    assert none is None and torch.equal(again, grad_w)
+    part, mag = dense @ w.double(), dense.abs() @ w.double().abs()
+    near(fmoe_native.reduce_slots_gate(None, None, gd, idxd, wd), part, mag, k + 1)
+    picked = torch.where((s2r >= 0).unsqueeze(1), rows.double()[s2r.clamp(min=0)], torch.zeros(1, dtype=torch.float64))
+    near(fmoe_native.reduce_slots_gate(rows.to(device), s2r.to(device), gd, idxd, wd), part + picked.view(n, k, d).sum(1),
+         mag + picked.abs().view(n, k, d).sum(1), 2 * k + 1)
+
+
+def test_naive_gate_of_many_experts_matches_the_dense_backward(device, monkeypatch):
+    """More experts than the fused linear takes: same choices, scores and gradients as with the linear layer apart."""
+    from fastermoe_amd.gates import NaiveGate
+    torch.manual_seed(5)
+    gate = NaiveGate(256, 200, 1, top_k=8).to(device)
+    x = torch.randn(1500, 256, device=device, requires_grad=True)
+    results = []
+    for flag in ("1", "0"):
+        monkeypatch.setenv("FMOE_GATE_LINEAR_FUSED", flag)
+        gate.zero_grad()
+        x.grad = None
+        idx, val = gate(x)
+        val.square().sum().backward()
+        results.append((idx, val, x.grad, gate.gate.weight.grad.clone(), gate.gate.bias.grad.clone()))
+    assert torch.equal(results[0][0], results[1][0])
+    for a, b in zip(results[0][1:], results[1][1:]):
+        assert torch.allclose(a, b, rtol=1e-4, atol=1e-4)
