@@ -1,9 +1,8 @@
-// Grouped GEMM over ragged expert segments for what the 16-byte-chunk kernel does not take
+// Grouped GEMM over ragged expert segments for what the 16-byte-chunk kernels do not take
 // (gfx950): double precision -- the float64 rows of the reference's test grid,
 // tests/test_numerical.py:84-94, cublasDgemm in cuda/utils/cublas_wrapper.h:46-93 -- on the fp64
-// matrix pipe (v_mfma_f64_16x16x4_f64), and the 16- and 32-bit types with feature sizes or
-// pointers off the 16-byte grid, converted to fp32 on the way into LDS and multiplied with
-// v_mfma_f32_16x16x4_f32.
+// matrix pipe (v_mfma_f64_16x16x4_f64), and float32 with feature sizes or pointers off the 16-byte
+// grid on v_mfma_f32_16x16x4_f32.  (16-bit types off that grid: gemm_unaligned.hip.)
 //
 // A workgroup of four waves (2 x 2) computes a 64 x 64 tile of C, 32 x 32 per wave (2 x 2 MFMA
 // blocks).  Slabs of 16 contraction elements go from memory through registers into LDS as
@@ -197,10 +196,8 @@ int launch_mfma_any(gemm::GemmParams &prm, int dtype, int product, int epilogue,
     switch (dtype) {
         case FMOE_F64: return launch_any_typed<double, double>(prm, product, epilogue, stream);
         case FMOE_F32: return launch_any_typed<float, float>(prm, product, epilogue, stream);
-        case FMOE_BF16: return launch_any_typed<__bf16, float>(prm, product, epilogue, stream);
-        case FMOE_F16: return launch_any_typed<_Float16, float>(prm, product, epilogue, stream);
     }
-    return fail(FMOE_EINVAL, "unknown dtype %d", dtype);
+    return fail(FMOE_EINVAL, "grouped GEMM: dtype %d is not a 32- or 64-bit float type", dtype);
 }
 
 }  // namespace fmoe

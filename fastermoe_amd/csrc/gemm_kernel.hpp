@@ -1329,8 +1329,9 @@ FMOE_DECLARE_MFMA(launch_mfma_f16_wgrad);
 FMOE_DECLARE_MFMA(launch_mfma_f32_fwd);
 FMOE_DECLARE_MFMA(launch_mfma_f32_dgrad);
 FMOE_DECLARE_MFMA(launch_mfma_f32_wgrad);
-// double precision, and any type with feature sizes or pointers off the 16-byte grid; all three products
-// (0 forward, 1 data gradient, 2 weight gradient): gemm_any.hip
+// Feature sizes or pointers off the 16-byte grid, all three products (0 forward, 1 data gradient, 2 weight gradient):
+// 16-bit types in gemm_unaligned.hip, 32-bit ones and double precision (whatever its sizes) in gemm_any.hip
+int launch_mfma_unaligned(gemm::GemmParams &prm, int dtype, int product, int epilogue, hipStream_t stream);
 int launch_mfma_any(gemm::GemmParams &prm, int dtype, int product, int epilogue, hipStream_t stream);
 
 }  // namespace fmoe

@@ -11,8 +11,8 @@
 //   wgrad    dW_e    = dY[seg]^T . X[seg]  contraction ragged (the segment)
 //
 // This file holds the host side: segment tables, launch plans per product and per
-// chunk and the stand-alone bias-gradient kernel that the any-shape kernel of gemm_any.hip (feature
-// sizes that are not a multiple of 16 bytes, fp64) needs.  The MFMA
+// chunk and the stand-alone bias-gradient kernel that the kernel of gemm_any.hip (fp64, and fp32 with feature
+// sizes that are not a multiple of 16 bytes) needs.  The MFMA
 // kernel itself (tiling, LDS layouts, software pipeline, epilogues) is in
 // gemm_kernel.hpp and is instantiated once per element type and product by
 // gemm_inst.hip.
@@ -135,6 +135,19 @@ TileShape pick_rows_tile_estimate(int64_t rows_cap, int64_t n_expert, int64_t n_
     return pick_tile((whole + std::min<int64_t>(n_expert, std::max<int64_t>(whole, 1)) / 2) * ceil_div(n_cols, 256));
 }
 
+// Row tiles of gemm_unaligned.hip, 64 or 128 rows high: the low ones where the high ones would leave part of the
+// chip idle (two workgroups fit a unit, so 512 tiles is one round).
+TileShape pick_unaligned_tile(const int64_t *counts, int64_t n_expert, int64_t row_lo, int64_t row_hi, int64_t n_cols) {
+    int64_t start = 0, row_tiles = 0;
+    for (int64_t e = 0; e < n_expert; ++e) {
+        const int64_t end = start + counts[e];
+        const int64_t lo = start < row_lo ? row_lo : start, hi = end > row_hi ? row_hi : end;
+        if (hi > lo) row_tiles += ceil_div(hi - lo, 128);
+        start = end;
+    }
+    return row_tiles * ceil_div(n_cols, 128) >= 512 ? TileShape{128, 128} : TileShape{64, 128};
+}
+
 // weight gradient: C is [out, in] per expert
 TileShape pick_wgrad_tile(int64_t n_experts_written, int64_t out_feat, int64_t in_feat) {
     return pick_tile(n_experts_written * ceil_div(out_feat, 256) * ceil_div(in_feat, 256));
@@ -221,9 +234,15 @@ std::mutex g_split_mutex;
 std::vector<SplitBuffer> g_split_buffers;
 int g_compute_units[16] = {};
 
+bool is_16bit(int dtype) { return dtype == FMOE_BF16 || dtype == FMOE_F16; }
+
 template <int PRODUCT>
 int dispatch(GemmParams &prm, int dtype, int epi, bool fast, hipStream_t stream) {
-    // double precision, and shapes off the 16-byte grid: the element-checked kernel of gemm_any.hip
+    // Shapes off the 16-byte grid: 16-bit types in gemm_unaligned.hip, the others and double precision on the
+    // element-checked kernel of gemm_any.hip.  bf16 on that one and on gemm_unaligned.hip, forward / data gradient /
+    // weight gradient: 1554 rows, 12 experts of 500 x 1302: 89 / 170 / 64 and 21 / 24 / 28 us; 16 rows, 8 experts of
+    // 1000 x 2001: 93 / 178 / 26 and 21 / 33 / 24; 8192 rows, 8 experts of 2047 x 4093: 3063 / 2800 / 2116 and 230 / 188 / 257.
+    if (!fast && is_16bit(dtype)) return launch_mfma_unaligned(prm, dtype, PRODUCT, epi, stream);
     if (!fast || dtype == FMOE_F64) return launch_mfma_any(prm, dtype, PRODUCT, epi, stream);
     switch (dtype * 3 + PRODUCT) {
         case FMOE_BF16 * 3 + kFwd: return launch_mfma_bf16_fwd(prm, epi, stream);
@@ -400,7 +419,8 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
     const bool fast = is_fast(a.dtype, {a.x, a.w, a.y, a.aux, a.bias}, {a.in_feat, a.out_feat});
     FMOE_REQUIRE(a.x_row_index == nullptr || linear_forward_can_gather(a),
                  "linear_forward: rows cannot be gathered in the loader for this shape");
-    const TileShape tile = pick_rows_tile(counts, n_expert, row_lo, row_hi, a.out_feat);
+    const TileShape tile = !fast && is_16bit(a.dtype) ? pick_unaligned_tile(counts, n_expert, row_lo, row_hi, a.out_feat)
+                                                      : pick_rows_tile(counts, n_expert, row_lo, row_hi, a.out_feat);
     for (int e0 = plan.first; e0 <= plan.last; e0 += kMaxGroupExperts) {
         const int e1 = std::min(plan.last, e0 + kMaxGroupExperts - 1);
         GemmParams prm{};
@@ -452,7 +472,8 @@ int grouped_linear_dgrad(const LinearDgradArgs &a, const int64_t *counts, int64_
     FMOE_REQUIRE(a.gy && a.w && a.gx, "linear_dgrad: NULL tensor");
     const Plan plan = plan_rows(counts, n_expert, row_lo, row_hi);
     const bool fast = is_fast(a.dtype, {a.gy, a.w, a.gx, a.aux}, {a.in_feat, a.out_feat});
-    const TileShape tile = pick_rows_tile(counts, n_expert, row_lo, row_hi, a.in_feat);
+    const TileShape tile = !fast && is_16bit(a.dtype) ? pick_unaligned_tile(counts, n_expert, row_lo, row_hi, a.in_feat)
+                                                      : pick_rows_tile(counts, n_expert, row_lo, row_hi, a.in_feat);
     for (int e0 = plan.first; e0 <= plan.last; e0 += kMaxGroupExperts) {
         const int e1 = std::min(plan.last, e0 + kMaxGroupExperts - 1);
         GemmParams prm{};
@@ -504,15 +525,15 @@ int grouped_linear_wgrad(const LinearWgradArgs &a, const int64_t *counts, int64_
         prm.block_m = tile.bm; prm.block_n = tile.bn;
         fill_table(&prm.tab, counts, e0, e1, row_lo, row_hi, tile.bm);
         prm.profile_class = kProfGemmWgrad; prm.profile_work = table_flop(prm.tab, a.in_feat, a.out_feat);
-        prm.P = a.x; prm.Q = a.gy; prm.C = a.gw; prm.bias_grad = fast ? a.gb : nullptr;
+        prm.P = a.x; prm.Q = a.gy; prm.C = a.gw; prm.bias_grad = fast || is_16bit(a.dtype) ? a.gb : nullptr;
         prm.ldp = a.in_feat; prm.ldq = a.out_feat; prm.ldc = a.in_feat;
         prm.c_expert_stride = a.in_feat * a.out_feat;
         prm.n_cols = (int)a.in_feat; prm.n_rows = (int)a.out_feat;
         prm.accumulate_first = (e0 == plan.first && plan.accumulate_first) ? 1 : 0;
         if (int rc = dispatch<kWgrad>(prm, a.dtype, kEpiStore, fast, stream)) return rc;
     }
-    // the MFMA kernel folds the bias gradient into its first column tiles; the any-shape path does not
-    if (a.gb && !fast)
+    // the 16- and 32-bit MFMA kernels fold the bias gradient into their first column tiles; gemm_any.hip does not
+    if (a.gb && !fast && !is_16bit(a.dtype))
         return grouped_bias_grad(a.gy, a.gb, a.out_feat, a.dtype, counts, n_expert, row_lo, row_hi, last_chunk, stream);
     return FMOE_OK;
 }
