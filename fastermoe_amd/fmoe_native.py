@@ -6,6 +6,7 @@ reference's ``exit()``), allocates outputs with torch, and enqueues the HIP
 kernels on torch's current stream through the C ABI.  Nothing here computes on
 the CPU and nothing falls back to torch operators.
 """
+import contextlib
 import ctypes
 
 import torch
@@ -17,12 +18,23 @@ _DTYPES = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _l
            torch.float64: _lib.F64}
 
 
+# A training step of the layer makes some 13 calls into the library, each with a stream, a device guard and half a
+# dozen pointers: plain integers (ctypes converts them to void *), the raw stream handle and a guard only
+# where the device differs cost 1 us a call where torch.cuda's objects cost 7.
 def _stream(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_CURRENT = contextlib.nullcontext()
+
+
+def _on(device):
+    """``torch.cuda.device(device)``; nothing where that device (a tensor's) is the current one already."""
+    return _CURRENT if device.index == torch._C._cuda_getDevice() else torch.cuda.device(device)
 
 
 def _dev(name, t, dtype=None):
@@ -73,7 +85,7 @@ def expert_count(gate_idx, expert_count):
     _dev("gate_idx", gate_idx, torch.int64)
     _dev("expert_count", expert_count, torch.int32)
     lib = _lib.load()
-    with torch.cuda.device(gate_idx.device):
+    with _on(gate_idx.device):
         check(lib.fmoe_expert_count(_ptr(gate_idx), _ptr(expert_count), gate_idx.numel(),
                                     expert_count.numel(), _stream(gate_idx)))
 
@@ -87,7 +99,7 @@ def assign_pos(cum_count, gate, pos):
     _dev("pos", pos, torch.int64)
     lib = _lib.load()
     n, e = gate.numel(), cum_count.numel()
-    with torch.cuda.device(gate.device):
+    with _on(gate.device):
         ws = _workspace(lib.fmoe_routing_workspace_bytes(n, e), gate.device)
         check(lib.fmoe_assign_pos(_ptr(cum_count), _ptr(gate), _ptr(pos), pos.numel(), n, e, _ptr(ws), ws.numel(),
                                   _stream(gate)))
@@ -112,7 +124,7 @@ def route_table(gate, n_expert, with_table=True):
     _dev("gate", gate, torch.int64)
     lib = _lib.load()
     n = gate.numel()
-    with torch.cuda.device(gate.device):
+    with _on(gate.device):
         cnt = torch.empty(n_expert, dtype=torch.int64, device=gate.device)
         pos = torch.empty(n, dtype=torch.int64, device=gate.device)
         s2r = torch.empty(n, dtype=torch.int64, device=gate.device)
@@ -144,7 +156,7 @@ def gate_topk_route(logits, top_k, score_mode=0, with_table=False):
     dt = _float_dtype("logits", logits)
     lib = _lib.load()
     dev = logits.device
-    with torch.cuda.device(dev):
+    with _on(dev):
         idx = torch.empty(n, top_k, dtype=torch.int64, device=dev)
         score = torch.empty(n, top_k, dtype=logits.dtype, device=dev)
         cnt = torch.empty(e, dtype=torch.int64, device=dev)
@@ -182,7 +194,7 @@ def gate_linear_topk_route(x, weight, bias, top_k, score_mode=0, with_table=Fals
         raise ValueError(f"gate_linear_topk_route does not take d_model={d}, n_expert={e}, top_k={top_k}, dtype={x.dtype}")
     lib = _lib.load()
     dev = x.device
-    with torch.cuda.device(dev):
+    with _on(dev):
         idx = torch.empty(n, top_k, dtype=torch.int64, device=dev)
         score = torch.empty(n, top_k, dtype=x.dtype, device=dev)
         cnt = torch.empty(e, dtype=torch.int64, device=dev)
@@ -216,7 +228,7 @@ def noisy_gate_forward(clean, raw, noise, top_k, eps):
     lib = _lib.load()
     dev = clean.device
     n_blocks = max(1, -(-n * top_k // 2048))
-    with torch.cuda.device(dev):
+    with _on(dev):
         idx = torch.empty(n, top_k, dtype=torch.int64, device=dev)
         gates = torch.empty(n, top_k, dtype=clean.dtype, device=dev)
         thr_val = torch.empty(n, 2, dtype=torch.float32, device=dev)
@@ -240,7 +252,7 @@ def noisy_gate_backward(clean, raw, noise, top_k, eps, topk_idx, gates, thr_val,
     _dev("grad_load", grad_load, torch.float32)
     n, e = clean.shape
     grad_clean, grad_raw = torch.empty_like(clean), torch.empty_like(clean)
-    with torch.cuda.device(clean.device):
+    with _on(clean.device):
         check(_lib.load().fmoe_noisy_gate_backward(_ptr(clean), _ptr(raw), _ptr(noise), float(eps), n, e, top_k, dt,
                                                    _ptr(topk_idx), _ptr(gates), _ptr(thr_val), _ptr(thr_idx),
                                                    _ptr(grad_gates), _ptr(grad_load), _ptr(grad_clean), _ptr(grad_raw),
@@ -257,7 +269,7 @@ def gate_topk_backward(grad_score, score, topk_idx, n_expert, score_mode=0):
     if score_mode == 1:
         _dev("score", score, grad_score.dtype)
     grad_logits = torch.empty(n, n_expert, dtype=grad_score.dtype, device=grad_score.device)
-    with torch.cuda.device(grad_score.device):
+    with _on(grad_score.device):
         check(_lib.load().fmoe_gate_topk_backward(_ptr(grad_score), _ptr(score if score_mode == 1 else None),
                                                   _ptr(topk_idx), _ptr(grad_logits), n, n_expert, k, dt, score_mode,
                                                   _stream(grad_score)))
@@ -285,7 +297,7 @@ def gate_weight_grad(grad_score, topk_idx, x, n_expert, with_bias):
     grad_b = torch.empty(n_expert, dtype=x.dtype, device=x.device) if with_bias else None
     if n == 0:
         return grad_w.zero_(), grad_b.zero_() if with_bias else None
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         ws = _workspace(lib.fmoe_gate_weight_grad_workspace_bytes(n, d, n_expert), x.device)
         check(lib.fmoe_gate_weight_grad(_ptr(grad_score), _ptr(topk_idx), _ptr(x), _ptr(grad_w), _ptr(grad_b), n, d, n_expert, k,
                                         dt, _ptr(ws), ws.numel(), _stream(x)))
@@ -308,7 +320,7 @@ def reduce_slots_gate(inp, slot_to_row, grad_score, topk_idx, weight):
         if inp.dtype != weight.dtype or inp.shape[1] != d or slot_to_row.numel() != n * k:
             raise ValueError("inp must be rows like weight's, slot_to_row must have one entry per slot")
     out = torch.empty(n, d, dtype=weight.dtype, device=weight.device)
-    with torch.cuda.device(weight.device):
+    with _on(weight.device):
         check(_lib.load().fmoe_reduce_slots_gate(_ptr(inp), _ptr(slot_to_row if inp is not None else None), _ptr(grad_score),
                                                  _ptr(topk_idx), _ptr(weight), _ptr(out), n, k, 0 if inp is None else inp.shape[0],
                                                  e, d, dt, _stream(weight)))
@@ -325,7 +337,7 @@ def limit_by_capacity(expert_count, capacity, n_expert, n_worker):
         raise ValueError("capacity must have n_expert entries")
     lib = _lib.load()
     out = torch.empty_like(expert_count)
-    with torch.cuda.device(expert_count.device):
+    with _on(expert_count.device):
         check(lib.fmoe_limit_by_capacity(_ptr(expert_count), _ptr(capacity), _ptr(out), n_expert, n_worker,
                                          _stream(expert_count)))
     return out
@@ -340,7 +352,7 @@ def prune_gate_by_capacity(gate_idx, expert_count, n_expert, n_worker):
     lib = _lib.load()
     out = torch.empty_like(gate_idx)
     n, e = gate_idx.numel(), expert_count.numel()
-    with torch.cuda.device(gate_idx.device):
+    with _on(gate_idx.device):
         ws = _workspace(lib.fmoe_routing_workspace_bytes(n, e), gate_idx.device)
         check(lib.fmoe_prune_gate_by_capacity(_ptr(gate_idx), _ptr(out), _ptr(expert_count), n, e, _ptr(ws),
                                               ws.numel(), _stream(gate_idx)))
@@ -362,7 +374,7 @@ def gather_rows(inp, index, n_out=None, index_div=1):
     _dev("index", index, torch.int64)
     n_out = index.numel() if n_out is None else n_out
     out = torch.empty(n_out, inp.shape[1], dtype=inp.dtype, device=inp.device)
-    with torch.cuda.device(inp.device):
+    with _on(inp.device):
         if index_div == 1:
             check(_lib.load().fmoe_gather_rows(_ptr(inp), _ptr(index), _ptr(out), n_out, inp.shape[0], inp.shape[1],
                                                dt, _stream(inp)))
@@ -376,7 +388,7 @@ def invert_index(pos, n_out):
     """inverse[pos[i]] = i, -1 elsewhere."""
     _dev("pos", pos, torch.int64)
     inv = torch.empty(n_out, dtype=torch.int64, device=pos.device)
-    with torch.cuda.device(pos.device):
+    with _on(pos.device):
         check(_lib.load().fmoe_invert_index(_ptr(pos), pos.numel(), _ptr(inv), n_out, _stream(pos)))
     return inv
 
@@ -388,7 +400,7 @@ def reduce_slots(inp, slot_to_row, n_tokens, top_k):
     if slot_to_row.numel() != n_tokens * top_k:
         raise ValueError("slot_to_row must have n_tokens * top_k entries")
     out = torch.empty(n_tokens, inp.shape[1], dtype=inp.dtype, device=inp.device)
-    with torch.cuda.device(inp.device):
+    with _on(inp.device):
         check(_lib.load().fmoe_reduce_slots(_ptr(inp), _ptr(slot_to_row), _ptr(out), n_tokens, top_k,
                                             inp.shape[0], inp.shape[1], dt, _stream(inp)))
     return out
@@ -402,7 +414,7 @@ def index_add_rows(inp, index, n_out):
         raise ValueError("index must have one entry per row of inp")
     lib = _lib.load()
     out = torch.empty(n_out, inp.shape[1], dtype=inp.dtype, device=inp.device)
-    with torch.cuda.device(inp.device):
+    with _on(inp.device):
         ws = _workspace(lib.fmoe_index_add_workspace_bytes(inp.shape[0], n_out), inp.device)
         check(lib.fmoe_index_add_rows(_ptr(inp), _ptr(index), _ptr(out), inp.shape[0], n_out, inp.shape[1], dt,
                                       _ptr(ws), ws.numel(), _stream(inp)))
@@ -422,7 +434,7 @@ def mask_restore(src, token_to_row, scale, fill, fill_row, n_tokens):
         if scale is not None:
             _dev("scale", scale, src.dtype)
     out = torch.empty(n_tokens, src.shape[1], dtype=src.dtype, device=src.device)
-    with torch.cuda.device(src.device):
+    with _on(src.device):
         check(_lib.load().fmoe_mask_restore(_ptr(src), _ptr(token_to_row), _ptr(scale if fill is not None else None),
                                             _ptr(fill), _ptr(fill_row if fill is not None else None), _ptr(out),
                                             n_tokens, src.shape[0], n_fill, src.shape[1], dt, _stream(src)))
@@ -434,7 +446,7 @@ def mask_scale_grad(grad_out, token_to_row, fill, fill_row):
     dt = _rows("grad_out", grad_out)
     _dev("fill", fill, grad_out.dtype)
     grad_scale = torch.empty(grad_out.shape[0], dtype=grad_out.dtype, device=grad_out.device)
-    with torch.cuda.device(grad_out.device):
+    with _on(grad_out.device):
         check(_lib.load().fmoe_mask_scale_grad(_ptr(grad_out), _ptr(token_to_row), _ptr(fill), _ptr(fill_row),
                                                _ptr(grad_scale), grad_out.shape[0], fill.shape[0], grad_out.shape[1],
                                                dt, _stream(grad_out)))
@@ -450,7 +462,7 @@ def combine_forward(x, score, n_tokens, top_k):
     if x.shape[0] != n_tokens * top_k or score.numel() != n_tokens * top_k:
         raise ValueError("x must have n_tokens*top_k rows and score n_tokens*top_k entries")
     out = torch.empty(n_tokens, x.shape[1], dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         check(_lib.load().fmoe_combine_forward(_ptr(x), _ptr(score), _ptr(out), n_tokens, top_k, x.shape[1], dt,
                                                _stream(x)))
     return out
@@ -465,7 +477,7 @@ def combine_backward(grad_out, x, score, n_tokens, top_k):
         raise ValueError(f"grad_out must be [{n_tokens}, {x.shape[1]}]")
     grad_x = torch.empty_like(x)
     grad_score = torch.empty(n_tokens, top_k, dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         check(_lib.load().fmoe_combine_backward(_ptr(grad_out), _ptr(x), _ptr(score), _ptr(grad_x), _ptr(grad_score),
                                                 n_tokens, top_k, x.shape[1], dt, _stream(x)))
     return grad_x, grad_score
@@ -480,7 +492,7 @@ def gather_combine_forward(rows, slot_to_row, score, n_tokens, top_k):
     if slot_to_row.numel() != n_tokens * top_k or score.numel() != n_tokens * top_k:
         raise ValueError("slot_to_row and score must have n_tokens*top_k entries")
     out = torch.empty(n_tokens, rows.shape[1], dtype=rows.dtype, device=rows.device)
-    with torch.cuda.device(rows.device):
+    with _on(rows.device):
         check(_lib.load().fmoe_gather_combine_forward(_ptr(rows), _ptr(slot_to_row), _ptr(score), _ptr(out), n_tokens,
                                                       top_k, rows.shape[0], rows.shape[1], dt, _stream(rows)))
     return out
@@ -498,7 +510,7 @@ def gather_combine_backward(grad_out, rows, slot_to_row, score, n_tokens, top_k)
         raise ValueError("slot_to_row and score must have n_tokens*top_k entries")
     grad_rows = torch.empty_like(rows)
     grad_score = torch.empty(n_tokens, top_k, dtype=rows.dtype, device=rows.device)
-    with torch.cuda.device(rows.device):
+    with _on(rows.device):
         check(_lib.load().fmoe_gather_combine_backward(_ptr(grad_out), _ptr(rows), _ptr(slot_to_row), _ptr(score),
                                                        _ptr(grad_rows), _ptr(grad_score), n_tokens, top_k,
                                                        rows.shape[0], rows.shape[1], dt, _stream(rows)))
@@ -539,7 +551,7 @@ def linear_forward(input_buf, expert_count, weight, bias=None):
     dt, n_expert, out_feat, in_feat = _check_linear(input_buf, expert_count, weight, bias)
     out = torch.empty(input_buf.shape[0], out_feat, dtype=input_buf.dtype, device=input_buf.device)
     cnt = _linear_counts(input_buf, expert_count, n_expert)
-    with torch.cuda.device(input_buf.device):
+    with _on(input_buf.device):
         check(_lib.load().fmoe_linear_forward(_ptr(input_buf), _ptr(weight), _ptr(bias), _ptr(out),
                                               ctypes.c_void_p(cnt.data_ptr()), n_expert, in_feat, out_feat, dt,
                                               _stream(input_buf)))
@@ -560,7 +572,7 @@ def linear_backward(grad_output_buf, input_buf, expert_count, weight, bias=None)
     grad_w = torch.empty_like(weight)
     grad_b = torch.empty(n_expert, out_feat, dtype=input_buf.dtype, device=input_buf.device) \
         if bias is not None else None
-    with torch.cuda.device(input_buf.device):
+    with _on(input_buf.device):
         check(_lib.load().fmoe_linear_backward(_ptr(grad_output_buf), _ptr(input_buf), _ptr(weight), _ptr(grad_in),
                                                _ptr(grad_w), _ptr(grad_b), ctypes.c_void_p(cnt.data_ptr()),
                                                n_expert, in_feat, out_feat, dt, _stream(input_buf)))
@@ -578,7 +590,7 @@ def linear_act_forward(input_buf, expert_count, weight, bias, activation, keep_p
     y = new()
     pre = new() if keep_pre else None
     cnt = _linear_counts(input_buf, expert_count, n_expert)
-    with torch.cuda.device(input_buf.device):
+    with _on(input_buf.device):
         check(_lib.load().fmoe_linear_act_forward(_ptr(input_buf), _ptr(weight), _ptr(bias), _ptr(pre), _ptr(y),
                                                   ctypes.c_void_p(cnt.data_ptr()), n_expert, in_feat, out_feat, dt,
                                                   activation, _stream(input_buf)))
@@ -604,7 +616,7 @@ def linear_dact_backward(grad_output_buf, expert_count, weight, pre, activation)
         if tuple(pre.shape) != (grad_output_buf.shape[0], in_feat):
             raise ValueError(f"pre must be [{grad_output_buf.shape[0]}, {in_feat}]")
     grad_x = torch.empty(grad_output_buf.shape[0], in_feat, dtype=grad_output_buf.dtype, device=grad_output_buf.device)
-    with torch.cuda.device(grad_output_buf.device):
+    with _on(grad_output_buf.device):
         check(_lib.load().fmoe_linear_dact_backward(_ptr(grad_output_buf), _ptr(weight),
                                                     _ptr(pre if activation != _lib.ACT_NONE else None), _ptr(grad_x),
                                                     ctypes.c_void_p(cnt.data_ptr()), n_expert, in_feat, out_feat, dt,
@@ -622,7 +634,7 @@ def linear_weight_backward(grad_output_buf, input_buf, expert_count, weight, bia
     grad_w = torch.empty_like(weight)
     grad_b = torch.empty(n_expert, out_feat, dtype=input_buf.dtype, device=input_buf.device) \
         if bias is not None else None
-    with torch.cuda.device(input_buf.device):
+    with _on(input_buf.device):
         check(_lib.load().fmoe_linear_backward(_ptr(grad_output_buf), _ptr(input_buf), _ptr(weight), None,
                                                _ptr(grad_w), _ptr(grad_b), ctypes.c_void_p(cnt.data_ptr()),
                                                n_expert, in_feat, out_feat, dt, _stream(input_buf)))
@@ -639,7 +651,7 @@ def segment_table(expert_count, rows_cap):
     lib = _lib.load()
     n_expert = expert_count.numel()
     nbytes = lib.fmoe_segment_table_bytes(int(rows_cap), n_expert)
-    with torch.cuda.device(expert_count.device):
+    with _on(expert_count.device):
         table = torch.empty(nbytes // 4, dtype=torch.int32, device=expert_count.device)
         check(lib.fmoe_segment_table_build(_ptr(expert_count), n_expert, int(rows_cap), _ptr(table), nbytes,
                                            _stream(expert_count)))
@@ -699,7 +711,7 @@ def linear_forward_dev(x, weight, bias, table, rows_cap, activation=_lib.ACT_NON
     new = lambda: torch.empty(rows_cap, out_feat, dtype=x.dtype, device=x.device)
     y = new()
     pre = new() if keep_pre else None
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         ws = _dev_workspace(in_feat, dt, x.device)
         check(_lib.load().fmoe_linear_forward_dev(_ptr(x), _ptr(row_index), int(index_div), x.shape[0], _ptr(weight),
                                                   _ptr(bias), _ptr(pre), _ptr(y), _ptr(table), n_expert, int(rows_cap),
@@ -724,7 +736,7 @@ def linear_dgrad_dev(grad_y, weight, table, rows_cap, pre=None, activation=_lib.
         if pre.dim() != 2 or pre.shape[0] < rows_cap or pre.shape[1] != in_feat:
             raise ValueError(f"pre must be [>= {rows_cap}, {in_feat}]")
     grad_x = torch.empty(rows_cap, in_feat, dtype=grad_y.dtype, device=grad_y.device)
-    with torch.cuda.device(grad_y.device):
+    with _on(grad_y.device):
         ws = _dev_workspace(out_feat, dt, grad_y.device)
         check(_lib.load().fmoe_linear_dgrad_dev(_ptr(grad_y), _ptr(weight),
                                                 _ptr(pre if activation != _lib.ACT_NONE else None), _ptr(grad_x),
@@ -744,7 +756,7 @@ def linear_wgrad_dev(grad_y, x, weight, table, rows_cap, with_bias):
     _check_table(table, n_expert, rows_cap)
     grad_w = torch.empty(n_expert, out_feat, in_feat, dtype=x.dtype, device=x.device)
     grad_b = torch.empty(n_expert, out_feat, dtype=x.dtype, device=x.device) if with_bias else None
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         check(_lib.load().fmoe_linear_wgrad_dev(_ptr(grad_y), _ptr(x), _ptr(grad_w), _ptr(grad_b), _ptr(table), n_expert,
                                                 int(rows_cap), in_feat, out_feat, dt, _stream(x)))
     return grad_w, grad_b
@@ -807,7 +819,7 @@ def fused_mlp_forward(inp, pos, slot_to_row, expert_count, w1, b1, w2, b2, top_k
     n_rows = int(cnt.sum())
     if n_rows > cap:
         raise ValueError(f"expert_count sums to {n_rows} but pos has {cap} entries")
-    with torch.cuda.device(inp.device):
+    with _on(inp.device):
         check(lib.fmoe_fused_mlp_forward(
             ctypes.byref(prm), _ptr(inp), _ptr(pos), _ptr(slot_to_row), ctypes.c_void_p(cnt.data_ptr()),
             n_tokens, top_k, n_rows, _ptr(buf_in), _ptr(buf_pre), _ptr(buf_mid), _ptr(buf_out), _ptr(out),
@@ -847,7 +859,7 @@ def fused_mlp_backward(grad_out, pos, slot_to_row, expert_count, w1, b1, w2, b2,
     grad_w1, grad_w2 = torch.empty_like(w1), torch.empty_like(w2)
     grad_b1 = torch.empty_like(b1) if b1 is not None else None
     grad_b2 = torch.empty_like(b2) if b2 is not None else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         check(_lib.load().fmoe_fused_mlp_backward(
             ctypes.byref(prm), _ptr(grad_out if slot_order else None), _ptr(pos), _ptr(slot_to_row),
             ctypes.c_void_p(cnt.data_ptr()),
