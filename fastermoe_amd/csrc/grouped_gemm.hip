@@ -17,6 +17,7 @@
 // gemm_kernel.hpp and is instantiated once per element type and product by
 // gemm_inst.hip.
 #include "gemm_ring.hpp"
+#include "gemm_skinny.hpp"
 #include "profile.hpp"
 
 #include <algorithm>
@@ -266,6 +267,18 @@ bool use_ring(const TileShape &tile, int dtype) {
     return tile.bm == 256 && tile.bn == 256 && (dtype == FMOE_BF16 || dtype == FMOE_F16) && !getenv("FMOE_GEMM_TILE");
 }
 
+// Whether a forward launch over a device table goes to gemm_skinny.hip: 16-bit types (no tile shape forced) and at
+// most two rows per expert on average, or eight where the weights make less than two rounds of 128 x 128 tiles (512 at
+// a time), whose last round is then badly filled.  Above that the rows' way from L2 into every 16 columns costs more than
+// the tiles' padding.  bf16, us on the tiles and here: 32 experts of 4096 x 1024, 2 / 32 / 256 rows: 26.7 / 57.4 / 69.9
+// and 13.8 / 36.3 / 55.5; 8 of 4096 x 14336, 8 / 32 / 64 / 128: 142 / 191 / 191 / 192 and 99 / 161 / 180 / 243; 256 of
+// 1024 x 2048, 256 / 512 / 1024: 134 / 179 / 205 and 124 / 170 / 210; 64 of 8192 x 2048, 64 / 128 / 256: 298 / 367 / 372
+// and 249 / 334 / 389.
+bool use_skinny(int64_t rows_cap, int64_t n_expert, int64_t out_feat, int dtype) {
+    if (!is_16bit(dtype) || getenv("FMOE_GEMM_TILE")) return false;
+    return rows_cap <= 2 * n_expert || (rows_cap <= 8 * n_expert && n_expert * ceil_div(out_feat, 128) < 1024);
+}
+
 template <int PRODUCT>
 int dispatch_ring(const GemmParams &g, int dtype, int epi, hipStream_t stream) {
     RingParams prm{};
@@ -403,6 +416,18 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
         const int64_t ws_need = linear_dev_workspace_bytes(a.in_feat, a.dtype);
         if (a.dev_workspace != nullptr && ws_need > 0 && a.dev_workspace_bytes >= ws_need && aligned16(a.dev_workspace))
             prm.dev_split_ws = (float *)a.dev_workspace;
+        if (use_skinny(a.dev_rows_cap, n_expert, a.out_feat, a.dtype)) {
+            SkinnyParams sk{};
+            sk.w = a.w; sk.x = a.x; sk.bias = a.bias; sk.y = a.y; sk.aux = a.aux;
+            sk.dev_tab = a.dev_tab;
+            sk.row_index = a.x_row_index; sk.x_total_rows = a.x_total_rows;
+            sk.div_mul = prm.q_div_mul; sk.div_shift = prm.q_div_shift;
+            sk.n_cols = prm.n_cols; sk.k_extent = prm.k_extent; sk.activation = prm.activation;
+            sk.tiles_n = (int)ceil_div(a.out_feat, kSkinnyCols);
+            sk.map_off = (int32_t)segtab::map128_off(a.dev_rows_cap, n_expert);
+            ProfileScope prof(prm.profile_class, prm.profile_work, stream);
+            return launch_skinny(sk, a.dtype, segtab::cap_tiles(a.dev_rows_cap, n_expert, 128), stream);
+        }
         // (what the persistent kernel is built for; the erf formula, "none" and ReLU with a saved pre-activation are rare)
         const bool ring_act = a.epilogue == kEpiStore || prm.activation == FMOE_ACT_GELU ||
                               (prm.activation == FMOE_ACT_RELU && a.aux == nullptr);

@@ -306,3 +306,44 @@ def test_persistent_kernel_products(case, dtype, device):
         close(gx_relu[r], back * (ps > 0), f"expert {ex}: relu derivative")
         close(gw[ex], gs.t() @ xs, f"expert {ex}: weight gradient")
         close(gb[ex], gs.sum(dim=0), f"expert {ex}: bias gradient")
+
+
+FEW_ROWS = [  # counts, contraction, columns: one to four blocks of 16 rows and more than 64 rows for an expert; contractions
+    # of one chunk, off the 32 elements of a product and the 128 of a unit, and of several units per wave
+    ([1], 8, 8),
+    ([2, 0, 1, 0, 0], 40, 24),
+    ([16, 0, 0, 17, 1, 15, 0], 136, 72),
+    ([33, 0, 0, 0, 0, 0], 96, 40),
+    ([0, 64, 0, 1, 0, 0, 0, 0, 0, 3], 1032, 264),
+    ([130, 0, 65, 0, 1] + [0] * 40, 520, 48),
+    ([1, 3] * 20, 2056, 136),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", range(len(FEW_ROWS)))
+def test_few_rows_per_expert(case, dtype, device):
+    """The forward product of decoding steps, over sorted rows and over rows read through an index (some of whose slots
+    are dropped), against the float64 oracle with the suite's tolerance of 16-bit types."""
+    counts, fin, fout = FEW_ROWS[case]
+    g = torch.Generator().manual_seed(case)
+    cnt, e, rows, k = torch.tensor(counts), len(counts), sum(counts), 3
+    slots = min(rows + 2, 8 * e)
+    table = fmoe_native.segment_table(cnt.to(device), slots)
+    tokens = torch.randn(rows, fin, generator=g).to(dtype)
+    w = (torch.randn(e, fout, fin, generator=g) / fin ** 0.5).to(dtype)
+    b = torch.randn(e, fout, generator=g).to(dtype)
+    index = torch.full((slots,), -1, dtype=torch.int64)
+    index[:rows] = torch.randint(0, rows * k, (rows,), generator=g)
+    tol = TOL[dtype]
+    for row_index in (None, index):
+        x = tokens if row_index is None else tokens[row_index[:rows] // k]
+        ref = omoe.per_expert_linear(x.double(), cnt, w.double(), b.double())
+        xd = tokens if row_index is not None else torch.cat([tokens, tokens.new_zeros(slots - rows, fin)])
+        args = dict(row_index=None if row_index is None else row_index.to(device), index_div=1 if row_index is None else k)
+        y, pre = fmoe_native.linear_forward_dev(xd.to(device), w.to(device), b.to(device), table, slots, _lib.ACT_GELU, True, **args)
+        assert rel_err(pre[:rows], ref) <= tol and rel_err(y[:rows], torch.nn.functional.gelu(ref)) <= tol
+        y, none = fmoe_native.linear_forward_dev(xd.to(device), w.to(device), b.to(device), table, slots, _lib.ACT_RELU, False, **args)
+        assert none is None and rel_err(y[:rows], ref.relu()) <= tol
+        y, _ = fmoe_native.linear_forward_dev(xd.to(device), w.to(device), None, table, slots, **args)
+        assert rel_err(y[:rows], omoe.per_expert_linear(x.double(), cnt, w.double(), None)) <= tol
