@@ -25,9 +25,11 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // wave of a SIMD sits at the barrier or waits for LDS; the workgroup takes the whole LDS of a
 // compute unit.  Tiles of 128 x 128: 2 x 2 (256 threads, 64 x 64 per wave) and half the LDS, so two
 // workgroups share a compute unit and one's first loads and epilogue run under the other's main
-// loop -- for launches whose tiles are short (few slabs) or few.
+// loop -- for launches whose tiles are short (few slabs) or few.  fp32 also comes in 64 x 64 (2 x 2 waves of one
+// 32 x 32 block, four workgroups per compute unit): its MFMA takes 256 cycles for what two 16-byte LDS reads
+// bring, so that the lower tile costs nothing and a launch of a few hundred tiles spreads evenly.
 constexpr int kWavesN = 2;
-constexpr int waves_m_of(int bn) { return bn == 128 ? 2 : 4; }
+constexpr int waves_m_of(int bn) { return bn <= 128 ? 2 : 4; }
 constexpr int threads_of(int bn) { return 64 * waves_m_of(bn) * kWavesN; }
 constexpr int kThreads = threads_of(256);  // workgroup size of the stand-alone bias-gradient kernel
 // The first kLoadWaves waves of a workgroup request the slabs.  The SIMD issues from its
@@ -321,7 +323,7 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
             int L;
             int main_tiles = prm.main_tiles, total_tiles = prm.total_tiles;
             if (dev) {
-                tm_total = dtab[BM == 256 ? segtab::kTiles256 : segtab::kTiles128];
+                tm_total = BM == 256 ? dtab[segtab::kTiles256] : dtab[segtab::kTiles128] * (128 / BM);
                 main_tiles = total_tiles = tm_total * prm.tiles_n;
                 if (prm.dev_cus > 0) {
                     const TailSplit ts = plan_tail_split(total_tiles, (prm.k_extent + BKE - 1) / BKE, prm.dev_cus, slab_weight_of<T>());
@@ -373,10 +375,17 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
                 // (the map's offset is known to the host, so this load waits for the tile count only)
                 typedef int i32x4 __attribute__((ext_vector_type(4)));
                 typedef const i32x4 __attribute__((address_space(4))) *DevTab4;
-                const i32x4 entry = *(DevTab4)(dtab + prm.dev_map_off + 4 * mt);
+                // (tiles of 64 rows: the halves of the map's 128; the second may have no rows)
+                constexpr int kPerEntry = BM == 64 ? 2 : 1;
+                const i32x4 entry = *(DevTab4)(dtab + prm.dev_map_off + 4 * (mt / kPerEntry));
                 ei = entry[0];
                 seg_lo = entry[1];
                 seg_hi = seg_lo + entry[2];
+                if constexpr (kPerEntry == 2) {
+                    seg_lo += (mt & 1) * BM;
+                    seg_hi = min(seg_hi, seg_lo + BM);
+                    if (seg_hi <= seg_lo) return;
+                }
             } else {
                 int lo = 0, hi = prm.tab.n;  // tile[lo] <= mt < tile[hi]
                 while (hi - lo > 1) {
@@ -882,8 +891,8 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
         if (fixup) {
             // the parts have been added up into part 0 by split_reduce_kernel; loads go out eight at a time
             const f32x4 *src = (const f32x4 *)prm.split_ws + (int64_t)tail_index * k_split * kTileVecs + wave * 64 + lane;
-            constexpr int kVecs = TI * TJ * kVecPerBlk, kBatch = 8;
-            static_assert(kVecs % kBatch == 0, "accumulator vectors are loaded in batches of eight");
+            constexpr int kVecs = TI * TJ * kVecPerBlk, kBatch = kVecs < 8 ? kVecs : 8;
+            static_assert(kVecs % kBatch == 0, "accumulator vectors are loaded in whole batches");
 #pragma unroll
             for (int j0 = 0; j0 < kVecs; j0 += kBatch) {
                 f32x4 val[kBatch];
@@ -1222,14 +1231,14 @@ int launch_tiles(GemmParams &prm, hipStream_t stream) {
             // the host does not know the tile count: with a workspace from the caller, every workgroup plans the
             // split itself, and the launch is sized for the most parts there can be (one per compute unit)
             prm.dev_cus = 0;
-            if (prm.dev_split_ws != nullptr && tail_split_possible(n_slabs, kWeight)) {
+            if (BM != 64 && prm.dev_split_ws != nullptr && tail_split_possible(n_slabs, kWeight)) {
                 prm.dev_cus = device_compute_units();
                 prm.split_ws = prm.dev_split_ws;
             }
             grid64 = ((int64_t)prm.total_tiles + 7) / 8 * 8 + prm.dev_cus;
         } else {
             const TailSplit ts = plan_tail_split(prm.total_tiles, n_slabs, device_compute_units(), kWeight);
-            if (ts.k_split > 1) {
+            if (BM != 64 && ts.k_split > 1) {
                 const int tail = prm.total_tiles - ts.main_tiles;
                 float *ws = split_workspace(stream, (size_t)tail * ts.k_split * BM * BN * sizeof(float));
                 if (ws != nullptr) {
@@ -1280,7 +1289,7 @@ int launch_tiles(GemmParams &prm, hipStream_t stream) {
 }
 
 // Tile counts, then the launch for the requested epilogue.  prm.block_m x prm.block_n (256 x 256,
-// 128 x 256 or 128 x 128, chosen by the host from the segment lengths) is the tile.
+// 128 x 256, 128 x 128 or, fp32 alone, 64 x 64, chosen by the host from the segment lengths) is the tile.
 // EPI_MASK lists the epilogues a product can be asked for, so that only those kernels
 // are built.
 template <typename T, int BM, int BN, int PS, int QS, int RG, int EPI_MASK>
@@ -1290,7 +1299,9 @@ int launch_for_height(GemmParams &prm, int epi, hipStream_t stream) {
     if (RG == kRaggedRows) {
         prm.tiles_m = 0;
         // device table: the most row tiles its rows can make (the kernel drops the surplus workgroups)
-        total = (prm.dev_tab ? segtab::cap_tiles(prm.dev_rows_cap, prm.tab.n, BM) : (int64_t)prm.tab.tile[prm.tab.n]) * prm.tiles_n;
+        constexpr int kMapRows = BM == 256 ? 256 : 128;
+        total = (prm.dev_tab ? segtab::cap_tiles(prm.dev_rows_cap, prm.tab.n, kMapRows) * (kMapRows / BM)
+                             : (int64_t)prm.tab.tile[prm.tab.n]) * prm.tiles_n;
         if (prm.dev_tab)
             prm.dev_map_off = (int32_t)(BM == 256 ? segtab::map256_off(prm.tab.n) : segtab::map128_off(prm.dev_rows_cap, prm.tab.n));
     } else {
@@ -1310,6 +1321,8 @@ int launch_for_height(GemmParams &prm, int epi, hipStream_t stream) {
 
 template <typename T, int PS, int QS, int RG, int EPI_MASK>
 int launch_by_epilogue(GemmParams &prm, int epi, hipStream_t stream) {
+    if constexpr (sizeof(T) == 4)
+        if (prm.block_m == 64 && prm.block_n == 64) return launch_for_height<T, 64, 64, PS, QS, RG, EPI_MASK>(prm, epi, stream);
     if (prm.block_m == 128 && prm.block_n == 128) return launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK>(prm, epi, stream);
     if (prm.block_m == 128 && prm.block_n == 256) return launch_for_height<T, 128, 256, PS, QS, RG, EPI_MASK>(prm, epi, stream);
     if (prm.block_m == 256 && prm.block_n == 256) return launch_for_height<T, 256, 256, PS, QS, RG, EPI_MASK>(prm, epi, stream);

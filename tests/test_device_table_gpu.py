@@ -347,3 +347,33 @@ def test_few_rows_per_expert(case, dtype, device):
         assert none is None and rel_err(y[:rows], ref.relu()) <= tol
         y, _ = fmoe_native.linear_forward_dev(xd.to(device), w.to(device), None, table, slots, **args)
         assert rel_err(y[:rows], omoe.per_expert_linear(x.double(), cnt, w.double(), None)) <= tol
+
+
+@pytest.mark.parametrize("fin,fout", [(4, 8), (60, 68), (64, 132), (100, 260)])
+@pytest.mark.parametrize("counts", [[1], [63, 0, 64, 65], [127, 128, 129, 0], [192, 193, 1], [300, 0, 5]])
+def test_float32_tiles_of_64(counts, fin, fout, device, monkeypatch):
+    """float32 in 64 x 64 tiles, which take the halves of the table's 128-row tiles: every product over the device table
+    and over host counts, the same bits from both, against the float64 oracle."""
+    monkeypatch.setenv("FMOE_GEMM_TILE", "64x64")
+    g = torch.Generator().manual_seed(sum(counts) + fin)
+    cnt, e, rows = torch.tensor(counts), len(counts), sum(counts)
+    table = fmoe_native.segment_table(cnt.to(device), rows)
+    x, gy = torch.randn(rows, fin, generator=g), torch.randn(rows, fout, generator=g)
+    w, b = torch.randn(e, fout, fin, generator=g) / fin ** 0.5, torch.randn(e, fout, generator=g)
+    pre_in = torch.randn(rows, fin, generator=g)
+    x64, w64, b64 = (t.double().requires_grad_(True) for t in (x, w, b))
+    ref = omoe.per_expert_linear(x64, cnt, w64, b64)
+    ref.backward(gy.double())
+    xd, wd, bd, gyd, pd = (t.to(device) for t in (x, w, b, gy, pre_in))
+    y, pre = fmoe_native.linear_forward_dev(xd, wd, bd, table, rows, _lib.ACT_GELU, True)
+    y_h, pre_h = fmoe_native.linear_act_forward(xd, cnt, wd, bd, _lib.ACT_GELU)
+    gx = fmoe_native.linear_dgrad_dev(gyd, wd, table, rows)
+    gx_act = fmoe_native.linear_dgrad_dev(gyd, wd, table, rows, pd, _lib.ACT_RELU)
+    gw, gb = fmoe_native.linear_wgrad_dev(gyd, xd, wd, table, rows, True)
+    gx_h, gw_h, gb_h = fmoe_native.linear_backward(gyd, xd, cnt, wd, bd)
+    for got, host in ((y, y_h), (pre, pre_h), (gx, gx_h), (gw, gw_h), (gb, gb_h)):
+        assert torch.equal(got, host)
+    tol = TOL[torch.float32]
+    assert rel_err(pre, ref) <= tol and rel_err(y, torch.nn.functional.gelu(ref)) <= tol
+    assert rel_err(gx, x64.grad) <= tol and rel_err(gx_act, x64.grad * (pre_in > 0)) <= tol
+    assert rel_err(gw, w64.grad) <= tol and rel_err(gb, b64.grad) <= tol
