@@ -10,12 +10,14 @@
 #include "common.hpp"
 #include "profile.hpp"
 #include "vec16.hpp"
+#include "wave_piece.hpp"
 
 namespace fmoe {
 namespace {
 
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
+constexpr int kBwdWaveVecs = 128;   // longest row that one wave of the backward takes by itself
 // row of x that slot s reads or writes: s itself, or idx[s] (negative or beyond n_rows: none)
 __device__ __forceinline__ int64_t slot_row(const int64_t *idx, int64_t s, int64_t n_rows) {
     if (idx == nullptr) return s;
@@ -29,10 +31,9 @@ __global__ __launch_bounds__(kBlock) void combine_fwd_vec_kernel(
     const u32x4 *__restrict__ x, const int64_t *__restrict__ idx, int64_t n_rows, const T *__restrict__ score,
     u32x4 *__restrict__ out, int64_t n_tokens, int top_k, int row_vecs, int pieces_per_row) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int64_t piece = (int64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    const int64_t t = piece / pieces_per_row;
+    const int64_t piece = wave_piece(kWavesPerBlock), t = div_small(piece, pieces_per_row);
     if (t >= n_tokens) return;
-    const int v = (int)(piece % pieces_per_row) * kWave + lane;
+    const int v = (int)(piece - t * pieces_per_row) * kWave + lane;
     if (v >= row_vecs) return;
     float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int j0 = 0; j0 < top_k; j0 += 8) {
@@ -72,9 +73,108 @@ __global__ __launch_bounds__(kBlock) void combine_fwd_elem_kernel(
     }
 }
 
-// backward: one workgroup per token.  grad_x[t*k+j,:] = score[t,j] * grad_out[t,:];
-// grad_score[t,j] = <grad_out[t,:], x[t*k+j,:]>, reduced lane -> wave -> workgroup in a
-// fixed order.
+// Backward: grad_x[t*k+j,:] = score[t,j] * grad_out[t,:]; grad_score[t,j] = <grad_out[t,:], x[t*k+j,:]>.
+// WPT waves share a token (the four of a workgroup, or one where a row is no more than two vectors to each of its lanes: the sum
+// then stays in the wave), K slots at a time and P vectors of each in flight per lane.
+// Sums are reduced lane -> wave -> workgroup in a fixed order.
+// Bound by reading and writing every slot's row once.  One workgroup per token and one slot after the other were bound by the chain
+// of loads, sums and barriers instead (a token's 128 vectors kept half the workgroup busy): bf16, 16384 tokens of
+// 1024, top-2: 47 -> 28 us; 32768 of 512, top-4: 134 -> 52; 8192 of 2048, top-8: 118 -> 110 (5.2 TB/s); 32768 of 4096, top-2:
+// 199 -> 194 (7 TB/s, part of it from the caches).
+template <typename T, int K, int P, int WPT>
+__global__ __launch_bounds__(kBlock) void combine_bwd_vec_kernel(
+    const u32x4 *__restrict__ grad_out, const u32x4 *__restrict__ x, const int64_t *__restrict__ idx, int64_t n_rows,
+    const T *__restrict__ score, u32x4 *__restrict__ grad_x, T *__restrict__ grad_score, int64_t n_tokens, int top_k,
+    int row_vecs) {
+    __shared__ float scratch[kWavesPerBlock][K];
+    constexpr int kTokens = kWavesPerBlock / WPT;
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int64_t t = (int64_t)blockIdx.x * kTokens + wave / WPT;
+    if (WPT == 1 && t >= n_tokens) return;
+    for (int j0 = 0; j0 < top_k; j0 += K) {
+        int64_t row[K];
+        float w[K], dot[K];
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const bool has = j0 + j < top_k;
+            row[j] = has ? slot_row(idx, t * top_k + j0 + j, n_rows) : -1;
+            w[j] = has ? (float)score[t * top_k + j0 + j] : 0.f;
+            dot[j] = 0.f;
+        }
+        for (int v0 = (wave % WPT) * kWave + lane; v0 < row_vecs; v0 += P * WPT * kWave) {
+            u32x4 gv[P], xv[P][K];
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const int v = v0 + p * WPT * kWave;
+                const bool in = v < row_vecs;
+                gv[p] = in ? grad_out[t * row_vecs + v] : u32x4{0, 0, 0, 0};
+#pragma unroll
+                for (int j = 0; j < K; ++j)
+                    xv[p][j] = in && row[j] >= 0 ? __builtin_nontemporal_load(&x[row[j] * row_vecs + v]) : u32x4{0, 0, 0, 0};
+            }
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const int v = v0 + p * WPT * kWave;
+                float g[8];
+                Vec<T>::unpack(gv[p], g);
+#pragma unroll
+                for (int j = 0; j < K; ++j) {
+                    if (row[j] < 0) continue;
+                    float f[8], r[8];
+                    Vec<T>::unpack(xv[p][j], f);
+#pragma unroll
+                    for (int i = 0; i < Vec<T>::N; ++i) {
+                        dot[j] += g[i] * f[i];
+                        r[i] = w[j] * g[i];
+                    }
+                    if (v < row_vecs) __builtin_nontemporal_store(Vec<T>::pack(r), &grad_x[row[j] * row_vecs + v]);
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+#pragma unroll
+            for (int off = kWave / 2; off > 0; off >>= 1) dot[j] += __shfl_down(dot[j], off, kWave);
+        if (WPT > 1) {
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < K; ++j)
+                if (lane == 0) scratch[wave][j] = dot[j];
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                dot[j] = 0.f;
+#pragma unroll
+                for (int u = 0; u < WPT; ++u) dot[j] += scratch[u][j];
+            }
+        }
+        if (lane == 0 && wave % WPT == 0) {
+#pragma unroll
+            for (int j = 0; j < K; ++j)
+                if (j0 + j < top_k) grad_score[t * top_k + j0 + j] = (T)dot[j];
+        }
+    }
+}
+
+template <typename T, int K, int P>
+void launch_combine_bwd(const void *grad_out, const void *x, const int64_t *idx, int64_t n_rows, const void *score, void *grad_x,
+                        void *grad_score, int64_t n_tokens, int64_t top_k, int row_vecs, hipStream_t st) {
+    auto launch = [&](auto kernel, int64_t blocks) {
+        kernel<<<(int)blocks, kBlock, 0, st>>>((const u32x4 *)grad_out, (const u32x4 *)x, idx, n_rows, (const T *)score,
+                                               (u32x4 *)grad_x, (T *)grad_score, n_tokens, (int)top_k, row_vecs);
+    };
+    if (row_vecs <= kBwdWaveVecs) launch(combine_bwd_vec_kernel<T, K, P, 1>, ceil_div(n_tokens, kWavesPerBlock));
+    else launch(combine_bwd_vec_kernel<T, K, P, kWavesPerBlock>, n_tokens);
+}
+
+template <typename T>
+void combine_bwd_vec(const void *grad_out, const void *x, const int64_t *idx, int64_t n_rows, const void *score, void *grad_x,
+                     void *grad_score, int64_t n_tokens, int64_t top_k, int row_vecs, hipStream_t st) {
+    auto go = top_k == 1 ? launch_combine_bwd<T, 1, 1> : top_k == 2 ? launch_combine_bwd<T, 2, 2>
+              : top_k <= 4 ? launch_combine_bwd<T, 4, 2> : launch_combine_bwd<T, 8, 1>;
+    go(grad_out, x, idx, n_rows, score, grad_x, grad_score, n_tokens, top_k, row_vecs, st);
+}
+
 template <typename Acc>
 __device__ __forceinline__ Acc block_sum(Acc v, Acc *scratch) {
 #pragma unroll
@@ -87,34 +187,6 @@ __device__ __forceinline__ Acc block_sum(Acc v, Acc *scratch) {
 #pragma unroll
     for (int w = 0; w < kWavesPerBlock; ++w) s += scratch[w];
     return s;
-}
-
-template <typename T>
-__global__ __launch_bounds__(kBlock) void combine_bwd_vec_kernel(
-    const u32x4 *__restrict__ grad_out, const u32x4 *__restrict__ x, const int64_t *__restrict__ idx, int64_t n_rows,
-    const T *__restrict__ score, u32x4 *__restrict__ grad_x, T *__restrict__ grad_score, int top_k, int row_vecs) {
-    __shared__ float scratch[kWavesPerBlock];
-    const int64_t t = blockIdx.x;
-    for (int j = 0; j < top_k; ++j) {
-        const float w = (float)score[t * top_k + j];
-        const int64_t row = slot_row(idx, t * top_k + j, n_rows);  // uniform over the workgroup
-        float dot = 0.f;
-        if (row >= 0) {
-            for (int v = threadIdx.x; v < row_vecs; v += kBlock) {
-                float g[8], f[8], r[8];
-                Vec<T>::unpack(grad_out[t * row_vecs + v], g);
-                Vec<T>::unpack(__builtin_nontemporal_load(&x[row * row_vecs + v]), f);
-#pragma unroll
-                for (int i = 0; i < Vec<T>::N; ++i) {
-                    dot += g[i] * f[i];
-                    r[i] = w * g[i];
-                }
-                __builtin_nontemporal_store(Vec<T>::pack(r), &grad_x[row * row_vecs + v]);
-            }
-        }
-        const float total = block_sum<float>(dot, scratch);
-        if (threadIdx.x == 0) grad_score[t * top_k + j] = (T)total;
-    }
 }
 
 template <typename T, typename Acc>
@@ -200,7 +272,7 @@ int combine_backward_impl(const char *who, const void *grad_out, const void *x, 
     ProfileScope prof(kProfCombine, (double)(2 * top_k + 1) * n_tokens * row_elems * dtype_bytes(dtype), st);
     if (vec_ok({grad_out, x, grad_x}, row_elems, dtype)) {
         const int row_vecs = (int)(row_elems * dtype_bytes(dtype) / 16);
-#define FMOE_CB(T) combine_bwd_vec_kernel<T><<<(int)n_tokens, kBlock, 0, st>>>((const u32x4 *)grad_out, (const u32x4 *)x, idx, n_rows, (const T *)score, (u32x4 *)grad_x, (T *)grad_score, (int)top_k, row_vecs)
+#define FMOE_CB(T) combine_bwd_vec<T>(grad_out, x, idx, n_rows, score, grad_x, grad_score, n_tokens, top_k, row_vecs, st)
         if (dtype == FMOE_F32) FMOE_CB(float);
         else if (dtype == FMOE_BF16) FMOE_CB(__bf16);
         else FMOE_CB(_Float16);

@@ -10,6 +10,7 @@
 // and no floating-point atomics are used.
 #include "permute.hpp"
 #include "profile.hpp"
+#include "wave_piece.hpp"
 
 namespace fmoe {
 namespace {
@@ -27,12 +28,11 @@ __global__ __launch_bounds__(kBlock) void gather_rows_vec_kernel(
     const u32x4 *__restrict__ inp, const int64_t *__restrict__ index, int64_t divisor,
     u32x4 *__restrict__ out, int64_t n_out, int64_t n_inp, int row_vecs, int pieces_per_row) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int64_t piece = (int64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    const int64_t row = piece / pieces_per_row;
+    const int64_t piece = wave_piece(kWavesPerBlock), row = div_small(piece, pieces_per_row);
     if (row >= n_out) return;
-    const int v0 = (int)(piece % pieces_per_row) * kPieceVecs;
+    const int v0 = (int)(piece - row * pieces_per_row) * kPieceVecs;
     int64_t src = index[row];
-    const bool live = src >= 0 && (src = src / divisor) < n_inp;
+    const bool live = src >= 0 && (src = div_small(src, divisor)) < n_inp;
     u32x4 val[kVecPerLane];
 #pragma unroll
     for (int j = 0; j < kVecPerLane; ++j) {
@@ -64,10 +64,9 @@ __global__ __launch_bounds__(kBlock) void scatter_rows_vec_kernel(
     const u32x4 *__restrict__ inp, const int64_t *__restrict__ index, u32x4 *__restrict__ out,
     int64_t n_in, int64_t n_out, int row_vecs, int pieces_per_row) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int64_t piece = (int64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    const int64_t row = piece / pieces_per_row;
+    const int64_t piece = wave_piece(kWavesPerBlock), row = div_small(piece, pieces_per_row);
     if (row >= n_in) return;
-    const int v0 = (int)(piece % pieces_per_row) * kPieceVecs;
+    const int v0 = (int)(piece - row * pieces_per_row) * kPieceVecs;
     const int64_t dst = index[row];
     if (dst < 0 || dst >= n_out) return;
     u32x4 val[kVecPerLane];
@@ -182,10 +181,9 @@ __global__ __launch_bounds__(kBlock) void reduce_slots_vec_kernel(
     const u32x4 *__restrict__ inp, const int64_t *__restrict__ slot_to_row, u32x4 *__restrict__ out,
     int64_t n_tokens, int top_k, int64_t n_inp, int row_vecs, int pieces_per_row) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int64_t piece = (int64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    const int64_t t = piece / pieces_per_row;
+    const int64_t piece = wave_piece(kWavesPerBlock), t = div_small(piece, pieces_per_row);
     if (t >= n_tokens) return;
-    const int v = (int)(piece % pieces_per_row) * kWave + lane;
+    const int v = (int)(piece - t * pieces_per_row) * kWave + lane;
     if (v >= row_vecs) return;
     float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int j0 = 0; j0 < top_k; j0 += kMaxTopKRegs) {
