@@ -53,7 +53,7 @@ class GateLinearTopK(Function):
     ``count_by_gate`` in one call that keeps the logits on chip.  Returns ``(topk_idx, topk_score)`` like
     :class:`GateTopK`; the routing rides on ``topk_idx``.  Gates of more experts than that call takes run the linear
     layer as a library product first.  Backward: straight from the gradient of the selected logits; a softmax over
-    them, or a shape these kernels do not take, goes through the dense gradient of the logits and library products."""
+    them, a shape these kernels do not take, or ``create_graph`` goes through the dense gradient of the logits and library products."""
 
     @staticmethod
     def forward(ctx, x, weight, bias, top_k, score_mode):
@@ -77,7 +77,9 @@ class GateLinearTopK(Function):
         x, weight, idx, score = ctx.saved_tensors
         score_mode, has_bias = ctx.moe_args
         grad_score = grad_score.contiguous()
-        if score_mode == 0 and fmoe_native.gate_grad_supported(x.shape[1], weight.shape[0], idx.shape[1], x.dtype):
+        # (a backward that is to be differentiated again needs the products as torch operators)
+        if (score_mode == 0 and not torch.is_grad_enabled()
+                and fmoe_native.gate_grad_supported(x.shape[1], weight.shape[0], idx.shape[1], x.dtype)):
             grad_x = grad_w = grad_b = None
             if ctx.needs_input_grad[0]:
                 grad_x = fmoe_native.reduce_slots_gate(None, None, grad_score, idx, weight)

@@ -454,3 +454,20 @@ def test_naive_gate_of_many_experts_matches_the_dense_backward(device, monkeypat
     assert torch.equal(results[0][0], results[1][0])
     for a, b in zip(results[0][1:], results[1][1:]):
         assert torch.allclose(a, b, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("n_expert", [16, 128])   # the linear inside the routing call, and as a library product
+def test_naive_gate_backward_can_be_differentiated_again(n_expert, device):
+    """A penalty on the gradient of the input reaches the gate's weight, as through the linear layer apart.  Bound:
+    float32 sums of 70 terms and a gradient rounded once."""
+    from fastermoe_amd.gates import NaiveGate
+    torch.manual_seed(n_expert)
+    gate = NaiveGate(64, n_expert, 1, top_k=2).to(device)
+    x = torch.randn(70, 64, device=device, requires_grad=True)
+    idx, val = gate(x)
+    grad_x, = torch.autograd.grad(val.sum(), x, create_graph=True)
+    grad_x.square().sum().backward()
+    w = gate.gate.weight.detach().double().cpu().requires_grad_(True)
+    picked = torch.zeros(70, n_expert, dtype=torch.float64).scatter_(1, idx.cpu().view(70, 2), 1.0)
+    (picked @ w).square().sum().backward()
+    assert torch.allclose(gate.gate.weight.grad.double().cpu(), w.grad, rtol=1e-5, atol=1e-5)
