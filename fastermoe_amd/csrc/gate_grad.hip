@@ -5,8 +5,8 @@
 // it, those entries are written into a dense [tokens, experts] matrix and go through two library products a few columns wide, two
 // reductions for the bias and one more pass over the input gradient to add the gate's part:
 //   grad_x[t] = experts' part + sum_j g[t,j] w[idx[t,j]]      grad_w[e] = sum over (t,j) with idx = e of g[t,j] x[t]
-// Here the first is folded into the sum over a token's rows that makes the experts' part (reduce_slots), and
-// the second is one pass over x with the matrix cores.
+// Here the first is a sum of top_k rows of w per token (the gate's own node; a caller that has the experts' part as rows
+// too gets both sums in one pass), and the second is one pass over x with the matrix cores.
 #include "common.hpp"
 #include "profile.hpp"
 #include "vec16.hpp"
