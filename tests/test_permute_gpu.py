@@ -167,6 +167,18 @@ def test_gather_combine_matches_gather_then_bmm(dtype, n, k, d, e, drop, device)
     assert torch.count_nonzero(sd.grad.view(-1)[s2r < 0]) == 0
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,k,d,e", [(1, 1, 8, 1), (5, 3, 512, 4), (6, 4, 1032, 5), (9, 9, 1024, 12), (7, 5, 520, 8),
+                                     (3, 17, 2056, 20), (2, 8, 4104, 9)])
+def test_combine_over_waves_and_slot_groups(dtype, n, k, d, e, device):
+    """Vector kernels of the combine at the edges of their split: rows of at most 128 vectors (one wave per
+    token) and longer ones (a workgroup), numbers of choices that are no multiple of the slots taken at a time, and last
+    workgroups that are not full; with dropped slots and without."""
+    for drop in (0.0, 0.3):
+        test_gather_combine_matches_gather_then_bmm(dtype, n, k, d, e, drop, device)
+    test_combine_matches_bmm(dtype, n, k, d, device)
+
+
 def test_full_size_round_trip(device):
     """config-4 sized rows: scatter then gather restores every kept slot, dropped slots are zero;
     linearity of the reduction."""
