@@ -94,24 +94,49 @@ void fill_table(SegmentTable *tab, const int64_t *counts, int e0, int e1, int64_
 // FMOE_GEMM_TILE=256x256|128x256|128x128|64x64 (the last for fp32 only) forces one shape (for tests and measurements).
 //
 // fp32 tiles take four times as long per slab and are bound by the matrix pipe whatever their shape, so there the
-// question is only how evenly the last round fills: low tiles for longer.  us for 64 x 64 / 128 x 128 / 256 x 256,
-// by the launch's number of 256 x 256 tiles.  Forward: 72 tiles (1024 rows, 16 experts of 768 x 3072): 85 / 107 / 190;
-// 144 (8192 rows, 8 of 512 x 1024): 89 / 113 / 132; 192 (8192 rows, 64 of 1024 x 1024): 216 / 212 / 260; 576 (8192 rows,
-// 8 of 2048 x 4096): 1168 / 1095 / 1144; 1152 (16384 rows, 16 of 1024 x 4096): 1163 / 1113 / 1267; 2112 (32768 rows,
-// 8 of 1024 x 4096): 2242 / 2147 / 2115.  Weight gradient: 64 (8 of 512 x 1024): 74 / 78 / 244; 128: 138 / 136 / 253;
-// 576 (16 of 768 x 3072): 74 / 73 / 80; 1024 (16 of 1024 x 4096): 1085 / 1020 / 993.
+// question is only how evenly they fill the chip: f32_rows_tile, f32_wgrad_tile.
 struct TileShape {
     int bm, bn;
 };
-constexpr int64_t kF32RowTiles64 = 160, kF32RowTiles128 = 1536, kF32WgradTiles64 = 100, kF32WgradTiles128 = 640;
-TileShape pick_tile(int64_t tiles_256, int dtype, int64_t f32_64, int64_t f32_128) {
-    if (const char *e = getenv("FMOE_GEMM_TILE")) {
-        if (!strcmp(e, "256x256")) return {256, 256};
-        if (!strcmp(e, "128x256")) return {128, 256};
-        if (!strcmp(e, "128x128")) return {128, 128};
-        if (!strcmp(e, "64x64") && dtype == FMOE_F32) return {64, 64};
-    }
-    if (dtype == FMOE_F32) return tiles_256 < f32_64 ? TileShape{64, 64} : tiles_256 < f32_128 ? TileShape{128, 128} : TileShape{256, 256};
+bool forced_tile(int dtype, TileShape *tile) {
+    const char *e = getenv("FMOE_GEMM_TILE");
+    if (!e) return false;
+    if (!strcmp(e, "256x256")) *tile = {256, 256};
+    else if (!strcmp(e, "128x256")) *tile = {128, 256};
+    else if (!strcmp(e, "128x128")) *tile = {128, 128};
+    else if (!strcmp(e, "64x64") && dtype == FMOE_F32) *tile = {64, 64};
+    else return false;
+    return true;
+}
+
+// Row-ragged products in fp32.  us for 64 x 64 / 128 x 128 / 256 x 256, by the launch's number of 256 x 256 tiles:
+// 72 tiles (1024 rows, 16 experts of 768 x 3072): 85 / 107 / 190; 144 (8192 rows, 8 of 512 x 1024): 89 / 113 / 132;
+// 192 (8192 rows, 64 of 1024 x 1024): 216 / 212 / 260; 576 (8192 rows, 8 of 2048 x 4096): 1168 / 1095 / 1144;
+// 1152 (16384 rows, 16 of 1024 x 4096): 1163 / 1113 / 1267; 2112 (32768 rows, 8 of 1024 x 4096): 2242 / 2147 / 2115.
+// Few tiles with a long contraction want the 128 x 128 ones, whose contraction is split over workgroups.  Tiles,
+// contraction, us for 64 x 64 / 128 x 128: 18, 3072: 108 / 84; 36, 4608: 642 / 631; 48, 4096: 505 / 497; but 39, 1984: 72 / 84; 42, 2816: 484 / 518;
+// 36, 1536: 83 / 111; 120, 3136: 353 / 381; 126, 1664: 193 / 211.
+TileShape f32_rows_tile(int64_t tiles_256, int64_t contraction) {
+    if (tiles_256 < 160 && contraction < 70 * tiles_256) return {64, 64};
+    return tiles_256 < 1536 ? TileShape{128, 128} : TileShape{256, 256};
+}
+
+// Weight gradients in fp32 (no contraction is split).  With a compute unit's tiles bound by its matrix pipe, a launch takes
+// as long as the unit with the most tile area: 64 x 64 where that is less by more than the 5 % its operands' extra reads
+// cost.  us for 64 x 64 / 128 x 128 / 256 x 256: 12 experts of 576 x 576, 76032 rows: 547 / 773 / 1468; 64 of 1408 x 704,
+// 17152 rows: 318 / 376 / 539; 8 of 2240 x 2240, 6016 rows: 497 / 521 / 559; 16 of 2048 x 512, 46336 rows: 757 / 714 / 708; 16 of
+// 2560 x 2560, 10035 rows: 1067 / 1003 / 1074.  Many tiles of a few rows per expert are bound by their stores and keep the
+// large tile: 32 of 2048 x 4096, 1024 rows: 405 / 372 / 342; 32 of 2304 x 4608, 768: 423 / 368 / 353; not 32 of
+// 2112 x 4224, 3072: 630 / 622 / 657.
+TileShape f32_wgrad_tile(int64_t experts, int64_t out_feat, int64_t in_feat, int64_t rows) {
+    if (experts * ceil_div(out_feat, 256) * ceil_div(in_feat, 256) >= 640 && rows < 48 * experts) return {256, 256};
+    constexpr int64_t kUnits = 256;
+    const int64_t low = ceil_div(experts * ceil_div(out_feat, 64) * ceil_div(in_feat, 64), kUnits) * 64 * 64;
+    const int64_t high = ceil_div(experts * ceil_div(out_feat, 128) * ceil_div(in_feat, 128), kUnits) * 128 * 128;
+    return 105 * low < 100 * high ? TileShape{64, 64} : TileShape{128, 128};
+}
+
+TileShape pick_tile(int64_t tiles_256) {
     if (tiles_256 >= 512) return {256, 256};
     return tiles_256 >= 256 ? TileShape{128, 256} : TileShape{128, 128};
 }
@@ -129,7 +154,10 @@ int kernel_activation(int activation) {
 }
 
 // ragged rows: tiles_256 counts every expert's rows rounded up to whole 256-row tiles
-TileShape pick_rows_tile(const int64_t *counts, int64_t n_expert, int64_t row_lo, int64_t row_hi, int64_t n_cols, int dtype) {
+TileShape pick_rows_tile(const int64_t *counts, int64_t n_expert, int64_t row_lo, int64_t row_hi, int64_t n_cols,
+                         int64_t contraction, int dtype) {
+    TileShape forced;
+    if (forced_tile(dtype, &forced)) return forced;
     int64_t start = 0, row_tiles = 0;
     for (int64_t e = 0; e < n_expert; ++e) {
         const int64_t end = start + counts[e];
@@ -137,14 +165,18 @@ TileShape pick_rows_tile(const int64_t *counts, int64_t n_expert, int64_t row_lo
         if (hi > lo) row_tiles += ceil_div(hi - lo, 256);
         start = end;
     }
-    return pick_tile(row_tiles * ceil_div(n_cols, 256), dtype, kF32RowTiles64, kF32RowTiles128);
+    const int64_t tiles = row_tiles * ceil_div(n_cols, 256);
+    return dtype == FMOE_F32 ? f32_rows_tile(tiles, contraction) : pick_tile(tiles);
 }
 
 // ragged rows over a device table: the host does not know the counts; rows_cap rows spread over
 // the experts make about rows_cap / 256 whole tiles plus a partial one for every other expert
-TileShape pick_rows_tile_estimate(int64_t rows_cap, int64_t n_expert, int64_t n_cols, int dtype) {
+TileShape pick_rows_tile_estimate(int64_t rows_cap, int64_t n_expert, int64_t n_cols, int64_t contraction, int dtype) {
+    TileShape forced;
+    if (forced_tile(dtype, &forced)) return forced;
     const int64_t whole = rows_cap / 256;
-    return pick_tile((whole + std::min<int64_t>(n_expert, std::max<int64_t>(whole, 1)) / 2) * ceil_div(n_cols, 256), dtype, kF32RowTiles64, kF32RowTiles128);
+    const int64_t tiles = (whole + std::min<int64_t>(n_expert, std::max<int64_t>(whole, 1)) / 2) * ceil_div(n_cols, 256);
+    return dtype == FMOE_F32 ? f32_rows_tile(tiles, contraction) : pick_tile(tiles);
 }
 
 // Row tiles of gemm_unaligned.hip, 64 or 128 rows high: the low ones where the high ones would leave part of the
@@ -161,8 +193,11 @@ TileShape pick_unaligned_tile(const int64_t *counts, int64_t n_expert, int64_t r
 }
 
 // weight gradient: C is [out, in] per expert
-TileShape pick_wgrad_tile(int64_t n_experts_written, int64_t out_feat, int64_t in_feat, int dtype) {
-    return pick_tile(n_experts_written * ceil_div(out_feat, 256) * ceil_div(in_feat, 256), dtype, kF32WgradTiles64, kF32WgradTiles128);
+TileShape pick_wgrad_tile(int64_t n_experts_written, int64_t out_feat, int64_t in_feat, int64_t rows, int dtype) {
+    TileShape forced;
+    if (forced_tile(dtype, &forced)) return forced;
+    if (dtype == FMOE_F32) return f32_wgrad_tile(n_experts_written, out_feat, in_feat, rows);
+    return pick_tile(n_experts_written * ceil_div(out_feat, 256) * ceil_div(in_feat, 256));
 }
 
 double table_flop(const SegmentTable &tab, int64_t in_feat, int64_t out_feat) {
@@ -412,7 +447,7 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
         const bool fast = is_fast(a.dtype, {a.x, a.w, a.y, a.aux, a.bias}, {a.in_feat, a.out_feat});
         FMOE_REQUIRE(a.x_row_index == nullptr || linear_forward_can_gather(a),
                      "linear_forward: rows cannot be gathered in the loader for this shape");
-        const TileShape tile = pick_rows_tile_estimate(a.dev_rows_cap, n_expert, a.out_feat, a.dtype);
+        const TileShape tile = pick_rows_tile_estimate(a.dev_rows_cap, n_expert, a.out_feat, a.in_feat, a.dtype);
         GemmParams prm{};
         if (int rc = device_table_launch("linear_forward", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast)) return rc;
         prm.block_m = tile.bm; prm.block_n = tile.bn;
@@ -456,7 +491,7 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
     FMOE_REQUIRE(a.x_row_index == nullptr || linear_forward_can_gather(a),
                  "linear_forward: rows cannot be gathered in the loader for this shape");
     const TileShape tile = !fast && is_16bit(a.dtype) ? pick_unaligned_tile(counts, n_expert, row_lo, row_hi, a.out_feat)
-                                                      : pick_rows_tile(counts, n_expert, row_lo, row_hi, a.out_feat, a.dtype);
+                                                      : pick_rows_tile(counts, n_expert, row_lo, row_hi, a.out_feat, a.in_feat, a.dtype);
     for (int e0 = plan.first; e0 <= plan.last; e0 += kMaxGroupExperts) {
         const int e1 = std::min(plan.last, e0 + kMaxGroupExperts - 1);
         GemmParams prm{};
@@ -483,7 +518,7 @@ int grouped_linear_dgrad(const LinearDgradArgs &a, const int64_t *counts, int64_
         if (a.dev_rows_cap == 0) return FMOE_OK;
         FMOE_REQUIRE(a.gy && a.w && a.gx, "linear_dgrad: NULL tensor");
         const bool fast = is_fast(a.dtype, {a.gy, a.w, a.gx, a.aux}, {a.in_feat, a.out_feat});
-        const TileShape tile = pick_rows_tile_estimate(a.dev_rows_cap, n_expert, a.in_feat, a.dtype);
+        const TileShape tile = pick_rows_tile_estimate(a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype);
         GemmParams prm{};
         if (int rc = device_table_launch("linear_dgrad", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast)) return rc;
         prm.block_m = tile.bm; prm.block_n = tile.bn;
@@ -509,7 +544,7 @@ int grouped_linear_dgrad(const LinearDgradArgs &a, const int64_t *counts, int64_
     const Plan plan = plan_rows(counts, n_expert, row_lo, row_hi);
     const bool fast = is_fast(a.dtype, {a.gy, a.w, a.gx, a.aux}, {a.in_feat, a.out_feat});
     const TileShape tile = !fast && is_16bit(a.dtype) ? pick_unaligned_tile(counts, n_expert, row_lo, row_hi, a.in_feat)
-                                                      : pick_rows_tile(counts, n_expert, row_lo, row_hi, a.in_feat, a.dtype);
+                                                      : pick_rows_tile(counts, n_expert, row_lo, row_hi, a.in_feat, a.out_feat, a.dtype);
     for (int e0 = plan.first; e0 <= plan.last; e0 += kMaxGroupExperts) {
         const int e1 = std::min(plan.last, e0 + kMaxGroupExperts - 1);
         GemmParams prm{};
@@ -534,7 +569,7 @@ int grouped_linear_wgrad(const LinearWgradArgs &a, const int64_t *counts, int64_
         FMOE_REQUIRE(a.gw && (a.dev_rows_cap == 0 || (a.gy && a.x)), "linear_wgrad: NULL tensor");
         // (with no rows at all the pointers may be NULL: every expert's contraction is empty and nothing is read)
         const bool fast = is_fast(a.dtype, {a.gy, a.x, a.gw}, {a.in_feat, a.out_feat});
-        const TileShape tile = pick_wgrad_tile(n_expert, a.out_feat, a.in_feat, a.dtype);
+        const TileShape tile = pick_wgrad_tile(n_expert, a.out_feat, a.in_feat, a.dev_rows_cap, a.dtype);
         GemmParams prm{};
         if (int rc = device_table_launch("linear_wgrad", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast)) return rc;
         prm.block_m = tile.bm; prm.block_n = tile.bn;
@@ -554,7 +589,7 @@ int grouped_linear_wgrad(const LinearWgradArgs &a, const int64_t *counts, int64_
     FMOE_REQUIRE(a.gw && (total == 0 || (a.gy && a.x)), "linear_wgrad: NULL tensor");
     const Plan plan = plan_contraction(counts, n_expert, row_lo, row_hi, last_chunk);
     const bool fast = is_fast(a.dtype, {a.gy, a.x, a.gw}, {a.in_feat, a.out_feat});
-    const TileShape tile = pick_wgrad_tile(plan.last - plan.first + 1, a.out_feat, a.in_feat, a.dtype);
+    const TileShape tile = pick_wgrad_tile(plan.last - plan.first + 1, a.out_feat, a.in_feat, row_hi - row_lo, a.dtype);
     for (int e0 = plan.first; e0 <= plan.last; e0 += kMaxGroupExperts) {
         const int e1 = std::min(plan.last, e0 + kMaxGroupExperts - 1);
         GemmParams prm{};
@@ -684,7 +719,7 @@ extern "C" int fmoe_linear_dev_supported(int64_t in_feat, int64_t out_feat, int 
 
 extern "C" int fmoe_linear_dev_reads_rows(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype) {
     if (!fmoe_linear_dev_supported(in_feat, out_feat, dtype) || rows_cap < 1 || n_expert < 1) return 0;
-    return use_ring(pick_rows_tile_estimate(rows_cap, n_expert, out_feat, dtype), dtype) ? 1 : 0;
+    return use_ring(pick_rows_tile_estimate(rows_cap, n_expert, out_feat, in_feat, dtype), dtype) ? 1 : 0;
 }
 
 extern "C" int64_t fmoe_linear_dev_workspace_bytes(int64_t contraction, int dtype) {
