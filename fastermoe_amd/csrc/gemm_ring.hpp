@@ -413,12 +413,12 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_ring_kernel(const R
                          "s_add_u32 m0, %0, %4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n.Lring_skip%=:"
                          :
                          : "s"(lds_addr), "v"(voff), "s"(rs), "s"(__builtin_amdgcn_readfirstlane((int)go)), "n"(it * 4096)
-                         : "memory", "scc");
+                         : "memory", "m0", "scc");
         } else {
             asm volatile("s_add_u32 m0, %0, %3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                          :
                          : "s"(lds_addr), "v"(voff), "s"(rs), "n"(it * 4096)
-                         : "memory", "scc");
+                         : "memory", "m0", "scc");
         }
         if (odd) op.run1 += step; else op.run0 += step;
     };
