@@ -58,13 +58,18 @@ class _Expert(nn.Module):
                 and fmoe_native.linear_dev_reads_rows(n_slots, n_expert, d_hidden, d_model, inp.dtype))
 
     def _device_tables_apply(self, inp):
+        r"""Whether the products over a device table take these tensors.  They want whole 16-byte chunks on
+        16-byte boundaries, in the sizes and in where the tensors begin: parameters that are views into one flat
+        buffer, or rows that begin inside another tensor, go the module's or the pipeline's way instead."""
         d_hidden, d_model = self.htoh4.weight.shape[1:]
         return (self._epilogue_activation() is not None and inp.is_cuda
                 and inp.dtype in (torch.float32, torch.bfloat16, torch.float16)
                 and self.htoh4.weight.dtype == inp.dtype and self.h4toh.weight.dtype == inp.dtype
                 and os.environ.get("FMOE_EXPERT_EPILOGUE", "1") != "0"
                 and os.environ.get("FMOE_DEVICE_TABLES", "1") != "0"
-                and fmoe_native.linear_dev_supported(d_model, d_hidden, inp.dtype))
+                and fmoe_native.linear_dev_supported(d_model, d_hidden, inp.dtype)
+                and all(t is None or t.data_ptr() % 16 == 0 for t in
+                        (inp, self.htoh4.weight, self.htoh4.bias, self.h4toh.weight, self.h4toh.bias)))
 
     def _epilogue_activation(self):
         from .fused_functions import _activation_code

@@ -6,7 +6,7 @@ rounded inputs, relative to the largest reference magnitude."""
 import pytest
 import torch
 
-from fastermoe_amd import _lib, fmoe_native
+from fastermoe_amd import FMoETransformerMLP, _lib, fmoe_native
 from oracle import moe as omoe
 from helpers import TOL, rel_err
 
@@ -71,3 +71,46 @@ def _check(dtype, counts, fin, fout, device, shift):
     p64 = pre_in.double().requires_grad_(True)
     torch.nn.functional.gelu(p64).backward(x64.grad)
     assert rel_err(fmoe_native.linear_dact_backward(gyd, cnt, wd, pd, _lib.ACT_GELU), p64.grad) <= tol
+
+
+@pytest.mark.parametrize("dtype,n,d,h,e,shift", [
+    (torch.bfloat16, 4096, 4096, 4096, 4, 4),   # sizes at which a fused layer leaves its chunks where it may
+    (torch.bfloat16, 300, 128, 256, 4, 1),
+    (torch.float32, 300, 128, 256, 4, 1),
+])
+@pytest.mark.parametrize("what", ["parameters", "input"])
+@pytest.mark.parametrize("fuse", [False, True])
+def test_layer_over_tensors_at_any_element(dtype, n, d, h, e, shift, what, fuse, device, monkeypatch):
+    """Expert weights and biases that are views into a larger buffer, or token rows that are: the same results as over
+    tensors of their own, fused and unfused.  Bound: the suite's tolerance of the type, twice (two runs with
+    their sums in different orders)."""
+    monkeypatch.delenv("FMOE_FUSE_GRAN", raising=False)
+    torch.manual_seed(shift)
+    with device:
+        moe = FMoETransformerMLP(num_expert=e, d_model=d, d_hidden=h, top_k=2)
+    moe = moe.to(dtype)
+    moe.enable_fuse = fuse
+    with torch.no_grad():
+        for lin in (moe.experts.htoh4, moe.experts.h4toh):
+            lin.weight.normal_(0, lin.weight.shape[2] ** -0.5)
+            lin.bias.normal_()
+    x = torch.randn(n, d, device=device).to(dtype)
+    grad = torch.randn(n, d, device=device).to(dtype)
+
+    def step(inp):
+        moe.zero_grad(set_to_none=True)
+        leaf = inp.detach().requires_grad_(True)
+        out = moe(leaf)
+        out.backward(grad)
+        return [out.detach(), leaf.grad] + [p.grad for p in moe.experts.parameters()]
+
+    want = step(x)
+    if what == "parameters":
+        for p in moe.experts.parameters():
+            p.data = _at(p.data, shift, device)
+            assert p.data_ptr() % 16 != 0
+    else:
+        x = _at(x, shift, device)
+        assert x.data_ptr() % 16 != 0
+    for got, ref in zip(step(x), want):
+        assert rel_err(got, ref) <= 2 * TOL[dtype]
