@@ -23,6 +23,17 @@ def ensure_comm(t, comm):
     return None
 
 
+def _whole_chunks(t):
+    """Whether ``t`` lies as the kernels over 16-byte chunks read it: contiguous, beginning on 16 bytes."""
+    return t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0)
+
+
+def _as_chunks(t):
+    """``t``, or a copy of it that satisfies :func:`_whole_chunks`.  What a forward saved does, but saved-tensor hooks may
+    hand back anything equal to it (a view into the buffer that an offloader packed it into)."""
+    return t if _whole_chunks(t) else t.clone(memory_format=torch.contiguous_format)
+
+
 class GateTopK(Function):
     r"""``torch.topk`` of the gate logits (and, with ``score_mode`` 1, the softmax over the selected
     logits) of fmoe/gates/naive_gate.py:26-42 with the routing of ``count_by_gate`` computed in
@@ -78,7 +89,7 @@ class GateLinearTopK(Function):
         score_mode, has_bias = ctx.moe_args
         grad_score = grad_score.contiguous()
         # (a backward that is to be differentiated again needs the products as torch operators)
-        if (score_mode == 0 and not torch.is_grad_enabled()
+        if (score_mode == 0 and not torch.is_grad_enabled() and _whole_chunks(x) and _whole_chunks(weight)
                 and fmoe_native.gate_grad_supported(x.shape[1], weight.shape[0], idx.shape[1], x.dtype)):
             grad_x = grad_w = grad_b = None
             if ctx.needs_input_grad[0]:
@@ -405,7 +416,7 @@ class MOERoutedMLP(Function):
 
     @staticmethod
     def backward(ctx, grad_out):
-        inp, rows, w1, b1, w2, b2, pos_buf, slot_to_row, table, pre, mid = ctx.saved_tensors
+        inp, rows, w1, b1, w2, b2, pos_buf, slot_to_row, table, pre, mid = map(_as_chunks, ctx.saved_tensors)
         top_k, activation, n_tokens = ctx.moe_args
         n_slots = pos_buf.numel()
         grad_out = grad_out.contiguous()

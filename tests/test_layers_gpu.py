@@ -1088,3 +1088,41 @@ def test_device_table_path_at_extreme_routings(case, dtype, device):
         for expert in range(e):
             if counts[expert] == 0:
                 assert torch.count_nonzero(got[name][expert]) == 0, (name, expert)
+
+
+@pytest.mark.parametrize("n,d,h,e,k", [(300, 128, 256, 4, 2), (200, 64, 64, 100, 2), (4096, 4096, 4096, 4, 2)])
+@pytest.mark.parametrize("fuse", [False, True])
+def test_saved_tensors_that_come_back_at_any_element(n, d, h, e, k, fuse, device, monkeypatch):
+    """Saved-tensor hooks may hand a backward anything equal to what it saved: here views into a packing buffer that
+    begin one element past a 16-byte boundary.  Same gradients as without hooks.  Bound: the suite's tolerance of
+    bfloat16 (the gate's gradients take the products of the library then)."""
+    monkeypatch.delenv("FMOE_FUSE_GRAN", raising=False)
+    torch.manual_seed(n + e)
+    with device:
+        moe = fmoe.FMoETransformerMLP(num_expert=e, d_model=d, d_hidden=h, top_k=k)
+    moe = moe.to(torch.bfloat16)
+    moe.enable_fuse = fuse
+    x = torch.randn(n, d, device=device).to(torch.bfloat16)
+    grad = torch.randn(n, d, device=device).to(torch.bfloat16)
+    moved = []
+
+    def pack(t):
+        if not t.is_floating_point():
+            return t
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        view = buf[1:].view(t.shape)
+        view.copy_(t)
+        moved.append(view.data_ptr() % 16)
+        return view
+
+    def step(hooks):
+        moe.zero_grad(set_to_none=True)
+        leaf = x.clone().requires_grad_(True)
+        with torch.autograd.graph.saved_tensors_hooks(pack if hooks else (lambda t: t), lambda t: t):
+            out = moe(leaf)
+        out.backward(grad)
+        return [leaf.grad] + [p.grad for p in moe.parameters()]
+
+    for got, want in zip(step(True), step(False)):
+        assert rel_err(got, want) <= TOL[torch.bfloat16]
+    assert moved and all(moved)
