@@ -390,7 +390,8 @@ class MOERoutedMLP(Function):
     back to the host: all GEMMs take the experts' row segments from ``table``, the device-side segment
     table of the routing's counts.  Small first GEMMs read token row ``pos_buf[r] // top_k`` for
     sorted row ``r`` in their loader (no scattered copy in the forward); large ones run on a kernel that wants
-    sorted rows, and the copy made for them serves the first linear's weight gradient too.  Returns the
+    sorted rows.  The copy made for them is not kept for the first linear's weight gradient, which makes its own: the
+    tokens, which the gate keeps anyway, are saved, not ``top_k`` times as many rows.  Returns the
     experts' output in expert-sorted order, one row per slot (``[n_slots, d_model]``; the rows past the
     routed ones are not written), for :class:`MOEGatherCombine` / :class:`MOEGather`.  With ``save`` false (nothing
     will be differentiated) the pre-activations are not written.
@@ -405,19 +406,20 @@ class MOERoutedMLP(Function):
         n_expert, d_hidden, d_model = w1.shape
         in_loader = (inp.numel() * inp.element_size() < (1 << 31)
                      and not fmoe_native.linear_dev_reads_rows(n_slots, n_expert, d_model, d_hidden, inp.dtype))
-        rows = None if in_loader else fmoe_native.gather_rows(inp, pos_buf, index_div=top_k)
-        mid, pre = fmoe_native.linear_forward_dev(inp if in_loader else rows, w1, b1, table, n_slots, activation, keep_pre,
+        src = inp if in_loader else fmoe_native.gather_rows(inp, pos_buf, index_div=top_k)
+        mid, pre = fmoe_native.linear_forward_dev(src, w1, b1, table, n_slots, activation, keep_pre,
                                                   row_index=pos_buf if in_loader else None, index_div=top_k)
+        del src   # (its memory serves the output, which is as large)
         out, _ = fmoe_native.linear_forward_dev(mid, w2, b2, table, n_slots)
         if save:
-            ctx.save_for_backward(inp if in_loader else None, rows, w1, b1, w2, b2, pos_buf, slot_to_row, table, pre, mid)
-        ctx.moe_args = top_k, activation, inp.shape[0]
+            ctx.save_for_backward(inp, w1, b1, w2, b2, pos_buf, slot_to_row, table, pre, mid)
+        ctx.moe_args = top_k, activation
         return out
 
     @staticmethod
     def backward(ctx, grad_out):
-        inp, rows, w1, b1, w2, b2, pos_buf, slot_to_row, table, pre, mid = map(_as_chunks, ctx.saved_tensors)
-        top_k, activation, n_tokens = ctx.moe_args
+        inp, w1, b1, w2, b2, pos_buf, slot_to_row, table, pre, mid = map(_as_chunks, ctx.saved_tensors)
+        top_k, activation = ctx.moe_args
         n_slots = pos_buf.numel()
         grad_out = grad_out.contiguous()
         g_pre = fmoe_native.linear_dgrad_dev(grad_out, w2, table, n_slots, pre if pre is not None else mid, activation)
@@ -425,9 +427,8 @@ class MOERoutedMLP(Function):
         g_inp = None
         if ctx.needs_input_grad[0]:
             g_rows = fmoe_native.linear_dgrad_dev(g_pre, w1, table, n_slots)
-            g_inp = fmoe_native.reduce_slots(g_rows, slot_to_row, n_tokens, top_k)
-        if rows is None:
-            rows = fmoe_native.gather_rows(inp, pos_buf, index_div=top_k)
+            g_inp = fmoe_native.reduce_slots(g_rows, slot_to_row, inp.shape[0], top_k)
+        rows = fmoe_native.gather_rows(inp, pos_buf, index_div=top_k)
         gw1, gb1 = fmoe_native.linear_wgrad_dev(g_pre, rows, w1, table, n_slots, b1 is not None)
         return g_inp, gw1, gb1, gw2, gb2, None, None, None, None, None, None
 

@@ -1126,3 +1126,26 @@ def test_saved_tensors_that_come_back_at_any_element(n, d, h, e, k, fuse, device
     for got, want in zip(step(True), step(False)):
         assert rel_err(got, want) <= TOL[torch.bfloat16]
     assert moved and all(moved)
+
+
+@pytest.mark.parametrize("fuse", [False, True])
+@pytest.mark.parametrize("n,d,h,e,k", [(4096, 2048, 4096, 8, 4), (4096, 2048, 1024, 64, 8)])
+def test_memory_held_between_forward_and_backward(n, d, h, e, k, fuse, device, monkeypatch):
+    """A training forward holds, per slot, the pre-activation, the hidden row and the experts' output row (the combine's
+    backward needs it), and per token the layer's output: no sorted copy of the input, which would be another row
+    per slot.  Allowed beside them: 1 MiB of scores, indices and tables, and the allocator's 2 MiB granularity for
+    each of the large tensors."""
+    monkeypatch.delenv("FMOE_FUSE_GRAN", raising=False)
+    with device:
+        moe = fmoe.FMoETransformerMLP(num_expert=e, d_model=d, d_hidden=h, top_k=k)
+    moe = moe.to(torch.bfloat16)
+    moe.enable_fuse = fuse
+    x = torch.randn(n, d, device=device).to(torch.bfloat16).requires_grad_(True)
+    moe(x).float().sum().backward()   # gradients and pools are there
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated(device)
+    out = moe(x)
+    held = torch.cuda.memory_allocated(device) - before
+    assert held <= 2 * (n * k * (2 * h + d) + n * d) + (1 << 20) + 4 * (2 << 20)
+    assert 2 * n * k * d > (1 << 20) + 4 * (2 << 20)   # (a sorted copy does not fit into that)
+    del out
