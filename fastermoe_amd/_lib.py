@@ -69,6 +69,8 @@ SIGNATURES = {
     "fmoe_linear_dev_supported": (_int, [_i64, _i64, _int]),
     "fmoe_linear_dev_reads_rows": (_int, [_i64, _i64, _i64, _i64, _int]),
     "fmoe_linear_dev_workspace_bytes": (_i64, [_i64, _int]),
+    "fmoe_linear_forward_dev_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _int, _int, _int, _int]),
+    "fmoe_linear_dgrad_dev_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _int, _int]),
     "fmoe_linear_forward_dev": (_int, [_vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp,
                                        _i64, _vp]),
     "fmoe_linear_dgrad_dev": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp, _i64, _vp]),

@@ -36,8 +36,8 @@ struct RingParams {
     int32_t n_cols, n_rows, k_extent, tiles_n, tiles_m;
     const int32_t *dev_tab;    // segtab layout
     int32_t dev_map_off, dev_order_off, n_expert;
-    // Ragged rows: the accumulators of tiles whose contraction is shared by several workgroups (null: none is shared), two
-    // tiles of floats per workgroup; ws_wgs workgroups run the launch (the number the second kernel plans with).
+    // Ragged rows: the accumulators of tiles whose contraction is shared by several workgroups (null: none is shared),
+    // ring_ws_tiles() tiles of floats; ws_wgs workgroups run the launch (the number the second kernel plans with).
     float *split_ws;
     int32_t ws_wgs;
 };
@@ -73,6 +73,10 @@ __host__ __device__ inline RingPlan ring_plan(int tiles, int per, int n_slabs, b
 }
 // whether any tile count makes ring_plan cut a contraction of n_slabs slabs
 inline bool ring_split_possible(int n_slabs) { return n_slabs - (n_slabs + kRingMaxParts - 1) / kRingMaxParts >= kRingSplitSaves; }
+// Where the part of run j that lies in tail tile i goes, in tiles of floats: from one part to the next j, i or both go up
+// by one, so the parts of an XCD (`per` runs at most, over at most per / 2 tiles) fit in per + per / 2 places.
+__host__ __device__ inline int ring_ws_slot(int xcd, int per, int run, int tail_tile) { return xcd * (per + per / 2) + run + tail_tile; }
+inline int64_t ring_ws_tiles(int wgs) { return (int64_t)(wgs / 8 + wgs / 8 / 2) * 8; }
 // the run that holds slab x of the tail's tail * n_slabs slabs; run j is [j * total / wgs, (j + 1) * total / wgs)
 __device__ __forceinline__ int ring_run_of(int x, int total, int wgs) { return ((x + 1) * wgs - 1) / total; }
 
@@ -293,7 +297,7 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_ring_kernel(const R
                 tl.partial = hi - lo < k_slabs;
                 tl.first_slab = lo - tail_tile * k_slabs;
                 tl.K = min(prm.k_extent - tl.first_slab * BKE, (hi - lo) * BKE);
-                tl.ws_slot = 2 * (xcd * per + slot) + (r > plan.full ? 1 : 0);
+                tl.ws_slot = ring_ws_slot(xcd, per, slot, tail_tile);
             }
         } else {
             const int grid = gridDim.x, fwd = xcd * per + slot, tpe = prm.tiles_m * prm.tiles_n;
@@ -717,9 +721,8 @@ __global__ __launch_bounds__(64) void ring_combine_kernel(const RingParams prm) 
 #pragma unroll
         for (int b = 0; b < kBatch; ++b) {
             const int j = j0 + b <= last ? j0 + b : last;
-            // workgroup j's part of this tile is its first item of the tail if its run begins in this tile
-            const int slot = 2 * (xcd * per + j) + (j * slabs / wgs / k_slabs == tail_tile ? 0 : 1);
-            const f32x4 *src = (const f32x4 *)prm.split_ws + (int64_t)slot * (kRingTile * kRingTile / 4) + wave * 64 + threadIdx.x;
+            const f32x4 *src = (const f32x4 *)prm.split_ws + (int64_t)ring_ws_slot(xcd, per, j, tail_tile) * (kRingTile * kRingTile / 4) +
+                               wave * 64 + threadIdx.x;
 #pragma unroll
             for (int x = 0; x < 8; ++x) v[b][x] = __builtin_nontemporal_load(src + (x * 4 + y) * kRingThreads);
         }
@@ -736,6 +739,9 @@ __global__ __launch_bounds__(64) void ring_combine_kernel(const RingParams prm) 
 #endif
 }
 
+// one workgroup per compute unit, the same number for each of the eight XCDs
+inline int ring_workgroups() { return std::max(8, device_compute_units() / 8 * 8); }
+
 template <typename T, int PS, int QS, int RG, int EPI, int ACT = FMOE_ACT_NONE, bool AUX = false>
 int launch_ring(RingParams prm, hipStream_t stream) {
     static std::atomic<int> configured[16];
@@ -748,8 +754,7 @@ int launch_ring(RingParams prm, hipStream_t stream) {
         configured[dev].store(err == hipSuccess ? 1 : 2, std::memory_order_release);
         FMOE_HIP_CHECK(err);
     }
-    // one workgroup per compute unit, the same number for each of the eight XCDs
-    const int grid = std::max(8, device_compute_units() / 8 * 8);
+    const int grid = ring_workgroups();
     prm.ws_wgs = grid;
     if (RG != kRaggedRows || !ring_split_possible((prm.k_extent + 63) / 64)) prm.split_ws = nullptr;
     kern<<<grid, kRingThreads, kRingLds, stream>>>(prm);

@@ -325,6 +325,42 @@ bool use_skinny(int64_t rows_cap, int64_t n_expert, int64_t out_feat, int dtype)
     return rows_cap <= 2 * n_expert || (rows_cap <= 8 * n_expert && n_expert * ceil_div(out_feat, 128) < 1024);
 }
 
+// The kernel of a row-ragged launch over a device table, and the workspace it can make use of.
+enum class DevKernel { kTiles, kSkinny, kRing };
+struct DevRoute {
+    DevKernel kernel;
+    TileShape tile;
+};
+DevRoute forward_route(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype, int epilogue,
+                       int activation, bool keep_pre, bool gathers) {
+    const TileShape tile = pick_rows_tile_estimate(rows_cap, n_expert, out_feat, in_feat, dtype);
+    if (use_skinny(rows_cap, n_expert, out_feat, dtype)) return {DevKernel::kSkinny, tile};
+    // (what the persistent kernel is built for; the erf formula, "none" and ReLU with a saved pre-activation are rare)
+    const bool ring_act = epilogue == kEpiStore || activation == FMOE_ACT_GELU || (activation == FMOE_ACT_RELU && !keep_pre);
+    return {use_ring(tile, dtype) && !gathers && ring_act ? DevKernel::kRing : DevKernel::kTiles, tile};
+}
+DevRoute dgrad_route(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype, int epilogue, int activation) {
+    const TileShape tile = pick_rows_tile_estimate(rows_cap, n_expert, in_feat, out_feat, dtype);
+    const bool ring_act = epilogue == kEpiStore || activation == FMOE_ACT_GELU || activation == FMOE_ACT_RELU;
+    return {use_ring(tile, dtype) && ring_act ? DevKernel::kRing : DevKernel::kTiles, tile};
+}
+int64_t route_workspace_bytes(const DevRoute &route, int64_t contraction, int dtype) {
+    const int eb = dtype_bytes(dtype);
+    const int n_slabs = (int)std::min<int64_t>(ceil_div(contraction, kSlabBytes / eb), 1 << 24);
+    // (contractions that the tiles would not split pay on neither kernel: 48 slabs and a tail of two tiles per XCD on the
+    // persistent one take 187 us cut and not cut)
+    if (route.kernel == DevKernel::kSkinny || !tail_split_possible(n_slabs, eb == 4 ? 2 : 1)) return 0;
+    const int64_t tile_bytes = (int64_t)route.tile.bm * route.tile.bn * (int64_t)sizeof(float);
+    if (route.kernel == DevKernel::kRing) return ring_split_possible(n_slabs) ? ring_ws_tiles(ring_workgroups()) * tile_bytes : 0;
+    // (a split never has more parts than compute units, and 64 x 64 tiles are never split)
+    return route.tile.bm == 64 ? 0 : device_compute_units() * tile_bytes;
+}
+// the caller's workspace where it is one, else null: the launch is not split
+float *route_workspace(const DevRoute &route, int64_t contraction, int dtype, void *ws, int64_t ws_bytes) {
+    const int64_t need = route_workspace_bytes(route, contraction, dtype);
+    return ws != nullptr && need > 0 && ws_bytes >= need && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0 ? (float *)ws : nullptr;
+}
+
 template <int PRODUCT>
 int dispatch_ring(const GemmParams &g, int dtype, int epi, hipStream_t stream) {
     RingParams prm{};
@@ -430,11 +466,9 @@ int device_table_launch(const char *who, GemmParams &prm, const int32_t *dev_tab
 int64_t linear_dev_workspace_bytes(int64_t contraction, int dtype) {
     const int eb = dtype_bytes(dtype);
     if (eb == 0 || dtype == FMOE_F64 || contraction < 1) return 0;
-    const int64_t per_slab = kSlabBytes / eb;
-    if (!tail_split_possible((int)std::min<int64_t>(ceil_div(contraction, per_slab), 1 << 24), eb == 4 ? 2 : 1)) return 0;
-    // one tile of fp32 accumulators per compute unit: a split never has more parts than that.  The persistent
-    // kernel's workgroups (16-bit types) leave up to two.
-    return (int64_t)device_compute_units() * 256 * 256 * (int64_t)sizeof(float) * (eb == 2 ? 2 : 1);
+    // the most that any launch of this contraction can use: 256 x 256 tiles, on the persistent kernel for 16-bit types
+    const DevRoute tiles{DevKernel::kTiles, {256, 256}}, ring{DevKernel::kRing, {256, 256}};
+    return std::max(route_workspace_bytes(tiles, contraction, dtype), eb == 2 ? route_workspace_bytes(ring, contraction, dtype) : 0);
 }
 
 int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, int64_t n_expert, int64_t row_lo,
@@ -447,10 +481,12 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
         const bool fast = is_fast(a.dtype, {a.x, a.w, a.y, a.aux, a.bias}, {a.in_feat, a.out_feat});
         FMOE_REQUIRE(a.x_row_index == nullptr || linear_forward_can_gather(a),
                      "linear_forward: rows cannot be gathered in the loader for this shape");
-        const TileShape tile = pick_rows_tile_estimate(a.dev_rows_cap, n_expert, a.out_feat, a.in_feat, a.dtype);
         GemmParams prm{};
         if (int rc = device_table_launch("linear_forward", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast)) return rc;
-        prm.block_m = tile.bm; prm.block_n = tile.bn;
+        prm.activation = kernel_activation(a.activation);
+        const DevRoute route = forward_route(a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype, a.epilogue, prm.activation,
+                                             a.aux != nullptr, a.x_row_index != nullptr);
+        prm.block_m = route.tile.bm; prm.block_n = route.tile.bn;
         prm.profile_class = kProfGemmFwd; prm.profile_work = 2.0 * (double)a.dev_rows_cap * (double)a.in_feat * (double)a.out_feat;
         prm.P = a.w; prm.Q = a.x; prm.C = a.y; prm.bias = a.bias; prm.aux = a.aux;
         prm.q_row_index = a.x_row_index; set_row_index_divisor(prm, a.x_index_div); prm.q_total_rows = a.x_total_rows;
@@ -458,11 +494,8 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
         prm.p_expert_stride = a.in_feat * a.out_feat;
         prm.bias_expert_stride = a.out_feat;
         prm.n_cols = (int)a.out_feat; prm.k_extent = (int)a.in_feat;
-        prm.activation = kernel_activation(a.activation);
-        const int64_t ws_need = linear_dev_workspace_bytes(a.in_feat, a.dtype);
-        if (a.dev_workspace != nullptr && ws_need > 0 && a.dev_workspace_bytes >= ws_need && aligned16(a.dev_workspace))
-            prm.dev_split_ws = (float *)a.dev_workspace;
-        if (use_skinny(a.dev_rows_cap, n_expert, a.out_feat, a.dtype)) {
+        prm.dev_split_ws = route_workspace(route, a.in_feat, a.dtype, a.dev_workspace, a.dev_workspace_bytes);
+        if (route.kernel == DevKernel::kSkinny) {
             SkinnyParams sk{};
             sk.w = a.w; sk.x = a.x; sk.bias = a.bias; sk.y = a.y; sk.aux = a.aux;
             sk.dev_tab = a.dev_tab;
@@ -474,10 +507,7 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
             ProfileScope prof(prm.profile_class, prm.profile_work, stream);
             return launch_skinny(sk, a.dtype, segtab::cap_tiles(a.dev_rows_cap, n_expert, 128), stream);
         }
-        // (what the persistent kernel is built for; the erf formula, "none" and ReLU with a saved pre-activation are rare)
-        const bool ring_act = a.epilogue == kEpiStore || prm.activation == FMOE_ACT_GELU ||
-                              (prm.activation == FMOE_ACT_RELU && a.aux == nullptr);
-        if (use_ring(tile, a.dtype) && a.x_row_index == nullptr && ring_act) return dispatch_ring<kFwd>(prm, a.dtype, a.epilogue, stream);
+        if (route.kernel == DevKernel::kRing) return dispatch_ring<kFwd>(prm, a.dtype, a.epilogue, stream);
         return dispatch<kFwd>(prm, a.dtype, a.epilogue, fast, stream);
     }
     int64_t total;
@@ -518,21 +548,18 @@ int grouped_linear_dgrad(const LinearDgradArgs &a, const int64_t *counts, int64_
         if (a.dev_rows_cap == 0) return FMOE_OK;
         FMOE_REQUIRE(a.gy && a.w && a.gx, "linear_dgrad: NULL tensor");
         const bool fast = is_fast(a.dtype, {a.gy, a.w, a.gx, a.aux}, {a.in_feat, a.out_feat});
-        const TileShape tile = pick_rows_tile_estimate(a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype);
         GemmParams prm{};
         if (int rc = device_table_launch("linear_dgrad", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast)) return rc;
-        prm.block_m = tile.bm; prm.block_n = tile.bn;
+        prm.activation = kernel_activation(a.activation);
+        const DevRoute route = dgrad_route(a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype, a.epilogue, prm.activation);
+        prm.block_m = route.tile.bm; prm.block_n = route.tile.bn;
         prm.profile_class = kProfGemmDgrad; prm.profile_work = 2.0 * (double)a.dev_rows_cap * (double)a.in_feat * (double)a.out_feat;
         prm.P = a.w; prm.Q = a.gy; prm.C = a.gx; prm.aux = const_cast<void *>(a.aux);
         prm.ldp = a.in_feat; prm.ldq = a.out_feat; prm.ldc = a.in_feat;
         prm.p_expert_stride = a.in_feat * a.out_feat;
         prm.n_cols = (int)a.in_feat; prm.k_extent = (int)a.out_feat;
-        prm.activation = kernel_activation(a.activation);
-        const int64_t ws_need = linear_dev_workspace_bytes(a.out_feat, a.dtype);
-        if (a.dev_workspace != nullptr && ws_need > 0 && a.dev_workspace_bytes >= ws_need && aligned16(a.dev_workspace))
-            prm.dev_split_ws = (float *)a.dev_workspace;
-        const bool ring_act = a.epilogue == kEpiStore || prm.activation == FMOE_ACT_GELU || prm.activation == FMOE_ACT_RELU;
-        if (use_ring(tile, a.dtype) && ring_act) return dispatch_ring<kDgrad>(prm, a.dtype, a.epilogue, stream);
+        prm.dev_split_ws = route_workspace(route, a.out_feat, a.dtype, a.dev_workspace, a.dev_workspace_bytes);
+        if (route.kernel == DevKernel::kRing) return dispatch_ring<kDgrad>(prm, a.dtype, a.epilogue, stream);
         return dispatch<kDgrad>(prm, a.dtype, a.epilogue, fast, stream);
     }
     int64_t total;
@@ -720,6 +747,22 @@ extern "C" int fmoe_linear_dev_supported(int64_t in_feat, int64_t out_feat, int 
 extern "C" int fmoe_linear_dev_reads_rows(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype) {
     if (!fmoe_linear_dev_supported(in_feat, out_feat, dtype) || rows_cap < 1 || n_expert < 1) return 0;
     return use_ring(pick_rows_tile_estimate(rows_cap, n_expert, out_feat, in_feat, dtype), dtype) ? 1 : 0;
+}
+
+extern "C" int64_t fmoe_linear_forward_dev_workspace_bytes(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat,
+                                                           int dtype, int activation, int keep_pre, int gathers) {
+    if (!fmoe_linear_dev_supported(in_feat, out_feat, dtype) || rows_cap < 1 || n_expert < 1) return 0;
+    const bool plain = activation == FMOE_ACT_NONE && !keep_pre;
+    return route_workspace_bytes(forward_route(rows_cap, n_expert, in_feat, out_feat, dtype, plain ? kEpiStore : kEpiBiasAct,
+                                               kernel_activation(activation), keep_pre != 0, gathers != 0), in_feat, dtype);
+}
+
+extern "C" int64_t fmoe_linear_dgrad_dev_workspace_bytes(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat,
+                                                         int dtype, int activation) {
+    if (!fmoe_linear_dev_supported(in_feat, out_feat, dtype) || rows_cap < 1 || n_expert < 1) return 0;
+    return route_workspace_bytes(dgrad_route(rows_cap, n_expert, in_feat, out_feat, dtype,
+                                             activation == FMOE_ACT_NONE ? kEpiStore : kEpiDAct, kernel_activation(activation)),
+                                 out_feat, dtype);
 }
 
 extern "C" int64_t fmoe_linear_dev_workspace_bytes(int64_t contraction, int dtype) {

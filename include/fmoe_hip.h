@@ -454,6 +454,21 @@ int fmoe_linear_dev_reads_rows(int64_t rows_cap, int64_t n_expert,
  * last round is then not split. */
 int64_t fmoe_linear_dev_workspace_bytes(int64_t contraction, int dtype);
 
+/* The same for one launch: what fmoe_linear_forward_dev (keep_pre: pre != NULL,
+ * gathers: x_row_index != NULL) and fmoe_linear_dgrad_dev can use with these
+ * arguments, never more than the general figure and 0 for the launches that
+ * split nothing.  Host only. */
+int64_t fmoe_linear_forward_dev_workspace_bytes(int64_t rows_cap,
+                                                int64_t n_expert,
+                                                int64_t in_feat,
+                                                int64_t out_feat, int dtype,
+                                                int activation, int keep_pre,
+                                                int gathers);
+int64_t fmoe_linear_dgrad_dev_workspace_bytes(int64_t rows_cap,
+                                              int64_t n_expert,
+                                              int64_t in_feat, int64_t out_feat,
+                                              int dtype, int activation);
+
 /* fmoe_linear_forward / fmoe_linear_act_forward over a device table:
  *   pre[seg_e] = x[seg_e] . w[e]^T + bias[e]  (stored when pre != NULL)
  *   y[seg_e]   = act(pre[seg_e])              (activation FMOE_ACT_NONE: y = pre)

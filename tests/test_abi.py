@@ -315,3 +315,36 @@ int main(void) {
     run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert run.returncode == 0, (run.returncode, run.stdout, run.stderr)
     assert run.stdout.split()[0] == "0" and run.stdout.split()[2] == "1024"
+
+
+def test_split_workspace_of_a_launch():
+    """Bytes that a launch over a device table can use, by its kernel: nothing for few rows per expert (weights straight
+    from memory) or for short contractions; a tile per compute unit; a tile and a half of 256 x 256 per compute unit
+    on the persistent kernel.  Never more than the figure that knows the contraction alone."""
+    lib = _lib.load()
+    cus = 256   # of a gfx950 device, and what the library assumes where there is none
+    tile = lambda m, n: m * n * 4
+
+    def fwd(rows, e, fin, fout, dt, act=_lib.ACT_NONE, pre=0, gathers=0):
+        got = lib.fmoe_linear_forward_dev_workspace_bytes(rows, e, fin, fout, dt, act, pre, gathers)
+        assert 0 <= got <= lib.fmoe_linear_dev_workspace_bytes(fin, dt)
+        return got
+
+    def dgrad(rows, e, fin, fout, dt, act=_lib.ACT_NONE):
+        got = lib.fmoe_linear_dgrad_dev_workspace_bytes(rows, e, fin, fout, dt, act)
+        assert 0 <= got <= lib.fmoe_linear_dev_workspace_bytes(fout, dt)
+        return got
+
+    assert fwd(2, 32, 4096, 1024, _lib.BF16) == 0                                # one decoded token
+    assert dgrad(2, 32, 1024, 4096, _lib.BF16) == cus * tile(128, 128)
+    assert fwd(2048, 32, 4096, 1024, _lib.BF16) == cus * tile(128, 128)
+    assert fwd(65536, 8, 4096, 14336, _lib.BF16) == cus * 3 // 2 * tile(256, 256)
+    assert fwd(65536, 8, 4096, 14336, _lib.F16, _lib.ACT_GELU, 1) == cus * 3 // 2 * tile(256, 256)
+    assert fwd(65536, 8, 4096, 14336, _lib.BF16, gathers=1) == cus * tile(256, 256)
+    assert fwd(65536, 8, 4096, 14336, _lib.BF16, _lib.ACT_RELU, 1) == cus * tile(256, 256)   # (not on the persistent kernel)
+    assert fwd(65536, 8, 1024, 14336, _lib.BF16) == 0                            # 16 slabs
+    assert fwd(4096, 16, 1024, 1024, _lib.F32) == 0                              # 64 x 64 tiles
+    assert fwd(65536, 8, 4100, 14336, _lib.BF16) == 0 and fwd(0, 8, 4096, 14336, _lib.BF16) == 0
+    assert lib.fmoe_linear_dev_workspace_bytes(4096, _lib.BF16) == cus * 3 // 2 * tile(256, 256)
+    assert lib.fmoe_linear_dev_workspace_bytes(4096, _lib.F32) == cus * tile(256, 256)
+    assert lib.fmoe_linear_dev_workspace_bytes(1024, _lib.BF16) == 0

@@ -1149,3 +1149,18 @@ def test_memory_held_between_forward_and_backward(n, d, h, e, k, fuse, device, m
     assert held <= 2 * (n * k * (2 * h + d) + n * d) + (1 << 20) + 4 * (2 << 20)
     assert 2 * n * k * d > (1 << 20) + 4 * (2 << 20)   # (a sorted copy does not fit into that)
     del out
+
+
+def test_decoding_takes_no_split_workspace(device):
+    """One token through a layer of the default size: both products read the weights straight from memory and share no
+    tile, so the allocator's peak stays at the step's own small tensors."""
+    with device:
+        moe = fmoe.FMoETransformerMLP(num_expert=32, d_model=1024, d_hidden=4096, top_k=2).to(torch.bfloat16)
+    x = torch.randn(1, 1024, device=device).to(torch.bfloat16)
+    with torch.no_grad():
+        moe(x)
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated(device)
+        torch.cuda.reset_peak_memory_stats(device)
+        moe(x)
+    assert torch.cuda.max_memory_allocated(device) - before < 1 << 20
