@@ -67,6 +67,7 @@ SIGNATURES = {
     "fmoe_segment_table_bytes": (_i64, [_i64, _i64]),
     "fmoe_segment_table_build": (_int, [_vp, _i64, _i64, _vp, _i64, _vp]),
     "fmoe_linear_dev_supported": (_int, [_i64, _i64, _int]),
+    "fmoe_linear_act_dev_reads_rows": (_int, [_i64, _i64, _i64, _i64, _int, _int, _int]),
     "fmoe_linear_dev_reads_rows": (_int, [_i64, _i64, _i64, _i64, _int]),
     "fmoe_linear_dev_workspace_bytes": (_i64, [_i64, _int]),
     "fmoe_linear_forward_dev_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _int, _int, _int, _int]),

@@ -744,9 +744,16 @@ extern "C" int fmoe_linear_dev_supported(int64_t in_feat, int64_t out_feat, int 
     return (in_feat % ce == 0 && out_feat % ce == 0 && in_feat * eb <= (1 << 22) && out_feat * eb <= (1 << 22)) ? 1 : 0;
 }
 
-extern "C" int fmoe_linear_dev_reads_rows(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype) {
+extern "C" int fmoe_linear_act_dev_reads_rows(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype,
+                                              int activation, int keep_pre) {
     if (!fmoe_linear_dev_supported(in_feat, out_feat, dtype) || rows_cap < 1 || n_expert < 1) return 0;
-    return use_ring(pick_rows_tile_estimate(rows_cap, n_expert, out_feat, in_feat, dtype), dtype) ? 1 : 0;
+    const bool plain = activation == FMOE_ACT_NONE && !keep_pre;
+    return forward_route(rows_cap, n_expert, in_feat, out_feat, dtype, plain ? kEpiStore : kEpiBiasAct, kernel_activation(activation),
+                         keep_pre != 0, false).kernel == DevKernel::kRing ? 1 : 0;
+}
+
+extern "C" int fmoe_linear_dev_reads_rows(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype) {
+    return fmoe_linear_act_dev_reads_rows(rows_cap, n_expert, in_feat, out_feat, dtype, FMOE_ACT_NONE, 0);
 }
 
 extern "C" int64_t fmoe_linear_forward_dev_workspace_bytes(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat,

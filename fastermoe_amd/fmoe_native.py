@@ -663,10 +663,10 @@ def linear_dev_supported(in_feat, out_feat, dtype):
     return dtype in _DTYPES and _lib.load().fmoe_linear_dev_supported(int(in_feat), int(out_feat), _DTYPES[dtype]) == 1
 
 
-def linear_dev_reads_rows(rows_cap, n_expert, in_feat, out_feat, dtype):
+def linear_dev_reads_rows(rows_cap, n_expert, in_feat, out_feat, dtype, activation=_lib.ACT_NONE, keep_pre=False):
     """Whether :func:`linear_forward_dev` for these sizes is faster over sorted rows than through ``row_index``."""
-    return _lib.load().fmoe_linear_dev_reads_rows(int(rows_cap), int(n_expert), int(in_feat), int(out_feat),
-                                                  _DTYPES[dtype]) == 1
+    return _lib.load().fmoe_linear_act_dev_reads_rows(int(rows_cap), int(n_expert), int(in_feat), int(out_feat),
+                                                      _DTYPES[dtype], activation, int(keep_pre)) == 1
 
 
 def _dev_workspace(nbytes, device):

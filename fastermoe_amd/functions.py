@@ -405,7 +405,7 @@ class MOERoutedMLP(Function):
         keep_pre = save and activation == _lib.ACT_GELU  # ReLU's derivative can be read off the output
         n_expert, d_hidden, d_model = w1.shape
         in_loader = (inp.numel() * inp.element_size() < (1 << 31)
-                     and not fmoe_native.linear_dev_reads_rows(n_slots, n_expert, d_model, d_hidden, inp.dtype))
+                     and not fmoe_native.linear_dev_reads_rows(n_slots, n_expert, d_model, d_hidden, inp.dtype, activation, keep_pre))
         src = inp if in_loader else fmoe_native.gather_rows(inp, pos_buf, index_div=top_k)
         mid, pre = fmoe_native.linear_forward_dev(src, w1, b1, table, n_slots, activation, keep_pre,
                                                   row_index=pos_buf if in_loader else None, index_div=top_k)

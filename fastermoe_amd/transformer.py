@@ -4,7 +4,7 @@ import os
 import torch
 import torch.nn as nn
 
-from . import fmoe_native
+from . import _lib, fmoe_native
 from .functions import MOEExpertMLP, MOERoutedMLP
 from .gates import NaiveGate
 from .layers import FMoE, FMoELinear
@@ -52,9 +52,11 @@ class _Expert(nn.Module):
         r"""Whether :meth:`routed_forward` beats the chunked pipeline: where both linears run on the persistent
         kernel and nobody asks for a number of chunks.  The pipeline hides the row permutes behind the
         products of its chunks, but needs the counts on the host and pays every chunk's last round of tiles."""
+        if "FMOE_FUSE_GRAN" in os.environ or not self._device_tables_apply(inp):
+            return False
         n_expert, d_hidden, d_model = self.htoh4.weight.shape
-        return ("FMOE_FUSE_GRAN" not in os.environ and self._device_tables_apply(inp)
-                and fmoe_native.linear_dev_reads_rows(n_slots, n_expert, d_model, d_hidden, inp.dtype)
+        code = self._epilogue_activation()
+        return (fmoe_native.linear_dev_reads_rows(n_slots, n_expert, d_model, d_hidden, inp.dtype, code, code == _lib.ACT_GELU)
                 and fmoe_native.linear_dev_reads_rows(n_slots, n_expert, d_hidden, d_model, inp.dtype))
 
     def _device_tables_apply(self, inp):

@@ -440,9 +440,14 @@ int fmoe_segment_table_build(const int64_t *expert_count, int64_t n_expert,
  * feature sizes that are multiples of 16 bytes), else 0.  Host only. */
 int fmoe_linear_dev_supported(int64_t in_feat, int64_t out_feat, int dtype);
 
-/* Whether fmoe_linear_forward_dev for these sizes runs on the kernel that reads
+/* Whether fmoe_linear_forward_dev for these sizes, with this activation and with
+ * (keep_pre) or without a pre-activation to store, runs on the kernel that reads
  * the rows of x in order (1: sorted rows are faster than x_row_index; 0:
- * either). */
+ * either).  FMOE_GELU_ERF=1 takes GELU off that kernel.  The second form is the
+ * one without activation. */
+int fmoe_linear_act_dev_reads_rows(int64_t rows_cap, int64_t n_expert,
+                                   int64_t in_feat, int64_t out_feat, int dtype,
+                                   int activation, int keep_pre);
 int fmoe_linear_dev_reads_rows(int64_t rows_cap, int64_t n_expert,
                                int64_t in_feat, int64_t out_feat, int dtype);
 

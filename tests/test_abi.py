@@ -348,3 +348,16 @@ def test_split_workspace_of_a_launch():
     assert lib.fmoe_linear_dev_workspace_bytes(4096, _lib.BF16) == cus * 3 // 2 * tile(256, 256)
     assert lib.fmoe_linear_dev_workspace_bytes(4096, _lib.F32) == cus * tile(256, 256)
     assert lib.fmoe_linear_dev_workspace_bytes(1024, _lib.BF16) == 0
+
+
+def test_sorted_rows_are_asked_for_by_the_activation_too(monkeypatch):
+    """Where the first product reads sorted rows depends on what its kernel is built for: the polynomial GELU with and
+    without its pre-activation and ReLU without, not the erf formula and not "none" with something to store."""
+    lib = _lib.load()
+    ask = lambda act, pre: lib.fmoe_linear_act_dev_reads_rows(65536, 8, 4096, 14336, _lib.BF16, act, pre)
+    assert ask(_lib.ACT_GELU, 1) == ask(_lib.ACT_GELU, 0) == ask(_lib.ACT_RELU, 0) == ask(_lib.ACT_NONE, 0) == 1
+    assert ask(_lib.ACT_RELU, 1) == ask(_lib.ACT_NONE, 1) == 0
+    assert lib.fmoe_linear_dev_reads_rows(65536, 8, 4096, 14336, _lib.BF16) == 1
+    monkeypatch.setenv("FMOE_GELU_ERF", "1")
+    assert ask(_lib.ACT_GELU, 1) == ask(_lib.ACT_GELU, 0) == 0
+    assert ask(_lib.ACT_RELU, 0) == 1
