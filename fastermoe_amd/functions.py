@@ -105,10 +105,13 @@ class GateLinearTopK(Function):
 
 
 def _plain_linear(linear):
-    """Whether calling ``linear`` is ``F.linear`` on its parameters and nothing else."""
+    """Whether calling ``linear`` is ``F.linear`` on its parameters and nothing else: no hook of its own, and none for
+    all modules (profilers and debuggers register those)."""
+    every = torch.nn.modules.module
     return (type(linear) is torch.nn.Linear and "forward" not in linear.__dict__
             and not (linear._forward_hooks or linear._forward_pre_hooks or linear._backward_hooks
-                     or linear._backward_pre_hooks))
+                     or linear._backward_pre_hooks or every._global_forward_hooks or every._global_forward_pre_hooks
+                     or every._global_backward_hooks or every._global_backward_pre_hooks))
 
 
 def gate_linear_topk(x, linear, top_k, score_mode=0):

@@ -471,3 +471,26 @@ def test_naive_gate_backward_can_be_differentiated_again(n_expert, device):
     picked = torch.zeros(70, n_expert, dtype=torch.float64).scatter_(1, idx.cpu().view(70, 2), 1.0)
     (picked @ w).square().sum().backward()
     assert torch.allclose(gate.gate.weight.grad.double().cpu(), w.grad, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("own", [True, False])
+def test_hooks_see_the_linear_layer_of_a_gate_of_many_experts(own, device):
+    """A forward hook on the gate's linear layer, or one for all modules, is called with its logits, as before the gate of
+    more than 64 experts took the layer's parameters straight."""
+    from fastermoe_amd.gates import NaiveGate
+    torch.manual_seed(8)
+    gate = NaiveGate(64, 100, 1, top_k=2).to(device)
+    x = torch.randn(30, 64, device=device)
+    seen = []
+
+    def hook(module, args, out):
+        if module is gate.gate:
+            seen.append(out.detach().clone())
+
+    handle = (gate.gate.register_forward_hook(hook) if own
+              else torch.nn.modules.module.register_module_forward_hook(hook))
+    try:
+        idx, val = gate(x)
+    finally:
+        handle.remove()
+    assert len(seen) == 1 and torch.equal(seen[0].gather(1, idx.view(30, 2)), val)
