@@ -34,6 +34,15 @@ def _as_chunks(t):
     return t if _whole_chunks(t) else t.clone(memory_format=torch.contiguous_format)
 
 
+def _attach_route(idx, n_expert, counts, pos_buf, slot_to_row, table=None):
+    """Leaves the routing (and segment table) of a gate's indices on them for :func:`_route_launch`, with the version of
+    the tensor that they are of.  Tensors made under ``torch.inference_mode`` count no versions, so a later write to
+    them would go unseen: those are routed anew."""
+    if not idx.is_inference():
+        idx._fmoe_route = (idx._version, n_expert, counts, pos_buf, slot_to_row)
+        idx._fmoe_table = table
+
+
 class GateTopK(Function):
     r"""``torch.topk`` of the gate logits (and, with ``score_mode`` 1, the softmax over the selected
     logits) of fmoe/gates/naive_gate.py:26-42 with the routing of ``count_by_gate`` computed in
@@ -48,8 +57,7 @@ class GateTopK(Function):
         ctx.save_for_backward(idx, score)
         ctx.moe_args = logits.shape[1], score_mode
         ctx.mark_non_differentiable(idx)
-        idx._fmoe_route = (idx._version, logits.shape[1], cnt, pos_buf, s2r)
-        idx._fmoe_table = table
+        _attach_route(idx, logits.shape[1], cnt, pos_buf, s2r, table)
         return idx, score
 
     @staticmethod
@@ -79,8 +87,7 @@ class GateLinearTopK(Function):
         ctx.save_for_backward(x, weight, idx, score)
         ctx.moe_args = score_mode, bias is not None
         ctx.mark_non_differentiable(idx)
-        idx._fmoe_route = (idx._version, weight.shape[0], cnt, pos_buf, s2r)
-        idx._fmoe_table = table
+        _attach_route(idx, weight.shape[0], cnt, pos_buf, s2r, table)
         return idx, score
 
     @staticmethod
@@ -147,7 +154,7 @@ class NoisyTopK(Function):
         ctx.save_for_backward(clean, raw, noise, idx, gates, thr_val, thr_idx)
         ctx.moe_args = top_k, eps
         ctx.mark_non_differentiable(idx)
-        idx._fmoe_route = (idx._version, clean.shape[1], cnt, pos_buf, s2r)
+        _attach_route(idx, clean.shape[1], cnt, pos_buf, s2r)
         return idx, gates, load
 
     @staticmethod

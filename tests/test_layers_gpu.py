@@ -1164,3 +1164,28 @@ def test_decoding_takes_no_split_workspace(device):
         torch.cuda.reset_peak_memory_stats(device)
         moe(x)
     assert torch.cuda.max_memory_allocated(device) - before < 1 << 20
+
+
+@pytest.mark.parametrize("gate", [NaiveGate, NoisyGate, SwitchGate])
+@pytest.mark.parametrize("e", [8, 100])
+@pytest.mark.parametrize("fuse", [False, True])
+def test_inference_mode(gate, e, fuse, device):
+    """Under torch.inference_mode, whose tensors count no versions, a layer gives what it gives under no_grad; indices that
+    are changed in place between gate and experts are routed as they are then."""
+    torch.manual_seed(e)
+    k = 2 if gate is NaiveGate else 1
+    with device:
+        moe = fmoe.FMoETransformerMLP(num_expert=e, d_model=64, d_hidden=128, top_k=k, gate=gate).eval()
+    moe.enable_fuse = fuse
+    x = torch.randn(200, 64, device=device)
+
+    def swap(idx, score, _):   # expert 0's tokens to expert 1 and back
+        idx.copy_(torch.where(idx == 0, 1, torch.where(idx == 1, 0, idx)))
+
+    for hook in (None, swap):
+        moe.gate_hook = hook
+        with torch.no_grad():
+            want = moe(x)
+        with torch.inference_mode():
+            got = moe(x)
+        assert torch.equal(got, want)
