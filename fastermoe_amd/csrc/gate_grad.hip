@@ -128,7 +128,15 @@ __global__ __launch_bounds__(kBlock) void gate_wgrad_kernel(const T *__restrict_
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lb = lane & 15, hq = lane >> 4;
     const int c0 = blockIdx.x * kCols;
     const int lo = blockIdx.y * tokens_per_range, hi = min(n_tokens, lo + tokens_per_range);
-    const bool with_bias = part_b != nullptr && blockIdx.x == 0 && wave == 0;
+    // The bias gradient, in the workgroups of the first columns.  16-bit types: one more column of products in the first
+    // wave.  float32: the rows of the LDS tile are added in double, as a chain of products over a long range is further from the
+    // exact sum than what it replaces (32768 tokens that all name 4 experts, relative error 1.0e-6; as one more
+    // pass of torch's sum over the dense gradient 7.7e-8; added like this 2.9e-8); lane and wave are expert and part of the tokens.
+    constexpr bool kWideBias = sizeof(T) == 4;
+    constexpr int kBiasExperts = EB <= 4 ? 64 : EB * 16, kBiasParts = kBlock / kBiasExperts, kBiasTok = kTok / kBiasParts;
+    const bool bias_wg = part_b != nullptr && blockIdx.x == 0, with_bias = !kWideBias && bias_wg && wave == 0;
+    const int bias_e = t % kBiasExperts, bias_part = t / kBiasExperts;
+    double bias_sum = 0.;
 
     for (int i = t; i < EB * 16 * kGS; i += kBlock) gt[i] = (T)0.f;
     f32x4 acc[EB][2], bacc[EB];
@@ -238,7 +246,13 @@ __global__ __launch_bounds__(kBlock) void gate_wgrad_kernel(const T *__restrict_
                     const float a = gf[(e * 16 + lb) * kGS + k];
                     acc[e][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b0, acc[e][0], 0, 0, 0);
                     acc[e][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b1, acc[e][1], 0, 0, 0);
-                    if (with_bias) bacc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, 1.f, bacc[e], 0, 0, 0);
+                }
+            }
+            if (bias_wg && bias_e < EB * 16) {
+#pragma unroll
+                for (int k = 0; k < kBiasTok; k += 4) {
+                    const f32x4 v = *(const f32x4 *)(gf + bias_e * kGS + bias_part * kBiasTok + k);
+                    bias_sum += ((double)v[0] + (double)v[1]) + ((double)v[2] + (double)v[3]);
                 }
             }
         }
@@ -261,9 +275,20 @@ __global__ __launch_bounds__(kBlock) void gate_wgrad_kernel(const T *__restrict_
             }
             if (with_bias && lb == 0) part_b[(int64_t)blockIdx.y * n_expert + ex] = bacc[e][i];
         }
+    if (kWideBias && bias_wg) {   // (uniform over the workgroup; the tiles were last read before the barrier that ends the loop)
+        double *sums = (double *)lds;   // [kBiasParts][kBiasExperts]
+        sums[t] = bias_sum;
+        __syncthreads();
+        if (t < kBiasExperts && t < n_expert) {
+#pragma unroll
+            for (int q = 1; q < kBiasParts; ++q) bias_sum += sums[q * kBiasExperts + t];
+            part_b[(int64_t)blockIdx.y * n_expert + t] = (float)bias_sum;
+        }
+    }
 }
 
-// adds the ranges' sums in ascending order: elements [0, n_w) are grad_w's, the n_b after them grad_b's
+// adds the ranges' sums in ascending order (float32 results: in double): elements [0, n_w) are grad_w's, the n_b after
+// them grad_b's
 template <typename T>
 __global__ __launch_bounds__(kBlock) void gate_wgrad_reduce_kernel(const float *__restrict__ part_w, const float *__restrict__ part_b,
                                                                    T *__restrict__ grad_w, T *__restrict__ grad_b, int64_t n_w,
@@ -272,13 +297,17 @@ __global__ __launch_bounds__(kBlock) void gate_wgrad_reduce_kernel(const float *
     if (i >= n_w + n_b) return;
     const float *src = i < n_w ? part_w + i : part_b + (i - n_w);
     const int64_t step = i < n_w ? n_w : n_b;
-    float sum = 0.f;
+    typename std::conditional<sizeof(T) == 4, double, float>::type sum = 0;
     for (int r0 = 0; r0 < ranges; r0 += 8) {
         float v[8];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) v[r] = r0 + r < ranges ? src[(int64_t)(r0 + r) * step] : 0.f;
+        for (int r = 0; r < 8; ++r) v[r] = src[(int64_t)min(r0 + r, ranges - 1) * step];
+        // (the eight loads are out before the first is waited for: with the conversion to double at each, or a condition around
+        // it, they go one by one, 19 us instead of 5 for 64 ranges)
 #pragma unroll
-        for (int r = 0; r < 8; ++r) sum += v[r];
+        for (int r = 0; r < 8; ++r) asm volatile("" : "+v"(v[r]));
+#pragma unroll
+        for (int r = 0; r < 8; ++r) sum += r0 + r < ranges ? v[r] : 0.f;
     }
     if (i < n_w) grad_w[i] = (T)sum;
     else grad_b[i - n_w] = (T)sum;
