@@ -8,15 +8,37 @@ namespace segtab {
 
 constexpr int kThreads = 1024;        // the workgroup that builds a table
 constexpr int kSmallExperts = 1024;   // most experts of small_table(): one per thread
+constexpr int kRankExperts = 192;     // most experts that are ordered by counting
 
 // LDS of small_table(): the three prefixes and the waves' sums
 struct SmallLds {
     int64_t row_sum[kThreads / kWave];
     int32_t wave_sum[2][kThreads / kWave];
     int32_t seg[kSmallExperts + 1];
-    int32_t pfx[2][kSmallExperts + 1];
+    __attribute__((aligned(8))) int32_t pfx[2][kSmallExperts + 1];   // (afterwards the exchange buffer of sort_descending)
     __attribute__((aligned(16))) int32_t rows[kSmallExperts];
 };
+
+// Sorts the workgroup's keys, one per thread, among its first n threads (a power of two of at least 64): thread i ends with the
+// i-th largest.  A bitonic network; partners in the same wave exchange by lane, others through buf [kThreads].
+__device__ __forceinline__ uint64_t sort_descending(uint64_t key, int n, uint64_t *buf) {
+    const int i = threadIdx.x;
+    for (int k = 2; k <= n; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            uint64_t other;
+            if (j < kWave) {
+                other = (uint64_t)__shfl_xor((unsigned long long)key, j, kWave);
+            } else {
+                buf[i] = key;
+                __syncthreads();
+                other = buf[i ^ j];
+                __syncthreads();
+            }
+            const bool keep_larger = ((i & j) == 0) == ((i & k) == 0);
+            key = (key > other) == keep_larger ? key : other;
+        }
+    return key;
+}
 
 // The whole table for at most kSmallExperts experts by one workgroup of kThreads threads, thread e
 // holding expert e's row count (others: anything).  The counts are clamped so that their sum never
@@ -98,15 +120,29 @@ __device__ __forceinline__ void small_table(int64_t count, int n_expert, int row
             *(int4 *)(map + 4 * (int64_t)i) = entry;
         }
     }
-    // the experts by descending rows: expert e's place is the number of experts that come before it
-    if (e < n_expert) {
+    // The experts by descending rows.  Up to kRankExperts an expert's place is counted, the number of experts that come
+    // before it; beyond, where the square of their number tells, the experts are sorted.  The whole table, counted and
+    // sorted: 129 experts 8.5 / 10.0 us, 256: 11.8 / 10.1, 512: 19.6 / 11.6, 1024: 44.6 / 13.8.
+    int4 *order = (int4 *)(tab + order_off(rows_cap, n_expert));
+    if (n_expert > kRankExperts) {
+        __syncthreads();   // the maps are done with lds.pfx
+        int n = kWave;
+        while (n < n_expert) n <<= 1;
+        // (of equal rows the lower expert first; threads without an expert sort last)
+        const uint64_t mine = e < n_expert ? ((uint64_t)(uint32_t)rows << 32) | (0xffffffffu - (uint32_t)e) : 0;
+        const uint64_t key = sort_descending(mine, n, (uint64_t *)&lds.pfx[0][0]);
+        if (e < n_expert) {
+            const int ex = (int)(0xffffffffu - (uint32_t)key);
+            order[e] = make_int4(ex, lds.seg[ex], (int)(key >> 32), 0);
+        }
+    } else if (e < n_expert) {
         int place = 0;
         for (int f = 0; f < n_expert; f += 4) {
             const int4 r = *(const int4 *)(lds.rows + f);
             place += (r.x > rows || (r.x == rows && f < e)) + (r.y > rows || (r.y == rows && f + 1 < e)) +
                      (r.z > rows || (r.z == rows && f + 2 < e)) + (r.w > rows || (r.w == rows && f + 3 < e));
         }
-        *(int4 *)(tab + order_off(rows_cap, n_expert) + 4 * (int64_t)place) = make_int4(e, (int)lo, rows, 0);
+        order[place] = make_int4(e, (int)lo, rows, 0);
     }
 }
 

@@ -377,3 +377,25 @@ def test_float32_tiles_of_64(counts, fin, fout, device, monkeypatch):
     assert rel_err(pre, ref) <= tol and rel_err(y, torch.nn.functional.gelu(ref)) <= tol
     assert rel_err(gx, x64.grad) <= tol and rel_err(gx_act, x64.grad * (pre_in > 0)) <= tol
     assert rel_err(gw, w64.grad) <= tol and rel_err(gb, b64.grad) <= tol
+
+
+@pytest.mark.parametrize("n_expert", [1, 2, 63, 64, 65, 255, 256, 257, 300, 512, 513, 1023, 1024, 1025, 1300])
+@pytest.mark.parametrize("kind", ["random", "equal", "few", "ascending"])
+def test_order_of_the_experts_by_their_rows(n_expert, kind, device):
+    """The table's list of {expert, first row, rows} in descending order of the rows, of equal ones the lower expert first;
+    beyond 1024 experts in expert order.  From the stand-alone table and from the one of a routing call: exact."""
+    g = torch.Generator().manual_seed(n_expert)
+    counts = {"random": torch.randint(0, 40, (n_expert,), generator=g), "equal": torch.full((n_expert,), 3),
+              "few": (torch.rand(n_expert, generator=g) < 0.05).long() * 7, "ascending": torch.arange(n_expert) % 50}[kind]
+    gate = torch.repeat_interleave(torch.arange(n_expert), counts)
+    gate = gate[torch.randperm(gate.numel(), generator=g)]
+    slots = gate.numel() + 1
+    gate = torch.cat([gate, torch.tensor([-1])])
+    first = np.concatenate([[0], np.cumsum(counts.numpy())[:-1]])
+    experts = sorted(range(n_expert), key=lambda e: (-int(counts[e]), e)) if n_expert <= 1024 else list(range(n_expert))
+    want = [(e, int(first[e]), int(counts[e]), 0) for e in experts]
+    for table in (fmoe_native.segment_table(counts.to(device), slots), fmoe_native.route_table(gate.to(device), n_expert)[3]):
+        t = table.cpu().numpy()
+        # (behind the map of the 128-row tiles, laid out for the most there can be)
+        at = int(t[5]) + 4 * (slots // 128 + min(n_expert, slots))
+        assert [tuple(r) for r in t[at:at + 4 * n_expert].reshape(-1, 4).tolist()] == want
