@@ -16,7 +16,7 @@
 //   * the tiles are dealt to the workgroups beforehand: row-ragged products in bands of row
 //     tiles shared by the XCDs; the weight gradient expert by expert in descending order of their rows (the table's
 //     order list), back and forth over the workgroups, so that every workgroup gets its share of long and
-//     short contractions;
+//     short contractions, and by cost where that leaves them uneven (ring_deal);
 //   * the bias gradient is one more column of products (a block of ones times the output gradient).
 #pragma once
 #include "gemm_kernel.hpp"
@@ -124,6 +124,128 @@ constexpr int kRingSlab = kRingTile * kSlabBytes;   // 32 KiB
 constexpr int kRingPBufs = 3, kRingQBase = kRingPBufs * kRingSlab;
 constexpr int kRingLds = (kRingPBufs + 2) * kRingSlab;
 typedef int ring_i32x4 __attribute__((ext_vector_type(4)));
+
+// How the tiles of a weight gradient are dealt: `rounds` back-and-forth rounds over all workgroups, then the `count` tiles from
+// `first` on (rounds == 0: rounds alone).
+struct RingDeal {
+    int rounds, first, count;
+};
+constexpr int kDealTileCost = 3;   // what a tile costs beside its slabs, in slabs (its epilogue, 4 to 5 us)
+constexpr int kDealSpread = 16;    // slabs by which the first round's tiles have to differ: planning takes 5 to 8 us, four or five slabs
+constexpr int kDealRounds = 8;     // most rounds before the rest is dealt by cost
+constexpr int kDealExperts = 1024, kDealGroups = 512;   // most experts and workgroups it is planned for
+__device__ __forceinline__ int ring_tile_cost(int rows) { return max(1, (rows + 63) >> 6) + kDealTileCost; }
+// tile of a back-and-forth round
+__device__ __forceinline__ int ring_zigzag(int round, int grid, int w) { return round * grid + ((round & 1) ? grid - 1 - w : w); }
+struct DealLds {
+    int cost[kDealExperts], pre[kDealExperts + 1];     // per expert of the order list, and its exclusive prefix
+    int wave_sum[8], round_max[kDealRounds + 1][8];    // (the last: all rounds)
+    int64_t wave_room[8], room[kDealGroups + 1];       // exclusive prefix of what the workgroups are below the mean
+};
+
+// Rounds alone give every workgroup as many tiles as any other, and where some experts have much more rows than the rest and
+// few tiles (fewer than there are workgroups, so that the first round mixes long tiles with short ones) the workgroups with the
+// long ones finish last.  There the first rounds, as many as make the longest list shortest, are followed by runs of
+// the remaining tiles cut by cost, for each workgroup as long as its rounds are below the mean.  us with one workgroup
+// per tile / rounds alone / this: 64 experts of 1456 x 1256, 12926 rows by a Zipf law: 143 / 157 / 133; 16 of 1472 x 2944,
+// 75724: 651 / 776 / 632; 128 of 640 x 2560, 14719: 193 / 207 / 181; 32 of 544 x 8040, all 39094 rows in one: 773 / 889 / 773.
+// Every workgroup plans the whole launch from the table, with the same numbers.  Simulated over sizes and
+// routings, the longest list is 1.05 times the mean (or the longest tile) on average; 1.15 with rounds alone, 1.03 if
+// every tile went to the least loaded workgroup.
+__device__ __forceinline__ RingDeal ring_deal(const RingParams &prm, int tiles_per_expert, int total, int grid, int w, DealLds &lds) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, n = prm.n_expert;
+    const int rounds = total / grid, rest = total - rounds * grid;
+    const RingDeal rounds_alone{0, 0, 0};
+    const int *order = prm.dev_tab + prm.dev_order_off;   // {expert, first row, rows, 0}
+    for (int e = t; e < n; e += 512) lds.cost[e] = ring_tile_cost(order[4 * e + 2]);
+    __syncthreads();
+    // thread t: the prefix up to experts 2 t and 2 t + 1
+    const int c0 = 2 * t < n ? lds.cost[2 * t] : 0, c1 = 2 * t + 1 < n ? lds.cost[2 * t + 1] : 0;
+    int v = c0 + c1;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int up = __shfl_up(v, off, 64);
+        if (lane >= off) v += up;
+    }
+    if (lane == 63) lds.wave_sum[wave] = v;
+    // thread t: the list of workgroup t
+    int load = 0;
+    for (int k = 0; k <= rounds; ++k) {
+        if (t < grid && (k < rounds || ring_zigzag(k, grid, t) < total)) load += lds.cost[ring_zigzag(k, grid, t) / tiles_per_expert];
+        if (k < kDealRounds || k == rounds) {
+            int m = load;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) m = max(m, __shfl_xor(m, off, 64));
+            if (lane == 0) {
+                if (k < kDealRounds) lds.round_max[k][wave] = m;
+                if (k == rounds) lds.round_max[kDealRounds][wave] = m;
+            }
+        }
+    }
+    __syncthreads();
+    for (int u = 0; u < wave; ++u) v += lds.wave_sum[u];
+    if (2 * t <= n) lds.pre[2 * t] = v - c0 - c1;
+    if (2 * t + 1 <= n) lds.pre[2 * t + 1] = v - c1;
+    if (t == 511 && n == kDealExperts) lds.pre[n] = v;
+    __syncthreads();
+    const int64_t all = (int64_t)lds.pre[n] * tiles_per_expert;
+    const int mean = (int)((all + grid - 1) / grid);
+    auto longest = [&](int k) {
+        int m = 0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) m = max(m, lds.round_max[k][u]);
+        return m;
+    };
+    int best = INT32_MAX, k_best = 0;
+    for (int k = 1; k <= kDealRounds && k * grid < total; ++k) {
+        const int est = max(longest(k - 1), mean + lds.cost[k * grid / tiles_per_expert] / 2);
+        if (est < best) {
+            best = est;
+            k_best = k;
+        }
+    }
+    // (by a sixteenth at least: runs by cost share less of their operands than rounds do)
+    if (k_best == 0 || (int64_t)longest(kDealRounds) * 16 <= (int64_t)best * 17) return rounds_alone;
+    // what each workgroup is below the mean after k_best rounds, and its prefix
+    int64_t room = 0;
+    if (t < grid) {
+        int have = 0;
+        for (int k = 0; k < k_best; ++k) have += lds.cost[ring_zigzag(k, grid, t) / tiles_per_expert];
+        room = max(0, mean - have);
+    }
+    int64_t r = room;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int64_t up = __shfl_up((long long)r, off, 64);
+        if (lane >= off) r += up;
+    }
+    if (lane == 63) lds.wave_room[wave] = r;
+    __syncthreads();
+    for (int u = 0; u < wave; ++u) r += lds.wave_room[u];
+    lds.room[t + 1] = r;
+    if (t == 0) lds.room[0] = 0;
+    __syncthreads();
+    const int n0 = k_best * grid;
+    const int64_t base = (int64_t)lds.pre[n0 / tiles_per_expert] * tiles_per_expert +
+                         (int64_t)lds.cost[n0 / tiles_per_expert] * (n0 % tiles_per_expert);
+    const int64_t total_room = lds.room[grid], left = all - base;
+    const double scale = (double)left / (double)total_room;
+    // the first tile whose middle lies at or past the cost that belongs to `room` (the same number on both sides of a border)
+    auto first_tile = [&](int64_t room_before) {
+        const int64_t at = base + (room_before == total_room ? left : (int64_t)((double)room_before * scale));
+        int lo = 0, hi = n;   // pre[lo] <= at / tiles_per_expert < pre[hi]
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if ((int64_t)lds.pre[mid] * tiles_per_expert <= at) lo = mid; else hi = mid;
+        }
+        const int c = lds.cost[lo];
+        const int64_t past = 2 * at - c - 2 * (int64_t)lds.pre[lo] * tiles_per_expert;
+        const int64_t i = past <= 0 ? 0 : (past + 2 * c - 1) / (2 * c);
+        return max(n0, lo * tiles_per_expert + (int)min(i, (int64_t)tiles_per_expert));
+    };
+    const int first = first_tile(lds.room[w]), end = w == grid - 1 ? total : first_tile(lds.room[w + 1]);
+    return RingDeal{k_best, first, max(0, end - first)};
+}
 
 // acc[x][y][i] is C(row 64 wm + 16 y + lb, column 128 wn + 16 x + 4 hq + i).  Sixteen rows at a time go
 // through 4 KiB of LDS (16-byte chunk c of row r at c ^ r) and out as whole 256-byte row pieces.
@@ -253,6 +375,8 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_ring_kernel(const R
     int n_items, tm_total;
     RingPlan plan{0, 0, 0};
     int run_lo = 0, run_hi = 0, k_slabs = 0;   // this workgroup's run of the tail's slabs
+    RingDeal deal{INT32_MAX, 0, 0};
+    int deal_w = xcd * per + slot;   // this workgroup's place in the dealing
     if (RAGGED == kRaggedRows) {
         tm_total = dtab[segtab::kTiles256];
         k_slabs = (prm.k_extent + BKE - 1) / BKE;
@@ -272,10 +396,30 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_ring_kernel(const R
     } else {
         tm_total = prm.tiles_m;
         const int total = prm.n_expert * prm.tiles_m * prm.tiles_n, grid = gridDim.x;
-        const int fwd = xcd * per + slot;
         const int rounds = uniform(total / grid), rest = total - rounds * grid;
-        const int last = (rounds & 1) ? grid - 1 - fwd : fwd;
-        n_items = rounds + (last < rest ? 1 : 0);
+        n_items = rounds + (ring_zigzag(rounds, grid, deal_w) < total ? 1 : 0);
+        if (rounds > 0 && rest + rounds > 1 && prm.n_expert <= kDealExperts && grid <= kDealGroups) {
+            // rounds alone are level enough where the first one is: its first and last tile differ by less than a sixteenth of a list
+            const int tpe = prm.tiles_m * prm.tiles_n;
+            const int longest = ring_tile_cost(dtab[prm.dev_order_off + 2]);
+            const int shortest = ring_tile_cost(dtab[prm.dev_order_off + 4 * uniform((grid - 1) / tpe) + 2]);
+            const float list = ((float)dtab[segtab::kRows] / 64.f + (kDealTileCost + 0.5f) * (float)prm.n_expert) * (float)tpe / (float)grid;
+            const int spread = uniform(longest) - uniform(shortest);
+            if (spread >= kDealSpread && (float)spread * 16.f > list) {
+                // (eight tiles in a row to an XCD, which share operands, then the next: as many long tiles as one expert has
+                // would otherwise all be on one or two XCDs, the 64 experts of ring_deal's comment 150 us instead of 133)
+                const int chunk = per % 8 == 0 ? 8 : 1;
+                const int w = (slot / chunk) * (8 * chunk) + xcd * chunk + slot % chunk;
+                const RingDeal planned = ring_deal(prm, tpe, total, grid, w, *(DealLds *)smem);
+                if (uniform(planned.rounds) > 0) {
+                    deal_w = uniform(w);
+                    deal.rounds = uniform(planned.rounds);
+                    deal.first = uniform(planned.first);
+                    n_items = deal.rounds + uniform(planned.count);
+                }
+                __syncthreads();   // the plan is read; the slabs take its place
+            }
+        }
     }
     if (n_items == 0) return;
 
@@ -300,8 +444,8 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_ring_kernel(const R
                 tl.ws_slot = ring_ws_slot(xcd, per, slot, tail_tile);
             }
         } else {
-            const int grid = gridDim.x, fwd = xcd * per + slot, tpe = prm.tiles_m * prm.tiles_n;
-            const int q = r * grid + ((r & 1) ? grid - 1 - fwd : fwd);
+            const int grid = gridDim.x, tpe = prm.tiles_m * prm.tiles_n;
+            const int q = r < deal.rounds ? ring_zigzag(r, grid, deal_w) : deal.first + (r - deal.rounds);
             ei = uniform(q / tpe);
             rem = q - ei * tpe;
             entry = *(DevTab4)(dtab + prm.dev_order_off + 4 * ei);

@@ -399,3 +399,44 @@ def test_order_of_the_experts_by_their_rows(n_expert, kind, device):
         # (behind the map of the 128-row tiles, laid out for the most there can be)
         at = int(t[5]) + 4 * (slots // 128 + min(n_expert, slots))
         assert [tuple(r) for r in t[at:at + 4 * n_expert].reshape(-1, 4).tolist()] == want
+
+
+UNEVEN = [  # experts, in, out, rows, routing: weight gradients whose tiles are dealt by cost, and some on either side of that rule
+    (64, 1456, 1256, 12926, "zipf"),
+    (32, 544, 8040, 3000, "one"),
+    (512, 264, 512, 9000, "few"),
+    (1024, 520, 256, 20000, "zipf"),
+    (1030, 256, 264, 5000, "zipf"),       # (more experts than the plan takes)
+    (8, 2600, 2600, 20000, "zipf"),
+    (16, 1296, 1800, 700, "one"),
+    (513, 256, 256, 30000, "one"),        # one tile per expert
+    (9, 2048, 2048, 3000, "even"),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("e,fin,fout,rows,routing", UNEVEN)
+def test_weight_gradient_of_uneven_experts(e, fin, fout, rows, routing, dtype, device):
+    """Every tile of the weight gradient is computed once, however the tiles are dealt to the persistent workgroups: into memory
+    that held NaN before, against float32 products, with the bound of the persistent kernel's other products."""
+    g = torch.Generator().manual_seed(e + rows)
+    p = {"zipf": torch.arange(1, e + 1).float() ** -1.2, "one": (torch.arange(e) == e // 3).float(),
+         "few": (torch.arange(e) % 37 == 5).float(), "even": torch.ones(e)}[routing]
+    counts = torch.bincount(torch.multinomial(p[torch.randperm(e, generator=g)], rows, replacement=True, generator=g), minlength=e)
+    slots = rows + 3
+    gd = torch.Generator(device=device).manual_seed(e)
+    x = torch.randn(slots, fin, device=device, generator=gd).to(dtype)
+    gy = torch.randn(slots, fout, device=device, generator=gd).to(dtype)
+    weight = torch.empty(e, fout, fin, dtype=dtype, device=device)
+    table = fmoe_native.segment_table(counts.to(device), slots)
+    for size in ((e, fout, fin), (e, fout)):
+        torch.full(size, float("nan"), dtype=dtype, device=device)   # (freed at once: the next tensor of this size takes its place)
+    gw, gb = fmoe_native.linear_wgrad_dev(gy, x, weight, table, slots, True)
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    lo = 0
+    for ex, n in enumerate(counts.tolist()):
+        gs, xs = gy[lo:lo + n].float(), x[lo:lo + n].float()
+        lo += n
+        for got, ref in ((gw[ex], gs.t() @ xs), (gb[ex], gs.sum(dim=0))):
+            bound = eps * ref.abs() + 1e-3 * ref.pow(2).mean().sqrt() if n else torch.zeros_like(ref)
+            assert bool(((got.float() - ref).abs() <= bound).all()), f"expert {ex} with {n} rows"
