@@ -130,9 +130,9 @@ TileShape f32_rows_tile(int64_t tiles_256, int64_t contraction) {
 // 2112 x 4224, 3072: 630 / 622 / 657.
 TileShape f32_wgrad_tile(int64_t experts, int64_t out_feat, int64_t in_feat, int64_t rows) {
     if (experts * ceil_div(out_feat, 256) * ceil_div(in_feat, 256) >= 640 && rows < 48 * experts) return {256, 256};
-    constexpr int64_t kUnits = 256;
-    const int64_t low = ceil_div(experts * ceil_div(out_feat, 64) * ceil_div(in_feat, 64), kUnits) * 64 * 64;
-    const int64_t high = ceil_div(experts * ceil_div(out_feat, 128) * ceil_div(in_feat, 128), kUnits) * 128 * 128;
+    const int64_t units = device_compute_units();
+    const int64_t low = ceil_div(experts * ceil_div(out_feat, 64) * ceil_div(in_feat, 64), units) * 64 * 64;
+    const int64_t high = ceil_div(experts * ceil_div(out_feat, 128) * ceil_div(in_feat, 128), units) * 128 * 128;
     return 105 * low < 100 * high ? TileShape{64, 64} : TileShape{128, 128};
 }
 
