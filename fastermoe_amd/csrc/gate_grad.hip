@@ -5,8 +5,8 @@
 // it, those entries are written into a dense [tokens, experts] matrix and go through two library products a few columns wide, two
 // reductions for the bias and one more pass over the input gradient to add the gate's part:
 //   grad_x[t] = experts' part + sum_j g[t,j] w[idx[t,j]]      grad_w[e] = sum over (t,j) with idx = e of g[t,j] x[t]
-// Here the first is a sum of top_k rows of w per token (the gate's own node; a caller that has the experts' part as rows
-// too gets both sums in one pass), and the second is one pass over x with the matrix cores.
+// Here the gate's part of the first is a sum of top_k rows of w per token (a caller that has the experts' part as rows gets
+// both sums in one pass; the layer does not call it so), and the second is one pass over x with the matrix cores.
 #include "common.hpp"
 #include "profile.hpp"
 #include "vec16.hpp"
@@ -25,9 +25,12 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 // ---- input gradient: reduce_slots plus the gate's part ---------------------------------------
 // A wave owns P pieces of 64 vectors (1 KiB) of one token's row and has all K P loads of rows and of w in flight together: the
-// slots' rows and experts are a dependent load before them, and with one piece per wave that latency was
-// the bound (32768 tokens of 4096 in bf16, top-2: 255 us with P = 1 and vector index loads, 153 with P = 4 and scalar ones, against
-// 137 for reduce_slots alone; w's rows come from the caches).  The two library steps it stands for took 99 (product) and 120 us (sum).
+// slots' experts (and rows) are a dependent load before them, scalar ones as they are the same for the wave, and w's rows come
+// from the caches.  The gate's node asks for its part alone (rows null), the sum with the experts' rows is for callers
+// that have them.  us for the gate's part with P = 1 / 2 / 4 (and with the rows, against reduce_slots alone): bf16, 32768 tokens of
+// 4096, 8 experts, top-2: 73 / 62 / 69 (147 / 141 / 150, 133), 16384 of 2048, 64 experts, top-1: 15.0 / 12.3 / 12.8
+// (27.9 / 25.5 / 26.7, 23.5), 16384 of 4096, top-4: 55 / 54 / 64; float32, 32768 of 4096, top-2: 115 / 87 / 81, top-4 at 16384:
+// 87 / 71 / 84.  As a library product over the dense gradient the first took 99.
 // Tokens or rows too few for that many waves take P = 1.
 template <typename T, int K, int P>
 __global__ __launch_bounds__(kBlock) void reduce_slots_gate_kernel(
@@ -85,7 +88,7 @@ template <typename T, int K>
 int launch_reduce_gate(const void *rows, const int64_t *slot_to_row, const void *grad_score, const int64_t *topk_idx, const void *w,
                        void *out, int64_t n_tokens, int64_t top_k, int64_t n_rows, int64_t n_expert, int64_t row_vecs,
                        hipStream_t st) {
-    constexpr int kPieces = K >= 8 ? 1 : K == 1 ? 4 : 8 / K;
+    constexpr int kPieces = K >= 8 ? 1 : K == 4 || sizeof(T) == 2 ? 2 : 4;
 #define FMOE_RG(P)                                                                                                                    \
     {                                                                                                                                 \
         const int64_t groups = ceil_div(row_vecs, (P) * kWave), blocks = ceil_div(n_tokens * groups, kWavesPerBlock);                  \
@@ -403,7 +406,8 @@ extern "C" int fmoe_reduce_slots_gate(const void *rows, const int64_t *slot_to_r
     FMOE_REQUIRE((row_elems * dtype_bytes(dtype)) % 16 == 0 && aligned16(rows) && aligned16(w) && aligned16(out),
                  "fmoe_reduce_slots_gate: rows must be whole 16-byte chunks");
     hipStream_t st = (hipStream_t)stream;
-    ProfileScope prof(kProfReduceSlots, (double)(top_k + 1) * n_tokens * row_elems * dtype_bytes(dtype), st);
+    // (bytes: the experts' rows and the result; the gate's part alone: its weight, once, and the result)
+    ProfileScope prof(kProfReduceSlots, (double)(slot_to_row ? (top_k + 1) * n_tokens : n_tokens + n_expert) * row_elems * dtype_bytes(dtype), st);
     const int64_t row_vecs = row_elems * dtype_bytes(dtype) / 16;
 #define FMOE_RGT(T, K)                                                                                                            \
     return launch_reduce_gate<T, K>(rows, slot_to_row, grad_score, topk_idx, w, out, n_tokens, top_k, n_rows, n_expert, row_vecs, st)

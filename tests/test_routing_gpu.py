@@ -508,3 +508,63 @@ def test_float32_gate_bias_gradient_keeps_its_precision(n, d, e, k, device):
     _, grad_b = fmoe_native.gate_weight_grad(grad, idx, x, e, True)
     want = torch.zeros(n, e, dtype=torch.float64, device=device).scatter_(1, idx, grad.double()).sum(dim=0)
     assert (grad_b.double() - want).norm() <= 2.0 ** -23 * want.norm()
+
+
+@pytest.mark.parametrize("dtype,n,d,k", [
+    (torch.bfloat16, 8192, 2056, 1), (torch.float16, 8192, 2056, 2), (torch.bfloat16, 4096, 1032, 4),   # two pieces per wave
+    (torch.float32, 8192, 1028, 1), (torch.float32, 8192, 1028, 2),                                     # four
+    (torch.float32, 8192, 516, 4), (torch.bfloat16, 8192, 2056, 8),                                     # two; one
+])
+def test_gate_input_gradient_of_long_rows(dtype, n, d, k, device):
+    """The gate's part of the input gradient where a wave takes several pieces of a row, at row lengths that leave the last wave
+    of a row partly empty, alone and with the experts' rows; tokens that name fewer experts.  Allowed per element: float32
+    sums and the rounding of the result."""
+    e = 16
+    g = torch.Generator(device=device).manual_seed(n + d + k)
+    w, grad = torch.randn(e, d, device=device, generator=g).to(dtype), torch.randn(n, k, device=device, generator=g).to(dtype)
+    idx = torch.rand(n, e, device=device, generator=g).topk(k, dim=1).indices
+    idx[::7, k - 1] = -1
+    rows = torch.randn(n * k, d, device=device, generator=g).to(dtype)
+    s2r = torch.randperm(n * k, device=device, generator=g)
+    s2r[::5] = -1
+    out_eps = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -11}[dtype]
+    dense = torch.zeros(n, e + 1, dtype=torch.float64, device=device).scatter_(1, idx + 1, grad.double())[:, 1:].contiguous()
+    part, mag = dense @ w.double(), dense.abs() @ w.double().abs()
+    picked = torch.where((s2r >= 0).unsqueeze(1), rows.double()[s2r.clamp(min=0)], 0.0).view(n, k, d)
+    for got, want, m in ((fmoe_native.reduce_slots_gate(None, None, grad, idx, w), part, mag),
+                         (fmoe_native.reduce_slots_gate(rows, s2r, grad, idx, w), part + picked.sum(1), mag + picked.abs().sum(1))):
+        assert bool(((got.double() - want).abs() <= 2 * out_eps * want.abs() + (2 * k + 1) * 2.0 ** -24 * m + 2.0 ** -25).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,e,k", [(300, 40, 12), (130, 256, 32), (70, 17, 17)])
+def test_gate_weight_gradient_of_many_choices(n, e, k, dtype, device):
+    """More choices per token than the entries that the weight gradient's kernel holds in registers from step to step."""
+    d = 136
+    g = torch.Generator(device=device).manual_seed(k)
+    x, grad = torch.randn(n, d, device=device, generator=g).to(dtype), torch.randn(n, k, device=device, generator=g).to(dtype)
+    idx = torch.rand(n, e, device=device, generator=g).topk(k, dim=1).indices
+    dense = torch.zeros(n, e, dtype=torch.float64, device=device).scatter_(1, idx, grad.double())
+    grad_w, grad_b = fmoe_native.gate_weight_grad(grad, idx, x, e, True)
+    eps = 2.0 ** -24 if dtype == torch.float32 else 2.0 ** -9
+    for got, want, mag in ((grad_w, dense.t() @ x.double(), dense.abs().t() @ x.double().abs()), (grad_b, dense.sum(0), dense.abs().sum(0))):
+        assert bool(((got.double() - want).abs() <= 2 * eps * want.abs() + n * 2.0 ** -24 * mag).all())
+
+
+def test_bytes_booked_for_the_gates_part(device):
+    """The profile counts the rows that a pass reads and writes: not the experts' rows where it is given none."""
+    import ctypes
+    from fastermoe_amd import _lib
+    lib = _lib.load()
+    n, e, d, k = 256, 8, 512, 2
+    w, grad = torch.randn(e, d, device=device), torch.randn(n, k, device=device)
+    idx = torch.rand(n, e, device=device).topk(k, dim=1).indices
+    rows, s2r = torch.randn(n * k, d, device=device), torch.arange(n * k, device=device)
+    classes = lib.fmoe_profile_classes()
+    for args, want in (((None, None), (n + e) * d * 4), ((rows, s2r), (k + 1) * n * d * 4)):
+        launches, ms, work = (ctypes.c_int64 * classes)(), (ctypes.c_double * classes)(), (ctypes.c_double * classes)()
+        _lib.check(lib.fmoe_profile_enable(1))
+        fmoe_native.reduce_slots_gate(*args, grad, idx, w)
+        _lib.check(lib.fmoe_profile_collect(*(ctypes.cast(a, ctypes.c_void_p) for a in (launches, ms, work)), classes))
+        _lib.check(lib.fmoe_profile_enable(0))
+        assert launches[6] == 1 and work[6] == want
