@@ -249,6 +249,7 @@ RING_CASES = [  # counts, in, out
     ([2300, 1900, 0, 3992], 8, 5000),            # one slab of one 16-byte chunk
     ([9000, 300], 4096, 4096),                   # an exact number of slabs; a tail cut along the contraction
     ([0] * 40 + [2, 1] * 30 + [700] * 12, 520, 1040),
+    ([(37 * i) % 211 for i in range(1100)], 264, 520),   # more experts than the table sorts
 ]
 
 

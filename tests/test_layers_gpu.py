@@ -1189,3 +1189,53 @@ def test_inference_mode(gate, e, fuse, device):
         with torch.inference_mode():
             got = moe(x)
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("act", [nn.GELU(), nn.ReLU()])
+@pytest.mark.parametrize("drop", [False, True])
+def test_fused_layer_without_chunks_equals_the_chunked_one(act, drop, device, monkeypatch):
+    """A fused layer whose products run on the persistent kernel leaves the chunked pipeline unless a number of chunks is asked
+    for: same outputs and gradients as with four chunks, with dropped slots and without.  Bound, in 2-norm: either
+    run rounds every value it stores to bfloat16, 2^-8 of it at most, so 2^-7 between the two.  (Not element by element: a
+    ReLU unit whose pre-activation is 1e-7 from zero may fall on either side in another order of the sum, and a
+    weight's gradient then has a term more.)  With the erf formula, which that kernel is not built for, GELU layers
+    keep their chunks."""
+    torch.manual_seed(11)
+    n, d, h, e, k = 4000, 4096, 4352, 6, 2
+    with device:
+        moe = fmoe.FMoETransformerMLP(num_expert=e, d_model=d, d_hidden=h, top_k=k, activation=act)
+    moe = moe.to(torch.bfloat16)
+    moe.enable_fuse = True
+    with torch.no_grad():
+        for lin in (moe.experts.htoh4, moe.experts.h4toh):
+            lin.weight.normal_(0, lin.weight.shape[2] ** -0.5)
+            lin.bias.normal_()
+    if drop:
+        whole = moe.gate.forward
+
+        def some(inp):
+            idx, score = whole(inp)
+            idx = idx.clone()
+            idx[::3, 0] = -1
+            return idx, score
+        moe.gate.forward = some
+    x = torch.randn(n, d, device=device).to(torch.bfloat16)
+    grad = torch.randn(n, d, device=device).to(torch.bfloat16)
+    results = []
+    for chunks in (None, "4"):
+        monkeypatch.delenv("FMOE_FUSE_GRAN", raising=False)
+        if chunks is not None:
+            monkeypatch.setenv("FMOE_FUSE_GRAN", chunks)
+        assert moe.experts.unchunked_is_faster(x, n * k) == (chunks is None)
+        moe.zero_grad(set_to_none=True)
+        leaf = x.clone().requires_grad_(True)
+        out = moe(leaf)
+        out.backward(grad)
+        with torch.no_grad():
+            infer = moe(x)
+        results.append([out.detach(), infer, leaf.grad] + [p.grad for p in moe.parameters()])
+    for a, b in zip(*results):
+        assert (a.float() - b.float()).norm() <= 2.0 ** -7 * b.float().norm()
+    monkeypatch.delenv("FMOE_FUSE_GRAN")
+    monkeypatch.setenv("FMOE_GELU_ERF", "1")
+    assert moe.experts.unchunked_is_faster(x, n * k) == isinstance(act, nn.ReLU)
