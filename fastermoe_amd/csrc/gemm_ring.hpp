@@ -16,7 +16,8 @@
 //   * the tiles are dealt to the workgroups beforehand: row-ragged products in bands of row
 //     tiles shared by the XCDs; the weight gradient expert by expert in descending order of their rows (the table's
 //     order list), back and forth over the workgroups, so that every workgroup gets its share of long and
-//     short contractions, and by cost where that leaves them uneven (ring_deal);
+//     short contractions, and by cost where that leaves them uneven (ring_deal); the gradients of experts without
+//     rows are filled with zeros outside the stream (ring_fill);
 //   * the bias gradient is one more column of products (a block of ones times the output gradient).
 #pragma once
 #include "gemm_kernel.hpp"
@@ -152,8 +153,8 @@ struct DealLds {
 // Every workgroup plans the whole launch from the table, with the same numbers.  Simulated over sizes and
 // routings, the longest list is 1.05 times the mean (or the longest tile) on average; 1.15 with rounds alone, 1.03 if
 // every tile went to the least loaded workgroup.
-__device__ __forceinline__ RingDeal ring_deal(const RingParams &prm, int tiles_per_expert, int total, int grid, int w, DealLds &lds) {
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, n = prm.n_expert;
+__device__ __forceinline__ RingDeal ring_deal(const RingParams &prm, int n, int tiles_per_expert, int total, int grid, int w, DealLds &lds) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;   // (n: experts with rows)
     const int rounds = total / grid, rest = total - rounds * grid;
     const RingDeal rounds_alone{0, 0, 0};
     const int *order = prm.dev_tab + prm.dev_order_off;   // {expert, first row, rows, 0}
@@ -245,6 +246,45 @@ __device__ __forceinline__ RingDeal ring_deal(const RingParams &prm, int tiles_p
     };
     const int first = first_tile(lds.room[w]), end = w == grid - 1 ? total : first_tile(lds.room[w + 1]);
     return RingDeal{k_best, first, max(0, end - first)};
+}
+
+// Experts of the order list whose weight gradients are dealt as tiles: those with rows, or all (see ring_fill).
+__device__ __forceinline__ int ring_live(const RingParams &prm, int grid) {
+    const int live = prm.dev_tab[segtab::kLive], tpe = prm.tiles_m * prm.tiles_n;
+    const bool whole = prm.n_rows % kRingTile == 0 && prm.n_cols % kRingTile == 0;
+    const bool nearly = 16 * (int64_t)prm.n_rows * prm.n_cols >= 15 * (int64_t)tpe * kRingTile * kRingTile;
+    return nearly && (4 * live > prm.n_expert || (whole && prm.n_expert * tpe >= 16 * grid)) ? prm.n_expert : live;
+}
+
+// Weight and bias gradients of the other experts, those of the order list from ring_live() on: zeros, 128 KiB at a time over all
+// workgroups.  As a tile such a piece would cost what a tile with a slab does, 5 us, however little of it has to be stored.  Waiting
+// for the stores of a piece together keeps the memory's queues short.  us with one workgroup per tile / as tiles / like this:
+// 5 rows over 128 experts of 96 x 3264: 22 / 35 / 17; 8 over 12 of 1248 x 2144: 15 / 20 / 15; 100 over 128 of 2000 x 2000:
+// 292 / 265 / 192; 7 over 32 of 1024 x 4096: 35 / 43 / 39.  Where tiles are (nearly) full they stay tiles if most experts have rows,
+// which leaves little to fill (64 over 16 of 1000 x 4000: 30 / 29 / 31), or if they are full and many, which go out through LDS as
+// fast (100 over 128 of 2048 x 2048: 178 / 179 / 187).
+template <typename T> __device__ __forceinline__ void ring_fill(const RingParams &prm, int place) {
+    constexpr int kStores = 16, kPieceVecs = kStores * kRingThreads;
+    const int t = threadIdx.x, grid = gridDim.x, n_live = ring_live(prm, grid);
+    const int64_t vecs = prm.c_expert_stride / 8;   // (an expert's gradient is dense, and both of its sizes are multiples of 8)
+    const int pieces = (int)((vecs + kPieceVecs - 1) / kPieceVecs);
+    const int total = (prm.n_expert - n_live) * pieces;   // (pieces of 128 KiB in memory, or one per expert: an int holds them)
+    // (the pieces go on where the tiles ended, so that workgroups with a tile less begin)
+    const int dealt = (int)((int64_t)n_live * prm.tiles_m * prm.tiles_n % grid);
+    for (int q = place >= dealt ? place - dealt : place + grid - dealt; q < total; q += grid) {
+        const int i = q / pieces;
+        const int64_t v0 = (int64_t)(q - i * pieces) * kPieceVecs, expert = prm.dev_tab[prm.dev_order_off + 4 * (n_live + i)];
+        u32x4 *dst = (u32x4 *)((T *)prm.C + expert * prm.c_expert_stride);
+#pragma unroll
+        for (int j = 0; j < kStores; ++j) {
+            const int64_t v = v0 + j * kRingThreads + t;
+            if (v < vecs) dst[v] = u32x4{0, 0, 0, 0};
+        }
+        if (v0 == 0 && prm.bias_grad != nullptr)
+            for (int r = t; r < prm.n_rows; r += kRingThreads) ((T *)prm.bias_grad)[expert * prm.n_rows + r] = (T)0.f;
+        __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+        __syncthreads();
+    }
 }
 
 // acc[x][y][i] is C(row 64 wm + 16 y + lb, column 128 wn + 16 x + 4 hq + i).  Sixteen rows at a time go
@@ -395,22 +435,23 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_ring_kernel(const R
         }
     } else {
         tm_total = prm.tiles_m;
-        const int total = prm.n_expert * prm.tiles_m * prm.tiles_n, grid = gridDim.x;
+        const int grid = gridDim.x, n_live = uniform(ring_live(prm, grid));
+        const int total = n_live * prm.tiles_m * prm.tiles_n;
         const int rounds = uniform(total / grid), rest = total - rounds * grid;
         n_items = rounds + (ring_zigzag(rounds, grid, deal_w) < total ? 1 : 0);
-        if (rounds > 0 && rest + rounds > 1 && prm.n_expert <= kDealExperts && grid <= kDealGroups) {
+        if (rounds > 0 && rest + rounds > 1 && n_live <= kDealExperts && grid <= kDealGroups) {
             // rounds alone are level enough where the first one is: its first and last tile differ by less than a sixteenth of a list
             const int tpe = prm.tiles_m * prm.tiles_n;
             const int longest = ring_tile_cost(dtab[prm.dev_order_off + 2]);
             const int shortest = ring_tile_cost(dtab[prm.dev_order_off + 4 * uniform((grid - 1) / tpe) + 2]);
-            const float list = ((float)dtab[segtab::kRows] / 64.f + (kDealTileCost + 0.5f) * (float)prm.n_expert) * (float)tpe / (float)grid;
+            const float list = ((float)dtab[segtab::kRows] / 64.f + (kDealTileCost + 0.5f) * (float)n_live) * (float)tpe / (float)grid;
             const int spread = uniform(longest) - uniform(shortest);
             if (spread >= kDealSpread && (float)spread * 16.f > list) {
                 // (eight tiles in a row to an XCD, which share operands, then the next: as many long tiles as one expert has
                 // would otherwise all be on one or two XCDs, the 64 experts of ring_deal's comment 150 us instead of 133)
                 const int chunk = per % 8 == 0 ? 8 : 1;
                 const int w = (slot / chunk) * (8 * chunk) + xcd * chunk + slot % chunk;
-                const RingDeal planned = ring_deal(prm, tpe, total, grid, w, *(DealLds *)smem);
+                const RingDeal planned = ring_deal(prm, n_live, tpe, total, grid, w, *(DealLds *)smem);
                 if (uniform(planned.rounds) > 0) {
                     deal_w = uniform(w);
                     deal.rounds = uniform(planned.rounds);
@@ -421,7 +462,10 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_ring_kernel(const R
             }
         }
     }
-    if (n_items == 0) return;
+    if (n_items == 0) {
+        if constexpr (RAGGED == kRaggedK) ring_fill<T>(prm, xcd * per + slot);
+        return;
+    }
 
     typedef RingTile<T> Tile;
     auto decode = [&](int r) {
@@ -823,6 +867,7 @@ __global__ __launch_bounds__(kRingThreads) void grouped_gemm_ring_kernel(const R
     };
     if (wave < kLoadWaves) run(std::true_type{});
     else run(std::false_type{});
+    if constexpr (RAGGED == kRaggedK) ring_fill<T>(prm, xcd * per + slot);
 #endif  // __HIP_DEVICE_COMPILE__
 }
 

@@ -29,7 +29,8 @@ struct SegmentTable {
 // GEMM through scalar loads.  All entries are int32:
 //   [0] n_expert   [1] rows (sum of the counts)   [2] row tiles of 256   [3] row tiles of 128
 //   [4] offset of the 256-row tile map            [5] offset of the 128-row tile map
-//   [6] rows_cap the table was laid out for       [7] 0
+//   [6] rows_cap the table was laid out for       [7] leading entries of `order` that have to be looked at: the experts
+//                                                     with rows (where the list is in expert order: all experts)
 //   [8 .. 8+E]           seg: first row of every expert, seg[E] = rows
 //   [.. +E+1] [.. +E+1]  exclusive prefix of the experts' row tiles, 256 and 128 rows high
 //   tile maps            one {expert, first row, rows, 0} per row tile, 16-byte aligned
@@ -39,7 +40,7 @@ struct SegmentTable {
 // workgroups beyond the table's tile count leave at once.
 namespace segtab {
 constexpr int kHeader = 8;
-constexpr int kRows = 1, kTiles256 = 2, kTiles128 = 3, kMap256 = 4, kMap128 = 5, kRowsCap = 6;
+constexpr int kRows = 1, kTiles256 = 2, kTiles128 = 3, kMap256 = 4, kMap128 = 5, kRowsCap = 6, kLive = 7;
 __host__ __device__ inline int64_t cap_tiles(int64_t rows_cap, int64_t n_expert, int block_rows) {
     return rows_cap / block_rows + (n_expert < rows_cap ? n_expert : rows_cap);
 }

@@ -102,7 +102,7 @@ __global__ __launch_bounds__(kTabBlock) void segment_table_kernel(const int64_t 
         tab[segtab::kMap256] = map256;
         tab[segtab::kMap128] = map128;
         tab[segtab::kRowsCap] = rows_cap;
-        tab[7] = 0;
+        tab[segtab::kLive] = n_expert;
     }
     // the prefixes written above are read back below by other threads of this workgroup
     __threadfence();

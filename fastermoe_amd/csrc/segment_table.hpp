@@ -13,7 +13,7 @@ constexpr int kRankExperts = 192;     // most experts that are ordered by counti
 // LDS of small_table(): the three prefixes and the waves' sums
 struct SmallLds {
     int64_t row_sum[kThreads / kWave];
-    int32_t wave_sum[2][kThreads / kWave];
+    int32_t wave_sum[2][kThreads / kWave], wave_live[kThreads / kWave];
     int32_t seg[kSmallExperts + 1];
     __attribute__((aligned(8))) int32_t pfx[2][kSmallExperts + 1];   // (afterwards the exchange buffer of sort_descending)
     __attribute__((aligned(16))) int32_t rows[kSmallExperts];
@@ -75,6 +75,8 @@ __device__ __forceinline__ void small_table(int64_t count, int n_expert, int row
         tv[k] = s;
         if (lane == kWave - 1) lds.wave_sum[k][wave] = s;
     }
+    const int live = __popcll(__ballot(rows > 0));
+    if (lane == 0) lds.wave_live[wave] = live;
     __syncthreads();
     for (int w = 0; w < wave; ++w) { tv[0] += lds.wave_sum[0][w]; tv[1] += lds.wave_sum[1][w]; }
     int32_t *seg = tab + seg_off(), *pfx256 = tab + pfx256_off(n_expert), *pfx128 = tab + pfx128_off(n_expert);
@@ -96,7 +98,10 @@ __device__ __forceinline__ void small_table(int64_t count, int n_expert, int row
         tab[kMap256] = map256;
         tab[kMap128] = map128;
         tab[kRowsCap] = rows_cap;
-        tab[7] = 0;
+        int all_live = 0;
+#pragma unroll
+        for (int w = 0; w < kThreads / kWave; ++w) all_live += lds.wave_live[w];
+        tab[kLive] = all_live;
     }
     __syncthreads();
 #pragma unroll

@@ -441,3 +441,38 @@ def test_weight_gradient_of_uneven_experts(e, fin, fout, rows, routing, dtype, d
         for got, ref in ((gw[ex], gs.t() @ xs), (gb[ex], gs.sum(dim=0))):
             bound = eps * ref.abs() + 1e-3 * ref.pow(2).mean().sqrt() if n else torch.zeros_like(ref)
             assert bool(((got.float() - ref).abs() <= bound).all()), f"expert {ex} with {n} rows"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts,fin,fout", [
+    ([0] * 600, 264, 520),                                        # no expert has rows
+    ([0] * 127 + [5], 96, 3264),
+    ([3] + [0] * 15 + [200] + [0] * 15, 1288, 1000),
+    ([0, 1] * 300, 8, 2056),                                      # gradients of one piece and a little
+    ([0] * 9 + [300] + [0] * 70, 2048, 1032),                     # whole pieces
+    ([0] * 1000 + [2] * 24, 256, 256),
+    ([0] * 1029 + [2], 256, 264),                                 # more experts than the table sorts
+])
+def test_weight_gradient_of_experts_without_rows(counts, fin, fout, dtype, device):
+    """Large launches fill the gradients of experts without rows apart from the products' tiles: exact zeros there, in memory
+    that held NaN before, and the float32 products, rounded, for the others; the table's count of experts with rows."""
+    counts = torch.tensor(counts)
+    e, slots = counts.numel(), int(counts.sum()) + 2
+    g = torch.Generator(device=device).manual_seed(e)
+    x = torch.randn(slots, fin, device=device, generator=g).to(dtype)
+    gy = torch.randn(slots, fout, device=device, generator=g).to(dtype)
+    weight = torch.empty(e, fout, fin, dtype=dtype, device=device)
+    table = fmoe_native.segment_table(counts.to(device), slots)
+    assert int(table[7]) == (int((counts > 0).sum()) if e <= 1024 else e)
+    for size in ((e, fout, fin), (e, fout)):
+        torch.full(size, float("nan"), dtype=dtype, device=device)   # (freed at once: the next tensor of this size takes its place)
+    gw, gb = fmoe_native.linear_wgrad_dev(gy, x, weight, table, slots, True)
+    empty = (counts == 0).to(device)
+    assert not gw[empty].any() and not gb[empty].any()
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    first = torch.cumsum(counts, 0) - counts
+    for ex in torch.nonzero(counts).flatten().tolist():
+        lo, n = int(first[ex]), int(counts[ex])
+        gs, xs = gy[lo:lo + n].float(), x[lo:lo + n].float()
+        for got, ref in ((gw[ex], gs.t() @ xs), (gb[ex], gs.sum(dim=0))):
+            assert bool(((got.float() - ref).abs() <= eps * ref.abs() + 1e-3 * ref.pow(2).mean().sqrt()).all()), f"expert {ex}"
