@@ -35,6 +35,13 @@ __global__ __launch_bounds__(kBlock) void combine_fwd_vec_kernel(
     if (t >= n_tokens) return;
     const int v = (int)(piece - t * pieces_per_row) * kWave + lane;
     if (v >= row_vecs) return;
+    // (float32 scores are read through the vector path, beside the rows: the compiler's scalar loads of what is the same for
+    // the whole wave take longer, top-1 combine of 40000 rows of 300: 24.6 us, like this 22.8, from indexed rows 25.9 and 24.4)
+    if constexpr (sizeof(T) == 4) {
+        int at = 0;
+        asm volatile("" : "+v"(at));
+        score += at;
+    }
     float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int j0 = 0; j0 < top_k; j0 += 8) {
         u32x4 val[8];
