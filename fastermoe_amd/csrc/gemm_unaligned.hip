@@ -10,7 +10,7 @@
 // 128 x 128 tiles (64 x 64 per wave), 64 x 128 where those would leave compute units without one; two slabs of
 // LDS, the next slab's chunks are requested before the products of the current one.  Bound by the latency of those
 // loads up to a few hundred rows per expert (1.2 us a slab) and by their way through registers above (8192 rows, 2047 x 4093:
-// 600 to 730 TFLOP/s).  Measured against the element-wise kernel it replaced: see the dispatch in grouped_gemm.hip.
+// 600 to 680 TFLOP/s).  Measured against the element-wise kernel it replaced: see the dispatch in grouped_gemm.hip.
 #include "gemm_kernel.hpp"
 
 namespace fmoe {
@@ -103,6 +103,21 @@ __global__ __launch_bounds__(kUaThreads) void grouped_gemm_unaligned_kernel(cons
         c_off = (int64_t)expert * prm.c_expert_stride + (int64_t)m0 * prm.ldc + n0;
     }
 
+    // An expert without rows: its tiles write zeros over equal parts of its gradient, which is dense (as a tile of no
+    // slabs, stored 16 bytes at a time off the grid: 1 row over 500 experts of 1483 x 70, 91 us, like this 23).
+    if (RAGGED == kRaggedK && K == 0 && !(prm.accumulate_first && ei == 0)) {
+        const int64_t size = (int64_t)prm.n_rows * prm.n_cols, per = (size + prm.tiles_m * prm.tiles_n - 1) / (prm.tiles_m * prm.tiles_n);
+        const int64_t lo = min(rem * per, size), hi = min(lo + per, size);
+        T *gw = (T *)prm.C + (int64_t)expert * prm.c_expert_stride;
+        const int64_t body = min(lo + (int64_t)((16 - ((uintptr_t)(gw + lo) & 15)) & 15) / 2, hi), vecs = (hi - body) / 8;
+        for (int64_t i = lo + t; i < body; i += kUaThreads) gw[i] = (T)0.f;
+        for (int64_t v = t; v < vecs; v += kUaThreads) ((u32x4 *)(gw + body))[v] = u32x4{0u, 0u, 0u, 0u};
+        for (int64_t i = body + 8 * vecs + t; i < hi; i += kUaThreads) gw[i] = (T)0.f;
+        if (rem == 0 && prm.bias_grad != nullptr)
+            for (int r = t; r < prm.n_rows; r += kUaThreads) ((T *)prm.bias_grad)[(int64_t)expert * prm.n_rows + r] = (T)0.f;
+        return;
+    }
+
     // -- memory -> registers -> LDS: thread t has chunk it * 256 + t of the slab
     auto chunk_index = [&](int shape, int it) { return shape == kKC ? (it * kUaThreads + t) >> 3 : (it * kUaThreads + t) >> 4; };
     // (its offsets from the slab's first element do not change: rows and chunks past a tile's end repeat the last one)
@@ -156,6 +171,10 @@ __global__ __launch_bounds__(kUaThreads) void grouped_gemm_unaligned_kernel(cons
         return u32x4{l2[0], l2[1], h2[0], h2[1]};
     };
 
+    // Block row y of a wave.  Ragged rows: every other one, so that both pairs of waves have some of an expert's few
+    // rows and the epilogue ends at the last of them.
+    auto row_block = [&](int y) { return RAGGED == kRaggedRows ? 2 * y + wm : TJ * wm + y; };
+
     f32x4 acc[TI][TJ], bacc[kBiasGrad ? TJ : 1];
 #pragma unroll
     for (int x = 0; x < TI; ++x)
@@ -191,7 +210,7 @@ __global__ __launch_bounds__(kUaThreads) void grouped_gemm_unaligned_kernel(cons
 #pragma unroll
             for (int x = 0; x < TI; ++x) pf[x] = frag(PSHAPE, buf, wn * TI + x, ks);
 #pragma unroll
-            for (int y = 0; y < TJ; ++y) qf[y] = frag(QSHAPE, buf + P_BYTES, wm * TJ + y, ks);
+            for (int y = 0; y < TJ; ++y) qf[y] = frag(QSHAPE, buf + P_BYTES, row_block(y), ks);
 #pragma unroll
             for (int x = 0; x < TI; ++x)
 #pragma unroll
@@ -204,12 +223,23 @@ __global__ __launch_bounds__(kUaThreads) void grouped_gemm_unaligned_kernel(cons
     }
     __syncthreads();
 
-    // -- epilogue: acc[x][y][i] is C(row 16 (TJ wm + y) + lb, column 64 wn + 16 x + 4 hq + i); sixteen rows at a
+    // -- epilogue: acc[x][y][i] is C(row 16 row_block(y) + lb, column 64 wn + 16 x + 4 hq + i); sixteen rows at a
     // time through 2 KiB of LDS per wave and out as 128-byte row pieces
     unsigned char *stg = smem + wave * 2048;
     T *C = (T *)prm.C + c_off, *aux = prm.aux ? (T *)prm.aux + c_off : nullptr;
     const bool accumulate = RAGGED == kRaggedK && prm.accumulate_first && ei == 0;
     const T *bias = prm.bias ? (const T *)prm.bias + (int64_t)expert * prm.bias_expert_stride + n0 : nullptr;
+    // (read once: in the loop, behind stores that might reach it as far as the compiler can tell, every use waited for those.  Forward
+    // with GELU, 8192 rows, 8 experts of 2047 x 4093: 275 -> 225 us; with the epilogue's end at an expert's last rows
+    // 556 rows, 64 of 38 x 1990: 50 -> 23)
+    float bias_of[TI][4];
+#pragma unroll
+    for (int x = 0; x < TI; ++x)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int col = 64 * wn + 16 * x + 4 * hq + i;
+            bias_of[x][i] = bias != nullptr && col < p_valid ? (float)bias[col] : 0.f;
+        }
     auto wave_sync = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -220,7 +250,7 @@ __global__ __launch_bounds__(kUaThreads) void grouped_gemm_unaligned_kernel(cons
         for (int i = 0; i < 2; ++i) {
             const int r = i * 8 + (lane >> 3), c = lane & 7;
             const u32x4 v = *(const u32x4 *)(stg + r * 128 + ((c ^ (r & 7)) << 4));
-            const int row = 16 * (TJ * wm + y) + r, col = 64 * wn + c * 8;
+            const int row = 16 * row_block(y) + r, col = 64 * wn + c * 8;
             if (row < q_valid && col < p_valid) {
                 T *p = to + (int64_t)row * prm.ldc + col;
                 if (col + 8 <= p_valid) {
@@ -237,7 +267,8 @@ __global__ __launch_bounds__(kUaThreads) void grouped_gemm_unaligned_kernel(cons
     };
 #pragma unroll
     for (int y = 0; y < TJ; ++y) {
-        const int row = 16 * (TJ * wm + y) + lb;
+        if (16 * row_block(y) >= q_valid) break;
+        const int row = 16 * row_block(y) + lb;
 #pragma unroll
         for (int kind = 1; kind >= 0; --kind) {   // 1: the pre-activation, 0: the result
             if (kind == 1 && (prm.epilogue != kEpiBiasAct || aux == nullptr)) continue;
@@ -248,8 +279,7 @@ __global__ __launch_bounds__(kUaThreads) void grouped_gemm_unaligned_kernel(cons
                 for (int i = 0; i < 4; ++i) {
                     const int col = 64 * wn + 16 * x + 4 * hq + i;
                     const bool in = row < q_valid && col < p_valid;
-                    float v = acc[x][y][i];
-                    if (bias != nullptr) v += col < p_valid ? (float)bias[col] : 0.f;
+                    float v = acc[x][y][i] + bias_of[x][i];
                     if (kind == 0 && prm.epilogue == kEpiBiasAct) v = apply_act<false>(v, prm.activation);
                     if (prm.epilogue == kEpiDAct) v *= act_grad<false>(in ? (float)aux[(int64_t)row * prm.ldc + col] : 0.f, prm.activation);
                     if (accumulate) v += in ? (float)C[(int64_t)row * prm.ldc + col] : 0.f;

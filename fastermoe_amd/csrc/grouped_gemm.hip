@@ -287,8 +287,8 @@ template <int PRODUCT>
 int dispatch(GemmParams &prm, int dtype, int epi, bool fast, hipStream_t stream) {
     // Shapes off the 16-byte grid: 16-bit types in gemm_unaligned.hip, the others and double precision on the
     // element-checked kernel of gemm_any.hip.  bf16 on that one and on gemm_unaligned.hip, forward / data gradient /
-    // weight gradient: 1554 rows, 12 experts of 500 x 1302: 89 / 170 / 64 and 21 / 24 / 28 us; 16 rows, 8 experts of
-    // 1000 x 2001: 93 / 178 / 26 and 21 / 33 / 24; 8192 rows, 8 experts of 2047 x 4093: 3063 / 2800 / 2116 and 230 / 188 / 257.
+    // weight gradient: 1554 rows, 12 experts of 500 x 1302: 89 / 170 / 64 and 15 / 24 / 21 us; 16 rows, 8 experts of
+    // 1000 x 2001: 93 / 178 / 26 and 17 / 32 / 20; 8192 rows, 8 experts of 2047 x 4093: 3063 / 2800 / 2116 and 203 / 228 / 218.
     if (!fast && is_16bit(dtype)) return launch_mfma_unaligned(prm, dtype, PRODUCT, epi, stream);
     if (!fast || dtype == FMOE_F64) return launch_mfma_any(prm, dtype, PRODUCT, epi, stream);
     switch (dtype * 3 + PRODUCT) {

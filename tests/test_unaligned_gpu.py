@@ -73,6 +73,28 @@ def _check(dtype, counts, fin, fout, device, shift):
     assert rel_err(fmoe_native.linear_dact_backward(gyd, cnt, wd, pd, _lib.ACT_GELU), p64.grad) <= tol
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts,fin,fout", [([0, 3, 0, 0], 1, 1), ([0, 1, 0], 3, 5), ([0] * 40 + [2] + [0] * 9, 1483, 70),
+                                             ([0, 5, 0, 0, 200], 129, 257)])
+def test_weight_gradients_of_experts_without_rows(dtype, counts, fin, fout, device):
+    """Zeros wherever an expert's gradient begins, into memory that held NaN before, and nothing beyond them."""
+    x = torch.randn(sum(counts), fin, device=device).to(dtype)
+    gy = torch.randn(sum(counts), fout, device=device).to(dtype)
+    w = torch.empty(len(counts), fout, fin, dtype=dtype, device=device)
+    b = torch.empty(len(counts), fout, dtype=dtype, device=device)
+    for size in (w.shape, b.shape):
+        torch.full(size, float("nan"), dtype=dtype, device=device)   # (freed at once: the next tensor of this size takes its place)
+    gw, gb = fmoe_native.linear_weight_backward(gy, x, torch.tensor(counts), w, b)
+    lo = 0
+    for ex, n in enumerate(counts):
+        gs, xs = gy[lo:lo + n].double(), x[lo:lo + n].double()
+        lo += n
+        if n:
+            assert rel_err(gw[ex], gs.t() @ xs) <= TOL[dtype] and rel_err(gb[ex], gs.sum(dim=0)) <= TOL[dtype]
+        else:
+            assert not gw[ex].any() and not gb[ex].any()
+
+
 @pytest.mark.parametrize("dtype,n,d,h,e,shift", [
     (torch.bfloat16, 4096, 4096, 4096, 4, 4),   # sizes at which a fused layer leaves its chunks where it may
     (torch.bfloat16, 300, 128, 256, 4, 1),
