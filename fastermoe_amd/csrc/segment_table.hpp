@@ -8,7 +8,7 @@ namespace segtab {
 
 constexpr int kThreads = 1024;        // the workgroup that builds a table
 constexpr int kSmallExperts = 1024;   // most experts of small_table(): one per thread
-constexpr int kRankExperts = 192;     // most experts that are ordered by counting
+constexpr int kRankExperts = 64;     // most experts that are ordered by counting
 
 // LDS of small_table(): the three prefixes and the waves' sums
 struct SmallLds {
@@ -19,25 +19,57 @@ struct SmallLds {
     __attribute__((aligned(16))) int32_t rows[kSmallExperts];
 };
 
+// The value of the lane whose number differs in bit J, by the cheapest exchange: within rows of 16 lanes in the vector pipe, of 32
+// by a swizzle with a constant pattern, else by address.
+template <int J> __device__ __forceinline__ unsigned int lane_xor(unsigned int v) {
+    if (J == 1) return __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);     // quad_perm 1 0 3 2
+    if (J == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true);     // quad_perm 2 3 0 1
+    if (J == 4)   // bits 0 to 2, then 0 and 1 back: row_half_mirror, quad_perm 3 2 1 0
+        return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true), 0x1b, 0xf, 0xf, true);
+    if (J == 8) return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, true);    // row_ror 8
+    if (J == 16) return __builtin_amdgcn_ds_swizzle(v, 0x401f);                     // and 31, or 0, xor 16
+    return __shfl_xor(v, J, kWave);
+}
+template <int J> __device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
+    return ((unsigned long long)lane_xor<J>((unsigned int)(v >> 32)) << 32) | lane_xor<J>((unsigned int)v);
+}
+
 // Sorts the workgroup's keys, one per thread, among its first n threads (a power of two of at least 64): thread i ends with the
 // i-th largest.  A bitonic network; partners in the same wave exchange by lane, others through buf [kThreads].
-__device__ __forceinline__ uint64_t sort_descending(uint64_t key, int n, uint64_t *buf) {
+template <typename Key> __device__ __forceinline__ Key sort_descending(Key key, int n, Key *buf) {
     const int i = threadIdx.x;
-    for (int k = 2; k <= n; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            uint64_t other;
-            if (j < kWave) {
-                other = (uint64_t)__shfl_xor((unsigned long long)key, j, kWave);
-            } else {
-                buf[i] = key;
-                __syncthreads();
-                other = buf[i ^ j];
-                __syncthreads();
-            }
+    for (int k = 2; k <= n; k <<= 1) {
+        auto take = [&](Key other, int j) {
             const bool keep_larger = ((i & j) == 0) == ((i & k) == 0);
             key = (key > other) == keep_larger ? key : other;
+        };
+        for (int j = k >> 1; j >= kWave; j >>= 1) {
+            buf[i] = key;
+            __syncthreads();
+            const Key other = buf[i ^ j];
+            __syncthreads();
+            take(other, j);
         }
+        if (k > 32) take(lane_xor<32>(key), 32);
+        if (k > 16) take(lane_xor<16>(key), 16);
+        if (k > 8) take(lane_xor<8>(key), 8);
+        if (k > 4) take(lane_xor<4>(key), 4);
+        if (k > 2) take(lane_xor<2>(key), 2);
+        take(lane_xor<1>(key), 1);
+    }
     return key;
+}
+
+// Thread e's place in the list of the experts by descending rows (of equal ones the lower expert first): the expert that belongs
+// there.  A key is an expert's rows above its number; 32 bits hold both up to 2^22 rows, half the exchanges of 64.
+template <typename Key> __device__ __forceinline__ int expert_in_order(int rows, int n_expert, Key *buf) {
+    constexpr int kBits = 10;   // kSmallExperts
+    const int e = threadIdx.x;
+    int n = kWave;
+    while (n < n_expert) n <<= 1;
+    // (threads without an expert sort last: their keys have the highest numbers)
+    const Key mine = ((Key)(e < n_expert ? rows : 0) << kBits) | (Key)((1 << kBits) - 1 - e);
+    return (1 << kBits) - 1 - (int)(sort_descending(mine, n, buf) & ((1 << kBits) - 1));
 }
 
 // The whole table for at most kSmallExperts experts by one workgroup of kThreads threads, thread e
@@ -127,19 +159,14 @@ __device__ __forceinline__ void small_table(int64_t count, int n_expert, int row
     }
     // The experts by descending rows.  Up to kRankExperts an expert's place is counted, the number of experts that come
     // before it; beyond, where the square of their number tells, the experts are sorted.  The whole table, counted and
-    // sorted: 129 experts 8.5 / 10.0 us, 256: 11.8 / 10.1, 512: 19.6 / 11.6, 1024: 44.6 / 13.8.
+    // sorted: up to 65 experts 7.6 us either way, 128: 8.6 / 7.6, 192: 10.3 / 8.1, 256: 11.8 / 8.1, 512: 19.6 / 9.1, 1024: 44.6 / 10.6
+    // (exchanges by address and 64-bit keys: 256: 10.3, 512: 12.0, 1024: 14.3).
     int4 *order = (int4 *)(tab + order_off(rows_cap, n_expert));
     if (n_expert > kRankExperts) {
         __syncthreads();   // the maps are done with lds.pfx
-        int n = kWave;
-        while (n < n_expert) n <<= 1;
-        // (of equal rows the lower expert first; threads without an expert sort last)
-        const uint64_t mine = e < n_expert ? ((uint64_t)(uint32_t)rows << 32) | (0xffffffffu - (uint32_t)e) : 0;
-        const uint64_t key = sort_descending(mine, n, (uint64_t *)&lds.pfx[0][0]);
-        if (e < n_expert) {
-            const int ex = (int)(0xffffffffu - (uint32_t)key);
-            order[e] = make_int4(ex, lds.seg[ex], (int)(key >> 32), 0);
-        }
+        const int ex = rows_cap < (1 << 22) ? expert_in_order<unsigned int>(rows, n_expert, (unsigned int *)&lds.pfx[0][0])
+                                            : expert_in_order<unsigned long long>(rows, n_expert, (unsigned long long *)&lds.pfx[0][0]);
+        if (e < n_expert) order[e] = make_int4(ex, lds.seg[ex], lds.rows[ex], 0);
     } else if (e < n_expert) {
         int place = 0;
         for (int f = 0; f < n_expert; f += 4) {

@@ -402,6 +402,20 @@ def test_order_of_the_experts_by_their_rows(n_expert, kind, device):
         assert [tuple(r) for r in t[at:at + 4 * n_expert].reshape(-1, 4).tolist()] == want
 
 
+@pytest.mark.parametrize("rows_cap", [(1 << 22) - 1, 1 << 22, 1 << 23])
+@pytest.mark.parametrize("n_expert", [193, 700, 1024])
+def test_order_of_experts_with_many_rows(n_expert, rows_cap, device):
+    """The same list on either side of the number of rows that sorts by 32-bit keys; one expert with nearly all rows."""
+    g = torch.Generator().manual_seed(n_expert)
+    counts = torch.randint(0, 3, (n_expert,), generator=g)
+    counts[n_expert // 2] = rows_cap - int(counts.sum()) + int(counts[n_expert // 2])
+    t = fmoe_native.segment_table(counts.to(device), rows_cap).cpu().numpy()
+    first = np.concatenate([[0], np.cumsum(counts.numpy())[:-1]])
+    want = [(e, int(first[e]), int(counts[e]), 0) for e in sorted(range(n_expert), key=lambda e: (-int(counts[e]), e))]
+    at = int(t[5]) + 4 * (rows_cap // 128 + n_expert)
+    assert [tuple(r) for r in t[at:at + 4 * n_expert].reshape(-1, 4).tolist()] == want
+
+
 UNEVEN = [  # experts, in, out, rows, routing: weight gradients whose tiles are dealt by cost, and some on either side of that rule
     (64, 1456, 1256, 12926, "zipf"),
     (32, 544, 8040, 3000, "one"),
