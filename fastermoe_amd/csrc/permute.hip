@@ -23,7 +23,11 @@ constexpr int kPieceVecs = kWave * kVecPerLane;  // 256 x 16 B = 4 KiB
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // ---- gather rows: out[r] = index[r] >= 0 ? inp[index[r]] : 0 -------------
-// row_vecs = 16-byte vectors per row.
+// row_vecs = 16-byte vectors per row.  AGAIN: a divisor makes several rows of one (the top_k copies of a token), so what is read
+// stays in the caches; rows that are read once pass them by.  us before (all passed by) and with it, sorted copies in
+// bf16: 8192 tokens of 2048, top-8: 83 and 74; 32768 of 4096, top-2: 176 and 154; with the weight gradient that reads the copy: 460
+// and 446, but top-1, 16384 of 2048: 126 and 132 with AGAIN.
+template <bool AGAIN>
 __global__ __launch_bounds__(kBlock) void gather_rows_vec_kernel(
     const u32x4 *__restrict__ inp, const int64_t *__restrict__ index, int64_t divisor,
     u32x4 *__restrict__ out, int64_t n_out, int64_t n_inp, int row_vecs, int pieces_per_row) {
@@ -38,7 +42,7 @@ __global__ __launch_bounds__(kBlock) void gather_rows_vec_kernel(
     for (int j = 0; j < kVecPerLane; ++j) {
         const int v = v0 + j * kWave + lane;
         val[j] = u32x4{0, 0, 0, 0};
-        if (live && v < row_vecs) val[j] = __builtin_nontemporal_load(&inp[src * row_vecs + v]);
+        if (live && v < row_vecs) val[j] = AGAIN ? inp[src * row_vecs + v] : __builtin_nontemporal_load(&inp[src * row_vecs + v]);
     }
 #pragma unroll
     for (int j = 0; j < kVecPerLane; ++j) {
@@ -346,7 +350,8 @@ int permute_gather_rows(const void *inp, const int64_t *index, int64_t divisor, 
         const int ppr = (int)ceil_div(row_vecs, kPieceVecs);
         const int64_t blocks = ceil_div(n_out * ppr, kWavesPerBlock);
         if (blocks > INT32_MAX) return fail(FMOE_ELIMIT, "gather_rows: grid too large");
-        gather_rows_vec_kernel<<<(int)blocks, kBlock, 0, st>>>((const u32x4 *)inp, index, divisor, (u32x4 *)out,
+        const auto kern = divisor > 1 ? gather_rows_vec_kernel<true> : gather_rows_vec_kernel<false>;
+        kern<<<(int)blocks, kBlock, 0, st>>>((const u32x4 *)inp, index, divisor, (u32x4 *)out,
                                                                 n_out, n_inp, row_vecs, ppr);
     } else {
         switch (dtype_bytes(dtype)) {
