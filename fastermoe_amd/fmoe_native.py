@@ -8,6 +8,7 @@ the CPU and nothing falls back to torch operators.
 """
 import contextlib
 import ctypes
+import os
 
 import torch
 
@@ -672,7 +673,6 @@ def linear_dev_reads_rows(rows_cap, n_expert, in_feat, out_feat, dtype, activati
 def _dev_workspace(nbytes, device):
     """The caller-side workspace of a row-ragged ``*_dev`` product (``None`` where the launch splits
     nothing); torch's caching allocator hands the same block back call after call."""
-    import os
     if nbytes == 0 or os.environ.get("FMOE_DEV_SPLIT", "1") == "0":
         return None
     return torch.empty(nbytes, dtype=torch.uint8, device=device)
@@ -712,8 +712,9 @@ def linear_forward_dev(x, weight, bias, table, rows_cap, activation=_lib.ACT_NON
     pre = new() if keep_pre else None
     with _on(x.device):
         lib = _lib.load()
-        ws = _dev_workspace(lib.fmoe_linear_forward_dev_workspace_bytes(int(rows_cap), n_expert, in_feat, out_feat, dt, activation,
-                                                                        int(keep_pre), int(row_index is not None)), x.device)
+        # (the cheaper question first: nothing of a short contraction is split)
+        ws = _dev_workspace(lib.fmoe_linear_dev_workspace_bytes(in_feat, dt) and lib.fmoe_linear_forward_dev_workspace_bytes(
+            int(rows_cap), n_expert, in_feat, out_feat, dt, activation, int(keep_pre), int(row_index is not None)), x.device)
         check(lib.fmoe_linear_forward_dev(_ptr(x), _ptr(row_index), int(index_div), x.shape[0], _ptr(weight), _ptr(bias),
                                           _ptr(pre), _ptr(y), _ptr(table), n_expert, int(rows_cap), in_feat, out_feat, dt,
                                           activation, _ptr(ws), 0 if ws is None else ws.numel(), _stream(x)))
@@ -738,8 +739,8 @@ def linear_dgrad_dev(grad_y, weight, table, rows_cap, pre=None, activation=_lib.
     grad_x = torch.empty(rows_cap, in_feat, dtype=grad_y.dtype, device=grad_y.device)
     with _on(grad_y.device):
         lib = _lib.load()
-        ws = _dev_workspace(lib.fmoe_linear_dgrad_dev_workspace_bytes(int(rows_cap), n_expert, in_feat, out_feat, dt, activation),
-                            grad_y.device)
+        ws = _dev_workspace(lib.fmoe_linear_dev_workspace_bytes(out_feat, dt) and lib.fmoe_linear_dgrad_dev_workspace_bytes(
+            int(rows_cap), n_expert, in_feat, out_feat, dt, activation), grad_y.device)
         check(lib.fmoe_linear_dgrad_dev(_ptr(grad_y), _ptr(weight), _ptr(pre if activation != _lib.ACT_NONE else None),
                                         _ptr(grad_x), _ptr(table), n_expert, int(rows_cap), in_feat, out_feat, dt, activation,
                                         _ptr(ws), 0 if ws is None else ws.numel(), _stream(grad_y)))
