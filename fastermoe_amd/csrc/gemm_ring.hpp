@@ -327,6 +327,10 @@ __device__ __forceinline__ void ring_epilogue(const RingParams &prm, const RingT
     };
     if constexpr (kDAct) request_aux(0);
     constexpr int kKinds = EPI == kEpiBiasAct ? 2 : 1;
+    // Weight gradients go out nontemporally: nothing of the launch reads them, and where they make up most of its traffic they
+    // would push the operands out of L2.  64 experts of 8192 x 2048, 64 / 256 / 512 rows each: 395 / 692 / 1067 us through the
+    // caches, 347 / 678 / 1036 like this.  (The other products' results are the next launch's input; nontemporal they gain nothing.)
+    constexpr int kPolicy = BIAS_GRAD ? 2 : 0;
 #pragma unroll
     for (int kind = kKinds - 1; kind >= 0; --kind) {   // 1: the pre-activation, 0: the result
         if (kind == 1 && !AUX) continue;
@@ -362,7 +366,7 @@ __device__ __forceinline__ void ring_epilogue(const RingParams &prm, const RingT
             for (int i = 0; i < 4; ++i) {
                 const int r = i * 4 + io_r;
                 const u32x4 v = *(const u32x4 *)(stg + r * 256 + ((io_c ^ r) << 4));
-                __builtin_amdgcn_raw_buffer_store_b128(v, rs, (int)io_offset(y, i), 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(v, rs, (int)io_offset(y, i), 0, kPolicy);
             }
             wave_sync();
         }
