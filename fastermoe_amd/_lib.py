@@ -87,6 +87,9 @@ SIGNATURES = {
     "fmoe_combine_backward": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "fmoe_gather_combine_forward": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp]),
     "fmoe_gather_combine_backward": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp]),
+    "fmoe_layer_sizes": (_int, [_i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
+    "fmoe_layer_forward": (_int, [_vp] * 17 + [_i64] * 5 + [_int] * 4 + [_vp, _i64, _vp]),
+    "fmoe_layer_backward": (_int, [_vp] * 21 + [_i64] * 5 + [_int] * 3 + [_vp, _i64, _vp]),
     "fmoe_profile_enable": (_int, [_int]),
     "fmoe_profile_classes": (_int, []),
     "fmoe_profile_collect": (_int, [_vp, _vp, _vp, _int]),
@@ -96,6 +99,7 @@ PROFILE_CLASSES = ["gemm_fwd", "gemm_dgrad", "gemm_wgrad", "bias_grad", "gather_
                    "reduce_slots", "index_add", "combine"]
 
 F32, BF16, F16, F64 = 0, 1, 2, 3
+GATE_LINEAR, GATE_LOGITS, GATE_ROUTED = 0, 1, 2
 ACT_NONE, ACT_RELU, ACT_GELU = 0, 1, 2
 
 _lib = None

@@ -764,6 +764,95 @@ def linear_wgrad_dev(grad_y, x, weight, table, rows_cap, with_bias):
     return grad_w, grad_b
 
 
+# ---- a whole layer pass in one call ----------------------------------------------------
+
+def layer_sizes(n_tokens, d_model, d_hidden, n_expert, top_k, dtype, activation, keep, gate):
+    """``(scratch bytes of a forward, of a backward, segment table bytes)`` of :func:`layer_forward` for these sizes,
+    or ``None`` where it does not take them (or one of the switches that keep the steps of a layer apart is set)."""
+    if dtype not in _DTYPES:
+        return None
+    sizes = (ctypes.c_int64 * 3)()
+    taken = _lib.load().fmoe_layer_sizes(n_tokens, d_model, d_hidden, n_expert, top_k, _DTYPES[dtype], activation, keep, gate, sizes)
+    return tuple(sizes) if taken == 1 else None
+
+
+class LayerRouting:
+    """Scores and routing of a pass: of a gate outside it (``score``, ``pos``, ``slot_to_row``, ``table``), or, with the
+    gate inside, places for them in one block (``kept``; ``None``: in the pass's scratch)."""
+
+    def __init__(self, score=None, pos=None, slot_to_row=None, table=None, kept=None):
+        self.tensors = (score, pos, slot_to_row, table)
+        self.kept = kept
+
+    @staticmethod
+    def _places(n_slots, table_bytes):
+        """Offsets of topk_idx, pos, slot_to_row, the table and the scores, each on 256 bytes."""
+        step, tab = -(-8 * n_slots // 256) * 256, -(-table_bytes // 256) * 256
+        return 0, step, 2 * step, 3 * step, 3 * step + tab
+
+    @classmethod
+    def block(cls, n_slots, table_bytes, element_size, device):
+        score_at = cls._places(n_slots, table_bytes)[4]
+        return cls(kept=torch.empty(score_at + n_slots * element_size, dtype=torch.uint8, device=device))
+
+    def pointers(self, n_slots, table_bytes):
+        """``(topk_idx, score, pos, slot_to_row, table)`` as the library takes them."""
+        if self.kept is None:
+            return (None,) + tuple(map(_ptr, self.tensors))
+        base = self.kept.data_ptr()
+        idx, pos, s2r, table, score = (base + at for at in self._places(n_slots, table_bytes))
+        return idx, score, pos, s2r, table
+
+    def gate_results(self, n_tokens, top_k, table_bytes, dtype):
+        """``(topk_idx, score)`` out of the block."""
+        n = n_tokens * top_k
+        score_at = self._places(n, table_bytes)[4]
+        return (self.kept[:8 * n].view(torch.int64).view(n_tokens, top_k),
+                self.kept[score_at:score_at + n * dtype.itemsize].view(dtype).view(n_tokens, top_k))
+
+
+def layer_forward(inp, gate_w, gate_b, logits, w1, b1, w2, b2, top_k, activation, keep, gate, sizes, routing):
+    """Gate, routing, experts and combine as one call, over tensors that the caller has checked against
+    :func:`layer_sizes` (contiguous, on 16 bytes, one type and device).  Returns ``(out, pre, mid, rows)``, the last three
+    ``None`` unless ``keep``."""
+    n, d = inp.shape
+    e, h = w1.shape[:2]
+    new = lambda r, c: torch.empty(r, c, dtype=inp.dtype, device=inp.device)
+    out = new(n, d)
+    pre = mid = rows = None
+    if keep:
+        pre = new(n * top_k, h) if activation == _lib.ACT_GELU else None
+        mid, rows = new(n * top_k, h), new(n * top_k, d)
+    scratch = torch.empty(sizes[0], dtype=torch.uint8, device=inp.device)
+    idx, score, pos, s2r, table = routing.pointers(n * top_k, sizes[2])
+    with _on(inp.device):
+        check(_lib.load().fmoe_layer_forward(
+            inp.data_ptr(), _ptr(gate_w), _ptr(gate_b), _ptr(logits), w1.data_ptr(), _ptr(b1), w2.data_ptr(), _ptr(b2), idx, score, pos,
+            s2r, table, _ptr(pre), _ptr(mid), _ptr(rows), out.data_ptr(), n, d, h, e, top_k, _DTYPES[inp.dtype], activation, keep, gate,
+            scratch.data_ptr(), sizes[0], _stream(inp)))
+    return out, pre, mid, rows
+
+
+def layer_backward(grad_out, inp, gate_w, w1, w2, top_k, activation, gate, sizes, routing, pre, mid, rows, grad_x, grad_score, grad_gate_w,
+                   grad_gate_b, grad_w1, grad_b1, grad_w2, grad_b2):
+    """Backward of :func:`layer_forward` into the gradients that are given (``None``: not wanted)."""
+    n, d = inp.shape
+    e, h = w1.shape[:2]
+    if tuple(grad_out.shape) != (n, d) or grad_out.dtype != inp.dtype:
+        raise ValueError(f"grad_out must be [{n}, {d}] of {inp.dtype}")
+    # (asked for again: the switches that change a product's kernel may have been set since the forward)
+    now = (ctypes.c_int64 * 3)()
+    _lib.load().fmoe_layer_sizes(n, d, h, e, top_k, _DTYPES[inp.dtype], activation, 1, gate, now)
+    scratch = torch.empty(now[1], dtype=torch.uint8, device=inp.device)
+    idx, score, pos, s2r, table = routing.pointers(n * top_k, sizes[2])
+    with _on(inp.device):
+        check(_lib.load().fmoe_layer_backward(
+            grad_out.data_ptr(), inp.data_ptr(), _ptr(gate_w), w1.data_ptr(), w2.data_ptr(), idx, score, pos, s2r, table, _ptr(pre),
+            mid.data_ptr(), rows.data_ptr(), _ptr(grad_x), _ptr(grad_score), _ptr(grad_gate_w), _ptr(grad_gate_b), _ptr(grad_w1),
+            _ptr(grad_b1), _ptr(grad_w2), _ptr(grad_b2), n, d, h, e, top_k, _DTYPES[inp.dtype], activation, gate, scratch.data_ptr(),
+            now[1], _stream(inp)))
+
+
 # ---- fused expert MLP (chunked, stream-overlapped pipeline) -------------------------
 
 def _mlp_params(w1, b1, w2, b2, activation):

@@ -111,14 +111,19 @@ class GateLinearTopK(Function):
         return grad_x, grad_w, grad_b, None, None
 
 
-def _plain_linear(linear):
-    """Whether calling ``linear`` is ``F.linear`` on its parameters and nothing else: no hook of its own, and none for
+def _no_hooks(module):
+    """Whether calling ``module`` is its class's ``forward`` and nothing else: no hook of its own, and none for
     all modules (profilers and debuggers register those)."""
     every = torch.nn.modules.module
-    return (type(linear) is torch.nn.Linear and "forward" not in linear.__dict__
-            and not (linear._forward_hooks or linear._forward_pre_hooks or linear._backward_hooks
-                     or linear._backward_pre_hooks or every._global_forward_hooks or every._global_forward_pre_hooks
+    return ("forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                     or module._backward_pre_hooks or every._global_forward_hooks or every._global_forward_pre_hooks
                      or every._global_backward_hooks or every._global_backward_pre_hooks))
+
+
+def _plain_linear(linear):
+    """Whether calling ``linear`` is ``F.linear`` on its parameters and nothing else."""
+    return type(linear) is torch.nn.Linear and _no_hooks(linear)
 
 
 def gate_linear_topk(x, linear, top_k, score_mode=0):
@@ -441,6 +446,97 @@ class MOERoutedMLP(Function):
         rows = fmoe_native.gather_rows(inp, pos_buf, index_div=top_k)
         gw1, gb1 = fmoe_native.linear_wgrad_dev(g_pre, rows, w1, table, n_slots, b1 is not None)
         return g_inp, gw1, gb1, gw2, gb2, None, None, None, None, None, None
+
+
+class MOELayer(Function):
+    r"""The layer between its input and its output as one autograd node: gate (``routing`` ``None``: the linear layer
+    ``gate_w``, ``gate_b`` and its top-k), :class:`MOERoutedMLP` and :class:`MOEGatherCombine`, each direction one call into
+    the library.  With a gate outside, ``score`` and ``routing = (pos_buf, slot_to_row, table)`` are its results.
+    Not in the reference; the same results as the nodes one by one, except that the gate's part of the input gradient is added
+    before the sum is rounded."""
+
+    @staticmethod
+    def forward(ctx, inp, gate_w, gate_b, score, w1, b1, w2, b2, routing, top_k, activation, gate, sizes):
+        inp = inp.contiguous()
+        if routing is None:
+            place = fmoe_native.LayerRouting.block(inp.shape[0] * top_k, sizes[2], inp.element_size(), inp.device)
+        else:
+            place = fmoe_native.LayerRouting(score, *routing)
+        out, pre, mid, rows = fmoe_native.layer_forward(inp, gate_w, gate_b, _gate_logits(gate, inp, gate_w, gate_b), w1, b1, w2, b2,
+                                                        top_k, activation, 1, gate, sizes, place)
+        ctx.save_for_backward(inp, gate_w, w1, w2, pre, mid, rows, place.kept, *place.tensors)
+        ctx.moe_args = top_k, activation, gate, sizes, [b is not None for b in (gate_b, b1, b2)]
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        inp, gate_w, w1, w2, pre, mid, rows, kept, *tensors = map(_as_chunks, ctx.saved_tensors)
+        top_k, activation, gate, sizes, (gate_bias, bias1, bias2) = ctx.moe_args
+        need = ctx.needs_input_grad
+        place = fmoe_native.LayerRouting(*tensors, kept=kept)
+        # (a backward that is to be differentiated again needs the gate's products as torch operators)
+        apart = kept is not None and torch.is_grad_enabled()
+        new = lambda wanted, *shape: torch.empty(shape, dtype=inp.dtype, device=inp.device) if wanted else None
+        (n, d), (e, h) = inp.shape, w1.shape[:2]
+        grad_x = new(need[0], n, d)
+        grad_score = new(kept is None or apart, n, top_k)
+        gate_wanted = kept is not None and not apart and (need[1] or need[2])
+        grad_gate_w, grad_gate_b = new(gate_wanted, e, d), new(gate_wanted and gate_bias, e)
+        first, second = need[4] or need[5], need[6] or need[7]
+        grad_w1, grad_b1 = new(first, e, h, d), new(first and bias1, e, h)
+        grad_w2, grad_b2 = new(second, e, d, h), new(second and bias2, e, d)
+        from ._lib import GATE_ROUTED
+        fmoe_native.layer_backward(grad_out.contiguous(), inp, gate_w, w1, w2, top_k, activation, GATE_ROUTED if apart else gate, sizes, place,
+                                   pre, mid, rows, grad_x, grad_score, grad_gate_w, grad_gate_b, grad_w1, grad_b1, grad_w2, grad_b2)
+        if apart:
+            idx, score = place.gate_results(n, top_k, sizes[2], inp.dtype)
+            g = fmoe_native.gate_topk_backward(grad_score, score, idx, e, 0)
+            grad_x = grad_x + g @ gate_w if need[0] else None
+            grad_gate_w = g.t() @ inp if need[1] else None
+            grad_gate_b = g.float().sum(dim=0).to(g.dtype) if gate_bias and need[2] else None
+        return (grad_x, grad_gate_w, grad_gate_b, grad_score if kept is None else None, grad_w1, grad_b1, grad_w2, grad_b2,
+                None, None, None, None, None)
+
+
+def _gate_logits(gate, inp, gate_w, gate_b):
+    """The logits of a gate whose linear layer stays a library product."""
+    from ._lib import GATE_LOGITS
+    return torch.nn.functional.linear(inp, gate_w, gate_b) if gate == GATE_LOGITS else None
+
+
+def layer_call(inp, gate_w, gate_b, score, w1, b1, w2, b2, routing, top_k, activation, gate):
+    r"""The layer's output through :class:`MOELayer`, or, where nothing will be differentiated, through the same call without
+    a node; ``None`` where the call does not take these tensors (see :func:`fmoe_native.layer_sizes`)."""
+    n, d = inp.shape
+    e, h = w1.shape[0], w1.shape[1]
+    params = [t for t in (gate_w, gate_b, score, w1, b1, w2, b2) if t is not None]
+    dtype, device = inp.dtype, inp.device
+    for t in params:
+        if t.dtype != dtype or t.device != device or not t.is_contiguous() or t.data_ptr() % 16 != 0:
+            return None
+    if (inp.data_ptr() % 16 != 0 or w1.shape != (e, h, d) or w2.shape != (e, d, h) or (b1 is not None and b1.shape != (e, h))
+            or (b2 is not None and b2.shape != (e, d)) or (gate_w is not None and gate_w.shape != (e, d))
+            or (gate_b is not None and gate_b.shape != (e,))):
+        return None
+    keep = torch.is_grad_enabled() and (inp.requires_grad or any(t.requires_grad for t in params))
+    sizes = fmoe_native.layer_sizes(n, d, h, e, top_k, dtype, activation, int(keep), gate)
+    if sizes is None:
+        return None
+    if keep:
+        return MOELayer.apply(inp, gate_w, gate_b, score, w1, b1, w2, b2, routing, top_k, activation, gate, sizes)
+    inp = inp.contiguous()
+    place = fmoe_native.LayerRouting() if routing is None else fmoe_native.LayerRouting(score, *routing)
+    return fmoe_native.layer_forward(inp, gate_w, gate_b, _gate_logits(gate, inp, gate_w, gate_b), w1, b1, w2, b2, top_k, activation, 0, gate,
+                                     sizes, place)[0]
+
+
+def nothing_watches(*tensors):
+    r"""Whether a call on these tensors is seen by autograd's plain reverse mode at most: no transform (vmap, forward
+    mode), trace, compiler, mode or tensor subclass that would have to see the operators of the layer one by one."""
+    return (all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors)
+            and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+            and torch._C._get_tracing_state() is None and not torch.compiler.is_compiling()
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0)
 
 
 class MOEGather(Function):

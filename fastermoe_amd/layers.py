@@ -8,8 +8,8 @@ import torch.nn as nn
 
 from . import fmoe_native
 from .functions import (AllGather, MaskRestore, MaskSelect, MOECache, MOECombine, MOEGather, MOEGatherCombine,
-                        MOELinear, MOEScatter, Slice, _PendingCounts, _prepare_forward_ex, _route_launch,
-                        _single_worker, ensure_comm, mask_index)
+                        MOELinear, MOEScatter, Slice, _no_hooks, _PendingCounts, _plain_linear, _prepare_forward_ex,
+                        _route_launch, _single_worker, ensure_comm, mask_index)
 from .gates import NaiveGate
 
 
@@ -88,6 +88,10 @@ def _fmoe_general_global_forward(inp, gate, expert_fn, policy_fn, experts, num_e
         routed = _route_launch(gate, num_expert, with_table=not enable_fuse)
         counts_dev, pos_buf, slot_to_row = routed[:3]
         if not enable_fuse:
+            if combine_score is not None:
+                x = experts.routed_layer(inp, None, None, combine_score, routed[1:], topk)
+                if x is not None:
+                    return x, torch.zeros(world_size * num_expert, dtype=torch.bool)
             x = experts.routed_forward(inp, pos_buf, slot_to_row, counts_dev, topk, routed[3])
             if x is not None:
                 stored_models = torch.zeros(world_size * num_expert, dtype=torch.bool)
@@ -260,6 +264,28 @@ class FMoE(nn.Module):
             scale = score.sum(dim=-1).contiguous()
         return MaskRestore.apply(y_k, keep_idx, token_to_row, scale, fill, fill_row)
 
+    def _gate_inside(self, inp):
+        r"""The whole layer as one call where its gate is a plain :class:`NaiveGate`, nothing between the steps is asked for
+        (a hook, a mask, another expert function) and the call takes the tensors; else ``None``."""
+        gate, experts = self.gate, self.experts
+        if (type(gate) is not NaiveGate or self.gate_hook is not None or self.mp_size > 1
+                or (self.mask is not None and self.mask_dict is not None) or not inp.is_cuda or inp.dim() != 2 or inp.shape[0] == 0
+                or gate.top_k != self.top_k or not self.experts_fused or not _own_expert_path(self.expert_fn, experts) or not _no_hooks(gate)):
+            return None
+        linear = gate._modules.get("gate")
+        if type(linear) is not nn.Linear or "weight" not in linear._parameters or "bias" not in linear._parameters:
+            return None
+        gate_w, gate_b = linear._parameters["weight"], linear._parameters["bias"]
+        if gate_w.shape[0] != self.num_expert:
+            return None
+        if not fmoe_native.gate_linear_supported(self.d_model, self.num_expert, self.top_k, inp.dtype):
+            # (more experts: the library makes the logits)
+            if not _plain_linear(linear) or torch.is_autocast_enabled():
+                return None
+        if self.enable_fuse and not experts.unchunked_is_faster(inp, inp.shape[0] * self.top_k):
+            return None
+        return experts.routed_layer(inp, gate_w, gate_b, None, None, self.top_k)
+
     def forward(self, inp):
         r"""Gate, route through the experts, and combine each token's ``top_k``
         expert outputs with the gate scores (fmoe/layers.py:272-326)."""
@@ -268,6 +294,9 @@ class FMoE(nn.Module):
         if self.mp_size > 1:
             inp = Slice.apply(inp, self.mp_rank, self.mp_size, self.mp_group)
 
+        out = self._gate_inside(inp)
+        if out is not None:
+            return out
         gate_top_k_idx, gate_score = self.gate(inp)
         if self.gate_hook is not None:
             self.gate_hook(gate_top_k_idx, gate_score, None)

@@ -5,7 +5,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib, fmoe_native
-from .functions import MOEExpertMLP, MOERoutedMLP
+from .functions import MOEExpertMLP, MOERoutedMLP, layer_call, nothing_watches
 from .gates import NaiveGate
 from .layers import FMoE, FMoELinear
 
@@ -47,6 +47,29 @@ class _Expert(nn.Module):
         params = (self.htoh4.weight, self.htoh4.bias, self.h4toh.weight, self.h4toh.bias)
         save = torch.is_grad_enabled() and (inp.requires_grad or any(p is not None and p.requires_grad for p in params))
         return MOERoutedMLP.apply(inp, *params, pos_buf, slot_to_row, table, top_k, code, save)
+
+    def routed_layer(self, inp, gate_w, gate_b, score, routing, top_k):
+        r"""The layer's output from its input as one call: with the gate's linear layer ``gate_w``, ``gate_b`` inside it, or
+        over the ``score`` and ``routing`` (``pos_buf``, ``slot_to_row`` and the segment table) of a gate outside.  ``None``
+        where that call does not apply: a subclass, replaced linears, another activation, tensors or sizes that it does not
+        take, or somebody who watches the operators."""
+        first, second = self._modules.get("htoh4"), self._modules.get("h4toh")
+        if type(self) is not _Expert or type(first) is not FMoELinear or type(second) is not FMoELinear:
+            return None
+        try:
+            params = [linear._parameters[name] for linear in (first, second) for name in ("weight", "bias")]
+        except KeyError:   # (parametrised, or a view that a sharding wrapper put there)
+            return None
+        code = self._epilogue_activation()
+        if code is None or params[0] is None or params[2] is None or not nothing_watches(inp, *(t for t in (gate_w, gate_b, score, *params) if t is not None)):
+            return None
+        if gate_w is None:
+            gate = _lib.GATE_ROUTED
+        elif fmoe_native.gate_linear_supported(inp.shape[1], gate_w.shape[0], top_k, inp.dtype):
+            gate = _lib.GATE_LINEAR
+        else:
+            gate = _lib.GATE_LOGITS
+        return layer_call(inp, gate_w, gate_b, score, *params, routing, top_k, code, gate)
 
     def unchunked_is_faster(self, inp, n_slots):
         r"""Whether :meth:`routed_forward` beats the chunked pipeline: where both linears run on the persistent
@@ -106,6 +129,8 @@ class FMoETransformerMLP(FMoE):
         self.mark_parallel_comm(expert_dp_comm)
 
     def forward(self, inp: torch.Tensor):
+        if inp.dim() == 2 and inp.shape[1] == self.d_model:
+            return super().forward(inp)
         original_shape = inp.shape
         inp = inp.reshape(-1, self.d_model)
         output = super().forward(inp)

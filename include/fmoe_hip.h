@@ -608,6 +608,64 @@ int fmoe_fused_mlp_backward(const fmoe_mlp_params *p, const void *grad_out,
                             void *grad_w2, void *grad_b2, int n_chunks,
                             void *stream);
 
+/* ---- a whole layer pass in one call ------------------------------------- */
+
+/* Where a layer pass takes its routing from: the gate's linear layer over x
+ * (gate_w, gate_b), the gate's logits, or a gate outside the call that hands in
+ * its scores and the routing of its indices. */
+#define FMOE_GATE_LINEAR 0
+#define FMOE_GATE_LOGITS 1
+#define FMOE_GATE_ROUTED 2
+
+/* 1 when the two calls below take these sizes (those of fmoe_linear_*_dev and,
+ * with the gate inside, of fmoe_gate_linear_topk_route / fmoe_gate_topk_route
+ * and fmoe_gate_weight_grad), else 0; also 0, with the sizes filled in, where the
+ * environment asks for the steps of a layer one by one (FMOE_FOLD_COMBINE=0,
+ * FMOE_EXPERT_EPILOGUE=0, FMOE_DEVICE_TABLES=0, FMOE_GATE_LINEAR_FUSED=0).
+ * sizes_host[0], [1]: bytes of scratch of a forward and, with keep, of a
+ * backward; [2]: bytes of a segment table.  Host only. */
+int fmoe_layer_sizes(int64_t n_tokens, int64_t d_model, int64_t d_hidden,
+                     int64_t n_expert, int64_t top_k, int dtype, int activation,
+                     int keep, int gate, int64_t *sizes_host);
+
+/* Gate, routing, both expert linears with the activation between them, and the
+ * score-weighted combine (FMoE.forward, fmoe/layers.py:272-326, at one worker),
+ * enqueued in one call: out [n_tokens, d_model].
+ *   topk_idx, pos, slot_to_row  int64 [n_tokens*top_k], topk_score, segment_table:
+ *       results with the gate inside, inputs with FMOE_GATE_ROUTED (topk_idx may
+ *       then be NULL); scores are the selected logits
+ *   keep != 0: what fmoe_layer_backward reads is left in pre (GELU only; else
+ *       NULL) and mid [n_tokens*top_k, d_hidden] and rows [n_tokens*top_k,
+ *       d_model].  keep == 0: those three and, with the gate inside, the routing
+ *       results are scratch and their pointers ignored.
+ *   scratch: 16-byte aligned. */
+int fmoe_layer_forward(const void *x, const void *gate_w, const void *gate_b,
+                       const void *logits, const void *w1, const void *b1,
+                       const void *w2, const void *b2, int64_t *topk_idx,
+                       void *topk_score, int64_t *pos, int64_t *slot_to_row,
+                       void *segment_table, void *pre, void *mid, void *rows,
+                       void *out, int64_t n_tokens, int64_t d_model,
+                       int64_t d_hidden, int64_t n_expert, int64_t top_k,
+                       int dtype, int activation, int keep, int gate,
+                       void *scratch, int64_t scratch_bytes, void *stream);
+
+/* Its backward.  Results, each NULL where it is not wanted: grad_x (with the
+ * gate inside: its part included, one rounding), grad_w1 (and grad_b1), grad_w2
+ * (and grad_b2); with the gate inside grad_gate_w (and grad_gate_b), else
+ * grad_score [n_tokens*top_k], which is always written.  Nothing of the forward
+ * is overwritten. */
+int fmoe_layer_backward(const void *grad_out, const void *x, const void *gate_w,
+                        const void *w1, const void *w2, const int64_t *topk_idx,
+                        const void *topk_score, const int64_t *pos,
+                        const int64_t *slot_to_row, const void *segment_table,
+                        const void *pre, const void *mid, const void *rows,
+                        void *grad_x, void *grad_score, void *grad_gate_w,
+                        void *grad_gate_b, void *grad_w1, void *grad_b1,
+                        void *grad_w2, void *grad_b2, int64_t n_tokens,
+                        int64_t d_model, int64_t d_hidden, int64_t n_expert,
+                        int64_t top_k, int dtype, int activation, int gate,
+                        void *scratch, int64_t scratch_bytes, void *stream);
+
 /* ---- per-launch timing of the library's kernels (off by default) ------- */
 
 /* Kernel classes, in the order of the arrays fmoe_profile_collect fills:
