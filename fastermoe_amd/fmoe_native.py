@@ -360,6 +360,27 @@ def prune_gate_by_capacity(gate_idx, expert_count, n_expert, n_worker):
     return out
 
 
+def limit_route(gate_idx, expert_count, slot_to_row, table, capacity):
+    """:func:`limit_by_capacity` and :func:`prune_gate_by_capacity` at one worker with one ``capacity``, and the routing of the
+    indices that stay, out of the routing (``expert_count``, ``slot_to_row``, segment ``table``) of ``gate_idx``.  Returns
+    ``(expert_count, gate_idx, pos_buf, slot_to_row, table)`` under the limit."""
+    _dev("gate_idx", gate_idx, torch.int64)
+    _dev("expert_count", expert_count, torch.int64)
+    _dev("slot_to_row", slot_to_row, torch.int64)
+    n, e = gate_idx.numel(), expert_count.numel()
+    if slot_to_row.numel() != n:
+        raise ValueError("slot_to_row must have one entry per slot")
+    _check_table(table, e, n)
+    lib = _lib.load()
+    with _on(gate_idx.device):
+        count, pruned = torch.empty_like(expert_count), torch.empty_like(gate_idx)
+        pos, s2r = torch.empty_like(slot_to_row), torch.empty_like(slot_to_row)
+        new_table, nbytes = _table_buffer(lib, n, e, gate_idx.device)
+        check(lib.fmoe_limit_route(_ptr(gate_idx), _ptr(slot_to_row), _ptr(expert_count), _ptr(table), n, e, int(capacity), _ptr(count),
+                                   _ptr(pruned), _ptr(pos), _ptr(s2r), _ptr(new_table), nbytes, _stream(gate_idx)))
+    return count, pruned, pos, s2r, new_table
+
+
 # ---- row permutes -------------------------------------------------------------
 
 def _rows(name, t):

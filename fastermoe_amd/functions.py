@@ -35,11 +35,11 @@ def _as_chunks(t):
 
 
 def _attach_route(idx, n_expert, counts, pos_buf, slot_to_row, table=None):
-    """Leaves the routing (and segment table) of a gate's indices on them for :func:`_route_launch`, with the version of
-    the tensor that they are of.  Tensors made under ``torch.inference_mode`` count no versions, so a later write to
+    """Leaves the routing (and segment table) of a gate's indices on them for :func:`_route_launch`, with the versions of
+    the tensor that they are of and of the counts, which capacity helpers hand out.  Tensors made under ``torch.inference_mode`` count no versions, so a later write to
     them would go unseen: those are routed anew."""
     if not idx.is_inference():
-        idx._fmoe_route = (idx._version, n_expert, counts, pos_buf, slot_to_row)
+        idx._fmoe_route = ((idx._version, counts._version), n_expert, counts, pos_buf, slot_to_row)
         idx._fmoe_table = table
 
 
@@ -194,7 +194,7 @@ def _route_launch(gate, num_expert, with_table=False):
     the segment table of the counts that the grouped GEMMs read."""
     with torch.no_grad():
         cached = getattr(gate, "_fmoe_route", None)
-        if cached is not None and cached[0] == gate._version and cached[1] == num_expert:
+        if cached is not None and cached[0] == (gate._version, cached[2]._version) and cached[1] == num_expert:
             if not with_table:
                 return cached[2:]
             table = getattr(gate, "_fmoe_table", None)

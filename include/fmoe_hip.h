@@ -260,6 +260,22 @@ int fmoe_prune_gate_by_capacity(const int64_t *gate_idx, int64_t *new_gate_idx,
                                 void *workspace, int64_t workspace_bytes,
                                 void *stream);
 
+/* limit_by_capacity and prune_gate_by_capacity at one worker with one capacity
+ * for all experts, and the routing of what is left (fmoe/gates/utils.py:9-26 and
+ * fmoe/functions.py:19-42), out of the routing without the limit: slot_to_row
+ * and expert_count as fmoe_route leaves them for gate_idx, segment_table of those
+ * counts and n_slots rows.  new_count[e] = min(expert_count[e], capacity); of an
+ * expert's slots those with the lowest flat index stay, the others' new_gate_idx
+ * is -1; new_pos, new_slot_to_row and new_table are the routing and the table of
+ * new_gate_idx.  At most 1024 experts; no output may alias an input. */
+int fmoe_limit_route(const int64_t *gate_idx, const int64_t *slot_to_row,
+                     const int64_t *expert_count, const void *segment_table,
+                     int64_t n_slots, int64_t n_expert, int64_t capacity,
+                     int64_t *new_count, int64_t *new_gate_idx,
+                     int64_t *new_pos, int64_t *new_slot_to_row, void *new_table,
+                     int64_t table_bytes, void *stream);
+
+
 /* ---- local scatter / gather (row permutes) ------------------------------ */
 
 /* out[r,:] = index[r] >= 0 ? inp[index[r],:] : 0   for r in [0, n_out).

@@ -568,3 +568,56 @@ def test_bytes_booked_for_the_gates_part(device):
         _lib.check(lib.fmoe_profile_collect(*(ctypes.cast(a, ctypes.c_void_p) for a in (launches, ms, work)), classes))
         _lib.check(lib.fmoe_profile_enable(0))
         assert launches[6] == 1 and work[6] == want
+
+
+@pytest.mark.parametrize("n,e,cap", [(1, 1, 0), (1, 4, 1), (64, 8, 3), (1000, 300, 2), (4097, 65, 64), (8192, 16, 1 << 30), (8192, 16, 400),
+                                     (8193, 64, 100), (40000, 1024, 40), (32768, 16, 2458), (5000, 8, 0)])
+@pytest.mark.parametrize("routed", [False, True])
+def test_limit_and_route_in_one_call(n, e, cap, routed, device):
+    """Counts, kept slots, their routing and the segment table under a capacity against the oracle and the routing of the pruned
+    indices, bit for bit; with the indices' routing at hand and without; entries that name no expert among them."""
+    from fastermoe_amd.functions import _attach_route, _route_launch
+    from fastermoe_amd.gates.utils import limit_by_capacity
+    rng = np.random.default_rng(n + e + cap)
+    p = np.arange(1, e + 1) ** -0.7
+    gate = rng.choice(e, size=n, p=p / p.sum()).astype(np.int64)
+    gate[rng.random(n) < 0.1] = -1
+    want_counts, _, want_idx = orouting.limit_and_prune(gate, e, cap)
+    if n > 100:
+        outside = rng.choice(np.flatnonzero(gate == -1), 2, replace=False)
+        gate[outside] = [e, 1 << 40]
+    idx = torch.from_numpy(gate).to(device)
+    if routed:
+        _attach_route(idx, e, *fmoe_native.route_table(idx, e))
+    counts, again, pruned = limit_by_capacity(idx, e, 1, cap)
+    assert counts is again and counts.dtype == torch.int64
+    assert np.array_equal(counts.cpu().numpy(), want_counts)
+    assert np.array_equal(pruned.cpu().numpy(), want_idx)
+    got = _route_launch(pruned, e, with_table=True)
+    assert got[0] is counts   # (the routing on the indices, not another one)
+    fresh = fmoe_native.route_table(pruned, e)
+    for a, b in zip(got[:3], fresh[:3]):
+        assert torch.equal(a, b)
+    rows, ints = int(want_counts.sum()), lambda t: t.cpu().numpy()
+    table, ref = ints(got[3]), ints(fresh[3])
+    assert table[1] == rows
+    head = 8 + 3 * (e + 1)
+    assert np.array_equal(table[:head], ref[:head])
+    for tiles, at in ((2, 4), (3, 5)):
+        lo, hi = table[at], table[at] + 4 * table[tiles]
+        assert np.array_equal(table[lo:hi], ref[lo:hi])
+    assert np.array_equal(table[-4 * e:], ref[-4 * e:])
+    counts.zero_()   # a caller's own use of the counts: the routing is made anew
+    assert torch.equal(_route_launch(pruned, e)[0], fresh[0])
+    _, _, bare = limit_by_capacity(idx.view(1, -1), e, 1, cap)
+    bare.fill_(0)    # and so it is after a write to the indices
+    assert int(_route_launch(bare, e)[0][0]) == n
+
+
+def test_capacity_of_gates_without_tokens_or_with_many_experts(device):
+    from fastermoe_amd.gates.utils import limit_by_capacity
+    counts, _, pruned = limit_by_capacity(torch.empty(0, 2, dtype=torch.int64, device=device), 4, 1, 3)
+    assert counts.tolist() == [0] * 4 and pruned.shape == (0, 2)
+    idx = torch.arange(3000, device=device) % 1500
+    counts, _, pruned = limit_by_capacity(idx, 1500, 1, 1)
+    assert counts.eq(1).all() and pruned[1500:].eq(-1).all() and torch.equal(pruned[:1500], idx[:1500])
