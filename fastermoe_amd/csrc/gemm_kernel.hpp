@@ -39,6 +39,11 @@ constexpr int kLoadWaves = 4;
 constexpr int kLoaders = 64 * kLoadWaves;
 constexpr int kRowsPerPass = kLoaders / 8;  // KC slabs: rows covered by one 16-byte load of every loading thread
 constexpr int kSlabBytes = 128;  // contraction bytes per row per slab
+// Who requests the slabs: waves that compute, or four of their own, in a workgroup that has a compute unit for itself (and LDS for
+// two slabs more ahead) or in one that shares it with a second.  See grouped_gemm_kernel, load_loop.
+enum Loaders { kLoadersCompute = 0, kLoadersAlone = 1, kLoadersShared = 2 };
+constexpr int ahead_of(int loaders) { return loaders == kLoadersAlone ? 2 : 0; }
+constexpr int extra_waves(int loaders) { return loaders == kLoadersCompute ? 0 : kLoadWaves; }
 constexpr int kGroupM = 4;       // row tiles that share a column tile consecutively (an XCD then runs 4 x 8 tiles at a time)
 
 enum Shape { kKC = 0, kMC = 1 };
@@ -216,7 +221,8 @@ struct GemmParams {
     int32_t dev_cus;
     float *dev_split_ws;
     int64_t dev_rows_cap;      // host only: rows the device table was laid out for
-    int32_t block_m, block_n;  // host only: tile height the segment table was built for (256 or 128) and tile width
+    int32_t block_m, block_n;  // host only: tile height the segment table was built for (256, 128 or 64) and tile width
+    int32_t loaders;           // host only: Loaders
     int32_t profile_class;     // host only: ProfileClass of this launch
     double profile_work;       // host only: flop of this launch
     SegmentTable tab;
@@ -283,11 +289,13 @@ template <typename T> __device__ __forceinline__ int mc_swz(int k) {
 }
 
 // ---- the kernel ---------------------------------------------------------------
-template <typename T, int BM, int BN, int PSHAPE, int QSHAPE, int RAGGED, int EPI>
-__global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const GemmParams prm) {
+template <typename T, int BM, int BN, int PSHAPE, int QSHAPE, int RAGGED, int EPI, int LOADERS>
+__global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS == kLoadersShared ? 4 : 1) void grouped_gemm_kernel(const GemmParams prm) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
     constexpr int kWavesM = waves_m_of(BN), kWaves = kWavesM * kWavesN;
-    constexpr int kThreads = threads_of(BN);
+    constexpr int kThreads = threads_of(BN);         // those that compute
+    constexpr int EXTRA = extra_waves(LOADERS);
+    static_assert(EXTRA == 0 || RAGGED == kRaggedRows, "waves that only load: the row-ragged products");
     static_assert(kWaves >= kLoadWaves && (kWaves & (kWaves - 1)) == 0, "wave layout");
     constexpr int CE = Elem<T>::kPerChunk;           // elements per 16-byte chunk
     constexpr int BKE = kSlabBytes / (int)sizeof(T); // elements per slab row
@@ -299,6 +307,7 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
     constexpr int NP = BN * 8 / kLoaders;            // 16-byte chunks per loading thread per slab
     constexpr int NQ = BM * 8 / kLoaders;
     constexpr int P_BYTES = BN * kSlabBytes, Q_BYTES = BM * kSlabBytes;
+    constexpr int kAhead = ahead_of(LOADERS);        // slabs requested beyond two
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
@@ -443,6 +452,8 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
     Cb = (T *)prm.C + aux_off;
 
     const int t = threadIdx.x;
+    // number among the loading threads (below 0: one that only computes)
+    const int lt = EXTRA ? t - kThreads : t;
     // a fixup launch runs one wave per workgroup; it stands in for wave blockIdx.x % kWaves of the tile's workgroup
     const int lane = t & 63, wave = fixup ? (int)(blockIdx.x % kWaves) : t >> 6;
     const int lb = lane & (MB - 1), hq = lane / MB;  // row inside an MFMA block, contraction chunk inside a step
@@ -479,10 +490,10 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
     constexpr int P_CPR = BN / CE, P_KPI = kLoaders / P_CPR;  // MC: chunks per k row, k rows per pass
     constexpr int Q_CPR = BM / CE, Q_KPI = kLoaders / Q_CPR;
     constexpr int kPassBytes = kLoaders * 16;  // LDS bytes filled by one 16-byte load of every loading thread
-    constexpr int kPBufs = 3;
+    constexpr int kPBufs = 3 + kAhead, kQBufs = 2 + kAhead;
     constexpr int Q_BASE = kPBufs * P_BYTES;
 
-    // Slot q = it*kLoaders + t of a slab is filled by thread t < kLoaders in pass it, so a wave fills
+    // Slot q = it*kLoaders + t of a slab is filled by loading thread t < kLoaders in pass it, so a wave fills
     // 1 KiB of consecutive LDS per load.  The swizzle is applied on the memory side: the
     // thread fetches the chunk that belongs in its slot.
     //   KC: slot q is row q/8, position q%8, and holds chunk (q%8) ^ swz(row)
@@ -490,26 +501,26 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
     uint32_t p_voff[NP], q_voff[NQ];
     int p_kc_chunk = 0, q_kc_chunk = 0;  // KC: logical chunk of this thread (same in every pass)
     if (PSHAPE == kKC) {
-        const int r = t >> 3;
-        p_kc_chunk = (t & 7) ^ swz(r);
+        const int r = lt >> 3;
+        p_kc_chunk = (lt & 7) ^ swz(r);
 #pragma unroll
         for (int it = 0; it < NP; ++it)
             p_voff[it] = (it * kRowsPerPass + r < p_valid)
                              ? (uint32_t)(((int64_t)(it * kRowsPerPass + r) * prm.ldp + p_kc_chunk * CE) * sizeof(T))
                              : kOutOfRange;
     } else {
-        const int kk = t / P_CPR;
+        const int kk = lt / P_CPR;
 #pragma unroll
         for (int it = 0; it < NP; ++it) {
-            const int c = (t % P_CPR) ^ mc_swz<T>(it * P_KPI + kk);
+            const int c = (lt % P_CPR) ^ mc_swz<T>(it * P_KPI + kk);
             p_voff[it] = (c * CE < p_valid)
                              ? (uint32_t)(((int64_t)(it * P_KPI + kk) * prm.ldp + c * CE) * sizeof(T))
                              : kOutOfRange;
         }
     }
     if (QSHAPE == kKC) {
-        const int r = t >> 3;
-        q_kc_chunk = (t & 7) ^ swz(r);
+        const int r = lt >> 3;
+        q_kc_chunk = (lt & 7) ^ swz(r);
         if (gather_q) {
             // the resource covers the whole token matrix (less than 2 GiB, checked by the host) from this
             // part's first contraction element on; a row index outside it reads as zeros
@@ -518,7 +529,7 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
             for (int it = 0; it < NQ; ++it) {
                 const int row = it * kRowsPerPass + r;
                 int64_t src = -1;
-                if (row < q_valid && t < kLoaders) {
+                if (row < q_valid && lt >= 0 && lt < kLoaders) {
                     // slot indices fit 31 bits (checked by the host), so idx / q_index_div is a multiply-high and
                     // a shift by constants the host derived from the divisor (a 64-bit division takes hundreds
                     // of instructions, and eight of them stood between a tile's start and its first loads)
@@ -538,10 +549,10 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
                                  : kOutOfRange;
         }
     } else {
-        const int kk = t / Q_CPR;
+        const int kk = lt / Q_CPR;
 #pragma unroll
         for (int it = 0; it < NQ; ++it) {
-            const int c = (t % Q_CPR) ^ mc_swz<T>(it * Q_KPI + kk);
+            const int c = (lt % Q_CPR) ^ mc_swz<T>(it * Q_KPI + kk);
             q_voff[it] = (c * CE < q_valid)
                              ? (uint32_t)(((int64_t)(it * Q_KPI + kk) * prm.ldq + c * CE) * sizeof(T))
                              : kOutOfRange;
@@ -556,7 +567,7 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
     constexpr bool kDmaAsm = (PSHAPE == kMC || QSHAPE == kMC);
     typedef int i32x4 __attribute__((ext_vector_type(4)));
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)smem;
-    const uint32_t wave_u = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wave_u = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), load_wave = EXTRA ? wave_u - kWaves : wave_u;
     auto dma_asm = [&](const T *origin, int64_t bytes, uint32_t lds_off, uint32_t voff) {
         const uint64_t a = (uint64_t)origin;
         i32x4 rs;
@@ -595,10 +606,10 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
         for (int it = 0; it < N; ++it) {
             if (it < it_lo || it >= it_hi) continue;
             if constexpr (kDmaAsm)
-                dma_asm(origin, bytes, lds_off + wave_u * 1024 + it * kPassBytes, voff[it] | past);
+                dma_asm(origin, bytes, lds_off + load_wave * 1024 + it * kPassBytes, voff[it] | past);
             else
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    rsrc, (__attribute__((address_space(3))) void *)(smem + lds_off + wave * 1024 + it * kPassBytes), 16,
+                    rsrc, (__attribute__((address_space(3))) void *)(smem + lds_off + (EXTRA ? load_wave : (uint32_t)wave) * 1024 + it * kPassBytes), 16,
                     voff[it] | past, 0, 0, 0);
         }
     };
@@ -619,6 +630,7 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
     // instead of after them, when every workgroup of the round asks memory at once.
     // Slot q of a part is row q/32, position q%32, and holds chunk (q%32) ^ (row%16).
     constexpr bool kAuxPrefetch = EPI == kEpiDAct && sizeof(T) == 2 && kDmaAsm && BN == 256;
+    static_assert(!kAuxPrefetch || EXTRA == 0, "the pre-activation tile is requested by waves that compute");
     constexpr int kAuxParts = BM / 64;
     const T *aux_tile = (const T *)prm.aux + aux_off;
     auto issue_aux = [&](int part, uint32_t lds_off) {
@@ -630,7 +642,7 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
                 const int c = (t & 31) ^ (rip & 15);
                 const bool ok = row < q_valid && c * CE < p_valid;
                 const uint32_t voff = ok ? (uint32_t)(((int64_t)row * prm.ldc + c * CE) * sizeof(T)) : kOutOfRange;
-                dma_asm(aux_tile, (int64_t)kOutOfRange, lds_off + wave_u * 1024 + it * kPassBytes, voff);
+                dma_asm(aux_tile, (int64_t)kOutOfRange, lds_off + load_wave * 1024 + it * kPassBytes, voff);
             }
         }
     };
@@ -738,7 +750,8 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
     constexpr int kPReadsPerFrag = (PSHAPE == kMC) ? (sizeof(T) == 2 ? 2 : 4) : 1;
     constexpr int kQReadsPerFrag = (QSHAPE == kMC) ? (sizeof(T) == 2 ? 2 : 4) : 1;
     constexpr int kMfma = PF * TJ * (sizeof(T) == 4 ? 4 : 1);   // MFMA instructions per phase
-    constexpr int kReadsPerMfma = 1;  // a phase's reads go out early, one per MFMA; the remaining MFMAs follow
+    // a phase's reads go out early, one per MFMA (two where they outnumber the MFMAs); the remaining MFMAs follow
+    constexpr int kReadsPerMfma = EXTRA > 0 && PF * kPReadsPerFrag + TJ * kQReadsPerFrag > kMfma ? 2 : 1;
     static_assert(NP % 2 == 0 && NP / 2 <= kMfma, "the P loads of a slab go out in two halves, one load per MFMA");
     // phases that carry the two halves: phase 3 carries the Q loads, phase 0 is left to let
     // the load queue drain (0 and 1 measured 0.5 % slower per step, all in phase 0 1 %)
@@ -787,34 +800,37 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
         constexpr bool kLoads = decltype(loads_tag)::value;  // this wave requests slabs
         constexpr int kNoWait = 63;
         if constexpr (kLoads) {
-            issue_p(0, 0);
-            issue_q(0, 0);
-            issue_p(BKE, 1);
-            issue_q(BKE, 1);
+#pragma unroll
+            for (int s = 0; s < 2 + kAhead; ++s) {
+                issue_p(s * BKE, s);
+                issue_q(s * BKE, s);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
-        wait_loads(std::integral_constant<int, kLoads ? NP + NQ : kNoWait>{});  // slab 0 has landed
+        wait_loads(std::integral_constant<int, kLoads ? (1 + kAhead) * (NP + NQ) : kNoWait>{});  // slab 0 has landed
         slab_barrier();
         if constexpr (kBias) add_q_chunks(0);
         read_phase(0, smem, smem + Q_BASE);
         __builtin_amdgcn_sched_barrier(0);
 
-        int pc = 0;
+        int pc = 0, qk = 0;
         for (int s = 0; s < n_slabs; ++s) {
             const int pn = pc == kPBufs - 1 ? 0 : pc + 1;
-            const int pf_buf = pn == kPBufs - 1 ? 0 : pn + 1;
+            // receives the P part of slab s + 2 + kAhead: the buffer before this slab's
+            const int pf_buf = kAhead == 0 ? (pn == kPBufs - 1 ? 0 : pn + 1) : (pc == 0 ? kPBufs - 1 : pc - 1);
+            const int qc = kAhead == 0 ? (s & 1) : qk, qn = kAhead == 0 ? ((s + 1) & 1) : (qk == kQBufs - 1 ? 0 : qk + 1);
             const unsigned char *sp = smem + pc * P_BYTES;
-            const unsigned char *sq = smem + Q_BASE + (s & 1) * Q_BYTES;
+            const unsigned char *sq = smem + Q_BASE + qc * Q_BYTES;
 #pragma unroll
             for (int ph = 0; ph + 1 < kPhases; ++ph) {
                 if (kLoads && ph == kPLoadPhaseA) {
                     const int past_end = s + 2 - n_slabs;  // >= 0: slab s+2 does not exist
                     if (kAuxPrefetch && aux_pref && past_end >= 0) issue_aux(past_end, (uint32_t)(pf_buf * P_BYTES));
-                    else issue_p((s + 2) * BKE, pf_buf, 0, NP / 2);
+                    else issue_p((s + 2 + kAhead) * BKE, pf_buf, 0, NP / 2);
                 }
                 if (kLoads && ph == kPLoadPhaseB) {  // the second half of the P loads (the pre-activation part went out whole)
                     const int past_end = s + 2 - n_slabs;
-                    if (!(kAuxPrefetch && aux_pref && past_end >= 0)) issue_p((s + 2) * BKE, pf_buf, NP / 2, NP);
+                    if (!(kAuxPrefetch && aux_pref && past_end >= 0)) issue_p((s + 2 + kAhead) * BKE, pf_buf, NP / 2, NP);
                 }
                 read_phase(ph + 1, sp, sq);
                 mma_phase(ph, 0, PF);
@@ -826,7 +842,8 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            wait_loads(std::integral_constant<int, kLoads ? NP : kNoWait>{});  // everything but the P loads of slab s+2
+            // everything but the P loads of slab s+2 (and of kAhead whole slabs, which those then follow)
+            wait_loads(std::integral_constant<int, kLoads ? NP + kAhead * (NP + NQ) : kNoWait>{});
             slab_barrier();
             if constexpr (kBias) add_q_chunks((s + 1) & 1);
             if constexpr (kLoads) {
@@ -834,9 +851,9 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
                 if (kAuxPrefetch && kAuxParts == 4 && aux_pref && past_end >= 0)
                     issue_aux(2 + past_end, (uint32_t)(Q_BASE + (s & 1) * Q_BYTES));
                 else
-                    issue_q((s + 2) * BKE, s & 1);
+                    issue_q((s + 2 + kAhead) * BKE, qc);
             }
-            read_phase(0, smem + pn * P_BYTES, smem + Q_BASE + ((s + 1) & 1) * Q_BYTES);
+            read_phase(0, smem + pn * P_BYTES, smem + Q_BASE + qn * Q_BYTES);
             mma_phase(kPhases - 1, 0, PF);
             constexpr int kQLoadsPerMfma = (NQ + kMfma - 1) / kMfma;
 #pragma unroll
@@ -847,15 +864,49 @@ __global__ __launch_bounds__(threads_of(BN)) void grouped_gemm_kernel(const Gemm
             }
             __builtin_amdgcn_sched_barrier(0);
             pc = pn;
+            qk = qn;
         }
         // the loads requested past the last slab (all out of range) must land before LDS is reused
         wait_loads(std::integral_constant<int, 0>{});
         slab_barrier();
     };
+    // The same slabs and barriers for a wave that only loads.  Where a launch leaves a compute unit one workgroup of four waves, a
+    // wave's loads (35 ns each, during which it issues nothing else), its LDS reads and its products follow one another;
+    // apart they overlap, and with the LDS of a whole unit four slabs are on their way.
+    auto load_loop = [&]() {
+#pragma unroll
+        for (int s = 0; s < 2 + kAhead; ++s) {
+            issue_p(s * BKE, s);
+            issue_q(s * BKE, s);
+        }
+        wait_loads(std::integral_constant<int, (1 + kAhead) * (NP + NQ)>{});
+        slab_barrier();
+        int pb = 2 + kAhead, qb = 0;
+        for (int s = 0; s < n_slabs; ++s) {
+            issue_p((s + 2 + kAhead) * BKE, pb);
+            wait_loads(std::integral_constant<int, NP + kAhead * (NP + NQ)>{});
+            slab_barrier();
+            issue_q((s + 2 + kAhead) * BKE, qb);
+            pb = pb == kPBufs - 1 ? 0 : pb + 1;
+            qb = qb == kQBufs - 1 ? 0 : qb + 1;
+        }
+        wait_loads(std::integral_constant<int, 0>{});
+        slab_barrier();
+    };
     auto run_loop = [&](auto with_bias) {
+        if constexpr (EXTRA > 0) {
+            main_loop(with_bias, std::false_type{});
+            return;
+        }
         if (wave_u < (uint32_t)kLoadWaves) main_loop(with_bias, std::true_type{});
         else main_loop(with_bias, std::false_type{});
     };
+    if constexpr (EXTRA > 0) {
+        if (wave_u >= (uint32_t)kWaves) {
+            load_loop();
+            return;
+        }
+    }
     bool want_bias = false;
     if constexpr (RAGGED == kRaggedK && QSHAPE == kMC) want_bias = prm.bias_grad != nullptr && nt == 0;
     if constexpr (RAGGED == kRaggedK && QSHAPE == kMC) {
@@ -1194,11 +1245,12 @@ __global__ __launch_bounds__(256) void split_reduce_dev_kernel(float *ws, const 
 int device_compute_units();
 float *split_workspace(hipStream_t stream, size_t bytes);
 
-template <typename T, int BM, int BN, int PS, int QS, int RG, int EPI>
+template <typename T, int BM, int BN, int PS, int QS, int RG, int EPI, int LOADERS>
 int launch_tiles(GemmParams &prm, hipStream_t stream) {
     constexpr int kWavesM = waves_m_of(BN), kThreads = threads_of(BN);
-    // three P and two Q slab buffers, or the epilogue's staging area (one [rows][row piece + 16 B] block per wave)
-    constexpr int smem_loop = (3 * BN + 2 * BM) * kSlabBytes;
+    // three P and two Q slab buffers (and those of the slabs further ahead), or the epilogue's staging area (one [rows][row piece + 16 B] block per wave)
+    constexpr int kAhead = ahead_of(LOADERS);
+    constexpr int smem_loop = ((3 + kAhead) * BN + (2 + kAhead) * BM) * kSlabBytes;
     constexpr int wave_cols_bytes = BN / kWavesN * (int)sizeof(T);
     constexpr int smem_wave_epi = (BM / kWavesM) * ((wave_cols_bytes < 256 ? wave_cols_bytes : 256) + 16);
     constexpr int smem_epi = kWavesM * kWavesN * smem_wave_epi;
@@ -1206,7 +1258,7 @@ int launch_tiles(GemmParams &prm, hipStream_t stream) {
     // the opt-in to more than 64 KiB of dynamic LDS is per device (and per kernel instantiation)
     // (0: not tried yet, 1: done, 2: failed -- a failure is reported by every later launch too)
     static std::atomic<int> configured[16];
-    auto kern = grouped_gemm_kernel<T, BM, BN, PS, QS, RG, EPI>;
+    auto kern = grouped_gemm_kernel<T, BM, BN, PS, QS, RG, EPI, LOADERS>;
     int dev = 0;
     FMOE_HIP_CHECK(hipGetDevice(&dev));
     FMOE_REQUIRE(dev >= 0 && dev < 16, "device index %d out of range", dev);
@@ -1258,7 +1310,7 @@ int launch_tiles(GemmParams &prm, hipStream_t stream) {
     if (grid64 > (int64_t)INT32_MAX) return fail(FMOE_ELIMIT, "grouped GEMM: grid of %lld workgroups", (long long)grid64);
     const int grid = (int)grid64;
     ProfileScope prof(prm.profile_class, prm.profile_work, stream);
-    kern<<<grid, kThreads, smem, stream>>>(prm);
+    kern<<<grid, kThreads + 64 * extra_waves(LOADERS), smem, stream>>>(prm);
     FMOE_LAUNCH_CHECK();
     if (prm.k_split > 1) {
         // the parts are complete when the first launch has ended: add them up, then run the epilogue,
@@ -1292,7 +1344,7 @@ int launch_tiles(GemmParams &prm, hipStream_t stream) {
 // 128 x 256, 128 x 128 or, fp32 alone, 64 x 64, chosen by the host from the segment lengths) is the tile.
 // EPI_MASK lists the epilogues a product can be asked for, so that only those kernels
 // are built.
-template <typename T, int BM, int BN, int PS, int QS, int RG, int EPI_MASK>
+template <typename T, int BM, int BN, int PS, int QS, int RG, int EPI_MASK, int LOADERS = kLoadersCompute>
 int launch_for_height(GemmParams &prm, int epi, hipStream_t stream) {
     prm.tiles_n = (int)ceil_div(prm.n_cols, BN);
     int64_t total;
@@ -1311,11 +1363,11 @@ int launch_for_height(GemmParams &prm, int epi, hipStream_t stream) {
     if (total > (int64_t)INT32_MAX - 8) return fail(FMOE_ELIMIT, "grouped GEMM: %lld tiles exceed the grid limit", (long long)total);
     prm.total_tiles = (int)total;
     if constexpr ((EPI_MASK >> kEpiStore) & 1)
-        if (epi == kEpiStore) return launch_tiles<T, BM, BN, PS, QS, RG, kEpiStore>(prm, stream);
+        if (epi == kEpiStore) return launch_tiles<T, BM, BN, PS, QS, RG, kEpiStore, LOADERS>(prm, stream);
     if constexpr ((EPI_MASK >> kEpiBiasAct) & 1)
-        if (epi == kEpiBiasAct) return launch_tiles<T, BM, BN, PS, QS, RG, kEpiBiasAct>(prm, stream);
+        if (epi == kEpiBiasAct) return launch_tiles<T, BM, BN, PS, QS, RG, kEpiBiasAct, LOADERS>(prm, stream);
     if constexpr ((EPI_MASK >> kEpiDAct) & 1)
-        if (epi == kEpiDAct) return launch_tiles<T, BM, BN, PS, QS, RG, kEpiDAct>(prm, stream);
+        if (epi == kEpiDAct) return launch_tiles<T, BM, BN, PS, QS, RG, kEpiDAct, LOADERS>(prm, stream);
     return fail(FMOE_EINVAL, "epilogue %d is not built for this product", epi);
 }
 
@@ -1323,7 +1375,14 @@ template <typename T, int PS, int QS, int RG, int EPI_MASK>
 int launch_by_epilogue(GemmParams &prm, int epi, hipStream_t stream) {
     if constexpr (sizeof(T) == 4)
         if (prm.block_m == 64 && prm.block_n == 64) return launch_for_height<T, 64, 64, PS, QS, RG, EPI_MASK>(prm, epi, stream);
-    if (prm.block_m == 128 && prm.block_n == 128) return launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK>(prm, epi, stream);
+    if constexpr (sizeof(T) == 2 && RG == kRaggedRows)
+        if (prm.block_n == 128) {
+            if (prm.block_m == 64) return launch_for_height<T, 64, 128, PS, QS, RG, EPI_MASK, kLoadersAlone>(prm, epi, stream);
+            return prm.loaders == kLoadersAlone ? launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK, kLoadersAlone>(prm, epi, stream)
+                                                : launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK, kLoadersShared>(prm, epi, stream);
+        }
+    if constexpr (sizeof(T) == 4 || RG == kRaggedK)
+        if (prm.block_m == 128 && prm.block_n == 128) return launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK>(prm, epi, stream);
     if (prm.block_m == 128 && prm.block_n == 256) return launch_for_height<T, 128, 256, PS, QS, RG, EPI_MASK>(prm, epi, stream);
     if (prm.block_m == 256 && prm.block_n == 256) return launch_for_height<T, 256, 256, PS, QS, RG, EPI_MASK>(prm, epi, stream);
     return fail(FMOE_EINVAL, "tile %d x %d is not built", prm.block_m, prm.block_n);

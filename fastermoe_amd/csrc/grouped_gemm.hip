@@ -85,25 +85,26 @@ void fill_table(SegmentTable *tab, const int64_t *counts, int e0, int e1, int64_
     tab->tile[tab->n] = tiles;
 }
 
-// Tile of a launch.  256 x 256 (one workgroup per compute unit) unless that gives too few tiles
-// to occupy the chip: then 128 x 256, and when even those number fewer than two per compute unit,
-// 128 x 128 (two workgroups per compute unit).  (Lower tiles to cut the padding of short segments
-// were measured and lost: with ~256 rows per expert the product is bound by streaming the weights,
-// which a lower tile re-reads more often; and 128 x 128 tiles lose a quarter of the rate of large
-// launches, because they read each operand from L2 and LDS more often per flop.)
-// FMOE_GEMM_TILE=256x256|128x256|128x128|64x64 (the last for fp32 only) forces one shape (for tests and measurements).
-//
-// fp32 tiles take four times as long per slab and are bound by the matrix pipe whatever their shape, so there the
-// question is only how evenly they fill the chip: f32_rows_tile, f32_wgrad_tile.
+// Tile of a launch.  Weight gradients of 16-bit types: 256 x 256 (one workgroup per compute unit) unless that gives too few tiles
+// to occupy the chip: then 128 x 256, and when even those number fewer than two per compute unit, 128 x 128 (two workgroups per
+// compute unit).  Their row-ragged products: rows_16bit_tile.  fp32 tiles take four times as long per slab and are bound by the
+// matrix pipe whatever their shape, so there the question is only how evenly they fill the chip: f32_rows_tile, f32_wgrad_tile.
+// FMOE_GEMM_TILE=256x256|128x256|128x128 forces one shape (for tests and measurements); for fp32 also 64x64, for the row-ragged
+// products of 16-bit types also 64x128 and, one workgroup per compute unit, 128x128+.
 struct TileShape {
     int bm, bn;
+    int loaders = kLoadersCompute;
+    bool many = false;   // enough 256 x 256 tiles for the persistent kernel
 };
-bool forced_tile(int dtype, TileShape *tile) {
+bool is_16bit(int dtype) { return dtype == FMOE_BF16 || dtype == FMOE_F16; }
+bool forced_tile(int dtype, bool rows, TileShape *tile) {
     const char *e = getenv("FMOE_GEMM_TILE");
     if (!e) return false;
     if (!strcmp(e, "256x256")) *tile = {256, 256};
     else if (!strcmp(e, "128x256")) *tile = {128, 256};
-    else if (!strcmp(e, "128x128")) *tile = {128, 128};
+    else if (!strcmp(e, "128x128")) *tile = {128, 128, rows && is_16bit(dtype) ? kLoadersShared : kLoadersCompute};
+    else if (!strcmp(e, "128x128+") && rows && is_16bit(dtype)) *tile = {128, 128, kLoadersAlone};
+    else if (!strcmp(e, "64x128") && rows && is_16bit(dtype)) *tile = {64, 128, kLoadersAlone};
     else if (!strcmp(e, "64x64") && dtype == FMOE_F32) *tile = {64, 64};
     else return false;
     return true;
@@ -136,9 +137,53 @@ TileShape f32_wgrad_tile(int64_t experts, int64_t out_feat, int64_t in_feat, int
     return 105 * low < 100 * high ? TileShape{64, 64} : TileShape{128, 128};
 }
 
+constexpr TileShape kManyTiles{256, 256, kLoadersCompute, true};
 TileShape pick_tile(int64_t tiles_256) {
-    if (tiles_256 >= 512) return {256, 256};
+    if (tiles_256 >= 512) return kManyTiles;
     return tiles_256 >= 256 ? TileShape{128, 256} : TileShape{128, 128};
+}
+
+// Row-ragged products in 16 bits with fewer than 512 tiles of 256 x 256: the shape with the least time by this estimate.  A round
+// of tiles that fills a share f of the chip's places takes start + slabs (alone + shared f) us, the accumulators' way out
+// included; the last round may be a partial one.  Below that the weights' way from memory is the bound.  The constants are fitted to
+// 204 products of 4 to 128 experts, 64 to 16384 rows and 512 to 8192 features, one fit per shape, a tenth of a launch's time
+// off on average; the shape that the estimate picks took 0.867 times what 128 x 128 tiles below 256 tiles of 256 x 256 and 128 x 256 from there on
+// did, the best of the five 0.84 times.  us for 64 x 128 / 128 x 128 alone / 128 x 128 shared / 128 x 256 / 256 x 256 (and 128 x 128 without
+// loading waves): 8 experts of 1024 x 4096, 1024 rows: 22 / 31 / 43 / - / - (51); 16 of 768 x 3072, 2000: 21 / 25 / 31 / 36 / 53 (37);
+// 8 of 2048 x 2048, 1600: 26 / 19 / 24 / 27 / 39 (28); 8 of 1024 x 1024, 4000: 23 / 21 / 18 / 17 / 25 (21); 12 of 2112 x 2112, 5000:
+// - / 69 / 62 / 59 / 47 (71); 8 of 2048 -> 1024, 8192: - / 50 / 50 / 54 / 42 (57); 64 of 2048 -> 8192, 509: 534 / 393 / 398 / 383 / 407 (378).
+struct RowShape {
+    TileShape tile;
+    int per_unit;                        // workgroups on a compute unit
+    double start, alone, shared, stream; // us, us per slab, TB/s
+};
+constexpr RowShape kRowShapes[] = {
+    {{64, 128, kLoadersAlone}, 1, 2.9, 0.21, 0.13, 3.9},     {{128, 128, kLoadersAlone}, 1, 3.3, 0.26, 0.24, 4.8},
+    {{128, 128, kLoadersShared}, 2, 3.1, 0.30, 0.71, 4.9},   {{128, 256, kLoadersCompute}, 1, 4.2, 0.38, 0.53, 5.2},
+    {{256, 256, kLoadersCompute}, 1, 6.9, 0.57, 0.83, 5.0},
+};
+template <typename RowTiles> TileShape rows_16bit_tile(RowTiles row_tiles, double weight_bytes, int64_t n_cols, int64_t contraction) {
+    const double slabs = (double)ceil_div(contraction, 64);
+    const int64_t units = device_compute_units();
+    double best = 0;
+    TileShape pick{};
+    for (const RowShape &s : kRowShapes) {
+        const int64_t tiles = row_tiles(s.tile.bm) * ceil_div(n_cols, s.tile.bn), places = units * s.per_unit;
+        const int64_t full = tiles / places, rest = tiles % places;
+        double us = (double)full * (s.start + slabs * (s.alone + s.shared));
+        if (rest) {
+            const TailSplit split = s.tile.bm == 64 ? TailSplit{0, 1, 0} : plan_tail_split((int)std::min<int64_t>(tiles, INT32_MAX), (int)slabs, (int)units);
+            if (split.k_split > 1 && full == 0)   // (and two short kernels after it)
+                us += 8 + s.start + split.split_slabs * (s.alone + s.shared * (double)(rest * split.k_split) / (double)places);
+            else
+                us += s.start + slabs * (s.alone + s.shared * (double)rest / (double)places);
+        }
+        // (a few large tiles cannot ask for the weights fast enough)
+        const double share = s.tile.bn == 256 ? std::min(1.0, (double)tiles * 1.6 / (double)units) : 1.0;
+        us = std::max(us + 3, weight_bytes * 1e-6 / (s.stream * share) + 4);
+        if (pick.bm == 0 || us < best) { best = us; pick = s.tile; }
+    }
+    return pick;
 }
 
 // The activation code the kernels see.  For results that are rounded to a 16-bit type GELU and its
@@ -157,26 +202,39 @@ int kernel_activation(int activation) {
 TileShape pick_rows_tile(const int64_t *counts, int64_t n_expert, int64_t row_lo, int64_t row_hi, int64_t n_cols,
                          int64_t contraction, int dtype) {
     TileShape forced;
-    if (forced_tile(dtype, &forced)) return forced;
-    int64_t start = 0, row_tiles = 0;
-    for (int64_t e = 0; e < n_expert; ++e) {
-        const int64_t end = start + counts[e];
-        const int64_t lo = start < row_lo ? row_lo : start, hi = end > row_hi ? row_hi : end;
-        if (hi > lo) row_tiles += ceil_div(hi - lo, 256);
-        start = end;
-    }
-    const int64_t tiles = row_tiles * ceil_div(n_cols, 256);
-    return dtype == FMOE_F32 ? f32_rows_tile(tiles, contraction) : pick_tile(tiles);
+    if (forced_tile(dtype, true, &forced)) return forced;
+    auto row_tiles = [&](int height) {
+        int64_t start = 0, tiles = 0;
+        for (int64_t e = 0; e < n_expert; ++e) {
+            const int64_t end = start + counts[e];
+            const int64_t lo = start < row_lo ? row_lo : start, hi = end > row_hi ? row_hi : end;
+            if (hi > lo) tiles += ceil_div(hi - lo, height);
+            start = end;
+        }
+        return tiles;
+    };
+    const int64_t tiles = row_tiles(256) * ceil_div(n_cols, 256);
+    if (dtype == FMOE_F32) return f32_rows_tile(tiles, contraction);
+    if (tiles >= 512) return kManyTiles;
+    const double live = (double)row_tiles(INT32_MAX);   // (experts with rows)
+    return rows_16bit_tile(row_tiles, live * (double)n_cols * (double)contraction * 2, n_cols, contraction);
 }
 
 // ragged rows over a device table: the host does not know the counts; rows_cap rows spread over
 // the experts make about rows_cap / 256 whole tiles plus a partial one for every other expert
 TileShape pick_rows_tile_estimate(int64_t rows_cap, int64_t n_expert, int64_t n_cols, int64_t contraction, int dtype) {
     TileShape forced;
-    if (forced_tile(dtype, &forced)) return forced;
+    if (forced_tile(dtype, true, &forced)) return forced;
     const int64_t whole = rows_cap / 256;
     const int64_t tiles = (whole + std::min<int64_t>(n_expert, std::max<int64_t>(whole, 1)) / 2) * ceil_div(n_cols, 256);
-    return dtype == FMOE_F32 ? f32_rows_tile(tiles, contraction) : pick_tile(tiles);
+    if (dtype == FMOE_F32) return f32_rows_tile(tiles, contraction);
+    if (tiles >= 512) return kManyTiles;
+    // every expert that can have a row, with its share of the rows and half a tile past the whole ones
+    const int64_t live = std::max<int64_t>(1, std::min(n_expert, rows_cap));
+    auto row_tiles = [&](int height) {
+        return (int64_t)((double)live * std::max(1.0, (double)rows_cap / ((double)live * height) + 0.5) + 0.5);
+    };
+    return rows_16bit_tile(row_tiles, (double)live * (double)n_cols * (double)contraction * 2, n_cols, contraction);
 }
 
 // Row tiles of gemm_unaligned.hip, 64 or 128 rows high: the low ones where the high ones would leave part of the
@@ -195,7 +253,7 @@ TileShape pick_unaligned_tile(const int64_t *counts, int64_t n_expert, int64_t r
 // weight gradient: C is [out, in] per expert
 TileShape pick_wgrad_tile(int64_t n_experts_written, int64_t out_feat, int64_t in_feat, int64_t rows, int dtype) {
     TileShape forced;
-    if (forced_tile(dtype, &forced)) return forced;
+    if (forced_tile(dtype, false, &forced)) return forced;
     if (dtype == FMOE_F32) return f32_wgrad_tile(n_experts_written, out_feat, in_feat, rows);
     return pick_tile(n_experts_written * ceil_div(out_feat, 256) * ceil_div(in_feat, 256));
 }
@@ -281,8 +339,6 @@ std::mutex g_split_mutex;
 std::vector<SplitBuffer> g_split_buffers;
 int g_compute_units[16] = {};
 
-bool is_16bit(int dtype) { return dtype == FMOE_BF16 || dtype == FMOE_F16; }
-
 template <int PRODUCT>
 int dispatch(GemmParams &prm, int dtype, int epi, bool fast, hipStream_t stream) {
     // Shapes off the 16-byte grid: 16-bit types in gemm_unaligned.hip, the others and double precision on the
@@ -310,7 +366,7 @@ int dispatch(GemmParams &prm, int dtype, int epi, bool fast, hipStream_t stream)
 // measured: 4 to 9 % faster at K = 4096, 7 to 14 % at K = 1024, 26 to 37 % on weight gradients of 64 to 256 rows per
 // expert.  32-bit tiles take four times as long per slab, so what happens between them hardly shows.
 bool use_ring(const TileShape &tile, int dtype) {
-    return tile.bm == 256 && tile.bn == 256 && (dtype == FMOE_BF16 || dtype == FMOE_F16) && !getenv("FMOE_GEMM_TILE");
+    return tile.many && is_16bit(dtype);
 }
 
 // Whether a forward launch over a device table goes to gemm_skinny.hip: 16-bit types (no tile shape forced) and at
@@ -467,7 +523,7 @@ int64_t linear_dev_workspace_bytes(int64_t contraction, int dtype) {
     const int eb = dtype_bytes(dtype);
     if (eb == 0 || dtype == FMOE_F64 || contraction < 1) return 0;
     // the most that any launch of this contraction can use: 256 x 256 tiles, on the persistent kernel for 16-bit types
-    const DevRoute tiles{DevKernel::kTiles, {256, 256}}, ring{DevKernel::kRing, {256, 256}};
+    const DevRoute tiles{DevKernel::kTiles, {256, 256}}, ring{DevKernel::kRing, kManyTiles};
     return std::max(route_workspace_bytes(tiles, contraction, dtype), eb == 2 ? route_workspace_bytes(ring, contraction, dtype) : 0);
 }
 
@@ -486,7 +542,7 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
         prm.activation = kernel_activation(a.activation);
         const DevRoute route = forward_route(a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype, a.epilogue, prm.activation,
                                              a.aux != nullptr, a.x_row_index != nullptr);
-        prm.block_m = route.tile.bm; prm.block_n = route.tile.bn;
+        prm.block_m = route.tile.bm; prm.block_n = route.tile.bn; prm.loaders = route.tile.loaders;
         prm.profile_class = kProfGemmFwd; prm.profile_work = 2.0 * (double)a.dev_rows_cap * (double)a.in_feat * (double)a.out_feat;
         prm.P = a.w; prm.Q = a.x; prm.C = a.y; prm.bias = a.bias; prm.aux = a.aux;
         prm.q_row_index = a.x_row_index; set_row_index_divisor(prm, a.x_index_div); prm.q_total_rows = a.x_total_rows;
@@ -525,7 +581,7 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
     for (int e0 = plan.first; e0 <= plan.last; e0 += kMaxGroupExperts) {
         const int e1 = std::min(plan.last, e0 + kMaxGroupExperts - 1);
         GemmParams prm{};
-        prm.block_m = tile.bm; prm.block_n = tile.bn;
+        prm.block_m = tile.bm; prm.block_n = tile.bn; prm.loaders = tile.loaders;
         fill_table(&prm.tab, counts, e0, e1, row_lo, row_hi, tile.bm);
         prm.profile_class = kProfGemmFwd; prm.profile_work = table_flop(prm.tab, a.in_feat, a.out_feat);
         prm.P = a.w; prm.Q = a.x; prm.C = a.y; prm.bias = a.bias; prm.aux = a.aux;
@@ -552,7 +608,7 @@ int grouped_linear_dgrad(const LinearDgradArgs &a, const int64_t *counts, int64_
         if (int rc = device_table_launch("linear_dgrad", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast)) return rc;
         prm.activation = kernel_activation(a.activation);
         const DevRoute route = dgrad_route(a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype, a.epilogue, prm.activation);
-        prm.block_m = route.tile.bm; prm.block_n = route.tile.bn;
+        prm.block_m = route.tile.bm; prm.block_n = route.tile.bn; prm.loaders = route.tile.loaders;
         prm.profile_class = kProfGemmDgrad; prm.profile_work = 2.0 * (double)a.dev_rows_cap * (double)a.in_feat * (double)a.out_feat;
         prm.P = a.w; prm.Q = a.gy; prm.C = a.gx; prm.aux = const_cast<void *>(a.aux);
         prm.ldp = a.in_feat; prm.ldq = a.out_feat; prm.ldc = a.in_feat;
@@ -575,7 +631,7 @@ int grouped_linear_dgrad(const LinearDgradArgs &a, const int64_t *counts, int64_
     for (int e0 = plan.first; e0 <= plan.last; e0 += kMaxGroupExperts) {
         const int e1 = std::min(plan.last, e0 + kMaxGroupExperts - 1);
         GemmParams prm{};
-        prm.block_m = tile.bm; prm.block_n = tile.bn;
+        prm.block_m = tile.bm; prm.block_n = tile.bn; prm.loaders = tile.loaders;
         fill_table(&prm.tab, counts, e0, e1, row_lo, row_hi, tile.bm);
         prm.profile_class = kProfGemmDgrad; prm.profile_work = table_flop(prm.tab, a.in_feat, a.out_feat);
         prm.P = a.w; prm.Q = a.gy; prm.C = a.gx; prm.aux = const_cast<void *>(a.aux);
@@ -599,7 +655,7 @@ int grouped_linear_wgrad(const LinearWgradArgs &a, const int64_t *counts, int64_
         const TileShape tile = pick_wgrad_tile(n_expert, a.out_feat, a.in_feat, a.dev_rows_cap, a.dtype);
         GemmParams prm{};
         if (int rc = device_table_launch("linear_wgrad", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast)) return rc;
-        prm.block_m = tile.bm; prm.block_n = tile.bn;
+        prm.block_m = tile.bm; prm.block_n = tile.bn; prm.loaders = tile.loaders;
         prm.profile_class = kProfGemmWgrad; prm.profile_work = 2.0 * (double)a.dev_rows_cap * (double)a.in_feat * (double)a.out_feat;
         prm.P = a.x; prm.Q = a.gy; prm.C = a.gw; prm.bias_grad = a.gb;
         prm.ldp = a.in_feat; prm.ldq = a.out_feat; prm.ldc = a.in_feat;
@@ -620,7 +676,7 @@ int grouped_linear_wgrad(const LinearWgradArgs &a, const int64_t *counts, int64_
     for (int e0 = plan.first; e0 <= plan.last; e0 += kMaxGroupExperts) {
         const int e1 = std::min(plan.last, e0 + kMaxGroupExperts - 1);
         GemmParams prm{};
-        prm.block_m = tile.bm; prm.block_n = tile.bn;
+        prm.block_m = tile.bm; prm.block_n = tile.bn; prm.loaders = tile.loaders;
         fill_table(&prm.tab, counts, e0, e1, row_lo, row_hi, tile.bm);
         prm.profile_class = kProfGemmWgrad; prm.profile_work = table_flop(prm.tab, a.in_feat, a.out_feat);
         prm.P = a.x; prm.Q = a.gy; prm.C = a.gw; prm.bias_grad = fast || is_16bit(a.dtype) ? a.gb : nullptr;
