@@ -46,7 +46,7 @@ template <typename T> __device__ __forceinline__ u32x4 load_part(const T *p, con
     return __builtin_bit_cast(u32x4, e);
 }
 
-// PSHAPE / QSHAPE: kKC = [index][contraction] in memory, kMC = [contraction][index]; host segment table only.
+// PSHAPE / QSHAPE: kKC = [index][contraction] in memory, kMC = [contraction][index].
 template <typename T, int BM, int PSHAPE, int QSHAPE, int RAGGED>
 __global__ __launch_bounds__(kUaThreads) void grouped_gemm_unaligned_kernel(const GemmParams prm) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
@@ -61,34 +61,56 @@ __global__ __launch_bounds__(kUaThreads) void grouped_gemm_unaligned_kernel(cons
     const int wm = wave >> 1, wn = wave & 1, lb = lane & 15, hq = lane >> 4;
 
     // -- which tile: a contiguous eighth of the logical order per XCD, kGroupM row tiles per column tile
-    const int per_xcd = (prm.total_tiles + 7) >> 3;
-    const int L = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per_xcd || L >= prm.total_tiles) return;
-    int ei = 0, rem = L, tm_total = prm.tiles_m;
+    // (over a device table the launch is sized for the most tiles there can be)
+    typedef const int32_t __attribute__((address_space(4))) *DevTab;    // read-only, uniform: scalar loads
+    const DevTab dtab = (DevTab)(uintptr_t)prm.dev_tab;
+    const bool dev = prm.dev_tab != nullptr;
+    int tm_total = prm.tiles_m, total_tiles = prm.total_tiles;
     if (RAGGED == kRaggedRows) {
-        tm_total = prm.tab.tile[prm.tab.n];
-    } else {
+        tm_total = dev ? dtab[segtab::kTiles128] * (128 / BM) : prm.tab.tile[prm.tab.n];
+        total_tiles = tm_total * prm.tiles_n;
+    }
+    const int per_xcd = (total_tiles + 7) >> 3;
+    const int L = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || L >= total_tiles) return;
+    int ei = 0, rem = L;
+    if (RAGGED == kRaggedK) {
         ei = L / (prm.tiles_m * prm.tiles_n);
         rem = L - ei * (prm.tiles_m * prm.tiles_n);
     }
     const int grp = rem / (kGroupM * prm.tiles_n), in_grp = rem - grp * kGroupM * prm.tiles_n;
     const int gsz = min(kGroupM, tm_total - grp * kGroupM);
     const int nt = in_grp / gsz, mt = grp * kGroupM + in_grp - nt * gsz;
-    if (RAGGED == kRaggedRows) {
+    int seg_lo, seg_hi, row0 = 0;   // (ragged rows over a device table: of this very tile)
+    if (RAGGED == kRaggedRows && dev) {
+        typedef int i32x4 __attribute__((ext_vector_type(4)));
+        typedef const i32x4 __attribute__((address_space(4))) *DevTab4;
+        constexpr int kPerEntry = 128 / BM;   // (tiles of 64 rows: the halves of the map's 128; the second may have no rows)
+        const i32x4 entry = *(DevTab4)(dtab + prm.dev_map_off + 4 * (mt / kPerEntry));
+        ei = entry[0];
+        seg_hi = entry[1] + entry[2];
+        row0 = seg_lo = entry[1] + (mt % kPerEntry) * BM;
+        if (seg_lo >= seg_hi) return;
+    } else if (RAGGED == kRaggedRows) {
         int lo = 0, hi = prm.tab.n;  // tile[lo] <= mt < tile[hi]
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
             if (prm.tab.tile[mid] <= mt) lo = mid; else hi = mid;
         }
         ei = lo;
+        seg_lo = prm.tab.seg[ei];
+        seg_hi = prm.tab.seg[ei + 1];
+        row0 = seg_lo + (mt - prm.tab.tile[ei]) * BM;
+    } else {
+        seg_lo = dev ? dtab[segtab::kHeader + ei] : prm.tab.seg[ei];
+        seg_hi = dev ? dtab[segtab::kHeader + ei + 1] : prm.tab.seg[ei + 1];
     }
-    const int expert = prm.tab.first_expert + ei, seg_lo = prm.tab.seg[ei], seg_hi = prm.tab.seg[ei + 1];
+    const int expert = prm.tab.first_expert + ei;
     const int n0 = nt * BN, p_valid = min(BN, prm.n_cols - n0);
     int K, q_valid, m0 = 0;
     const T *P, *Q;
     int64_t c_off;
     if (RAGGED == kRaggedRows) {
-        const int row0 = seg_lo + (mt - prm.tab.tile[ei]) * BM;
         q_valid = min(BM, seg_hi - row0);
         K = prm.k_extent;
         P = (const T *)prm.P + (int64_t)expert * prm.p_expert_stride + (PSHAPE == kKC ? (int64_t)n0 * prm.ldp : (int64_t)n0);
@@ -302,7 +324,14 @@ int launch_unaligned_tiles(GemmParams &prm, int epilogue, hipStream_t stream) {
     prm.epilogue = epilogue;
     prm.tiles_n = (int)ceil_div(prm.n_cols, kUaBN);
     prm.tiles_m = RG == kRaggedRows ? 0 : (int)ceil_div(prm.n_rows, BM);
-    const int64_t total = (RG == kRaggedRows ? (int64_t)prm.tab.tile[prm.tab.n] : (int64_t)prm.tab.n * prm.tiles_m) * prm.tiles_n;
+    int64_t row_tiles = (int64_t)prm.tab.n * prm.tiles_m;
+    if (RG == kRaggedRows && prm.dev_tab != nullptr) {
+        row_tiles = segtab::cap_tiles(prm.dev_rows_cap, prm.tab.n, 128) * (128 / BM);
+        prm.dev_map_off = (int32_t)segtab::map128_off(prm.dev_rows_cap, prm.tab.n);
+    } else if (RG == kRaggedRows) {
+        row_tiles = prm.tab.tile[prm.tab.n];
+    }
+    const int64_t total = row_tiles * prm.tiles_n;
     if (total > (int64_t)INT32_MAX - 8) return fail(FMOE_ELIMIT, "grouped GEMM: %lld tiles exceed the grid limit", (long long)total);
     if (total == 0) return FMOE_OK;
     prm.total_tiles = (int)total;
@@ -328,7 +357,7 @@ template <typename T> int launch_unaligned_typed(GemmParams &prm, int product, i
 }  // namespace
 
 // product: 0 forward, 1 data gradient, 2 weight gradient (with the bias gradient).  Ragged rows: prm.block_m (64 or 128)
-// is the tile height that prm.tab was filled in for.
+// is the tile height, for which prm.tab was filled in (a device table serves both).
 int launch_mfma_unaligned(gemm::GemmParams &prm, int dtype, int product, int epilogue, hipStream_t stream) {
     if (dtype == FMOE_BF16) return launch_unaligned_typed<__bf16>(prm, product, epilogue, stream);
     if (dtype == FMOE_F16) return launch_unaligned_typed<_Float16>(prm, product, epilogue, stream);

@@ -249,6 +249,10 @@ TileShape pick_unaligned_tile(const int64_t *counts, int64_t n_expert, int64_t r
     }
     return row_tiles * ceil_div(n_cols, 128) >= 512 ? TileShape{128, 128} : TileShape{64, 128};
 }
+TileShape unaligned_tile_estimate(int64_t rows_cap, int64_t n_expert, int64_t n_cols) {
+    const int64_t row_tiles = rows_cap / 128 + std::min(n_expert, rows_cap) / 2;
+    return row_tiles * ceil_div(n_cols, 128) >= 512 ? TileShape{128, 128} : TileShape{64, 128};
+}
 
 // weight gradient: C is [out, in] per expert
 TileShape pick_wgrad_tile(int64_t n_experts_written, int64_t out_feat, int64_t in_feat, int64_t rows, int dtype) {
@@ -506,8 +510,8 @@ bool linear_forward_can_gather(const LinearForwardArgs &a) {
 
 // checks shared by the launches over a device table; fills the parts of prm that say so
 int device_table_launch(const char *who, GemmParams &prm, const int32_t *dev_tab, int64_t rows_cap, int64_t n_expert,
-                        bool fast) {
-    FMOE_REQUIRE(fast, "%s: a launch over a device segment table needs 16-byte aligned tensors, feature sizes that are "
+                        bool taken) {
+    FMOE_REQUIRE(taken, "%s: a launch over a device segment table needs 16-byte aligned tensors, feature sizes that are "
                        "multiples of 16 bytes and a 16- or 32-bit float type", who);
     FMOE_REQUIRE(n_expert >= 1 && n_expert <= (int64_t)(1 << 24) && rows_cap >= 0 && rows_cap <= (int64_t)INT32_MAX - 65536,
                  "%s: n_expert=%lld rows_cap=%lld", who, (long long)n_expert, (long long)rows_cap);
@@ -538,10 +542,12 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
         FMOE_REQUIRE(a.x_row_index == nullptr || linear_forward_can_gather(a),
                      "linear_forward: rows cannot be gathered in the loader for this shape");
         GemmParams prm{};
-        if (int rc = device_table_launch("linear_forward", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast)) return rc;
+        const bool any_grid = !fast && a.dev_any_grid && is_16bit(a.dtype) && a.x_row_index == nullptr;
+        if (int rc = device_table_launch("linear_forward", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast || any_grid)) return rc;
         prm.activation = kernel_activation(a.activation);
-        const DevRoute route = forward_route(a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype, a.epilogue, prm.activation,
-                                             a.aux != nullptr, a.x_row_index != nullptr);
+        const DevRoute route = any_grid ? DevRoute{DevKernel::kTiles, unaligned_tile_estimate(a.dev_rows_cap, n_expert, a.out_feat)}
+                                        : forward_route(a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype, a.epilogue, prm.activation,
+                                                        a.aux != nullptr, a.x_row_index != nullptr);
         prm.block_m = route.tile.bm; prm.block_n = route.tile.bn; prm.loaders = route.tile.loaders;
         prm.profile_class = kProfGemmFwd; prm.profile_work = 2.0 * (double)a.dev_rows_cap * (double)a.in_feat * (double)a.out_feat;
         prm.P = a.w; prm.Q = a.x; prm.C = a.y; prm.bias = a.bias; prm.aux = a.aux;
@@ -550,6 +556,7 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
         prm.p_expert_stride = a.in_feat * a.out_feat;
         prm.bias_expert_stride = a.out_feat;
         prm.n_cols = (int)a.out_feat; prm.k_extent = (int)a.in_feat;
+        if (any_grid) return dispatch<kFwd>(prm, a.dtype, a.epilogue, false, stream);
         prm.dev_split_ws = route_workspace(route, a.in_feat, a.dtype, a.dev_workspace, a.dev_workspace_bytes);
         if (route.kernel == DevKernel::kSkinny) {
             SkinnyParams sk{};
@@ -605,15 +612,18 @@ int grouped_linear_dgrad(const LinearDgradArgs &a, const int64_t *counts, int64_
         FMOE_REQUIRE(a.gy && a.w && a.gx, "linear_dgrad: NULL tensor");
         const bool fast = is_fast(a.dtype, {a.gy, a.w, a.gx, a.aux}, {a.in_feat, a.out_feat});
         GemmParams prm{};
-        if (int rc = device_table_launch("linear_dgrad", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast)) return rc;
+        const bool any_grid = !fast && a.dev_any_grid && is_16bit(a.dtype);
+        if (int rc = device_table_launch("linear_dgrad", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast || any_grid)) return rc;
         prm.activation = kernel_activation(a.activation);
-        const DevRoute route = dgrad_route(a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype, a.epilogue, prm.activation);
+        const DevRoute route = any_grid ? DevRoute{DevKernel::kTiles, unaligned_tile_estimate(a.dev_rows_cap, n_expert, a.in_feat)}
+                                        : dgrad_route(a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype, a.epilogue, prm.activation);
         prm.block_m = route.tile.bm; prm.block_n = route.tile.bn; prm.loaders = route.tile.loaders;
         prm.profile_class = kProfGemmDgrad; prm.profile_work = 2.0 * (double)a.dev_rows_cap * (double)a.in_feat * (double)a.out_feat;
         prm.P = a.w; prm.Q = a.gy; prm.C = a.gx; prm.aux = const_cast<void *>(a.aux);
         prm.ldp = a.in_feat; prm.ldq = a.out_feat; prm.ldc = a.in_feat;
         prm.p_expert_stride = a.in_feat * a.out_feat;
         prm.n_cols = (int)a.in_feat; prm.k_extent = (int)a.out_feat;
+        if (any_grid) return dispatch<kDgrad>(prm, a.dtype, a.epilogue, false, stream);
         prm.dev_split_ws = route_workspace(route, a.out_feat, a.dtype, a.dev_workspace, a.dev_workspace_bytes);
         if (route.kernel == DevKernel::kRing) return dispatch_ring<kDgrad>(prm, a.dtype, a.epilogue, stream);
         return dispatch<kDgrad>(prm, a.dtype, a.epilogue, fast, stream);
@@ -654,7 +664,8 @@ int grouped_linear_wgrad(const LinearWgradArgs &a, const int64_t *counts, int64_
         const bool fast = is_fast(a.dtype, {a.gy, a.x, a.gw}, {a.in_feat, a.out_feat});
         const TileShape tile = pick_wgrad_tile(n_expert, a.out_feat, a.in_feat, a.dev_rows_cap, a.dtype);
         GemmParams prm{};
-        if (int rc = device_table_launch("linear_wgrad", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast)) return rc;
+        const bool any_grid = !fast && a.dev_any_grid && is_16bit(a.dtype);
+        if (int rc = device_table_launch("linear_wgrad", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast || any_grid)) return rc;
         prm.block_m = tile.bm; prm.block_n = tile.bn; prm.loaders = tile.loaders;
         prm.profile_class = kProfGemmWgrad; prm.profile_work = 2.0 * (double)a.dev_rows_cap * (double)a.in_feat * (double)a.out_feat;
         prm.P = a.x; prm.Q = a.gy; prm.C = a.gw; prm.bias_grad = a.gb;
@@ -662,7 +673,7 @@ int grouped_linear_wgrad(const LinearWgradArgs &a, const int64_t *counts, int64_
         prm.c_expert_stride = a.in_feat * a.out_feat;
         prm.n_cols = (int)a.in_feat; prm.n_rows = (int)a.out_feat;
         prm.accumulate_first = 0;
-        if (use_ring(tile, a.dtype)) return dispatch_ring<kWgrad>(prm, a.dtype, kEpiStore, stream);
+        if (!any_grid && use_ring(tile, a.dtype)) return dispatch_ring<kWgrad>(prm, a.dtype, kEpiStore, stream);
         return dispatch<kWgrad>(prm, a.dtype, kEpiStore, fast, stream);
     }
     int64_t total;

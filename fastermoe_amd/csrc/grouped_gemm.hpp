@@ -79,6 +79,8 @@ struct LinearForwardArgs {
     // round of tiles (without it such a round is not split)
     void *dev_workspace = nullptr;
     int64_t dev_workspace_bytes = 0;
+    // with dev_tab: 16-bit tensors and feature sizes off the 16-byte grid are taken too (gemm_unaligned.hip)
+    bool dev_any_grid = false;
 };
 
 // Bytes of workspace with which a launch over a device table can split its last round of tiles along a
@@ -100,6 +102,7 @@ struct LinearDgradArgs {
     int64_t dev_rows_cap = 0;
     void *dev_workspace = nullptr;
     int64_t dev_workspace_bytes = 0;
+    bool dev_any_grid = false;
 };
 
 struct LinearWgradArgs {
@@ -111,6 +114,7 @@ struct LinearWgradArgs {
     int dtype;
     const int32_t *dev_tab = nullptr;  // as in LinearForwardArgs
     int64_t dev_rows_cap = 0;
+    bool dev_any_grid = false;
 };
 
 // counts[e] rows for experts [0, n_expert), restricted to rows [row_lo, row_hi)

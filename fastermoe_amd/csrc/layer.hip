@@ -8,7 +8,7 @@
 // tensors that it hands in.  Blocks whose lives do not overlap share memory: the sorted input is the output rows' place before the
 // second linear writes them, and in the backward one block of rows is in turn the gradient of the experts' output, the
 // experts' input gradient and the sorted input.
-#include "common.hpp"
+#include "grouped_gemm.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -38,8 +38,11 @@ struct Carver {
     }
 };
 
+// whether rows are whole 16-byte chunks; where they are not, 16-bit types go through gemm_unaligned.hip, over sorted rows
+bool on_grid(const Sizes &s) { return fmoe_linear_dev_supported(s.d_model, s.d_hidden, s.dtype) == 1; }
+
 bool reads_token_rows(const Sizes &s, bool keep_pre) {
-    return s.n_tokens * s.d_model * s.eb < ((int64_t)1 << 31) &&
+    return on_grid(s) && s.n_tokens * s.d_model * s.eb < ((int64_t)1 << 31) &&
            !fmoe_linear_act_dev_reads_rows(s.n_slots, s.n_expert, s.d_model, s.d_hidden, s.dtype, s.activation, keep_pre);
 }
 
@@ -106,9 +109,9 @@ bool taken(const Sizes &s, int gate) {
     if (s.n_tokens < 1 || s.d_model < 1 || s.d_hidden < 1 || s.n_expert < 1 || s.top_k < 1 || s.eb == 0 || s.dtype == FMOE_F64) return false;
     if (s.n_tokens > (int64_t)INT32_MAX / s.top_k - 65536 || s.n_expert > (1 << 24)) return false;
     if (s.activation < FMOE_ACT_NONE || s.activation > FMOE_ACT_GELU) return false;
-    if (!fmoe_linear_dev_supported(s.d_model, s.d_hidden, s.dtype)) return false;
+    if (!on_grid(s) && (s.dtype == FMOE_F32 || s.d_model * s.eb > (1 << 22) || s.d_hidden * s.eb > (1 << 22))) return false;
     if (gate == FMOE_GATE_ROUTED) return true;
-    if (!fmoe_gate_grad_supported(s.d_model, s.n_expert, s.top_k, s.dtype)) return false;
+    if (gate == FMOE_GATE_LINEAR && !fmoe_gate_grad_supported(s.d_model, s.n_expert, s.top_k, s.dtype)) return false;
     if (gate == FMOE_GATE_LINEAR) return fmoe_gate_linear_supported(s.d_model, s.n_expert, s.top_k, s.dtype) == 1;
     return gate == FMOE_GATE_LOGITS && (s.top_k == 1 || s.top_k == 2 || s.top_k == 4 || s.top_k == 8) && s.top_k <= s.n_expert && s.n_expert <= 8192;
 }
@@ -117,6 +120,41 @@ bool taken(const Sizes &s, int gate) {
 bool apart(int gate) {
     return switched_off("FMOE_FOLD_COMBINE") || switched_off("FMOE_EXPERT_EPILOGUE") || switched_off("FMOE_DEVICE_TABLES") ||
            (gate != FMOE_GATE_ROUTED && switched_off("FMOE_GATE_LINEAR_FUSED"));
+}
+
+// one expert linear over the sorted rows of a segment table
+int linear_forward(const Sizes &s, const void *x, const int64_t *row_index, const void *w, const void *b, void *pre, void *y,
+                   const void *table, int64_t in_feat, int64_t out_feat, int activation, void *ws, int64_t ws_bytes, hipStream_t st) {
+    const bool plain = activation == FMOE_ACT_NONE && pre == nullptr;
+    LinearForwardArgs a{x, w, b, y, pre, in_feat, out_feat, s.dtype, plain ? kEpiStore : kEpiBiasAct, activation};
+    a.x_row_index = row_index;
+    a.x_index_div = row_index ? s.top_k : 1;
+    a.x_total_rows = row_index ? s.n_tokens : 0;
+    a.dev_tab = (const int32_t *)table;
+    a.dev_rows_cap = s.n_slots;
+    a.dev_workspace = ws_bytes ? ws : nullptr;
+    a.dev_workspace_bytes = ws_bytes;
+    a.dev_any_grid = true;
+    return grouped_linear_forward(a, nullptr, s.n_expert, 0, s.n_slots, st);
+}
+int linear_dgrad(const Sizes &s, const void *gy, const void *w, const void *pre, void *gx, const void *table, int64_t in_feat,
+                 int64_t out_feat, int activation, void *ws, int64_t ws_bytes, hipStream_t st) {
+    const bool act = activation != FMOE_ACT_NONE;
+    LinearDgradArgs d{gy, w, gx, act ? pre : nullptr, in_feat, out_feat, s.dtype, act ? kEpiDAct : kEpiStore, activation};
+    d.dev_tab = (const int32_t *)table;
+    d.dev_rows_cap = s.n_slots;
+    d.dev_workspace = ws_bytes ? ws : nullptr;
+    d.dev_workspace_bytes = ws_bytes;
+    d.dev_any_grid = true;
+    return grouped_linear_dgrad(d, nullptr, s.n_expert, 0, s.n_slots, st);
+}
+int linear_wgrad(const Sizes &s, const void *gy, const void *x, void *gw, void *gb, const void *table, int64_t in_feat, int64_t out_feat,
+                 hipStream_t st) {
+    LinearWgradArgs g{gy, x, gw, gb, in_feat, out_feat, s.dtype};
+    g.dev_tab = (const int32_t *)table;
+    g.dev_rows_cap = s.n_slots;
+    g.dev_any_grid = true;
+    return grouped_linear_wgrad(g, nullptr, s.n_expert, 0, s.n_slots, true, st);
 }
 
 Sizes sizes_of(int64_t n_tokens, int64_t d_model, int64_t d_hidden, int64_t n_expert, int64_t top_k, int dtype, int activation) {
@@ -179,12 +217,11 @@ extern "C" int fmoe_layer_forward(const void *x, const void *gate_w, const void 
         rc = fmoe_gather_rows_div(x, pos, top_k, rows, s.n_slots, n_tokens, d_model, dtype, stream);
         if (rc != FMOE_OK) return rc;
     }
-    rc = fmoe_linear_forward_dev(token_rows ? x : rows, token_rows ? pos : nullptr, top_k, token_rows ? n_tokens : s.n_slots, w1, b1,
-                                 keep_pre ? pre : nullptr, mid, segment_table, n_expert, s.n_slots, d_model, d_hidden, dtype, activation,
-                                 f.split1 ? f.split_ws : nullptr, f.split1, stream);
+    hipStream_t st = (hipStream_t)stream;
+    rc = linear_forward(s, token_rows ? x : rows, token_rows ? pos : nullptr, w1, b1, keep_pre ? pre : nullptr, mid, segment_table, d_model,
+                        d_hidden, activation, f.split_ws, f.split1, st);
     if (rc != FMOE_OK) return rc;
-    rc = fmoe_linear_forward_dev(mid, nullptr, 1, s.n_slots, w2, b2, nullptr, rows, segment_table, n_expert, s.n_slots, d_hidden, d_model,
-                                 dtype, FMOE_ACT_NONE, f.split2 ? f.split_ws : nullptr, f.split2, stream);
+    rc = linear_forward(s, mid, nullptr, w2, b2, nullptr, rows, segment_table, d_hidden, d_model, FMOE_ACT_NONE, f.split_ws, f.split2, st);
     if (rc != FMOE_OK) return rc;
     return fmoe_gather_combine_forward(rows, slot_to_row, topk_score, out, n_tokens, top_k, s.n_slots, d_model, dtype, stream);
 }
@@ -208,22 +245,21 @@ extern "C" int fmoe_layer_backward(const void *grad_out, const void *x, const vo
     const void *saved_pre = activation == FMOE_ACT_GELU ? pre : mid;   // (ReLU's derivative can be read off its output)
     FMOE_REQUIRE(grad_out && x && w1 && w2 && topk_score && pos && slot_to_row && segment_table && saved_pre && mid && rows && grad_score &&
                      (!gated || (topk_idx && gate_w)), "fmoe_layer_backward: NULL pointer");
+    hipStream_t st = (hipStream_t)stream;
     int rc = fmoe_gather_combine_backward(grad_out, rows, slot_to_row, topk_score, b.rows, grad_score, n_tokens, top_k, s.n_slots, d_model,
                                           dtype, stream);
     if (rc != FMOE_OK) return rc;
     const bool first = grad_x != nullptr || grad_w1 != nullptr;   // whether the first linear's output gradient is wanted
     if (first) {
-        rc = fmoe_linear_dgrad_dev(b.rows, w2, saved_pre, b.grad_pre, segment_table, n_expert, s.n_slots, d_hidden, d_model, dtype, activation,
-                                   b.split2 ? b.ws : nullptr, b.split2, stream);
+        rc = linear_dgrad(s, b.rows, w2, saved_pre, b.grad_pre, segment_table, d_hidden, d_model, activation, b.ws, b.split2, st);
         if (rc != FMOE_OK) return rc;
     }
     if (grad_w2 != nullptr) {
-        rc = fmoe_linear_wgrad_dev(b.rows, mid, grad_w2, grad_b2, segment_table, n_expert, s.n_slots, d_hidden, d_model, dtype, stream);
+        rc = linear_wgrad(s, b.rows, mid, grad_w2, grad_b2, segment_table, d_hidden, d_model, st);
         if (rc != FMOE_OK) return rc;
     }
     if (grad_x != nullptr) {
-        rc = fmoe_linear_dgrad_dev(b.grad_pre, w1, nullptr, b.rows, segment_table, n_expert, s.n_slots, d_model, d_hidden, dtype, FMOE_ACT_NONE,
-                                   b.split1 ? b.ws : nullptr, b.split1, stream);
+        rc = linear_dgrad(s, b.grad_pre, w1, nullptr, b.rows, segment_table, d_model, d_hidden, FMOE_ACT_NONE, b.ws, b.split1, st);
         if (rc != FMOE_OK) return rc;
         // (the gate's part of the input gradient is added in the same pass, before the one rounding)
         rc = gated ? fmoe_reduce_slots_gate(b.rows, slot_to_row, grad_score, topk_idx, gate_w, grad_x, n_tokens, top_k, s.n_slots, n_expert,
@@ -234,7 +270,7 @@ extern "C" int fmoe_layer_backward(const void *grad_out, const void *x, const vo
     if (grad_w1 != nullptr) {
         rc = fmoe_gather_rows_div(x, pos, top_k, b.rows, s.n_slots, n_tokens, d_model, dtype, stream);
         if (rc != FMOE_OK) return rc;
-        rc = fmoe_linear_wgrad_dev(b.grad_pre, b.rows, grad_w1, grad_b1, segment_table, n_expert, s.n_slots, d_model, d_hidden, dtype, stream);
+        rc = linear_wgrad(s, b.grad_pre, b.rows, grad_w1, grad_b1, segment_table, d_model, d_hidden, st);
         if (rc != FMOE_OK) return rc;
     }
     if (gated && grad_gate_w != nullptr)

@@ -474,8 +474,10 @@ class MOELayer(Function):
         top_k, activation, gate, sizes, (gate_bias, bias1, bias2) = ctx.moe_args
         need = ctx.needs_input_grad
         place = fmoe_native.LayerRouting(*tensors, kept=kept)
-        # (a backward that is to be differentiated again needs the gate's products as torch operators)
-        apart = kept is not None and torch.is_grad_enabled()
+        # (a backward that is to be differentiated again needs the gate's products as torch operators, and so do gates that the
+        # kernels do not take)
+        apart = kept is not None and (torch.is_grad_enabled() or not fmoe_native.gate_grad_supported(
+            inp.shape[1], gate_w.shape[0], top_k, inp.dtype))
         new = lambda wanted, *shape: torch.empty(shape, dtype=inp.dtype, device=inp.device) if wanted else None
         (n, d), (e, h) = inp.shape, w1.shape[:2]
         grad_x = new(need[0], n, d)

@@ -633,9 +633,9 @@ int fmoe_fused_mlp_backward(const fmoe_mlp_params *p, const void *grad_out,
 #define FMOE_GATE_LOGITS 1
 #define FMOE_GATE_ROUTED 2
 
-/* 1 when the two calls below take these sizes (those of fmoe_linear_*_dev and,
- * with the gate inside, of fmoe_gate_linear_topk_route / fmoe_gate_topk_route
- * and fmoe_gate_weight_grad), else 0; also 0, with the sizes filled in, where the
+/* 1 when the two calls below take these sizes (those of fmoe_linear_*_dev, any
+ * feature sizes for 16-bit types, and, with the gate inside, those of
+ * fmoe_gate_linear_topk_route / fmoe_gate_topk_route), else 0; also 0, with the sizes filled in, where the
  * environment asks for the steps of a layer one by one (FMOE_FOLD_COMBINE=0,
  * FMOE_EXPERT_EPILOGUE=0, FMOE_DEVICE_TABLES=0, FMOE_GATE_LINEAR_FUSED=0).
  * sizes_host[0], [1]: bytes of scratch of a forward and, with keep, of a
@@ -669,7 +669,9 @@ int fmoe_layer_forward(const void *x, const void *gate_w, const void *gate_b,
  * gate inside: its part included, one rounding), grad_w1 (and grad_b1), grad_w2
  * (and grad_b2); with the gate inside grad_gate_w (and grad_gate_b), else
  * grad_score [n_tokens*top_k], which is always written.  Nothing of the forward
- * is overwritten. */
+ * is overwritten.  A gate that fmoe_gate_grad_supported does not take is
+ * differentiated outside: FMOE_GATE_ROUTED then serves here whatever the forward
+ * ran with. */
 int fmoe_layer_backward(const void *grad_out, const void *x, const void *gate_w,
                         const void *w1, const void *w2, const int64_t *topk_idx,
                         const void *topk_score, const int64_t *pos,
