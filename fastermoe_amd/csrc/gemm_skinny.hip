@@ -1,8 +1,8 @@
-// Grouped forward product Y[seg_e] = act(X[seg_e] . W_e^T + b_e) for few rows per expert, 16-bit types over a device
+// Grouped forward product Y[seg_e] = act(X[seg_e] . W_e^T + b_e) for few rows per expert, 16- and 32-bit types over a device
 // segment table (gfx950): decoding steps, where every weight is read once and meets a handful of rows.
 //
-// Bound by the weights' way from memory, so nothing is staged: a wave loads a 16 x 32 block of weights with one 16-byte
-// load per lane straight into the registers of a 16 x 16 x 32 MFMA, and the rows the same way (from L2, where they stay).
+// Bound by the weights' way from memory, so nothing is staged: a wave loads a block of 16 rows of 64 bytes of weights with one 16-byte
+// load per lane straight into the registers of a 16 x 16 x 32 MFMA (float32: of four 16 x 16 x 4), and the rows the same way (from L2, where they stay).
 // A workgroup of four waves has 16 columns of one row tile; the waves take the contraction in turns of one unit,
 // so that together they read whole lines of each weight row, with the next unit's loads under way before the products of
 // the current one, and add up their accumulators through LDS in a fixed order.  With 16 waves per compute unit
@@ -17,9 +17,20 @@ namespace {
 
 constexpr int kSkThreads = 256, kSkWaves = 4, kSkMaxBlocks = 4;   // most blocks of 16 rows of a wave
 
+// one 16 x 16 block over 64 bytes of contraction; acc as for the 16 x 16 x 32 form
+template <typename T> __device__ __forceinline__ void mma_step(f32x4 &acc, const u32x4 &w, const u32x4 &x) { Elem<T>::mma(acc, w, x); }
+template <> __device__ __forceinline__ void mma_step<float>(f32x4 &acc, const u32x4 &w, const u32x4 &x) {
+    // product j takes element j of every lane's four: contraction elements j, 4 + j, 8 + j and 12 + j of the step
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w[j]), __uint_as_float(x[j]), acc, 0, 0, 0);
+}
+
 template <typename T>
 __global__ __launch_bounds__(kSkThreads, 4) void grouped_gemm_skinny_kernel(const SkinnyParams prm) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
+    constexpr int EB = (int)sizeof(T), CE = 16 / EB, kStep = 64 / EB;   // elements per lane's load and per step
+    typedef std::conditional_t<sizeof(T) == 2, u32x2, u32x4> Vec4;        // four elements
     constexpr uint32_t kOutOfRange = 0x80000000u;
     constexpr int kRsrcFlags = 0x00020000;   // raw buffer, 32-bit data format
     typedef const int32_t __attribute__((address_space(4))) *DevTab;    // read-only, uniform: scalar loads
@@ -38,15 +49,15 @@ __global__ __launch_bounds__(kSkThreads, 4) void grouped_gemm_skinny_kernel(cons
 
     // weights: rows past the last column lie past the end of the resource and read as zero
     const T *W = (const T *)prm.w + ((int64_t)expert * prm.n_cols + n0) * K;
-    const int w_bytes = min(kSkinnyCols, prm.n_cols - n0) * K * 2;
+    const int w_bytes = min(kSkinnyCols, prm.n_cols - n0) * K * EB;
     const __amdgpu_buffer_rsrc_t w_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(W), 0, w_bytes, kRsrcFlags);
-    const uint32_t w_off = (uint32_t)(lb * K * 2 + hq * 16);
+    const uint32_t w_off = (uint32_t)(lb * K * EB + hq * 16);
     const bool gather = prm.row_index != nullptr;
     const T *X = (const T *)prm.x + (gather ? (int64_t)0 : (int64_t)first * K);
-    const int x_bytes = gather ? (int)(prm.x_total_rows * K * 2) : rows * K * 2;
+    const int x_bytes = gather ? (int)(prm.x_total_rows * K * EB) : rows * K * EB;
     const __amdgpu_buffer_rsrc_t x_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(X), 0, x_bytes, kRsrcFlags);
 
-    // RB blocks of 16 rows from row r0 of the tile on; STEPS contraction steps of 32 elements to a unit
+    // RB blocks of 16 rows from row r0 of the tile on; STEPS contraction steps of 64 bytes to a unit
     auto pass = [&](auto rb_tag, auto steps_tag, int r0) {
         constexpr int RB = decltype(rb_tag)::value, STEPS = decltype(steps_tag)::value;
         uint32_t x_off[RB];
@@ -61,7 +72,7 @@ __global__ __launch_bounds__(kSkThreads, 4) void grouped_gemm_skinny_kernel(cons
                     src = prm.div_shift < 0 ? idx : (int64_t)(__umulhi((uint32_t)idx, prm.div_mul) >> prm.div_shift);
                 if (src >= prm.x_total_rows) src = -1;
             }
-            x_off[y] = src >= 0 ? (uint32_t)(src * K * 2 + hq * 16) : kOutOfRange;
+            x_off[y] = src >= 0 ? (uint32_t)(src * K * EB + hq * 16) : kOutOfRange;
         }
         f32x4 acc[RB];
 #pragma unroll
@@ -70,22 +81,22 @@ __global__ __launch_bounds__(kSkThreads, 4) void grouped_gemm_skinny_kernel(cons
         auto load = [&](Unit &u, int unit) {
 #pragma unroll
             for (int s = 0; s < STEPS; ++s) {
-                const int k = (unit * STEPS + s) * 32;
-                // sign bit set where this lane's eight elements lie past the contraction (and for every unit past it)
-                const uint32_t past = (uint32_t)(K - 1 - k - hq * 8) & kOutOfRange;
-                u.w[s] = __builtin_amdgcn_raw_buffer_load_b128(w_rs, (int)((w_off + k * 2) | past), 0, 0);
+                const int k = (unit * STEPS + s) * kStep;
+                // sign bit set where this lane's elements lie past the contraction (and for every unit past it)
+                const uint32_t past = (uint32_t)(K - 1 - k - hq * CE) & kOutOfRange;
+                u.w[s] = __builtin_amdgcn_raw_buffer_load_b128(w_rs, (int)((w_off + k * EB) | past), 0, 0);
 #pragma unroll
                 for (int y = 0; y < RB; ++y)
-                    u.x[s][y] = __builtin_amdgcn_raw_buffer_load_b128(x_rs, (int)((x_off[y] + k * 2) | past), 0, 0);
+                    u.x[s][y] = __builtin_amdgcn_raw_buffer_load_b128(x_rs, (int)((x_off[y] + k * EB) | past), 0, 0);
             }
         };
         auto multiply = [&](const Unit &u) {
 #pragma unroll
             for (int s = 0; s < STEPS; ++s)
 #pragma unroll
-                for (int y = 0; y < RB; ++y) Elem<T>::mma(acc[y], u.w[s], u.x[s][y]);
+                for (int y = 0; y < RB; ++y) mma_step<T>(acc[y], u.w[s], u.x[s][y]);
         };
-        const int n_units = (K + 32 * STEPS - 1) / (32 * STEPS);
+        const int n_units = (K + kStep * STEPS - 1) / (kStep * STEPS);
         Unit a, b;
         int unit = wave;
         load(a, unit);
@@ -108,9 +119,9 @@ __global__ __launch_bounds__(kSkThreads, 4) void grouped_gemm_skinny_kernel(cons
         if (wave > 0) return;   // (from this pass)
         // acc[y][i] is C(row 16 y + lb, column 4 hq + i)
         const int col = n0 + 4 * hq;
-        alignas(8) T b4[4] = {};
+        alignas(16) T b4[4] = {};
         if (prm.bias != nullptr && col < prm.n_cols)
-            *(u32x2 *)b4 = *(const u32x2 *)((const T *)prm.bias + (int64_t)expert * prm.n_cols + col);
+            *(Vec4 *)b4 = *(const Vec4 *)((const T *)prm.bias + (int64_t)expert * prm.n_cols + col);
 #pragma unroll
         for (int y = 0; y < RB; ++y) {
             f32x4 v = acc[y];
@@ -118,16 +129,16 @@ __global__ __launch_bounds__(kSkThreads, 4) void grouped_gemm_skinny_kernel(cons
             for (int w = 0; w < kSkWaves - 1; ++w) v += part[w][y][lane];
             const int row = r0 + 16 * y + lb;
             if (row >= rows || col >= prm.n_cols) continue;
-            alignas(8) T pre[4], res[4];
+            alignas(16) T pre[4], res[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float p = v[i] + (float)b4[i];
                 pre[i] = (T)p;
-                res[i] = (T)apply_act<true>(p, prm.activation);
+                res[i] = (T)apply_act<sizeof(T) == 2>(p, prm.activation);
             }
             const int64_t at = (int64_t)(first + row) * prm.n_cols + col;
-            if (prm.aux != nullptr) *(u32x2 *)((T *)prm.aux + at) = *(const u32x2 *)pre;
-            *(u32x2 *)((T *)prm.y + at) = *(const u32x2 *)res;
+            if (prm.aux != nullptr) *(Vec4 *)((T *)prm.aux + at) = *(const Vec4 *)pre;
+            *(Vec4 *)((T *)prm.y + at) = *(const Vec4 *)res;
         }
     };
     typedef std::integral_constant<int, 1> One;
@@ -149,8 +160,9 @@ __global__ __launch_bounds__(kSkThreads, 4) void grouped_gemm_skinny_kernel(cons
 int launch_skinny(const SkinnyParams &prm, int dtype, int64_t row_tiles, hipStream_t stream) {
     const int64_t grid = row_tiles * prm.tiles_n;
     if (grid > (int64_t)INT32_MAX) return fail(FMOE_ELIMIT, "grouped GEMM: grid of %lld workgroups", (long long)grid);
-    FMOE_REQUIRE(dtype == FMOE_BF16 || dtype == FMOE_F16, "grouped GEMM: dtype %d is not a 16-bit float type", dtype);
-    if (dtype == FMOE_BF16) grouped_gemm_skinny_kernel<__bf16><<<(unsigned)grid, kSkThreads, 0, stream>>>(prm);
+    FMOE_REQUIRE(dtype == FMOE_BF16 || dtype == FMOE_F16 || dtype == FMOE_F32, "grouped GEMM: dtype %d is not a 16- or 32-bit float type", dtype);
+    if (dtype == FMOE_F32) grouped_gemm_skinny_kernel<float><<<(unsigned)grid, kSkThreads, 0, stream>>>(prm);
+    else if (dtype == FMOE_BF16) grouped_gemm_skinny_kernel<__bf16><<<(unsigned)grid, kSkThreads, 0, stream>>>(prm);
     else grouped_gemm_skinny_kernel<_Float16><<<(unsigned)grid, kSkThreads, 0, stream>>>(prm);
     FMOE_LAUNCH_CHECK();
     return FMOE_OK;

@@ -373,15 +373,19 @@ bool use_ring(const TileShape &tile, int dtype) {
     return tile.many && is_16bit(dtype);
 }
 
-// Whether a forward launch over a device table goes to gemm_skinny.hip: 16-bit types (no tile shape forced) and at
+// Whether a forward launch over a device table goes to gemm_skinny.hip (no tile shape forced).  16-bit types: at
 // most two rows per expert on average, or eight where the weights make less than two rounds of 128 x 128 tiles (512 at
 // a time), whose last round is then badly filled.  Above that the rows' way from L2 into every 16 columns costs more than
 // the tiles' padding.  bf16, us on the tiles and here: 32 experts of 4096 x 1024, 2 / 32 / 256 rows: 26.7 / 57.4 / 69.9
 // and 13.8 / 36.3 / 55.5; 8 of 4096 x 14336, 8 / 32 / 64 / 128: 142 / 191 / 191 / 192 and 99 / 161 / 180 / 243; 256 of
 // 1024 x 2048, 256 / 512 / 1024: 134 / 179 / 205 and 124 / 170 / 210; 64 of 8192 x 2048, 64 / 128 / 256: 298 / 367 / 372
 // and 249 / 334 / 389.
+// float32, where a tile's padding costs products and not only places: at most 40 rows per expert on average.  us on the tiles and here:
+// 8 experts of 2048 x 8192, 2 / 16 / 32 / 48 rows each: 260 / 260 / 265 / 266 and 109 / 151 / 209 / 280; 32 of 1024 x 1024, 2 / 32 / 48:
+// 75 / 70 / 70 and 31 / 51 / 66; 4 of 768 x 3072, 2 / 32 / 64: 54 / 54 / 31 and 11 / 17 / 26.
 bool use_skinny(int64_t rows_cap, int64_t n_expert, int64_t out_feat, int dtype) {
-    if (!is_16bit(dtype) || getenv("FMOE_GEMM_TILE")) return false;
+    if ((!is_16bit(dtype) && dtype != FMOE_F32) || getenv("FMOE_GEMM_TILE")) return false;
+    if (dtype == FMOE_F32) return rows_cap <= 40 * n_expert;
     return rows_cap <= 2 * n_expert || (rows_cap <= 8 * n_expert && n_expert * ceil_div(out_feat, 128) < 1024);
 }
 

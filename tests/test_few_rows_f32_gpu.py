@@ -1,0 +1,53 @@
+"""The forward product for few rows per expert in float32 (weights straight from memory to the matrix pipe)."""
+import pytest
+import torch
+
+from fastermoe_amd import _lib, fmoe_native
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 0, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 130]   # blocks of 16 rows, passes of 64, a tile of 128 and the next
+
+
+@pytest.mark.parametrize("k,n", [(4, 4), (16, 16), (20, 36), (68, 20), (256, 64), (1028, 132)])
+@pytest.mark.parametrize("act", [_lib.ACT_NONE, _lib.ACT_RELU, _lib.ACT_GELU])
+def test_few_rows_in_float32(k, n, act, device):
+    """Against float64, element by element: 2 k + 8 roundings of float32 of the terms' absolute sum bound any order of the
+    products, the waves' sums and the bias; GELU's own formula is within 1.5e-7 of its argument's size."""
+    counts = torch.tensor(EDGES)
+    e, rows = len(EDGES), sum(EDGES)
+    slots = rows + 5
+    assert slots <= 40 * e   # (the rule's line)
+    g = torch.Generator().manual_seed(k + n)
+    x = torch.randn(slots, k, generator=g).to(device)
+    w = (torch.randn(e, n, k, generator=g) / k ** 0.5).to(device)
+    b = torch.randn(e, n, generator=g).to(device)
+    table = fmoe_native.segment_table(counts.to(device), slots)
+    index = torch.randint(0, 3 * slots, (slots,), generator=g)
+    index[torch.rand(slots, generator=g) < 0.1] = -1
+    index = index.to(device)
+    picked = torch.where(index[:, None] >= 0, x[(index // 3).clamp(min=0)], torch.zeros_like(x))
+    for src, kw in ((x, {}), (picked, dict(row_index=index, index_div=3))):
+        y, pre = fmoe_native.linear_forward_dev(x, w, b, table, slots, act, act != _lib.ACT_NONE, **kw)
+        lo = 0
+        for i, c in enumerate(EDGES):
+            a, we = src[lo:lo + c].double(), w[i].double()
+            ref = a @ we.t() + b[i].double()
+            bound = (2 * k + 8) * 2.0 ** -24 * (a.abs() @ we.abs().t() + b[i].double().abs())
+            got = (pre if pre is not None else y)[lo:lo + c].double()
+            assert ((got - ref).abs() <= bound).all()
+            if act == _lib.ACT_RELU:
+                assert torch.equal(y[lo:lo + c], pre[lo:lo + c].clamp(min=0))
+            if act == _lib.ACT_GELU:
+                want = torch.nn.functional.gelu(pre[lo:lo + c].double())
+                assert ((y[lo:lo + c].double() - want).abs() <= 4e-7 * (1 + pre[lo:lo + c].double().abs())).all()
+            lo += c
+
+
+def test_the_rows_past_the_counts_are_left_alone(device):
+    counts = torch.tensor([3, 0, 2], device=device)
+    table = fmoe_native.segment_table(counts, 64)
+    x, w = torch.randn(64, 32, device=device), torch.randn(3, 48, 32, device=device)
+    full, _ = fmoe_native.linear_forward_dev(x, w, None, table, 64)
+    ref = torch.cat([x[:3].double() @ w[0].double().t(), x[3:5].double() @ w[2].double().t()])
+    assert (full[:5].double() - ref).abs().max() <= 1e-5 * ref.abs().max()
