@@ -9,6 +9,7 @@
 #include <atomic>
 #include <mutex>
 #include <type_traits>
+#include <utility>
 
 namespace fmoe {
 namespace gemm {
@@ -25,9 +26,8 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // wave of a SIMD sits at the barrier or waits for LDS; the workgroup takes the whole LDS of a
 // compute unit.  Tiles of 128 x 128: 2 x 2 (256 threads, 64 x 64 per wave) and half the LDS, so two
 // workgroups share a compute unit and one's first loads and epilogue run under the other's main
-// loop -- for launches whose tiles are short (few slabs) or few.  fp32 also comes in 64 x 64 (2 x 2 waves of one
-// 32 x 32 block, four workgroups per compute unit): its MFMA takes 256 cycles for what two 16-byte LDS reads
-// bring, so that the lower tile costs nothing and a launch of a few hundred tiles spreads evenly.
+// loop -- for launches whose tiles are short (few slabs) or few.  fp32 comes in 128 x 128 and in 64 x 64 (2 x 2 waves of one
+// 32 x 32 block, four workgroups per compute unit), over which a launch of a few tiles spreads more evenly.
 constexpr int kWavesN = 2;
 constexpr int waves_m_of(int bn) { return bn <= 128 ? 2 : 4; }
 constexpr int threads_of(int bn) { return 64 * waves_m_of(bn) * kWavesN; }
@@ -54,7 +54,7 @@ template <typename T> struct Elem;
 
 // The 16-bit types use the 16 x 16 x 32 MFMA (4 accumulator registers per block): for the same
 // flops it moves half as many accumulator registers as 32 x 32 x 16, and under the chip's
-// power limit that buys clock.  fp32 uses 32 x 32 x 2.
+// power limit that buys clock.  fp32 uses 32 x 32 x 2 where its bf16 parts do not do (Split8).
 template <> struct Elem<__bf16> {
     static constexpr int kPerChunk = 8;
     static constexpr int kBlk = 16;  // rows and columns of one MFMA block
@@ -86,6 +86,53 @@ template <> struct Elem<float> {
             acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(p[j]), __uint_as_float(q[j]), acc, 0, 0, 0);
     }
 };
+
+// fp32 products on the bf16 matrix pipe.  A float is the exact sum of three bf16 numbers, each the rounding of what the ones before
+// it left (8 significant bits each, down to 2^-110; below that what is left out is at most 2^-134).  Of the nine products of two such
+// sums the three smallest, at most 2^-25 of the whole, are left out; the other six go into the fp32 accumulator, small ones first:
+// 6 x 32 cycles for 16 contraction elements of a 32 x 32 block, where the fp32 MFMA takes 8 x 64, and six roundings of the accumulator
+// instead of eight.  Distance from float64 beside the fp32 MFMA's (relative 2-norms, 15 sizes from 512 to 40000 rows): 0.83 to 0.87 of it for every
+// forward, data gradient and weight gradient, e.g. 2.4 / 2.9e-7 at K = 512, 3.5 / 4.1e-7 at 1024, 4.9 / 5.7e-7 at 2048.
+// What bounds it: the power limit for large launches (six bf16 products to one: 190 TFLOP/s are 1140 of bf16 ones), else loads into LDS
+// and tiles that do not fill the chip.  Forward / data gradient / weight gradient in us, before and now: 8192 rows, 8 experts of 2048 x 4096: 1095 / 1094 /
+// 1051 and 787 / 765 / 729; of 512 x 1024: 96 / 105 / 83 and 77 / 74 / 58; 1024 rows, 16 of 768 x 3072: 85 / 107 / 75 and 67 / 74 / 52.
+// An infinity, a NaN or a number that rounds to a bf16 infinity makes the accumulator a NaN or an infinity: such tiles are computed again on the fp32 MFMA
+// (grouped_gemm_kernel).
+struct Raw8 {      // 8 contraction elements of one row: two 16-byte chunks
+    u32x4 c[2];
+};
+struct Split8 {    // the same as three bf16 numbers each
+    u32x4 hi, mid, lo;
+};
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+// The arithmetic of one fragment in five stages of 4 to 8 instructions, which the main loop places between MFMAs.  `left` holds the
+// floats, then what the parts so far leave of them: v - 1 x own half + 0 x the other, one v_dot2_f32_bf16 each.  (The pair
+// -1, 0 comes from a register: as an operand it turns into the inline constant -1.0, which is the pair 0, -1.)
+constexpr int kSplitStages = 5;
+__device__ __forceinline__ void split_stage(int stage, Raw8 &left, Split8 &s) {
+    uint32_t low = 0x0000bf80u;
+    asm("" : "+s"(low));
+    u32x4 &part = stage < 2 ? s.hi : stage < 4 ? s.mid : s.lo;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int c = j >> 1, i = 2 * (j & 1);
+        f32x2 v = {__uint_as_float(left.c[c][i]), __uint_as_float(left.c[c][i + 1])};
+        if ((stage & 1) == 0) {
+            part[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+        } else {
+            const bf16x2 r = __builtin_bit_cast(bf16x2, (uint32_t)part[j]);
+            left.c[c][i] = __float_as_uint(__builtin_amdgcn_fdot2_f32_bf16(r, __builtin_bit_cast(bf16x2, low), v[0], false));
+            left.c[c][i + 1] = __float_as_uint(__builtin_amdgcn_fdot2_f32_bf16(r, __builtin_bit_cast(bf16x2, 0xbf800000u), v[1], false));
+        }
+    }
+}
+// product 0..5 of two such sums
+__device__ __forceinline__ void mma_part(int product, f32x16 &acc, const Split8 &p, const Split8 &q) {
+    const u32x4 a = product == 0 ? p.lo : product == 2 || product == 3 ? p.mid : p.hi;
+    const u32x4 b = product == 1 ? q.lo : product == 2 || product == 4 ? q.mid : q.hi;
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+}
 
 // erf by Abramowitz & Stegun 7.1.26 (|error| <= 1.5e-7): a reciprocal, an exponential and
 // five multiply-adds instead of the library routine's branches.  The same exponential,
@@ -171,6 +218,14 @@ template <bool kNarrow> __device__ __forceinline__ float act_grad(float x, int a
         return g.cdf + x * g.pdf;
     }
     return 1.f;
+}
+
+// f(0), f(1), .. f(N - 1), each argument a compile-time constant
+template <typename F, int... I> __device__ __forceinline__ void for_each_index(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F> __device__ __forceinline__ void for_each_index(F &&f) {
+    for_each_index(f, std::make_integer_sequence<int, N>{});
 }
 
 // ---- kernel arguments -------------------------------------------------------
@@ -303,6 +358,7 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
     constexpr int MB = Elem<T>::kBlk;                // MFMA block edge
     constexpr int TI = WN / MB, TJ = WM / MB;        // MFMA blocks per wave (cols, rows)
     constexpr int kAccRegs = MB * MB / 64;           // accumulator registers per block
+    constexpr bool kSplit = sizeof(T) == 4;          // products of bf16 parts, see Split8
     constexpr int kChunksPerStep = 64 / MB;          // 16-byte contraction chunks one MFMA step consumes per row
     constexpr int NP = BN * 8 / kLoaders;            // 16-byte chunks per loading thread per slab
     constexpr int NQ = BM * 8 / kLoaders;
@@ -617,9 +673,9 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
         issue_part(std::integral_constant<int, PSHAPE>{}, Pb, prm.ldp, p_kc_chunk, p_voff, std::integral_constant<int, NP>{}, k0,
                    (uint32_t)(buf * P_BYTES), it_lo, it_hi);
     };
-    auto issue_q = [&](int k0, int buf) {
+    auto issue_q = [&](int k0, int buf, int it_lo = 0, int it_hi = 1 << 20) {
         issue_part(std::integral_constant<int, QSHAPE>{}, Qb, prm.ldq, q_kc_chunk, q_voff, std::integral_constant<int, NQ>{}, k0,
-                   (uint32_t)(Q_BASE + buf * Q_BYTES), 0, 1 << 20, gather_q ? q_gather_bytes : (int64_t)1 << 40);
+                   (uint32_t)(Q_BASE + buf * Q_BYTES), it_lo, it_hi, gather_q ? q_gather_bytes : (int64_t)1 << 40);
     };
 
     // Data-grad with the activation derivative, 16-bit types: the tile of saved
@@ -727,9 +783,9 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
             for (int r = 0; r < kAccRegs; ++r) acc[x][y][r] = 0.f;
 
     // Main loop, one basic block per slab, software-pipelined by hand.  A slab is worked
-    // through in four phases.  fp32 (32 x 32 blocks): a phase is one contraction step over
-    // all block columns.  16-bit (16 x 16 blocks): a phase is half the block columns of one
-    // of the slab's two contraction steps, so the Q fragments are read every other phase.
+    // through in four phases.  fp32 in 64 x 64 (one block column): in two, the first of which also does what is said of the
+    // second and third below, each one contraction step.  Else a phase is half the block columns of one of the slab's two contraction steps (16-bit elements: 32
+    // of them, fp32 in bf16 parts: 16), so the Q fragments are read every other phase.
     // P buffer pc holds slab s, pn slab s+1, pf_buf receives slab s+2; Q buffer s%2 holds
     // slab s.  Per slab:
     //   phase 0     : MFMAs of the phase, LDS reads of phase 1 between them
@@ -745,41 +801,96 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
     // covers the reads that follow the barrier (with part of phase 3 ahead of the barrier
     // the step measured 0.8 % slower).  Past the last slab the
     // loads return zeros and land in buffers nobody reads, which keeps the body branch-free.
-    constexpr int kPhases = 4;
-    constexpr int PF = (MB == 32) ? TI : TI / 2;                // block columns per phase
-    constexpr int kPReadsPerFrag = (PSHAPE == kMC) ? (sizeof(T) == 2 ? 2 : 4) : 1;
-    constexpr int kQReadsPerFrag = (QSHAPE == kMC) ? (sizeof(T) == 2 ? 2 : 4) : 1;
-    constexpr int kMfma = PF * TJ * (sizeof(T) == 4 ? 4 : 1);   // MFMA instructions per phase
+    constexpr bool kWhole = TI == 1;                            // a phase is a whole contraction step
+    constexpr int kPhases = kWhole ? 2 : 4;
+    constexpr int PF = kWhole ? TI : TI / 2;                    // block columns per phase
+    constexpr int kPReadsPerFrag = ((PSHAPE == kMC) ? (sizeof(T) == 2 ? 2 : 4) : 1) * (kSplit ? 2 : 1);
+    constexpr int kQReadsPerFrag = ((QSHAPE == kMC) ? (sizeof(T) == 2 ? 2 : 4) : 1) * (kSplit ? 2 : 1);
+    constexpr int kMfma = PF * TJ * (kSplit ? 6 : sizeof(T) == 4 ? 4 : 1);   // MFMA instructions per phase
     // a phase's reads go out early, one per MFMA (two where they outnumber the MFMAs); the remaining MFMAs follow
-    constexpr int kReadsPerMfma = EXTRA > 0 && PF * kPReadsPerFrag + TJ * kQReadsPerFrag > kMfma ? 2 : 1;
-    static_assert(NP % 2 == 0 && NP / 2 <= kMfma, "the P loads of a slab go out in two halves, one load per MFMA");
+    constexpr int kReadsPerMfma = (EXTRA > 0 || kSplit) && PF * kPReadsPerFrag + TJ * kQReadsPerFrag > kMfma ? 2 : 1;
+    static_assert(NP % 2 == 0 && (kWhole ? NP : NP / 2) <= kMfma, "the P loads of a slab go out in two halves, one load per MFMA");
     // phases that carry the two halves: phase 3 carries the Q loads, phase 0 is left to let
     // the load queue drain (0 and 1 measured 0.5 % slower per step, all in phase 0 1 %)
-    constexpr int kPLoadPhaseA = 1, kPLoadPhaseB = 2;
+    constexpr int kPLoadPhaseA = kWhole ? 0 : 1, kPLoadPhaseB = kWhole ? 0 : 2, kPLoadsPerPhase = kWhole ? NP : NP / 2;
     // contraction step, first block column, Q fragment buffer of a phase; does it start a step
-    auto phase_ks = [](int ph) { return MB == 32 ? ph : ph >> 1; };
-    auto phase_x0 = [](int ph) { return MB == 32 ? 0 : (ph & 1) * PF; };
-    auto phase_qbuf = [](int ph) { return MB == 32 ? (ph & 1) : ((ph >> 1) & 1); };
-    auto phase_reads_q = [](int ph) { return MB == 32 || (ph & 1) == 0; };
+    auto phase_ks = [](int ph) { return kWhole ? ph : ph >> 1; };
+    auto phase_x0 = [](int ph) { return kWhole ? 0 : (ph & 1) * PF; };
+    auto phase_qbuf = [](int ph) { return kWhole ? (ph & 1) : ((ph >> 1) & 1); };
+    auto phase_reads_q = [](int ph) { return kWhole || (ph & 1) == 0; };
     auto phase_reads = [&](int ph) { return PF * kPReadsPerFrag + (phase_reads_q(ph) ? TJ * kQReadsPerFrag : 0); };
+
+    constexpr int kSplitFrom = kMfma / 4;   // the MFMA by which a phase's fragments are there to be taken apart
 
     const int n_slabs = (K + BKE - 1) / BKE;
     const bool aux_pref = kAuxPrefetch && n_slabs >= 2 && split_part < 0 && !fixup;  // both tail slabs exist
-    u32x4 pf[2][PF], qf[2][TJ];
+    typedef typename std::conditional<kSplit, Raw8, u32x4>::type Frag;
+    Frag pf[2][PF], qf[2][TJ];
+    Split8 p_parts[2][kSplit ? PF : 1], q_parts[2][kSplit ? TJ : 1];
+    auto read_frag = [&](const unsigned char *slab, int shape, int extent, int r0, int ks) -> Frag {
+        if constexpr (kSplit) return Raw8{{frag(slab, shape, extent, r0, 2 * ks), frag(slab, shape, extent, r0, 2 * ks + 1)}};
+        else return frag(slab, shape, extent, r0, ks);
+    };
     // the fragments of phase ph, in the order its MFMAs (x outer, y inner) first need them
     auto read_phase = [&](int ph, const unsigned char *sp, const unsigned char *sq) {
         if (phase_reads_q(ph)) {
 #pragma unroll
-            for (int y = 0; y < TJ; ++y) qf[phase_qbuf(ph)][y] = frag(sq, QSHAPE, BM, wave_m0 + y * MB, phase_ks(ph));
+            for (int y = 0; y < TJ; ++y) qf[phase_qbuf(ph)][y] = read_frag(sq, QSHAPE, BM, wave_m0 + y * MB, phase_ks(ph));
         }
 #pragma unroll
-        for (int x = 0; x < PF; ++x) pf[ph & 1][x] = frag(sp, PSHAPE, BN, wave_n0 + (phase_x0(ph) + x) * MB, phase_ks(ph));
+        for (int x = 0; x < PF; ++x) pf[ph & 1][x] = read_frag(sp, PSHAPE, BN, wave_n0 + (phase_x0(ph) + x) * MB, phase_ks(ph));
     };
-    auto mma_phase = [&](int ph, int x_lo, int x_hi) {
+    auto mma_phase = [&](int ph, auto exact) {
+        if constexpr (!kSplit) {
 #pragma unroll
-        for (int x = x_lo; x < x_hi; ++x)
+            for (int x = 0; x < PF; ++x)
 #pragma unroll
-            for (int y = 0; y < TJ; ++y) Elem<T>::mma(acc[phase_x0(ph) + x][y], pf[ph & 1][x], qf[phase_qbuf(ph)][y]);
+                for (int y = 0; y < TJ; ++y) Elem<T>::mma(acc[phase_x0(ph) + x][y], pf[ph & 1][x], qf[phase_qbuf(ph)][y]);
+        } else if constexpr (decltype(exact)::value) {
+#pragma unroll
+            for (int x = 0; x < PF; ++x)
+#pragma unroll
+                for (int y = 0; y < TJ; ++y)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        Elem<T>::mma(acc[phase_x0(ph) + x][y], pf[ph & 1][x].c[h], qf[phase_qbuf(ph)][y].c[h]);
+        }
+    };
+    // fp32 in bf16 parts: fragment f of a phase (the Q fragments it reads first, then its P fragments), its 16-byte reads and its stages
+    auto phase_frags = [&](int ph) { return PF + (phase_reads_q(ph) ? TJ : 0); };
+    auto read_half = [&](int ph, int f, int h, const unsigned char *sp, const unsigned char *sq) {
+        if constexpr (kSplit) {
+            const int x = phase_reads_q(ph) ? f - TJ : f;
+            if (x < 0) qf[phase_qbuf(ph)][f].c[h] = frag(sq, QSHAPE, BM, wave_m0 + f * MB, 2 * phase_ks(ph) + h);
+            else pf[ph & 1][x].c[h] = frag(sp, PSHAPE, BN, wave_n0 + (phase_x0(ph) + x) * MB, 2 * phase_ks(ph) + h);
+        }
+    };
+    auto stage_frag = [&](int ph, int f, int stage) {
+        if constexpr (kSplit) {
+            const int x = phase_reads_q(ph) ? f - TJ : f;
+            if (x < 0) split_stage(stage, qf[phase_qbuf(ph)][f], q_parts[phase_qbuf(ph)][f]);
+            else split_stage(stage, pf[ph & 1][x], p_parts[ph & 1][x]);
+        }
+    };
+    // Phase ph, one MFMA after the other, and between them the reads of phase `next` from sp and sq, this phase's loads (load(i): the
+    // one after MFMA i) and the stages that take the next phase's fragments apart.  A fragment's stages follow one another with
+    // those of the others in between, so that none waits for the one before it.
+    auto split_phase = [&](auto ph_tag, auto next_tag, const unsigned char *sp, const unsigned char *sq, auto load) {
+        if constexpr (kSplit) {
+            constexpr int ph = decltype(ph_tag)::value, next = decltype(next_tag)::value;
+            constexpr int kSpan = kMfma - kSplitFrom, frags = PF + (kWhole || (next & 1) == 0 ? TJ : 0), stages = frags * kSplitStages;
+            for_each_index<kMfma>([&](auto mfma) {
+                constexpr int i = decltype(mfma)::value;
+                if constexpr (i < frags) { read_half(next, i, 0, sp, sq); read_half(next, i, 1, sp, sq); }
+                constexpr int block = i % (PF * TJ), x = block / TJ, y = block % TJ;
+                mma_part(i / (PF * TJ), acc[phase_x0(ph) + x][y], p_parts[ph & 1][x], q_parts[phase_qbuf(ph)][y]);
+                load(i);
+                constexpr int from = i <= kSplitFrom ? 0 : ((i - kSplitFrom) * stages + kSpan - 1) / kSpan;
+                constexpr int to = i < kSplitFrom ? 0 : ((i + 1 - kSplitFrom) * stages + kSpan - 1) / kSpan;
+                for_each_index<to - from>([&](auto c) { stage_frag(next, (from + c) % frags, (from + c) / frags); });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        }
     };
     // s_waitcnt vmcnt(n) lgkmcnt(0): at most n of this wave's loads still in flight, all LDS reads done
     auto wait_loads = [&](auto n_tag) {
@@ -795,7 +906,7 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    auto main_loop = [&](auto with_bias, auto loads_tag) {
+    auto main_loop = [&](auto with_bias, auto loads_tag, auto exact) {
         constexpr bool kBias = decltype(with_bias)::value;
         constexpr bool kLoads = decltype(loads_tag)::value;  // this wave requests slabs
         constexpr int kNoWait = 63;
@@ -810,7 +921,12 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
         wait_loads(std::integral_constant<int, kLoads ? (1 + kAhead) * (NP + NQ) : kNoWait>{});  // slab 0 has landed
         slab_barrier();
         if constexpr (kBias) add_q_chunks(0);
+        constexpr bool kParts = kSplit && !decltype(exact)::value;
         read_phase(0, smem, smem + Q_BASE);
+        if constexpr (kParts) {
+#pragma unroll
+            for (int c = 0; c < phase_frags(0) * kSplitStages; ++c) stage_frag(0, c % phase_frags(0), c / phase_frags(0));
+        }
         __builtin_amdgcn_sched_barrier(0);
 
         int pc = 0, qk = 0;
@@ -821,8 +937,17 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
             const int qc = kAhead == 0 ? (s & 1) : qk, qn = kAhead == 0 ? ((s + 1) & 1) : (qk == kQBufs - 1 ? 0 : qk + 1);
             const unsigned char *sp = smem + pc * P_BYTES;
             const unsigned char *sq = smem + Q_BASE + qc * Q_BYTES;
+            if constexpr (kParts) {
+                for_each_index<kPhases - 1>([&](auto ph) {
+                    split_phase(ph, std::integral_constant<int, ph + 1>{}, sp, sq, [&](int i) {
+                        if (!kLoads) return;
+                        if (ph == kPLoadPhaseA && i < kPLoadsPerPhase) issue_p((s + 2 + kAhead) * BKE, pf_buf, i, i + 1);
+                        else if (ph == kPLoadPhaseB && i < kPLoadsPerPhase) issue_p((s + 2 + kAhead) * BKE, pf_buf, NP / 2 + i, NP / 2 + i + 1);
+                    });
+                });
+            }
 #pragma unroll
-            for (int ph = 0; ph + 1 < kPhases; ++ph) {
+            for (int ph = 0; !kParts && ph + 1 < kPhases; ++ph) {
                 if (kLoads && ph == kPLoadPhaseA) {
                     const int past_end = s + 2 - n_slabs;  // >= 0: slab s+2 does not exist
                     if (kAuxPrefetch && aux_pref && past_end >= 0) issue_aux(past_end, (uint32_t)(pf_buf * P_BYTES));
@@ -833,12 +958,12 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
                     if (!(kAuxPrefetch && aux_pref && past_end >= 0)) issue_p((s + 2 + kAhead) * BKE, pf_buf, NP / 2, NP);
                 }
                 read_phase(ph + 1, sp, sq);
-                mma_phase(ph, 0, PF);
+                mma_phase(ph, exact);
 #pragma unroll
                 for (int i = 0; i < kMfma; ++i) {
                     if (i * kReadsPerMfma < phase_reads(ph + 1)) __builtin_amdgcn_sched_group_barrier(0x100, kReadsPerMfma, 0);  // LDS reads
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                       // one MFMA
-                    if (kLoads && (ph == kPLoadPhaseA || ph == kPLoadPhaseB) && i < NP / 2) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // one load
+                    if (kLoads && (ph == kPLoadPhaseA || ph == kPLoadPhaseB) && i < kPLoadsPerPhase) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // one load
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -846,6 +971,15 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
             wait_loads(std::integral_constant<int, kLoads ? NP + kAhead * (NP + NQ) : kNoWait>{});
             slab_barrier();
             if constexpr (kBias) add_q_chunks((s + 1) & 1);
+            constexpr int kQLoadsPerMfma = (NQ + kMfma - 1) / kMfma;
+            if constexpr (kParts) {
+                split_phase(std::integral_constant<int, kPhases - 1>{}, std::integral_constant<int, 0>{}, smem + pn * P_BYTES, smem + Q_BASE + qn * Q_BYTES, [&](int i) {
+                    if (kLoads && i * kQLoadsPerMfma < NQ) issue_q((s + 2 + kAhead) * BKE, qc, i * kQLoadsPerMfma, (i + 1) * kQLoadsPerMfma);
+                });
+                pc = pn;
+                qk = qn;
+                continue;
+            }
             if constexpr (kLoads) {
                 const int past_end = s + 2 - n_slabs;
                 if (kAuxPrefetch && kAuxParts == 4 && aux_pref && past_end >= 0)
@@ -854,8 +988,7 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
                     issue_q((s + 2 + kAhead) * BKE, qc);
             }
             read_phase(0, smem + pn * P_BYTES, smem + Q_BASE + qn * Q_BYTES);
-            mma_phase(kPhases - 1, 0, PF);
-            constexpr int kQLoadsPerMfma = (NQ + kMfma - 1) / kMfma;
+            mma_phase(kPhases - 1, exact);
 #pragma unroll
             for (int i = 0; i < kMfma; ++i) {
                 if (i * kReadsPerMfma < phase_reads(0)) __builtin_amdgcn_sched_group_barrier(0x100, kReadsPerMfma, 0);
@@ -893,27 +1026,62 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
         wait_loads(std::integral_constant<int, 0>{});
         slab_barrier();
     };
-    auto run_loop = [&](auto with_bias) {
+    auto run_loop = [&](auto with_bias, auto exact) {
         if constexpr (EXTRA > 0) {
-            main_loop(with_bias, std::false_type{});
+            main_loop(with_bias, std::false_type{}, exact);
             return;
         }
-        if (wave_u < (uint32_t)kLoadWaves) main_loop(with_bias, std::true_type{});
-        else main_loop(with_bias, std::false_type{});
+        if (wave_u < (uint32_t)kLoadWaves) main_loop(with_bias, std::true_type{}, exact);
+        else main_loop(with_bias, std::false_type{}, exact);
+    };
+    // whether any wave of the workgroup says so; LDS is free where it is asked
+    auto any_wave = [&](bool say) {
+        int *flags = (int *)smem;
+        const bool any = __builtin_amdgcn_ballot_w64(say) != 0;
+        if (lane == 0 && wave_u < (uint32_t)kWaves) flags[wave_u] = any;
+        __syncthreads();
+        int all = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) all |= flags[w];
+        __syncthreads();
+        return __builtin_amdgcn_readfirstlane(all) != 0;
     };
     if constexpr (EXTRA > 0) {
         if (wave_u >= (uint32_t)kWaves) {
             load_loop();
+            if constexpr (kSplit)
+                if (any_wave(false)) load_loop();
             return;
         }
     }
     bool want_bias = false;
     if constexpr (RAGGED == kRaggedK && QSHAPE == kMC) want_bias = prm.bias_grad != nullptr && nt == 0;
     if constexpr (RAGGED == kRaggedK && QSHAPE == kMC) {
-        if (want_bias) run_loop(std::true_type{});
-        else run_loop(std::false_type{});
+        if (want_bias) run_loop(std::true_type{}, std::false_type{});
+        else run_loop(std::false_type{}, std::false_type{});
     } else {
-        if (!fixup) run_loop(std::false_type{});
+        if (!fixup) run_loop(std::false_type{}, std::false_type{});
+    }
+    if constexpr (kSplit) {
+        // a tile with a NaN or an infinity once more, as the fp32 MFMA has it (the bias gradient's sums come from the elements themselves)
+        if (!fixup) {
+            float none = 0.f;
+#pragma unroll
+            for (int x = 0; x < TI; ++x)
+#pragma unroll
+                for (int y = 0; y < TJ; ++y)
+#pragma unroll
+                    for (int r = 0; r < kAccRegs; ++r) none = fmaf(acc[x][y][r], 0.f, none);
+            if (any_wave(none != 0.f)) {   // (0 x infinity and 0 x NaN are NaN)
+#pragma unroll
+                for (int x = 0; x < TI; ++x)
+#pragma unroll
+                    for (int y = 0; y < TJ; ++y)
+#pragma unroll
+                        for (int r = 0; r < kAccRegs; ++r) acc[x][y][r] = 0.f;
+                run_loop(std::false_type{}, std::true_type{});
+            }
+        }
     }
 
     // Split tail tiles.  Part p of tail tile i keeps its accumulators in
@@ -1036,6 +1204,9 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
         }
     };
     // staging -> memory
+    // (fp32 weight gradients nontemporally: nothing of the launch reads them.  8 experts of 2048 x 8192, 2 / 32 / 64 rows each: 134 / 165 / 196
+    // us through the caches, 116 / 141 / 172 like this)
+    constexpr int kPolicy = RAGGED == kRaggedK && sizeof(T) == 4 ? 2 : 0;
     auto stage_out = [&](T *dst, int col_base) {
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(dst, 0, (int)kOutOfRange, kRsrcFlags);
 #pragma unroll
@@ -1045,7 +1216,7 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
             for (int i = 0; i < kIoBatch; ++i) v[i] = *(const u32x4 *)(stg + ((i0 + i) * kIoRows + io_r) * kStgRow + io_c * 16);
 #pragma unroll
             for (int i = 0; i < kIoBatch; ++i)
-                __builtin_amdgcn_raw_buffer_store_b128(v[i], rs, (int)tile_offset((i0 + i) * kIoRows + io_r, col_base), 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(v[i], rs, (int)tile_offset((i0 + i) * kIoRows + io_r, col_base), 0, kPolicy);
         }
     };
     // accumulator side: 4 consecutive columns of one row
@@ -1341,7 +1512,7 @@ int launch_tiles(GemmParams &prm, hipStream_t stream) {
 }
 
 // Tile counts, then the launch for the requested epilogue.  prm.block_m x prm.block_n (256 x 256,
-// 128 x 256, 128 x 128 or, fp32 alone, 64 x 64, chosen by the host from the segment lengths) is the tile.
+// 128 x 256, 128 x 128, 64 x 128; fp32: 128 x 128, 64 x 64; chosen by the host from the segment lengths) is the tile.
 // EPI_MASK lists the epilogues a product can be asked for, so that only those kernels
 // are built.
 template <typename T, int BM, int BN, int PS, int QS, int RG, int EPI_MASK, int LOADERS = kLoadersCompute>
@@ -1373,19 +1544,24 @@ int launch_for_height(GemmParams &prm, int epi, hipStream_t stream) {
 
 template <typename T, int PS, int QS, int RG, int EPI_MASK>
 int launch_by_epilogue(GemmParams &prm, int epi, hipStream_t stream) {
-    if constexpr (sizeof(T) == 4)
-        if (prm.block_m == 64 && prm.block_n == 64) return launch_for_height<T, 64, 64, PS, QS, RG, EPI_MASK>(prm, epi, stream);
-    if constexpr (sizeof(T) == 2 && RG == kRaggedRows)
+    if constexpr (sizeof(T) == 4) {
+        if (prm.block_n == 64) return launch_for_height<T, 64, 64, PS, QS, RG, EPI_MASK>(prm, epi, stream);
+        if constexpr (RG == kRaggedRows)
+            if (prm.loaders == kLoadersAlone) return launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK, kLoadersAlone>(prm, epi, stream);
+        return launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK>(prm, epi, stream);
+    } else {
+    if constexpr (RG == kRaggedRows)
         if (prm.block_n == 128) {
             if (prm.block_m == 64) return launch_for_height<T, 64, 128, PS, QS, RG, EPI_MASK, kLoadersAlone>(prm, epi, stream);
             return prm.loaders == kLoadersAlone ? launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK, kLoadersAlone>(prm, epi, stream)
                                                 : launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK, kLoadersShared>(prm, epi, stream);
         }
-    if constexpr (sizeof(T) == 4 || RG == kRaggedK)
+    if constexpr (RG == kRaggedK)
         if (prm.block_m == 128 && prm.block_n == 128) return launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK>(prm, epi, stream);
     if (prm.block_m == 128 && prm.block_n == 256) return launch_for_height<T, 128, 256, PS, QS, RG, EPI_MASK>(prm, epi, stream);
     if (prm.block_m == 256 && prm.block_n == 256) return launch_for_height<T, 256, 256, PS, QS, RG, EPI_MASK>(prm, epi, stream);
     return fail(FMOE_EINVAL, "tile %d x %d is not built", prm.block_m, prm.block_n);
+    }
 }
 
 }  // namespace gemm

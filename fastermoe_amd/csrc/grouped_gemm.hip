@@ -87,10 +87,10 @@ void fill_table(SegmentTable *tab, const int64_t *counts, int e0, int e1, int64_
 
 // Tile of a launch.  Weight gradients of 16-bit types: 256 x 256 (one workgroup per compute unit) unless that gives too few tiles
 // to occupy the chip: then 128 x 256, and when even those number fewer than two per compute unit, 128 x 128 (two workgroups per
-// compute unit).  Their row-ragged products: rows_16bit_tile.  fp32 tiles take four times as long per slab and are bound by the
-// matrix pipe whatever their shape, so there the question is only how evenly they fill the chip: f32_rows_tile, f32_wgrad_tile.
-// FMOE_GEMM_TILE=256x256|128x256|128x128 forces one shape (for tests and measurements); for fp32 also 64x64, for the row-ragged
-// products of 16-bit types also 64x128 and, one workgroup per compute unit, 128x128+.
+// compute unit).  Row-ragged products: rows_tile.  fp32 has no tiles 256 wide (128 x 128 came within 4 % of 256 x 256 where
+// that was ahead); its weight gradients: f32_wgrad_tile.
+// FMOE_GEMM_TILE=256x256|128x256|128x128 forces one shape (for tests and measurements; fp32 takes 128x128 for the first two); for fp32
+// also 64x64, for the row-ragged products 128x128+ (one workgroup per compute unit) and, 16-bit types alone, 64x128.
 struct TileShape {
     int bm, bn;
     int loaders = kLoadersCompute;
@@ -100,41 +100,25 @@ bool is_16bit(int dtype) { return dtype == FMOE_BF16 || dtype == FMOE_F16; }
 bool forced_tile(int dtype, bool rows, TileShape *tile) {
     const char *e = getenv("FMOE_GEMM_TILE");
     if (!e) return false;
-    if (!strcmp(e, "256x256")) *tile = {256, 256};
-    else if (!strcmp(e, "128x256")) *tile = {128, 256};
+    const bool f32 = dtype == FMOE_F32;
+    if (!strcmp(e, "256x256")) *tile = f32 ? TileShape{128, 128} : TileShape{256, 256};
+    else if (!strcmp(e, "128x256")) *tile = f32 ? TileShape{128, 128} : TileShape{128, 256};
     else if (!strcmp(e, "128x128")) *tile = {128, 128, rows && is_16bit(dtype) ? kLoadersShared : kLoadersCompute};
-    else if (!strcmp(e, "128x128+") && rows && is_16bit(dtype)) *tile = {128, 128, kLoadersAlone};
+    else if (!strcmp(e, "128x128+") && rows) *tile = {128, 128, kLoadersAlone};
     else if (!strcmp(e, "64x128") && rows && is_16bit(dtype)) *tile = {64, 128, kLoadersAlone};
-    else if (!strcmp(e, "64x64") && dtype == FMOE_F32) *tile = {64, 64};
+    else if (!strcmp(e, "64x64") && f32) *tile = {64, 64};
     else return false;
     return true;
 }
 
-// Row-ragged products in fp32.  us for 64 x 64 / 128 x 128 / 256 x 256, by the launch's number of 256 x 256 tiles:
-// 72 tiles (1024 rows, 16 experts of 768 x 3072): 85 / 107 / 190; 144 (8192 rows, 8 of 512 x 1024): 89 / 113 / 132;
-// 192 (8192 rows, 64 of 1024 x 1024): 216 / 212 / 260; 576 (8192 rows, 8 of 2048 x 4096): 1168 / 1095 / 1144;
-// 1152 (16384 rows, 16 of 1024 x 4096): 1163 / 1113 / 1267; 2112 (32768 rows, 8 of 1024 x 4096): 2242 / 2147 / 2115.
-// Few tiles with a long contraction want the 128 x 128 ones, whose contraction is split over workgroups.  Tiles,
-// contraction, us for 64 x 64 / 128 x 128: 18, 3072: 108 / 84; 36, 4608: 642 / 631; 48, 4096: 505 / 497; but 39, 1984: 72 / 84; 42, 2816: 484 / 518;
-// 36, 1536: 83 / 111; 120, 3136: 353 / 381; 126, 1664: 193 / 211.
-TileShape f32_rows_tile(int64_t tiles_256, int64_t contraction) {
-    if (tiles_256 < 160 && contraction < 70 * tiles_256) return {64, 64};
-    return tiles_256 < 1536 ? TileShape{128, 128} : TileShape{256, 256};
-}
-
-// Weight gradients in fp32 (no contraction is split).  With a compute unit's tiles bound by its matrix pipe, a launch takes
-// as long as the unit with the most tile area: 64 x 64 where that is less by more than the 5 % its operands' extra reads
-// cost.  us for 64 x 64 / 128 x 128 / 256 x 256: 12 experts of 576 x 576, 76032 rows: 547 / 773 / 1468; 64 of 1408 x 704,
-// 17152 rows: 318 / 376 / 539; 8 of 2240 x 2240, 6016 rows: 497 / 521 / 559; 16 of 2048 x 512, 46336 rows: 757 / 714 / 708; 16 of
-// 2560 x 2560, 10035 rows: 1067 / 1003 / 1074.  Many tiles of a few rows per expert are bound by their stores and keep the
-// large tile: 32 of 2048 x 4096, 1024 rows: 405 / 372 / 342; 32 of 2304 x 4608, 768: 423 / 368 / 353; not 32 of
-// 2112 x 4224, 3072: 630 / 622 / 657.
-TileShape f32_wgrad_tile(int64_t experts, int64_t out_feat, int64_t in_feat, int64_t rows) {
-    if (experts * ceil_div(out_feat, 256) * ceil_div(in_feat, 256) >= 640 && rows < 48 * experts) return {256, 256};
+// Weight gradients in fp32 (no contraction is split): 128 x 128, or 64 x 64 where the compute unit with the most tile area then has less by
+// more than the 30 % that their operands' extra reads cost.  us for 64 x 64 / 128 x 128: 8 experts of
+// 576 x 512, 1600 rows: 22 / 25; 4 of 768 x 512, 25552: 197 / 258; 16 of 1472 x 704, 9893: 167 / 149; 8 of 2048 x 4096, 8192: 951 / 729.
+TileShape f32_wgrad_tile(int64_t experts, int64_t out_feat, int64_t in_feat) {
     const int64_t units = device_compute_units();
     const int64_t low = ceil_div(experts * ceil_div(out_feat, 64) * ceil_div(in_feat, 64), units) * 64 * 64;
     const int64_t high = ceil_div(experts * ceil_div(out_feat, 128) * ceil_div(in_feat, 128), units) * 128 * 128;
-    return 105 * low < 100 * high ? TileShape{64, 64} : TileShape{128, 128};
+    return 130 * low < 100 * high ? TileShape{64, 64} : TileShape{128, 128};
 }
 
 constexpr TileShape kManyTiles{256, 256, kLoadersCompute, true};
@@ -162,19 +146,30 @@ constexpr RowShape kRowShapes[] = {
     {{128, 128, kLoadersShared}, 2, 3.1, 0.30, 0.71, 4.9},   {{128, 256, kLoadersCompute}, 1, 4.2, 0.38, 0.53, 5.2},
     {{256, 256, kLoadersCompute}, 1, 6.9, 0.57, 0.83, 5.0},
 };
-template <typename RowTiles> TileShape rows_16bit_tile(RowTiles row_tiles, double weight_bytes, int64_t n_cols, int64_t contraction) {
-    const double slabs = (double)ceil_div(contraction, 64);
+// fp32, three bf16 products to one (Split8 in gemm_kernel.hpp), slabs of 32 elements: fitted in the same way to 220 products of 4 to 128
+// experts, 64 to 32768 rows and 512 to 13056 features, off by a tenth; the shape picked takes 1.02 times what the best one does, 64 x 64 alone
+// 1.16, 128 x 128 two to a unit 1.09, one to a unit 1.07 times.  us for the three (and on the fp32 MFMA, best of 64 x 64, 128 x 128 and
+// 256 x 256): 4 experts of 640 -> 512, 251 rows: 18 / 33 / 29; 4 of 832 -> 3328, 547: 55 / 46 / 42; 8 of 1024 -> 512, 8192: 79 / 73 / 73 (98); 32 of
+// 640 -> 1344, 2635: 63 / 59 / 61; 8 of 2048 -> 4096, 8192: 1063 / 787 / 816 (1095).
+constexpr RowShape kRowShapesF32[] = {
+    {{64, 64}, 4, 2.25, 0.58, 1.38, 2.45}, {{128, 128}, 2, 10.3, 0.68, 1.78, 2.85}, {{128, 128, kLoadersAlone}, 1, 8.4, 0.78, 0.40, 3.04},
+};
+template <int N, typename RowTiles> TileShape rows_tile(const RowShape (&shapes)[N], RowTiles row_tiles, double live, int64_t n_cols,
+                                                        int64_t contraction, int element_bytes) {
+    const double slabs = (double)ceil_div(contraction, kSlabBytes / element_bytes);
+    const double weight_bytes = live * (double)n_cols * (double)contraction * element_bytes;
     const int64_t units = device_compute_units();
     double best = 0;
     TileShape pick{};
-    for (const RowShape &s : kRowShapes) {
+    for (const RowShape &s : shapes) {
         const int64_t tiles = row_tiles(s.tile.bm) * ceil_div(n_cols, s.tile.bn), places = units * s.per_unit;
         const int64_t full = tiles / places, rest = tiles % places;
         double us = (double)full * (s.start + slabs * (s.alone + s.shared));
         if (rest) {
-            const TailSplit split = s.tile.bm == 64 ? TailSplit{0, 1, 0} : plan_tail_split((int)std::min<int64_t>(tiles, INT32_MAX), (int)slabs, (int)units);
+            const TailSplit split = s.tile.bm == 64 ? TailSplit{0, 1, 0} : plan_tail_split((int)std::min<int64_t>(tiles, INT32_MAX), (int)slabs, (int)units,
+                                                                                          element_bytes == 4 ? slab_weight_of<float>() : 1);
             if (split.k_split > 1 && full == 0)   // (and two short kernels after it)
-                us += 8 + s.start + split.split_slabs * (s.alone + s.shared * (double)(rest * split.k_split) / (double)places);
+                us += 8 + s.start + split.split_slabs * (s.alone + s.shared * std::min(1.0, (double)(rest * split.k_split) / (double)places));
             else
                 us += s.start + slabs * (s.alone + s.shared * (double)rest / (double)places);
         }
@@ -184,6 +179,10 @@ template <typename RowTiles> TileShape rows_16bit_tile(RowTiles row_tiles, doubl
         if (pick.bm == 0 || us < best) { best = us; pick = s.tile; }
     }
     return pick;
+}
+template <typename RowTiles> TileShape rows_tile(int dtype, RowTiles row_tiles, double live, int64_t n_cols, int64_t contraction) {
+    return dtype == FMOE_F32 ? rows_tile(kRowShapesF32, row_tiles, live, n_cols, contraction, 4)
+                             : rows_tile(kRowShapes, row_tiles, live, n_cols, contraction, 2);
 }
 
 // The activation code the kernels see.  For results that are rounded to a 16-bit type GELU and its
@@ -213,11 +212,8 @@ TileShape pick_rows_tile(const int64_t *counts, int64_t n_expert, int64_t row_lo
         }
         return tiles;
     };
-    const int64_t tiles = row_tiles(256) * ceil_div(n_cols, 256);
-    if (dtype == FMOE_F32) return f32_rows_tile(tiles, contraction);
-    if (tiles >= 512) return kManyTiles;
-    const double live = (double)row_tiles(INT32_MAX);   // (experts with rows)
-    return rows_16bit_tile(row_tiles, live * (double)n_cols * (double)contraction * 2, n_cols, contraction);
+    if (dtype != FMOE_F32 && row_tiles(256) * ceil_div(n_cols, 256) >= 512) return kManyTiles;
+    return rows_tile(dtype, row_tiles, (double)row_tiles(INT32_MAX) /* experts with rows */, n_cols, contraction);
 }
 
 // ragged rows over a device table: the host does not know the counts; rows_cap rows spread over
@@ -227,14 +223,13 @@ TileShape pick_rows_tile_estimate(int64_t rows_cap, int64_t n_expert, int64_t n_
     if (forced_tile(dtype, true, &forced)) return forced;
     const int64_t whole = rows_cap / 256;
     const int64_t tiles = (whole + std::min<int64_t>(n_expert, std::max<int64_t>(whole, 1)) / 2) * ceil_div(n_cols, 256);
-    if (dtype == FMOE_F32) return f32_rows_tile(tiles, contraction);
-    if (tiles >= 512) return kManyTiles;
+    if (dtype != FMOE_F32 && tiles >= 512) return kManyTiles;
     // every expert that can have a row, with its share of the rows and half a tile past the whole ones
     const int64_t live = std::max<int64_t>(1, std::min(n_expert, rows_cap));
     auto row_tiles = [&](int height) {
         return (int64_t)((double)live * std::max(1.0, (double)rows_cap / ((double)live * height) + 0.5) + 0.5);
     };
-    return rows_16bit_tile(row_tiles, (double)live * (double)n_cols * (double)contraction * 2, n_cols, contraction);
+    return rows_tile(dtype, row_tiles, (double)live, n_cols, contraction);
 }
 
 // Row tiles of gemm_unaligned.hip, 64 or 128 rows high: the low ones where the high ones would leave part of the
@@ -255,10 +250,10 @@ TileShape unaligned_tile_estimate(int64_t rows_cap, int64_t n_expert, int64_t n_
 }
 
 // weight gradient: C is [out, in] per expert
-TileShape pick_wgrad_tile(int64_t n_experts_written, int64_t out_feat, int64_t in_feat, int64_t rows, int dtype) {
+TileShape pick_wgrad_tile(int64_t n_experts_written, int64_t out_feat, int64_t in_feat, int dtype) {
     TileShape forced;
     if (forced_tile(dtype, false, &forced)) return forced;
-    if (dtype == FMOE_F32) return f32_wgrad_tile(n_experts_written, out_feat, in_feat, rows);
+    if (dtype == FMOE_F32) return f32_wgrad_tile(n_experts_written, out_feat, in_feat);
     return pick_tile(n_experts_written * ceil_div(out_feat, 256) * ceil_div(in_feat, 256));
 }
 
@@ -380,12 +375,13 @@ bool use_ring(const TileShape &tile, int dtype) {
 // and 13.8 / 36.3 / 55.5; 8 of 4096 x 14336, 8 / 32 / 64 / 128: 142 / 191 / 191 / 192 and 99 / 161 / 180 / 243; 256 of
 // 1024 x 2048, 256 / 512 / 1024: 134 / 179 / 205 and 124 / 170 / 210; 64 of 8192 x 2048, 64 / 128 / 256: 298 / 367 / 372
 // and 249 / 334 / 389.
-// float32, where a tile's padding costs products and not only places: at most 40 rows per expert on average.  us on the tiles and here:
-// 8 experts of 2048 x 8192, 2 / 16 / 32 / 48 rows each: 260 / 260 / 265 / 266 and 109 / 151 / 209 / 280; 32 of 1024 x 1024, 2 / 32 / 48:
-// 75 / 70 / 70 and 31 / 51 / 66; 4 of 768 x 3072, 2 / 32 / 64: 54 / 54 / 31 and 11 / 17 / 26.
+// float32: at most 24 rows per expert on average, or 40 where the 128 x 128 tiles would number less than half the compute units.  us on the best
+// tiles and here: 8 experts of 2048 x 8192, 2 / 16 / 24 / 32 rows each: 166 / 197 / 196 / 203 and 96 / 154 / 185 / 225; 32 of 1024 x 1024,
+// 16 / 24 / 32: 50 / 49 / 49 and 46 / 48 / 60; 16 of 640 x 2560: 46 / 46 / 46 and 33 / 39 / 48; 4 of 768 x 3072, 2 / 32 / 40: 27 / 28 / 28 and 15 / 21 / 23.
 bool use_skinny(int64_t rows_cap, int64_t n_expert, int64_t out_feat, int dtype) {
     if ((!is_16bit(dtype) && dtype != FMOE_F32) || getenv("FMOE_GEMM_TILE")) return false;
-    if (dtype == FMOE_F32) return rows_cap <= 40 * n_expert;
+    if (dtype == FMOE_F32)
+        return rows_cap <= 24 * n_expert || (rows_cap <= 40 * n_expert && n_expert * ceil_div(out_feat, 128) * 2 < device_compute_units());
     return rows_cap <= 2 * n_expert || (rows_cap <= 8 * n_expert && n_expert * ceil_div(out_feat, 128) < 1024);
 }
 
@@ -666,7 +662,7 @@ int grouped_linear_wgrad(const LinearWgradArgs &a, const int64_t *counts, int64_
         FMOE_REQUIRE(a.gw && (a.dev_rows_cap == 0 || (a.gy && a.x)), "linear_wgrad: NULL tensor");
         // (with no rows at all the pointers may be NULL: every expert's contraction is empty and nothing is read)
         const bool fast = is_fast(a.dtype, {a.gy, a.x, a.gw}, {a.in_feat, a.out_feat});
-        const TileShape tile = pick_wgrad_tile(n_expert, a.out_feat, a.in_feat, a.dev_rows_cap, a.dtype);
+        const TileShape tile = pick_wgrad_tile(n_expert, a.out_feat, a.in_feat, a.dtype);
         GemmParams prm{};
         const bool any_grid = !fast && a.dev_any_grid && is_16bit(a.dtype);
         if (int rc = device_table_launch("linear_wgrad", prm, a.dev_tab, a.dev_rows_cap, n_expert, fast || any_grid)) return rc;
@@ -687,7 +683,7 @@ int grouped_linear_wgrad(const LinearWgradArgs &a, const int64_t *counts, int64_
     FMOE_REQUIRE(a.gw && (total == 0 || (a.gy && a.x)), "linear_wgrad: NULL tensor");
     const Plan plan = plan_contraction(counts, n_expert, row_lo, row_hi, last_chunk);
     const bool fast = is_fast(a.dtype, {a.gy, a.x, a.gw}, {a.in_feat, a.out_feat});
-    const TileShape tile = pick_wgrad_tile(plan.last - plan.first + 1, a.out_feat, a.in_feat, row_hi - row_lo, a.dtype);
+    const TileShape tile = pick_wgrad_tile(plan.last - plan.first + 1, a.out_feat, a.in_feat, a.dtype);
     for (int e0 = plan.first; e0 <= plan.last; e0 += kMaxGroupExperts) {
         const int e1 = std::min(plan.last, e0 + kMaxGroupExperts - 1);
         GemmParams prm{};
