@@ -87,7 +87,7 @@ void fill_table(SegmentTable *tab, const int64_t *counts, int e0, int e1, int64_
 
 // Tile of a launch.  Weight gradients of 16-bit types: 256 x 256 (one workgroup per compute unit) unless that gives too few tiles
 // to occupy the chip: then 128 x 256, and when even those number fewer than two per compute unit, 128 x 128 (two workgroups per
-// compute unit).  Row-ragged products: rows_tile.  fp32 has no tiles 256 wide (128 x 128 came within 4 % of 256 x 256 where
+// compute unit).  Row-ragged products: rows_16bit_tile, rows_f32_tile.  fp32 has no tiles 256 wide (128 x 128 came within 4 % of 256 x 256 where
 // that was ahead); its weight gradients: f32_wgrad_tile.
 // FMOE_GEMM_TILE=256x256|128x256|128x128 forces one shape (for tests and measurements; fp32 takes 128x128 for the first two); for fp32
 // also 64x64, for the row-ragged products 128x128+ (one workgroup per compute unit) and, 16-bit types alone, 64x128.
@@ -146,30 +146,19 @@ constexpr RowShape kRowShapes[] = {
     {{128, 128, kLoadersShared}, 2, 3.1, 0.30, 0.71, 4.9},   {{128, 256, kLoadersCompute}, 1, 4.2, 0.38, 0.53, 5.2},
     {{256, 256, kLoadersCompute}, 1, 6.9, 0.57, 0.83, 5.0},
 };
-// fp32, three bf16 products to one (Split8 in gemm_kernel.hpp), slabs of 32 elements: fitted in the same way to 220 products of 4 to 128
-// experts, 64 to 32768 rows and 512 to 13056 features, off by a tenth; the shape picked takes 1.02 times what the best one does, 64 x 64 alone
-// 1.16, 128 x 128 two to a unit 1.09, one to a unit 1.07 times.  us for the three (and on the fp32 MFMA, best of 64 x 64, 128 x 128 and
-// 256 x 256): 4 experts of 640 -> 512, 251 rows: 18 / 33 / 29; 4 of 832 -> 3328, 547: 55 / 46 / 42; 8 of 1024 -> 512, 8192: 79 / 73 / 73 (98); 32 of
-// 640 -> 1344, 2635: 63 / 59 / 61; 8 of 2048 -> 4096, 8192: 1063 / 787 / 816 (1095).
-constexpr RowShape kRowShapesF32[] = {
-    {{64, 64}, 4, 2.25, 0.58, 1.38, 2.45}, {{128, 128}, 2, 10.3, 0.68, 1.78, 2.85}, {{128, 128, kLoadersAlone}, 1, 8.4, 0.78, 0.40, 3.04},
-};
-template <int N, typename RowTiles> TileShape rows_tile(const RowShape (&shapes)[N], RowTiles row_tiles, double live, int64_t n_cols,
-                                                        int64_t contraction, int element_bytes) {
-    const double slabs = (double)ceil_div(contraction, kSlabBytes / element_bytes);
-    const double weight_bytes = live * (double)n_cols * (double)contraction * element_bytes;
+template <typename RowTiles> TileShape rows_16bit_tile(RowTiles row_tiles, double weight_bytes, int64_t n_cols, int64_t contraction) {
+    const double slabs = (double)ceil_div(contraction, 64);
     const int64_t units = device_compute_units();
     double best = 0;
     TileShape pick{};
-    for (const RowShape &s : shapes) {
+    for (const RowShape &s : kRowShapes) {
         const int64_t tiles = row_tiles(s.tile.bm) * ceil_div(n_cols, s.tile.bn), places = units * s.per_unit;
         const int64_t full = tiles / places, rest = tiles % places;
         double us = (double)full * (s.start + slabs * (s.alone + s.shared));
         if (rest) {
-            const TailSplit split = s.tile.bm == 64 ? TailSplit{0, 1, 0} : plan_tail_split((int)std::min<int64_t>(tiles, INT32_MAX), (int)slabs, (int)units,
-                                                                                          element_bytes == 4 ? slab_weight_of<float>() : 1);
+            const TailSplit split = s.tile.bm == 64 ? TailSplit{0, 1, 0} : plan_tail_split((int)std::min<int64_t>(tiles, INT32_MAX), (int)slabs, (int)units);
             if (split.k_split > 1 && full == 0)   // (and two short kernels after it)
-                us += 8 + s.start + split.split_slabs * (s.alone + s.shared * std::min(1.0, (double)(rest * split.k_split) / (double)places));
+                us += 8 + s.start + split.split_slabs * (s.alone + s.shared * (double)(rest * split.k_split) / (double)places);
             else
                 us += s.start + slabs * (s.alone + s.shared * (double)rest / (double)places);
         }
@@ -180,9 +169,37 @@ template <int N, typename RowTiles> TileShape rows_tile(const RowShape (&shapes)
     }
     return pick;
 }
-template <typename RowTiles> TileShape rows_tile(int dtype, RowTiles row_tiles, double live, int64_t n_cols, int64_t contraction) {
-    return dtype == FMOE_F32 ? rows_tile(kRowShapesF32, row_tiles, live, n_cols, contraction, 4)
-                             : rows_tile(kRowShapes, row_tiles, live, n_cols, contraction, 2);
+
+// The same for fp32 (products out of bf16 parts: Split8 in gemm_kernel.hpp; slabs of 32 elements).  A compute unit takes its m tiles
+// per_unit at a time, each such round start + slabs (alone + shared m / per_unit) us long, and as long as the fullest unit has tiles; the
+// parts of a tail whose contraction is shared come after them.  Fitted to 220 products of 4 to 128 experts, 64 to 32768 rows and 512 to 13056
+// features, then moved to where the shape picked is the best one most often: it takes 1.01 times what that does, 64 x 64 alone 1.16, 128 x 128 two to a
+// unit 1.09, one to a unit 1.07 times.  us for the three (and before, on the fp32 MFMA): 4 experts of 640 -> 512, 251 rows: 18 / 33 / 29; 4 of 832 -> 3328,
+// 547: 55 / 46 / 42; 32 of 640 -> 1344, 2635: 63 / 59 / 61; 8 of 1024 -> 512, 8192: 79 / 92 / 92 (98); 8 of 2048 -> 4096, 8192: 1063 / 787 / 816 (1095).
+struct F32RowShape {
+    TileShape tile;
+    int per_unit;
+    double start, alone, shared, tail, stream; // us, us per slab, us, TB/s
+};
+constexpr F32RowShape kF32RowShapes[] = {
+    {{64, 64}, 4, 1.4, 0.32, 2.07, 0, 2.4}, {{128, 128}, 2, 4.0, 0.03, 2.47, 19, 4.4}, {{128, 128, kLoadersAlone}, 1, 4.3, 0.24, 0.96, 14, 3.3},
+};
+template <typename RowTiles> TileShape rows_f32_tile(RowTiles row_tiles, double weight_bytes, int64_t n_cols, int64_t contraction) {
+    const int64_t slabs = ceil_div(contraction, kSlabBytes / 4), units = device_compute_units();
+    double best = 0;
+    TileShape pick{};
+    for (const F32RowShape &s : kF32RowShapes) {
+        const int64_t tiles = row_tiles(s.tile.bm) * ceil_div(n_cols, s.tile.bn);
+        const TailSplit split = s.tile.bm == 64 ? TailSplit{(int)std::min<int64_t>(tiles, INT32_MAX), 1, 0}
+                                                : plan_tail_split((int)std::min<int64_t>(tiles, INT32_MAX), (int)slabs, (int)units);
+        const int64_t fullest = ceil_div(split.main_tiles, units), rounds = fullest / s.per_unit, rest = fullest % s.per_unit;
+        auto round = [&](int64_t m) { return s.start + (double)slabs * (s.alone + s.shared * (double)m / s.per_unit); };
+        double us = (double)rounds * round(s.per_unit) + (rest ? round(rest) : 0);
+        if (split.k_split > 1) us += s.tail + split.split_slabs * (s.alone + s.shared / s.per_unit);
+        us = std::max(us + 3, weight_bytes * 1e-6 / s.stream + 4);
+        if (pick.bm == 0 || us < best) { best = us; pick = s.tile; }
+    }
+    return pick;
 }
 
 // The activation code the kernels see.  For results that are rounded to a 16-bit type GELU and its
@@ -212,8 +229,10 @@ TileShape pick_rows_tile(const int64_t *counts, int64_t n_expert, int64_t row_lo
         }
         return tiles;
     };
-    if (dtype != FMOE_F32 && row_tiles(256) * ceil_div(n_cols, 256) >= 512) return kManyTiles;
-    return rows_tile(dtype, row_tiles, (double)row_tiles(INT32_MAX) /* experts with rows */, n_cols, contraction);
+    const double weights = (double)row_tiles(INT32_MAX) * (double)n_cols * (double)contraction;   // (of experts with rows)
+    if (dtype == FMOE_F32) return rows_f32_tile(row_tiles, weights * 4, n_cols, contraction);
+    if (row_tiles(256) * ceil_div(n_cols, 256) >= 512) return kManyTiles;
+    return rows_16bit_tile(row_tiles, weights * 2, n_cols, contraction);
 }
 
 // ragged rows over a device table: the host does not know the counts; rows_cap rows spread over
@@ -229,7 +248,8 @@ TileShape pick_rows_tile_estimate(int64_t rows_cap, int64_t n_expert, int64_t n_
     auto row_tiles = [&](int height) {
         return (int64_t)((double)live * std::max(1.0, (double)rows_cap / ((double)live * height) + 0.5) + 0.5);
     };
-    return rows_tile(dtype, row_tiles, (double)live, n_cols, contraction);
+    const double weights = (double)live * (double)n_cols * (double)contraction;
+    return dtype == FMOE_F32 ? rows_f32_tile(row_tiles, weights * 4, n_cols, contraction) : rows_16bit_tile(row_tiles, weights * 2, n_cols, contraction);
 }
 
 // Row tiles of gemm_unaligned.hip, 64 or 128 rows high: the low ones where the high ones would leave part of the
@@ -409,7 +429,7 @@ int64_t route_workspace_bytes(const DevRoute &route, int64_t contraction, int dt
     const int n_slabs = (int)std::min<int64_t>(ceil_div(contraction, kSlabBytes / eb), 1 << 24);
     // (contractions that the tiles would not split pay on neither kernel: 48 slabs and a tail of two tiles per XCD on the
     // persistent one take 187 us cut and not cut)
-    if (route.kernel == DevKernel::kSkinny || !tail_split_possible(n_slabs, eb == 4 ? 2 : 1)) return 0;
+    if (route.kernel == DevKernel::kSkinny || !tail_split_possible(n_slabs)) return 0;
     const int64_t tile_bytes = (int64_t)route.tile.bm * route.tile.bn * (int64_t)sizeof(float);
     if (route.kernel == DevKernel::kRing) return ring_split_possible(n_slabs) ? ring_ws_tiles(ring_workgroups()) * tile_bytes : 0;
     // (a split never has more parts than compute units, and 64 x 64 tiles are never split)
