@@ -381,34 +381,64 @@ __device__ __forceinline__ void topk_insert(float (&val)[K], int (&idx)[K], floa
     }
 }
 
-// Merges the sorted lists of the G lanes of a group (G consecutive lanes, a power of two of at least K):
-// K rounds of taking the best head of all lists -- the larger value, of equal ones the lower expert --
-// after which every lane of the group holds the group's K best in out_val / out_idx.  That is the
-// order topk_insert gives a single lane that sees all the experts in ascending order.
-template <int K, int G>
-__device__ __forceinline__ void topk_merge(float (&val)[K], int (&idx)[K], float (&out_val)[K], int (&out_idx)[K]) {
+// A (logit, expert) pair as one unsigned number that orders as the gate selects: the larger logit first, of equal ones the lower
+// expert, NaN as -inf, -0 as 0.  Zero is no pair at all (an empty place), below every pair.  The logits are values of T: 16 bits of
+// them and 16 of the expert make 32, float32 takes 64.  Keeping, exchanging and taking the larger of two pairs is then a
+// maximum instead of two compares and four selects.
+template <typename T> struct TopkKey {
+    typedef typename std::conditional<sizeof(T) == 2, uint32_t, unsigned long long>::type Key;
+    static constexpr int kHalf = 4 * (int)sizeof(Key);   // bits of the expert, and of the logit
+    static constexpr uint32_t kSign = 1u << (8 * sizeof(T) - 1), kMask = 2 * kSign - 1;
+    static __device__ __forceinline__ Key make(float x, int e) {
+        x = x != x ? -__builtin_inff() : x + 0.f;
+        uint32_t bits;
+        if constexpr (sizeof(T) == 2) bits = __builtin_bit_cast(uint16_t, (T)x);
+        else bits = __builtin_bit_cast(uint32_t, x);
+        bits = (bits & kSign) ? ~bits & kMask : bits | kSign;
+        return ((Key)bits << kHalf) | (Key)((1u << 16) - 1 - (uint32_t)e);
+    }
+    static __device__ __forceinline__ int expert(Key key) { return key == 0 ? -1 : (int)((1u << 16) - 1 - ((uint32_t)key & 0xffffu)); }
+    static __device__ __forceinline__ float logit(Key key) {
+        if (key == 0) return -__builtin_inff();
+        uint32_t bits = (uint32_t)(key >> kHalf);
+        bits = (bits & kSign) ? bits & ~kSign : ~bits & kMask;
+        if constexpr (sizeof(T) == 2) return (float)__builtin_bit_cast(T, (uint16_t)bits);
+        else return __builtin_bit_cast(float, bits);
+    }
+};
+static_assert(kMaxExpert < (1 << 16), "an expert's number takes 16 bits of a key");
+
+// Keeps the K largest keys in descending order.
+template <typename Key, int K> __device__ __forceinline__ void key_insert(Key (&keys)[K], Key x) {
 #pragma unroll
     for (int j = 0; j < K; ++j) {
-        float bv = idx[0] >= 0 ? val[0] : -__builtin_inff();
-        int bi = idx[0] >= 0 ? idx[0] : INT32_MAX;
+        const Key larger = keys[j] > x ? keys[j] : x;
+        x = keys[j] > x ? x : keys[j];
+        keys[j] = larger;
+    }
+}
+
+// Merges the sorted lists of the G lanes of a group (G consecutive lanes, a power of two of at least K; all lanes of
+// the wave take part): K rounds of taking the largest head of all lists, after which every lane of the group holds the group's K
+// best in val / idx.  Keys of different experts differ, so that only the list which gave the head drops it.
+template <typename T, int K, int G>
+__device__ __forceinline__ void topk_merge(typename TopkKey<T>::Key (&keys)[K], float (&val)[K], int (&idx)[K]) {
+    typedef typename TopkKey<T>::Key Key;
 #pragma unroll
-        for (int off = 1; off < G; off <<= 1) {
-            const float ov = __shfl_xor(bv, off, kWave);
-            const int oi = __shfl_xor(bi, off, kWave);
-            const bool take = ov > bv || (ov == bv && oi < bi);
-            bv = take ? ov : bv;
-            bi = take ? oi : bi;
-        }
-        out_val[j] = bv;
-        out_idx[j] = bi == INT32_MAX ? -1 : bi;
-        const bool pop = idx[0] >= 0 && idx[0] == bi;
+    for (int j = 0; j < K; ++j) {
+        Key best = keys[0];
+        auto take = [&](Key other) { best = other > best ? other : best; };
+        if constexpr (G > 1) take(segtab::lane_xor<1>(best));
+        if constexpr (G > 2) take(segtab::lane_xor<2>(best));
+        if constexpr (G > 4) take(segtab::lane_xor<4>(best));
+        if constexpr (G > 8) take(segtab::lane_xor<8>(best));
+        if constexpr (G > 16) take(segtab::lane_xor<16>(best));
+        if constexpr (G > 32) take(segtab::lane_xor<32>(best));
+        val[j] = TopkKey<T>::logit(best);
+        idx[j] = TopkKey<T>::expert(best);
+        const bool pop = keys[0] == best;
 #pragma unroll
-        for (int i = 0; i < K; ++i) {
-            const float nv = i + 1 < K ? val[i + 1 < K ? i + 1 : i] : -__builtin_inff();
-            const int ni = i + 1 < K ? idx[i + 1 < K ? i + 1 : i] : -1;
-            val[i] = pop ? nv : val[i];
-            idx[i] = pop ? ni : idx[i];
-        }
+        for (int i = 0; i < K; ++i) keys[i] = pop ? (i + 1 < K ? keys[i + 1 < K ? i + 1 : i] : (Key)0) : keys[i];
     }
 }
 
@@ -444,12 +474,12 @@ __device__ __forceinline__ void topk_store(int sub, int64_t token, const int (&i
 // Top-k of the gate logits and the scores of the selected experts.
 //
 // G lanes share a token: each keeps the K largest of its part of the row (16-byte pieces when the rows
-// are aligned) in a sorted register list -- an insertion is K compare-selects, and a later logit
-// only displaces a strictly smaller one -- and the G lists are merged in K rounds of lane exchanges, so
-// the choices come out in descending order of the logit, ties to the lower expert.  With one lane per token
-// (the routing histogram in the same kernel, 2048 slots per workgroup) a row of 256 logits was a chain
-// of 256 insertions on a few waves: 71 us for 64 tokens and 77 us for 8192 at top-8; 16 lanes per token take
-// 13 us for either, and the histogram is left to the routing kernels.
+// are aligned) in a sorted register list of keys, and the G lists are merged in K rounds of lane exchanges, so
+// the choices come out in descending order of the logit, ties to the lower expert.  Bound by that chain: with one lane per
+// token (the routing histogram in the same kernel, 2048 slots per workgroup) a row of 256 logits was 256 insertions on a few
+// waves, 71 us for 64 tokens and 77 us for 8192 at top-8; 16 lanes per token took 12.4 and 12.8 with logits and experts
+// compared and exchanged (by address) apart, and take 5.0 and 5.2 as keys exchanged in the vector pipe.  The histogram is left to
+// the routing kernels.
 template <typename T, int K, int G>
 __global__ __launch_bounds__(kBlock) void gate_topk_kernel(
     const T *__restrict__ logits, int64_t n_tokens, int n_expert, int score_mode, int vector_rows,
@@ -458,21 +488,23 @@ __global__ __launch_bounds__(kBlock) void gate_topk_kernel(
     const int sub = threadIdx.x % G;
     const int64_t token = (int64_t)blockIdx.x * (kBlock / G) + threadIdx.x / G;
     const T *row = logits + (token < n_tokens ? token : n_tokens - 1) * n_expert;
-    float val[K], best[K], score[K];
-    int idx[K], chosen[K];
+    float best[K], score[K];
+    int chosen[K];
+    typedef TopkKey<T> Pair;
+    typename Pair::Key keys[K];
 #pragma unroll
-    for (int j = 0; j < K; ++j) { val[j] = -__builtin_inff(); idx[j] = -1; }
+    for (int j = 0; j < K; ++j) keys[j] = 0;
     if (vector_rows) {
         for (int e = sub * kVec; e < n_expert; e += G * kVec) {
             alignas(16) T chunk[kVec];
             *(uint4 *)chunk = *(const uint4 *)(row + e);
 #pragma unroll
-            for (int c = 0; c < kVec; ++c) topk_insert<K>(val, idx, (float)chunk[c], e + c);
+            for (int c = 0; c < kVec; ++c) key_insert(keys, Pair::make((float)chunk[c], e + c));
         }
     } else {
-        for (int e = sub; e < n_expert; e += G) topk_insert<K>(val, idx, (float)row[e], e);
+        for (int e = sub; e < n_expert; e += G) key_insert(keys, Pair::make((float)row[e], e));
     }
-    topk_merge<K, G>(val, idx, best, chosen);
+    topk_merge<T, K, G>(keys, best, chosen);
     topk_scores<K>(best, chosen, score_mode, score);
     if (token < n_tokens) topk_store<T, K>(sub, token, chosen, score, topk_idx, topk_score);
 }
@@ -612,18 +644,20 @@ __global__ __launch_bounds__(kBlock) void gate_linear_topk_kernel(
     constexpr int kSub = kBlock / kGateTokens;   // lanes per token
     const int t = threadIdx.x / kSub, sub = threadIdx.x % kSub;
     const int64_t token = token0 + t;
-    float val[K], best[K], score[K];
-    int idx[K], chosen[K];
+    float best[K], score[K];
+    int chosen[K];
+    typedef TopkKey<T> Pair;
+    typename Pair::Key keys[K];
 #pragma unroll
-    for (int j = 0; j < K; ++j) { val[j] = -__builtin_inff(); idx[j] = -1; }
+    for (int j = 0; j < K; ++j) keys[j] = 0;
     const int ws = n_eb * 16 * kGateStride;   // one wave's tile
     for (int e = sub; e < n_expert; e += kSub) {
         const float *p = part_lds + e * kGateStride + t;
         float logit = ((p[0] + p[ws]) + p[2 * ws]) + p[3 * ws];
         if (bias != nullptr) logit += (float)bias[e];
-        topk_insert<K>(val, idx, (float)(T)logit, e);
+        key_insert(keys, Pair::make((float)(T)logit, e));
     }
-    topk_merge<K, kSub>(val, idx, best, chosen);
+    topk_merge<T, K, kSub>(keys, best, chosen);
     topk_scores<K>(best, chosen, score_mode, score);
     if (token < n_tokens) topk_store<T, K>(sub, token, chosen, score, topk_idx, topk_score);
 }

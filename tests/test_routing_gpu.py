@@ -271,6 +271,25 @@ def test_naive_gate_hands_its_routing_to_the_layer(device):
     assert torch.allclose(val2, torch.gather(logits, 1, idx2), rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("e,k", [(8, 8), (64, 4), (65, 8), (250, 8), (256, 2), (513, 8), (8192, 8)])
+def test_gate_topk_orders_equal_and_special_logits(dtype, e, k, device):
+    """Many equal logits, both zeros, infinities, NaN (as -inf) and the smallest subnormals: by descending logit, of equal ones the
+    lower expert, as sorting the pairs gives on the CPU; the scores are the logits."""
+    gen = torch.Generator().manual_seed(e + k)
+    tiny = 2.0 ** {torch.float32: -149, torch.bfloat16: -133, torch.float16: -24}[dtype]
+    pool = torch.tensor([0.0, -0.0, 1.5, -1.5, float("inf"), -float("inf"), float("nan"), tiny, -tiny, 3.0, -3.0], dtype=torch.float64)
+    logits = pool[torch.randint(len(pool), (37, e), generator=gen)].to(dtype)
+    logits[0] = -float("inf")
+    logits[1] = torch.arange(e, dtype=torch.float64).neg().to(dtype)
+    idx, score = fmoe_native.gate_topk_route(logits.to(device), k, 0)[:2]
+    values = logits.double()
+    values = torch.where(values.isnan(), torch.full_like(values, -float("inf")), values)
+    want = torch.stack([torch.tensor(sorted(range(e), key=lambda i: (-row[i], i))[:k]) for row in values.tolist()])
+    assert torch.equal(idx.cpu(), want)
+    assert torch.equal(score.double().cpu(), values.gather(1, want))
+
+
 def test_gate_topk_with_masked_out_logits(device):
     """Logits of -inf (experts masked out by a caller) and NaN: a token with fewer than top_k finite
     logits still names top_k distinct experts -- the finite ones first, then the lowest-numbered of
