@@ -20,6 +20,7 @@
 #include "common.hpp"
 #include "segment_table.hpp"
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -285,6 +286,118 @@ __global__ __launch_bounds__(kSmallBlock) void route_small_kernel(
         if (i < n_slots && i >= routed) pos[i] = -1;
     }
     if (table != nullptr) segtab::small_table(total, n_expert, n_slots, table, table_lds);
+}
+
+// The same for experts that one wave holds, one per lane: past the one barrier behind the histogram every wave has the counts, their
+// prefixes and its own first rows in registers, and writes its slots and its part of the table without waiting for another.
+// Bound by launch and latency: the barriers, exchanges by address and walks over other waves' sums of the kernel above were most of its
+// time.  The largest of 16 waves walks 8 steps, as there; few slots take fewer waves.
+// us of the kernel above and of this one, slots and experts: 2, 32: 8.2 / 4.0; 509, 64: 12.7 / 6.6; 2000, 16: 9.0 / 5.7; 8192, 8: 14.8 / 10.3.
+constexpr int kFewExperts = kWave;
+// Prefix sum (with the lane's own value) over the wave, all lanes taking part: within rows of 16 lanes, then over the rows
+__device__ __forceinline__ int32_t wave_prefix(int32_t v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);    // row_shr 1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast 15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast 31 into rows 2 and 3
+    return v;
+}
+__global__ __launch_bounds__(kSmallBlock) void route_few_experts_kernel(
+    const int64_t *__restrict__ gate, int n_slots, int n_expert, int nbits, int64_t *__restrict__ expert_count,
+    int64_t *__restrict__ pos, int64_t *__restrict__ slot_to_row, int32_t *__restrict__ table) {
+    __shared__ int32_t bins[kSmallWaves][kFewExperts], next_row[kSmallWaves][kFewExperts];
+    const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave), waves = (int)blockDim.x / kWave;
+    const int steps = (n_slots + (int)blockDim.x - 1) / (int)blockDim.x;   // kStepsPerWave at most
+    const int wave_base = wave * steps * kWave;
+    int keys[kStepsPerWave];
+#pragma unroll
+    for (int s = 0; s < kStepsPerWave; ++s) {
+        const int i = wave_base + s * kWave + lane;
+        int64_t g = -1;
+        if (s < steps && i < n_slots) g = gate[i];
+        keys[s] = (g >= 0 && g < n_expert) ? (int)g : -1;
+    }
+    bins[wave][lane] = 0;
+    wave_lds_sync();
+    uint64_t peers[kStepsPerWave];
+#pragma unroll
+    for (int s = 0; s < kStepsPerWave; ++s) {
+        peers[s] = 0;
+        if (s < steps) {
+            peers[s] = match_mask(keys[s], keys[s] >= 0, nbits);
+            wave_bins_add(bins[wave], keys[s], keys[s] >= 0, peers[s]);
+        }
+    }
+    __syncthreads();
+    // lane e: expert e's slots of the waves before this one, all its slots, and the prefix over the experts
+    const int e = lane;
+    int32_t before = 0, rows = 0;
+#pragma unroll
+    for (int w = 0; w < kSmallWaves; ++w) {
+        const int32_t c = w < waves ? bins[w][e] : 0;
+        before += w < wave ? c : 0;
+        rows += c;
+    }
+    const int32_t hi = wave_prefix(rows), lo = hi - rows;
+    const int routed = __builtin_amdgcn_readlane(hi, kWave - 1);
+    int32_t *mine = next_row[wave];   // (the other waves may still be reading this one's bins)
+    mine[e] = hi - 1 - before;
+    wave_lds_sync();
+#pragma unroll
+    for (int s = 0; s < kStepsPerWave; ++s) {
+        if (s >= steps) break;
+        const int i = wave_base + s * kWave + lane;
+        const bool valid = keys[s] >= 0;
+        int row = -1;
+        if (valid) row = mine[keys[s]] - __popcll(peers[s] & lanes_below());
+        wave_lds_sync();   // every lane has read its expert's next row before the lowest peers lower it
+        if (valid && (peers[s] & lanes_below()) == 0) mine[keys[s]] -= __popcll(peers[s]);
+        wave_lds_sync();
+        if (valid) pos[row] = i;
+        if (slot_to_row && i < n_slots) slot_to_row[i] = row;
+        if (i < n_slots && i >= routed) pos[i] = -1;
+    }
+    if (wave == 1 && e < n_expert) expert_count[e] = rows;
+    if (table == nullptr) return;
+    // (the rows of all experts are at most n_slots, the table's capacity: nothing to clamp; tiles of both sizes fit 16 bits each)
+    const int32_t tiles[2] = {(rows + 255) / 256, (rows + 127) / 128};
+    const int32_t ends = wave_prefix(tiles[0] | tiles[1] << 16), all = __builtin_amdgcn_readlane(ends, kWave - 1);
+    const int32_t first[2] = {(ends & 0xffff) - tiles[0], (ends >> 16) - tiles[1]};
+    const int map256 = (int)segtab::map256_off(n_expert), map128 = (int)segtab::map128_off(n_slots, n_expert);
+    if (wave == 0) {   // the experts by descending rows
+        const int ex = segtab::expert_in_order<unsigned int>(rows, n_expert, nullptr);   // (one wave: nothing goes through a buffer)
+        const int first_row = __shfl(lo, ex, kWave), ex_rows = __shfl(rows, ex, kWave);
+        if (e < n_expert) ((int4 *)(table + segtab::order_off(n_slots, n_expert)))[e] = make_int4(ex, first_row, ex_rows, 0);
+    } else if (wave == 1) {
+        const int live = __popcll(__ballot(rows > 0));
+        if (e < n_expert) {
+            table[segtab::seg_off() + e] = lo;
+            table[segtab::pfx256_off(n_expert) + e] = first[0];
+            table[segtab::pfx128_off(n_expert) + e] = first[1];
+        }
+        if (e == 0) {
+            table[segtab::seg_off() + n_expert] = routed;
+            table[segtab::pfx256_off(n_expert) + n_expert] = all & 0xffff;
+            table[segtab::pfx128_off(n_expert) + n_expert] = all >> 16;
+            table[0] = n_expert;
+            table[segtab::kRows] = routed;
+            table[segtab::kTiles256] = all & 0xffff;
+            table[segtab::kTiles128] = all >> 16;
+            table[segtab::kMap256] = map256;
+            table[segtab::kMap128] = map128;
+            table[segtab::kRowsCap] = n_slots;
+            table[segtab::kLive] = live;
+        }
+    }
+    // every wave writes its share of each expert's row tiles
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int tile_rows = k == 0 ? 256 : 128;
+        int4 *map = (int4 *)(table + (k == 0 ? map256 : map128)) + first[k];
+        for (int j = wave; j < tiles[k]; j += waves) map[j] = make_int4(e, lo + j * tile_rows, min(rows - j * tile_rows, tile_rows), 0);
+    }
 }
 
 // ---------------------------------------------------------------- apply ----
@@ -1064,6 +1177,13 @@ int route_launch(const int64_t *gate, int64_t n_slots, int64_t n_expert, int64_t
                  int64_t *slot_to_row, int32_t *table, const RouteScratch &s, hipStream_t st) {
     const int E = (int)n_expert;
     // (the single workgroup's tables: 17 int32 per expert, 35 KiB of LDS at 512 experts beside the segment table's)
+    if (n_slots <= kSmallSlots && E <= kFewExperts) {
+        // a wave per 64 slots, up to 16; at least four, which share the writing of the table
+        const int waves = std::min(kSmallWaves, std::max(4, (int)ceil_div(n_slots, kWave)));
+        route_few_experts_kernel<<<1, waves * kWave, 0, st>>>(gate, (int)n_slots, E, ilog2_ceil(n_expert), expert_count, pos, slot_to_row, table);
+        FMOE_LAUNCH_CHECK();
+        return FMOE_OK;
+    }
     if (n_slots <= kSmallSlots && E <= 512) {
         route_small_kernel<<<1, kSmallBlock, (kSmallWaves + 1) * E * sizeof(int32_t), st>>>(
             gate, (int)n_slots, E, ilog2_ceil(n_expert), expert_count, pos, slot_to_row, table);

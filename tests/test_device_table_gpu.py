@@ -74,6 +74,33 @@ def test_route_with_its_segment_table(n_slots, n_expert, device):
         assert np.array_equal(got[key][:, :3], ref[key]), key
 
 
+@pytest.mark.parametrize("n_expert", [1, 2, 63, 64, 65])
+@pytest.mark.parametrize("n_slots", [1, 64, 65, 257, 1023, 4097, 8192])
+@pytest.mark.parametrize("spread", ["even", "one", "none"])
+def test_table_of_the_routing_against_the_one_of_its_counts(n_slots, n_expert, spread, device):
+    """The table that comes with the routing of few slots, on both sides of one expert per lane, is word for word the one that its
+    own kernel builds of the counts: header, prefixes, tiles and the experts by descending rows."""
+    g = torch.Generator().manual_seed(n_slots * 67 + n_expert)
+    gate = torch.randint(-1, n_expert, (n_slots,), generator=g)
+    if spread != "even":
+        gate[torch.rand(n_slots, generator=g) < 0.9] = n_expert - 1 if spread == "one" else -1
+    cnt, pos, s2r, table = fmoe_native.route_table(gate.to(device), n_expert)
+    ref_pos, ref_cnt = orouting.count_by_gate(gate.numpy(), n_expert)
+    total = int(ref_cnt.sum())
+    assert np.array_equal(cnt.cpu().numpy(), ref_cnt)
+    assert np.array_equal(pos[:total].cpu().numpy(), ref_pos) and (pos[total:] == -1).all()
+    inv = np.full(n_slots, -1, dtype=np.int64)
+    inv[ref_pos] = np.arange(total)
+    assert np.array_equal(s2r.cpu().numpy(), inv)
+    got, want = table.cpu().numpy(), fmoe_native.segment_table(cnt, n_slots).cpu().numpy()
+    assert got.size == want.size
+    head = HEADER + 3 * (n_expert + 1)
+    assert np.array_equal(got[:head], want[:head])
+    assert np.array_equal(got[-4 * n_expert:], want[-4 * n_expert:])
+    for key in ("tiles256", "tiles128"):
+        assert np.array_equal(_unpack(table, n_expert)[key], _unpack(torch.from_numpy(want), n_expert)[key]), key
+
+
 @pytest.mark.parametrize("name", sorted(CONFIG_COUNTS))
 def test_segment_table_at_the_configurations(name, device):
     g = torch.Generator().manual_seed(11)
