@@ -624,28 +624,29 @@ __global__ __launch_bounds__(kBlock) void gate_topk_kernel(
 
 // The gate's linear layer, its top-k and the scores in one kernel, for up to 64 experts: the logits
 // x W^T + b (fmoe/gates/naive_gate.py:26-31) are formed in registers and LDS and never written
-// to memory.  A workgroup owns kGateTokens tokens; its four waves split the contraction (wave w
-// takes the steps w, w + 4, ... of 128 bytes per row) and feed the MFMA straight from global
+// to memory.  A workgroup owns 16 kTB tokens; its kGateWaves waves split the contraction (wave w
+// takes the steps w, w + kGateWaves, ... of 128 bytes per row) and feed the MFMA straight from global
 // memory -- for the 16 x 16 block shapes a lane's operand is 16 contiguous bytes of one row of W
 // (expert lb of a 16-expert block) or of x (token lb of a 16-token block), so there is no staging
-// -- then leave their partial [expert][token] tiles in LDS.  Eight lanes per token add the four
+// -- then leave their partial [expert][token] tiles in LDS.  The token's lanes add the waves'
 // partials of the token's logits in wave order (a fixed order), add the bias, round to the
 // element type (what the layer's own output would have been) and keep the K largest exactly as
 // gate_topk_kernel does.  The routing histogram is left to the routing kernels that follow:
 // the contraction wants many small workgroups, the histogram few large ones.
 // For few tokens the kernel is one chain of load latencies per workgroup, so a group's loads go out
 // before the group ahead of it is multiplied.
-constexpr int kGateTokens = 32, kGateMaxExpert = 64, kGateStride = kGateTokens + 4;
+constexpr int kGateMaxExpert = 64;
+constexpr int gate_stride(int tokens) { return tokens + 4; }
 
-template <typename T, int K, int kEB>
-__global__ __launch_bounds__(kBlock) void gate_linear_topk_kernel(
+template <typename T, int K, int kEB, int kTB, int kGateWaves>   // 16-expert blocks there are accumulators for, 16-token blocks, waves
+__global__ __launch_bounds__(kGateWaves * kWave) void gate_linear_topk_kernel(
     const T *__restrict__ x, const T *__restrict__ w, const T *__restrict__ bias, int64_t n_tokens, int d,
     int n_expert, int score_mode, int64_t *__restrict__ topk_idx, T *__restrict__ topk_score) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
     typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-    extern __shared__ float part_lds[];   // [kWavesPerBlock][16 n_eb][kGateStride]
-    constexpr int kTB = kGateTokens / 16;   // kEB: 16-expert blocks this instantiation holds accumulators for
+    extern __shared__ float part_lds[];   // [kGateWaves][16 n_eb][kGateStride]
+    constexpr int kGateTokens = 16 * kTB, kGateStride = gate_stride(kGateTokens);
     constexpr int kPer = 16 / (int)sizeof(T);       // elements per 16-byte operand
     constexpr int kStep = 8 * kPer;                 // contraction elements per step of a wave (128 bytes per row)
     const int lane = lane_id(), wave = threadIdx.x / kWave, lb = lane & 15, hq = lane >> 4;
@@ -692,8 +693,8 @@ __global__ __launch_bounds__(kBlock) void gate_linear_topk_kernel(
     };
     // rows outside the problem read row 0 (and are dropped at the end): no bounds checks on the way.
     // A wave's step covers 128 bytes of every row -- whole cache lines, as two 64-byte halves (the
-    // operands of two products) -- and the four waves take the steps in turn.
-    constexpr int kUnroll = 2, kStride = kWavesPerBlock * kStep;
+    // operands of two products) -- and the waves take the steps in turn.
+    constexpr int kUnroll = 2, kStride = kGateWaves * kStep;
     // Workgroups start at different places of the contraction and wrap around: in step with each
     // other they would all ask for the same columns of their rows at the same time, which lie a whole
     // row length apart and so fall on a few memory channels.  (The order of the fp32 additions
@@ -754,7 +755,7 @@ __global__ __launch_bounds__(kBlock) void gate_linear_topk_kernel(
                 if (eb < n_eb) part_lds[((wave * n_eb + eb) * 16 + 4 * hq + r) * kGateStride + tb * 16 + lb] = acc[eb][tb][r];
     __syncthreads();
 
-    constexpr int kSub = kBlock / kGateTokens;   // lanes per token
+    constexpr int kSub = kGateWaves * kWave / kGateTokens;   // lanes per token
     const int t = threadIdx.x / kSub, sub = threadIdx.x % kSub;
     const int64_t token = token0 + t;
     float best[K], score[K];
@@ -766,7 +767,9 @@ __global__ __launch_bounds__(kBlock) void gate_linear_topk_kernel(
     const int ws = n_eb * 16 * kGateStride;   // one wave's tile
     for (int e = sub; e < n_expert; e += kSub) {
         const float *p = part_lds + e * kGateStride + t;
-        float logit = ((p[0] + p[ws]) + p[2 * ws]) + p[3 * ws];
+        float logit = p[0];
+#pragma unroll
+        for (int u = 1; u < kGateWaves; ++u) logit += p[u * ws];
         if (bias != nullptr) logit += (float)bias[e];
         key_insert(keys, Pair::make((float)(T)logit, e));
     }
@@ -1432,20 +1435,30 @@ namespace {
 template <typename T>
 int launch_gate_linear(const void *x, const void *w, const void *bias, int64_t n_tokens, int d, int E, int top_k,
                        int score_mode, int64_t *topk_idx, void *topk_score, hipStream_t st) {
-    const unsigned grid = (unsigned)ceil_div(n_tokens, kGateTokens);
-    const size_t lds = (size_t)kWavesPerBlock * ((E + 15) / 16 * 16) * kGateStride * sizeof(float);
+    // Up to 16 tokens per compute unit: 16 tokens to a workgroup of eight waves, which is half the chain of load latencies; with more,
+    // 32 to one of four, which reads w half as often.  us with 32 and four / 16 and eight: one token, 32 experts of 1024: 5.4 / 4.4; 509, 64
+    // of 2048: 21.4 / 16.7; 1000, 16 of 768: 7.4 / 5.7; 4096, 8 of 512, float32: 6.6 / 5.3.
+    constexpr int64_t kFewTokens = 16 * 256;
+    const bool few = n_tokens <= kFewTokens;
+    const int tokens = few ? 16 : 32, waves = few ? 8 : 4;
+    const unsigned grid = (unsigned)ceil_div(n_tokens, tokens);
+    const size_t lds = (size_t)waves * ((E + 15) / 16 * 16) * gate_stride(tokens) * sizeof(float);
     // (accumulators for 1, 2 or 4 blocks of 16 experts: fewer registers, more waves per compute unit)
+#define FMOE_GATE_LINEAR_LAUNCH_AS(KK, EB, TB, WAVES)                                                                       \
+    gate_linear_topk_kernel<T, KK, EB, TB, WAVES><<<grid, WAVES * kWave, lds, st>>>((const T *)x, (const T *)w, (const T *)bias, \
+                                                                                  n_tokens, d, E, score_mode, topk_idx, (T *)topk_score)
 #define FMOE_GATE_LINEAR_LAUNCH(KK)                                                                                         \
     do {                                                                                                                    \
-        if (E <= 16)                                                                                                        \
-            gate_linear_topk_kernel<T, KK, 1><<<grid, kBlock, lds, st>>>((const T *)x, (const T *)w, (const T *)bias,        \
-                                                                         n_tokens, d, E, score_mode, topk_idx, (T *)topk_score); \
-        else if (E <= 32)                                                                                                   \
-            gate_linear_topk_kernel<T, KK, 2><<<grid, kBlock, lds, st>>>((const T *)x, (const T *)w, (const T *)bias,        \
-                                                                         n_tokens, d, E, score_mode, topk_idx, (T *)topk_score); \
-        else                                                                                                                \
-            gate_linear_topk_kernel<T, KK, 4><<<grid, kBlock, lds, st>>>((const T *)x, (const T *)w, (const T *)bias,        \
-                                                                         n_tokens, d, E, score_mode, topk_idx, (T *)topk_score); \
+        if (E <= 16) {                                                                                                      \
+            if (few) FMOE_GATE_LINEAR_LAUNCH_AS(KK, 1, 1, 8);                                                               \
+            else FMOE_GATE_LINEAR_LAUNCH_AS(KK, 1, 2, 4);                                                                   \
+        } else if (E <= 32) {                                                                                               \
+            if (few) FMOE_GATE_LINEAR_LAUNCH_AS(KK, 2, 1, 8);                                                               \
+            else FMOE_GATE_LINEAR_LAUNCH_AS(KK, 2, 2, 4);                                                                   \
+        } else {                                                                                                            \
+            if (few) FMOE_GATE_LINEAR_LAUNCH_AS(KK, 4, 1, 8);                                                               \
+            else FMOE_GATE_LINEAR_LAUNCH_AS(KK, 4, 2, 4);                                                                   \
+        }                                                                                                                   \
     } while (0)
     switch (top_k) {
         case 1: FMOE_GATE_LINEAR_LAUNCH(1); break;
@@ -1455,6 +1468,7 @@ int launch_gate_linear(const void *x, const void *w, const void *bias, int64_t n
         default: return fail(FMOE_ELIMIT, "gate linear top-k: top_k=%d is not 1, 2, 4 or 8", top_k);
     }
 #undef FMOE_GATE_LINEAR_LAUNCH
+#undef FMOE_GATE_LINEAR_LAUNCH_AS
     FMOE_LAUNCH_CHECK();
     return FMOE_OK;
 }

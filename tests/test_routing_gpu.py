@@ -316,6 +316,9 @@ def test_gate_topk_with_masked_out_logits(device):
     (1000, 72, 5, 4, True),        # experts not a multiple of 16, tokens not a multiple of a workgroup's share,
                                    # contraction not a multiple of a wave's step
     (33, 8, 2, 2, True),
+    (16, 2048, 64, 8, False),      # one workgroup of 16 tokens, and one token into the second
+    (17, 1032, 33, 4, True),
+    (4097, 136, 17, 2, True),      # past the sizes that take 16 tokens to a workgroup
     (100, 264, 64, 8, True),
     (0, 64, 4, 2, True),
 ])
