@@ -304,26 +304,33 @@ __device__ __forceinline__ int32_t wave_prefix(int32_t v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast 31 into rows 2 and 3
     return v;
 }
-__global__ __launch_bounds__(kSmallBlock) void route_few_experts_kernel(
-    const int64_t *__restrict__ gate, int n_slots, int n_expert, int nbits, int64_t *__restrict__ expert_count,
-    int64_t *__restrict__ pos, int64_t *__restrict__ slot_to_row, int32_t *__restrict__ table) {
-    __shared__ int32_t bins[kSmallWaves][kFewExperts], next_row[kSmallWaves][kFewExperts];
+struct RouteOut {   // results of a routing; slot_to_row and table may be null
+    int64_t *expert_count, *pos, *slot_to_row;
+    int32_t *table;
+};
+// gate_of(i): slot i's expert; bins, next_row: [kWaves or more][kFewExperts] of LDS each.  The workgroup has at most kWaves waves, and at
+// least n_slots / (64 kSteps) and two.
+template <int kWaves, int kSteps, typename GateOf>
+__device__ __forceinline__ void route_few_experts(const GateOf &gate_of, int n_slots, int n_expert, int nbits, const RouteOut &out,
+                                                  int32_t (*bins)[kFewExperts], int32_t (*next_row)[kFewExperts]) {
+    int64_t *const expert_count = out.expert_count, *const pos = out.pos, *const slot_to_row = out.slot_to_row;
+    int32_t *const table = out.table;
     const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave), waves = (int)blockDim.x / kWave;
-    const int steps = (n_slots + (int)blockDim.x - 1) / (int)blockDim.x;   // kStepsPerWave at most
+    const int steps = (n_slots + (int)blockDim.x - 1) / (int)blockDim.x;   // kSteps at most
     const int wave_base = wave * steps * kWave;
-    int keys[kStepsPerWave];
+    int keys[kSteps];
 #pragma unroll
-    for (int s = 0; s < kStepsPerWave; ++s) {
+    for (int s = 0; s < kSteps; ++s) {
         const int i = wave_base + s * kWave + lane;
         int64_t g = -1;
-        if (s < steps && i < n_slots) g = gate[i];
+        if (s < steps && i < n_slots) g = gate_of(i);
         keys[s] = (g >= 0 && g < n_expert) ? (int)g : -1;
     }
     bins[wave][lane] = 0;
     wave_lds_sync();
-    uint64_t peers[kStepsPerWave];
+    uint64_t peers[kSteps];
 #pragma unroll
-    for (int s = 0; s < kStepsPerWave; ++s) {
+    for (int s = 0; s < kSteps; ++s) {
         peers[s] = 0;
         if (s < steps) {
             peers[s] = match_mask(keys[s], keys[s] >= 0, nbits);
@@ -335,7 +342,7 @@ __global__ __launch_bounds__(kSmallBlock) void route_few_experts_kernel(
     const int e = lane;
     int32_t before = 0, rows = 0;
 #pragma unroll
-    for (int w = 0; w < kSmallWaves; ++w) {
+    for (int w = 0; w < kWaves; ++w) {
         const int32_t c = w < waves ? bins[w][e] : 0;
         before += w < wave ? c : 0;
         rows += c;
@@ -346,7 +353,7 @@ __global__ __launch_bounds__(kSmallBlock) void route_few_experts_kernel(
     mine[e] = hi - 1 - before;
     wave_lds_sync();
 #pragma unroll
-    for (int s = 0; s < kStepsPerWave; ++s) {
+    for (int s = 0; s < kSteps; ++s) {
         if (s >= steps) break;
         const int i = wave_base + s * kWave + lane;
         const bool valid = keys[s] >= 0;
@@ -398,6 +405,12 @@ __global__ __launch_bounds__(kSmallBlock) void route_few_experts_kernel(
         int4 *map = (int4 *)(table + (k == 0 ? map256 : map128)) + first[k];
         for (int j = wave; j < tiles[k]; j += waves) map[j] = make_int4(e, lo + j * tile_rows, min(rows - j * tile_rows, tile_rows), 0);
     }
+}
+
+__global__ __launch_bounds__(kSmallBlock) void route_few_experts_kernel(const int64_t *__restrict__ gate, int n_slots, int n_expert, int nbits,
+                                                                       RouteOut out) {
+    __shared__ int32_t bins[kSmallWaves][kFewExperts], next_row[kSmallWaves][kFewExperts];
+    route_few_experts<kSmallWaves, kStepsPerWave>([&](int i) { return gate[i]; }, n_slots, n_expert, nbits, out, bins, next_row);
 }
 
 // ---------------------------------------------------------------- apply ----
@@ -638,10 +651,11 @@ __global__ __launch_bounds__(kBlock) void gate_topk_kernel(
 constexpr int kGateMaxExpert = 64;
 constexpr int gate_stride(int tokens) { return tokens + 4; }
 
-template <typename T, int K, int kEB, int kTB, int kGateWaves>   // 16-expert blocks there are accumulators for, 16-token blocks, waves
+// kEB: 16-expert blocks there are accumulators for; kTB: 16-token blocks; kRoute: one workgroup, which also routes (`route`)
+template <typename T, int K, int kEB, int kTB, int kGateWaves, bool kRoute>
 __global__ __launch_bounds__(kGateWaves * kWave) void gate_linear_topk_kernel(
     const T *__restrict__ x, const T *__restrict__ w, const T *__restrict__ bias, int64_t n_tokens, int d,
-    int n_expert, int score_mode, int64_t *__restrict__ topk_idx, T *__restrict__ topk_score) {
+    int n_expert, int score_mode, int64_t *__restrict__ topk_idx, T *__restrict__ topk_score, RouteOut route, int nbits) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
     typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -776,6 +790,23 @@ __global__ __launch_bounds__(kGateWaves * kWave) void gate_linear_topk_kernel(
     topk_merge<T, K, kSub>(keys, best, chosen);
     topk_scores<K>(best, chosen, score_mode, score);
     if (token < n_tokens) topk_store<T, K>(sub, token, chosen, score, topk_idx, topk_score);
+    // Where this workgroup has all the tokens it routes them too: a launch less, which on a decoding step takes longer than its work.
+    // One token, 32 experts of 1024: 4.4 and 4.0 us of two kernels, 7.1 of one; the step 39.8 and 37.7.
+    if constexpr (kRoute) {
+        constexpr int kSlots = kGateTokens * K;
+        static_assert(kSlots <= kGateWaves * kWave, "a slot per thread");
+        static_assert(kSlots + 2 * kGateWaves * kFewExperts <= kGateWaves * 16 * kGateStride, "fits where one expert block's logits were");
+        __syncthreads();   // the logits have been read
+        int32_t *slot_expert = (int32_t *)part_lds;
+        int32_t(*tables)[kFewExperts] = (int32_t(*)[kFewExperts])(slot_expert + kSlots);
+        int mine = chosen[0];
+#pragma unroll
+        for (int j = 1; j < K; ++j) mine = sub == j ? chosen[j] : mine;
+        if (sub < K) slot_expert[t * K + sub] = mine;
+        __syncthreads();
+        route_few_experts<kGateWaves, 1>([&](int i) { return (int64_t)slot_expert[i]; }, (int)n_tokens * K, n_expert, nbits, route, tables,
+                                         tables + kGateWaves);
+    }
 }
 
 // ----------------------------------------------------------- noisy gate ----
@@ -1183,7 +1214,8 @@ int route_launch(const int64_t *gate, int64_t n_slots, int64_t n_expert, int64_t
     if (n_slots <= kSmallSlots && E <= kFewExperts) {
         // a wave per 64 slots, up to 16; at least four, which share the writing of the table
         const int waves = std::min(kSmallWaves, std::max(4, (int)ceil_div(n_slots, kWave)));
-        route_few_experts_kernel<<<1, waves * kWave, 0, st>>>(gate, (int)n_slots, E, ilog2_ceil(n_expert), expert_count, pos, slot_to_row, table);
+        route_few_experts_kernel<<<1, waves * kWave, 0, st>>>(gate, (int)n_slots, E, ilog2_ceil(n_expert),
+                                                             RouteOut{expert_count, pos, slot_to_row, table});
         FMOE_LAUNCH_CHECK();
         return FMOE_OK;
     }
@@ -1434,30 +1466,35 @@ namespace {
 
 template <typename T>
 int launch_gate_linear(const void *x, const void *w, const void *bias, int64_t n_tokens, int d, int E, int top_k,
-                       int score_mode, int64_t *topk_idx, void *topk_score, hipStream_t st) {
+                       int score_mode, int64_t *topk_idx, void *topk_score, const RouteOut &route, bool *routed, hipStream_t st) {
     // Up to 16 tokens per compute unit: 16 tokens to a workgroup of eight waves, which is half the chain of load latencies; with more,
     // 32 to one of four, which reads w half as often.  us with 32 and four / 16 and eight: one token, 32 experts of 1024: 5.4 / 4.4; 509, 64
     // of 2048: 21.4 / 16.7; 1000, 16 of 768: 7.4 / 5.7; 4096, 8 of 512, float32: 6.6 / 5.3.
     constexpr int64_t kFewTokens = 16 * 256;
     const bool few = n_tokens <= kFewTokens;
+    *routed = n_tokens <= 16;   // (one workgroup)
+    const int nbits = ilog2_ceil(E);
     const int tokens = few ? 16 : 32, waves = few ? 8 : 4;
     const unsigned grid = (unsigned)ceil_div(n_tokens, tokens);
     const size_t lds = (size_t)waves * ((E + 15) / 16 * 16) * gate_stride(tokens) * sizeof(float);
     // (accumulators for 1, 2 or 4 blocks of 16 experts: fewer registers, more waves per compute unit)
-#define FMOE_GATE_LINEAR_LAUNCH_AS(KK, EB, TB, WAVES)                                                                       \
-    gate_linear_topk_kernel<T, KK, EB, TB, WAVES><<<grid, WAVES * kWave, lds, st>>>((const T *)x, (const T *)w, (const T *)bias, \
-                                                                                  n_tokens, d, E, score_mode, topk_idx, (T *)topk_score)
+#define FMOE_GATE_LINEAR_LAUNCH_AS(KK, EB, TB, WAVES, ROUTE)                                                                       \
+    gate_linear_topk_kernel<T, KK, EB, TB, WAVES, ROUTE><<<grid, WAVES * kWave, lds, st>>>((const T *)x, (const T *)w, (const T *)bias, \
+                                                                                  n_tokens, d, E, score_mode, topk_idx, (T *)topk_score, route, nbits)
 #define FMOE_GATE_LINEAR_LAUNCH(KK)                                                                                         \
     do {                                                                                                                    \
         if (E <= 16) {                                                                                                      \
-            if (few) FMOE_GATE_LINEAR_LAUNCH_AS(KK, 1, 1, 8);                                                               \
-            else FMOE_GATE_LINEAR_LAUNCH_AS(KK, 1, 2, 4);                                                                   \
+            if (*routed) FMOE_GATE_LINEAR_LAUNCH_AS(KK, 1, 1, 8, true);                                      \
+            else if (few) FMOE_GATE_LINEAR_LAUNCH_AS(KK, 1, 1, 8, false);                                                               \
+            else FMOE_GATE_LINEAR_LAUNCH_AS(KK, 1, 2, 4, false);                                                                   \
         } else if (E <= 32) {                                                                                               \
-            if (few) FMOE_GATE_LINEAR_LAUNCH_AS(KK, 2, 1, 8);                                                               \
-            else FMOE_GATE_LINEAR_LAUNCH_AS(KK, 2, 2, 4);                                                                   \
+            if (*routed) FMOE_GATE_LINEAR_LAUNCH_AS(KK, 2, 1, 8, true);                                      \
+            else if (few) FMOE_GATE_LINEAR_LAUNCH_AS(KK, 2, 1, 8, false);                                                               \
+            else FMOE_GATE_LINEAR_LAUNCH_AS(KK, 2, 2, 4, false);                                                                   \
         } else {                                                                                                            \
-            if (few) FMOE_GATE_LINEAR_LAUNCH_AS(KK, 4, 1, 8);                                                               \
-            else FMOE_GATE_LINEAR_LAUNCH_AS(KK, 4, 2, 4);                                                                   \
+            if (*routed) FMOE_GATE_LINEAR_LAUNCH_AS(KK, 4, 1, 8, true);                                      \
+            else if (few) FMOE_GATE_LINEAR_LAUNCH_AS(KK, 4, 1, 8, false);                                                               \
+            else FMOE_GATE_LINEAR_LAUNCH_AS(KK, 4, 2, 4, false);                                                                   \
         }                                                                                                                   \
     } while (0)
     switch (top_k) {
@@ -1520,13 +1557,15 @@ extern "C" int fmoe_gate_linear_topk_route_table(const void *x, const void *w, c
     FMOE_REQUIRE(aligned16(x) && aligned16(w), "fmoe_gate_linear_topk_route: x and w must be 16-byte aligned");
     RouteScratch s;
     if (int rc = carve(workspace, workspace_bytes, n_slots, n_expert, &s)) return rc;
+    const RouteOut route{expert_count, pos, slot_to_row, (int32_t *)segment_table};
+    bool routed = false;
     int rc = FMOE_OK;
     switch (dtype) {
-        case FMOE_F32: rc = launch_gate_linear<float>(x, w, bias, n_tokens, (int)d_model, (int)n_expert, (int)top_k, score_mode, topk_idx, topk_score, st); break;
-        case FMOE_BF16: rc = launch_gate_linear<__bf16>(x, w, bias, n_tokens, (int)d_model, (int)n_expert, (int)top_k, score_mode, topk_idx, topk_score, st); break;
-        default: rc = launch_gate_linear<_Float16>(x, w, bias, n_tokens, (int)d_model, (int)n_expert, (int)top_k, score_mode, topk_idx, topk_score, st); break;
+        case FMOE_F32: rc = launch_gate_linear<float>(x, w, bias, n_tokens, (int)d_model, (int)n_expert, (int)top_k, score_mode, topk_idx, topk_score, route, &routed, st); break;
+        case FMOE_BF16: rc = launch_gate_linear<__bf16>(x, w, bias, n_tokens, (int)d_model, (int)n_expert, (int)top_k, score_mode, topk_idx, topk_score, route, &routed, st); break;
+        default: rc = launch_gate_linear<_Float16>(x, w, bias, n_tokens, (int)d_model, (int)n_expert, (int)top_k, score_mode, topk_idx, topk_score, route, &routed, st); break;
     }
-    if (rc) return rc;
+    if (rc || routed) return rc;
     return route_launch(topk_idx, n_slots, n_expert, expert_count, pos, slot_to_row, (int32_t *)segment_table, s, st);
 }
 

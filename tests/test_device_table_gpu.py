@@ -101,6 +101,27 @@ def test_table_of_the_routing_against_the_one_of_its_counts(n_slots, n_expert, s
         assert np.array_equal(_unpack(table, n_expert)[key], _unpack(torch.from_numpy(want), n_expert)[key]), key
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n_tokens", [1, 7, 15, 16, 17])
+@pytest.mark.parametrize("n_expert,top_k", [(1, 1), (8, 8), (33, 2), (64, 4), (64, 8)])
+def test_gate_that_routes_its_own_tokens(n_tokens, n_expert, top_k, dtype, device):
+    """A gate with one workgroup's tokens routes them in the same launch: routing and table of its choices, word for word those
+    of the routing kernels."""
+    g = torch.Generator().manual_seed(n_tokens * 65 + n_expert)
+    x, w = torch.randn(n_tokens, 264, generator=g).to(dtype), torch.randn(n_expert, 264, generator=g).to(dtype)
+    idx, _score, *got = fmoe_native.gate_linear_topk_route(x.to(device), w.to(device), None, top_k, 0, with_table=True)
+    ref_pos, ref_cnt = orouting.count_by_gate(idx.cpu().numpy(), n_expert)
+    assert np.array_equal(got[0].cpu().numpy(), ref_cnt) and np.array_equal(got[1].cpu().numpy(), ref_pos)
+    want = fmoe_native.route_table(idx, n_expert)
+    assert all(torch.equal(a, b) for a, b in zip(got[:3], want[:3]))
+    got, want = got[3].cpu().numpy(), want[3].cpu().numpy()
+    assert got.size == want.size
+    head = HEADER + 3 * (n_expert + 1)
+    assert np.array_equal(got[:head], want[:head]) and np.array_equal(got[-4 * n_expert:], want[-4 * n_expert:])
+    for key in ("tiles256", "tiles128"):
+        assert np.array_equal(_unpack(torch.from_numpy(got), n_expert)[key], _unpack(torch.from_numpy(want), n_expert)[key]), key
+
+
 @pytest.mark.parametrize("name", sorted(CONFIG_COUNTS))
 def test_segment_table_at_the_configurations(name, device):
     g = torch.Generator().manual_seed(11)
