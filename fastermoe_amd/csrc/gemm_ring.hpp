@@ -913,8 +913,10 @@ __global__ __launch_bounds__(64) void ring_combine_kernel(const RingParams prm) 
         f32x4 v[kBatch][8];
 #pragma unroll
         for (int b = 0; b < kBatch; ++b) {
-            const int j = j0 + b <= last ? j0 + b : last;
-            const f32x4 *src = (const f32x4 *)prm.split_ws + (int64_t)ring_ws_slot(xcd, per, j, tail_tile) * (kRingTile * kRingTile / 4) +
+            // (the same for the workgroup; with the last part read again in a missing one's place the launch took 21.4 us instead of
+            // 14.8 on 64 tail tiles of 4 columns of tiles, K = 4096)
+            if (j0 + b > last) continue;
+            const f32x4 *src = (const f32x4 *)prm.split_ws + (int64_t)ring_ws_slot(xcd, per, j0 + b, tail_tile) * (kRingTile * kRingTile / 4) +
                                wave * 64 + threadIdx.x;
 #pragma unroll
             for (int x = 0; x < 8; ++x) v[b][x] = __builtin_nontemporal_load(src + (x * 4 + y) * kRingThreads);
