@@ -9,6 +9,7 @@
 // second linear writes them, and in the backward one block of rows is in turn the gradient of the experts' output, the
 // experts' input gradient and the sorted input.
 #include "grouped_gemm.hpp"
+#include "permute.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -122,6 +123,13 @@ bool apart(int gate) {
            (gate != FMOE_GATE_ROUTED && switched_off("FMOE_GATE_LINEAR_FUSED"));
 }
 
+// The sorted copy of the token rows.  Rows past the routed ones are left alone: the products read the segments of the table only.
+int sort_rows(const Sizes &s, const void *x, const int64_t *pos, const int64_t *slot_to_row, void *rows, hipStream_t st) {
+    if (s.top_k > 1 && s.d_model * s.eb % 16 == 0 && aligned16(x) && aligned16(rows))
+        return permute_spread_rows(x, slot_to_row, s.top_k, rows, s.n_tokens, s.n_slots, s.d_model, s.dtype, st);
+    return permute_gather_rows(x, pos, s.top_k, rows, s.n_slots, s.n_tokens, s.d_model, s.dtype, st);
+}
+
 // one expert linear over the sorted rows of a segment table
 int linear_forward(const Sizes &s, const void *x, const int64_t *row_index, const void *w, const void *b, void *pre, void *y,
                    const void *table, int64_t in_feat, int64_t out_feat, int activation, void *ws, int64_t ws_bytes, hipStream_t st) {
@@ -214,7 +222,7 @@ extern "C" int fmoe_layer_forward(const void *x, const void *gate_w, const void 
     if (rc != FMOE_OK) return rc;
     const bool token_rows = reads_token_rows(s, keep_pre);
     if (!token_rows) {
-        rc = fmoe_gather_rows_div(x, pos, top_k, rows, s.n_slots, n_tokens, d_model, dtype, stream);
+        rc = sort_rows(s, x, pos, slot_to_row, rows, (hipStream_t)stream);
         if (rc != FMOE_OK) return rc;
     }
     hipStream_t st = (hipStream_t)stream;
@@ -268,7 +276,7 @@ extern "C" int fmoe_layer_backward(const void *grad_out, const void *x, const vo
         if (rc != FMOE_OK) return rc;
     }
     if (grad_w1 != nullptr) {
-        rc = fmoe_gather_rows_div(x, pos, top_k, b.rows, s.n_slots, n_tokens, d_model, dtype, stream);
+        rc = sort_rows(s, x, pos, slot_to_row, b.rows, st);
         if (rc != FMOE_OK) return rc;
         rc = linear_wgrad(s, b.grad_pre, b.rows, grad_w1, grad_b1, segment_table, d_model, d_hidden, st);
         if (rc != FMOE_OK) return rc;

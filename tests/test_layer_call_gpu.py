@@ -114,9 +114,10 @@ def test_feature_sizes_off_the_grid(dtype, n, d, h, e, k, device, monkeypatch):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("fuse", [False, True])
-@pytest.mark.parametrize("n,d,h,e,k", [(513, 128, 256, 8, 2), (8192, 512, 2048, 16, 4)])
+@pytest.mark.parametrize("n,d,h,e,k", [(513, 128, 256, 8, 2), (8192, 512, 2048, 16, 4), (203, 1544, 64, 12, 9), (65, 1032, 1304, 32, 17)])
 def test_gate_outside_the_call(n, d, h, e, k, fuse, device, monkeypatch):
     """A gate that drops slots (none of expert rows may be read for them), and a hook on a plain one."""
+    torch.full((64 << 20,), float("nan"), dtype=torch.bfloat16, device=device)   # (the rows past the routed ones are whatever was there)
     x = torch.randn(n, d, device=device).to(torch.bfloat16).requires_grad_(True)
     grad = torch.randn(n, d, device=device).to(torch.bfloat16)
     moe = build(device, torch.bfloat16, d, h, e, k, gate=DroppingGate, fuse=fuse)
