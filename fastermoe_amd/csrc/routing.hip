@@ -169,7 +169,7 @@ __global__ __launch_bounds__(kRouteScanBlock) void route_scan_kernel(
     __shared__ segtab::SmallLds table_lds;
     if (threadIdx.x == 0) carry_s = 0;
     __syncthreads();
-    int32_t run = 0;
+    int32_t run = 0, upto = 0;   // this thread's expert's count and the prefix with it, of the last round
     for (int e0 = 0; e0 < n_expert; e0 += kRouteScanBlock) {
         const int e = e0 + threadIdx.x;
         run = 0;
@@ -188,30 +188,25 @@ __global__ __launch_bounds__(kRouteScanBlock) void route_scan_kernel(
             expert_count[e] = run;
         }
         // inclusive scan of `run` over the workgroup
-        int32_t v = run;
-#pragma unroll
-        for (int off = 1; off < kWave; off <<= 1) {
-            const int32_t up = __shfl_up(v, off, kWave);
-            if (lane_id() >= off) v += up;
-        }
+        const int32_t v = segtab::wave_prefix(run);
         const int wave = threadIdx.x / kWave;
         if (lane_id() == kWave - 1) wave_sum[wave] = v;
         __syncthreads();
-        int32_t before = carry_s;
-        for (int w = 0; w < wave; ++w) before += wave_sum[w];
-        if (e < n_expert) cum_incl[e] = v + before;
+        upto = v + carry_s + segtab::sums_before(wave_sum, wave);
+        if (e < n_expert) cum_incl[e] = upto;
         __syncthreads();
-        if (threadIdx.x == kRouteScanBlock - 1) carry_s = v + before;
+        if (threadIdx.x == kRouteScanBlock - 1) carry_s = upto;
         __syncthreads();
     }
-    if (table != nullptr) segtab::small_table(run, n_expert, rows_cap, table, table_lds);
+    if (table != nullptr) segtab::small_table<true>(run, n_expert, rows_cap, table, table_lds, upto);
 }
 
 // Few slots: histogram, scan, placement and segment table in one launch of one workgroup.  Wave w owns
 // the slots [w * 64 steps, (w + 1) * 64 steps) and keeps its keys and match masks in registers between
 // the passes; its table in LDS is a histogram first and the running ranks afterwards, as in
 // block_hist_kernel and rank_apply_kernel.  The four separate launches took 26 us for 64 slots, 34 us for
-// 509 and 25 us for 8192, nearly all of it launch and memory latency; this one takes 8, 10 and 13 us.
+// 509 and 25 us for 8192, nearly all of it launch and memory latency; this one took 8, 10 and 13 us.  512 slots of 256 experts:
+// 12.0 us with prefix sums by exchanges by address and walks over the other waves' sums, 9.0 with both in the vector pipe.
 // Up to kSmallSlots a wave has no more steps to walk than one of rank_apply_kernel's.
 constexpr int kSmallBlock = segtab::kThreads, kSmallWaves = kSmallBlock / kWave;
 constexpr int kSmallSlots = kSmallBlock * kStepsPerWave;   // 8192
@@ -258,15 +253,10 @@ __global__ __launch_bounds__(kSmallBlock) void route_small_kernel(
         }
         expert_count[e] = total;
     }
-    int32_t v = total;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const int32_t up = __shfl_up(v, off, kWave);
-        if (lane_id() >= off) v += up;
-    }
+    int32_t v = segtab::wave_prefix(total);
     if (lane_id() == kWave - 1) wave_sum[wave] = v;
     __syncthreads();
-    for (int w = 0; w < wave; ++w) v += wave_sum[w];
+    v += segtab::sums_before(wave_sum, wave);
     if (e < n_expert) cum[e] = v;
     __syncthreads();
     const int routed = cum[n_expert - 1];
@@ -285,25 +275,16 @@ __global__ __launch_bounds__(kSmallBlock) void route_small_kernel(
         if (slot_to_row && i < n_slots) slot_to_row[i] = row;
         if (i < n_slots && i >= routed) pos[i] = -1;
     }
-    if (table != nullptr) segtab::small_table(total, n_expert, n_slots, table, table_lds);
+    if (table != nullptr) segtab::small_table<true>(total, n_expert, n_slots, table, table_lds, v);
 }
 
 // The same for experts that one wave holds, one per lane: past the one barrier behind the histogram every wave has the counts, their
 // prefixes and its own first rows in registers, and writes its slots and its part of the table without waiting for another.
 // Bound by launch and latency: the barriers, exchanges by address and walks over other waves' sums of the kernel above were most of its
 // time.  The largest of 16 waves walks 8 steps, as there; few slots take fewer waves.
-// us of the kernel above and of this one, slots and experts: 2, 32: 8.2 / 4.0; 509, 64: 12.7 / 6.6; 2000, 16: 9.0 / 5.7; 8192, 8: 14.8 / 10.3.
+// us of the kernel above (with its prefix sums by exchanges) and of this one, slots and experts: 2, 32: 8.2 / 4.0; 509, 64: 12.7 / 6.6;
+// 2000, 16: 9.0 / 5.7; 8192, 8: 14.8 / 10.3.
 constexpr int kFewExperts = kWave;
-// Prefix sum (with the lane's own value) over the wave, all lanes taking part: within rows of 16 lanes, then over the rows
-__device__ __forceinline__ int32_t wave_prefix(int32_t v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);    // row_shr 1, 2, 4, 8
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast 15 into rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast 31 into rows 2 and 3
-    return v;
-}
 struct RouteOut {   // results of a routing; slot_to_row and table may be null
     int64_t *expert_count, *pos, *slot_to_row;
     int32_t *table;
@@ -347,7 +328,7 @@ __device__ __forceinline__ void route_few_experts(const GateOf &gate_of, int n_s
         before += w < wave ? c : 0;
         rows += c;
     }
-    const int32_t hi = wave_prefix(rows), lo = hi - rows;
+    const int32_t hi = segtab::wave_prefix(rows), lo = hi - rows;
     const int routed = __builtin_amdgcn_readlane(hi, kWave - 1);
     int32_t *mine = next_row[wave];   // (the other waves may still be reading this one's bins)
     mine[e] = hi - 1 - before;
@@ -370,7 +351,7 @@ __device__ __forceinline__ void route_few_experts(const GateOf &gate_of, int n_s
     if (table == nullptr) return;
     // (the rows of all experts are at most n_slots, the table's capacity: nothing to clamp; tiles of both sizes fit 16 bits each)
     const int32_t tiles[2] = {(rows + 255) / 256, (rows + 127) / 128};
-    const int32_t ends = wave_prefix(tiles[0] | tiles[1] << 16), all = __builtin_amdgcn_readlane(ends, kWave - 1);
+    const int32_t ends = segtab::wave_prefix(tiles[0] | tiles[1] << 16), all = __builtin_amdgcn_readlane(ends, kWave - 1);
     const int32_t first[2] = {(ends & 0xffff) - tiles[0], (ends >> 16) - tiles[1]};
     const int map256 = (int)segtab::map256_off(n_expert), map128 = (int)segtab::map128_off(n_slots, n_expert);
     if (wave == 0) {   // the experts by descending rows
@@ -1042,7 +1023,7 @@ __global__ __launch_bounds__(kSmallBlock) void limit_table_kernel(
         kept = min(count[e], (int64_t)cap);
         new_count[e] = kept;
     }
-    segtab::small_table(kept, n_expert, n_slots, table, lds);
+    segtab::small_table<false>(kept, n_expert, n_slots, table, lds);
     if (n_slots > kSmallSlots) return;
     // (lds.seg was written before the barriers inside)
     const int routed = lds.seg[n_expert];

@@ -18,7 +18,7 @@ constexpr int kTabBlock = segtab::kThreads;
 __global__ __launch_bounds__(kTabBlock) void small_table_kernel(const int64_t *__restrict__ counts, int n_expert,
                                                                 int rows_cap, int32_t *__restrict__ tab) {
     __shared__ segtab::SmallLds lds;
-    segtab::small_table((int)threadIdx.x < n_expert ? counts[threadIdx.x] : 0, n_expert, rows_cap, tab, lds);
+    segtab::small_table<false>((int)threadIdx.x < n_expert ? counts[threadIdx.x] : 0, n_expert, rows_cap, tab, lds);
 }
 
 // More experts: one workgroup.  Pass 1: per expert (in chunks of kTabBlock, carrying the running sums) the

@@ -72,59 +72,86 @@ template <typename Key> __device__ __forceinline__ int expert_in_order(int rows,
     return (1 << kBits) - 1 - (int)(sort_descending(mine, n, buf) & ((1 << kBits) - 1));
 }
 
+// Prefix sum (with the lane's own value) over the wave, all lanes taking part: within rows of 16 lanes, then over the rows
+__device__ __forceinline__ int32_t wave_prefix(int32_t v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);    // row_shr 1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast 15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast 31 into rows 2 and 3
+    return v;
+}
+// The sum of the first `wave` of at most 16 sums in LDS, all lanes taking part: read together and added by lanes, where a walk over them was a
+// chain of up to fifteen LDS latencies.
+__device__ __forceinline__ int32_t sums_before(const int32_t *sums, int wave) {
+    static_assert(kThreads / kWave <= 16, "a row of lanes holds the sums");
+    const int lane = threadIdx.x & (kWave - 1);
+    int32_t v = lane < wave ? sums[lane] : 0;
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);    // row_shr 1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    return __builtin_amdgcn_readlane(v, 15);
+}
+
 // The whole table for at most kSmallExperts experts by one workgroup of kThreads threads, thread e
 // holding expert e's row count (others: anything).  The counts are clamped so that their sum never
 // exceeds rows_cap.  The prefixes stay in LDS, where the row tiles find their expert by binary
 // search: read back from memory, the ten dependent loads of that search were most of the table's
-// 9.7 us at 8 experts.
-__device__ __forceinline__ void small_table(int64_t count, int n_expert, int rows_cap, int32_t *__restrict__ tab, SmallLds &lds) {
+// 9.7 us at 8 experts.  kExact: the counts are the caller's own, none is negative, their sum is at most rows_cap and `upto` is their
+// prefix sum with this thread's own.
+template <bool kExact>
+__device__ __forceinline__ void small_table(int64_t count, int n_expert, int rows_cap, int32_t *__restrict__ tab, SmallLds &lds,
+                                            int32_t upto = 0) {
     const int e = threadIdx.x, lane = e & (kWave - 1), wave = e / kWave;
-    int64_t c64 = e < n_expert ? count : 0;
-    c64 = c64 < 0 ? 0 : (c64 > rows_cap ? rows_cap : c64);
-    int64_t v = c64;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const int64_t up = __shfl_up(v, off, kWave);
-        if (lane >= off) v += up;
+    int32_t lo, hi;
+    if constexpr (kExact) {
+        hi = upto;
+        lo = e < n_expert ? upto - (int32_t)count : upto;
+    } else {
+        int64_t c64 = e < n_expert ? count : 0;
+        c64 = c64 < 0 ? 0 : (c64 > rows_cap ? rows_cap : c64);
+        int64_t v = c64;
+    #pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+            const int64_t up = __shfl_up(v, off, kWave);
+            if (lane >= off) v += up;
+        }
+        if (lane == kWave - 1) lds.row_sum[wave] = v;
+        __syncthreads();
+        for (int w = 0; w < wave; ++w) v += lds.row_sum[w];
+        const int64_t before = v - c64;
+        lo = (int32_t)(before > rows_cap ? rows_cap : before);
+        hi = (int32_t)(v > rows_cap ? rows_cap : v);
     }
-    if (lane == kWave - 1) lds.row_sum[wave] = v;
-    __syncthreads();
-    for (int w = 0; w < wave; ++w) v += lds.row_sum[w];
-    int64_t lo = v - c64;
-    lo = lo > rows_cap ? rows_cap : lo;
-    const int64_t hi = v > rows_cap ? rows_cap : v;
-    const int32_t rows = (int32_t)(hi - lo);
+    const int32_t rows = hi - lo;
     const int32_t t[2] = {(rows + 255) / 256, (rows + 127) / 128};
     int32_t tv[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-        int32_t s = t[k];
-#pragma unroll
-        for (int off = 1; off < kWave; off <<= 1) {
-            const int32_t up = __shfl_up(s, off, kWave);
-            if (lane >= off) s += up;
-        }
-        tv[k] = s;
-        if (lane == kWave - 1) lds.wave_sum[k][wave] = s;
+        tv[k] = wave_prefix(t[k]);
+        if (lane == kWave - 1) lds.wave_sum[k][wave] = tv[k];
     }
     const int live = __popcll(__ballot(rows > 0));
     if (lane == 0) lds.wave_live[wave] = live;
     __syncthreads();
-    for (int w = 0; w < wave; ++w) { tv[0] += lds.wave_sum[0][w]; tv[1] += lds.wave_sum[1][w]; }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) tv[k] += sums_before(lds.wave_sum[k], wave);
     int32_t *seg = tab + seg_off(), *pfx256 = tab + pfx256_off(n_expert), *pfx128 = tab + pfx128_off(n_expert);
     const int map256 = (int)map256_off(n_expert), map128 = (int)map128_off(rows_cap, n_expert);
     lds.rows[e] = e < n_expert ? rows : -1;
     if (e < n_expert) {
-        lds.seg[e] = seg[e] = (int32_t)lo;
+        lds.seg[e] = seg[e] = lo;
         lds.pfx[0][e] = pfx256[e] = tv[0] - t[0];
         lds.pfx[1][e] = pfx128[e] = tv[1] - t[1];
     }
     if (e == n_expert - 1) {
-        lds.seg[n_expert] = seg[n_expert] = (int32_t)hi;
+        lds.seg[n_expert] = seg[n_expert] = hi;
         lds.pfx[0][n_expert] = pfx256[n_expert] = tv[0];
         lds.pfx[1][n_expert] = pfx128[n_expert] = tv[1];
         tab[0] = n_expert;
-        tab[kRows] = (int32_t)hi;
+        tab[kRows] = hi;
         tab[kTiles256] = tv[0];
         tab[kTiles128] = tv[1];
         tab[kMap256] = map256;
@@ -174,7 +201,7 @@ __device__ __forceinline__ void small_table(int64_t count, int n_expert, int row
             place += (r.x > rows || (r.x == rows && f < e)) + (r.y > rows || (r.y == rows && f + 1 < e)) +
                      (r.z > rows || (r.z == rows && f + 2 < e)) + (r.w > rows || (r.w == rows && f + 3 < e));
         }
-        order[place] = make_int4(e, (int)lo, rows, 0);
+        order[place] = make_int4(e, lo, rows, 0);
     }
 }
 
