@@ -44,6 +44,9 @@ constexpr int kSlabBytes = 128;  // contraction bytes per row per slab
 enum Loaders { kLoadersCompute = 0, kLoadersAlone = 1, kLoadersShared = 2 };
 constexpr int ahead_of(int loaders) { return loaders == kLoadersAlone ? 2 : 0; }
 constexpr int extra_waves(int loaders) { return loaders == kLoadersCompute ? 0 : kLoadWaves; }
+// Two workgroups to a compute unit: at most 128 registers with waves that only load, 256 for fp32, whose two accumulators would otherwise
+// take up to 311 (nothing is spilled).
+constexpr int waves_per_simd(int loaders, int element, int bn) { return loaders == kLoadersShared ? 4 : element == 4 && bn == 128 ? 2 : 1; }
 constexpr int kGroupM = 4;       // row tiles that share a column tile consecutively (an XCD then runs 4 x 8 tiles at a time)
 
 enum Shape { kKC = 0, kMC = 1 };
@@ -87,17 +90,24 @@ template <> struct Elem<float> {
     }
 };
 
-// fp32 products on the bf16 matrix pipe.  A float is the exact sum of three bf16 numbers, each the rounding of what the ones before
-// it left (8 significant bits each, down to 2^-110; below that what is left out is at most 2^-134).  Of the nine products of two such
-// sums the three smallest, at most 2^-25 of the whole, are left out; the other six go into the fp32 accumulator, small ones first:
-// 6 x 32 cycles for 16 contraction elements of a 32 x 32 block, where the fp32 MFMA takes 8 x 64, and six roundings of the accumulator
-// instead of eight.  Distance from float64 beside the fp32 MFMA's (relative 2-norms, 15 sizes from 512 to 40000 rows): 0.83 to 0.87 of it for every
-// forward, data gradient and weight gradient, e.g. 2.4 / 2.9e-7 at K = 512, 3.5 / 4.1e-7 at 1024, 4.9 / 5.7e-7 at 2048.
-// What bounds it: the power limit for large launches (six bf16 products to one: 190 TFLOP/s are 1140 of bf16 ones), else loads into LDS
-// and tiles that do not fill the chip.  Forward / data gradient / weight gradient in us, before and now: 8192 rows, 8 experts of 2048 x 4096: 1095 / 1094 /
-// 1051 and 787 / 765 / 729; of 512 x 1024: 96 / 105 / 83 and 77 / 74 / 58; 1024 rows, 16 of 768 x 3072: 85 / 107 / 75 and 67 / 74 / 52.
+// fp32 products on the bf16 matrix pipe.  A float is the sum of three bf16 numbers, each the rounding of what the ones before
+// it left (8 significant bits each): exactly from 2^-110 up, to 2^-134 below.  Of the nine products of two such sums the three
+// smallest, at most 2^-25 of the whole, are left out; the other six take 6 x 32 cycles for 16 contraction elements of a 32 x 32
+// block, where the fp32 MFMA takes 8 x 64.  Only the largest goes into the accumulator; the five lesser ones have one of their own
+// (`low`), 2^-8 of its size, which is added at the end.  So 16 elements round the accumulator twice (the instruction adds up 8 at a time) and
+// the fp32 MFMA 16 times.
+// Distance from float64 in the fp32 MFMA's (2-norms of forward and both gradients on all three tiles, 4 to 16384 terms, contractions that no two
+// workgroups share; in brackets with all six products in one accumulator): normal operands 0.32 to 0.68 (0.46 to 0.93); of one sign 0.35 to 0.74
+// (0.50 to 0.82); ReLU's by normal ones 0.35 to 0.79 (0.61 to 1.22); GELU's by uniform ones 0.33 to 0.69 (0.44 to 0.93); normal ones times powers of two
+// from -20 to 20, on one side 0.49 to 0.84 (0.79 to 1.07) from 16 terms on and at most 1.15 (1.17) below, on both 0.74 to 0.97 (1.06 to 1.21) from 32 on
+// and at most 1.23 (1.24) below.  The signed mean of the error is at most 0.01 (0.06 to 0.4) of the distance on normal operands: what the
+// instruction cuts off lies on one side.
 // An infinity, a NaN or a number that rounds to a bf16 infinity makes the accumulator a NaN or an infinity: such tiles are computed again on the fp32 MFMA
 // (grouped_gemm_kernel).
+// What bounds it: the power limit for large launches (six bf16 products to one: 183 TFLOP/s are 1100 of bf16 ones), else loads into LDS
+// and tiles that do not fill the chip.  Forward / data gradient / weight gradient in us on the fp32 MFMA and here, repeated on the same operands: 8192
+// rows, 8 experts of 2048 x 4096: 1089 / 1058 / 1020 and 846 / 799 / 748; of
+// 512 x 1024: 96 / 90 / 78 and 79 / 84 / 55; 1024 rows, 16 of 768 x 3072: 82 / 115 / 74 and 65 / 70 / 48.  The second accumulator takes none of that.
 struct Raw8 {      // 8 contraction elements of one row: two 16-byte chunks
     u32x4 c[2];
 };
@@ -343,7 +353,7 @@ template <typename T> __device__ __forceinline__ int mc_swz(int k) {
 
 // ---- the kernel ---------------------------------------------------------------
 template <typename T, int BM, int BN, int PSHAPE, int QSHAPE, int RAGGED, int EPI, int LOADERS>
-__global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS == kLoadersShared ? 4 : 1) void grouped_gemm_kernel(const GemmParams prm) {
+__global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_per_simd(LOADERS, (int)sizeof(T), BN)) void grouped_gemm_kernel(const GemmParams prm) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
     constexpr int kWavesM = waves_m_of(BN), kWaves = kWavesM * kWavesN;
     constexpr int kThreads = threads_of(BN);         // those that compute
@@ -779,6 +789,7 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
         for (int y = 0; y < TJ; ++y)
 #pragma unroll
             for (int r = 0; r < kAccRegs; ++r) acc[x][y][r] = 0.f;
+    f32x16 low[kSplit ? TI : 1][kSplit ? TJ : 1] = {};   // the sum of the lesser products, see Split8
 
     // Main loop, one basic block per slab, software-pipelined by hand.  A slab is worked
     // through in four phases.  fp32 in 64 x 64 (one block column): in two, the first of which also does what is said of the
@@ -866,8 +877,9 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
     auto stage_frag = [&](int ph, int f, int stage) {
         if constexpr (kSplit) {
             const int x = phase_reads_q(ph) ? f - TJ : f;
-            if (x < 0) split_stage(stage, qf[phase_qbuf(ph)][f], q_parts[phase_qbuf(ph)][f]);
-            else split_stage(stage, pf[ph & 1][x], p_parts[ph & 1][x]);
+            Raw8 &left = x < 0 ? qf[phase_qbuf(ph)][f] : pf[ph & 1][x];
+            Split8 &parts = x < 0 ? q_parts[phase_qbuf(ph)][f] : p_parts[ph & 1][x];
+            split_stage(stage, left, parts);
         }
     };
     // Phase ph, one MFMA after the other, and between them the reads of phase `next` from sp and sq, this phase's loads (load(i): the
@@ -881,7 +893,8 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
                 constexpr int i = decltype(mfma)::value;
                 if constexpr (i < frags) { read_half(next, i, 0, sp, sq); read_half(next, i, 1, sp, sq); }
                 constexpr int block = i % (PF * TJ), x = block / TJ, y = block % TJ;
-                mma_part(i / (PF * TJ), acc[phase_x0(ph) + x][y], p_parts[ph & 1][x], q_parts[phase_qbuf(ph)][y]);
+                constexpr int product = i / (PF * TJ);
+                mma_part(product, (product == 5 ? acc : low)[phase_x0(ph) + x][y], p_parts[ph & 1][x], q_parts[phase_qbuf(ph)][y]);
                 load(i);
                 constexpr int from = i <= kSplitFrom ? 0 : ((i - kSplitFrom) * stages + kSpan - 1) / kSpan;
                 constexpr int to = i < kSplitFrom ? 0 : ((i + 1 - kSplitFrom) * stages + kSpan - 1) / kSpan;
@@ -1069,7 +1082,10 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), LOADERS
 #pragma unroll
                 for (int y = 0; y < TJ; ++y)
 #pragma unroll
-                    for (int r = 0; r < kAccRegs; ++r) none = fmaf(acc[x][y][r], 0.f, none);
+                    for (int r = 0; r < kAccRegs; ++r) {
+                        acc[x][y][r] += low[x][y][r];
+                        none = fmaf(acc[x][y][r], 0.f, none);
+                    }
             if (any_wave(none != 0.f)) {   // (0 x infinity and 0 x NaN are NaN)
 #pragma unroll
                 for (int x = 0; x < TI; ++x)

@@ -101,3 +101,29 @@ def test_few_and_many_rows_take_a_shape_by_themselves(device, monkeypatch):
             assert ((got.double() - ref).abs() <= (terms + 2) * 2.0 ** -24 * size).all()
         pre = fmoe_native.linear_forward_dev(x, w, None, table, sum(counts), _lib.ACT_GELU, True)[1]
         assert torch.equal(pre, fmoe_native.linear_forward_dev(x, w, None, table, sum(counts))[0])
+
+
+def of_kind(kind, rows, cols, g, device):
+    z = torch.randn(rows, cols, generator=g)
+    return {"normal": z, "relu": z.clamp(min=0), "one sign": z.abs()}[kind].to(device)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("left,right", [("normal", "normal"), ("relu", "normal"), ("one sign", "one sign")])
+def test_the_accumulator_is_rounded_by_one_product_only(left, right, tile, device, monkeypatch):
+    """The largest of the six products rounds the accumulator once per 8 elements: m = K / 8 roundings of 2^-24 / sqrt(3) of what has
+    been added up, sqrt(i / m) of the sum after i of them (less where all terms have one sign), come to 2^-24 sqrt(m / 6) of it.  With all six products in one
+    accumulator, and on the fp32 matrix instruction, it is more than that, and the roundings of the former lie to one side: 0.09 to 0.2 of the distance."""
+    monkeypatch.setenv("FMOE_GEMM_TILE", tile)
+    r, k, n = 256, 2048, 192
+    g = torch.Generator().manual_seed(17)
+    a, b = of_kind(left, r, k, g, device), of_kind(right, n, k, g, device)
+    ref = a.double() @ b.double().t()
+    rows, terms = (fmoe_native.segment_table(torch.tensor([c]).to(device), c) for c in (r, k))
+    for got in (fmoe_native.linear_forward_dev(a, b.view(1, n, k), None, rows, r)[0],
+                fmoe_native.linear_dgrad_dev(a, b.t().contiguous().view(1, k, n), rows, r),
+                fmoe_native.linear_wgrad_dev(a.t().contiguous(), b.t().contiguous(), torch.empty(1, r, n, device=device), terms, k, False)[0][0]):
+        err = got.double() - ref
+        assert err.norm() <= 2.0 ** -24 * (k / 8 / 6) ** 0.5 * ref.norm()
+        if right == "normal":
+            assert err.mean().abs() <= err.square().mean().sqrt() / 16
