@@ -102,12 +102,14 @@ template <> struct Elem<float> {
 // from -20 to 20, on one side 0.49 to 0.84 (0.79 to 1.07) from 16 terms on and at most 1.15 (1.17) below, on both 0.74 to 0.97 (1.06 to 1.21) from 32 on
 // and at most 1.23 (1.24) below.  The signed mean of the error is at most 0.01 (0.06 to 0.4) of the distance on normal operands: what the
 // instruction cuts off lies on one side.
-// An infinity, a NaN or a number that rounds to a bf16 infinity makes the accumulator a NaN or an infinity: such tiles are computed again on the fp32 MFMA
-// (grouped_gemm_kernel).
+// An infinity, a NaN or a number that rounds to a bf16 infinity makes the accumulator a NaN or an infinity, and a row or column whose elements are
+// all below 2^-95 would lose digits: such tiles are computed again on the fp32 MFMA (grouped_gemm_kernel).  Elements below 2^-110 beside
+// larger ones of their row lose what lies below 2^-134.
 // What bounds it: the power limit for large launches (six bf16 products to one: 183 TFLOP/s are 1100 of bf16 ones), else loads into LDS
 // and tiles that do not fill the chip.  Forward / data gradient / weight gradient in us on the fp32 MFMA and here, repeated on the same operands: 8192
-// rows, 8 experts of 2048 x 4096: 1089 / 1058 / 1020 and 846 / 799 / 748; of
-// 512 x 1024: 96 / 90 / 78 and 79 / 84 / 55; 1024 rows, 16 of 768 x 3072: 82 / 115 / 74 and 65 / 70 / 48.  The second accumulator takes none of that.
+// rows, 8 experts of 2048 x 4096: 1089 / 1058 / 1020 and 859 / 807 / 752; of
+// 512 x 1024: 96 / 90 / 78 and 79 / 84 / 56; 1024 rows, 16 of 768 x 3072: 82 / 115 / 74 and 66 / 71 / 48.  The second accumulator takes none of that, the
+// look-out for rows of tiny elements 1 %.
 struct Raw8 {      // 8 contraction elements of one row: two 16-byte chunks
     u32x4 c[2];
 };
@@ -120,6 +122,7 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 // floats, then what the parts so far leave of them: v - 1 x own half + 0 x the other, one v_dot2_f32_bf16 each.  (The pair
 // -1, 0 comes from a register: as an operand it turns into the inline constant -1.0, which is the pair 0, -1.)
 constexpr int kSplitStages = 5;
+constexpr uint32_t kTinyBits = 32u << 7;   // 2^-95 in bf16
 __device__ __forceinline__ void split_stage(int stage, Raw8 &left, Split8 &s) {
     uint32_t low = 0x0000bf80u;
     asm("" : "+s"(low));
@@ -790,6 +793,7 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
 #pragma unroll
             for (int r = 0; r < kAccRegs; ++r) acc[x][y][r] = 0.f;
     f32x16 low[kSplit ? TI : 1][kSplit ? TJ : 1] = {};   // the sum of the lesser products, see Split8
+    uint32_t p_seen[TI] = {}, q_seen[TJ] = {};           // the first parts of this lane's rows, or-ed
 
     // Main loop, one basic block per slab, software-pipelined by hand.  A slab is worked
     // through in four phases.  fp32 in 64 x 64 (one block column): in two, the first of which also does what is said of the
@@ -879,6 +883,11 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
             const int x = phase_reads_q(ph) ? f - TJ : f;
             Raw8 &left = x < 0 ? qf[phase_qbuf(ph)][f] : pf[ph & 1][x];
             Split8 &parts = x < 0 ? q_parts[phase_qbuf(ph)][f] : p_parts[ph & 1][x];
+            if (stage == kSplitStages - 1) {
+                uint32_t &seen = x < 0 ? q_seen[f] : p_seen[phase_x0(ph) + x];
+                seen |= parts.hi[0] | parts.hi[1];
+                seen |= parts.hi[2] | parts.hi[3];
+            }
             split_stage(stage, left, parts);
         }
     };
@@ -1074,7 +1083,8 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
         if (!fixup) run_loop(std::false_type{}, std::false_type{});
     }
     if constexpr (kSplit) {
-        // a tile with a NaN or an infinity once more, as the fp32 MFMA has it (the bias gradient's sums come from the elements themselves)
+        // a tile with a NaN, an infinity or a row of tiny elements once more, as the fp32 MFMA has it (the bias gradient's sums come from the
+        // elements themselves)
         if (!fixup) {
             float none = 0.f;
 #pragma unroll
@@ -1086,7 +1096,18 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
                         acc[x][y][r] += low[x][y][r];
                         none = fmaf(acc[x][y][r], 0.f, none);
                     }
-            if (any_wave(none != 0.f)) {   // (0 x infinity and 0 x NaN are NaN)
+            bool again = none != 0.f;   // (0 x infinity and 0 x NaN are NaN)
+            // the exponents are all below a power of two exactly where the or of them is
+            auto tiny = [&](uint32_t seen) {
+                seen |= (uint32_t)__shfl_xor((int)seen, MB, 64);   // (the row's other chunks)
+                seen = (seen | seen >> 16) & 0x7fffu;
+                return seen != 0 && seen < kTinyBits;
+            };
+#pragma unroll
+            for (int x = 0; x < TI; ++x) again |= tiny(p_seen[x]);
+#pragma unroll
+            for (int y = 0; y < TJ; ++y) again |= tiny(q_seen[y]);
+            if (any_wave(again)) {
 #pragma unroll
                 for (int x = 0; x < TI; ++x)
 #pragma unroll

@@ -127,3 +127,26 @@ def test_the_accumulator_is_rounded_by_one_product_only(left, right, tile, devic
         assert err.norm() <= 2.0 ** -24 * (k / 8 / 6) ** 0.5 * ref.norm()
         if right == "normal":
             assert err.mean().abs() <= err.square().mean().sqrt() / 16
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("power", [-96, -112, -120, -126])
+def test_rows_of_tiny_elements(power, tile, device, monkeypatch):
+    """Rows of either operand that are small throughout keep float32's digits (2^-24 sqrt(K) of the products' root of summed squares bounds the random walk
+    of K roundings); the other rows, and rows of zeros, are as without them."""
+    monkeypatch.setenv("FMOE_GEMM_TILE", tile)
+    counts, k, n = [130, 3, 70], 512, 136
+    x, w, gy, table = operands(counts, k, n, device, 23)
+    x[5] *= 2.0 ** power
+    x[:, 9] *= 2.0 ** power
+    x[132] = 0
+    w[2, 77] *= 2.0 ** power
+    gy[150:] *= 2.0 ** power
+    gy[:, 3] *= 2.0 ** power
+    want, _ = reference(x, w, gy, counts)
+    fwd, dgrad, wgrad = zip(products(x, w, gy, table)[:3], want[:3])
+    parts = {"row": [t[5] for t in fwd], "zeros": [t[132] for t in fwd], "weight": [t[133:, 77] for t in fwd], "gradient rows": [t[150:] for t in dgrad],
+             "input column": [t[..., 9] for t in wgrad], "gradient column": [t[:, 3] for t in wgrad], "all": fwd, "all d": dgrad, "all w": wgrad}
+    for name, (got, ref) in parts.items():
+        subnormal = 2.0 ** -149 * ref.numel() ** 0.5
+        assert (got.double() - ref).norm() <= 2.0 ** -24 * k ** 0.5 * ref.norm() + subnormal, name
