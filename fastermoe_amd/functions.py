@@ -7,6 +7,7 @@ outside this package and raises ``NotImplementedError``.
 """
 import torch
 from torch.autograd import Function
+from torch.utils._device import DeviceContext
 
 from . import fmoe_native
 
@@ -532,13 +533,30 @@ def layer_call(inp, gate_w, gate_b, score, w1, b1, w2, b2, routing, top_k, activ
                                      sizes, place)[0]
 
 
+def saving_is_watched():
+    r"""Whether saved-tensor hooks are in force where something may be saved: an offloader's, or an activation checkpoint's, which
+    compares what a forward and its second run save.  The second run may go without the hooks and modes of the first, so what is
+    saved must not depend on them then."""
+    return torch.is_grad_enabled() and torch._C._autograd._top_saved_tensors_default_hooks(True) is not None
+
+
+def _modes_watch():
+    """Whether a mode is in force that would have to see the operators: not one that only names the device of new tensors
+    (``with torch.device(...)``, ``torch.set_default_device``)."""
+    if torch._C._len_torch_dispatch_stack() != 0:
+        return True
+    return (torch._C._len_torch_function_stack() != 0
+            and any(type(mode) is not DeviceContext for mode in torch.overrides._get_current_function_mode_stack()))
+
+
 def nothing_watches(*tensors):
     r"""Whether a call on these tensors is seen by autograd's plain reverse mode at most: no transform (vmap, forward
-    mode), trace, compiler, mode or tensor subclass that would have to see the operators of the layer one by one."""
+    mode), trace, compiler, mode or tensor subclass that would have to see the operators of the layer one by one.  Modes count only
+    where :func:`saving_is_watched` is false."""
     return (all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors)
             and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
             and torch._C._get_tracing_state() is None and not torch.compiler.is_compiling()
-            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0)
+            and (not _modes_watch() or saving_is_watched()))
 
 
 class MOEGather(Function):

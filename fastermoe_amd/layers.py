@@ -9,7 +9,7 @@ import torch.nn as nn
 from . import fmoe_native
 from .functions import (AllGather, MaskRestore, MaskSelect, MOECache, MOECombine, MOEGather, MOEGatherCombine,
                         MOELinear, MOEScatter, Slice, _no_hooks, _PendingCounts, _plain_linear, _prepare_forward_ex,
-                        _route_launch, _single_worker, ensure_comm, mask_index)
+                        _route_launch, _single_worker, ensure_comm, mask_index, saving_is_watched)
 from .gates import NaiveGate
 
 
@@ -266,11 +266,13 @@ class FMoE(nn.Module):
 
     def _gate_inside(self, inp):
         r"""The whole layer as one call where its gate is a plain :class:`NaiveGate`, nothing between the steps is asked for
-        (a hook, a mask, another expert function) and the call takes the tensors; else ``None``."""
+        (a hook, a mask, another expert function) and the call takes the tensors; else ``None``.  Where saving is watched the gate is
+        called apart: hooks of modules may be there in one of two runs only, and the experts save the same either way."""
         gate, experts = self.gate, self.experts
         if (type(gate) is not NaiveGate or self.gate_hook is not None or self.mp_size > 1
                 or (self.mask is not None and self.mask_dict is not None) or not inp.is_cuda or inp.dim() != 2 or inp.shape[0] == 0
-                or gate.top_k != self.top_k or not self.experts_fused or not _own_expert_path(self.expert_fn, experts) or not _no_hooks(gate)):
+                or gate.top_k != self.top_k or not self.experts_fused or not _own_expert_path(self.expert_fn, experts) or not _no_hooks(gate)
+                or saving_is_watched()):
             return None
         linear = gate._modules.get("gate")
         if type(linear) is not nn.Linear or "weight" not in linear._parameters or "bias" not in linear._parameters:

@@ -1,10 +1,12 @@
 """The layer as one call (``MOELayer`` / ``fmoe_layer_forward`` / ``fmoe_layer_backward``) against the same layer step by
 step: the kernels are the same, so everything is equal bit by bit but the input's gradient, whose gate part is added before
 the one rounding instead of after two."""
+import contextlib
 import copy
 
 import pytest
 import torch
+import torch.utils.checkpoint
 
 import fastermoe_amd as fmoe
 from fastermoe_amd import _lib, fmoe_native, functions
@@ -190,6 +192,69 @@ def test_inference_takes_no_node_and_transforms_keep_theirs(e, device):
     moe.requires_grad_(False)
     out = moe(x)
     assert not out.requires_grad and torch.equal(out, want)
+
+
+class WatchingDispatch(torch.utils._python_dispatch.TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+@contextlib.contextmanager
+def module_hook():
+    handle = torch.nn.modules.module.register_module_forward_pre_hook(lambda module, args: None)
+    try:
+        yield
+    finally:
+        handle.remove()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("inside", ["forward", "backward"])
+@pytest.mark.parametrize("watcher", ["device", "function mode", "dispatch mode", "module hook"])
+def test_a_checkpointed_layer_saves_the_same_in_both_runs(watcher, inside, device):
+    """The second run of a checkpoint does not see the modes and hooks that were in force around the first, or sees others."""
+    make = {"device": lambda: torch.device("cuda"), "function mode": Watching, "dispatch mode": WatchingDispatch, "module hook": module_hook}[watcher]
+    n, d, h, e, k = 96, 64, 128, 8, 2
+    moe = build(device, torch.bfloat16, d, h, e, k)
+    x = torch.randn(n, d, device=device).to(torch.bfloat16).requires_grad_(True)
+    grad = torch.randn(n, d, device=device).to(torch.bfloat16)
+    _, want, wants = step(moe, x, grad, False)
+    moe.zero_grad(set_to_none=True)
+    with (make() if inside == "forward" else contextlib.nullcontext()):
+        out = torch.utils.checkpoint.checkpoint(moe, x, use_reentrant=False)
+    with (make() if inside == "backward" else contextlib.nullcontext()):
+        out.backward(grad)
+    for name, p in moe.named_parameters():
+        assert torch.equal(p.grad, wants[name]), name
+    assert (x.grad.double() - want.double()).abs().max() <= 2 * EPS[torch.bfloat16] * want.double().abs().max()   # (as in compare)
+
+
+@pytest.mark.gpu
+def test_a_default_device_keeps_the_one_call(device, monkeypatch):
+    moe = build(device, torch.bfloat16, 64, 128, 8, 2)
+    x = torch.randn(5, 64, device=device).to(torch.bfloat16).requires_grad_(True)
+    seen = []
+    real = functions.MOELayer.apply
+    monkeypatch.setattr(functions.MOELayer, "apply", lambda *a: (seen.append(len(a[8] or ())), real(*a))[1])
+    with torch.device(device):
+        moe(x)
+    assert seen == [0]   # (the gate inside)
+
+
+def test_what_watches():
+    t = torch.zeros(1)
+    hooks = lambda: torch.autograd.graph.saved_tensors_hooks(lambda v: v, lambda v: v)
+    assert functions.nothing_watches(t) and not functions.saving_is_watched()
+    with torch.device("cpu"):
+        assert functions.nothing_watches(t)
+        with Watching():
+            assert not functions.nothing_watches(t)
+            with hooks():
+                assert functions.nothing_watches(t) and functions.saving_is_watched()
+    with WatchingDispatch():
+        assert not functions.nothing_watches(t)
+    with hooks(), torch.no_grad():
+        assert not functions.saving_is_watched()
 
 
 def test_sizes_say_what_is_taken(monkeypatch):
