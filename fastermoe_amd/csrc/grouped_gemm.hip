@@ -395,13 +395,19 @@ bool use_ring(const TileShape &tile, int dtype) {
 // and 13.8 / 36.3 / 55.5; 8 of 4096 x 14336, 8 / 32 / 64 / 128: 142 / 191 / 191 / 192 and 99 / 161 / 180 / 243; 256 of
 // 1024 x 2048, 256 / 512 / 1024: 134 / 179 / 205 and 124 / 170 / 210; 64 of 8192 x 2048, 64 / 128 / 256: 298 / 367 / 372
 // and 249 / 334 / 389.
-// float32: at most 24 rows per expert on average, or 40 where the 128 x 128 tiles would number less than half the compute units.  us on the best
-// tiles and here: 8 experts of 2048 x 8192, 2 / 16 / 24 / 32 rows each: 166 / 197 / 196 / 203 and 96 / 154 / 185 / 225; 32 of 1024 x 1024,
-// 16 / 24 / 32: 50 / 49 / 49 and 46 / 48 / 60; 16 of 640 x 2560: 46 / 46 / 46 and 33 / 39 / 48; 4 of 768 x 3072, 2 / 32 / 40: 27 / 28 / 28 and 15 / 21 / 23.
-bool use_skinny(int64_t rows_cap, int64_t n_expert, int64_t out_feat, int dtype) {
+// float32: at most 24 rows per expert on average, 12 of contractions from 4096 on and 32 of shorter ones where the 128 x 128 tiles would number less
+// than half the compute units; as many as one pass takes in all (64) whatever the contraction.  The host does not know the counts, and an expert with more rows than a pass takes
+// walks its contraction again, so the lines are drawn where a skewed gate (shares 1 / rank^1.2) loses little.  us on the best tiles and
+// here with equal counts, then with skewed ones, weights from memory: 8 experts of 2048 -> 8192, 8 rows each: 205 / 125, 197 / 124; 24: 206 / 183, 206 / 194; 8 of
+// 8192 -> 2048, 12: 185 / 141, 183 / 175; 16: 186 / 153, 187 / 192; 24: 189 / 195, 188 / 305; 16 of 4096 -> 1024, 16: 101 / 79, 97 / 134; 24: 102 / 99, 101 / 144; 32 of 1024 -> 1024,
+// 8: 48 / 38, 47 / 45; 24: 50 / 52, 72 / 56; 64 of 1024 -> 4096, 16: 365 / 290, 356 / 309; 4 of 2048 -> 1024, 32: 37 / 20, 38 / 32; 40: 38 / 32, 38 / 54.  Where one expert
+// has all the rows the tiles are ahead: 64 of 1024 -> 4096, 256 rows: 25 / 42; 1024: 57 / 150.
+bool use_skinny(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype) {
     if ((!is_16bit(dtype) && dtype != FMOE_F32) || getenv("FMOE_GEMM_TILE")) return false;
-    if (dtype == FMOE_F32)
-        return rows_cap <= 24 * n_expert || (rows_cap <= 40 * n_expert && n_expert * ceil_div(out_feat, 128) * 2 < device_compute_units());
+    if (dtype == FMOE_F32) {
+        if (in_feat >= 4096 && rows_cap > 64) return rows_cap <= 12 * n_expert;
+        return rows_cap <= 24 * n_expert || (rows_cap <= 32 * n_expert && n_expert * ceil_div(out_feat, 128) * 2 < device_compute_units());
+    }
     return rows_cap <= 2 * n_expert || (rows_cap <= 8 * n_expert && n_expert * ceil_div(out_feat, 128) < 1024);
 }
 
@@ -414,7 +420,7 @@ struct DevRoute {
 DevRoute forward_route(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype, int epilogue,
                        int activation, bool keep_pre, bool gathers) {
     const TileShape tile = pick_rows_tile_estimate(rows_cap, n_expert, out_feat, in_feat, dtype);
-    if (use_skinny(rows_cap, n_expert, out_feat, dtype)) return {DevKernel::kSkinny, tile};
+    if (use_skinny(rows_cap, n_expert, in_feat, out_feat, dtype)) return {DevKernel::kSkinny, tile};
     // (what the persistent kernel is built for; the erf formula, "none" and ReLU with a saved pre-activation are rare)
     const bool ring_act = epilogue == kEpiStore || activation == FMOE_ACT_GELU || (activation == FMOE_ACT_RELU && !keep_pre);
     return {use_ring(tile, dtype) && !gathers && ring_act ? DevKernel::kRing : DevKernel::kTiles, tile};

@@ -350,6 +350,15 @@ def test_split_workspace_of_a_launch():
     assert lib.fmoe_linear_dev_workspace_bytes(1024, _lib.BF16) == 0
 
 
+def test_few_rows_in_float32_stay_on_tiles_where_a_skewed_gate_would_lose():
+    """The kernel for few rows asks for no workspace, tiles whose contraction can be shared do."""
+    lib = _lib.load()
+    ask = lambda rows, e, fin, fout: lib.fmoe_linear_forward_dev_workspace_bytes(rows, e, fin, fout, _lib.F32, _lib.ACT_NONE, 0, 0)
+    assert ask(96, 8, 8192, 2048) == 0 and ask(97, 8, 8192, 2048) > 0 and ask(64, 4, 8192, 2048) == 0 and ask(65, 4, 8192, 2048) > 0
+    assert ask(192, 16, 4096, 1024) == 0 and ask(193, 16, 4096, 1024) > 0
+    assert ask(192, 8, 2560, 8192) == 0 and ask(193, 8, 2560, 8192) > 0
+
+
 def test_sorted_rows_are_asked_for_by_the_activation_too(monkeypatch):
     """Where the first product reads sorted rows depends on what its kernel is built for: the polynomial GELU with and
     without its pre-activation and ReLU without, not the erf formula and not "none" with something to store."""

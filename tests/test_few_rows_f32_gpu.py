@@ -6,7 +6,8 @@ from fastermoe_amd import _lib, fmoe_native
 
 pytestmark = pytest.mark.gpu
 
-EDGES = [1, 0, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 130]   # blocks of 16 rows, passes of 64, a tile of 128 and the next
+# blocks of 16 rows, passes of 64, a tile of 128 and the next; experts without rows keep the average below the rule's line
+EDGES = [1, 0, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 130] + [0] * 9
 
 
 @pytest.mark.parametrize("k,n", [(4, 4), (16, 16), (20, 36), (68, 20), (256, 64), (1028, 132)])
@@ -17,7 +18,7 @@ def test_few_rows_in_float32(k, n, act, device):
     counts = torch.tensor(EDGES)
     e, rows = len(EDGES), sum(EDGES)
     slots = rows + 5
-    assert slots <= 40 * e   # (the rule's line)
+    assert slots <= 24 * e   # (the rule's line)
     g = torch.Generator().manual_seed(k + n)
     x = torch.randn(slots, k, generator=g).to(device)
     w = (torch.randn(e, n, k, generator=g) / k ** 0.5).to(device)
