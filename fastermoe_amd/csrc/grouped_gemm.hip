@@ -129,22 +129,24 @@ TileShape pick_tile(int64_t tiles_256) {
 
 // Row-ragged products in 16 bits with fewer than 512 tiles of 256 x 256: the shape with the least time by this estimate.  A round
 // of tiles that fills a share f of the chip's places takes start + slabs (alone + shared f) us, the accumulators' way out
-// included; the last round may be a partial one.  Below that the weights' way from memory is the bound.  The constants are fitted to
-// 204 products of 4 to 128 experts, 64 to 16384 rows and 512 to 8192 features, one fit per shape, a tenth of a launch's time
-// off on average; the shape that the estimate picks took 0.867 times what 128 x 128 tiles below 256 tiles of 256 x 256 and 128 x 256 from there on
-// did, the best of the five 0.84 times.  us for 64 x 128 / 128 x 128 alone / 128 x 128 shared / 128 x 256 / 256 x 256 (and 128 x 128 without
-// loading waves): 8 experts of 1024 x 4096, 1024 rows: 22 / 31 / 43 / - / - (51); 16 of 768 x 3072, 2000: 21 / 25 / 31 / 36 / 53 (37);
-// 8 of 2048 x 2048, 1600: 26 / 19 / 24 / 27 / 39 (28); 8 of 1024 x 1024, 4000: 23 / 21 / 18 / 17 / 25 (21); 12 of 2112 x 2112, 5000:
-// - / 69 / 62 / 59 / 47 (71); 8 of 2048 -> 1024, 8192: - / 50 / 50 / 54 / 42 (57); 64 of 2048 -> 8192, 509: 534 / 393 / 398 / 383 / 407 (378).
+// included; the last round may be a partial one.  The weights' way from memory comes on top, as far as the rounds do not hide it.  The constants are
+// fitted to 300 products of 4 to 128 experts, 90 to 14000 rows and 512 to 8192 features, a tenth of a launch's time off on average, with
+// weights that change from call to call, as in a model.  (Repeated on the same ones up to 256 MB of them stay in the memory-side cache, and low
+// tiles, which read them more often, look better than they are: constants fitted like that picked shapes that took 1.042 times what the best of the five
+// does on 120 other products, these 1.035, and 0.90 times what 128 x 128 tiles below 256 tiles of 256 x 256 and 128 x 256 from there on did.)  us for 64 x 128 /
+// 128 x 128 alone / 128 x 128 shared / 128 x 256 / 256 x 256 (and 128 x 128 without loading waves): 8 experts of 4096 -> 1024, 1024 rows: 33 / 37 / 38 /
+// 37 / 48 (37); 16 of 768 -> 3072, 2000: 49 / 43 / 40 / 41 / 29 (37); of 3072 -> 768: 42 / 38 / 40 / 52 / 65 (41); 8 of 2048 -> 2048, 1600: 38 / 26 / 29 / 34 /
+// 47 (30); 8 of 1024 -> 1024, 4000: 27 / 26 / 21 / 21 / 29 (24); 12 of 2112 -> 2112, 5000: 103 / 83 / 72 / 67 / 54 (77); 8 of 2048 -> 1024, 8192:
+// 65 / 58 / 58 / 58 / 48 (60); 64 of 2048 -> 8192, 509: 516 / 397 / 399 / 377 / 429 (377).
 struct RowShape {
     TileShape tile;
     int per_unit;                        // workgroups on a compute unit
-    double start, alone, shared, stream; // us, us per slab, TB/s
+    double start, alone, shared, stream; // us, us per slab, TB/s (of what the rounds do not hide)
 };
 constexpr RowShape kRowShapes[] = {
-    {{64, 128, kLoadersAlone}, 1, 2.9, 0.21, 0.13, 3.9},     {{128, 128, kLoadersAlone}, 1, 3.3, 0.26, 0.24, 4.8},
-    {{128, 128, kLoadersShared}, 2, 3.1, 0.30, 0.71, 4.9},   {{128, 256, kLoadersCompute}, 1, 4.2, 0.38, 0.53, 5.2},
-    {{256, 256, kLoadersCompute}, 1, 6.9, 0.57, 0.83, 5.0},
+    {{64, 128, kLoadersAlone}, 1, 3.2, 0.185, 0.14, 5.8},    {{128, 128, kLoadersAlone}, 1, 3.6, 0.31, 0.26, 30},
+    {{128, 128, kLoadersShared}, 2, 4.5, 0.25, 0.83, 17},    {{128, 256, kLoadersCompute}, 1, 4.4, 0.48, 0.45, 24},
+    {{256, 256, kLoadersCompute}, 1, 7.4, 0.81, 0.50, 40},
 };
 template <typename RowTiles> TileShape rows_16bit_tile(RowTiles row_tiles, double weight_bytes, int64_t n_cols, int64_t contraction) {
     const double slabs = (double)ceil_div(contraction, 64);
@@ -164,7 +166,7 @@ template <typename RowTiles> TileShape rows_16bit_tile(RowTiles row_tiles, doubl
         }
         // (a few large tiles cannot ask for the weights fast enough)
         const double share = s.tile.bn == 256 ? std::min(1.0, (double)tiles * 1.6 / (double)units) : 1.0;
-        us = std::max(us + 3, weight_bytes * 1e-6 / (s.stream * share) + 4);
+        us += weight_bytes * 1e-6 / (s.stream * share);
         if (pick.bm == 0 || us < best) { best = us; pick = s.tile; }
     }
     return pick;
