@@ -144,7 +144,7 @@ struct RowShape {
     double start, alone, shared, stream; // us, us per slab, TB/s (of what the rounds do not hide)
 };
 constexpr RowShape kRowShapes[] = {
-    {{64, 128, kLoadersAlone}, 1, 3.2, 0.185, 0.14, 5.8},    {{128, 128, kLoadersAlone}, 1, 3.6, 0.31, 0.26, 30},
+    {{64, 128, kLoadersAlone}, 1, 3.2, 0.18, 0.14, 6.2},     {{128, 128, kLoadersAlone}, 1, 3.4, 0.31, 0.26, 30},
     {{128, 128, kLoadersShared}, 2, 4.5, 0.25, 0.83, 17},    {{128, 256, kLoadersCompute}, 1, 4.4, 0.48, 0.45, 24},
     {{256, 256, kLoadersCompute}, 1, 7.4, 0.81, 0.50, 40},
 };
