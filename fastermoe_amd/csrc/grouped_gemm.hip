@@ -554,9 +554,10 @@ int device_table_launch(const char *who, GemmParams &prm, const int32_t *dev_tab
 int64_t linear_dev_workspace_bytes(int64_t contraction, int dtype) {
     const int eb = dtype_bytes(dtype);
     if (eb == 0 || dtype == FMOE_F64 || contraction < 1) return 0;
-    // the most that any launch of this contraction can use: 256 x 256 tiles, on the persistent kernel for 16-bit types
-    const DevRoute tiles{DevKernel::kTiles, {256, 256}}, ring{DevKernel::kRing, kManyTiles};
-    return std::max(route_workspace_bytes(tiles, contraction, dtype), eb == 2 ? route_workspace_bytes(ring, contraction, dtype) : 0);
+    // the most that any launch of this contraction can use: the largest tiles, for 16-bit types also on the persistent kernel
+    if (dtype == FMOE_F32) return route_workspace_bytes({DevKernel::kTiles, {128, 128}}, contraction, dtype);
+    return std::max(route_workspace_bytes({DevKernel::kTiles, {256, 256}}, contraction, dtype),
+                    route_workspace_bytes({DevKernel::kRing, kManyTiles}, contraction, dtype));
 }
 
 int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, int64_t n_expert, int64_t row_lo,

@@ -346,7 +346,8 @@ def test_split_workspace_of_a_launch():
     assert fwd(4096, 16, 1024, 1024, _lib.F32) == 0                              # 64 x 64 tiles
     assert fwd(65536, 8, 4100, 14336, _lib.BF16) == 0 and fwd(0, 8, 4096, 14336, _lib.BF16) == 0
     assert lib.fmoe_linear_dev_workspace_bytes(4096, _lib.BF16) == cus * 3 // 2 * tile(256, 256)
-    assert lib.fmoe_linear_dev_workspace_bytes(4096, _lib.F32) == cus * tile(256, 256)
+    assert lib.fmoe_linear_dev_workspace_bytes(4096, _lib.F32) == cus * tile(128, 128)   # (float32 has no larger tiles)
+    assert fwd(65536, 8, 4096, 4096, _lib.F32) == cus * tile(128, 128)
     assert lib.fmoe_linear_dev_workspace_bytes(1024, _lib.BF16) == 0
 
 
