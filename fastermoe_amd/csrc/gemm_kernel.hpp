@@ -1445,10 +1445,8 @@ __global__ __launch_bounds__(256) void split_reduce_dev_kernel(float *ws, const 
     }
 }
 
-// Host-side services of grouped_gemm.hip: compute units of the current device, and a per-stream
-// buffer for the partial accumulators of split tail tiles (allocated on first use, kept until
-// the process ends; NULL when the allocation fails, in which case nothing is split).
-int device_compute_units();
+// Host-side service of grouped_gemm.hip: a per-stream buffer for the partial accumulators of split tail tiles (allocated on
+// first use, kept until the process ends; NULL when the allocation fails, in which case nothing is split).
 float *split_workspace(hipStream_t stream, size_t bytes);
 
 template <typename T, int BM, int BN, int PS, int QS, int RG, int EPI, int LOADERS>

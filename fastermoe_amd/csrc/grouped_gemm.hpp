@@ -24,6 +24,10 @@ struct SegmentTable {
     int32_t tile[kMaxGroupExperts + 1];   // prefix of row tiles (ragged-M launches)
 };
 
+namespace gemm {
+int device_compute_units();   // of the current device; 256 where there is none
+}  // namespace gemm
+
 // Segment table in device memory, for launches that must not wait for the expert counts to
 // reach the host: built by segment_table_kernel from the routing's counts, read by the grouped
 // GEMM through scalar loads.  All entries are int32:

@@ -1451,8 +1451,7 @@ int launch_gate_linear(const void *x, const void *w, const void *bias, int64_t n
     // Up to 16 tokens per compute unit: 16 tokens to a workgroup of eight waves, which is half the chain of load latencies; with more,
     // 32 to one of four, which reads w half as often.  us with 32 and four / 16 and eight: one token, 32 experts of 1024: 5.4 / 4.4; 509, 64
     // of 2048: 21.4 / 16.7; 1000, 16 of 768: 7.4 / 5.7; 4096, 8 of 512, float32: 6.6 / 5.3.
-    constexpr int64_t kFewTokens = 16 * 256;
-    const bool few = n_tokens <= kFewTokens;
+    const bool few = n_tokens <= 16 * gemm::device_compute_units();
     *routed = n_tokens <= 16;   // (one workgroup)
     const int nbits = ilog2_ceil(E);
     const int tokens = few ? 16 : 32, waves = few ? 8 : 4;
