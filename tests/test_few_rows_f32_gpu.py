@@ -45,10 +45,19 @@ def test_few_rows_in_float32(k, n, act, device):
             lo += c
 
 
-def test_the_rows_past_the_counts_are_left_alone(device):
+@pytest.mark.parametrize("act", [_lib.ACT_NONE, _lib.ACT_GELU])
+def test_the_rows_past_the_counts_are_left_alone(act, device, monkeypatch):
+    """Outputs that begin as a value no product makes still hold it past the counts, bit for bit."""
     counts = torch.tensor([3, 0, 2], device=device)
     table = fmoe_native.segment_table(counts, 64)
     x, w = torch.randn(64, 32, device=device), torch.randn(3, 48, 32, device=device)
-    full, _ = fmoe_native.linear_forward_dev(x, w, None, table, 64)
+    marker = -1.25e33
+    real = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: real(*a, **k).fill_(marker) if k.get("dtype") == torch.float32 else real(*a, **k))
+    y, pre = fmoe_native.linear_forward_dev(x, w, None, table, 64, act, act != _lib.ACT_NONE)
     ref = torch.cat([x[:3].double() @ w[0].double().t(), x[3:5].double() @ w[2].double().t()])
+    full = y if pre is None else pre
     assert (full[:5].double() - ref).abs().max() <= 1e-5 * ref.abs().max()
+    for t in (y, pre):
+        if t is not None:
+            assert t.shape[0] == 64 and (t[:5] != marker).all() and (t[5:] == torch.tensor(marker, device=device)).all()

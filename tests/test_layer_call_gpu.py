@@ -116,10 +116,15 @@ def test_feature_sizes_off_the_grid(dtype, n, d, h, e, k, device, monkeypatch):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("fuse", [False, True])
-@pytest.mark.parametrize("n,d,h,e,k", [(513, 128, 256, 8, 2), (8192, 512, 2048, 16, 4), (203, 1544, 64, 12, 9), (65, 1032, 1304, 32, 17)])
+@pytest.mark.parametrize("n,d,h,e,k", [(513, 128, 256, 8, 2), (8192, 512, 2048, 16, 4), (203, 1544, 64, 12, 9), (65, 1032, 1304, 32, 17),
+                                       (2048, 1024, 4096, 16, 2)])
 def test_gate_outside_the_call(n, d, h, e, k, fuse, device, monkeypatch):
-    """A gate that drops slots (none of expert rows may be read for them), and a hook on a plain one."""
-    torch.full((64 << 20,), float("nan"), dtype=torch.bfloat16, device=device)   # (the rows past the routed ones are whatever was there)
+    """A gate that drops slots (none of expert rows may be read for them), and a hook on a plain one.  All memory that a pass allocates begins as
+    NaN: the rows past the routed ones are written by nothing.  (The last size has 1024 tiles of 256 x 256 of weight gradients, on the persistent kernel.)"""
+    real = torch.empty
+    blank = lambda *a, **kw: real(*a, **kw).view(torch.uint8).fill_(255).view(kw["dtype"])
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: blank(*a, **kw) if kw.get("dtype") in (torch.uint8, torch.bfloat16)
+                        and torch.device(kw.get("device", "cpu")).type == "cuda" else real(*a, **kw))
     x = torch.randn(n, d, device=device).to(torch.bfloat16).requires_grad_(True)
     grad = torch.randn(n, d, device=device).to(torch.bfloat16)
     moe = build(device, torch.bfloat16, d, h, e, k, gate=DroppingGate, fuse=fuse)
@@ -130,6 +135,28 @@ def test_gate_outside_the_call(n, d, h, e, k, fuse, device, monkeypatch):
     hooked.gate_hook = lambda idx, score, _: got.append((idx, score))
     compare(hooked, x, grad, int(one_call), monkeypatch)
     assert len(got) == 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_the_input_gradient_rounded_once_is_nearer_to_float64(dtype, device):
+    """The sum of the experts' and the gate's part is rounded once, the steps round both parts and their sum."""
+    n, d, h, e, k = 1500, 256, 512, 8, 2
+    moe = build(device, dtype, d, h, e, k, torch.nn.ReLU())
+    x = torch.randn(n, d, device=device).to(dtype).requires_grad_(True)
+    grad = torch.randn(n, d, device=device).to(dtype)
+    idx = moe.gate(x.detach())[0]
+    exact = copy.deepcopy(moe).double()
+    leaf = x.detach().double().requires_grad_(True)
+    score, one, two = exact.gate.gate(leaf).gather(1, idx), exact.experts.htoh4, exact.experts.h4toh
+    out = torch.zeros_like(leaf)
+    for i in range(e):
+        t, j = (idx == i).nonzero(as_tuple=True)
+        y = torch.relu(leaf[t] @ one.weight[i].t() + one.bias[i]) @ two.weight[i].t() + two.bias[i]
+        out = out.index_add(0, t, y * score[t, j][:, None])
+    want, = torch.autograd.grad(out, leaf, grad.double())
+    once, thrice = ((step(moe, x, grad, watched)[1].double() - want).norm() for watched in (False, True))
+    assert once <= thrice
 
 
 @pytest.mark.gpu
