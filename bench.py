@@ -35,7 +35,8 @@ CONFIGS = {
                     text="config5: 8192 tokens, d2048/h1024, 256 experts top-8, biased logits"),
 }
 
-PEAK = {"bf16": 2500.0, "f32": 157.3}  # dense MFMA TFLOP/s, MI355X
+# dense MFMA TFLOP/s, MI355X; a float32 product is six bf16 ones on the bf16 pipe (the fp32 pipe, which it does not use, has 157.3)
+PEAK = {"bf16": 2500.0, "f32": round(2500.0 / 6, 1)}
 # HBM-side bytes per launch of the grouped GEMM at config 4 (rocprofv3 FETCH_SIZE + WRITE_SIZE, each scaled by
 # what the same counter reads for a copy kernel of known size: 1.984 and 1.000); measured offline, not in this
 # script -- the counters need their own profiler runs.  Per class the mean over its launches of a step: forward

@@ -44,8 +44,8 @@ constexpr int kSlabBytes = 128;  // contraction bytes per row per slab
 enum Loaders { kLoadersCompute = 0, kLoadersAlone = 1, kLoadersShared = 2 };
 constexpr int ahead_of(int loaders) { return loaders == kLoadersAlone ? 2 : 0; }
 constexpr int extra_waves(int loaders) { return loaders == kLoadersCompute ? 0 : kLoadWaves; }
-// Two workgroups to a compute unit: at most 128 registers with waves that only load, 256 for fp32, whose two accumulators would otherwise
-// take up to 311 (nothing is spilled).
+// Two workgroups to a compute unit: at most 128 registers with waves that only load (3 to 9 of them are spilled, to 16 to 28 bytes per lane, outside the
+// slab loop: by the tile's start and the epilogues), 256 for fp32, whose two accumulators would otherwise take up to 311 (none is spilled).
 constexpr int waves_per_simd(int loaders, int element, int bn) { return loaders == kLoadersShared ? 4 : element == 4 && bn == 128 ? 2 : 1; }
 constexpr int kGroupM = 4;       // row tiles that share a column tile consecutively (an XCD then runs 4 x 8 tiles at a time)
 

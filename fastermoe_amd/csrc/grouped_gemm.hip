@@ -175,8 +175,8 @@ template <typename RowTiles> TileShape rows_16bit_tile(RowTiles row_tiles, doubl
 // The same for fp32 (products out of bf16 parts: Split8 in gemm_kernel.hpp; slabs of 32 elements).  A compute unit takes its m tiles
 // per_unit at a time, each such round start + slabs (alone + shared m / per_unit) us long, and as long as the fullest unit has tiles; the
 // parts of a tail whose contraction is shared come after them.  Fitted to 220 products of 4 to 128 experts, 64 to 32768 rows and 512 to 13056
-// features, then moved to where the shape picked is the best one most often: it takes 1.01 times what that does, 64 x 64 alone 1.16, 128 x 128 two to a
-// unit 1.09, one to a unit 1.07 times.  us for the three (and before, on the fp32 MFMA): 4 experts of 640 -> 512, 251 rows: 18 / 33 / 29; 4 of 832 -> 3328,
+// features, then moved to where the shape picked is the best one most often: repeated on the same weights it takes 1.01 times what that does, with
+// weights that change from call to call (120 other products) 1.02 times, 64 x 64 alone 1.18, 128 x 128 two to a unit 1.07, one to a unit 1.08 times.  Repeated, us for the three (and before, on the fp32 MFMA): 4 experts of 640 -> 512, 251 rows: 18 / 33 / 29; 4 of 832 -> 3328,
 // 547: 55 / 46 / 42; 32 of 640 -> 1344, 2635: 63 / 59 / 61; 8 of 1024 -> 512, 8192: 79 / 92 / 92 (98); 8 of 2048 -> 4096, 8192: 1063 / 787 / 816 (1095).
 struct F32RowShape {
     TileShape tile;
@@ -385,7 +385,7 @@ int dispatch(GemmParams &prm, int dtype, int epi, bool fast, hipStream_t stream)
 // Whether a launch over a device table goes to the persistent kernel of gemm_ring.hpp: 16-bit types and enough
 // tiles for 256 x 256 ones (and no tile shape forced).  There it was at least level on every product
 // measured: 4 to 9 % faster at K = 4096, 7 to 14 % at K = 1024, 26 to 37 % on weight gradients of 64 to 256 rows per
-// expert.  32-bit tiles take four times as long per slab, so what happens between them hardly shows.
+// expert.  Not built for 32-bit types, whose tiles are no larger than 128 x 128.
 bool use_ring(const TileShape &tile, int dtype) {
     return tile.many && is_16bit(dtype);
 }
@@ -539,8 +539,8 @@ bool linear_forward_can_gather(const LinearForwardArgs &a) {
 // checks shared by the launches over a device table; fills the parts of prm that say so
 int device_table_launch(const char *who, GemmParams &prm, const int32_t *dev_tab, int64_t rows_cap, int64_t n_expert,
                         bool taken) {
-    FMOE_REQUIRE(taken, "%s: a launch over a device segment table needs 16-byte aligned tensors, feature sizes that are "
-                       "multiples of 16 bytes and a 16- or 32-bit float type", who);
+    FMOE_REQUIRE(taken, "%s: a launch over a device segment table needs a 16- or 32-bit float type, 16-byte aligned tensors and feature "
+                       "sizes that are multiples of 16 bytes (in a layer's call 16-bit types need the type only)", who);
     FMOE_REQUIRE(n_expert >= 1 && n_expert <= (int64_t)(1 << 24) && rows_cap >= 0 && rows_cap <= (int64_t)INT32_MAX - 65536,
                  "%s: n_expert=%lld rows_cap=%lld", who, (long long)n_expert, (long long)rows_cap);
     FMOE_REQUIRE((reinterpret_cast<uintptr_t>(dev_tab) & 15u) == 0, "%s: the segment table must be 16-byte aligned", who);
