@@ -127,17 +127,18 @@ TileShape pick_tile(int64_t tiles_256) {
     return tiles_256 >= 256 ? TileShape{128, 256} : TileShape{128, 128};
 }
 
-// Row-ragged products in 16 bits with fewer than 512 tiles of 256 x 256: the shape with the least time by this estimate.  A round
-// of tiles that fills a share f of the chip's places takes start + slabs (alone + shared f) us, the accumulators' way out
-// included; the last round may be a partial one.  The weights' way from memory comes on top, as far as the rounds do not hide it.  The constants are
-// fitted to 300 products of 4 to 128 experts, 90 to 14000 rows and 512 to 8192 features, a tenth of a launch's time off on average, with
-// weights that change from call to call, as in a model.  (Repeated on the same ones up to 256 MB of them stay in the memory-side cache, and low
-// tiles, which read them more often, look better than they are: constants fitted like that picked shapes that took 1.042 times what the best of the five
-// does on 120 other products, these 1.035, and 0.90 times what 128 x 128 tiles below 256 tiles of 256 x 256 and 128 x 256 from there on did.)  us for 64 x 128 /
-// 128 x 128 alone / 128 x 128 shared / 128 x 256 / 256 x 256 (and 128 x 128 without loading waves): 8 experts of 4096 -> 1024, 1024 rows: 33 / 37 / 38 /
-// 37 / 48 (37); 16 of 768 -> 3072, 2000: 49 / 43 / 40 / 41 / 29 (37); of 3072 -> 768: 42 / 38 / 40 / 52 / 65 (41); 8 of 2048 -> 2048, 1600: 38 / 26 / 29 / 34 /
-// 47 (30); 8 of 1024 -> 1024, 4000: 27 / 26 / 21 / 21 / 29 (24); 12 of 2112 -> 2112, 5000: 103 / 83 / 72 / 67 / 54 (77); 8 of 2048 -> 1024, 8192:
-// 65 / 58 / 58 / 58 / 48 (60); 64 of 2048 -> 8192, 509: 516 / 397 / 399 / 377 / 429 (377).
+// Row-ragged products in 16 bits with fewer than 512 tiles of 256 x 256: the shape with the least time by this estimate.  A round of tiles
+// that fills a share f of the chip's places takes start + slabs (alone + shared f) us, the accumulators' way out included; the last round
+// may be a partial one.  The weights' way from memory comes on top, as far as the rounds do not hide it.  The constants are fitted to 300
+// products of 4 to 128 experts, 90 to 14000 rows and 512 to 8192 features, a tenth of a launch's time off on average, with weights that
+// change from call to call, as in a model.  (Repeated on the same ones up to 256 MB of them stay in the memory-side cache, and low tiles,
+// which read them more often, look better than they are: constants fitted like that picked shapes that took 1.042 times what the best of
+// the five does on 120 other products, these 1.035, and 0.90 times what 128 x 128 tiles below 256 tiles of 256 x 256 and 128 x 256 from
+// there on did.) us for 64 x 128 / 128 x 128 alone / 128 x 128 shared / 128 x 256 / 256 x 256 (and 128 x 128 without loading waves): 8
+// experts of 4096 -> 1024, 1024 rows: 33 / 37 / 38 / 37 / 48 (37); 16 of 768 -> 3072, 2000: 49 / 43 / 40 / 41 / 29 (37); of 3072 -> 768: 42
+// / 38 / 40 / 52 / 65 (41); 8 of 2048 -> 2048, 1600: 38 / 26 / 29 / 34 / 47 (30); 8 of 1024 -> 1024, 4000: 27 / 26 / 21 / 21 / 29 (24); 12
+// of 2112 -> 2112, 5000: 103 / 83 / 72 / 67 / 54 (77); 8 of 2048 -> 1024, 8192: 65 / 58 / 58 / 58 / 48 (60); 64 of 2048 -> 8192, 509: 516 /
+// 397 / 399 / 377 / 429 (377).
 struct RowShape {
     TileShape tile;
     int per_unit;                        // workgroups on a compute unit
@@ -174,10 +175,12 @@ template <typename RowTiles> TileShape rows_16bit_tile(RowTiles row_tiles, doubl
 
 // The same for fp32 (products out of bf16 parts: Split8 in gemm_kernel.hpp; slabs of 32 elements).  A compute unit takes its m tiles
 // per_unit at a time, each such round start + slabs (alone + shared m / per_unit) us long, and as long as the fullest unit has tiles; the
-// parts of a tail whose contraction is shared come after them.  Fitted to 220 products of 4 to 128 experts, 64 to 32768 rows and 512 to 13056
-// features, then moved to where the shape picked is the best one most often: repeated on the same weights it takes 1.01 times what that does, with
-// weights that change from call to call (120 other products) 1.02 times, 64 x 64 alone 1.18, 128 x 128 two to a unit 1.07, one to a unit 1.08 times.  Repeated, us for the three (and before, on the fp32 MFMA): 4 experts of 640 -> 512, 251 rows: 18 / 33 / 29; 4 of 832 -> 3328,
-// 547: 55 / 46 / 42; 32 of 640 -> 1344, 2635: 63 / 59 / 61; 8 of 1024 -> 512, 8192: 79 / 92 / 92 (98); 8 of 2048 -> 4096, 8192: 1063 / 787 / 816 (1095).
+// parts of a tail whose contraction is shared come after them.  Fitted to 220 products of 4 to 128 experts, 64 to 32768 rows and 512 to
+// 13056 features, then moved to where the shape picked is the best one most often: repeated on the same weights it takes 1.01 times what
+// that does, with weights that change from call to call (120 other products) 1.02 times, 64 x 64 alone 1.18, 128 x 128 two to a unit 1.07,
+// one to a unit 1.08 times.  Repeated, us for the three (and before, on the fp32 MFMA): 4 experts of 640 -> 512, 251 rows: 18 / 33 / 29; 4
+// of 832 -> 3328, 547: 55 / 46 / 42; 32 of 640 -> 1344, 2635: 63 / 59 / 61; 8 of 1024 -> 512, 8192: 79 / 92 / 92 (98); 8 of 2048 -> 4096,
+// 8192: 1063 / 787 / 816 (1095).
 struct F32RowShape {
     TileShape tile;
     int per_unit;
@@ -397,13 +400,14 @@ bool use_ring(const TileShape &tile, int dtype) {
 // and 13.8 / 36.3 / 55.5; 8 of 4096 x 14336, 8 / 32 / 64 / 128: 142 / 191 / 191 / 192 and 99 / 161 / 180 / 243; 256 of
 // 1024 x 2048, 256 / 512 / 1024: 134 / 179 / 205 and 124 / 170 / 210; 64 of 8192 x 2048, 64 / 128 / 256: 298 / 367 / 372
 // and 249 / 334 / 389.
-// float32: at most 24 rows per expert on average, 12 of contractions from 4096 on and 32 of shorter ones where the 128 x 128 tiles would number less
-// than half the compute units; as many as one pass takes in all (64) whatever the contraction.  The host does not know the counts, and an expert with more rows than a pass takes
-// walks its contraction again, so the lines are drawn where a skewed gate (shares 1 / rank^1.2) loses little.  us on the best tiles and
-// here with equal counts, then with skewed ones, weights from memory: 8 experts of 2048 -> 8192, 8 rows each: 205 / 125, 197 / 124; 24: 206 / 183, 206 / 194; 8 of
-// 8192 -> 2048, 12: 185 / 141, 183 / 175; 16: 186 / 153, 187 / 192; 24: 189 / 195, 188 / 305; 16 of 4096 -> 1024, 16: 101 / 79, 97 / 134; 24: 102 / 99, 101 / 144; 32 of 1024 -> 1024,
-// 8: 48 / 38, 47 / 45; 24: 50 / 52, 72 / 56; 64 of 1024 -> 4096, 16: 365 / 290, 356 / 309; 4 of 2048 -> 1024, 32: 37 / 20, 38 / 32; 40: 38 / 32, 38 / 54.  Where one expert
-// has all the rows the tiles are ahead: 64 of 1024 -> 4096, 256 rows: 25 / 42; 1024: 57 / 150.
+// float32: at most 24 rows per expert on average, 12 of contractions from 4096 on and 32 of shorter ones where the 128 x 128 tiles would
+// number less than half the compute units; as many as one pass takes in all (64) whatever the contraction.  The host does not know the
+// counts, and an expert with more rows than a pass takes walks its contraction again, so the lines are drawn where a skewed gate (shares 1
+// / rank^1.2) loses little.  us on the best tiles and here with equal counts, then with skewed ones, weights from memory: 8 experts of 2048
+// -> 8192, 8 rows each: 205 / 125, 197 / 124; 24: 206 / 183, 206 / 194; 8 of 8192 -> 2048, 12: 185 / 141, 183 / 175; 16: 186 / 153, 187 /
+// 192; 24: 189 / 195, 188 / 305; 16 of 4096 -> 1024, 16: 101 / 79, 97 / 134; 24: 102 / 99, 101 / 144; 32 of 1024 -> 1024, 8: 48 / 38, 47 /
+// 45; 24: 50 / 52, 72 / 56; 64 of 1024 -> 4096, 16: 365 / 290, 356 / 309; 4 of 2048 -> 1024, 32: 37 / 20, 38 / 32; 40: 38 / 32, 38 / 54.
+// Where one expert has all the rows the tiles are ahead: 64 of 1024 -> 4096, 256 rows: 25 / 42; 1024: 57 / 150.
 bool use_skinny(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype) {
     if ((!is_16bit(dtype) && dtype != FMOE_F32) || getenv("FMOE_GEMM_TILE")) return false;
     if (dtype == FMOE_F32) {
