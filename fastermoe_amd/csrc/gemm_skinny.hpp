@@ -13,12 +13,12 @@ struct SkinnyParams {
     int64_t x_total_rows;
     uint32_t div_mul;
     int32_t div_shift;
-    int32_t n_cols, k_extent, tiles_n, map_off, activation;
+    int32_t n_cols, k_extent, activation;
+    int32_t order_off, tiles_n, extra_groups;   // set by the launch: the table's list of experts, workgroups of a row group, see launch()
 };
-constexpr int kSkinnyCols = 16;   // columns of a workgroup
 
-// row_tiles: the most 128-row tiles the table can have
-int launch_skinny(const SkinnyParams &prm, int dtype, int64_t row_tiles, hipStream_t stream);
+// rows_cap: the rows that the table was laid out for
+int launch_skinny(const SkinnyParams &prm, int dtype, int64_t rows_cap, int64_t n_expert, hipStream_t stream);
 
 }  // namespace gemm
 }  // namespace fmoe

@@ -393,28 +393,23 @@ bool use_ring(const TileShape &tile, int dtype) {
     return tile.many && is_16bit(dtype);
 }
 
-// Whether a forward launch over a device table goes to gemm_skinny.hip (no tile shape forced).  16-bit types: at
-// most two rows per expert on average, or eight where the weights make less than two rounds of 128 x 128 tiles (512 at
-// a time), whose last round is then badly filled.  Above that the rows' way from L2 into every 16 columns costs more than
-// the tiles' padding.  bf16, us on the tiles and here: 32 experts of 4096 x 1024, 2 / 32 / 256 rows: 26.7 / 57.4 / 69.9
-// and 13.8 / 36.3 / 55.5; 8 of 4096 x 14336, 8 / 32 / 64 / 128: 142 / 191 / 191 / 192 and 99 / 161 / 180 / 243; 256 of
-// 1024 x 2048, 256 / 512 / 1024: 134 / 179 / 205 and 124 / 170 / 210; 64 of 8192 x 2048, 64 / 128 / 256: 298 / 367 / 372
-// and 249 / 334 / 389.
-// float32: at most 24 rows per expert on average, 12 of contractions from 4096 on and 32 of shorter ones where the 128 x 128 tiles would
-// number less than half the compute units; as many as one pass takes in all (64) whatever the contraction.  The host does not know the
-// counts, and an expert with more rows than a pass takes walks its contraction again, so the lines are drawn where a skewed gate (shares 1
-// / rank^1.2) loses little.  us on the best tiles and here with equal counts, then with skewed ones, weights from memory: 8 experts of 2048
-// -> 8192, 8 rows each: 205 / 125, 197 / 124; 24: 206 / 183, 206 / 194; 8 of 8192 -> 2048, 12: 185 / 141, 183 / 175; 16: 186 / 153, 187 /
-// 192; 24: 189 / 195, 188 / 305; 16 of 4096 -> 1024, 16: 101 / 79, 97 / 134; 24: 102 / 99, 101 / 144; 32 of 1024 -> 1024, 8: 48 / 38, 47 /
-// 45; 24: 50 / 52, 72 / 56; 64 of 1024 -> 4096, 16: 365 / 290, 356 / 309; 4 of 2048 -> 1024, 32: 37 / 20, 38 / 32; 40: 38 / 32, 38 / 54.
-// Where one expert has all the rows the tiles are ahead: 64 of 1024 -> 4096, 256 rows: 25 / 42; 1024: 57 / 150.
+// Whether a forward launch over a device table goes to gemm_skinny.hip (no tile shape forced).  The host does not know the counts: an
+// expert with more than 32 rows has its weights read again, from the caches, so the lines lie where a skewed gate loses little.
+// 16-bit types: at most four rows per expert on average, or twelve where the weights make less than two rounds of 128 x 128 tiles (512 at a
+// time), whose last round is then badly filled.  us on the tiles and here, weights from memory: 128 experts of 1088 x 4352, 1 row
+// each: 177 / 123; 256 of 2048 x 1024, 2: 184 / 140, of 1024 x 2048: 203 / 146; 64 of 1664 x 3328, 2.7: 154 / 108; 64 of 1408 x 1408, 3.6: 59 /
+// 39; 128 of 1280 x 1280, 3.5, a third of the rows one expert's: 26 / 29; 256 of 1536 x 1536, 8, a fifth of them one's: 82 / 117 (even counts at
+// 8: 64 of 2048 x 8192 384 / 333, 256 of 1088 x 2176 258 / 227).  Fewer tiles: 8 of 4096 x 14336, 8 rows: 187 / 138; 8 of 14336 x 4096, 8 / 12:
+// 176 / 146, 176 / 156; 12 of 512 x 1792, 12: 11.3 / 8.1; 16 of 768 x 3072, 12, at random / shares 1 / rank^1.2: 23.4 / 19.5, 24.1 / 20.5; of 3072
+// x 768: 31.5 / 21.8, 34.7 / 29.1; 32 of 768 x 3072, 13, a third of them one's: 41 / 36, of 3072 x 768: 36 / 41; 32 of 1024 x 1024, 15: 19.7 / 20.1.
+// float32: at most 32 rows per expert on average, 24 of contractions from 4096 on.  64 experts of 1216 x 1216, 1 row each: 105 / 44; 8 of
+// 1792 x 6272, 1.5: 140 / 46; 32 of 1024 x 3584, 16: 194 / 102; 64 of 1280 x 1280, 14, a third of the rows one's: 116 / 82; 256 of 1408 x 704,
+// 24: 402 / 300; 12 of 2432 x 1216, 27: 80 / 42; 32 of 1024 x 1024, 32: 51 / 51; 8 of 2048 x 8192, 48: 225 / 232; 8 of 8192 x 2048, 24, at random /
+// skewed: 190 / 119, 193 / 156.
 bool use_skinny(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype) {
     if ((!is_16bit(dtype) && dtype != FMOE_F32) || getenv("FMOE_GEMM_TILE")) return false;
-    if (dtype == FMOE_F32) {
-        if (in_feat >= 4096 && rows_cap > 64) return rows_cap <= 12 * n_expert;
-        return rows_cap <= 24 * n_expert || (rows_cap <= 32 * n_expert && n_expert * ceil_div(out_feat, 128) * 2 < device_compute_units());
-    }
-    return rows_cap <= 2 * n_expert || (rows_cap <= 8 * n_expert && n_expert * ceil_div(out_feat, 128) < 1024);
+    if (dtype == FMOE_F32) return rows_cap <= (in_feat >= 4096 ? 24 : 32) * n_expert;
+    return rows_cap <= 4 * n_expert || (rows_cap <= 12 * n_expert && n_expert * ceil_div(out_feat, 128) < 1024);
 }
 
 // The kernel of a row-ragged launch over a device table, and the workspace it can make use of.
@@ -598,10 +593,8 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
             sk.row_index = a.x_row_index; sk.x_total_rows = a.x_total_rows;
             sk.div_mul = prm.q_div_mul; sk.div_shift = prm.q_div_shift;
             sk.n_cols = prm.n_cols; sk.k_extent = prm.k_extent; sk.activation = prm.activation;
-            sk.tiles_n = (int)ceil_div(a.out_feat, kSkinnyCols);
-            sk.map_off = (int32_t)segtab::map128_off(a.dev_rows_cap, n_expert);
             ProfileScope prof(prm.profile_class, prm.profile_work, stream);
-            return launch_skinny(sk, a.dtype, segtab::cap_tiles(a.dev_rows_cap, n_expert, 128), stream);
+            return launch_skinny(sk, a.dtype, a.dev_rows_cap, n_expert, stream);
         }
         if (route.kernel == DevKernel::kRing) return dispatch_ring<kFwd>(prm, a.dtype, a.epilogue, stream);
         return dispatch<kFwd>(prm, a.dtype, a.epilogue, fast, stream);
