@@ -402,13 +402,17 @@ bool use_ring(const TileShape &tile, int dtype) {
 // 8: 64 of 2048 x 8192 384 / 333, 256 of 1088 x 2176 258 / 227).  Fewer tiles: 8 of 4096 x 14336, 8 rows: 187 / 138; 8 of 14336 x 4096, 8 / 12:
 // 176 / 146, 176 / 156; 12 of 512 x 1792, 12: 11.3 / 8.1; 16 of 768 x 3072, 12, at random / shares 1 / rank^1.2: 23.4 / 19.5, 24.1 / 20.5; of 3072
 // x 768: 31.5 / 21.8, 34.7 / 29.1; 32 of 768 x 3072, 13, a third of them one's: 41 / 36, of 3072 x 768: 36 / 41; 32 of 1024 x 1024, 15: 19.7 / 20.1.
-// float32: at most 32 rows per expert on average, 24 of contractions from 4096 on.  64 experts of 1216 x 1216, 1 row each: 105 / 44; 8 of
-// 1792 x 6272, 1.5: 140 / 46; 32 of 1024 x 3584, 16: 194 / 102; 64 of 1280 x 1280, 14, a third of the rows one's: 116 / 82; 256 of 1408 x 704,
-// 24: 402 / 300; 12 of 2432 x 1216, 27: 80 / 42; 32 of 1024 x 1024, 32: 51 / 51; 8 of 2048 x 8192, 48: 225 / 232; 8 of 8192 x 2048, 24, at random /
-// skewed: 190 / 119, 193 / 156.
+// float32: at most 24 rows per expert on average, 12 of contractions from 4096 on and 32 of shorter ones where the 128 x 128 tiles would
+// number less than half the compute units; as many as two passes take in all (64) whatever the contraction.  64 experts of 1216 x 1216, 1 row
+// each: 105 / 44; 8 of 1792 x 6272, 1.5: 140 / 46; 32 of 1024 x 3584, 16: 194 / 102; 64 of 1280 x 1280, 14, a third of the rows one's: 116 / 82; 256
+// of 1408 x 704, 24: 402 / 300; 12 of 2432 x 1216, 27: 80 / 42; 32 of 1024 x 1024, 32: 51 / 51; 8 of 2048 x 8192, 48: 225 / 232; 8 of 8192 x 2048, 24,
+// at random / skewed: 190 / 119, 193 / 156.
 bool use_skinny(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype) {
     if ((!is_16bit(dtype) && dtype != FMOE_F32) || getenv("FMOE_GEMM_TILE")) return false;
-    if (dtype == FMOE_F32) return rows_cap <= (in_feat >= 4096 ? 24 : 32) * n_expert;
+    if (dtype == FMOE_F32) {
+        if (in_feat >= 4096 && rows_cap > 64) return rows_cap <= 12 * n_expert;
+        return rows_cap <= 24 * n_expert || (rows_cap <= 32 * n_expert && n_expert * ceil_div(out_feat, 128) * 2 < device_compute_units());
+    }
     return rows_cap <= 4 * n_expert || (rows_cap <= 12 * n_expert && n_expert * ceil_div(out_feat, 128) < 1024);
 }
 
