@@ -43,6 +43,9 @@ SIGNATURES = {
                                                  _vp, _i64, _vp, _i64, _vp]),
     "fmoe_gate_topk_backward": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _int, _vp]),
     "fmoe_gate_grad_supported": (_int, [_i64, _i64, _i64, _int]),
+    "fmoe_gate_grad_any_supported": (_int, [_i64, _i64, _i64, _int]),
+    "fmoe_gate_weight_grad_any": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _i64, _vp]),
+    "fmoe_reduce_slots_gate_any": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp]),
     "fmoe_gate_weight_grad_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "fmoe_gate_weight_grad": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _i64, _vp]),
     "fmoe_reduce_slots_gate": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp]),

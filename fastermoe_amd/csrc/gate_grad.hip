@@ -7,7 +7,7 @@
 //   grad_x[t] = experts' part + sum_j g[t,j] w[idx[t,j]]      grad_w[e] = sum over (t,j) with idx = e of g[t,j] x[t]
 // Here the gate's part of the first is a sum of top_k rows of w per token (a caller that has the experts' part as rows gets
 // both sums in one pass; the layer does not call it so), and the second is one pass over x with the matrix cores.
-#include "common.hpp"
+#include "gate_grad.hpp"
 #include "profile.hpp"
 #include "vec16.hpp"
 
@@ -32,11 +32,21 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 // (27.9 / 25.5 / 26.7, 23.5), 16384 of 4096, top-4: 55 / 54 / 64; float32, 32768 of 4096, top-2: 115 / 87 / 81, top-4 at 16384:
 // 87 / 71 / 84.  As a library product over the dense gradient the first took 99.
 // Tokens or rows too few for that many waves take P = 1.
-template <typename T, int K, int P>
+// ANY (16-bit types): rows of any length, read 16 bytes at a time wherever they lie; row_vecs counts the last, partial piece.
+template <typename T, int K, int P, bool ANY>
 __global__ __launch_bounds__(kBlock) void reduce_slots_gate_kernel(
     const u32x4 *__restrict__ rows, const int64_t *__restrict__ slot_to_row, const T *__restrict__ grad_score,
     const int64_t *__restrict__ topk_idx, const u32x4 *__restrict__ w, u32x4 *__restrict__ out, int64_t n_tokens, int top_k,
-    int64_t n_rows, int n_expert, int row_vecs, int groups_per_row) {
+    int64_t n_rows, int n_expert, int row_vecs, int groups_per_row, int row_elems) {
+    // vector v of row r
+    auto load = [&](const u32x4 *base, int64_t r, int v, auto once) {
+        if constexpr (ANY) {
+            return load_some((const T *)base + r * row_elems + v * 8, row_elems - v * 8);
+        } else {
+            const u32x4 *at = &base[r * row_vecs + v];
+            if constexpr (decltype(once)::value) return __builtin_nontemporal_load(at); else return *at;
+        }
+    };
     const int lane = threadIdx.x & (kWave - 1);
     // one token per wave: its slots' rows, experts and gradients are scalar loads
     const uint32_t group = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave);
@@ -57,8 +67,8 @@ __global__ __launch_bounds__(kBlock) void reduce_slots_gate_kernel(
 #pragma unroll
             for (int p = 0; p < P; ++p) {
                 const int v = v0 + p * kWave;
-                val[p][j] = live && v < row_vecs ? __builtin_nontemporal_load(&rows[src * row_vecs + v]) : u32x4{0, 0, 0, 0};
-                wv[p][j] = named && v < row_vecs ? w[e * row_vecs + v] : u32x4{0, 0, 0, 0};
+                val[p][j] = live && v < row_vecs ? load(rows, src, v, std::true_type{}) : u32x4{0, 0, 0, 0};
+                wv[p][j] = named && v < row_vecs ? load(w, e, v, std::false_type{}) : u32x4{0, 0, 0, 0};
             }
         }
 #pragma unroll
@@ -80,23 +90,25 @@ __global__ __launch_bounds__(kBlock) void reduce_slots_gate_kernel(
         if (v >= row_vecs) continue;
 #pragma unroll
         for (int i = 0; i < Vec<T>::N; ++i) acc[p][i] += gate[p][i];
-        __builtin_nontemporal_store(Vec<T>::pack(acc[p]), &out[t * row_vecs + v]);
+        if constexpr (ANY) store_some((T *)out + t * row_elems + v * 8, Vec<T>::pack(acc[p]), row_elems - v * 8);
+        else __builtin_nontemporal_store(Vec<T>::pack(acc[p]), &out[t * row_vecs + v]);
     }
 }
 
-template <typename T, int K>
+template <typename T, int K, bool ANY>
 int launch_reduce_gate(const void *rows, const int64_t *slot_to_row, const void *grad_score, const int64_t *topk_idx, const void *w,
-                       void *out, int64_t n_tokens, int64_t top_k, int64_t n_rows, int64_t n_expert, int64_t row_vecs,
+                       void *out, int64_t n_tokens, int64_t top_k, int64_t n_rows, int64_t n_expert, int64_t row_elems,
                        hipStream_t st) {
+    const int64_t row_vecs = ceil_div(row_elems * (int64_t)sizeof(T), 16);
     constexpr int kPieces = K >= 8 ? 1 : K == 4 || sizeof(T) == 2 ? 2 : 4;
 #define FMOE_RG(P)                                                                                                                    \
     {                                                                                                                                 \
         const int64_t groups = ceil_div(row_vecs, (P) * kWave), blocks = ceil_div(n_tokens * groups, kWavesPerBlock);                  \
         if (blocks > INT32_MAX / kWavesPerBlock) return fail(FMOE_ELIMIT, "fmoe_reduce_slots_gate: grid too large");                   \
-        reduce_slots_gate_kernel<T, K, P><<<(int)blocks, kBlock, 0, st>>>((const u32x4 *)rows, slot_to_row, (const T *)grad_score,     \
+        reduce_slots_gate_kernel<T, K, P, ANY><<<(int)blocks, kBlock, 0, st>>>((const u32x4 *)rows, slot_to_row, (const T *)grad_score,     \
                                                                          topk_idx, (const u32x4 *)w, (u32x4 *)out, n_tokens,          \
                                                                          (int)top_k, n_rows, (int)n_expert, (int)row_vecs,            \
-                                                                         (int)groups);                                                \
+                                                                         (int)groups, (int)row_elems);                                \
     }
     if (kPieces > 1 && row_vecs >= kPieces * kWave && n_tokens * row_vecs >= (int64_t)kPieces * kWave * 4096) FMOE_RG(kPieces)
     else FMOE_RG(1)
@@ -117,7 +129,7 @@ constexpr int kCols = 128;
 template <typename T> constexpr int tokens_per_step() { return sizeof(T) == 2 ? 64 : 32; }
 template <typename T> constexpr int g_stride() { return tokens_per_step<T>() + 16 / (int)sizeof(T); }   // elements per expert
 
-template <typename T, int EB>   // EB: blocks of 16 experts
+template <typename T, int EB, bool ANY>   // EB: blocks of 16 experts; ANY (16-bit types): rows of x of any length
 __global__ __launch_bounds__(kBlock) void gate_wgrad_kernel(const T *__restrict__ grad_score, const int64_t *__restrict__ topk_idx,
                                                             const T *__restrict__ x, float *__restrict__ part_w,
                                                             float *__restrict__ part_b, int n_tokens, int d, int n_expert, int top_k,
@@ -154,7 +166,10 @@ __global__ __launch_bounds__(kBlock) void gate_wgrad_kernel(const T *__restrict_
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
             const int q = i * kBlock + t, k = q / CPR, c = q % CPR;
-            ahead[i] = (t0 + k < hi && c0 + c * CE < d) ? *(const u32x4 *)(x + (int64_t)(t0 + k) * d + c0 + c * CE) : u32x4{0, 0, 0, 0};
+            const T *at = x + (int64_t)(t0 + k) * d + c0 + c * CE;
+            const bool in = t0 + k < hi && c0 + c * CE < d;
+            if constexpr (ANY) ahead[i] = in ? load_some(at, d - (c0 + c * CE)) : u32x4{0, 0, 0, 0};
+            else ahead[i] = in ? *(const u32x4 *)at : u32x4{0, 0, 0, 0};
         }
     };
     // this step's first kHeld entries per thread are loaded a step ahead and kept until they are cleared again
@@ -329,7 +344,7 @@ int wgrad_ranges(int64_t n_tokens, int64_t d, int64_t n_expert) {
     return (int)(r < 1 ? 1 : r);
 }
 
-template <typename T>
+template <typename T, bool ANY>
 int launch_wgrad(const void *grad_score, const int64_t *topk_idx, const void *x, void *grad_w, void *grad_b, int64_t n_tokens,
                  int64_t d, int64_t n_expert, int64_t top_k, float *ws, hipStream_t st) {
     const int ranges = wgrad_ranges(n_tokens, d, n_expert);
@@ -340,7 +355,7 @@ int launch_wgrad(const void *grad_score, const int64_t *topk_idx, const void *x,
     const int eb = n_expert <= 16 ? 1 : n_expert <= 32 ? 2 : n_expert <= 64 ? 4 : n_expert <= 128 ? 8 : 16;
     const size_t lds = (tokens_per_step<T>() * kCols + eb * 16 * g_stride<T>()) * sizeof(T);
 #define FMOE_GW(EB)                                                                                                          \
-    gate_wgrad_kernel<T, EB><<<grid, kBlock, lds, st>>>((const T *)grad_score, topk_idx, (const T *)x, part_w, part_b,        \
+    gate_wgrad_kernel<T, EB, ANY><<<grid, kBlock, lds, st>>>((const T *)grad_score, topk_idx, (const T *)x, part_w, part_b,        \
                                                         (int)n_tokens, (int)d, (int)n_expert, (int)top_k, per_range)
     switch (eb) {
         case 1: FMOE_GW(1); break;
@@ -359,6 +374,67 @@ int launch_wgrad(const void *grad_score, const int64_t *topk_idx, const void *x,
 }
 
 }  // namespace
+
+bool gate_grad_any_grid(int64_t d_model, int64_t n_expert, int64_t top_k, int dtype) {
+    return fmoe_gate_grad_supported(d_model, n_expert, top_k, dtype) == 1 ||
+           (dtype_bytes(dtype) == 2 && n_expert >= 1 && n_expert <= kMaxGateExpert && top_k >= 1 && top_k <= n_expert && d_model >= 1 &&
+            d_model < (1 << 24));
+}
+
+int gate_weight_grad(const void *grad_score, const int64_t *topk_idx, const void *x, void *grad_w, void *grad_b, int64_t n_tokens,
+                     int64_t d_model, int64_t n_expert, int64_t top_k, int dtype, void *workspace, int64_t workspace_bytes, hipStream_t st) {
+    FMOE_REQUIRE(n_tokens >= 1 && n_tokens * top_k <= (int64_t)INT32_MAX, "fmoe_gate_weight_grad: n_tokens=%lld", (long long)n_tokens);
+    FMOE_REQUIRE(grad_score && topk_idx && x && grad_w && aligned16(x), "fmoe_gate_weight_grad: NULL or misaligned pointer");
+    const int64_t need = fmoe_gate_weight_grad_workspace_bytes(n_tokens, d_model, n_expert);
+    if (workspace == nullptr || workspace_bytes < need)
+        return fail(FMOE_EWORKSPACE, "fmoe_gate_weight_grad: needs %lld bytes of workspace, got %lld", (long long)need,
+                    (long long)workspace_bytes);
+    FMOE_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 3u) == 0, "fmoe_gate_weight_grad: the workspace must be 4-byte aligned");
+    float *ws = (float *)workspace;
+    const bool any = (d_model * dtype_bytes(dtype)) % 16 != 0;
+#define FMOE_GWL(T, ANY) return launch_wgrad<T, ANY>(grad_score, topk_idx, x, grad_w, grad_b, n_tokens, d_model, n_expert, top_k, ws, st)
+    if (dtype == FMOE_F32) FMOE_GWL(float, false);
+    if (dtype == FMOE_BF16) {
+        if (any) FMOE_GWL(__bf16, true);
+        FMOE_GWL(__bf16, false);
+    }
+    if (any) FMOE_GWL(_Float16, true);
+    FMOE_GWL(_Float16, false);
+#undef FMOE_GWL
+}
+
+int reduce_slots_gate(const void *rows, const int64_t *slot_to_row, const void *grad_score, const int64_t *topk_idx, const void *w, void *out,
+                      int64_t n_tokens, int64_t top_k, int64_t n_rows, int64_t n_expert, int64_t row_elems, int dtype, hipStream_t st) {
+    FMOE_REQUIRE(dtype == FMOE_F32 || dtype == FMOE_BF16 || dtype == FMOE_F16, "fmoe_reduce_slots_gate: dtype %d", dtype);
+    FMOE_REQUIRE(n_tokens >= 0 && top_k >= 1 && n_rows >= 0 && n_expert >= 1 && row_elems >= 0, "fmoe_reduce_slots_gate: bad sizes");
+    if (n_tokens == 0 || row_elems == 0) return FMOE_OK;
+    if (n_tokens > (int64_t)INT32_MAX || top_k > 65536 || row_elems > (int64_t)(1 << 28) || n_expert > (int64_t)(1 << 24))
+        return fail(FMOE_ELIMIT, "fmoe_reduce_slots_gate: sizes beyond the supported range");
+    FMOE_REQUIRE(grad_score && topk_idx && w && out && (rows || n_rows == 0 || slot_to_row == nullptr), "fmoe_reduce_slots_gate: NULL pointer");
+    const bool any = (row_elems * dtype_bytes(dtype)) % 16 != 0;
+    FMOE_REQUIRE(!any || dtype != FMOE_F32, "fmoe_reduce_slots_gate: rows must be whole 16-byte chunks");
+    // (bytes: the experts' rows and the result; the gate's part alone: its weight, once, and the result)
+    ProfileScope prof(kProfReduceSlots, (double)(slot_to_row ? (top_k + 1) * n_tokens : n_tokens + n_expert) * row_elems * dtype_bytes(dtype), st);
+#define FMOE_RGT(T, K, ANY)                                                                                                       \
+    return launch_reduce_gate<T, K, ANY>(rows, slot_to_row, grad_score, topk_idx, w, out, n_tokens, top_k, n_rows, n_expert, row_elems, st)
+#define FMOE_RGK(T, ANY)                                                                                                          \
+    {                                                                                                                             \
+        if (top_k == 1) FMOE_RGT(T, 1, ANY);                                                                                      \
+        if (top_k == 2) FMOE_RGT(T, 2, ANY);                                                                                      \
+        if (top_k <= 4) FMOE_RGT(T, 4, ANY);                                                                                      \
+        FMOE_RGT(T, 8, ANY);                                                                                                      \
+    }
+    if (dtype == FMOE_F32) FMOE_RGK(float, false)
+    if (dtype == FMOE_BF16) {
+        if (any) FMOE_RGK(__bf16, true)
+        FMOE_RGK(__bf16, false)
+    }
+    if (any) FMOE_RGK(_Float16, true)
+    FMOE_RGK(_Float16, false)
+#undef FMOE_RGK
+#undef FMOE_RGT
+}
+
 }  // namespace fmoe
 
 using namespace fmoe;
@@ -380,47 +456,37 @@ extern "C" int fmoe_gate_weight_grad(const void *grad_score, const int64_t *topk
     if (!fmoe_gate_grad_supported(d_model, n_expert, top_k, dtype))
         return fail(FMOE_ELIMIT, "fmoe_gate_weight_grad: d_model=%lld n_expert=%lld top_k=%lld dtype=%d is not taken", (long long)d_model,
                     (long long)n_expert, (long long)top_k, dtype);
-    FMOE_REQUIRE(n_tokens >= 1 && n_tokens * top_k <= (int64_t)INT32_MAX, "fmoe_gate_weight_grad: n_tokens=%lld", (long long)n_tokens);
-    FMOE_REQUIRE(grad_score && topk_idx && x && grad_w && aligned16(x), "fmoe_gate_weight_grad: NULL or misaligned pointer");
-    const int64_t need = fmoe_gate_weight_grad_workspace_bytes(n_tokens, d_model, n_expert);
-    if (workspace == nullptr || workspace_bytes < need)
-        return fail(FMOE_EWORKSPACE, "fmoe_gate_weight_grad: needs %lld bytes of workspace, got %lld", (long long)need,
-                    (long long)workspace_bytes);
-    FMOE_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 3u) == 0, "fmoe_gate_weight_grad: the workspace must be 4-byte aligned");
-    float *ws = (float *)workspace;
-    hipStream_t st = (hipStream_t)stream;
-    if (dtype == FMOE_F32) return launch_wgrad<float>(grad_score, topk_idx, x, grad_w, grad_b, n_tokens, d_model, n_expert, top_k, ws, st);
-    if (dtype == FMOE_BF16) return launch_wgrad<__bf16>(grad_score, topk_idx, x, grad_w, grad_b, n_tokens, d_model, n_expert, top_k, ws, st);
-    return launch_wgrad<_Float16>(grad_score, topk_idx, x, grad_w, grad_b, n_tokens, d_model, n_expert, top_k, ws, st);
+    return gate_weight_grad(grad_score, topk_idx, x, grad_w, grad_b, n_tokens, d_model, n_expert, top_k, dtype, workspace, workspace_bytes,
+                            (hipStream_t)stream);
+}
+
+extern "C" int fmoe_gate_grad_any_supported(int64_t d_model, int64_t n_expert, int64_t top_k, int dtype) {
+    return gate_grad_any_grid(d_model, n_expert, top_k, dtype) ? 1 : 0;
+}
+
+extern "C" int fmoe_gate_weight_grad_any(const void *grad_score, const int64_t *topk_idx, const void *x, void *grad_w, void *grad_b,
+                                         int64_t n_tokens, int64_t d_model, int64_t n_expert, int64_t top_k, int dtype, void *workspace,
+                                         int64_t workspace_bytes, void *stream) {
+    if (!gate_grad_any_grid(d_model, n_expert, top_k, dtype))
+        return fail(FMOE_ELIMIT, "fmoe_gate_weight_grad_any: d_model=%lld n_expert=%lld top_k=%lld dtype=%d is not taken", (long long)d_model,
+                    (long long)n_expert, (long long)top_k, dtype);
+    return gate_weight_grad(grad_score, topk_idx, x, grad_w, grad_b, n_tokens, d_model, n_expert, top_k, dtype, workspace, workspace_bytes,
+                            (hipStream_t)stream);
+}
+
+extern "C" int fmoe_reduce_slots_gate_any(const void *rows, const int64_t *slot_to_row, const void *grad_score, const int64_t *topk_idx,
+                                          const void *w, void *out, int64_t n_tokens, int64_t top_k, int64_t n_rows, int64_t n_expert,
+                                          int64_t row_elems, int dtype, void *stream) {
+    FMOE_REQUIRE(aligned16(rows) && aligned16(w) && aligned16(out), "fmoe_reduce_slots_gate_any: misaligned pointer");
+    return reduce_slots_gate(rows, slot_to_row, grad_score, topk_idx, w, out, n_tokens, top_k, n_rows, n_expert, row_elems, dtype,
+                             (hipStream_t)stream);
 }
 
 extern "C" int fmoe_reduce_slots_gate(const void *rows, const int64_t *slot_to_row, const void *grad_score, const int64_t *topk_idx,
                                       const void *w, void *out, int64_t n_tokens, int64_t top_k, int64_t n_rows, int64_t n_expert,
                                       int64_t row_elems, int dtype, void *stream) {
-    FMOE_REQUIRE(dtype == FMOE_F32 || dtype == FMOE_BF16 || dtype == FMOE_F16, "fmoe_reduce_slots_gate: dtype %d", dtype);
-    FMOE_REQUIRE(n_tokens >= 0 && top_k >= 1 && n_rows >= 0 && n_expert >= 1 && row_elems >= 0, "fmoe_reduce_slots_gate: bad sizes");
-    if (n_tokens == 0 || row_elems == 0) return FMOE_OK;
-    if (n_tokens > (int64_t)INT32_MAX || top_k > 65536 || row_elems > (int64_t)(1 << 28) || n_expert > (int64_t)(1 << 24))
-        return fail(FMOE_ELIMIT, "fmoe_reduce_slots_gate: sizes beyond the supported range");
-    FMOE_REQUIRE(grad_score && topk_idx && w && out && (rows || n_rows == 0 || slot_to_row == nullptr), "fmoe_reduce_slots_gate: NULL pointer");
     FMOE_REQUIRE((row_elems * dtype_bytes(dtype)) % 16 == 0 && aligned16(rows) && aligned16(w) && aligned16(out),
                  "fmoe_reduce_slots_gate: rows must be whole 16-byte chunks");
-    hipStream_t st = (hipStream_t)stream;
-    // (bytes: the experts' rows and the result; the gate's part alone: its weight, once, and the result)
-    ProfileScope prof(kProfReduceSlots, (double)(slot_to_row ? (top_k + 1) * n_tokens : n_tokens + n_expert) * row_elems * dtype_bytes(dtype), st);
-    const int64_t row_vecs = row_elems * dtype_bytes(dtype) / 16;
-#define FMOE_RGT(T, K)                                                                                                            \
-    return launch_reduce_gate<T, K>(rows, slot_to_row, grad_score, topk_idx, w, out, n_tokens, top_k, n_rows, n_expert, row_vecs, st)
-#define FMOE_RGK(T)                                                                                                               \
-    {                                                                                                                             \
-        if (top_k == 1) FMOE_RGT(T, 1);                                                                                           \
-        if (top_k == 2) FMOE_RGT(T, 2);                                                                                           \
-        if (top_k <= 4) FMOE_RGT(T, 4);                                                                                           \
-        FMOE_RGT(T, 8);                                                                                                           \
-    }
-    if (dtype == FMOE_F32) FMOE_RGK(float)
-    if (dtype == FMOE_BF16) FMOE_RGK(__bf16)
-    FMOE_RGK(_Float16)
-#undef FMOE_RGK
-#undef FMOE_RGT
+    return reduce_slots_gate(rows, slot_to_row, grad_score, topk_idx, w, out, n_tokens, top_k, n_rows, n_expert, row_elems, dtype,
+                             (hipStream_t)stream);
 }

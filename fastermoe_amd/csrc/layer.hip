@@ -8,6 +8,7 @@
 // tensors that it hands in.  Blocks whose lives do not overlap share memory: the sorted input is the output rows' place before the
 // second linear writes them, and in the backward one block of rows is in turn the gradient of the experts' output, the
 // experts' input gradient and the sorted input.
+#include "gate_grad.hpp"
 #include "grouped_gemm.hpp"
 #include "permute.hpp"
 
@@ -270,8 +271,8 @@ extern "C" int fmoe_layer_backward(const void *grad_out, const void *x, const vo
         rc = linear_dgrad(s, b.grad_pre, w1, nullptr, b.rows, segment_table, d_model, d_hidden, FMOE_ACT_NONE, b.ws, b.split1, st);
         if (rc != FMOE_OK) return rc;
         // (the gate's part of the input gradient is added in the same pass, before the one rounding)
-        rc = gated ? fmoe_reduce_slots_gate(b.rows, slot_to_row, grad_score, topk_idx, gate_w, grad_x, n_tokens, top_k, s.n_slots, n_expert,
-                                            d_model, dtype, stream)
+        rc = gated ? reduce_slots_gate(b.rows, slot_to_row, grad_score, topk_idx, gate_w, grad_x, n_tokens, top_k, s.n_slots, n_expert,
+                                       d_model, dtype, st)
                    : fmoe_reduce_slots(b.rows, slot_to_row, grad_x, n_tokens, top_k, s.n_slots, d_model, dtype, stream);
         if (rc != FMOE_OK) return rc;
     }
@@ -282,7 +283,7 @@ extern "C" int fmoe_layer_backward(const void *grad_out, const void *x, const vo
         if (rc != FMOE_OK) return rc;
     }
     if (gated && grad_gate_w != nullptr)
-        rc = fmoe_gate_weight_grad(grad_score, topk_idx, x, grad_gate_w, grad_gate_b, n_tokens, d_model, n_expert, top_k, dtype, b.ws,
-                                   b.gate_bytes, stream);
+        rc = gate_weight_grad(grad_score, topk_idx, x, grad_gate_w, grad_gate_b, n_tokens, d_model, n_expert, top_k, dtype, b.ws,
+                              b.gate_bytes, st);
     return rc;
 }

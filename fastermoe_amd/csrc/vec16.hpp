@@ -57,4 +57,31 @@ template <> struct Vec<_Float16> {
     }
 };
 
+// The first n of the 16-bit elements at p, which may lie anywhere, zeros after them (8 <= n: all eight); nothing past them is read.
+template <typename T> __device__ __forceinline__ u32x4 load_some(const T *p, int64_t n) {
+    static_assert(sizeof(T) == 2, "16-bit element types");
+    if (n >= 8) {
+        u32x4 v;
+        __builtin_memcpy(&v, p, 16);
+        return v;
+    }
+    alignas(16) uint16_t e[8] = {};
+#pragma unroll
+    for (int j = 0; j < 7; ++j)
+        if (j < n) e[j] = ((const uint16_t *)p)[j];
+    return __builtin_bit_cast(u32x4, e);
+}
+template <typename T> __device__ __forceinline__ void store_some(T *p, const u32x4 &v, int64_t n) {
+    static_assert(sizeof(T) == 2, "16-bit element types");
+    if (n >= 8) {
+        __builtin_memcpy(p, &v, 16);
+        return;
+    }
+    alignas(16) uint16_t e[8];
+    __builtin_memcpy(e, &v, 16);
+#pragma unroll
+    for (int j = 0; j < 7; ++j)
+        if (j < n) ((uint16_t *)p)[j] = e[j];
+}
+
 }  // namespace fmoe

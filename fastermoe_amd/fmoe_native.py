@@ -283,9 +283,15 @@ def gate_grad_supported(d_model, n_expert, top_k, dtype):
                                                                      _DTYPES[dtype]) == 1
 
 
-def gate_weight_grad(grad_score, topk_idx, x, n_expert, with_bias):
+def gate_grad_any_supported(d_model, n_expert, top_k, dtype):
+    """The same with ``any_grid``; :func:`layer_backward` differentiates these gates."""
+    return dtype in _DTYPES and _lib.load().fmoe_gate_grad_any_supported(int(d_model), int(n_expert), int(top_k),
+                                                                         _DTYPES[dtype]) == 1
+
+
+def gate_weight_grad(grad_score, topk_idx, x, n_expert, with_bias, any_grid=False):
     """Gradients ``(grad_w [E, d_model], grad_b [E] or None)`` of the gate's linear layer from the gradient
-    ``[N, k]`` of the selected logits."""
+    ``[N, k]`` of the selected logits.  ``any_grid``: rows of 16-bit types that are no whole 16-byte chunks are taken too."""
     dt = _rows("x", x)
     _dev("grad_score", grad_score, x.dtype)
     _dev("topk_idx", topk_idx, torch.int64)
@@ -300,14 +306,16 @@ def gate_weight_grad(grad_score, topk_idx, x, n_expert, with_bias):
         return grad_w.zero_(), grad_b.zero_() if with_bias else None
     with _on(x.device):
         ws = _workspace(lib.fmoe_gate_weight_grad_workspace_bytes(n, d, n_expert), x.device)
-        check(lib.fmoe_gate_weight_grad(_ptr(grad_score), _ptr(topk_idx), _ptr(x), _ptr(grad_w), _ptr(grad_b), n, d, n_expert, k,
-                                        dt, _ptr(ws), ws.numel(), _stream(x)))
+        call = lib.fmoe_gate_weight_grad_any if any_grid else lib.fmoe_gate_weight_grad
+        check(call(_ptr(grad_score), _ptr(topk_idx), _ptr(x), _ptr(grad_w), _ptr(grad_b), n, d, n_expert, k, dt, _ptr(ws), ws.numel(),
+                   _stream(x)))
     return grad_w, grad_b
 
 
-def reduce_slots_gate(inp, slot_to_row, grad_score, topk_idx, weight):
+def reduce_slots_gate(inp, slot_to_row, grad_score, topk_idx, weight, any_grid=False):
     """:func:`reduce_slots` plus the gate's part of the input gradient,
-    ``sum_j grad_score[t,j] * weight[topk_idx[t,j]]``; ``inp`` and ``slot_to_row`` ``None``: that part alone."""
+    ``sum_j grad_score[t,j] * weight[topk_idx[t,j]]``; ``inp`` and ``slot_to_row`` ``None``: that part alone.  ``any_grid`` as
+    in :func:`gate_weight_grad`."""
     dt = _rows("weight", weight)
     _dev("grad_score", grad_score, weight.dtype)
     _dev("topk_idx", topk_idx, torch.int64)
@@ -322,9 +330,10 @@ def reduce_slots_gate(inp, slot_to_row, grad_score, topk_idx, weight):
             raise ValueError("inp must be rows like weight's, slot_to_row must have one entry per slot")
     out = torch.empty(n, d, dtype=weight.dtype, device=weight.device)
     with _on(weight.device):
-        check(_lib.load().fmoe_reduce_slots_gate(_ptr(inp), _ptr(slot_to_row if inp is not None else None), _ptr(grad_score),
-                                                 _ptr(topk_idx), _ptr(weight), _ptr(out), n, k, 0 if inp is None else inp.shape[0],
-                                                 e, d, dt, _stream(weight)))
+        lib = _lib.load()
+        call = lib.fmoe_reduce_slots_gate_any if any_grid else lib.fmoe_reduce_slots_gate
+        check(call(_ptr(inp), _ptr(slot_to_row if inp is not None else None), _ptr(grad_score), _ptr(topk_idx), _ptr(weight), _ptr(out),
+                   n, k, 0 if inp is None else inp.shape[0], e, d, dt, _stream(weight)))
     return out
 
 

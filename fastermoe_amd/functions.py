@@ -98,12 +98,12 @@ class GateLinearTopK(Function):
         grad_score = grad_score.contiguous()
         # (a backward that is to be differentiated again needs the products as torch operators)
         if (score_mode == 0 and not torch.is_grad_enabled() and _whole_chunks(x) and _whole_chunks(weight)
-                and fmoe_native.gate_grad_supported(x.shape[1], weight.shape[0], idx.shape[1], x.dtype)):
+                and fmoe_native.gate_grad_any_supported(x.shape[1], weight.shape[0], idx.shape[1], x.dtype)):
             grad_x = grad_w = grad_b = None
             if ctx.needs_input_grad[0]:
-                grad_x = fmoe_native.reduce_slots_gate(None, None, grad_score, idx, weight)
+                grad_x = fmoe_native.reduce_slots_gate(None, None, grad_score, idx, weight, any_grid=True)
             if ctx.needs_input_grad[1] or (has_bias and ctx.needs_input_grad[2]):
-                grad_w, grad_b = fmoe_native.gate_weight_grad(grad_score, idx, x, weight.shape[0], has_bias)
+                grad_w, grad_b = fmoe_native.gate_weight_grad(grad_score, idx, x, weight.shape[0], has_bias, any_grid=True)
             return grad_x, grad_w, grad_b, None, None
         g = fmoe_native.gate_topk_backward(grad_score, score, idx, weight.shape[0], score_mode)
         grad_x = g @ weight if ctx.needs_input_grad[0] else None
@@ -138,10 +138,10 @@ def gate_linear_topk(x, linear, top_k, score_mode=0):
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
         if fmoe_native.gate_linear_supported(x.shape[1], w.shape[0], top_k, x.dtype):
             return GateLinearTopK.apply(x, w, b, top_k, score_mode)
-        # more experts: the library makes the logits, their gradient still is never formed
+        # more experts, or rows off the 16-byte grid: the library makes the logits, their gradient still is never formed
         if (_plain_linear(linear) and score_mode == 0 and x.shape[0] > 0 and not torch.is_autocast_enabled()
                 and fmoe_native.gate_topk_supported(w.shape[0], top_k, x.dtype)
-                and fmoe_native.gate_grad_supported(x.shape[1], w.shape[0], top_k, x.dtype)):
+                and fmoe_native.gate_grad_any_supported(x.shape[1], w.shape[0], top_k, x.dtype)):
             return GateLinearTopK.apply(x, w, b, top_k, score_mode)
     return gate_topk(linear(x), top_k, score_mode)
 
@@ -477,7 +477,7 @@ class MOELayer(Function):
         place = fmoe_native.LayerRouting(*tensors, kept=kept)
         # (a backward that is to be differentiated again needs the gate's products as torch operators, and so do gates that the
         # kernels do not take)
-        apart = kept is not None and (torch.is_grad_enabled() or not fmoe_native.gate_grad_supported(
+        apart = kept is not None and (torch.is_grad_enabled() or not fmoe_native.gate_grad_any_supported(
             inp.shape[1], gate_w.shape[0], top_k, inp.dtype))
         new = lambda wanted, *shape: torch.empty(shape, dtype=inp.dtype, device=inp.device) if wanted else None
         (n, d), (e, h) = inp.shape, w1.shape[:2]

@@ -204,6 +204,22 @@ int fmoe_reduce_slots_gate(const void *rows, const int64_t *slot_to_row,
                            int64_t top_k, int64_t n_rows, int64_t n_expert,
                            int64_t row_elems, int dtype, void *stream);
 
+/* The same with rows of any length in 16-bit types: d_model, or row_elems, need
+ * be no whole number of 16-byte chunks; all tensors begin on 16 bytes.  Where
+ * they are whole chunks the kernels and results are those of the functions above. */
+int fmoe_gate_grad_any_supported(int64_t d_model, int64_t n_expert,
+                                 int64_t top_k, int dtype);
+int fmoe_gate_weight_grad_any(const void *grad_score, const int64_t *topk_idx,
+                          const void *x, void *grad_w, void *grad_b,
+                          int64_t n_tokens, int64_t d_model, int64_t n_expert,
+                          int64_t top_k, int dtype, void *workspace,
+                          int64_t workspace_bytes, void *stream);
+int fmoe_reduce_slots_gate_any(const void *rows, const int64_t *slot_to_row,
+                           const void *grad_score, const int64_t *topk_idx,
+                           const void *w, void *out, int64_t n_tokens,
+                           int64_t top_k, int64_t n_rows, int64_t n_expert,
+                           int64_t row_elems, int dtype, void *stream);
+
 /* Noisy top-k gating in training mode (Shazeer et al. 2017; the behaviour of
  * fmoe/gates/noisy_gate.py:113-144) after the two linear products, in one
  * pass: with std = softplus(raw) + eps and noisy = clean + noise * std (clean,
@@ -669,7 +685,7 @@ int fmoe_layer_forward(const void *x, const void *gate_w, const void *gate_b,
  * gate inside: its part included, one rounding), grad_w1 (and grad_b1), grad_w2
  * (and grad_b2); with the gate inside grad_gate_w (and grad_gate_b), else
  * grad_score [n_tokens*top_k], which is always written.  Nothing of the forward
- * is overwritten.  A gate that fmoe_gate_grad_supported does not take is
+ * is overwritten.  A gate that fmoe_gate_grad_any_supported does not take is
  * differentiated outside: FMOE_GATE_ROUTED then serves here whatever the forward
  * ran with. */
 int fmoe_layer_backward(const void *grad_out, const void *x, const void *gate_w,
