@@ -49,6 +49,10 @@ constexpr int extra_waves(int loaders) { return loaders == kLoadersCompute ? 0 :
 constexpr int waves_per_simd(int loaders, int element, int bn) { return loaders == kLoadersShared ? 4 : element == 4 && bn == 128 ? 2 : 1; }
 constexpr int kGroupM = 4;       // row tiles that share a column tile consecutively (an XCD then runs 4 x 8 tiles at a time)
 
+// Cache policy of an operand's loads: through the caches, or (nontemporal) leaving no trace in them, which whole lines that are read once
+// get from memory at 6.9 TB/s instead of 6.2.
+constexpr int kPolicyCached = 0, kPolicyOnce = 2;
+
 enum Shape { kKC = 0, kMC = 1 };
 enum Ragged { kRaggedRows = 0, kRaggedK = 1 };
 
@@ -291,6 +295,7 @@ struct GemmParams {
     int64_t dev_rows_cap;      // host only: rows the device table was laid out for
     int32_t block_m, block_n;  // host only: tile height the segment table was built for (256, 128 or 64) and tile width
     int32_t loaders;           // host only: Loaders
+    int32_t weights_once;      // host only: the column operand past the caches, see reads_weights_once() in grouped_gemm.hip
     int32_t profile_class;     // host only: ProfileClass of this launch
     double profile_work;       // host only: flop of this launch
     SegmentTable tab;
@@ -355,7 +360,8 @@ template <typename T> __device__ __forceinline__ int mc_swz(int k) {
 }
 
 // ---- the kernel ---------------------------------------------------------------
-template <typename T, int BM, int BN, int PSHAPE, int QSHAPE, int RAGGED, int EPI, int LOADERS>
+// P_POLICY: of the column operand's loads, kPolicyCached or kPolicyOnce
+template <typename T, int BM, int BN, int PSHAPE, int QSHAPE, int RAGGED, int EPI, int LOADERS, int P_POLICY>
 __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_per_simd(LOADERS, (int)sizeof(T), BN)) void grouped_gemm_kernel(const GemmParams prm) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
     constexpr int kWavesM = waves_m_of(BN), kWaves = kWavesM * kWavesN;
@@ -635,7 +641,8 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
     typedef int i32x4 __attribute__((ext_vector_type(4)));
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)smem;
     const uint32_t wave_u = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), load_wave = EXTRA ? wave_u - kWaves : wave_u;
-    auto dma_asm = [&](const T *origin, int64_t bytes, uint32_t lds_off, uint32_t voff) {
+    typedef std::integral_constant<int, kPolicyCached> Cached;
+    auto dma_asm = [&](const T *origin, int64_t bytes, uint32_t lds_off, uint32_t voff, auto policy) {
         const uint64_t a = (uint64_t)origin;
         i32x4 rs;
         rs[0] = (int)(uint32_t)a;
@@ -646,17 +653,24 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
         rs[1] = __builtin_amdgcn_readfirstlane(rs[1]);
         rs[2] = __builtin_amdgcn_readfirstlane(rs[2]);
         const uint32_t lds_addr = __builtin_amdgcn_readfirstlane(lds_base + lds_off);
-        asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                     :
-                     : "s"(lds_addr), "v"(voff), "s"(rs)
-                     : "memory", "m0");
+        if constexpr (decltype(policy)::value == kPolicyOnce) {
+            asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
+                         :
+                         : "s"(lds_addr), "v"(voff), "s"(rs)
+                         : "memory", "m0");
+        } else {
+            asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                         :
+                         : "s"(lds_addr), "v"(voff), "s"(rs)
+                         : "memory", "m0");
+        }
     };
 
     // One operand's part of the slab that starts at contraction index k0, into LDS offset
     // lds_off.  KC: the resource starts at contraction index k0 of the tile's first row and
     // the chunk is dropped when it lies past K.  MC: the resource starts at contraction row
     // k0 and is exactly as long as the rows that remain, so rows past K read as zero.
-    auto issue_part = [&](auto shape_tag, const T *tile, int64_t ld, int kc_chunk, const uint32_t *voff, auto n_tag, int k0,
+    auto issue_part = [&](auto shape_tag, const T *tile, int64_t ld, int kc_chunk, const uint32_t *voff, auto n_tag, auto policy, int k0,
                           uint32_t lds_off, int it_lo = 0, int it_hi = 1 << 20, int64_t kc_extent = (int64_t)1 << 40) {
         constexpr int SHAPE = decltype(shape_tag)::value;
         constexpr int N = decltype(n_tag)::value;
@@ -673,19 +687,20 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
         for (int it = 0; it < N; ++it) {
             if (it < it_lo || it >= it_hi) continue;
             if constexpr (kDmaAsm)
-                dma_asm(origin, bytes, lds_off + load_wave * 1024 + it * kPassBytes, voff[it] | past);
+                dma_asm(origin, bytes, lds_off + load_wave * 1024 + it * kPassBytes, voff[it] | past, policy);
             else
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(
                     rsrc, (__attribute__((address_space(3))) void *)(smem + lds_off + (EXTRA ? load_wave : (uint32_t)wave) * 1024 + it * kPassBytes), 16,
-                    voff[it] | past, 0, 0, 0);
+                    voff[it] | past, 0, 0, decltype(policy)::value);
         }
     };
     auto issue_p = [&](int k0, int buf, int it_lo = 0, int it_hi = 1 << 20) {
-        issue_part(std::integral_constant<int, PSHAPE>{}, Pb, prm.ldp, p_kc_chunk, p_voff, std::integral_constant<int, NP>{}, k0,
+        issue_part(std::integral_constant<int, PSHAPE>{}, Pb, prm.ldp, p_kc_chunk, p_voff, std::integral_constant<int, NP>{},
+                   std::integral_constant<int, P_POLICY>{}, k0,
                    (uint32_t)(buf * P_BYTES), it_lo, it_hi);
     };
     auto issue_q = [&](int k0, int buf, int it_lo = 0, int it_hi = 1 << 20) {
-        issue_part(std::integral_constant<int, QSHAPE>{}, Qb, prm.ldq, q_kc_chunk, q_voff, std::integral_constant<int, NQ>{}, k0,
+        issue_part(std::integral_constant<int, QSHAPE>{}, Qb, prm.ldq, q_kc_chunk, q_voff, std::integral_constant<int, NQ>{}, Cached{}, k0,
                    (uint32_t)(Q_BASE + buf * Q_BYTES), it_lo, it_hi, gather_q ? q_gather_bytes : (int64_t)1 << 40);
     };
 
@@ -709,7 +724,7 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
                 const int c = (t & 31) ^ (rip & 15);
                 const bool ok = row < q_valid && c * CE < p_valid;
                 const uint32_t voff = ok ? (uint32_t)(((int64_t)row * prm.ldc + c * CE) * sizeof(T)) : kOutOfRange;
-                dma_asm(aux_tile, (int64_t)kOutOfRange, lds_off + load_wave * 1024 + it * kPassBytes, voff);
+                dma_asm(aux_tile, (int64_t)kOutOfRange, lds_off + load_wave * 1024 + it * kPassBytes, voff, Cached{});
             }
         }
     };
@@ -1449,7 +1464,7 @@ __global__ __launch_bounds__(256) void split_reduce_dev_kernel(float *ws, const 
 // first use, kept until the process ends; NULL when the allocation fails, in which case nothing is split).
 float *split_workspace(hipStream_t stream, size_t bytes);
 
-template <typename T, int BM, int BN, int PS, int QS, int RG, int EPI, int LOADERS>
+template <typename T, int BM, int BN, int PS, int QS, int RG, int EPI, int LOADERS, int P_POLICY>
 int launch_tiles(GemmParams &prm, hipStream_t stream) {
     constexpr int kWavesM = waves_m_of(BN), kThreads = threads_of(BN);
     // three P and two Q slab buffers (and those of the slabs further ahead), or the epilogue's staging area (one [rows][row piece + 16 B] block per wave)
@@ -1462,7 +1477,7 @@ int launch_tiles(GemmParams &prm, hipStream_t stream) {
     // the opt-in to more than 64 KiB of dynamic LDS is per device (and per kernel instantiation)
     // (0: not tried yet, 1: done, 2: failed -- a failure is reported by every later launch too)
     static std::atomic<int> configured[16];
-    auto kern = grouped_gemm_kernel<T, BM, BN, PS, QS, RG, EPI, LOADERS>;
+    auto kern = grouped_gemm_kernel<T, BM, BN, PS, QS, RG, EPI, LOADERS, P_POLICY>;
     int dev = 0;
     FMOE_HIP_CHECK(hipGetDevice(&dev));
     FMOE_REQUIRE(dev >= 0 && dev < 16, "device index %d out of range", dev);
@@ -1547,7 +1562,7 @@ int launch_tiles(GemmParams &prm, hipStream_t stream) {
 // 128 x 256, 128 x 128, 64 x 128; fp32: 128 x 128, 64 x 64; chosen by the host from the segment lengths) is the tile.
 // EPI_MASK lists the epilogues a product can be asked for, so that only those kernels
 // are built.
-template <typename T, int BM, int BN, int PS, int QS, int RG, int EPI_MASK, int LOADERS = kLoadersCompute>
+template <typename T, int BM, int BN, int PS, int QS, int RG, int EPI_MASK, int LOADERS = kLoadersCompute, int P_POLICY = kPolicyCached>
 int launch_for_height(GemmParams &prm, int epi, hipStream_t stream) {
     prm.tiles_n = (int)ceil_div(prm.n_cols, BN);
     int64_t total;
@@ -1566,12 +1581,23 @@ int launch_for_height(GemmParams &prm, int epi, hipStream_t stream) {
     if (total > (int64_t)INT32_MAX - 8) return fail(FMOE_ELIMIT, "grouped GEMM: %lld tiles exceed the grid limit", (long long)total);
     prm.total_tiles = (int)total;
     if constexpr ((EPI_MASK >> kEpiStore) & 1)
-        if (epi == kEpiStore) return launch_tiles<T, BM, BN, PS, QS, RG, kEpiStore, LOADERS>(prm, stream);
+        if (epi == kEpiStore) return launch_tiles<T, BM, BN, PS, QS, RG, kEpiStore, LOADERS, P_POLICY>(prm, stream);
     if constexpr ((EPI_MASK >> kEpiBiasAct) & 1)
-        if (epi == kEpiBiasAct) return launch_tiles<T, BM, BN, PS, QS, RG, kEpiBiasAct, LOADERS>(prm, stream);
+        if (epi == kEpiBiasAct) return launch_tiles<T, BM, BN, PS, QS, RG, kEpiBiasAct, LOADERS, P_POLICY>(prm, stream);
     if constexpr ((EPI_MASK >> kEpiDAct) & 1)
-        if (epi == kEpiDAct) return launch_tiles<T, BM, BN, PS, QS, RG, kEpiDAct, LOADERS>(prm, stream);
+        if (epi == kEpiDAct) return launch_tiles<T, BM, BN, PS, QS, RG, kEpiDAct, LOADERS, P_POLICY>(prm, stream);
     return fail(FMOE_EINVAL, "epilogue %d is not built for this product", epi);
+}
+
+// the row-ragged shapes of 16-bit types
+template <typename T, int PS, int QS, int EPI_MASK, int P_POLICY> int launch_16bit_rows(GemmParams &prm, int epi, hipStream_t stream) {
+    if (prm.block_n == 128) {
+        if (prm.block_m == 64) return launch_for_height<T, 64, 128, PS, QS, kRaggedRows, EPI_MASK, kLoadersAlone, P_POLICY>(prm, epi, stream);
+        return prm.loaders == kLoadersAlone ? launch_for_height<T, 128, 128, PS, QS, kRaggedRows, EPI_MASK, kLoadersAlone, P_POLICY>(prm, epi, stream)
+                                            : launch_for_height<T, 128, 128, PS, QS, kRaggedRows, EPI_MASK, kLoadersShared, P_POLICY>(prm, epi, stream);
+    }
+    if (prm.block_m == 128) return launch_for_height<T, 128, 256, PS, QS, kRaggedRows, EPI_MASK, kLoadersCompute, P_POLICY>(prm, epi, stream);
+    return launch_for_height<T, 256, 256, PS, QS, kRaggedRows, EPI_MASK, kLoadersCompute, P_POLICY>(prm, epi, stream);
 }
 
 template <typename T, int PS, int QS, int RG, int EPI_MASK>
@@ -1582,16 +1608,19 @@ int launch_by_epilogue(GemmParams &prm, int epi, hipStream_t stream) {
             if (prm.loaders == kLoadersAlone) return launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK, kLoadersAlone>(prm, epi, stream);
         return launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK>(prm, epi, stream);
     } else {
+    const bool built = (prm.block_m == 64 && prm.block_n == 128) || ((prm.block_m == 128 || prm.block_m == 256) && prm.block_n == 256) ||
+                       (prm.block_m == 128 && prm.block_n == 128);
     if constexpr (RG == kRaggedRows)
-        if (prm.block_n == 128) {
-            if (prm.block_m == 64) return launch_for_height<T, 64, 128, PS, QS, RG, EPI_MASK, kLoadersAlone>(prm, epi, stream);
-            return prm.loaders == kLoadersAlone ? launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK, kLoadersAlone>(prm, epi, stream)
-                                                : launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK, kLoadersShared>(prm, epi, stream);
+        if (built) {
+            return prm.weights_once ? launch_16bit_rows<T, PS, QS, EPI_MASK, kPolicyOnce>(prm, epi, stream)
+                                    : launch_16bit_rows<T, PS, QS, EPI_MASK, kPolicyCached>(prm, epi, stream);
         }
     if constexpr (RG == kRaggedK)
         if (prm.block_m == 128 && prm.block_n == 128) return launch_for_height<T, 128, 128, PS, QS, RG, EPI_MASK>(prm, epi, stream);
-    if (prm.block_m == 128 && prm.block_n == 256) return launch_for_height<T, 128, 256, PS, QS, RG, EPI_MASK>(prm, epi, stream);
-    if (prm.block_m == 256 && prm.block_n == 256) return launch_for_height<T, 256, 256, PS, QS, RG, EPI_MASK>(prm, epi, stream);
+    if constexpr (RG == kRaggedK) {
+        if (prm.block_m == 128 && prm.block_n == 256) return launch_for_height<T, 128, 256, PS, QS, RG, EPI_MASK>(prm, epi, stream);
+        if (prm.block_m == 256 && prm.block_n == 256) return launch_for_height<T, 256, 256, PS, QS, RG, EPI_MASK>(prm, epi, stream);
+    }
     return fail(FMOE_EINVAL, "tile %d x %d is not built", prm.block_m, prm.block_n);
     }
 }

@@ -1,0 +1,30 @@
+"""Products over a device table whose weights are read past the caches, where the average expert has one row tile."""
+import pytest
+import torch
+
+from fastermoe_amd import _lib, fmoe_native
+
+pytestmark = pytest.mark.gpu
+
+
+# on both sides of the line, which lies at 6/7 of a tile's height (64, 128 or 256 rows), ragged and skewed counts
+@pytest.mark.parametrize("tile", ["64x128", "128x128", "128x128+", "128x256", "256x256"])
+@pytest.mark.parametrize("counts", [[3, 0, 40, 17], [300, 1, 0, 2], [108, 110, 109, 110], [219, 219, 219, 220], [256, 255, 257, 300]])
+@pytest.mark.parametrize("k,n", [(64, 256), (200, 136)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_results_are_those_of_the_host_counts(tile, counts, k, n, dtype, device, monkeypatch):
+    """Where a load leaves traces makes no difference to what it reads: bit for bit the launch from host counts, which reads through the caches."""
+    monkeypatch.setenv("FMOE_GEMM_TILE", tile)
+    e, rows = len(counts), sum(counts)
+    g = torch.Generator().manual_seed(k + rows)
+    x = torch.randn(rows, k, generator=g).to(dtype).to(device)
+    w = (torch.randn(e, n, k, generator=g) / k ** 0.5).to(dtype).to(device)
+    b = torch.randn(e, n, generator=g).to(dtype).to(device)
+    gy = torch.randn(rows, n, generator=g).to(dtype).to(device)
+    host = torch.tensor(counts)
+    table = fmoe_native.segment_table(host.to(device), rows)
+    y, pre = fmoe_native.linear_forward_dev(x, w, b, table, rows, _lib.ACT_GELU, True)
+    ref, ref_pre = fmoe_native.linear_act_forward(x, host, w, b, _lib.ACT_GELU)
+    assert torch.equal(y, ref) and torch.equal(pre, ref_pre)
+    gx = fmoe_native.linear_dgrad_dev(gy, w, table, rows)
+    assert torch.equal(gx, fmoe_native.linear_backward(gy, x, host, w, b)[0])
