@@ -127,6 +127,28 @@ def load():
     return lib
 
 
+_layer_call = None
+
+
+def load_layer_call():
+    """The extension module ``fastermoe_amd/lib/_layer_call.so``, which calls the library's layer from Python's tensors."""
+    global _layer_call
+    if _layer_call is None:
+        path = os.path.join(_HERE, "lib", "_layer_call.so")
+        if not os.path.exists(path):
+            raise ImportError(f"{path} is missing: the host extension has not been built (run `python -m fastermoe_amd.build`)")
+        import importlib.machinery
+        import importlib.util
+        import torch  # noqa: F401  (its libraries have to be there first)
+        lib = load()
+        loader = importlib.machinery.ExtensionFileLoader("_layer_call", path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_layer_call", loader))
+        loader.exec_module(module)
+        module.bind(*(ctypes.cast(fn, _vp).value for fn in (lib.fmoe_layer_sizes, lib.fmoe_layer_forward)))
+        _layer_call = module
+    return _layer_call
+
+
 class FmoeHipError(RuntimeError):
     pass
 

@@ -9,12 +9,14 @@ by side.
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "lib", "libfmoe_hip.so")
+LAYER_CALL = os.path.join(HERE, "lib", "_layer_call.so")   # host code over torch's tensors
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
@@ -54,6 +56,17 @@ def _compile(unit):
     return proc.returncode, obj, log
 
 
+def _build_layer_call():
+    """The extension module of csrc/layer_call.cpp."""
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{sysconfig.get_path('include')}", *(f"-I{p}" for p in include_paths()), os.path.join(CSRC, "layer_call.cpp"), "-o", LAYER_CALL,
+           *(f"-L{p}" for p in library_paths()), "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10"]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    return proc.returncode, "_layer_call.so", proc.stdout
+
+
 def build(jobs=None, verbose=False):
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(os.path.dirname(LIB), exist_ok=True)
@@ -61,7 +74,8 @@ def build(jobs=None, verbose=False):
     jobs = jobs or min(8, os.cpu_count() or 1)
     failed = False
     with ThreadPoolExecutor(max_workers=jobs) as pool:
-        for rc, obj, log in pool.map(_compile, units):
+        host = pool.submit(_build_layer_call)
+        for rc, obj, log in [*pool.map(_compile, units), host.result()]:
             if log.strip() and (verbose or rc != 0):
                 print(f"--- {obj}\n{log}", file=sys.stderr)
             failed |= rc != 0

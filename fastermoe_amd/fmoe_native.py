@@ -796,6 +796,17 @@ def linear_wgrad_dev(grad_y, x, weight, table, rows_cap, with_bias):
 
 # ---- a whole layer pass in one call ----------------------------------------------------
 
+def layer_infer(inp, gate_w, gate_b, score, routing, w1, b1, w2, b2, top_k, activation, gate):
+    """The layer's output where nothing will be differentiated (``routing``: ``pos_buf``, ``slot_to_row`` and the segment table of a gate
+    outside, whose scores ``score`` are), or ``None`` where the call does not take these tensors."""
+    pos, slot_to_row, table = routing if routing is not None else (None, None, None)
+    with _on(inp.device):
+        out = _lib.load_layer_call().infer(inp, gate_w, gate_b, score, pos, slot_to_row, table, w1, b1, w2, b2, top_k, activation, gate, _stream(inp))
+    if type(out) is int:
+        check(out)
+    return out
+
+
 def layer_sizes(n_tokens, d_model, d_hidden, n_expert, top_k, dtype, activation, keep, gate):
     """``(scratch bytes of a forward, of a backward, segment table bytes)`` of :func:`layer_forward` for these sizes,
     or ``None`` where it does not take them (or one of the switches that keep the steps of a layer apart is set)."""
@@ -841,24 +852,22 @@ class LayerRouting:
                 self.kept[score_at:score_at + n * dtype.itemsize].view(dtype).view(n_tokens, top_k))
 
 
-def layer_forward(inp, gate_w, gate_b, logits, w1, b1, w2, b2, top_k, activation, keep, gate, sizes, routing):
+def layer_forward(inp, gate_w, gate_b, logits, w1, b1, w2, b2, top_k, activation, gate, sizes, routing):
     """Gate, routing, experts and combine as one call, over tensors that the caller has checked against
     :func:`layer_sizes` (contiguous, on 16 bytes, one type and device).  Returns ``(out, pre, mid, rows)``, the last three
-    ``None`` unless ``keep``."""
+    for the backward (``pre`` ``None`` where ``mid`` tells as much)."""
     n, d = inp.shape
     e, h = w1.shape[:2]
     new = lambda r, c: torch.empty(r, c, dtype=inp.dtype, device=inp.device)
     out = new(n, d)
-    pre = mid = rows = None
-    if keep:
-        pre = new(n * top_k, h) if activation == _lib.ACT_GELU else None
-        mid, rows = new(n * top_k, h), new(n * top_k, d)
+    pre = new(n * top_k, h) if activation == _lib.ACT_GELU else None
+    mid, rows = new(n * top_k, h), new(n * top_k, d)
     scratch = torch.empty(sizes[0], dtype=torch.uint8, device=inp.device)
     idx, score, pos, s2r, table = routing.pointers(n * top_k, sizes[2])
     with _on(inp.device):
         check(_lib.load().fmoe_layer_forward(
             inp.data_ptr(), _ptr(gate_w), _ptr(gate_b), _ptr(logits), w1.data_ptr(), _ptr(b1), w2.data_ptr(), _ptr(b2), idx, score, pos,
-            s2r, table, _ptr(pre), _ptr(mid), _ptr(rows), out.data_ptr(), n, d, h, e, top_k, _DTYPES[inp.dtype], activation, keep, gate,
+            s2r, table, _ptr(pre), mid.data_ptr(), rows.data_ptr(), out.data_ptr(), n, d, h, e, top_k, _DTYPES[inp.dtype], activation, 1, gate,
             scratch.data_ptr(), sizes[0], _stream(inp)))
     return out, pre, mid, rows
 
