@@ -359,6 +359,54 @@ template <typename T> __device__ __forceinline__ int mc_swz(int k) {
     return sizeof(T) == 2 ? ((k & 3) << 2) | (((k >> 3) & 1) << 1) : 0;
 }
 
+// The row tiles of a device table of 128-row tiles apart: those of more than 64 rows, in their order, and the low ones, at most one
+// for each expert.  Low tiles go last, so that they are the second ones of their compute units: the first workgroups of an XCD get
+// a unit each, and with the table's order the second ones are as often as not full tiles, for which the launch
+// then waits (8 experts of 1024 -> 512, about 1024 rows each: 84 us in the table's order, low tiles or not; 71 with the low ones last).
+// Lane i holds experts i, 64 + i, ..; all of it is read in one go, where the map of tiles has to wait for their number.
+struct LowTiles {
+    static constexpr int kChunks = 4, kMaxExperts = 64 * kChunks;
+    int first[kChunks], rows[kChunks], before[kChunks], low_before[kChunks];   // per expert: first row, rows, full and low tiles before
+    int n_low;
+    static __device__ __forceinline__ bool is_low(int rows) { return (rows & 127) != 0 && (rows & 127) <= 64; }
+    __device__ __forceinline__ void read(const int32_t *tab, int n_expert) {
+        const int lane = threadIdx.x & 63;
+        const int32_t *seg = tab + segtab::seg_off(), *pfx = tab + segtab::pfx128_off(n_expert);
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) {
+            const int e = c * 64 + lane;
+            first[c] = e < n_expert ? seg[e] : 0;
+            rows[c] = e < n_expert ? seg[e + 1] - first[c] : 0;
+            before[c] = e < n_expert ? pfx[e] : 0;
+        }
+        n_low = 0;
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) {
+            const uint64_t low = __builtin_amdgcn_ballot_w64(is_low(rows[c]));
+            low_before[c] = n_low + __popcll(low & ((1ull << lane) - 1));
+            before[c] -= low_before[c];
+            n_low += __popcll(low);
+        }
+    }
+    // expert and rows of full or low row tile t
+    __device__ __forceinline__ void find(bool from_low, int t, int &expert, int &row_lo, int &row_hi) const {
+        expert = row_lo = row_hi = 0;
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) {
+            const bool low = is_low(rows[c]);
+            const int n_full = (rows[c] + 127) / 128 - low;
+            const uint64_t hit = __builtin_amdgcn_ballot_w64(from_low ? low && low_before[c] == t : t >= before[c] && t < before[c] + n_full);
+            if (hit != 0) {
+                const int lane = __builtin_ctzll(hit);
+                const int lo = __builtin_amdgcn_readlane(first[c], lane), n = __builtin_amdgcn_readlane(rows[c], lane);
+                expert = c * 64 + lane;
+                row_lo = lo + (from_low ? n & ~127 : (t - __builtin_amdgcn_readlane(before[c], lane)) * 128);
+                row_hi = min(lo + n, row_lo + 128);
+            }
+        }
+    }
+};
+
 // ---- the kernel ---------------------------------------------------------------
 // P_POLICY: of the column operand's loads, kPolicyCached or kPolicyOnce
 template <typename T, int BM, int BN, int PSHAPE, int QSHAPE, int RAGGED, int EPI, int LOADERS, int P_POLICY>
@@ -381,6 +429,8 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
     constexpr int NQ = BM * 8 / kLoaders;
     constexpr int P_BYTES = BN * kSlabBytes, Q_BYTES = BM * kSlabBytes;
     constexpr int kAhead = ahead_of(LOADERS);        // slabs requested beyond two
+    // fp32 row-ragged tiles of at most half their rows: see low_tile_loop
+    constexpr bool kLowTiles = kSplit && RAGGED == kRaggedRows && TI == 2;
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
@@ -399,6 +449,8 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
     const DevTab dtab = (DevTab)(uintptr_t)prm.dev_tab;
     const bool dev = prm.dev_tab != nullptr;
     int seg_lo, seg_hi;
+    LowTiles low_tiles;
+    bool low_last = false, from_low = false;
     {
         int tm_total, rem;
         if (RAGGED == kRaggedRows) {
@@ -417,7 +469,21 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
                 tm_total = prm.tab.tile[prm.tab.n];
             }
             const int main_grid = (main_tiles + 7) & ~7;
-            if (fixup) {
+            low_last = kLowTiles && dev && k_split == 1 && !fixup && prm.tab.n <= LowTiles::kMaxExperts;
+            if (low_last) {
+                if constexpr (kLowTiles) {
+                    low_tiles.read(prm.dev_tab, prm.tab.n);
+                    // an equal number of full ones to each XCD, and low ones up to an equal number of all
+                    const int per_xcd = main_grid >> 3, xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
+                    if (i >= per_xcd) return;
+                    const int full = (tm_total - low_tiles.n_low) * prm.tiles_n, share = (full + 7) >> 3;
+                    const int first = min(full, xcd * share), n_full = min(full, (xcd + 1) * share) - first;
+                    from_low = i >= n_full;
+                    L = from_low ? xcd * per_xcd - first + i - n_full : first + i;
+                    if (from_low && L >= total_tiles - full) return;
+                    tm_total = from_low ? low_tiles.n_low : tm_total - low_tiles.n_low;
+                }
+            } else if (fixup) {
                 tail_index = blockIdx.x / kWaves;  // one one-wave workgroup per wave of a tail tile
                 // (device table: the launch was sized for the most tail tiles there can be)
                 if (dev && (k_split == 1 || tail_index >= total_tiles - main_tiles)) return;
@@ -452,7 +518,9 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
         mt = first_m + in_grp % gsz;
         nt = in_grp / gsz;
         if (RAGGED == kRaggedRows) {
-            if (dev) {
+            if (kLowTiles && low_last) {
+                low_tiles.find(from_low, mt, ei, seg_lo, seg_hi);
+            } else if (dev) {
                 // {expert, first row, rows} of row tile mt
                 // (the map's offset is known to the host, so this load waits for the tile count only)
                 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -530,7 +598,14 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
     // a fixup launch runs one wave per workgroup; it stands in for wave blockIdx.x % kWaves of the tile's workgroup
     const int lane = t & 63, wave = fixup ? (int)(blockIdx.x % kWaves) : t >> 6;
     const int lb = lane & (MB - 1), hq = lane / MB;  // row inside an MFMA block, contraction chunk inside a step
-    const int wave_m0 = (wave / kWavesN) * WM, wave_n0 = (wave % kWavesN) * WN;
+    int wave_m0 = (wave / kWavesN) * WM, wave_n0 = (wave % kWavesN) * WN;
+    int wave_n_end = BN;   // columns of the tile from here on are not this wave's
+    const bool low_tile = kLowTiles && q_valid <= BM / 2 && split_part < 0 && !fixup;
+    if (low_tile) {
+        wave_m0 = 0;
+        wave_n0 = wave * MB;
+        wave_n_end = wave_n0 + MB;
+    }
 
     // An expert without rows has a zero weight gradient (and bias gradient): write the
     // tile with plain coalesced stores and skip the whole pipeline.
@@ -941,7 +1016,7 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    auto main_loop = [&](auto with_bias, auto loads_tag, auto exact) {
+    auto main_loop = [&](auto with_bias, auto loads_tag, auto exact) __attribute__((always_inline)) {
         constexpr bool kBias = decltype(with_bias)::value;
         constexpr bool kLoads = decltype(loads_tag)::value;  // this wave requests slabs
         constexpr int kNoWait = 63;
@@ -1038,6 +1113,90 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
         wait_loads(std::integral_constant<int, 0>{});
         slab_barrier();
     };
+    // The same for a tile of at most 64 rows, the remainder of an expert's rows.  Laid out like a full one, half the
+    // waves would work on rows that are not there while the others take as long as in a full tile; here each wave has all
+    // rows (NY blocks of 32) of a quarter of the columns, acc[0], and the same order of products per element.
+    // A slab is two phases of one contraction step each.
+    // Bound by its chain of LDS reads, parts and products: 0.7 us per slab alone on a unit, where a full tile takes 1.6.  8192 rows of 8
+    // experts of 512 x 1024, four of them 6 to 36 rows past 1024 (272 tiles of 32 slabs on 256 units), with the order of
+    // LowTiles: data gradient and second product 84 -> 71 us, the first (16 slabs) 71 -> 64; 55 where all have 1024.
+    auto low_tile_loop = [&](auto rows_tag, auto loads_tag) __attribute__((always_inline)) {
+        if constexpr (kLowTiles) {
+            constexpr int NY = decltype(rows_tag)::value, kProducts = 6 * NY, kFrags = NY + 1, kStages = kFrags * kSplitStages;
+            constexpr bool kLoads = decltype(loads_tag)::value;
+            constexpr int kQLoads = NY;   // (each brings 32 rows; the others nothing but zeros)
+            static_assert(QSHAPE == kKC && kRowsPerPass == MB, "a load for each block of rows");
+            constexpr int kFrom = kProducts / 4, kSpan = kProducts - kFrom;
+            static_assert(NP <= kProducts && kQLoads <= kProducts && kFrags <= kProducts, "one load and one fragment per product");
+            auto fetch = [&](auto ks_tag, int f, const unsigned char *sp, const unsigned char *sq) {
+                constexpr int ks = decltype(ks_tag)::value;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if (f < NY) qf[ks][f].c[h] = frag(sq, QSHAPE, BM, f * MB, 2 * ks + h);
+                    else pf[ks][0].c[h] = frag(sp, PSHAPE, BN, wave_n0, 2 * ks + h);
+                }
+            };
+            auto take_apart = [&](auto ks_tag, int f, int stage) {
+                constexpr int ks = decltype(ks_tag)::value;
+                Split8 &parts = f < NY ? q_parts[ks][f] : p_parts[ks][0];
+                if (stage == kSplitStages - 1) {
+                    uint32_t &seen = f < NY ? q_seen[f] : p_seen[0];
+                    seen |= parts.hi[0] | parts.hi[1];
+                    seen |= parts.hi[2] | parts.hi[3];
+                }
+                split_stage(stage, f < NY ? qf[ks][f] : pf[ks][0], parts);
+            };
+            // products of contraction step ks, reads of the other one from sp and sq, load(i) after product i
+            auto phase = [&](auto ks_tag, const unsigned char *sp, const unsigned char *sq, auto load) {
+                constexpr int ks = decltype(ks_tag)::value;
+                std::integral_constant<int, 1 - ks> next;
+                for_each_index<kProducts>([&](auto mfma) {
+                    constexpr int i = decltype(mfma)::value, y = i % NY, product = i / NY;
+                    if constexpr (i < kFrags) fetch(next, i, sp, sq);
+                    mma_part(product, product == 5 ? acc[0][y] : low[0][y], p_parts[ks][0], q_parts[ks][y]);
+                    load(i);
+                    constexpr int from = i <= kFrom ? 0 : ((i - kFrom) * kStages + kSpan - 1) / kSpan;
+                    constexpr int to = i < kFrom ? 0 : ((i + 1 - kFrom) * kStages + kSpan - 1) / kSpan;
+                    for_each_index<to - from>([&](auto c) { take_apart(next, (from + c) % kFrags, (from + c) / kFrags); });
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+            };
+            const std::integral_constant<int, 0> step0;
+            const std::integral_constant<int, 1> step1;
+            if constexpr (kLoads) {
+#pragma unroll
+                for (int s = 0; s < 2 + kAhead; ++s) {
+                    issue_p(s * BKE, s);
+                    issue_q(s * BKE, s, 0, kQLoads);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            wait_loads(std::integral_constant<int, kLoads ? (1 + kAhead) * (NP + kQLoads) : 63>{});
+            slab_barrier();
+#pragma unroll
+            for (int f = 0; f < kFrags; ++f) fetch(step0, f, smem, smem + Q_BASE);
+#pragma unroll
+            for (int c = 0; c < kStages; ++c) take_apart(step0, c % kFrags, c / kFrags);
+            __builtin_amdgcn_sched_barrier(0);
+            int pc = 0, qc = 0;
+            for (int s = 0; s < n_slabs; ++s) {
+                const int pn = pc == kPBufs - 1 ? 0 : pc + 1, qn = qc == kQBufs - 1 ? 0 : qc + 1;
+                const int pf_buf = kAhead == 0 ? (pn == kPBufs - 1 ? 0 : pn + 1) : (pc == 0 ? kPBufs - 1 : pc - 1);
+                phase(step0, smem + pc * P_BYTES, smem + Q_BASE + qc * Q_BYTES, [&](int i) {
+                    if (kLoads && i < NP) issue_p((s + 2 + kAhead) * BKE, pf_buf, i, i + 1);
+                });
+                wait_loads(std::integral_constant<int, kLoads ? NP + kAhead * (NP + kQLoads) : 63>{});
+                slab_barrier();
+                phase(step1, smem + pn * P_BYTES, smem + Q_BASE + qn * Q_BYTES, [&](int i) {
+                    if (kLoads && i < kQLoads) issue_q((s + 2 + kAhead) * BKE, qc, i, i + 1);
+                });
+                pc = pn;
+                qc = qn;
+            }
+            wait_loads(std::integral_constant<int, 0>{});
+            slab_barrier();
+        }
+    };
     // The same slabs and barriers for a wave that only loads.  Where a launch leaves a compute unit one workgroup of four waves, a
     // wave's loads (35 ns each, during which it issues nothing else), its LDS reads and its products follow one another;
     // apart they overlap, and with the LDS of a whole unit four slabs are on their way.
@@ -1061,7 +1220,7 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
         wait_loads(std::integral_constant<int, 0>{});
         slab_barrier();
     };
-    auto run_loop = [&](auto with_bias, auto exact) {
+    auto run_loop = [&](auto with_bias, auto exact) __attribute__((always_inline)) {
         if constexpr (EXTRA > 0) {
             main_loop(with_bias, std::false_type{}, exact);
             return;
@@ -1095,7 +1254,14 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
         if (want_bias) run_loop(std::true_type{}, std::false_type{});
         else run_loop(std::false_type{}, std::false_type{});
     } else {
-        if (!fixup) run_loop(std::false_type{}, std::false_type{});
+        if constexpr (kLowTiles) {
+            const std::integral_constant<bool, EXTRA == 0> loads;   // (all four waves, or others)
+            if (low_tile && q_valid <= MB) low_tile_loop(std::integral_constant<int, 1>{}, loads);
+            else if (low_tile) low_tile_loop(std::integral_constant<int, 2>{}, loads);
+            else if (!fixup) run_loop(std::false_type{}, std::false_type{});
+        } else {
+            if (!fixup) run_loop(std::false_type{}, std::false_type{});
+        }
     }
     if constexpr (kSplit) {
         // a tile with a NaN, an infinity or a row of tiny elements once more, as the fp32 MFMA has it (the bias gradient's sums come from the
@@ -1129,6 +1295,11 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
                     for (int y = 0; y < TJ; ++y)
 #pragma unroll
                         for (int r = 0; r < kAccRegs; ++r) acc[x][y][r] = 0.f;
+                if (low_tile) {   // (as a full tile)
+                    wave_m0 = (wave / kWavesN) * WM;
+                    wave_n0 = (wave % kWavesN) * WN;
+                    wave_n_end = BN;
+                }
                 run_loop(std::false_type{}, std::true_type{});
             }
         }
@@ -1236,7 +1407,7 @@ __global__ __launch_bounds__(threads_of(BN) + 64 * extra_waves(LOADERS), waves_p
     constexpr int kIoSteps = WM / kIoRows, kIoBatch = kIoSteps < 8 ? kIoSteps : 8;
     static_assert(kIoSteps % kIoBatch == 0, "row groups of a wave's sub-tile come in whole batches");
     auto tile_offset = [&](int r, int col_base) -> uint32_t {
-        return (wave_m0 + r < q_valid && col_base + io_c * CE < p_valid)
+        return (wave_m0 + r < q_valid && col_base + io_c * CE < min(p_valid, wave_n_end))
                    ? (uint32_t)(((int64_t)(wave_m0 + r) * prm.ldc + col_base + io_c * CE) * (int64_t)sizeof(T))
                    : kOutOfRange;
     };
