@@ -423,8 +423,12 @@ bool use_skinny(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out
 // 3328 -> 3328, 96, a fifth of the rows one's: 204 / 183; 32 of 2048 -> 4096, 106: 164 / 152; 16 of 2560 -> 2560, 216 (tiles of 256): 80 / 73; past
 // the line 128 of 1664 -> 832, 136 (tiles of 128): 136 / 151; 12 of 3328 -> 960, 264: 53 / 66; 4 of 4352 -> 1088, 320: 35 / 40.  (The
 // persistent kernel's launches have more row tiles: all their weights past the caches cost 64 experts with shares 1 / rank^1.2 of 16384 rows 7 %.)
-bool reads_weights_once(const TileShape &tile, int64_t rows_cap, int64_t n_expert, int dtype) {
-    return is_16bit(dtype) && rows_cap * 7 <= n_expert * tile.bm * 6;
+// Weights that the memory-side cache (256 MiB) can hold together with the layer's other linear stay as they were: loads past the caches
+// drop them from it, and the next product that reads them waits for memory (16 experts of 768 x 3072, 2000 rows, a training step
+// after another: forward of the second linear 24.6 us, 37.9 after a data gradient that read past the caches and took no less time itself).
+constexpr int64_t kHeldWeightBytes = (int64_t)128 << 20;
+bool reads_weights_once(const TileShape &tile, int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out_feat, int dtype) {
+    return is_16bit(dtype) && rows_cap * 7 <= n_expert * tile.bm * 6 && n_expert * in_feat * out_feat * 2 > kHeldWeightBytes;
 }
 
 // The kernel of a row-ragged launch over a device table, and the workspace it can make use of.
@@ -592,7 +596,7 @@ int grouped_linear_forward(const LinearForwardArgs &a, const int64_t *counts, in
                                         : forward_route(a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype, a.epilogue, prm.activation,
                                                         a.aux != nullptr, a.x_row_index != nullptr);
         prm.block_m = route.tile.bm; prm.block_n = route.tile.bn; prm.loaders = route.tile.loaders;
-        prm.weights_once = fast && reads_weights_once(route.tile, a.dev_rows_cap, n_expert, a.dtype);
+        prm.weights_once = fast && reads_weights_once(route.tile, a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype);
         prm.profile_class = kProfGemmFwd; prm.profile_work = 2.0 * (double)a.dev_rows_cap * (double)a.in_feat * (double)a.out_feat;
         prm.P = a.w; prm.Q = a.x; prm.C = a.y; prm.bias = a.bias; prm.aux = a.aux;
         prm.q_row_index = a.x_row_index; set_row_index_divisor(prm, a.x_index_div); prm.q_total_rows = a.x_total_rows;
@@ -660,7 +664,7 @@ int grouped_linear_dgrad(const LinearDgradArgs &a, const int64_t *counts, int64_
         const DevRoute route = any_grid ? DevRoute{DevKernel::kTiles, unaligned_tile_estimate(a.dev_rows_cap, n_expert, a.in_feat)}
                                         : dgrad_route(a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype, a.epilogue, prm.activation);
         prm.block_m = route.tile.bm; prm.block_n = route.tile.bn; prm.loaders = route.tile.loaders;
-        prm.weights_once = fast && reads_weights_once(route.tile, a.dev_rows_cap, n_expert, a.dtype);
+        prm.weights_once = fast && reads_weights_once(route.tile, a.dev_rows_cap, n_expert, a.in_feat, a.out_feat, a.dtype);
         prm.profile_class = kProfGemmDgrad; prm.profile_work = 2.0 * (double)a.dev_rows_cap * (double)a.in_feat * (double)a.out_feat;
         prm.P = a.w; prm.Q = a.gy; prm.C = a.gx; prm.aux = const_cast<void *>(a.aux);
         prm.ldp = a.in_feat; prm.ldq = a.out_feat; prm.ldc = a.in_feat;

@@ -7,6 +7,31 @@ from fastermoe_amd import _lib, fmoe_native
 pytestmark = pytest.mark.gpu
 
 
+def operands(counts, k, n, dtype, device):
+    rows = sum(counts)
+    g = torch.Generator(device=device).manual_seed(k + rows)
+    new = lambda *s: torch.randn(*s, generator=g, device=device).to(dtype)
+    return new(rows, k), new(len(counts), n, k) / k ** 0.5, new(len(counts), n), new(rows, n)
+
+
+# (loads past the caches begin at weights of 128 MiB; the smaller ones stay in the caches on either side of the line)
+@pytest.mark.parametrize("tile", ["64x128", "128x128", "128x128+", "128x256", "256x256"])
+@pytest.mark.parametrize("counts", [[3, 0, 40, 17], [49, 50, 1, 0], [219, 219, 219, 220]])
+def test_results_with_large_weights(tile, counts, device, monkeypatch):
+    monkeypatch.setenv("FMOE_GEMM_TILE", tile)
+    k, n = 4104, 4168
+    x, w, b, gy = operands(counts, k, n, torch.bfloat16, device)
+    assert w.numel() * 2 > 128 << 20
+    host = torch.tensor(counts)
+    table = fmoe_native.segment_table(host.to(device), sum(counts))
+    y, pre = fmoe_native.linear_forward_dev(x, w, b, table, sum(counts), _lib.ACT_GELU, True)
+    ref, ref_pre = fmoe_native.linear_act_forward(x, host, w, b, _lib.ACT_GELU)
+    gx, ref_gx = fmoe_native.linear_dgrad_dev(gy, w, table, sum(counts)), fmoe_native.linear_backward(gy, x, host, w, b)[0]
+    # (the host's launches may split a tail's contraction: its terms in another order, 4168 roundings of 2^-24 at most, and one of 2^-8)
+    for got, want in ((pre, ref_pre), (y, ref), (gx, ref_gx)):
+        assert (got.float() - want.float()).norm() <= 2.0 ** -8 * want.float().norm()
+
+
 # on both sides of the line, which lies at 6/7 of a tile's height (64, 128 or 256 rows), ragged and skewed counts
 @pytest.mark.parametrize("tile", ["64x128", "128x128", "128x128+", "128x256", "256x256"])
 @pytest.mark.parametrize("counts", [[3, 0, 40, 17], [300, 1, 0, 2], [108, 110, 109, 110], [219, 219, 219, 220], [256, 255, 257, 300]])
