@@ -32,6 +32,10 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 // (27.9 / 25.5 / 26.7, 23.5), 16384 of 4096, top-4: 55 / 54 / 64; float32, 32768 of 4096, top-2: 115 / 87 / 81, top-4 at 16384:
 // 87 / 71 / 84.  As a library product over the dense gradient the first took 99.
 // Tokens or rows too few for that many waves take P = 1.
+// More than two slots: 16-bit types two at a time, so that seven or eight waves fit a SIMD where the loads of all slots and pieces at once leave four
+// (top-8, 8192 tokens of 2048, 256 experts: 71.7 -> 56.4 us, 32768 of 512: 72.0 -> 58.2; top-4, 16384 of 4096: 120.5 -> 113.4, 8192 of
+// 1024: 17.8 either way; the order of the sums is the same).  float32 as many as there are, whose rows are twice the bytes for the same sums (8192 of
+// 2048, top-8: 103.4, two at a time 107.3).
 // ANY (16-bit types): rows of any length, read 16 bytes at a time wherever they lie; row_vecs counts the last, partial piece.
 template <typename T, int K, int P, bool ANY>
 __global__ __launch_bounds__(kBlock) void reduce_slots_gate_kernel(
@@ -100,7 +104,7 @@ int launch_reduce_gate(const void *rows, const int64_t *slot_to_row, const void 
                        void *out, int64_t n_tokens, int64_t top_k, int64_t n_rows, int64_t n_expert, int64_t row_elems,
                        hipStream_t st) {
     const int64_t row_vecs = ceil_div(row_elems * (int64_t)sizeof(T), 16);
-    constexpr int kPieces = K >= 8 ? 1 : K == 4 || sizeof(T) == 2 ? 2 : 4;
+    constexpr int kPieces = K >= 8 ? 1 : K == 4 || sizeof(T) == 2 ? 2 : 4;   // (K 4 and 8: float32)
 #define FMOE_RG(P)                                                                                                                    \
     {                                                                                                                                 \
         const int64_t groups = ceil_div(row_vecs, (P) * kWave), blocks = ceil_div(n_tokens * groups, kWavesPerBlock);                  \
@@ -420,11 +424,13 @@ int reduce_slots_gate(const void *rows, const int64_t *slot_to_row, const void *
 #define FMOE_RGK(T, ANY)                                                                                                          \
     {                                                                                                                             \
         if (top_k == 1) FMOE_RGT(T, 1, ANY);                                                                                      \
-        if (top_k == 2) FMOE_RGT(T, 2, ANY);                                                                                      \
-        if (top_k <= 4) FMOE_RGT(T, 4, ANY);                                                                                      \
-        FMOE_RGT(T, 8, ANY);                                                                                                      \
+        FMOE_RGT(T, 2, ANY);                                                                                                      \
     }
-    if (dtype == FMOE_F32) FMOE_RGK(float, false)
+    if (dtype == FMOE_F32) {
+        if (top_k > 4) FMOE_RGT(float, 8, false);
+        if (top_k > 2) FMOE_RGT(float, 4, false);
+        FMOE_RGK(float, false)
+    }
     if (dtype == FMOE_BF16) {
         if (any) FMOE_RGK(__bf16, true)
         FMOE_RGK(__bf16, false)
