@@ -48,3 +48,24 @@ def test_the_entry_points_for_whole_chunks_still_refuse(device):
         fmoe_native.gate_weight_grad(x[:, :1].contiguous(), idx, x, 4, False)
     with pytest.raises(Exception):
         fmoe_native.reduce_slots_gate(None, None, x[:, :1].contiguous(), idx, x, any_grid=False)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,d,k", [(70, 64, 3), (9, 1024, 5), (4200, 1024, 3), (4200, 1032, 7)])
+def test_sums_over_an_odd_number_of_slots(n, d, k, dtype, device):
+    """Slots are taken two (float32: four, eight) at a time: what is left at the end, dropped slots among them, with one and with several
+    pieces of a row per wave.  float32 sums of 2 k terms, then one rounding."""
+    g = torch.Generator(device=device).manual_seed(n + k)
+    e = 9
+    idx = torch.randn(n, e, device=device, generator=g).topk(k).indices
+    idx[::7, k - 1] = -1
+    rows = torch.randn(n * k, d, device=device, generator=g).to(dtype)
+    w, grad = torch.randn(e, d, device=device, generator=g).to(dtype), torch.randn(n, k, device=device, generator=g).to(dtype)
+    s2r = fmoe_native.route(idx, e)[2].view(-1)
+    got = fmoe_native.reduce_slots_gate(rows, s2r, grad, idx, w)
+    live = (idx >= 0).unsqueeze(-1)
+    picked = torch.where(live, rows.double()[s2r.clamp(min=0)].view(n, k, d), 0.0)
+    part = torch.where(live, w.double()[idx.clamp(min=0)] * grad.double().unsqueeze(-1), 0.0)
+    want, mag = picked.sum(1) + part.sum(1), picked.abs().sum(1) + part.abs().sum(1)
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}[dtype]
+    assert ((got.double() - want).abs() <= (2 * k + 1) * 2.0 ** -24 * mag + ulp * want.abs() + 2.0 ** -24).all()
