@@ -61,8 +61,8 @@ __global__ __launch_bounds__(kSkThreads, COL_BLOCKS == 4 ? 3 : 4) void grouped_g
     const DevTab dtab = (DevTab)(uintptr_t)prm.dev_tab;
     int place = __builtin_amdgcn_readfirstlane(blockIdx.x / prm.tiles_n);
     const int n0 = (blockIdx.x - place * prm.tiles_n) * (COL_BLOCKS * 16), K = prm.k_extent;
-    const DevTab4 order = (DevTab4)(dtab + prm.order_off);   // {expert, first row, rows}
-    const int live = dtab[segtab::kLive];
+    const DevTab4 order = (DevTab4)(dtab + prm.order_off);   // {expert, first row, rows}: of an expert, or (not APART) of a tile of at most 128 rows
+    const int live = dtab[APART ? segtab::kLive : segtab::kTiles128];
     int r0 = 0;   // first row
     i32x4 entry;
     if (APART && place < prm.extra_groups) {
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(kSkThreads, COL_BLOCKS == 4 ? 3 : 4) void grouped_g
         r0 = (skip + 1) * kSkRows;
     } else {
         place -= prm.extra_groups;
-        entry = order[place];   // (asked for together with their number; the launch has as many places as experts can have rows)
+        entry = order[place];   // (asked for together with their number; the launch has as many places as experts can have rows, or as there can be tiles)
         asm volatile("" : "+s"(entry));
         if (place >= live) return;
     }
@@ -281,13 +281,15 @@ template <typename T> int skinny_blocks(const SkinnyParams &prm, int64_t experts
 
 template <typename T> int launch(const SkinnyParams &params, int64_t rows_cap, int64_t n_expert, hipStream_t stream) {
     SkinnyParams prm = params;
-    prm.order_off = (int32_t)segtab::order_off(rows_cap, n_expert);
     // An expert's groups of rows go to workgroups of their own, where the experts come in order of their rows: the further groups first,
     // which leave at once where there are none.  128 experts of 1280 x 1280, 448 rows, 144 of them one expert's: 37 us in turn, 29 apart; 64 of 1280 x
     // 1280 in float32, 900 and 274: 116 and 82.
+    // More experts are in no order, and those with rows are found through the map of row tiles, at most as many as there are rows: 8192 experts of 64 x
+    // 1024, 8 slots: 9 us on 256 workgroups, where a place for each expert makes 262144 and 71; 2048 of 512 x 512, 64 slots: 9 and 17.
     const bool apart = n_expert <= segtab::kSmallExperts;
+    prm.order_off = (int32_t)(apart ? segtab::order_off(rows_cap, n_expert) : segtab::map128_off(rows_cap, n_expert));
     prm.extra_groups = apart ? (int32_t)(rows_cap / kSkRows) : 0;
-    const int64_t experts = apart ? std::min(rows_cap, n_expert) : n_expert;
+    const int64_t experts = apart ? std::min(rows_cap, n_expert) : segtab::cap_tiles(rows_cap, n_expert, 128);
     const int blocks = apart ? skinny_blocks<T>(prm, experts) : 2;
     prm.tiles_n = (int)ceil_div(prm.n_cols, 16 * blocks);
     const int64_t grid = (experts + prm.extra_groups) * prm.tiles_n;

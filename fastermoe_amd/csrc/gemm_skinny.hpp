@@ -14,7 +14,7 @@ struct SkinnyParams {
     uint32_t div_mul;
     int32_t div_shift;
     int32_t n_cols, k_extent, activation;
-    int32_t order_off, tiles_n, extra_groups;   // set by the launch: the table's list of experts, workgroups of a row group, see launch()
+    int32_t order_off, tiles_n, extra_groups;   // set by the launch: the table's list of experts (or its map of row tiles), see launch()
 };
 
 // rows_cap: the rows that the table was laid out for

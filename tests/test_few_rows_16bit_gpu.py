@@ -11,11 +11,12 @@ pytestmark = pytest.mark.gpu
 EDGES = [1, 0, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 130] + [0] * 120
 FEW = [1, 0, 2]
 MANY = [1, 0, 17, 40] + [0] * 1100 + [33]   # past 1024 experts, which are not in order of their rows
+TILES = [128, 129, 0, 300] + [0] * 1100 + [1, 256]   # there: experts of one row tile and of several
 
 
 # one, two and four blocks of 16 columns to a workgroup; contractions that end inside a line of 128 bytes, a unit, a turn of the waves
 @pytest.mark.parametrize("k,n,counts", [(8, 16, FEW), (264, 40, FEW), (72, 24, EDGES), (136, 200, EDGES), (1032, 264, EDGES), (520, 8200, FEW),
-                                        (200, 8136, EDGES), (72, 24, MANY)])
+                                        (200, 8136, EDGES), (72, 24, MANY), (72, 72, TILES)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_few_rows_in_16_bits(k, n, counts, dtype, device):
     """Against float64, element by element: 2 k + 8 roundings of float32 of the terms' absolute sum bound any order of the products,

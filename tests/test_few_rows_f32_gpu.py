@@ -8,15 +8,26 @@ pytestmark = pytest.mark.gpu
 
 # blocks of 16 rows, passes of 64, a tile of 128 and the next; experts without rows keep the average below the rule's line
 EDGES = [1, 0, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 130] + [0] * 9
+# past 1024 experts, which are not in order of their rows: row tiles of 128
+TILES = [1, 0, 17, 128, 129, 300] + [0] * 1100 + [33]
 
 
 @pytest.mark.parametrize("k,n", [(4, 4), (16, 16), (20, 36), (68, 20), (256, 64), (1028, 132)])
 @pytest.mark.parametrize("act", [_lib.ACT_NONE, _lib.ACT_RELU, _lib.ACT_GELU])
 def test_few_rows_in_float32(k, n, act, device):
+    against_float64(EDGES, k, n, act, device)
+
+
+@pytest.mark.parametrize("k,n", [(20, 36), (260, 68)])
+def test_few_rows_of_more_experts_than_the_table_sorts(k, n, device):
+    against_float64(TILES, k, n, _lib.ACT_RELU, device)
+
+
+def against_float64(sizes, k, n, act, device):
     """Against float64, element by element: 2 k + 8 roundings of float32 of the terms' absolute sum bound any order of the
     products, the waves' sums and the bias; GELU's own formula is within 1.5e-7 of its argument's size."""
-    counts = torch.tensor(EDGES)
-    e, rows = len(EDGES), sum(EDGES)
+    counts = torch.tensor(sizes)
+    e, rows = len(sizes), sum(sizes)
     slots = rows + 5
     assert slots <= 24 * e   # (the rule's line)
     g = torch.Generator().manual_seed(k + n)
@@ -31,7 +42,7 @@ def test_few_rows_in_float32(k, n, act, device):
     for src, kw in ((x, {}), (picked, dict(row_index=index, index_div=3))):
         y, pre = fmoe_native.linear_forward_dev(x, w, b, table, slots, act, act != _lib.ACT_NONE, **kw)
         lo = 0
-        for i, c in enumerate(EDGES):
+        for i, c in enumerate(sizes):
             a, we = src[lo:lo + c].double(), w[i].double()
             ref = a @ we.t() + b[i].double()
             bound = (2 * k + 8) * 2.0 ** -24 * (a.abs() @ we.abs().t() + b[i].double().abs())
