@@ -96,12 +96,6 @@ __global__ __launch_bounds__(kSkThreads, COL_BLOCKS == 4 ? 3 : 4) void grouped_g
     const __amdgpu_buffer_rsrc_t w_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(W), 0, w_bytes, kRsrcFlags);
     const uint32_t w_off = (uint32_t)(row8 * K * EB + chunk * 16), eight_rows = (uint32_t)(8 * K * EB);
     const bool gather = prm.row_index != nullptr;
-    const T *X = (const T *)prm.x + (gather ? (int64_t)0 : (int64_t)first * K);
-    const int x_bytes = gather ? (int)(prm.x_total_rows * K * EB) : rows * K * EB;
-    const __amdgpu_buffer_rsrc_t x_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(X), 0, x_bytes, kRsrcFlags);
-
-    const __amdgpu_buffer_rsrc_t index_rs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<int64_t *>(gather ? prm.row_index + first : nullptr), 0, gather ? rows * 8 : 0, kRsrcFlags);
 
     // NB blocks of 16 columns from column c0 of the workgroup on times RB blocks of 16 rows from the expert's row r0 on; a unit is LINES times
     // 128 bytes of contraction.  POLICY: of the weights' loads
@@ -110,6 +104,14 @@ __global__ __launch_bounds__(kSkThreads, COL_BLOCKS == 4 ? 3 : 4) void grouped_g
         constexpr int POLICY = decltype(policy_tag)::value;
         static_assert(NB * RB <= 2 * COL_BLOCKS && NB <= kSkWaves, "the waves' sums");
         struct Unit { u32x4 w[LINES][NB][2], x[LINES][RB][2]; };
+        // The rows, in a resource that begins at the pass's first or at the tile's: all of an expert can be more than the 2 GiB that offsets reach (bit
+        // 31 marks one as out of range), these are at most 32 or 128 of 4 MiB.  A gathered matrix is less than 2 GiB as a whole.
+        const int base = APART ? r0 : 0, base_rows = APART ? min(rows - r0, 16 * RB) : rows;
+        const int64_t base_at = (int64_t)first + base;
+        const __amdgpu_buffer_rsrc_t x_rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<T *>((const T *)prm.x + (gather ? (int64_t)0 : base_at * K)), 0, (int)(gather ? prm.x_total_rows : (int64_t)base_rows) * K * EB, kRsrcFlags);
+        const __amdgpu_buffer_rsrc_t index_rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<int64_t *>(gather ? prm.row_index + base_at : nullptr), 0, gather ? base_rows * 8 : 0, kRsrcFlags);
         const uint32_t w_base = w_off + (uint32_t)c0 * (uint32_t)(K * EB);
         const int n_units = (K + kLine * LINES - 1) / (kLine * LINES);
         const int turn = __builtin_amdgcn_readfirstlane((int)(blockIdx.x % (uint32_t)n_units));   // the unit it begins with
@@ -137,7 +139,7 @@ __global__ __launch_bounds__(kSkThreads, COL_BLOCKS == 4 ? 3 : 4) void grouped_g
 #pragma unroll
         for (int y = 0; y < RB; ++y)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) index[y][h] = __builtin_amdgcn_raw_buffer_load_b64(index_rs, (r0 + 16 * y + 8 * h + row8) * 8, 0, 0);
+            for (int h = 0; h < 2; ++h) index[y][h] = __builtin_amdgcn_raw_buffer_load_b64(index_rs, (r0 - base + 16 * y + 8 * h + row8) * 8, 0, 0);
         load_w(a, unit);
         __builtin_amdgcn_sched_barrier(0);
         uint32_t x_off[RB][2];
@@ -145,9 +147,9 @@ __global__ __launch_bounds__(kSkThreads, COL_BLOCKS == 4 ? 3 : 4) void grouped_g
         for (int y = 0; y < RB; ++y)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int row = r0 + 16 * y + 8 * h + row8;
+                const int row = r0 - base + 16 * y + 8 * h + row8;
                 uint32_t src = row;
-                bool valid = row < rows;
+                bool valid = row < base_rows;
                 if (gather) {
                     const uint32_t idx = index[y][h][0];
                     src = prm.div_shift < 0 ? idx : __umulhi(idx, prm.div_mul) >> prm.div_shift;

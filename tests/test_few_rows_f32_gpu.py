@@ -72,3 +72,25 @@ def test_the_rows_past_the_counts_are_left_alone(act, device, monkeypatch):
     for t in (y, pre):
         if t is not None:
             assert t.shape[0] == 64 and (t[:5] != marker).all() and (t[5:] == torch.tensor(marker, device=device)).all()
+
+
+# (the second: past 1024 experts, and past 4 GiB)
+@pytest.mark.parametrize("e,rows", [(1024, 12288), (2048, 24576)])
+def test_rows_of_one_expert_past_two_gib(e, rows, device):
+    """All rows are one expert's, more than 32-bit offsets reach.  Small whole numbers: sums below 2^24, exact in any order.  The last rows are
+    infinite, so that a row which reads them in place of what lies past its contraction is not a number."""
+    k, n, one = 43720, 4, e - 3
+    assert (1 << 31) * (rows // 12288) < rows * k * 4 and rows <= 12 * e and 6 * k < 1 << 24
+    g = torch.Generator(device=device).manual_seed(e)
+    x = torch.empty(rows, k, device=device)
+    for part in x.split(2048):
+        part.copy_(torch.randint(-1, 3, part.shape, device=device, generator=g, dtype=torch.int8))
+    x[-8:] = float("inf")
+    w = torch.zeros(e, n, k, device=device)
+    w[one] = torch.randint(-3, 4, (n, k), device=device, generator=g).float()
+    counts = torch.zeros(e, dtype=torch.int64)
+    counts[one] = rows
+    table = fmoe_native.segment_table(counts.to(device), rows)
+    y = fmoe_native.linear_forward_dev(x, w, None, table, rows)[0]
+    for got, part in zip(y[:-8].split(2048), x[:-8].split(2048)):
+        assert torch.equal(got, (part.double() @ w[one].double().t()).float())
