@@ -387,6 +387,9 @@ bool gate_grad_any_grid(int64_t d_model, int64_t n_expert, int64_t top_k, int dt
 
 int gate_weight_grad(const void *grad_score, const int64_t *topk_idx, const void *x, void *grad_w, void *grad_b, int64_t n_tokens,
                      int64_t d_model, int64_t n_expert, int64_t top_k, int dtype, void *workspace, int64_t workspace_bytes, hipStream_t st) {
+    if (!gate_grad_any_grid(d_model, n_expert, top_k, dtype))
+        return fail(FMOE_ELIMIT, "fmoe_gate_weight_grad: d_model=%lld n_expert=%lld top_k=%lld dtype=%d is not taken", (long long)d_model,
+                    (long long)n_expert, (long long)top_k, dtype);
     FMOE_REQUIRE(n_tokens >= 1 && n_tokens * top_k <= (int64_t)INT32_MAX, "fmoe_gate_weight_grad: n_tokens=%lld", (long long)n_tokens);
     FMOE_REQUIRE(grad_score && topk_idx && x && grad_w && aligned16(x), "fmoe_gate_weight_grad: NULL or misaligned pointer");
     const int64_t need = fmoe_gate_weight_grad_workspace_bytes(n_tokens, d_model, n_expert);
@@ -416,7 +419,8 @@ int reduce_slots_gate(const void *rows, const int64_t *slot_to_row, const void *
         return fail(FMOE_ELIMIT, "fmoe_reduce_slots_gate: sizes beyond the supported range");
     FMOE_REQUIRE(grad_score && topk_idx && w && out && (rows || n_rows == 0 || slot_to_row == nullptr), "fmoe_reduce_slots_gate: NULL pointer");
     const bool any = (row_elems * dtype_bytes(dtype)) % 16 != 0;
-    FMOE_REQUIRE(!any || dtype != FMOE_F32, "fmoe_reduce_slots_gate: rows must be whole 16-byte chunks");
+    FMOE_REQUIRE((!any || dtype != FMOE_F32) && aligned16(rows) && aligned16(w) && aligned16(out),
+                 "fmoe_reduce_slots_gate: misaligned pointer, or rows that are no whole 16-byte chunks");
     // (bytes: the experts' rows and the result; the gate's part alone: its weight, once, and the result)
     ProfileScope prof(kProfReduceSlots, (double)(slot_to_row ? (top_k + 1) * n_tokens : n_tokens + n_expert) * row_elems * dtype_bytes(dtype), st);
 #define FMOE_RGT(T, K, ANY)                                                                                                       \
@@ -473,9 +477,6 @@ extern "C" int fmoe_gate_grad_any_supported(int64_t d_model, int64_t n_expert, i
 extern "C" int fmoe_gate_weight_grad_any(const void *grad_score, const int64_t *topk_idx, const void *x, void *grad_w, void *grad_b,
                                          int64_t n_tokens, int64_t d_model, int64_t n_expert, int64_t top_k, int dtype, void *workspace,
                                          int64_t workspace_bytes, void *stream) {
-    if (!gate_grad_any_grid(d_model, n_expert, top_k, dtype))
-        return fail(FMOE_ELIMIT, "fmoe_gate_weight_grad_any: d_model=%lld n_expert=%lld top_k=%lld dtype=%d is not taken", (long long)d_model,
-                    (long long)n_expert, (long long)top_k, dtype);
     return gate_weight_grad(grad_score, topk_idx, x, grad_w, grad_b, n_tokens, d_model, n_expert, top_k, dtype, workspace, workspace_bytes,
                             (hipStream_t)stream);
 }
@@ -483,7 +484,6 @@ extern "C" int fmoe_gate_weight_grad_any(const void *grad_score, const int64_t *
 extern "C" int fmoe_reduce_slots_gate_any(const void *rows, const int64_t *slot_to_row, const void *grad_score, const int64_t *topk_idx,
                                           const void *w, void *out, int64_t n_tokens, int64_t top_k, int64_t n_rows, int64_t n_expert,
                                           int64_t row_elems, int dtype, void *stream) {
-    FMOE_REQUIRE(aligned16(rows) && aligned16(w) && aligned16(out), "fmoe_reduce_slots_gate_any: misaligned pointer");
     return reduce_slots_gate(rows, slot_to_row, grad_score, topk_idx, w, out, n_tokens, top_k, n_rows, n_expert, row_elems, dtype,
                              (hipStream_t)stream);
 }

@@ -254,6 +254,12 @@ extern "C" int fmoe_layer_backward(const void *grad_out, const void *x, const vo
     const void *saved_pre = activation == FMOE_ACT_GELU ? pre : mid;   // (ReLU's derivative can be read off its output)
     FMOE_REQUIRE(grad_out && x && w1 && w2 && topk_score && pos && slot_to_row && segment_table && saved_pre && mid && rows && grad_score &&
                      (!gated || (topk_idx && gate_w)), "fmoe_layer_backward: NULL pointer");
+    // (what the gate's kernels would refuse, before anything is enqueued)
+    if (gated && grad_gate_w != nullptr && !gate_grad_any_grid(d_model, n_expert, top_k, dtype))
+        return fail(FMOE_ELIMIT, "fmoe_layer_backward: gradients of a gate of d_model=%lld n_expert=%lld top_k=%lld dtype=%d are not taken",
+                    (long long)d_model, (long long)n_expert, (long long)top_k, dtype);
+    FMOE_REQUIRE(!gated || grad_x == nullptr || (aligned16(gate_w) && aligned16(grad_x)), "fmoe_layer_backward: misaligned gate_w or grad_x");
+    FMOE_REQUIRE(!gated || grad_gate_w == nullptr || aligned16(x), "fmoe_layer_backward: misaligned x");
     hipStream_t st = (hipStream_t)stream;
     int rc = fmoe_gather_combine_backward(grad_out, rows, slot_to_row, topk_score, b.rows, grad_score, n_tokens, top_k, s.n_slots, d_model,
                                           dtype, stream);

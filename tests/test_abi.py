@@ -371,3 +371,30 @@ def test_sorted_rows_are_asked_for_by_the_activation_too(monkeypatch):
     monkeypatch.setenv("FMOE_GELU_ERF", "1")
     assert ask(_lib.ACT_GELU, 1) == ask(_lib.ACT_GELU, 0) == 0
     assert ask(_lib.ACT_RELU, 0) == 1
+
+
+def test_layer_backward_refuses_a_gate_before_any_launch():
+    """Gradients of a gate of more than 256 experts, and a gate's weight, input or input gradient off 16 bytes: refused by the call itself (a launch
+    would fail otherwise here, where there is no device).  Without the weight's gradient more experts are taken."""
+    lib = _lib.load()
+    n, d, h, k = 4, 64, 128, 2
+    at = 1 << 20   # (never read)
+
+    def call(e, dtype=_lib.BF16, wanted=("grad_x", "grad_gate_w"), **change):
+        ptr = dict.fromkeys(("grad_out", "x", "gate_w", "w1", "w2", "topk_idx", "topk_score", "pos", "slot_to_row", "segment_table", "pre", "mid",
+                             "rows"), at)
+        ptr.update({name: at if name in wanted else None for name in ("grad_x", "grad_score", "grad_gate_w", "grad_gate_b", "grad_w1", "grad_b1",
+                                                                      "grad_w2", "grad_b2")})
+        ptr.update(change)
+        rc = lib.fmoe_layer_backward(*ptr.values(), n, d, h, e, k, dtype, _lib.ACT_GELU, _lib.GATE_LOGITS, at, 1 << 40, None)
+        return rc, lib.fmoe_last_error()
+
+    for e in (257, 8192):
+        rc, why = call(e)
+        assert rc == -2 and b"fmoe_layer_backward" in why   # FMOE_ELIMIT
+    for change in ({"gate_w": at + 2}, {"grad_x": at + 8}, {"x": at + 8}):
+        rc, why = call(256, **change)
+        assert rc == -1 and b"misaligned" in why
+    if not torch.cuda.is_available():
+        for e, wanted in ((256, ("grad_x", "grad_gate_w")), (8192, ("grad_x",))):
+            assert b"fmoe_layer_backward" not in call(e, wanted=wanted)[1]   # (no refusal: the launch fails)
