@@ -411,7 +411,7 @@ int gate_weight_grad(const void *grad_score, const int64_t *topk_idx, const void
 }
 
 int reduce_slots_gate(const void *rows, const int64_t *slot_to_row, const void *grad_score, const int64_t *topk_idx, const void *w, void *out,
-                      int64_t n_tokens, int64_t top_k, int64_t n_rows, int64_t n_expert, int64_t row_elems, int dtype, hipStream_t st) {
+                      int64_t n_tokens, int64_t top_k, int64_t n_rows, int64_t n_expert, int64_t row_elems, int dtype, bool any_grid, hipStream_t st) {
     FMOE_REQUIRE(dtype == FMOE_F32 || dtype == FMOE_BF16 || dtype == FMOE_F16, "fmoe_reduce_slots_gate: dtype %d", dtype);
     FMOE_REQUIRE(n_tokens >= 0 && top_k >= 1 && n_rows >= 0 && n_expert >= 1 && row_elems >= 0, "fmoe_reduce_slots_gate: bad sizes");
     if (n_tokens == 0 || row_elems == 0) return FMOE_OK;
@@ -419,7 +419,7 @@ int reduce_slots_gate(const void *rows, const int64_t *slot_to_row, const void *
         return fail(FMOE_ELIMIT, "fmoe_reduce_slots_gate: sizes beyond the supported range");
     FMOE_REQUIRE(grad_score && topk_idx && w && out && (rows || n_rows == 0 || slot_to_row == nullptr), "fmoe_reduce_slots_gate: NULL pointer");
     const bool any = (row_elems * dtype_bytes(dtype)) % 16 != 0;
-    FMOE_REQUIRE((!any || dtype != FMOE_F32) && aligned16(rows) && aligned16(w) && aligned16(out),
+    FMOE_REQUIRE((!any || (any_grid && dtype != FMOE_F32)) && aligned16(rows) && aligned16(w) && aligned16(out),
                  "fmoe_reduce_slots_gate: misaligned pointer, or rows that are no whole 16-byte chunks");
     // (bytes: the experts' rows and the result; the gate's part alone: its weight, once, and the result)
     ProfileScope prof(kProfReduceSlots, (double)(slot_to_row ? (top_k + 1) * n_tokens : n_tokens + n_expert) * row_elems * dtype_bytes(dtype), st);
@@ -484,15 +484,13 @@ extern "C" int fmoe_gate_weight_grad_any(const void *grad_score, const int64_t *
 extern "C" int fmoe_reduce_slots_gate_any(const void *rows, const int64_t *slot_to_row, const void *grad_score, const int64_t *topk_idx,
                                           const void *w, void *out, int64_t n_tokens, int64_t top_k, int64_t n_rows, int64_t n_expert,
                                           int64_t row_elems, int dtype, void *stream) {
-    return reduce_slots_gate(rows, slot_to_row, grad_score, topk_idx, w, out, n_tokens, top_k, n_rows, n_expert, row_elems, dtype,
+    return reduce_slots_gate(rows, slot_to_row, grad_score, topk_idx, w, out, n_tokens, top_k, n_rows, n_expert, row_elems, dtype, true,
                              (hipStream_t)stream);
 }
 
 extern "C" int fmoe_reduce_slots_gate(const void *rows, const int64_t *slot_to_row, const void *grad_score, const int64_t *topk_idx,
                                       const void *w, void *out, int64_t n_tokens, int64_t top_k, int64_t n_rows, int64_t n_expert,
                                       int64_t row_elems, int dtype, void *stream) {
-    FMOE_REQUIRE((row_elems * dtype_bytes(dtype)) % 16 == 0 && aligned16(rows) && aligned16(w) && aligned16(out),
-                 "fmoe_reduce_slots_gate: rows must be whole 16-byte chunks");
-    return reduce_slots_gate(rows, slot_to_row, grad_score, topk_idx, w, out, n_tokens, top_k, n_rows, n_expert, row_elems, dtype,
+    return reduce_slots_gate(rows, slot_to_row, grad_score, topk_idx, w, out, n_tokens, top_k, n_rows, n_expert, row_elems, dtype, false,
                              (hipStream_t)stream);
 }

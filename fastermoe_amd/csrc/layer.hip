@@ -278,7 +278,7 @@ extern "C" int fmoe_layer_backward(const void *grad_out, const void *x, const vo
         if (rc != FMOE_OK) return rc;
         // (the gate's part of the input gradient is added in the same pass, before the one rounding)
         rc = gated ? reduce_slots_gate(b.rows, slot_to_row, grad_score, topk_idx, gate_w, grad_x, n_tokens, top_k, s.n_slots, n_expert,
-                                       d_model, dtype, st)
+                                       d_model, dtype, true, st)
                    : fmoe_reduce_slots(b.rows, slot_to_row, grad_x, n_tokens, top_k, s.n_slots, d_model, dtype, stream);
         if (rc != FMOE_OK) return rc;
     }

@@ -398,3 +398,16 @@ def test_layer_backward_refuses_a_gate_before_any_launch():
     if not torch.cuda.is_available():
         for e, wanted in ((256, ("grad_x", "grad_gate_w")), (8192, ("grad_x",))):
             assert b"fmoe_layer_backward" not in call(e, wanted=wanted)[1]   # (no refusal: the launch fails)
+
+
+@pytest.mark.parametrize("entry", ["fmoe_reduce_slots_gate", "fmoe_reduce_slots_gate_any"])
+def test_sums_over_no_slots_need_no_whole_chunks(entry):
+    """A call without tokens, or with rows of no elements, has nothing to do wherever its tensors lie; with something to do it refuses what it always did."""
+    lib = _lib.load()
+    call = lambda n, elems, dtype, w=1 << 20: getattr(lib, entry)(None, None, 1 << 20, 1 << 20, w, 1 << 20, n, 2, 0, 4, elems, dtype, None)
+    for dtype in (_lib.BF16, _lib.F16, _lib.F32):
+        assert call(0, 7, dtype) == 0 and call(0, 8, dtype, w=(1 << 20) + 2) == 0 and call(5, 0, dtype, w=(1 << 20) + 2) == 0
+        assert call(5, 8, dtype, w=(1 << 20) + 2) == -1 and call(-1, 8, dtype) == -1
+    assert call(5, 7, _lib.F32) == -1 and call(5, 8, 99) == -1 and call(0, 8, 99) == -1
+    if entry == "fmoe_reduce_slots_gate":
+        assert call(5, 7, _lib.BF16) == -1
