@@ -10,8 +10,9 @@
 //     sixteen rows, the operands' own shape, read nontemporally: 5.5, as the halves of a line are fetched apart);
 //   * the rows' loads, which take as many places in a unit's queue of loads as the weights' do, serve two or four blocks of 16 columns
 //     (one block: 362 us for that layer's pass, without the rows' loads 300);
-//   * each workgroup begins its contraction one unit further on than the one before, so that they don't all ask the same channels for
-//     the same columns at once (162 -> 142 us for 14336 x 4096);
+//   * each workgroup of an expert begins its contraction one unit further on than the one before, so that they don't all ask the same
+//     channels for the same columns at once (162 -> 142 us for 14336 x 4096); where it begins is its expert's and its columns' own, so that a row's
+//     sum, in the order of the units from there on, does not depend on how many rows other experts have;
 //   * the compiler may not move a unit's loads behind the products of the one before, which left none in flight at their end.
 // Where it is used, and what it measured: use_skinny() in grouped_gemm.hip.
 #include "gemm_skinny.hpp"
@@ -60,7 +61,7 @@ __global__ __launch_bounds__(kSkThreads, COL_BLOCKS == 4 ? 3 : 4) void grouped_g
 
     const DevTab dtab = (DevTab)(uintptr_t)prm.dev_tab;
     int place = __builtin_amdgcn_readfirstlane(blockIdx.x / prm.tiles_n);
-    const int n0 = (blockIdx.x - place * prm.tiles_n) * (COL_BLOCKS * 16), K = prm.k_extent;
+    const int tile_n = blockIdx.x - place * prm.tiles_n, n0 = tile_n * (COL_BLOCKS * 16), K = prm.k_extent;
     const DevTab4 order = (DevTab4)(dtab + prm.order_off);   // {expert, first row, rows}: of an expert, or (not APART) of a tile of at most 128 rows
     const int live = dtab[APART ? segtab::kLive : segtab::kTiles128];
     int r0 = 0;   // first row
@@ -85,6 +86,8 @@ __global__ __launch_bounds__(kSkThreads, COL_BLOCKS == 4 ? 3 : 4) void grouped_g
     }
     const int expert = entry[0], first = entry[1], rows = entry[2];
     if (rows == 0) return;
+    // where its contraction begins, by expert and columns alone: a row's sum does not depend on the rows that other experts have
+    const uint32_t start = __builtin_amdgcn_readfirstlane((uint32_t)expert * (uint32_t)prm.tiles_n + (uint32_t)tile_n);
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int lb = lane & 15, hq = lane >> 4;
     // A load takes 128 bytes of eight rows, this lane 16 bytes of row lane % 8 (see pair_to_steps)
@@ -114,7 +117,7 @@ __global__ __launch_bounds__(kSkThreads, COL_BLOCKS == 4 ? 3 : 4) void grouped_g
             const_cast<int64_t *>(gather ? prm.row_index + base_at : nullptr), 0, gather ? base_rows * 8 : 0, kRsrcFlags);
         const uint32_t w_base = w_off + (uint32_t)c0 * (uint32_t)(K * EB);
         const int n_units = (K + kLine * LINES - 1) / (kLine * LINES);
-        const int turn = __builtin_amdgcn_readfirstlane((int)(blockIdx.x % (uint32_t)n_units));   // the unit it begins with
+        const int turn = __builtin_amdgcn_readfirstlane((int)(start % (uint32_t)n_units));   // the unit it begins with
         // (offsets past the contraction, as of every unit past it, have the sign bit set)
         auto line_offset = [&](int unit, int l) -> uint32_t {
             const int at = unit + turn < n_units ? unit + turn : unit + turn - n_units;
@@ -254,17 +257,17 @@ __global__ __launch_bounds__(kSkThreads, COL_BLOCKS == 4 ? 3 : 4) void grouped_g
         pass(All{}, One{}, std::integral_constant<int, COL_BLOCKS == 1 ? 2 : 1>{}, Nontemporal{}, 0, 0);
         return;
     }
-    const int cols = min(COL_BLOCKS * 16, prm.n_cols - n0);
-    for (int c0 = 0; c0 < cols; c0 += 16 * UpToTwo::value) {
+    auto up_to_two = [&](int c0) {
         if (rows <= kSkRows) {
             pass(UpToTwo{}, Two{}, One{}, Nontemporal{}, c0, 0);
         } else if constexpr (APART) {
             pass(UpToTwo{}, Two{}, One{}, Cached{}, c0, r0);
         } else {
-            for (; r0 < rows; r0 += kSkRows) pass(UpToTwo{}, Two{}, One{}, Cached{}, c0, r0);
-            r0 = 0;
+            for (int row = 0; row < rows; row += kSkRows) pass(UpToTwo{}, Two{}, One{}, Cached{}, c0, row);
         }
-    }
+    };
+    up_to_two(0);
+    if (COL_BLOCKS > 2 && prm.n_cols - n0 > 32) up_to_two(32);
 #endif
 }
 
