@@ -7,7 +7,8 @@
 // up their accumulators through LDS in a fixed order.  What it takes to come near the 6.9 TB/s that such loads alone reach here
 // (8 experts of 4096 x 14336, 8 rows each: 189 us before, 137 now; of 14336 x 4096: 187 and 142):
 //   * a load takes whole lines, 128 bytes of eight rows, and leaves no trace in the caches (6.2 TB/s through them; 64 bytes of
-//     sixteen rows, the operands' own shape, read nontemporally: 5.5, as the halves of a line are fetched apart);
+//     sixteen rows, the operands' own shape, read nontemporally: 5.5, as the halves of a line are fetched apart), unless the weights are read
+//     again soon and fit there (weights_cached);
 //   * the rows' loads, which take as many places in a unit's queue of loads as the weights' do, serve two or four blocks of 16 columns
 //     (one block: 362 us for that layer's pass, without the rows' loads 300);
 //   * each workgroup of an expert begins its contraction one unit further on than the one before, so that they don't all ask the same
@@ -254,11 +255,13 @@ __global__ __launch_bounds__(kSkThreads, COL_BLOCKS == 4 ? 3 : 4) void grouped_g
     // (Two units have to fit 168 registers: scratch memory costs launches that never touch it a tenth of their time.  The weights of an
     // expert with several groups are read again, from the caches.)
     if (rows <= 16) {
-        pass(All{}, One{}, std::integral_constant<int, COL_BLOCKS == 1 ? 2 : 1>{}, Nontemporal{}, 0, 0);
+        const std::integral_constant<int, COL_BLOCKS == 1 ? 2 : 1> lines;
+        if (prm.weights_cached) pass(All{}, One{}, lines, Cached{}, 0, 0);
+        else pass(All{}, One{}, lines, Nontemporal{}, 0, 0);
         return;
     }
     auto up_to_two = [&](int c0) {
-        if (rows <= kSkRows) {
+        if (rows <= kSkRows && !prm.weights_cached) {
             pass(UpToTwo{}, Two{}, One{}, Nontemporal{}, c0, 0);
         } else if constexpr (APART) {
             pass(UpToTwo{}, Two{}, One{}, Cached{}, c0, r0);

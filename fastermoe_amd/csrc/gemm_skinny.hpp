@@ -14,6 +14,7 @@ struct SkinnyParams {
     uint32_t div_mul;
     int32_t div_shift;
     int32_t n_cols, k_extent, activation;
+    int32_t weights_cached;       // not 0: the weights through the caches, see caches_few_row_weights() in grouped_gemm.hip
     int32_t order_off, tiles_n, extra_groups;   // set by the launch: the table's list of experts (or its map of row tiles), see launch()
 };
 

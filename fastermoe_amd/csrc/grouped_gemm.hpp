@@ -85,6 +85,8 @@ struct LinearForwardArgs {
     int64_t dev_workspace_bytes = 0;
     // with dev_tab: 16-bit tensors and feature sizes off the 16-byte grid are taken too (gemm_unaligned.hip)
     bool dev_any_grid = false;
+    // with dev_tab: nothing will read the weights again soon, as a backward would
+    bool dev_weights_once = false;
 };
 
 // Bytes of workspace with which a launch over a device table can split its last round of tiles along a

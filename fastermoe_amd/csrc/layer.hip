@@ -133,7 +133,7 @@ int sort_rows(const Sizes &s, const void *x, const int64_t *pos, const int64_t *
 
 // one expert linear over the sorted rows of a segment table
 int linear_forward(const Sizes &s, const void *x, const int64_t *row_index, const void *w, const void *b, void *pre, void *y,
-                   const void *table, int64_t in_feat, int64_t out_feat, int activation, void *ws, int64_t ws_bytes, hipStream_t st) {
+                   const void *table, int64_t in_feat, int64_t out_feat, int activation, bool keep, void *ws, int64_t ws_bytes, hipStream_t st) {
     const bool plain = activation == FMOE_ACT_NONE && pre == nullptr;
     LinearForwardArgs a{x, w, b, y, pre, in_feat, out_feat, s.dtype, plain ? kEpiStore : kEpiBiasAct, activation};
     a.x_row_index = row_index;
@@ -144,6 +144,7 @@ int linear_forward(const Sizes &s, const void *x, const int64_t *row_index, cons
     a.dev_workspace = ws_bytes ? ws : nullptr;
     a.dev_workspace_bytes = ws_bytes;
     a.dev_any_grid = true;
+    a.dev_weights_once = !keep;
     return grouped_linear_forward(a, nullptr, s.n_expert, 0, s.n_slots, st);
 }
 int linear_dgrad(const Sizes &s, const void *gy, const void *w, const void *pre, void *gx, const void *table, int64_t in_feat,
@@ -228,9 +229,9 @@ extern "C" int fmoe_layer_forward(const void *x, const void *gate_w, const void 
     }
     hipStream_t st = (hipStream_t)stream;
     rc = linear_forward(s, token_rows ? x : rows, token_rows ? pos : nullptr, w1, b1, keep_pre ? pre : nullptr, mid, segment_table, d_model,
-                        d_hidden, activation, f.split_ws, f.split1, st);
+                        d_hidden, activation, keep != 0, f.split_ws, f.split1, st);
     if (rc != FMOE_OK) return rc;
-    rc = linear_forward(s, mid, nullptr, w2, b2, nullptr, rows, segment_table, d_hidden, d_model, FMOE_ACT_NONE, f.split_ws, f.split2, st);
+    rc = linear_forward(s, mid, nullptr, w2, b2, nullptr, rows, segment_table, d_hidden, d_model, FMOE_ACT_NONE, keep != 0, f.split_ws, f.split2, st);
     if (rc != FMOE_OK) return rc;
     return fmoe_gather_combine_forward(rows, slot_to_row, topk_score, out, n_tokens, top_k, s.n_slots, d_model, dtype, stream);
 }

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from fastermoe_amd import fmoe_native
+from fastermoe_amd import _lib, fmoe_native, functions
 
 pytestmark = pytest.mark.gpu
 
@@ -33,3 +33,29 @@ def test_a_row_has_the_same_sum_whatever_the_other_experts_have(k, n, dtype, dev
         for other in results[1:]:
             assert torch.equal(other, results[0])
         assert torch.equal(results[0][0], results[0][rows - 1])
+
+
+# an expert's rows on both sides of a block's 16, a group's 32 and the next; one, two and (16 bits) four blocks of columns to a workgroup
+COUNTS = [1, 0, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 130] + [0] * 120
+
+
+@pytest.mark.parametrize("d,h", [(24, 40), (136, 200), (264, 8200)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_inference_and_training_have_the_same_result(d, h, dtype, device):
+    """Weights past the caches where nothing is differentiated, through them where a backward will read them: what is read is the same, bit for bit."""
+    e, n = len(COUNTS), sum(COUNTS)
+    assert n <= 4 * e and 2 * e * d * h < 1 << 30   # (the rule's line; either side of what the caches hold)
+    g = torch.Generator().manual_seed(d)
+    idx = torch.repeat_interleave(torch.arange(e), torch.tensor(COUNTS))[torch.randperm(n, generator=g)].unsqueeze(1).to(device)
+    new = lambda *s: torch.randn(*s, generator=g).to(dtype).to(device)
+    x, score, w1, b1, w2, b2 = new(n, d), new(n, 1), new(e, h, d) / d ** 0.5, new(e, h), new(e, d, h) / h ** 0.5, new(e, d)
+    counts, pos, slot_to_row = fmoe_native.route(idx, e)
+    routing = pos, slot_to_row.view(-1), fmoe_native.segment_table(counts, n)
+    args = x, None, None, score, w1, b1, w2, b2, routing, 1, _lib.ACT_RELU, _lib.GATE_ROUTED
+    with torch.no_grad():
+        once = functions.layer_call(*args)
+    w1.requires_grad_(True)
+    kept = functions.layer_call(*args)
+    assert kept.requires_grad and not once.requires_grad and torch.equal(kept.detach(), once)
+    rows = torch.cat([torch.relu(x[t] @ w1[i].t() + b1[i]) @ w2[i].t() + b2[i] for t, i in zip(range(3), idx[:3, 0].tolist())]).view(3, d)
+    assert (once[:3] - rows * score[:3]).float().norm() <= 0.02 * (rows * score[:3]).float().norm()
