@@ -6,6 +6,8 @@ raises, and every operator of the package fails with it.  Build it with
 """
 import ctypes
 import os
+import sys
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # FMOE_HIP_LIB points at another build of the same library (e.g. an experiment)
@@ -127,24 +129,32 @@ def load():
     return lib
 
 
-_layer_call = None
+_layer_call = False   # not asked for yet
 
 
 def load_layer_call():
-    """The extension module ``fastermoe_amd/lib/_layer_call.so``, which calls the library's layer from Python's tensors."""
+    """The extension module ``fastermoe_amd/lib/_layer_call.so``, which calls the library's layer from Python's tensors.  ``None``, and one
+    warning, where there is none for this torch and Python: the library needs neither, and its layer is then called from Python."""
     global _layer_call
-    if _layer_call is None:
-        path = os.path.join(_HERE, "lib", "_layer_call.so")
-        if not os.path.exists(path):
-            raise ImportError(f"{path} is missing: the host extension has not been built (run `python -m fastermoe_amd.build`)")
+    if _layer_call is False:
         import importlib.machinery
         import importlib.util
-        import torch  # noqa: F401  (its libraries have to be there first)
-        lib = load()
-        loader = importlib.machinery.ExtensionFileLoader("_layer_call", path)
-        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_layer_call", loader))
-        loader.exec_module(module)
-        module.bind(*(ctypes.cast(fn, _vp).value for fn in (lib.fmoe_layer_sizes, lib.fmoe_layer_forward)))
+        import torch   # (its libraries have to be there first)
+        path = os.path.join(_HERE, "lib", "_layer_call.so")
+        here = f"{torch.__version__} {sys.implementation.cache_tag}"
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("_layer_call", path)
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_layer_call", loader))
+            loader.exec_module(module)
+            built_for = getattr(module, "built_for", "another torch")
+            if built_for != here:
+                raise ImportError(f"{path} was built for {built_for}, this is {here}")
+        except ImportError as why:
+            warnings.warn(f"inference calls the layer from Python, some 10 us slower: {why} (run `python -m fastermoe_amd.build`)", RuntimeWarning)
+            module = None
+        else:
+            lib = load()
+            module.bind(*(ctypes.cast(fn, _vp).value for fn in (lib.fmoe_layer_sizes, lib.fmoe_layer_forward)))
         _layer_call = module
     return _layer_call
 

@@ -60,8 +60,9 @@ def _build_layer_call():
     """The extension module of csrc/layer_call.cpp."""
     import torch
     from torch.utils.cpp_extension import include_paths, library_paths
+    built_for = f"{torch.__version__} {sys.implementation.cache_tag}"   # what _lib.load_layer_call() compares
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           f"-I{sysconfig.get_path('include')}", *(f"-I{p}" for p in include_paths()), os.path.join(CSRC, "layer_call.cpp"), "-o", LAYER_CALL,
+           f'-DFMOE_BUILT_FOR="{built_for}"', f"-I{sysconfig.get_path('include')}", *(f"-I{p}" for p in include_paths()), os.path.join(CSRC, "layer_call.cpp"), "-o", LAYER_CALL,
            *(f"-L{p}" for p in library_paths()), "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10"]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     return proc.returncode, "_layer_call.so", proc.stdout

@@ -106,4 +106,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_layer_call", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__layer_call() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__layer_call() {
+    PyObject *m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddStringConstant(m, "built_for", FMOE_BUILT_FOR) < 0) Py_CLEAR(m);   // (torch's and Python's versions)
+    return m;
+}

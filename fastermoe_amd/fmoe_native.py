@@ -798,7 +798,7 @@ def linear_wgrad_dev(grad_y, x, weight, table, rows_cap, with_bias):
 
 def layer_infer(inp, gate_w, gate_b, score, routing, w1, b1, w2, b2, top_k, activation, gate):
     """The layer's output where nothing will be differentiated (``routing``: ``pos_buf``, ``slot_to_row`` and the segment table of a gate
-    outside, whose scores ``score`` are), or ``None`` where the call does not take these tensors."""
+    outside, whose scores ``score`` are), or ``None`` where the call does not take these tensors.  Needs :func:`_lib.load_layer_call`."""
     pos, slot_to_row, table = routing if routing is not None else (None, None, None)
     with _on(inp.device):
         out = _lib.load_layer_call().infer(inp, gate_w, gate_b, score, pos, slot_to_row, table, w1, b1, w2, b2, top_k, activation, gate, _stream(inp))
@@ -852,22 +852,24 @@ class LayerRouting:
                 self.kept[score_at:score_at + n * dtype.itemsize].view(dtype).view(n_tokens, top_k))
 
 
-def layer_forward(inp, gate_w, gate_b, logits, w1, b1, w2, b2, top_k, activation, gate, sizes, routing):
+def layer_forward(inp, gate_w, gate_b, logits, w1, b1, w2, b2, top_k, activation, keep, gate, sizes, routing):
     """Gate, routing, experts and combine as one call, over tensors that the caller has checked against
     :func:`layer_sizes` (contiguous, on 16 bytes, one type and device).  Returns ``(out, pre, mid, rows)``, the last three
-    for the backward (``pre`` ``None`` where ``mid`` tells as much)."""
+    for the backward (``pre`` ``None`` where ``mid`` tells as much), all ``None`` unless ``keep``."""
     n, d = inp.shape
     e, h = w1.shape[:2]
     new = lambda r, c: torch.empty(r, c, dtype=inp.dtype, device=inp.device)
     out = new(n, d)
-    pre = new(n * top_k, h) if activation == _lib.ACT_GELU else None
-    mid, rows = new(n * top_k, h), new(n * top_k, d)
+    pre = mid = rows = None
+    if keep:
+        pre = new(n * top_k, h) if activation == _lib.ACT_GELU else None
+        mid, rows = new(n * top_k, h), new(n * top_k, d)
     scratch = torch.empty(sizes[0], dtype=torch.uint8, device=inp.device)
     idx, score, pos, s2r, table = routing.pointers(n * top_k, sizes[2])
     with _on(inp.device):
         check(_lib.load().fmoe_layer_forward(
             inp.data_ptr(), _ptr(gate_w), _ptr(gate_b), _ptr(logits), w1.data_ptr(), _ptr(b1), w2.data_ptr(), _ptr(b2), idx, score, pos,
-            s2r, table, _ptr(pre), mid.data_ptr(), rows.data_ptr(), out.data_ptr(), n, d, h, e, top_k, _DTYPES[inp.dtype], activation, 1, gate,
+            s2r, table, _ptr(pre), _ptr(mid), _ptr(rows), out.data_ptr(), n, d, h, e, top_k, _DTYPES[inp.dtype], activation, keep, gate,
             scratch.data_ptr(), sizes[0], _stream(inp)))
     return out, pre, mid, rows
 

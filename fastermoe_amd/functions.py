@@ -9,7 +9,7 @@ import torch
 from torch.autograd import Function
 from torch.utils._device import DeviceContext
 
-from . import fmoe_native
+from . import _lib, fmoe_native
 
 
 def _single_worker(world_size, what):
@@ -464,7 +464,7 @@ class MOELayer(Function):
         else:
             place = fmoe_native.LayerRouting(score, *routing)
         out, pre, mid, rows = fmoe_native.layer_forward(inp, gate_w, gate_b, _gate_logits(gate, inp, gate_w, gate_b), w1, b1, w2, b2,
-                                                        top_k, activation, gate, sizes, place)
+                                                        top_k, activation, 1, gate, sizes, place)
         ctx.save_for_backward(inp, gate_w, w1, w2, pre, mid, rows, place.kept, *place.tensors)
         ctx.moe_args = top_k, activation, gate, sizes, [b is not None for b in (gate_b, b1, b2)]
         return out
@@ -510,7 +510,8 @@ def _gate_logits(gate, inp, gate_w, gate_b):
 def layer_call(inp, gate_w, gate_b, score, w1, b1, w2, b2, routing, top_k, activation, gate):
     r"""The layer's output through :class:`MOELayer`, or, where nothing will be differentiated, through the same call without
     a node; ``None`` where the call does not take these tensors (see :func:`fmoe_native.layer_sizes`)."""
-    if not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (inp, gate_w, gate_b, score, w1, b1, w2, b2))):
+    keep = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (inp, gate_w, gate_b, score, w1, b1, w2, b2))
+    if not keep and _lib.load_layer_call() is not None:
         return fmoe_native.layer_infer(inp, gate_w, gate_b, score, routing, w1, b1, w2, b2, top_k, activation, gate)
     n, d = inp.shape
     e, h = w1.shape[0], w1.shape[1]
@@ -523,9 +524,14 @@ def layer_call(inp, gate_w, gate_b, score, w1, b1, w2, b2, routing, top_k, activ
             or (b2 is not None and b2.shape != (e, d)) or (gate_w is not None and gate_w.shape != (e, d))
             or (gate_b is not None and gate_b.shape != (e,))):
         return None
-    sizes = fmoe_native.layer_sizes(n, d, h, e, top_k, dtype, activation, 1, gate)
+    sizes = fmoe_native.layer_sizes(n, d, h, e, top_k, dtype, activation, int(keep), gate)
     if sizes is None:
         return None
+    if not keep:
+        inp = inp.contiguous()
+        place = fmoe_native.LayerRouting() if routing is None else fmoe_native.LayerRouting(score, *routing)
+        return fmoe_native.layer_forward(inp, gate_w, gate_b, _gate_logits(gate, inp, gate_w, gate_b), w1, b1, w2, b2, top_k, activation, 0,
+                                         gate, sizes, place)[0]
     return MOELayer.apply(inp, gate_w, gate_b, score, w1, b1, w2, b2, routing, top_k, activation, gate, sizes)
 
 

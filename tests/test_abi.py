@@ -411,3 +411,30 @@ def test_sums_over_no_slots_need_no_whole_chunks(entry):
     assert call(5, 7, _lib.F32) == -1 and call(5, 8, 99) == -1 and call(0, 8, 99) == -1
     if entry == "fmoe_reduce_slots_gate":
         assert call(5, 7, _lib.BF16) == -1
+
+
+@pytest.mark.parametrize("there", ["nothing", "no library", "another torch"])
+def test_without_the_extension_module_there_is_a_warning_and_no_failure(there, tmp_path, monkeypatch):
+    """The library needs no torch; the module that calls its layer from tensors is for one torch and Python.  Where it is missing, cannot be loaded or is
+    another's, the callers get None, and one warning."""
+    import shutil
+    import warnings
+    (tmp_path / "lib").mkdir()
+    path = tmp_path / "lib" / "_layer_call.so"
+    if there == "no library":
+        path.write_bytes(b"\x7fELF and no more")
+    if there == "another torch":
+        shutil.copy(os.path.join(os.path.dirname(_lib.__file__), "lib", "_layer_call.so"), path)
+        monkeypatch.setattr(torch, "__version__", "1.2.3")
+    monkeypatch.setattr(_lib, "_HERE", str(tmp_path))
+    monkeypatch.setattr(_lib, "_layer_call", False)
+    with pytest.warns(RuntimeWarning, match="_layer_call.so" if there != "another torch" else "this is 1.2.3"):
+        assert _lib.load_layer_call() is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.load_layer_call() is None
+
+
+def test_the_extension_module_is_for_this_torch(monkeypatch):
+    monkeypatch.setattr(_lib, "_layer_call", False)
+    assert callable(_lib.load_layer_call().infer)

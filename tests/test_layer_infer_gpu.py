@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from fastermoe_amd import _lib, fmoe_native
+from fastermoe_amd import _lib, fmoe_native, functions
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +41,21 @@ def test_a_failing_call_raises(device):
         fmoe_native.layer_infer(**dict(tensors(device), gate=_lib.GATE_ROUTED))   # no routing is given
     with pytest.raises(TypeError):
         fmoe_native.layer_infer(**dict(tensors(device), gate_w=1))
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float16, 52), (torch.float32, 64)])
+@pytest.mark.parametrize("outside", [False, True])
+def test_without_the_extension_module_the_result_is_the_same(dtype, d, outside, device, monkeypatch):
+    """The layer's call from Python: bit for bit, with the gate inside (off the 16-byte grid: its logits a library product) and outside."""
+    gate = _lib.GATE_LINEAR if d % 8 == 0 else _lib.GATE_LOGITS
+    t = tensors(device, d=d, dtype=dtype, h=128 if d % 8 == 0 else 100)
+    if outside:
+        idx, score = torch.randn(5, 4, device=device).topk(2).indices, torch.randn(5, 2, device=device).to(dtype)
+        cnt, pos, slot_to_row = fmoe_native.route(idx, 4)
+        t.update(gate_w=None, gate_b=None, score=score, routing=(pos, slot_to_row.view(-1), fmoe_native.segment_table(cnt, 10)))
+        gate = _lib.GATE_ROUTED
+    args = [t[k] for k in ("inp", "gate_w", "gate_b", "score", "w1", "b1", "w2", "b2", "routing", "top_k", "activation")] + [gate]
+    with torch.no_grad():
+        native = functions.layer_call(*args)
+        monkeypatch.setattr(_lib, "_layer_call", None)
+        assert native is not None and torch.equal(functions.layer_call(*args), native)
