@@ -34,6 +34,12 @@ int dtype_code(at::ScalarType t) {
 bool on_16_bytes(const at::Tensor &t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0; }
 void *pointer(const at::Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
 
+// The interpreter's lock, given back while this lives
+struct WithoutLock {
+    PyThreadState *state = PyEval_SaveThread();
+    ~WithoutLock() { PyEval_RestoreThread(state); }
+};
+
 PyObject *bind(PyObject *, PyObject *args) {
     unsigned long long sizes, forward;
     if (!PyArg_ParseTuple(args, "KK", &sizes, &forward)) return nullptr;
@@ -80,18 +86,23 @@ PyObject *infer(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     int64_t sizes[3] = {};
     if (layer_sizes(n, d, h, e, top_k, dtype, (int)activation, 0, (int)gate, sizes) != 1) Py_RETURN_NONE;
 
-    const at::Tensor inp = given.contiguous();
-    const at::Tensor logits = gate == FMOE_GATE_LOGITS ? at::linear(inp, gate_w, gate_b.defined() ? std::optional<at::Tensor>(gate_b) : std::nullopt) : at::Tensor();
-    const at::TensorOptions like = at::TensorOptions().dtype(inp.scalar_type()).device(inp.device());
-    at::Tensor out = at::empty({n, d}, like);
-    const at::Tensor scratch = at::empty({sizes[0]}, like.dtype(at::kByte));
+    // Other threads of the interpreter go on from here, as they do in torch's own operators: an allocation may wait for the device, and the
+    // library product of the logits, like the launches, for a full queue.
+    at::Tensor out;
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = layer_forward(pointer(inp), pointer(gate_w), pointer(gate_b), pointer(logits), pointer(w1), pointer(b1), pointer(w2), pointer(b2), nullptr,
-                       pointer(score), (int64_t *)pointer(pos), (int64_t *)pointer(slot_to_row), pointer(table), nullptr, nullptr, nullptr,
-                       pointer(out), n, d, h, e, top_k, dtype, (int)activation, 0, (int)gate, pointer(scratch), sizes[0],
-                       reinterpret_cast<void *>(static_cast<uintptr_t>(stream)));
-    Py_END_ALLOW_THREADS
+    {
+        const WithoutLock no_lock;
+        const at::Tensor inp = given.contiguous();
+        const at::Tensor logits = gate == FMOE_GATE_LOGITS
+                                      ? at::linear(inp, gate_w, gate_b.defined() ? std::optional<at::Tensor>(gate_b) : std::nullopt) : at::Tensor();
+        const at::TensorOptions like = at::TensorOptions().dtype(inp.scalar_type()).device(inp.device());
+        out = at::empty({n, d}, like);
+        const at::Tensor scratch = at::empty({sizes[0]}, like.dtype(at::kByte));
+        rc = layer_forward(pointer(inp), pointer(gate_w), pointer(gate_b), pointer(logits), pointer(w1), pointer(b1), pointer(w2), pointer(b2), nullptr,
+                           pointer(score), (int64_t *)pointer(pos), (int64_t *)pointer(slot_to_row), pointer(table), nullptr, nullptr, nullptr,
+                           pointer(out), n, d, h, e, top_k, dtype, (int)activation, 0, (int)gate, pointer(scratch), sizes[0],
+                           reinterpret_cast<void *>(static_cast<uintptr_t>(stream)));
+    }
     if (rc != FMOE_OK) return PyLong_FromLong(rc);
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS

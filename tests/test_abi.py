@@ -438,3 +438,46 @@ def test_without_the_extension_module_there_is_a_warning_and_no_failure(there, t
 def test_the_extension_module_is_for_this_torch(monkeypatch):
     monkeypatch.setattr(_lib, "_layer_call", False)
     assert callable(_lib.load_layer_call().infer)
+
+
+def test_the_extension_module_lets_other_threads_run():
+    """While it works on tensors, here in the product of the logits, another thread of the interpreter goes on: no pause between two of its steps
+    is as long as half that product.  (The library's entry points are stand-ins, so that it needs no device.)"""
+    import ctypes
+    import threading
+    import time
+    lib, module = _lib.load(), _lib.load_layer_call()
+    restype, argtypes = _lib.SIGNATURES["fmoe_layer_sizes"]
+    sizes = ctypes.CFUNCTYPE(restype, *argtypes)(lambda *a: ctypes.cast(a[-1], ctypes.POINTER(ctypes.c_int64)).__setitem__(0, 16) or 1)
+    restype, argtypes = _lib.SIGNATURES["fmoe_layer_forward"]
+    forward = ctypes.CFUNCTYPE(restype, *argtypes)(lambda *a: -7)
+    n, d, e = 4096, 2048, 1024
+    x, gate_w = torch.randn(n, d), torch.randn(e, d)
+    w1, w2 = torch.zeros(e, 1, d), torch.zeros(e, d, 1)
+    threads, steps, done = torch.get_num_threads(), [], threading.Event()
+
+    def other():
+        while not done.is_set():
+            steps.append(time.perf_counter())
+            time.sleep(0.001)
+
+    address = lambda fn: ctypes.cast(fn, ctypes.c_void_p).value
+    torch.set_num_threads(1)
+    try:
+        module.bind(address(sizes), address(forward))
+        torch.nn.functional.linear(x, gate_w)
+        begin = time.perf_counter()
+        torch.nn.functional.linear(x, gate_w)
+        product = time.perf_counter() - begin
+        thread = threading.Thread(target=other)
+        thread.start()
+        time.sleep(0.01)
+        rc = module.infer(x, gate_w, None, None, None, None, None, w1, None, w2, None, 1, _lib.ACT_RELU, _lib.GATE_LOGITS, 0)
+        time.sleep(0.01)
+    finally:
+        done.set()
+        module.bind(address(lib.fmoe_layer_sizes), address(lib.fmoe_layer_forward))
+        torch.set_num_threads(threads)
+    thread.join()
+    assert rc == -7 and product > 0.02
+    assert max(b - a for a, b in zip(steps, steps[1:])) < product / 2, product
