@@ -6,13 +6,14 @@ from fastermoe_amd import _lib, fmoe_native
 
 pytestmark = pytest.mark.gpu
 
-# blocks of 16 rows, passes of 64, a tile of 128 and the next; experts without rows keep the average below the rule's line
+# blocks of 16 rows, groups of 32, a tile of 128 and the next; experts without rows keep the average below the rule's line
 EDGES = [1, 0, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 130] + [0] * 9
 # past 1024 experts, which are not in order of their rows: row tiles of 128
 TILES = [1, 0, 17, 128, 129, 300] + [0] * 1100 + [33]
 
 
-@pytest.mark.parametrize("k,n", [(4, 4), (16, 16), (20, 36), (68, 20), (256, 64), (1028, 132)])
+# (one block of 16 columns to a workgroup, and two where 22 experts make a workgroup of them for each of 256 compute units)
+@pytest.mark.parametrize("k,n", [(4, 4), (16, 16), (20, 36), (68, 20), (256, 64), (1028, 132), (68, 388), (260, 356)])
 @pytest.mark.parametrize("act", [_lib.ACT_NONE, _lib.ACT_RELU, _lib.ACT_GELU])
 def test_few_rows_in_float32(k, n, act, device):
     against_float64(EDGES, k, n, act, device)
