@@ -5,8 +5,8 @@
 // it, those entries are written into a dense [tokens, experts] matrix and go through two library products a few columns wide, two
 // reductions for the bias and one more pass over the input gradient to add the gate's part:
 //   grad_x[t] = experts' part + sum_j g[t,j] w[idx[t,j]]      grad_w[e] = sum over (t,j) with idx = e of g[t,j] x[t]
-// Here the gate's part of the first is a sum of top_k rows of w per token (a caller that has the experts' part as rows gets
-// both sums in one pass; the layer does not call it so), and the second is one pass over x with the matrix cores.
+// Here the gate's part of the first is a sum of top_k rows of w per token (a caller that has the experts' part as rows, as the layer's
+// backward does, gets both sums in one pass), and the second is one pass over x with the matrix cores.
 #include "gate_grad.hpp"
 #include "profile.hpp"
 #include "vec16.hpp"
@@ -24,17 +24,18 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 // ---- input gradient: reduce_slots plus the gate's part ---------------------------------------
-// A wave owns P pieces of 64 vectors (1 KiB) of one token's row and has all K P loads of rows and of w in flight together: the
-// slots' experts (and rows) are a dependent load before them, scalar ones as they are the same for the wave, and w's rows come
-// from the caches.  The gate's node asks for its part alone (rows null), the sum with the experts' rows is for callers
-// that have them.  us for the gate's part with P = 1 / 2 / 4 (and with the rows, against reduce_slots alone): bf16, 32768 tokens of
+// A wave owns P pieces of 64 vectors (1 KiB) of one token's row and takes its slots K at a time, with all K P loads of rows and of w in
+// flight together: the slots' experts (and rows) are a dependent load before them, scalar ones as they are the same for the wave, and w's
+// rows come from the caches.  The layer's backward hands in the experts' rows, the gate's own node asks for its part alone (rows null).
+// us for the gate's part with P = 1 / 2 / 4 and all slots at a time (and with the rows, against reduce_slots alone): bf16, 32768 tokens of
 // 4096, 8 experts, top-2: 73 / 62 / 69 (147 / 141 / 150, 133), 16384 of 2048, 64 experts, top-1: 15.0 / 12.3 / 12.8
 // (27.9 / 25.5 / 26.7, 23.5), 16384 of 4096, top-4: 55 / 54 / 64; float32, 32768 of 4096, top-2: 115 / 87 / 81, top-4 at 16384:
 // 87 / 71 / 84.  As a library product over the dense gradient the first took 99.
 // Tokens or rows too few for that many waves take P = 1.
 // More than two slots: 16-bit types two at a time, so that seven or eight waves fit a SIMD where the loads of all slots and pieces at once leave four
 // (top-8, 8192 tokens of 2048, 256 experts: 71.7 -> 56.4 us, 32768 of 512: 72.0 -> 58.2; top-4, 16384 of 4096: 120.5 -> 113.4, 8192 of
-// 1024: 17.8 either way; the order of the sums is the same).  float32 as many as there are, whose rows are twice the bytes for the same sums (8192 of
+// 1024: 17.8 either way; launches that leave the chip waves to spare wait twice, 64 tokens of 2048, top-8: 5.7 -> 6.1; the order of the sums
+// is the same).  float32 as many as there are, whose rows are twice the bytes for the same sums (8192 of
 // 2048, top-8: 103.4, two at a time 107.3).
 // ANY (16-bit types): rows of any length, read 16 bytes at a time wherever they lie; row_vecs counts the last, partial piece.
 template <typename T, int K, int P, bool ANY>

@@ -402,6 +402,8 @@ bool use_ring(const TileShape &tile, int dtype) {
 // 8: 64 of 2048 x 8192 384 / 333, 256 of 1088 x 2176 258 / 227).  Fewer tiles: 8 of 4096 x 14336, 8 rows: 187 / 138; 8 of 14336 x 4096, 8 / 12:
 // 176 / 146, 176 / 156; 12 of 512 x 1792, 12: 11.3 / 8.1; 16 of 768 x 3072, 12, at random / shares 1 / rank^1.2: 23.4 / 19.5, 24.1 / 20.5; of 3072
 // x 768: 31.5 / 21.8, 34.7 / 29.1; 32 of 768 x 3072, 13, a third of them one's: 41 / 36, of 3072 x 768: 36 / 41; 32 of 1024 x 1024, 15: 19.7 / 20.1.
+// What the lines cost where a gate sends all rows to one expert (weights read again per 32 rows, where one round of tiles has them once): 8 of 4096 x
+// 14336, 96 rows: 39 / 89; 32 of 768 x 3072, 384: 13 / 18; 256 of 2048 x 1024, 1024: 23 / 32; 64 of 4096 x 1024, 256: 39 / 32.
 // float32: at most 24 rows per expert on average, 12 of contractions from 4096 on and 32 of shorter ones where the 128 x 128 tiles would
 // number less than half the compute units; as many as two passes take in all (64) whatever the contraction.  64 experts of 1216 x 1216, 1 row
 // each: 105 / 44; 8 of 1792 x 6272, 1.5: 140 / 46; 32 of 1024 x 3584, 16: 194 / 102; 64 of 1280 x 1280, 14, a third of the rows one's: 116 / 82; 256
@@ -421,7 +423,8 @@ bool use_skinny(int64_t rows_cap, int64_t n_expert, int64_t in_feat, int64_t out
 // in L2, lose what that costs; the line lies where an even spread rarely makes a second tile.  us through the caches and past them, weights
 // from memory, forward (the data gradients gain as much): 256 experts of 768 -> 3072, 9.5 rows each: 275 / 251; 64 of 2048 -> 1024, 30: 72 / 67; 32 of
 // 3328 -> 3328, 96, a fifth of the rows one's: 204 / 183; 32 of 2048 -> 4096, 106: 164 / 152; 16 of 2560 -> 2560, 216 (tiles of 256): 80 / 73; past
-// the line 128 of 1664 -> 832, 136 (tiles of 128): 136 / 151; 12 of 3328 -> 960, 264: 53 / 66; 4 of 4352 -> 1088, 320: 35 / 40.  (The
+// the line 128 of 1664 -> 832, 136 (tiles of 128): 136 / 151; 12 of 3328 -> 960, 264: 53 / 66; 4 of 4352 -> 1088, 320: 35 / 40.  Where all rows are
+// one expert's: 128 of 2048 -> 2048, 40 on average: 53 / 65; 64 of 2048 -> 8192, 16: 37 / 40.  (The
 // persistent kernel's launches have more row tiles: all their weights past the caches cost 64 experts with shares 1 / rank^1.2 of 16384 rows 7 %.)
 // Weights that the memory-side cache (256 MiB) can hold together with the layer's other linear stay as they were: loads past the caches
 // drop them from it, and the next product that reads them waits for memory (16 experts of 768 x 3072, 2000 rows, a training step

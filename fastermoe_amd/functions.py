@@ -71,8 +71,8 @@ class GateTopK(Function):
 class GateLinearTopK(Function):
     r"""``nn.Linear`` -> ``torch.topk`` (-> softmax) of fmoe/gates/naive_gate.py:26-42 and the routing of
     ``count_by_gate`` in one call that keeps the logits on chip.  Returns ``(topk_idx, topk_score)`` like
-    :class:`GateTopK`; the routing rides on ``topk_idx``.  Gates of more experts than that call takes run the linear
-    layer as a library product first.  Backward: straight from the gradient of the selected logits; a softmax over
+    :class:`GateTopK`; the routing rides on ``topk_idx``.  Gates of more experts than that call takes, or with 16-bit rows
+    off the 16-byte grid, run the linear layer as a library product first.  Backward: straight from the gradient of the selected logits; a softmax over
     them, a shape these kernels do not take, or ``create_graph`` goes through the dense gradient of the logits and library products."""
 
     @staticmethod
@@ -130,7 +130,8 @@ def _plain_linear(linear):
 def gate_linear_topk(x, linear, top_k, score_mode=0):
     r"""Top-k indices and scores of ``linear(x)`` for an ``nn.Linear`` gate: one fused call when the
     shape is taken (CUDA tensors, at most 64 experts, ``top_k`` 1, 2, 4 or 8, rows of whole 16-byte
-    chunks; ``FMOE_GATE_LINEAR_FUSED=0`` switches it off), else the layer followed by :func:`gate_topk`."""
+    chunks; ``FMOE_GATE_LINEAR_FUSED=0`` switches it off); one node over a library product where the gate's gradients take the shape
+    (up to 256 experts, 16-bit rows of any length); else the layer followed by :func:`gate_topk`."""
     import os
     w, b = linear.weight, linear.bias
     if (x.is_cuda and x.dim() == 2 and w.is_cuda and w.dtype == x.dtype and (b is None or b.dtype == x.dtype)
