@@ -150,11 +150,11 @@ def load_layer_call():
             if built_for != here:
                 raise ImportError(f"{path} was built for {built_for}, this is {here}")
         except ImportError as why:
+            _layer_call = None   # (before the warning, which may be an error)
             warnings.warn(f"inference calls the layer from Python, some 10 us slower: {why} (run `python -m fastermoe_amd.build`)", RuntimeWarning)
-            module = None
-        else:
-            lib = load()
-            module.bind(*(ctypes.cast(fn, _vp).value for fn in (lib.fmoe_layer_sizes, lib.fmoe_layer_forward)))
+            return None
+        lib = load()
+        module.bind(*(ctypes.cast(fn, _vp).value for fn in (lib.fmoe_layer_sizes, lib.fmoe_layer_forward)))
         _layer_call = module
     return _layer_call
 

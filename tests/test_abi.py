@@ -430,6 +430,10 @@ def test_without_the_extension_module_there_is_a_warning_and_no_failure(there, t
     monkeypatch.setattr(_lib, "_layer_call", False)
     with pytest.warns(RuntimeWarning, match="_layer_call.so" if there != "another torch" else "this is 1.2.3"):
         assert _lib.load_layer_call() is None
+    monkeypatch.setattr(_lib, "_layer_call", False)
+    with warnings.catch_warnings(), pytest.raises(RuntimeWarning):   # (where warnings are errors: once)
+        warnings.simplefilter("error")
+        _lib.load_layer_call()
     with warnings.catch_warnings():
         warnings.simplefilter("error")
         assert _lib.load_layer_call() is None
